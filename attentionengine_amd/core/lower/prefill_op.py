@@ -13,6 +13,7 @@ import os
 import torch
 
 from ..runtime import hip_rt as rt
+from ..runtime import host
 from ..transform.core import _convert_mask_to_block_mask, is_causal_mask
 from . import lower as L
 from .mask import plan_mask
@@ -136,6 +137,8 @@ class PrefillOp:
             raise NotImplementedError("too many rowscales / custom inputs")
         self.final_rowscales = {}
         self.block_mask = None
+        # calls of a shape that has run before (csrc/ae_host.cpp)
+        self._host = host.new_host(self.D, self.DV, self.dtype, self.functors.customs, self.n_rowscales)
         self._variants = {}   # (mask_mode, even_q, even_kv) -> (module, cfg, config_src)
         self._plans = {}      # (B|1, H|1, Sq, Skv) -> MaskPlan with device table
         self.meta_shape = (_dim(q_meta.shape[0], 1), _dim(q_meta.shape[1], 1), _dim(q_meta.shape[2], 0),
@@ -163,6 +166,7 @@ class PrefillOp:
         self.tiles = L.PrefillTiles()
         self._variants.clear()
         self._plans.clear()
+        self._host.clear()
         self._bwd = None            # (the backward reads this operator's mask plans: built again on demand)
         self.gave_way_to_generic = True
         return True
@@ -322,7 +326,15 @@ class PrefillOp:
     # ---- launch ----------------------------------------------------------------------------
     def __call__(self, q, k, v, *extra):
         """Forward; records the autograd edge when a gradient of q, k or v is wanted (the reference's
-        generated ``_attention`` autograd function, attn_tl.py:530-640)."""
+        generated ``_attention`` autograd function, attn_tl.py:530-640).  A call whose shape has run before is
+        checked and launched natively (csrc/ae_host.cpp), autograd edge included."""
+        if extra and extra[-1] is self.block_mask and self.block_mask is not None and not self.extern_block_mask:
+            done = self._host.run(q, k, v, *extra[:-1])        # (the mask inferred from mask_mod itself: see _forward_once)
+        else:
+            done = self._host.run(q, k, v, *extra)
+        if done is not None:
+            self.final_rowscales = dict(zip(self.functors.final_rowscale_names, done[1:]))
+            return done[0]
         if torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in (q, k, v)):
             return _PrefillFunction.apply(self, q, k, v, *extra)
         return self._forward(q, k, v, *extra)
@@ -442,6 +454,11 @@ class PrefillOp:
                 rt.prefill_fwd(kern, p, cfg, stream)
         self.final_rowscales = dict(zip(self.functors.final_rowscale_names, rowscales))
         self._keepalive = keep
+        if extern_mask is None and self.DV_launch == self.DV and not self._clock_stamps():
+            host.add_forward(self._host, host.PREFILL_SPLIT if n_split > 1 else host.PREFILL, B, Sq, Hq, Hkv, Skv, dev, module,
+                             kern, cfg, combine=module.kernel("ae_decode_combine_kernel") if n_split > 1 else None,
+                             ccfg=ccfg if n_split > 1 else None, n_split=n_split, kv_per_split=kv_per_split,
+                             table=table if mode == 2 else None, mask_block=(mbm, mbn), env=("AE_CLOCK_STAMPS",))
         return out
 
 

@@ -1,6 +1,7 @@
 """Build steps for the native side of the package.
 
   build_library()       g++ + hipcc -> csrc/libae_hip.so (the C ABI of include/ae_hip.h)
+  build_host()          g++ -> csrc/_ae_host.so (the native host path of repeated calls, linked against it)
   check_templates()     hipcc --offload-arch=gfx950 -c of every kernel template, with headers
                         generated for a representative configuration (offline "does it build")
 
@@ -20,6 +21,7 @@ REPO = osp.dirname(PKG)
 INCLUDE = osp.join(REPO, "include")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 LIB = osp.join(CSRC, "libae_hip.so")
+HOST = osp.join(CSRC, "_ae_host.so")
 
 # device flags shared with the hipRTC path (core/runtime/hip_rt.py: COMPILE_OPTS)
 DEVICE_FLAGS = ["-O3", "-std=c++17", "-fno-math-errno", "-fno-trapping-math", "-fno-signed-zeros",
@@ -54,6 +56,21 @@ def build_library(verbose=False):
     return LIB
 
 
+def build_host():
+    """csrc/ae_host.cpp -> csrc/_ae_host.so: a Python extension on torch's C++ interface and libae_hip.so."""
+    import sysconfig
+    import torch
+    t = osp.dirname(torch.__file__)
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          f"-I{INCLUDE}", f"-isystem{t}/include", f"-isystem{t}/include/torch/csrc/api/include", f"-isystem{ROCM}/include",
+          f"-isystem{sysconfig.get_paths()['include']}", osp.join(CSRC, "ae_host.cpp"),
+          f"-L{CSRC}", "-lae_hip", f"-L{t}/lib", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python",
+          "-Wl,-rpath,$ORIGIN", "-o", HOST + ".tmp"])
+    os.replace(HOST + ".tmp", HOST)
+    return HOST
+
+
 def check_templates(header_sets, verbose=False):
     """Cross-compile kernel templates for gfx950 with hipcc.
 
@@ -77,7 +94,7 @@ def check_templates(header_sets, verbose=False):
 
 
 if __name__ == "__main__":
-    print("built", build_library(verbose=True))
+    print("built", build_library(verbose=True), build_host())
     sys.path.insert(0, REPO)
     import __graft_entry__ as g
     check_templates(g.representative_headers(), verbose=True)
