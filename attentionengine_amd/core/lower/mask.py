@@ -108,8 +108,10 @@ class MaskPlan:
     apply the elementwise mask, 2 = visit, fully visible.
     """
 
-    def __init__(self, mode: int, table=None, block_m: int = 0, block_n: int = 0, elementwise: bool = False):
+    def __init__(self, mode: int, table=None, block_m: int = 0, block_n: int = 0, elementwise: bool = False, band=None):
         self.mode = mode
+        # (lo, hi) where the mask of mode 2 is exactly lo <= q_idx - kv_idx <= hi (hi None: no far edge at this size)
+        self.band = band
         self.table = table
         self.block_m = block_m
         self.block_n = block_n
@@ -136,6 +138,8 @@ def plan_mask(mask_mod, lowered: LoweredMask, B: int, H: int, Sq: int, Skv: int,
     n_kt = (Skv + tile_n - 1) // tile_n
     table = torch.zeros(mb, mh, n_qt, n_kt, dtype=torch.int8)
     exactly_causal = True
+    band = (mb, mh) == (1, 1) and elementwise
+    d_lo, d_hi, seen = Sq + Skv, -(Sq + Skv), 0       # extremes of q - kv over the visible positions, and their number
     chunk_rows = max(tile_m, (chunk_rows // tile_m) * tile_m)
     kv = torch.arange(Skv).view(1, 1, 1, Skv)
     bb = torch.arange(mb).view(mb, 1, 1, 1)
@@ -149,6 +153,15 @@ def plan_mask(mask_mod, lowered: LoweredMask, B: int, H: int, Sq: int, Skv: int,
         m = m.to(torch.bool).expand(mb, mh, r1 - r0, Skv)
         if exactly_causal:
             exactly_causal = bool(torch.equal(m, (q >= kv).expand_as(m)))
+        if band:
+            rows = m[0, 0]
+            any_row = rows.any(dim=1)
+            if bool(any_row.any()):
+                qr = torch.arange(r0, r1)[any_row]
+                first = rows[any_row].to(torch.int8).argmax(dim=1)
+                last = Skv - 1 - rows[any_row].flip(1).to(torch.int8).argmax(dim=1)
+                d_lo, d_hi = min(d_lo, int((qr - last).min())), max(d_hi, int((qr - first).max()))
+            seen += int(rows.sum())
         # a block cut by the sequence end is "full" when every in-range element is visible
         vis = _count_blocks(m, tile_m, tile_n)
         tot = _count_blocks(torch.ones(1, 1, r1 - r0, Skv, dtype=torch.bool), tile_m, tile_n)
@@ -163,7 +176,16 @@ def plan_mask(mask_mod, lowered: LoweredMask, B: int, H: int, Sq: int, Skv: int,
         # mask_value != "-inf": the forward only skips tiles (attn_tl.py:124-137 guards the
         # elementwise test with is_inf_mask); visited tiles are treated as fully visible.
         table = torch.where(table > 0, torch.full_like(table, 2), table)
+    if band and seen and seen == band_size(Sq, Skv, d_lo, d_hi):
+        return MaskPlan(2, table.contiguous(), tile_m, tile_n, elementwise, (d_lo, None if d_hi >= Sq - 1 else d_hi))
     return MaskPlan(2, table.contiguous(), tile_m, tile_n, elementwise)
+
+
+def band_size(Sq: int, Skv: int, lo: int, hi: int) -> int:
+    """Number of positions of a [Sq, Skv] grid with lo <= q - kv <= hi.  A mask whose visible positions all lie in the
+    band and are as many as the band has is the band."""
+    q = torch.arange(Sq)
+    return int(((q - lo).clamp(max=Skv - 1) - (q - hi).clamp(min=0) + 1).clamp(min=0).sum())
 
 
 def _count_blocks(mask: torch.Tensor, bm: int, bn: int) -> torch.Tensor:

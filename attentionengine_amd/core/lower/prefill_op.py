@@ -177,7 +177,8 @@ class PrefillOp:
         n_split, _ = self.plan_splits(B, H, Sq, Skv)
         _, _, cfg_src = self._variant(mode, Sq % self.tiles.block_m == 0, Skv % self.tiles.block_n == 0, n_split,
                                       self._table_rows(self.mask_block[0] if self.extern_block_mask else plan.block_m),
-                                      plan.heavy_last and not self.extern_block_mask)
+                                      plan.heavy_last and not self.extern_block_mask,
+                                      None if self.extern_block_mask else self._band(plan))
         self.source = cfg_src + "\n" + self.functor_src
         if infer_mask and mask_mod is not None and not self.extern_block_mask:
             self.block_mask = self._reference_block_mask(B, H, Sq, Skv)
@@ -225,7 +226,7 @@ class PrefillOp:
             plan = plan_mask(self.mask_mod, self.functors.mask, B, H, Sq, Skv, self.tiles.block_m,
                              self.tiles.block_n, elementwise=self.elementwise_mask)
             self._plans[key] = plan
-        if device is not None and plan.table is not None and plan.table.device != device:
+        if device is not None and plan.table is not None and plan.table.device != device and self._band(plan) is None:
             plan.table = plan.table.to(device)
         return plan
 
@@ -290,10 +291,16 @@ class PrefillOp:
         rows = max(1, -(-self.tiles.block_m // int(mask_block_m)))
         return next(r for r in (1, 2, 4, 8) if r >= min(rows, 8))
 
-    def _variant(self, mask_mode, even_q, even_kv, n_split=1, table_rows=1, heavy_last=False):
+    def _band(self, plan):
+        """The mask's band (MaskPlan.band) where the kernel takes one instead of the tile table."""
+        return plan.band if self.tiles.template == "ae_prefill.hip" else None
+
+    def _variant(self, mask_mode, even_q, even_kv, n_split=1, table_rows=1, heavy_last=False, band=None):
+        if mask_mode != 2 or band is not None:
+            table_rows = 1
         if mask_mode != 2:
-            table_rows, heavy_last = 1, False
-        key = (mask_mode, even_q, even_kv, n_split, table_rows, bool(heavy_last))
+            heavy_last = False
+        key = (mask_mode, even_q, even_kv, n_split, table_rows, bool(heavy_last), band)
         v = self._variants.get(key)
         if v is None:
             has_mask_mod = self.elementwise_mask and mask_mode != 1
@@ -306,6 +313,9 @@ class PrefillOp:
                 cfg_src += "#define AE_MASK_VALUE_ZERO 1\n"
             if mask_mode == 2:
                 cfg_src += f"#define AE_TT_ROWS {table_rows}\n#define AE_HEAVY_LAST {1 if heavy_last else 0}\n"
+            if band is not None:
+                cfg_src += (f"#define AE_BAND 1\n#define AE_BAND_LO ({band[0]})\n"
+                            f"#define AE_BAND_HI {'0x7fffffff' if band[1] is None else f'({band[1]})'}\n")
             if n_split > 1:
                 cfg_src += f"#define AE_NSPLIT {n_split}\n#define AE_COMBINE_THREADS {self.COMBINE_THREADS}\n"
             if self._clock_stamps():
@@ -319,7 +329,8 @@ class PrefillOp:
                              threads=64 * self.tiles.n_waves,
                              lds_bytes=self.tiles.lds_bytes(self.D, self.DV_launch) + self._kv_custom_scratch(), head_dim=self.D,
                              head_dim_v=self.DV_launch, elem_bytes=2, n_rowscales=self.n_rowscales,
-                             mask_mode=mask_mode, table_rows=table_rows if mask_mode == 2 else 0)
+                             mask_mode=mask_mode if band is None else 1,      # (a band is analytic: no table comes with the call)
+                             table_rows=table_rows if mask_mode == 2 and band is None else 0)
             v = self._variants[key] = (module, cfg, cfg_src)
         return v
 
@@ -399,14 +410,14 @@ class PrefillOp:
             if table.dtype != torch.int8:
                 table = table.to(torch.int8)
             table = table.to(dev).contiguous()
-            mode, mbm, mbn = 2, bm, bn
+            mode, mbm, mbn, band = 2, bm, bn, None
         else:
             plan = self._plan(B, Hq, Sq, Skv, dev)
-            mode, table, mbm, mbn = plan.mode, plan.table, plan.block_m, plan.block_n
+            mode, table, mbm, mbn, band = plan.mode, plan.table, plan.block_m, plan.block_n, self._band(plan)
         n_split, kv_per_split = self.plan_splits(B, Hq, Sq, Skv)
         module, cfg, _ = self._variant(mode, Sq % self.tiles.block_m == 0, Skv % self.tiles.block_n == 0, n_split,
                                        self._table_rows(mbm) if mode == 2 else 1,
-                                       extern_mask is None and plan.heavy_last)
+                                       extern_mask is None and plan.heavy_last, band)
         kern = module.kernel("ae_prefill_kernel")
 
         out = torch.empty((B, Sq, Hq, self.DV), dtype=self.dtype, device=dev)
@@ -425,7 +436,7 @@ class PrefillOp:
             t = t.to(device=dev, dtype=desc.torch_dtype).contiguous()
             keep.append(t)
             p.custom[i] = t.data_ptr()
-        if mode == 2:
+        if mode == 2 and band is None:
             p.block_mask = table.data_ptr()
             p.mask_b, p.mask_h, p.mask_nq, p.mask_nkv = table.shape
             p.mask_block_m, p.mask_block_n = mbm, mbn
@@ -458,7 +469,7 @@ class PrefillOp:
             host.add_forward(self._host, host.PREFILL_SPLIT if n_split > 1 else host.PREFILL, B, Sq, Hq, Hkv, Skv, dev, module,
                              kern, cfg, combine=module.kernel("ae_decode_combine_kernel") if n_split > 1 else None,
                              ccfg=ccfg if n_split > 1 else None, n_split=n_split, kv_per_split=kv_per_split,
-                             table=table if mode == 2 else None, mask_block=(mbm, mbn), env=("AE_CLOCK_STAMPS",))
+                             table=table if mode == 2 and band is None else None, mask_block=(mbm, mbn), env=("AE_CLOCK_STAMPS",))
         return out
 
 

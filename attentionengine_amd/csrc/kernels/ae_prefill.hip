@@ -52,6 +52,25 @@
 #define AE_HEAVY_LAST 0      // 1: the tile table gives late q tiles more work than early ones
 #endif
 
+// AE_BAND 1 (AE_MASK_MODE 2 in the configuration): the host has shown that mask_mod is exactly
+// AE_BAND_LO <= q_idx - kv_idx <= AE_BAND_HI (core/lower/mask.py: sliding windows, shifted causal masks, a causal mask
+// over unequal lengths).  Such a mask needs no table and no call of ae_mask_mod: the tile range of a q tile is a
+// subtraction, a tile crosses at most two edges, and an edge costs one compare with a literal and one select per
+// score.  A wave none of whose rows sees a tile does not multiply it.  B2 H32 S4096 D128 fp16, window of 256, through
+// the table: 127 us (2.1 TB/s); as a band: 87 us.
+#ifndef AE_BAND
+#define AE_BAND 0
+#endif
+#if AE_BAND
+#undef AE_MASK_MODE
+#define AE_MASK_MODE 3
+#endif
+#define AE_ANALYTIC (AE_MASK_MODE == 1 || AE_MASK_MODE == 3)
+#if AE_MASK_MODE == 1
+#define AE_BAND_LO 0
+#define AE_BAND_HI 0x7fffffff
+#endif
+
 // value given to score positions past seqlen_kv before the user functors run: -inf, or 0 for graphs
 // declared with mask_value="0" (no additive -inf mask anywhere, attn_tl.py:124-137 / lower.py:637)
 #if defined(AE_MASK_VALUE_ZERO) && AE_MASK_VALUE_ZERO
@@ -175,7 +194,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #endif
   const int xcd = wg & 7;
   const int slot = wg >> 3;
-#if AE_MASK_MODE == 1 || (AE_MASK_MODE == 2 && AE_HEAVY_LAST)
+#if AE_MASK_MODE == 1 || AE_HEAVY_LAST
   // causal: q tiles differ in work by up to n_qt : 1, so ids go heaviest tile first across ALL heads
   // (longest-job-first keeps the tail short); the heads of one XCD still meet in its L2.  A tile table whose
   // late q tiles are the long ones (AE_HEAVY_LAST, found on the host: causal variants, long sliding windows)
@@ -229,10 +248,16 @@ void ae_prefill_kernel(const ae_attn_params p) {
   // ---- KV tile range ---------------------------------------------------------------------
   const int n_kvt = (p.seqlen_kv + AE_BN - 1) / AE_BN;
   int j_end = n_kvt;
-#if AE_MASK_MODE == 1
+#if AE_ANALYTIC
+  int j_first = 0;        // first tile with a key that some row of the q tile sees
   {
-    int lim = (q0 + AE_BM + AE_BN - 1) / AE_BN;  // attn_tl.py:113-115
-    j_end = lim < n_kvt ? lim : n_kvt;
+    int last_kv = q0 + AE_BM - 1 - AE_BAND_LO;   // attn_tl.py:113-115
+    last_kv = last_kv < p.seqlen_kv ? last_kv : p.seqlen_kv - 1;
+    j_end = last_kv < 0 ? 0 : last_kv / AE_BN + 1;
+#if AE_BAND_HI != 0x7fffffff
+    const int first_kv = q0 - AE_BAND_HI;
+    j_first = first_kv > 0 ? first_kv / AE_BN : 0;
+#endif
   }
 #endif
 #if AE_MASK_MODE == 2
@@ -346,7 +371,13 @@ void ae_prefill_kernel(const ae_attn_params p) {
     const int lim = j_begin + p.kv_per_split / AE_BN;
     j_end = lim < j_end ? lim : j_end;
   }
+#if AE_ANALYTIC
+  int j = j_begin > j_first ? j_begin : j_first;
+#else
   int j = next_tile(j_begin);
+#endif
+#elif AE_ANALYTIC
+  int j = j_first;
 #else
   int j = next_tile(0);
 #endif
@@ -405,6 +436,16 @@ void ae_prefill_kernel(const ae_attn_params p) {
       for (int db = 0; db < AE_NDB; db++) asm volatile("" : "+a"(oacc[rb][db]));
 #endif
 
+#if AE_ANALYTIC && !defined(AE_HAS_KV_PREFETCH) && AE_WAVES_PER_EU >= 2
+    // (wave uniform: some row of this wave sees a key of the tile.  Not where the functors also fetch custom inputs
+    // tile by tile, which has to go on; not in the builds that fill the register file with one wave, which spill)
+    bool active = kv0 <= q0w + AE_WROWS - 1 - AE_BAND_LO;
+#if AE_BAND_HI != 0x7fffffff
+    active = active && kv0 + AE_BN - 1 >= q0w - AE_BAND_HI;
+#endif
+    if (active)
+#endif
+    {
     // ---- S^T = K Q^T: every K fragment feeds one MFMA per row block -------------------------
     ae_f32x16 sacc[AE_RB][AE_NB];
 #pragma unroll
@@ -436,13 +477,21 @@ void ae_prefill_kernel(const ae_attn_params p) {
       const int kvb = ctx[rb].kv_base;
 
       // ---- mask (additive -inf before score_mod, attn_tl.py:124-137) --------------------------
+#if !AE_ANALYTIC
       bool masked_here = false;    // some score of this row block was tested on this tile
-#if AE_MASK_MODE == 1
-      if (kv0 + AE_BN - 1 > q0w + rb * 32) {  // tile crosses the diagonal of this row block
-        masked_here = true;
+#endif
+#if AE_ANALYTIC
+      const int qd = qrow[rb] - kvb;            // q - kv of score e is qd - ae_kv_off(e)
+      if (kv0 + AE_BN - 1 > q0w + rb * 32 - AE_BAND_LO) {  // tile crosses the diagonal of this row block
 #pragma unroll
-        for (int e = 0; e < AE_NS; e++) s[e] = (qrow[rb] >= kvb + ae_kv_off(e)) ? s[e] : AE_NEG_INF;
+        for (int e = 0; e < AE_NS; e++) s[e] = (qd >= ae_kv_off(e) + AE_BAND_LO) ? s[e] : AE_NEG_INF;
       }
+#if AE_BAND_HI != 0x7fffffff
+      if (kv0 < q0w + rb * 32 + 31 - AE_BAND_HI) {         // ... the far edge of the band
+#pragma unroll
+        for (int e = 0; e < AE_NS; e++) s[e] = (qd <= ae_kv_off(e) + AE_BAND_HI) ? s[e] : AE_NEG_INF;
+      }
+#endif
 #elif AE_MASK_MODE == 2 && !(defined(AE_MASK_VALUE_ZERO) && AE_MASK_VALUE_ZERO)
       if (__builtin_amdgcn_ballot_w64(cls[rb] != 2) != 0) {   // some row of this block does not see the whole tile
         masked_here = true;
@@ -466,12 +515,23 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #endif
 #if !AE_EVEN_KV
       if (kv0 + AE_BN > p.seqlen_kv) {
-        masked_here = true;
 #pragma unroll
         for (int e = 0; e < AE_NS; e++) s[e] = (kvb + ae_kv_off(e) < p.seqlen_kv) ? s[e] : AE_KV_PAD;
       }
 #endif
-      if (masked_here) {           // (an untested tile is visible to every row)
+#if AE_ANALYTIC
+      {
+        // the row's visible keys of this tile are an interval
+        int lo_kv = kv0, hi_kv = kv0 + AE_BN - 1;
+        hi_kv = hi_kv < p.seqlen_kv ? hi_kv : p.seqlen_kv - 1;
+        hi_kv = hi_kv < qrow[rb] - AE_BAND_LO ? hi_kv : qrow[rb] - AE_BAND_LO;
+#if AE_BAND_HI != 0x7fffffff
+        lo_kv = lo_kv > qrow[rb] - AE_BAND_HI ? lo_kv : qrow[rb] - AE_BAND_HI;
+#endif
+        seen[rb] = lo_kv <= hi_kv ? 1.f : seen[rb];
+      }
+#else
+      if (masked_here) {           // (an untested tile is visible to every row; a tile that the end of the sequence cuts holds a key)
         float top = s[0];
 #pragma unroll
         for (int e = 1; e < AE_NS; e++) top = __builtin_fmaxf(top, s[e]);
@@ -479,6 +539,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
       } else {
         seen[rb] = 1.f;
       }
+#endif
 
       // ---- user functors ----------------------------------------------------------------------
 #if defined(AE_HAS_KV_PREFETCH) && AE_KV_COALESCED
@@ -548,6 +609,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #pragma unroll
         for (int rb = 0; rb < AE_RB; rb++) oacc[rb][db] = ae_mfma32(vf, pf[rb][kk], oacc[rb][db]);
       }
+    }
     }
 
     // the next tile must have landed before anyone reads it: direct loads are tracked by vmcnt
