@@ -165,7 +165,7 @@ AE_DEV void ae_q_rows_to_lds(const char* qg, ae_lds_byte* qs, int lane, int row0
 }
 
 extern "C" __global__ __launch_bounds__(AE_NT)
-__attribute__((amdgpu_waves_per_eu(AE_WAVES_PER_EU, AE_WAVES_PER_EU)))
+__attribute__((amdgpu_waves_per_eu(AE_WAVES_PER_EU)))
 void ae_prefill_kernel(const ae_attn_params p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ae_smem[];
   ae_lds_byte* lds = (ae_lds_byte*)ae_smem;
