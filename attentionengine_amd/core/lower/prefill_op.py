@@ -16,6 +16,7 @@ from ..runtime import hip_rt as rt
 from ..runtime import host
 from ..transform.core import _convert_mask_to_block_mask, is_causal_mask
 from . import lower as L
+from .lower_decode import combine_rows
 from .mask import plan_mask
 
 
@@ -448,7 +449,7 @@ class PrefillOp:
             p.partial_o, p.partial_rs = partial_o.data_ptr(), partial_rs.data_ptr()
             p.num_splits, p.kv_per_split = n_split, kv_per_split
             keep += [partial_o, partial_rs]
-            ccfg = rt.TileCfg(block_m=1, block_n=n_split, threads=self.COMBINE_THREADS, lds_bytes=0,
+            ccfg = rt.TileCfg(block_m=combine_rows(self.COMBINE_THREADS, self.DV), block_n=n_split, threads=self.COMBINE_THREADS, lds_bytes=0,
                               head_dim=self.D, head_dim_v=self.DV, elem_bytes=2,
                               n_rowscales=self.n_rowscales, mask_mode=0)
             rt.prefill_split_fwd(kern, module.kernel("ae_decode_combine_kernel"), p, cfg, ccfg, stream)

@@ -398,6 +398,12 @@ int ae_prefill_fwd(ae_kernel* k, const ae_attn_params* p, const ae_tile_cfg* cfg
   return ae_launch(k, p, sizeof *p, grid, block, (uint32_t)cfg->lds_bytes, stream);
 }
 
+// workgroups of the merge kernel for `rows` output rows of a batch entry: block_m rows each (ae_combine.h)
+static uint32_t combine_grid(int32_t rows, const ae_tile_cfg* c) {
+  const int32_t per = c->block_m > 0 ? c->block_m : 1;
+  return (uint32_t)((rows + per - 1) / per);
+}
+
 // launch == false: only the argument checks (ae_decode_fwd_noalloc runs them before it touches the device)
 static int decode_fwd_impl(ae_kernel* split, ae_kernel* combine, const ae_attn_params* p,
                            const ae_tile_cfg* cfg, const ae_tile_cfg* combine_cfg, void* stream, bool launch) {
@@ -475,7 +481,7 @@ static int decode_fwd_impl(ae_kernel* split, ae_kernel* combine, const ae_attn_p
   if (!launch) return AE_OK;
   rc = ae_launch(split, p, sizeof *p, grid, block, (uint32_t)cfg->lds_bytes, stream);
   if (rc || merged) return rc;
-  uint32_t cgrid[3] = {(uint32_t)p->heads_q, (uint32_t)p->batch, 1};
+  uint32_t cgrid[3] = {combine_grid(p->heads_q, combine_cfg), (uint32_t)p->batch, 1};
   uint32_t cblock[3] = {(uint32_t)combine_cfg->threads, 1, 1};
   return ae_launch(combine, p, sizeof *p, cgrid, cblock, (uint32_t)combine_cfg->lds_bytes, stream);
 }
@@ -536,7 +542,7 @@ int ae_prefill_split_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_par
   // tells it to write the merged row scales in [B, Hq, Sq] order
   ae_attn_params cp = *p;
   cp.heads_q = (int32_t)rows;
-  uint32_t cgrid[3] = {(uint32_t)rows, (uint32_t)p->batch, 1};
+  uint32_t cgrid[3] = {combine_grid((int32_t)rows, combine_cfg), (uint32_t)p->batch, 1};
   uint32_t cblock[3] = {(uint32_t)combine_cfg->threads, 1, 1};
   return ae_launch(combine, &cp, sizeof cp, cgrid, cblock, (uint32_t)combine_cfg->lds_bytes, stream);
 }
@@ -609,7 +615,7 @@ int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params
   uint32_t block[3] = {(uint32_t)cfg->threads, 1, 1};
   rc = ae_launch(split, p, sizeof *p, grid, block, (uint32_t)cfg->lds_bytes, stream);
   if (rc || direct) return rc;
-  uint32_t cgrid[3] = {(uint32_t)p->heads_q, (uint32_t)p->batch, 1};
+  uint32_t cgrid[3] = {combine_grid(p->heads_q, combine_cfg), (uint32_t)p->batch, 1};
   uint32_t cblock[3] = {(uint32_t)combine_cfg->threads, 1, 1};
   return ae_launch(combine, p, sizeof *p, cgrid, cblock, (uint32_t)combine_cfg->lds_bytes, stream);
 }

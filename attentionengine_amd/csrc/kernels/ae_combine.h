@@ -3,13 +3,21 @@
 #ifndef AE_COMBINE_H
 #define AE_COMBINE_H
 
-// Merge of the per-split partials: grid (Hq, B), one workgroup per output row.
+#define AE_COMBINE_ROWS (AE_COMBINE_THREADS / (AE_DV / 4) > 0 ? AE_COMBINE_THREADS / (AE_DV / 4) : 1)
+static_assert(AE_DV % 4 == 0, "four value columns a thread");
+
+// Merge of the per-split partials: grid (ceil(Hq / AE_COMBINE_ROWS), B).  Bound by its chain of dependent memory
+// trips (row scales, then partial results), not by bytes, so a thread owns four neighbouring value columns (16-byte
+// loads, one pass over DV 512 with 128 threads where one column a thread took four) and a workgroup holds as many
+// rows as its threads have room for (ae_tile_cfg.block_m of the combine configuration).
 // out[b,0,h,:] = sum_k partial_o[b,h,k,:] * o_scale[k], o_scale = combine(final_rowscales[k])
 // (attn_gqa_decode_tl.py:224-266; generic form core/template/tl_template/attn/attn_decode_tl.py:184-189).
 extern "C" __global__ __launch_bounds__(AE_COMBINE_THREADS)
 void ae_decode_combine_kernel(const ae_attn_params p) {
-  const int h = blockIdx.x;
+  constexpr int TPR = AE_DV / 4 < AE_COMBINE_THREADS ? AE_DV / 4 : AE_COMBINE_THREADS;      // threads per row
+  const int h = AE_COMBINE_ROWS == 1 ? blockIdx.x : blockIdx.x * AE_COMBINE_ROWS + threadIdx.x / TPR;
   const int b = blockIdx.y;
+  if (threadIdx.x >= AE_COMBINE_ROWS * TPR || h >= p.heads_q) return;
   const int64_t row = ((int64_t)b * p.heads_q + h) * AE_NSPLIT;
   // Paged cache (per-entry lengths): only the first ceil(length / kv_per_split) splits of an entry hold keys and
   // wrote partial results; an entry with at most one wrote `out` itself.
@@ -31,30 +39,35 @@ void ae_decode_combine_kernel(const ae_attn_params p) {
   float merged[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1];
   ae_combine(rs, w, merged);
   ae_elem* optr = (ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)h * p.o_stride_h;
-  for (int dv = threadIdx.x; dv < AE_DV; dv += AE_COMBINE_THREADS) {
+  for (int dv = (threadIdx.x % TPR) * 4; dv < AE_DV; dv += TPR * 4) {
     // The partial results are read 16 splits at a time, unconditionally, so that the loads of a group all go
     // out before the first one is waited for (one memory round trip per group instead of one per split: the
     // merge of 32 splits 18 -> 4 us).  Splits that wrote nothing re-read the last one that did, with weight 0.
-    float acc = 0.f;
+    ae_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     constexpr int G = AE_NSPLIT < 16 ? AE_NSPLIT : 16;
 #pragma unroll
     for (int k0 = 0; k0 < AE_NSPLIT; k0 += G) {
-      float val[G];
+      ae_f32x4 val[G];
 #pragma unroll
       for (int i = 0; i < G; i++) {
         const int k = k0 + i < AE_NSPLIT ? k0 + i : AE_NSPLIT - 1;
         const int kc = k < n_used ? k : n_used - 1;
-        val[i] = p.partial_o[(row + kc) * AE_DV + dv];
+        val[i] = *(const ae_f32x4*)(p.partial_o + (row + kc) * AE_DV + dv);
       }
 #pragma unroll
       for (int i = 0; i < G; i++) {
         const int k = k0 + i;
-        acc += val[i] * ((k < AE_NSPLIT && k < n_used) ? w[k < AE_NSPLIT ? k : 0] : 0.f);
+        const float wk = (k < AE_NSPLIT && k < n_used) ? w[k < AE_NSPLIT ? k : 0] : 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; c++) acc[c] += val[i][c] * wk;
       }
     }
-    optr[dv] = (ae_elem)acc;
+    ae_elem4 r;
+#pragma unroll
+    for (int c = 0; c < 4; c++) r[c] = (ae_elem)acc[c];
+    *(ae_elem4*)(optr + dv) = r;
   }
-  if (threadIdx.x == 0) {
+  if (threadIdx.x % TPR == 0) {
     // One-token decode: row scales [B, Hq].  Split-KV prefill (p.seqlen_q > 1: its launch hands the (q position,
     // head) pairs over as p.heads_q = Sq * Hq "heads", h = s * Hq + head): row scales [B, Hq, Sq], the layout of
     // the unsplit kernels.
