@@ -58,6 +58,17 @@
 #define AE_MERGE_LAST 0
 #endif
 static_assert(!(AE_MERGE_IN_WG && AE_MERGE_LAST), "one way to merge");
+// 1 (where combine() is the log-sum-exp merge, whose result does not depend on the grouping): the waves of a workgroup
+// merge their partial results in LDS first and ONE partial result per workgroup goes to memory: AE_NSPLIT is then the
+// number of workgroups (p.num_splits / AE_NWAVES), with either form of the merge that follows.
+// A kv axis can then be shared out over four times as many workgroups for the same merge traffic, which is what a
+// batch of one to four needs: with one workgroup per 8 kv heads and 8 shares each wave walked eight tiles one memory
+// trip after the other (8.7 of 16.4 us of B1 Hq32 Hkv8 Skv8192).
+#ifndef AE_WG_FIRST
+#define AE_WG_FIRST 0
+#endif
+static_assert(!(AE_WG_FIRST && AE_MERGE_IN_WG), "grouped merge: for partial results of several workgroups");
+static_assert(!AE_WG_FIRST || AE_N_ROWSCALES == 1, "the log-sum-exp merge has one row scale");
 static_assert(!AE_MERGE_IN_WG || AE_NSPLIT == AE_NWAVES, "the workgroup merges exactly its own waves' partial results");
 static_assert(AE_D % 32 == 0, "head dim must be a multiple of 32");
 static_assert(AE_DV % 16 == 0, "value head dim must be a multiple of 16");
@@ -260,7 +271,7 @@ void ae_decode_split_kernel(const ae_attn_params p) {
 #pragma unroll
     for (int i = 0; i < AE_N_ROWSCALES; i++) frs[i] = AE_NEG_INF;
   }
-#if AE_MERGE_IN_WG
+#if AE_MERGE_IN_WG || AE_WG_FIRST
   {
     // (the wave's V tile region is its own, and its last transposed reads have returned: O was computed from them)
     __attribute__((address_space(3))) float* mo = (__attribute__((address_space(3))) float*)vs;
@@ -276,6 +287,52 @@ void ae_decode_split_kernel(const ae_attn_params p) {
       for (int i = 0; i < AE_N_ROWSCALES; i++) mrs[(i * AE_NWAVES + wave) * 16 + l16] = frs[i];
     }
     __syncthreads();
+#if AE_WG_FIRST
+    // this workgroup's partial result of the tile's heads -> memory (device scope: see below)
+    const int tile_heads = group - ht * 16 < 16 ? group - ht * 16 : 16;
+    const int64_t tile_row0 = ((int64_t)b * p.heads_q + hk * group + ht * 16) * AE_NSPLIT;
+#if AE_MERGE_LAST
+    constexpr int kDeviceScope = 16;
+    __amdgpu_buffer_rsrc_t po_buf = __builtin_amdgcn_make_buffer_rsrc(
+        p.partial_o + tile_row0 * AE_DV, 0, tile_heads * AE_NSPLIT * AE_DV * 4, 0x00020000);
+#endif
+    const bool no_keys = wg_base >= p.seqlen_kv;        // (else the workgroup's first wave has some)
+    for (int idx = tid; idx < tile_heads * (AE_DV / 4); idx += AE_NT) {
+      const int hl = idx / (AE_DV / 4), dv = (idx % (AE_DV / 4)) * 4;
+      float rs[AE_NWAVES];
+#pragma unroll
+      for (int k = 0; k < AE_NWAVES; k++) rs[k] = mrs[k * 16 + hl];
+      const float top = ae_arr_max<AE_NWAVES>(rs);
+      float w[AE_NWAVES];
+#pragma unroll
+      for (int k = 0; k < AE_NWAVES; k++) w[k] = ae_exp(rs[k] - top);
+      float merged = ae_log(ae_arr_sum<AE_NWAVES>(w)) + top;
+      ae_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < AE_NWAVES; k++) {
+        const ae_f32x4 v = *(__attribute__((address_space(3))) ae_f32x4*)(
+            (__attribute__((address_space(3))) float*)((ae_lds_byte*)ae_smem + k * AE_V_WAVE_BYTES) + hl * AE_DV + dv);
+        const float wk = ae_exp(rs[k] - merged);
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[r] += v[r] * wk;
+      }
+      if (no_keys) {
+        acc = (ae_f32x4){0.f, 0.f, 0.f, 0.f};
+        merged = AE_NEG_INF;
+      }
+      const int row_in_tile = hl * AE_NSPLIT + blockIdx.x;
+#if AE_MERGE_LAST
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(ae_u32x4, acc), po_buf, (row_in_tile * AE_DV + dv) * 4, 0,
+                                             kDeviceScope);
+      if (dv == 0)
+        __hip_atomic_store(p.partial_rs + tile_row0 + row_in_tile, merged, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#else
+      *(ae_f32x4*)(p.partial_o + (tile_row0 + row_in_tile) * AE_DV + dv) = acc;
+      if (dv == 0) p.partial_rs[tile_row0 + row_in_tile] = merged;
+#endif
+    }
+    (void)split;
+#else
     for (int idx = tid; idx < 16 * AE_DV; idx += AE_NT) {
       const int hl = idx / AE_DV, dv = idx % AE_DV;
       if (ht * 16 + hl >= group) continue;
@@ -301,6 +358,7 @@ void ae_decode_split_kernel(const ae_attn_params p) {
     }
     (void)split;
     return;
+#endif
   }
 #endif
 #if AE_MERGE_LAST
@@ -310,9 +368,10 @@ void ae_decode_split_kernel(const ae_attn_params p) {
   // invalidates the whole L2: measured at several microseconds a workgroup, twice the call at batch 4).
   constexpr int kDeviceScope = 16;     // the sc1 bit of a buffer instruction's cache policy
   const int tile_heads = group - ht * 16 < 16 ? group - ht * 16 : 16;
-  const int64_t tile_row0 = ((int64_t)b * p.heads_q + hk * group + ht * 16) * p.num_splits;
+  const int64_t tile_row0 = ((int64_t)b * p.heads_q + hk * group + ht * 16) * AE_NSPLIT;
   __amdgpu_buffer_rsrc_t po_buf = __builtin_amdgcn_make_buffer_rsrc(
-      p.partial_o + tile_row0 * AE_DV, 0, tile_heads * p.num_splits * AE_DV * 4, 0x00020000);
+      p.partial_o + tile_row0 * AE_DV, 0, tile_heads * AE_NSPLIT * AE_DV * 4, 0x00020000);
+#if !AE_WG_FIRST
   if (head_ok) {
     const int row_in_tile = l16 * p.num_splits + split;
 #pragma unroll
@@ -328,6 +387,7 @@ void ae_decode_split_kernel(const ae_attn_params p) {
                            frs[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
+#endif
   {
     // Every wave waits until its stores above have been acknowledged (stores count in vmcnt; the barrier alone
     // does not wait for them: a workgroup-scope release on this target orders only what the waves of one CU see),
@@ -357,7 +417,7 @@ void ae_decode_split_kernel(const ae_attn_params p) {
       for (int i = 0; i < AE_N_ROWSCALES; i++)
 #pragma unroll
         for (int k = 0; k < AE_NSPLIT; k++)
-          rs[i][k] = __hip_atomic_load(p.partial_rs + (int64_t)i * p.batch * p.heads_q * p.num_splits + tile_row0 +
+          rs[i][k] = __hip_atomic_load(p.partial_rs + (int64_t)i * p.batch * p.heads_q * AE_NSPLIT + tile_row0 +
                                            hl * AE_NSPLIT + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       constexpr int G = AE_NSPLIT < 16 ? AE_NSPLIT : 16;     // partial results in flight at a time
       ae_f32x4 val[G];
@@ -396,7 +456,7 @@ void ae_decode_split_kernel(const ae_attn_params p) {
       }
     }
   }
-#else
+#elif !AE_WG_FIRST
   if (head_ok) {
     const int64_t row = ((int64_t)b * p.heads_q + hq) * p.num_splits + split;
     float* po = p.partial_o + row * AE_DV;
