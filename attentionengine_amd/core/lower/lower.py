@@ -598,14 +598,23 @@ class PrefillTiles:
     k_pad: int = 0
     v_pad: int = 0
     rows_per_wave: int = 32
+    kv_groups: int = 1                 # sets of n_waves waves that share the kv axis (AE_KW of ae_prefill.hip)
     kv_stages: int = 2                 # K / V tile stages in LDS (AE_KV_STAGES of the pipelined kernel: 2 or 3)
 
     @property
     def block_m(self):
         return self.rows_per_wave * self.n_waves
 
+    @property
+    def threads(self):
+        return 64 * self.n_waves * self.kv_groups
+
     def lds_bytes(self, d: int, dv: int) -> int:
-        stages = self.kv_stages * self.block_n * ((2 * d + self.k_pad) + (2 * dv + self.v_pad))
+        stages = self.kv_groups * self.kv_stages * self.block_n * ((2 * d + self.k_pad) + (2 * dv + self.v_pad))
+        if self.kv_groups > 1:
+            # the groups' O (fp32) and row state meet in LDS after the loop
+            waves = self.kv_groups * self.n_waves
+            stages = max(stages, waves * 32 * dv * 4 + waves * 3 * 64 * 4)
         if self.template == "ae_prefill_pipe.hip":
             # behind the tile stages every wave has room for its 64 Q rows (later its 64 O rows), which travel
             # through LDS as whole rows (AE_QO_BYTES of the kernel)
@@ -700,6 +709,39 @@ def choose_prefill_tiles(d: int, dv: int, seqlen_q: int = 0, softmax=None, batch
     return t
 
 
+def kv_group_tiles(d: int, dv: int, batch_heads: int, seqlen_q: int, seqlen_kv: int, banded: bool):
+    """Tiles whose waves share the kv axis (AE_KW of ae_prefill.hip), or None where the launch is large enough to fill
+    the chip with whole kv axes.  Written as rows x kv groups x keys of a tile: 32 x 4 x 32, 64 x 4 x 32, 64 x 2 x 32 and
+    128 x 2 x 64.  The first two hold 128 KiB of LDS at head dim 128 (one workgroup a CU) and half of it at 64 (two):
+    they pay while all workgroups are resident at once, fewer rows first; a causal or banded launch, whose workgroups end
+    at different times, a little beyond.  Measured (us, default tiles -> these): bf16 D128 causal, Hq32 S333 13.8 -> 10.4
+    (64 x 4), S600 20.0 -> 16.7, S1000 29.1 -> 24.2 (64 x 2), S1500 44.6 -> 39.7 (128 x 2); H16 S333 13.5 -> 8.7 (32 x 4);
+    D64 H32 S333 10.7 -> 7.3; but B4 H32 S333 17.4 -> 20 with any of them."""
+    def wgs(rows):
+        return batch_heads * -(-seqlen_q // rows)
+    slots = _MI355X_CUS if max(d, dv) > 64 else 2 * _MI355X_CUS
+    if wgs(32) <= slots:
+        return PrefillTiles(n_waves=1, kv_groups=4, block_n=32)
+    if seqlen_kv >= 192 and wgs(64) <= (slots * 5 // 4 if banded else _MI355X_CUS):
+        return PrefillTiles(n_waves=2, kv_groups=4, block_n=32)
+    if banded and seqlen_kv >= 512 and max(d, dv) > 64 and wgs(64) <= 2 * slots:
+        return PrefillTiles(n_waves=2, kv_groups=2, block_n=32)
+    if seqlen_kv >= 512 and wgs(128) <= (_MI355X_CUS * 3 // 2 if banded else _MI355X_CUS):
+        return PrefillTiles(kv_groups=2)
+    return None
+
+
+def kv_group_tiles_split(seqlen_q: int):
+    """The same for launches that also split the kv axis over workgroups (a few query tokens against a long cache): the
+    query rows decide.  fp16 D128: B8 H32 Sq4 Skv4096 110 -> 95 us, B1 H32 Sq16 Skv16000 55 -> 46 (32 x 4 x 32); B2 H16 Sq40
+    Skv3000 19.1 -> 17.7 (64 x 2 x 32); from 65 rows on the 128-row tiles already read the cache at 5.8 TB/s."""
+    if seqlen_q <= 32:
+        return PrefillTiles(n_waves=1, kv_groups=4, block_n=32)
+    if seqlen_q <= 64:
+        return PrefillTiles(n_waves=2, kv_groups=2, block_n=32)
+    return None
+
+
 def render_config(d: int, dv: int, dtype, tiles: PrefillTiles, mask_mode: int, has_mask_mod: bool,
                   n_rowscales: int, o_scale_one: bool, even_q: bool, even_kv: bool, softmax=None,
                   elementwise: bool = False, exact_scale=None) -> str:
@@ -726,6 +768,8 @@ def render_config(d: int, dv: int, dtype, tiles: PrefillTiles, mask_mode: int, h
         f"#define AE_DV {dv}",
         f"#define AE_BN {tiles.block_n}",
         f"#define AE_NWAVES {tiles.n_waves}",
+        *([f"#define AE_KW {tiles.kv_groups}", f"#define AE_KW_SOFTMAX {1 if softmax is not None else 0}"]
+          if tiles.kv_groups > 1 else []),
         f"#define AE_DTYPE_BF16 {1 if dtype == torch.bfloat16 else 0}",
         f"#define AE_MASK_MODE {mask_mode}",
         f"#define AE_HAS_MASK_MOD {1 if has_mask_mod else 0}",

@@ -86,8 +86,11 @@ class PrefillOp:
         # the pipelined kernel's (B2 H32 S4096 D128, sliding window of 256: 0.13 against 0.31 ms; a random block
         # mask that keeps 27 %: 0.22 against 0.35 ms).  tune=True still measures both.
         if self.tiles.rows_per_wave == 64 and os.environ.get("AE_PREFILL_KERNEL", "") != "pipelined" and (
-                self.extern_block_mask or (mask_mod is not None and self._probe_mask_mode(q_meta, v_meta) == 2)):
+                self.extern_block_mask or (mask_mod is not None and self._probe_mask(q_meta, v_meta).mode == 2)):
             self.tiles = L.PrefillTiles()
+        groups = self._groups = self._kv_group_choice(q_meta, v_meta, split_kv)
+        if groups is not None:
+            self.tiles = groups
         # tune=True (attn_tl.py:465-521 of the reference): the tile configuration comes from the record of
         # this problem in tune_file, or is measured at the first call and recorded there.  Launches whose
         # tiles are bound to something else (split-KV, an external block mask) keep the fixed choice.
@@ -117,7 +120,8 @@ class PrefillOp:
             if not hasattr(online_func, "combine"):
                 raise NotImplementedError("split-KV needs OnlineFunc.combine to merge the partial results")
             from .lower_decode import lower_combine
-            self.tiles = L.PrefillTiles()          # the generic kernel carries the split-KV mode
+            if tiles is None and groups is None:
+                self.tiles = L.PrefillTiles()      # the generic kernel carries the split-KV mode
             self.functor_src += lower_combine(online_func, self.functors.final_rowscale_names)
         if self.extern_block_mask and self.tiles.rows_per_wave != 32 and (
                 self.mask_block[1] % self.tiles.block_n or
@@ -184,17 +188,36 @@ class PrefillOp:
         if infer_mask and mask_mod is not None and not self.extern_block_mask:
             self.block_mask = self._reference_block_mask(B, H, Sq, Skv)
 
-    def _probe_mask_mode(self, q_meta, v_meta):
-        """Mode of the mask plan at the declared sequence lengths (4096 where they are dynamic), for batch entry
-        and head 0: 2 = the mask needs a tile table."""
+    def _probe_mask(self, q_meta, v_meta):
+        """The mask plan at the declared sequence lengths (4096 where they are dynamic), for batch entry and head 0:
+        mode 2 = the mask needs a tile table (or is a band)."""
         sq, skv = _dim(q_meta.shape[2], 4096), _dim(v_meta.shape[2], 4096)
-        return plan_mask(self.mask_mod, self.functors.mask, 1, 1, sq, skv, 128, 64,
-                         elementwise=self.elementwise_mask).mode
+        return plan_mask(self.mask_mod, self.functors.mask, 1, 1, sq, skv, 128, 64, elementwise=self.elementwise_mask)
+
+    def _kv_group_choice(self, q_meta, v_meta, split_kv):
+        """Tiles whose waves share the kv axis, where this engine's graph, mask and declared extents allow and want them:
+        a merge the kernel knows (the proven online softmax, or no row state), no mask table, no tensor read per score."""
+        sq, skv = _dim(q_meta.shape[2], 0), _dim(v_meta.shape[2], 0)
+        bh = _dim(q_meta.shape[0], 0) * _dim(q_meta.shape[1], 0)
+        if (not sq or not skv or not bh or self.extern_block_mask or self.D not in (64, 128) or self.DV not in (64, 128)
+                or not (self._pipe_softmax is not None or self._pipe_elementwise)
+                or any(c.per_kv for c in self.functors.customs) or os.environ.get("AE_PREFILL_KERNEL", "")):
+            return None
+        if split_kv:
+            return L.kv_group_tiles_split(sq) if self.mask_mod is None else None
+        found = L.kv_group_tiles(self.D, self.DV, bh, sq, skv, self.mask_mod is not None)
+        if found is not None and self.mask_mod is not None:
+            plan = self._probe_mask(q_meta, v_meta)
+            lm = self.functors.mask
+            if lm.uses_b or lm.uses_h or not (plan.mode == 1 or plan.band is not None):
+                return None
+        return found
 
     # ---- tuning ------------------------------------------------------------------------
     def _tune_candidates(self):
         from . import tuner
-        return tuner.prefill_candidates(self.D, self.DV_launch, self._pipe_softmax, self._pipe_elementwise)
+        cands = tuner.prefill_candidates(self.D, self.DV_launch, self._pipe_softmax, self._pipe_elementwise)
+        return cands if self._groups is None else cands + [self._groups]
 
     def _tune(self, q, k, v, *extra):
         """Measures every candidate tile configuration on the caller's tensors, becomes the fastest one and
@@ -307,7 +330,7 @@ class PrefillOp:
             has_mask_mod = self.elementwise_mask and mask_mode != 1
             cfg_src = L.render_config(self.D, self.DV_launch, self.dtype, self.tiles, mask_mode, has_mask_mod,
                                       self.n_rowscales, self.functors.o_scale_one, even_q, even_kv,
-                                      self._pipe_softmax if self.tiles.rows_per_wave == 64 else None,
+                                      self._pipe_softmax if (self.tiles.rows_per_wave == 64 or self.tiles.kv_groups > 1) else None,
                                       elementwise=self._pipe_elementwise and self.tiles.rows_per_wave == 64,
                                       exact_scale=self.exact_scale)
             if self.mask_value_zero:
@@ -327,7 +350,7 @@ class PrefillOp:
                                        # the builds in which a spilled tuple came back wrong: 256 accumulator registers
                                        strict_spills=self.tiles.template == "ae_prefill.hip" and self.DV_launch > 256)
             cfg = rt.TileCfg(block_m=self.tiles.block_m, block_n=self.tiles.block_n,
-                             threads=64 * self.tiles.n_waves,
+                             threads=self.tiles.threads,
                              lds_bytes=self.tiles.lds_bytes(self.D, self.DV_launch) + self._kv_custom_scratch(), head_dim=self.D,
                              head_dim_v=self.DV_launch, elem_bytes=2, n_rowscales=self.n_rowscales,
                              mask_mode=mask_mode if band is None else 1,      # (a band is analytic: no table comes with the call)
@@ -415,6 +438,13 @@ class PrefillOp:
         else:
             plan = self._plan(B, Hq, Sq, Skv, dev)
             mode, table, mbm, mbn, band = plan.mode, plan.table, plan.block_m, plan.block_n, self._band(plan)
+        if mode == 2 and band is None and self.tiles.kv_groups > 1:
+            # (a shape other than the declared one whose mask needs a table, or a block mask of the caller's)
+            self.tiles = L.PrefillTiles()
+            self._variants.clear()
+            self._plans.clear()
+            self._host.clear()
+            return self._forward_once(q, k, v, *extra, *(() if extern_mask is None else (extern_mask,)))
         n_split, kv_per_split = self.plan_splits(B, Hq, Sq, Skv)
         module, cfg, _ = self._variant(mode, Sq % self.tiles.block_m == 0, Skv % self.tiles.block_n == 0, n_split,
                                        self._table_rows(mbm) if mode == 2 else 1,

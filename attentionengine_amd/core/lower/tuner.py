@@ -121,7 +121,7 @@ def prefill_candidates(d, dv, softmax, elementwise):
 
 
 def encode_tiles(t):
-    return [t.block_m, t.block_n, t.kv_stages, 64 * t.n_waves, t.waves_per_eu, t.template]
+    return [t.block_m, t.block_n, t.kv_stages, t.threads, t.waves_per_eu, t.template]
 
 
 def decode_tiles(tuned_config, candidates):

@@ -57,7 +57,7 @@
 // over unequal lengths).  Such a mask needs no table and no call of ae_mask_mod: the tile range of a q tile is a
 // subtraction, a tile crosses at most two edges, and an edge costs one compare with a literal and one select per
 // score.  A wave none of whose rows sees a tile does not multiply it.  B2 H32 S4096 D128 fp16, window of 256, through
-// the table: 127 us (2.1 TB/s); as a band: 87 us.
+// the table: 127 us (2.1 TB/s); as a band: 91 us.
 #ifndef AE_BAND
 #define AE_BAND 0
 #endif
@@ -69,6 +69,21 @@
 #if AE_MASK_MODE == 1
 #define AE_BAND_LO 0
 #define AE_BAND_HI 0x7fffffff
+#endif
+
+// AE_KW > 1: the waves of a workgroup also share the kv axis.  AE_NWAVES waves own 32 query rows each, as always; AE_KW
+// such sets of waves ("kv groups") walk the kv tiles in turn, each with its own pair of LDS stages, and meet at the end:
+// every wave leaves its unscaled O in LDS, rescales a share of the value columns to the common reference and sums it
+// over the groups.  For launches whose q tiles do not fill the chip - one prompt of a few hundred tokens, a chunk of
+// query tokens against a long cache -, where a wave alone on its SIMD takes 1.5 us for a 64-key tile (LDS latency, MFMA
+// latency and the softmax one after the other) and the kv axis is a serial chain of them: B1 Hq32 S333 causal, 96
+// workgroups, 9.4 of 13.4 us in six tiles.  Needs a merge that the kernel knows: AE_KW_SOFTMAX 1 the proven online softmax
+// (fields AE_SM_M, AE_SM_R), 0 no row state (O is summed).  Not with a tile table.
+#ifndef AE_KW
+#define AE_KW 1
+#endif
+#ifndef AE_KW_SOFTMAX
+#define AE_KW_SOFTMAX 0
 #endif
 
 // value given to score positions past seqlen_kv before the user functors run: -inf, or 0 for graphs
@@ -84,7 +99,8 @@
 #endif
 #define AE_WROWS (AE_RB * 32)     // query rows per wave
 #define AE_BM (AE_NWAVES * AE_WROWS)
-#define AE_NT (AE_NWAVES * 64)
+#define AE_GT (AE_NWAVES * 64)     // threads of a kv group
+#define AE_NT (AE_GT * AE_KW)
 #define AE_NB (AE_BN / 32)        // 32-wide kv blocks per tile
 #define AE_NS (AE_NB * 16)        // score elements per lane per tile
 #define AE_NDB (AE_DV / 32)       // 32-wide dv blocks
@@ -96,8 +112,8 @@
 #define AE_STAGE_BYTES (AE_K_BYTES + AE_V_BYTES)
 #define AE_KCPR (AE_D / 8)        // 16-byte chunks per K row
 #define AE_VCPR (AE_DV / 8)
-#define AE_K_LOADS ((AE_BN * AE_KCPR) / AE_NT)   // direct loads per lane per K tile
-#define AE_V_LOADS ((AE_BN * AE_VCPR) / AE_NT)
+#define AE_K_LOADS ((AE_BN * AE_KCPR) / AE_GT)   // direct loads per lane per K tile
+#define AE_V_LOADS ((AE_BN * AE_VCPR) / AE_GT)
 #define AE_V_RPI (64 / AE_VCPR)
 #define AE_VPPR (AE_VCPR / 2)     // 32-byte pairs per V row
 // the pairs of a V row are exchanged by the row's low bits: at most three of them, so that rows 8 apart (the
@@ -107,8 +123,10 @@
 static_assert(AE_D % 16 == 0, "head dim must be a multiple of 16");
 static_assert(AE_DV % 32 == 0, "value head dim must be a multiple of 32");
 static_assert(AE_BN % 32 == 0, "kv tile must be a multiple of 32");
-static_assert((AE_BN * AE_KCPR) % AE_NT == 0, "K tile must split evenly over the workgroup");
-static_assert((AE_BN * AE_VCPR) % AE_NT == 0, "V tile must split evenly over the workgroup");
+static_assert((AE_BN * AE_KCPR) % AE_GT == 0, "K tile must split evenly over the waves that load it");
+static_assert((AE_BN * AE_VCPR) % AE_GT == 0, "V tile must split evenly over the waves that load it");
+static_assert(AE_KW == 1 || (AE_MASK_MODE != 2 && AE_RB == 1 && AE_NO % (4 * AE_KW) == 0 && AE_WAVES_PER_EU >= 2),
+              "kv groups: 32 rows a wave, no tile table, a whole number of 4-column pieces of O per group");
 static_assert(AE_K_LOADS >= 1 && AE_K_LOADS <= 8 && AE_V_LOADS >= 1 && AE_V_LOADS <= 8, "one burst per tile and wave");
 static_assert(AE_KCPR == 8 || AE_KCPR == 16 || AE_KCPR == 32 || AE_KCPR % 8 == 4 || AE_KCPR % 16 == 8,
               "swizzle is written for K rows of 128, 256 or 512 bytes, or an odd multiple of 64 or 128 bytes");
@@ -141,7 +159,7 @@ AE_DEV int ae_k_swz(int c, int row) {
 #define AE_Q_LOADS ((AE_WROWS * AE_KCPR) / 64)     // direct loads per lane for the wave's Q rows
 #define AE_Q_VIA_LDS (AE_BM * AE_KSTR <= AE_STAGE_BYTES)
 #define AE_O_LOADS ((AE_WROWS * AE_VCPR) / 64)
-#define AE_O_VIA_LDS (AE_NSPLIT == 1 && AE_NO <= 128 && AE_BM * AE_VSTR <= 2 * AE_STAGE_BYTES)
+#define AE_O_VIA_LDS (AE_NSPLIT == 1 && AE_KW == 1 && AE_NO <= 128 && AE_BM * AE_VSTR <= 2 * AE_STAGE_BYTES)
 
 // the wave's Q rows -> qs, in bursts of up to eight loads.  qg: row q0c of this (batch, head), 4 KiB low (see
 // ae_load_lds16_burst_base); row0 = first row of the wave - q0c; rows past `last` (relative to q0c) re-read it.
@@ -168,11 +186,17 @@ extern "C" __global__ __launch_bounds__(AE_NT)
 __attribute__((amdgpu_waves_per_eu(AE_WAVES_PER_EU)))
 void ae_prefill_kernel(const ae_attn_params p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ae_smem[];
-  ae_lds_byte* lds = (ae_lds_byte*)ae_smem;
-
   const int tid = threadIdx.x;
   const int lane = tid & 63;
+#if AE_KW == 1
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  ae_lds_byte* lds = (ae_lds_byte*)ae_smem;
+#else
+  const int wave_wg = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wave_wg / AE_NWAVES;         // kv group
+  const int wave = wave_wg % AE_NWAVES;       // ... and which 32 rows
+  ae_lds_byte* lds = (ae_lds_byte*)ae_smem + kg * (2 * AE_STAGE_BYTES);
+#endif
   const int l32 = lane & 31;
   const int hf = lane >> 5;
 
@@ -382,6 +406,15 @@ void ae_prefill_kernel(const ae_attn_params p) {
   int j = next_tile(0);
 #endif
   bool any_tile = j < j_end;
+#if AE_KW > 1
+  // group kg takes tiles j0 + kg, j0 + kg + AE_KW, ...; all groups make the same number of trips (the barriers)
+  const int j_trips = j_end + kg;
+  j += kg;
+#define AE_J_LIVE (j < j_end)
+#else
+  const int j_trips = j_end;
+#define AE_J_LIVE true
+#endif
   int cls[AE_RB];          // class of tile j for this lane's row of each row block
   // 1 once this lane's row of a row block has met a key it may see.  A row that never does - inside a q tile whose
   // other rows do: block masks finer than the q tile, masks such as q - 100 >= kv - ends with out = 0 and row
@@ -391,7 +424,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
   for (int rb = 0; rb < AE_RB; rb++) seen[rb] = 0.f;
 #pragma unroll
   for (int rb = 0; rb < AE_RB; rb++) cls[rb] = row_class(j, rb);
-  if (any_tile) load_tile(j, 0);
+  if (any_tile && AE_J_LIVE) load_tile(j, 0);
 #ifdef AE_HAS_KV_PREFETCH
   if (any_tile) {
 #pragma unroll
@@ -414,8 +447,8 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #endif
 
   int stage = 0;
-  while (j < j_end) {
-    const int jn = next_tile(j + 1);
+  while (j < j_trips) {
+    const int jn = next_tile(j + AE_KW);
     int cls_n[AE_RB];
 #pragma unroll
     for (int rb = 0; rb < AE_RB; rb++) cls_n[rb] = row_class(jn, rb);
@@ -443,7 +476,9 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #if AE_BAND_HI != 0x7fffffff
     active = active && kv0 + AE_BN - 1 >= q0w - AE_BAND_HI;
 #endif
-    if (active)
+    if (active && AE_J_LIVE)
+#elif AE_KW > 1
+    if (AE_J_LIVE)
 #endif
     {
     // ---- S^T = K Q^T: every K fragment feeds one MFMA per row block -------------------------
@@ -622,7 +657,104 @@ void ae_prefill_kernel(const ae_attn_params p) {
   }
 
   // ---- epilogue -------------------------------------------------------------------------------
-#if AE_NO > 128 && AE_NSPLIT == 1
+#if AE_KW > 1
+  // Every wave leaves its O and its row state in LDS (the stages are free: the loop ended with a barrier; element e of
+  // lane l at 16 * ((e / 4) * 64 + l) + 4 * (e % 4), so that all accesses are 16 bytes a lane in lane order), then takes
+  // the elements [kg * AE_NE, (kg + 1) * AE_NE) of its rows over all groups.
+  {
+    constexpr int AE_NE = AE_NO / AE_KW;
+    typedef __attribute__((address_space(3))) ae_f32x4 lds_f4;
+    typedef __attribute__((address_space(3))) float lds_f;
+    ae_lds_byte* xo = (ae_lds_byte*)ae_smem;                                  // [wave][AE_NO * 64] floats
+    lds_f* xs = (lds_f*)(xo + AE_KW * AE_NWAVES * AE_NO * 256);               // [wave][m, r, seen][64]
+#pragma unroll
+    for (int e = 0; e < AE_NO; e += 4) {
+      const ae_f32x16& a = oacc[0][e >> 4];
+      *(lds_f4*)(xo + wave_wg * (AE_NO * 256) + (e >> 2) * 1024 + lane * 16) =
+          (ae_f32x4){a[e & 15], a[(e & 15) + 1], a[(e & 15) + 2], a[(e & 15) + 3]};
+    }
+#if AE_KW_SOFTMAX
+    xs[(wave_wg * 3 + 0) * 64 + lane] = st[0].AE_SM_M;
+    xs[(wave_wg * 3 + 1) * 64 + lane] = st[0].AE_SM_R;
+#endif
+    xs[(wave_wg * 3 + 2) * 64 + lane] = seen[0];
+    __syncthreads();
+    float w[AE_KW];
+    bool row_seen = false;
+#if AE_KW_SOFTMAX
+    float mg[AE_KW], top = AE_NEG_INF, r_sum = 0.f;
+#endif
+#pragma unroll
+    for (int k = 0; k < AE_KW; k++) {
+      const int wk = (k * AE_NWAVES + wave) * 3;
+      const float sk = xs[(wk + 2) * 64 + lane];
+      row_seen = row_seen || ae_group_max(sk) > 0.f;
+      w[k] = 1.f;
+#if AE_KW_SOFTMAX
+      // (a group that met no visible key of the row has r = 0 and O = 0: its reference does not count)
+      mg[k] = sk > 0.f ? xs[wk * 64 + lane] : AE_NEG_INF;
+      top = __builtin_fmaxf(top, mg[k]);
+#endif
+    }
+#if AE_KW_SOFTMAX
+#pragma unroll
+    for (int k = 0; k < AE_KW; k++) {
+      w[k] = mg[k] > AE_NEG_INF ? ae_exp(mg[k] - top) : 0.f;
+      r_sum += w[k] > 0.f ? xs[((k * AE_NWAVES + wave) * 3 + 1) * 64 + lane] * w[k] : 0.f;
+    }
+    st[0].AE_SM_M = top;
+    st[0].AE_SM_R = r_sum;
+#endif
+    float o[AE_NE];
+#pragma unroll
+    for (int e = 0; e < AE_NE; e++) o[e] = 0.f;
+#pragma unroll
+    for (int k = 0; k < AE_KW; k++)
+#pragma unroll
+      for (int e = 0; e < AE_NE; e += 4) {
+        const ae_f32x4 v = *(const lds_f4*)(xo + (k * AE_NWAVES + wave) * (AE_NO * 256) + ((kg * AE_NE + e) >> 2) * 1024 + lane * 16);
+#pragma unroll
+        for (int t = 0; t < 4; t++) o[e + t] += w[k] > 0.f ? v[t] * w[k] : 0.f;
+      }
+    float frs[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1];
+    frs[0] = 0.f;
+    if (any_tile && row_seen) {
+      ae_epilogue<AE_NE>(o, st[0], frs, ctx[0], cust[0]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < AE_NE; e++) o[e] = 0.f;
+#pragma unroll
+      for (int i = 0; i < AE_N_ROWSCALES; i++) frs[i] = AE_NEG_INF;
+    }
+    if (q_ok[0]) {
+#if AE_NSPLIT > 1
+      const int64_t prow = ((((int64_t)b * p.seqlen_q + qrow[0]) * p.heads_q + h) * AE_NSPLIT) + split;
+      float* po = p.partial_o + prow * AE_DV;
+#else
+      ae_elem* po = (ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)qrow[0] * p.o_stride_s + (int64_t)h * p.o_stride_h;
+#endif
+#pragma unroll
+      for (int e = 0; e < AE_NE; e += 4) {
+        const int ea = kg * AE_NE + e;                      // element ea .. ea + 3: four neighbouring columns
+        const int col = (ea >> 4) * 32 + ((ea & 15) >> 2) * 8 + hf * 4;
+#if AE_NSPLIT > 1
+        *(ae_f32x4*)(po + col) = (ae_f32x4){o[e], o[e + 1], o[e + 2], o[e + 3]};
+#else
+        *(ae_elem4*)(po + col) = (ae_elem4){(ae_elem)o[e], (ae_elem)o[e + 1], (ae_elem)o[e + 2], (ae_elem)o[e + 3]};
+#endif
+      }
+      if (hf == 0 && kg == 0) {
+#pragma unroll
+        for (int i = 0; i < AE_N_ROWSCALES; i++)
+#if AE_NSPLIT > 1
+          p.partial_rs[(int64_t)i * p.batch * p.seqlen_q * p.heads_q * AE_NSPLIT + prow] = frs[i];
+#else
+          p.rowscale_out[i][((int64_t)b * p.heads_q + h) * p.seqlen_q + qrow[0]] = frs[i];
+#endif
+      }
+    }
+  }
+#elif AE_NO > 128 && AE_NSPLIT == 1
   // wide value heads: the epilogue functor (elementwise over the value columns) runs one 32-column block at a
   // time; a copy of all of O next to its accumulators would not fit the register file
 #pragma unroll

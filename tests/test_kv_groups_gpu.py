@@ -1,0 +1,83 @@
+"""Prefill tiles whose waves share the kv axis (AE_KW of csrc/kernels/ae_prefill.hip): every tile shape of
+core/lower/lower.py kv_group_tiles against the oracle, where groups run out of tiles, rows and keys end inside a tile,
+and rows see nothing."""
+import math
+
+import pytest
+import torch
+
+import attn_cases as C
+from attn_engine import AttentionEngine
+from core import CustomIO, meta_tensor
+from core.lower.lower import PrefillTiles, kv_group_tiles, kv_group_tiles_split
+from core.lower.prefill_op import PrefillOp
+from oracle import attention_ref as R
+from oracle import masks as OM
+
+TILES = [PrefillTiles(n_waves=1, kv_groups=4, block_n=32), PrefillTiles(n_waves=2, kv_groups=4, block_n=32),
+         PrefillTiles(n_waves=2, kv_groups=2, block_n=32), PrefillTiles(kv_groups=2)]
+
+
+def test_the_choice_follows_the_number_of_workgroups():
+    assert kv_group_tiles(128, 128, 32, 8, 8, True) == TILES[0]
+    assert kv_group_tiles(128, 128, 32, 333, 333, True) == TILES[1]
+    assert kv_group_tiles(64, 64, 32, 333, 333, True) == TILES[0]
+    assert kv_group_tiles(128, 128, 32, 1000, 1000, True) == TILES[2]
+    assert kv_group_tiles(128, 128, 32, 1500, 1500, True) == TILES[3]
+    assert kv_group_tiles(128, 128, 16, 1200, 1200, False) == TILES[3]
+    assert kv_group_tiles(128, 128, 64, 4096, 4096, True) is None
+    assert kv_group_tiles_split(32) == TILES[0] and kv_group_tiles_split(64) == TILES[2]
+    assert kv_group_tiles_split(128) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tiles", TILES, ids=lambda t: f"{t.block_m}x{t.kv_groups}x{t.block_n}")
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16)])
+@pytest.mark.parametrize("mask", ["none", "causal", "window", "shifted"])
+def test_kv_groups_against_the_oracle(cuda_device, tiles, D, dtype, mask):
+    mod = {"none": None, "causal": C.causal_mask, "window": C.make_sliding_window_mask(50),
+           "shifted": C.causal_shifted_mask}[mask]
+    for B, H, Hkv, S in ((1, 2, 2, 1), (1, 2, 1, 31), (2, 2, 2, 65), (1, 4, 2, 129), (2, 3, 3, 300)):
+        print(f"case kv groups {tiles.block_m}x{tiles.kv_groups}x{tiles.block_n} D{D} {mask} B{B} H{H} S{S}", flush=True)
+        if mask == "shifted" and S <= 128:
+            continue                                             # (nothing is visible)
+        q, k, v = C.make_inputs(B, S, S, H, Hkv, D, D, dtype, seed=S)
+        meta = (meta_tensor(B, H, S, D, dtype=dtype), meta_tensor(B, Hkv, S, D, dtype=dtype), meta_tensor(B, Hkv, S, D, dtype=dtype))
+        op = PrefillOp(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), mod, C.OnlineSoftmax(), "-inf", tiles=tiles)
+        assert op.tiles == tiles and "#define AE_KW " in op.source
+        out = op(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+        lse = op.final_rowscales["lse"].cpu()
+        vis = None if mod is None else torch.from_numpy(OM.dense_mask_grid(mod, B, H, S, S))
+        ref, rlse = R.softmax_attention(q, k, v, causal=False, mask=vis)
+        seen = torch.isfinite(rlse)
+        assert (out - ref.nan_to_num(0.0)).abs().max().item() <= 2e-2
+        assert torch.equal(torch.isfinite(lse), seen)
+        assert (lse[seen] - rlse[seen]).abs().max().item() <= 1e-3
+        assert (lse[~seen] == float("-inf")).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Sq,Skv", [(1, 40), (1, 1000), (31, 129), (33, 700), (64, 2100)])
+def test_kv_groups_of_split_launches(cuda_device, Sq, Skv):
+    B, H, D, dtype = 1, 3, 128, torch.float16
+    q, k, v = C.make_inputs(B, Sq, Skv, H, H, D, D, dtype, seed=7)
+    meta = (meta_tensor(B, H, Sq, D, dtype=dtype), meta_tensor(B, H, Skv, D, dtype=dtype), meta_tensor(B, H, Skv, D, dtype=dtype))
+    mod = AttentionEngine(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), None, C.OnlineSoftmax())
+    assert mod._op.tiles == kv_group_tiles_split(Sq)
+    out = mod(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+    ref, lse = R.softmax_attention(q, k, v, causal=False)
+    assert (out - ref).abs().max().item() <= 2e-2
+    assert (mod.final_rowscales["lse"].cpu() - lse).abs().max().item() <= 1e-3
+
+
+@pytest.mark.gpu
+def test_kv_groups_of_graphs_without_row_state(cuda_device):
+    B, H, S, D, dtype = 1, 2, 200, 64, torch.float16
+    q, k, v = C.make_inputs(B, S, S, H, H, D, D, dtype, seed=3)
+    meta = (meta_tensor(B, H, S, D, dtype=dtype),) * 3
+    mod = AttentionEngine(meta, CustomIO({"softmax_bias": (1,)}), C.make_sigmoid_score_mod(1 / math.sqrt(D)), None,
+                          C.OnlineIdentity())
+    assert mod._op.tiles.kv_groups == 4
+    out = mod(q.cuda(), k.cuda(), v.cuda(), torch.tensor([-2.0], device="cuda"))
+    ref = R.sigmoid_attention(q, k, v, bias=-2.0)
+    assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
