@@ -52,7 +52,8 @@ void ae_decode_combine_kernel(const ae_attn_params p) {
       for (int i = 0; i < G; i++) {
         const int k = k0 + i < AE_NSPLIT ? k0 + i : AE_NSPLIT - 1;
         const int kc = k < n_used ? k : n_used - 1;
-        val[i] = *(const ae_f32x4*)(p.partial_o + (row + kc) * AE_DV + dv);
+        // (read once: past the caches, see ae_mla_decode_ws.hip)
+        val[i] = __builtin_nontemporal_load((const ae_f32x4*)(p.partial_o + (row + kc) * AE_DV + dv));
       }
 #pragma unroll
       for (int i = 0; i < G; i++) {

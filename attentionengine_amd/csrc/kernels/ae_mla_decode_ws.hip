@@ -78,6 +78,10 @@ static_assert(AE_DV % 128 == 0 && AE_DV <= AE_D1, "V must be a prefix of the lat
 static_assert(AE_CPR % 8 == 0 && AE_CPR1 % 8 == 0, "chunk groups of eight must not straddle the two K tensors");
 static_assert((AE_BN * AE_CPR) % 64 == 0, "tile must be a whole number of 1 KiB blocks");
 static_assert(AE_L1 <= 8 && AE_L2 >= 1 && AE_BLOCKS >= AE_LOADS, "two bursts of at most eight loads per wave and tile");
+// chunk exchange of the results in LDS: inside groups that divide a head's chunks (16 where there are as many)
+#define AE_OSW1 ((AE_DVW / 8) & -(AE_DVW / 8))
+#define AE_OSW (AE_OSW1 < 16 ? AE_OSW1 - 1 : 15)
+static_assert(AE_DV * AE_HEADS_PER_WG * 4 <= AE_NSTAGE * AE_STAGE_BYTES, "the results of 64 heads fit the tile stages");
 static_assert(AE_NSTAGE >= 3, "a tile is multiplied by K one trip before it is multiplied as V");
 
 #ifndef AE_PAGED
@@ -584,9 +588,15 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   const unsigned long long ae_w2 = __builtin_amdgcn_s_memrealtime();     // the last trip is done
 #endif
 
+  // (... of every value wave: the score waves have left, and the tile stages take the results)
+  __syncthreads();
+  ae_lds_byte* obuf = lds + dvw * (AE_HEADS_PER_WG * AE_DVW * 4);
+  const int heads_left = group - ht * AE_HEADS_PER_WG;          // heads of the tile that exist
+  const int heads_here = heads_left < AE_HEADS_PER_WG ? heads_left : AE_HEADS_PER_WG;
   // ---- per-split epilogue: lane owns head 32*hb + l32, value columns AE_DVW*dvw + 32*db + 8*(r/4) + 4*hf + r%4
 #pragma unroll
   for (int hb = 0; hb < 2; hb++) {
+    if (hb * 32 >= heads_here) break;                           // (wave uniform)
     const int head_in_group = ht * AE_HEADS_PER_WG + hb * 32 + l32;
     const bool head_ok = head_in_group < group;
     const int hq = hk * group + (head_ok ? head_in_group : 0);
@@ -616,38 +626,62 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #pragma unroll
       for (int i = 0; i < AE_N_ROWSCALES; i++) frs[i] = AE_NEG_INF;
     }
-    if (!head_ok) continue;
+    // row scales: this lane's own head
+    if (head_ok && hf == 0 && dvw == 0) {
+      const int64_t row = ((int64_t)b * p.heads_q + hq) * p.num_splits + split;
+#pragma unroll
+      for (int i = 0; i < AE_N_ROWSCALES; i++) {
+        if (!direct) p.partial_rs[(int64_t)i * p.batch * p.heads_q * p.num_splits + row] = frs[i];
+        else if (p.rowscale_out[i]) p.rowscale_out[i][(int64_t)b * p.heads_q + hq] = frs[i];
+      }
+    }
+    // O leaves through LDS, a head's AE_DVW columns as one contiguous piece (512 bytes fp32, 256 bytes in the output
+    // type).  Stored straight from the accumulators it is 16 (8) bytes of each of 64 heads per instruction: lines that
+    // are written in eight pieces, which the L2 has to put together (partial results of B4 H128, 8 MB: 2.8 us a
+    // workgroup).  The partial results are stored past the cache (nontemporal, and read so by the merge kernel): their
+    // lines are read once, on another XCD; left dirty they are written back between the two launches and again when the
+    // next call's stores meet them.  B4 H128 Skv2048: call 24.7 -> 20.2 us.  16-byte chunks of a row are exchanged by the head number, so neither side meets a bank twice.
+    const int hl = hb * 32 + l32;
     if (direct) {
-    ae_elem* optr = (ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)hq * p.o_stride_h + dvw * AE_DVW;
 #pragma unroll
-    for (int db = 0; db < AE_NDB; db++)
+      for (int db = 0; db < AE_NDB; db++)
 #pragma unroll
-      for (int rg = 0; rg < 4; rg++) {
-        ae_elem4 w;
+        for (int rg = 0; rg < 4; rg++) {
+          ae_elem4 w;
 #pragma unroll
-        for (int i = 0; i < 4; i++) w[i] = (ae_elem)o[db * 16 + rg * 4 + i];
-        *(ae_elem4*)(optr + db * 32 + rg * 8 + hf * 4) = w;
-      }
-    if (hf == 0 && dvw == 0) {
+          for (int i = 0; i < 4; i++) w[i] = (ae_elem)o[db * 16 + rg * 4 + i];
+          *(__attribute__((address_space(3))) ae_elem4*)(obuf + hl * (AE_DVW * 2) + (((db * 4 + rg) ^ (hl & AE_OSW)) << 4) + hf * 8) = w;
+        }
+    } else {
 #pragma unroll
-      for (int i = 0; i < AE_N_ROWSCALES; i++)
-        if (p.rowscale_out[i]) p.rowscale_out[i][(int64_t)b * p.heads_q + hq] = frs[i];
+      for (int db = 0; db < AE_NDB; db++)
+#pragma unroll
+        for (int rg = 0; rg < 4; rg++) {
+          const ae_f32x4 w = {o[db * 16 + rg * 4 + 0], o[db * 16 + rg * 4 + 1], o[db * 16 + rg * 4 + 2], o[db * 16 + rg * 4 + 3]};
+          *(__attribute__((address_space(3))) ae_f32x4*)(obuf + hl * (AE_DVW * 4) + (((db * 8 + rg * 2 + hf) ^ (hl & AE_OSW)) << 4)) = w;
+        }
     }
-    continue;
-    }
-    const int64_t row = ((int64_t)b * p.heads_q + hq) * p.num_splits + split;
-    float* po = p.partial_o + row * AE_DV + dvw * AE_DVW;
-#pragma unroll
-    for (int db = 0; db < AE_NDB; db++)
-#pragma unroll
-      for (int rg = 0; rg < 4; rg++) {
-        ae_f32x4 w = {o[db * 16 + rg * 4 + 0], o[db * 16 + rg * 4 + 1], o[db * 16 + rg * 4 + 2], o[db * 16 + rg * 4 + 3]};
-        *(ae_f32x4*)(po + db * 32 + rg * 8 + hf * 4) = w;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the wave's own region: its LDS writes have been made)
+  {
+    if (direct) {
+      constexpr int CPH = AE_DVW / 8;                         // 16-byte chunks of a head's piece
+      ae_elem* ob = (ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)(hk * group + ht * AE_HEADS_PER_WG) * p.o_stride_h + dvw * AE_DVW;
+#pragma unroll 4
+      for (int i = 0; i * 64 < heads_here * CPH; i++) {
+        const int hl = (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
+        const ae_elem8 w = *(const __attribute__((address_space(3))) ae_elem8*)(obuf + hl * (AE_DVW * 2) + ((c ^ (hl & AE_OSW)) << 4));
+        if (hl < heads_here) *(ae_elem8*)(ob + (int64_t)hl * p.o_stride_h + c * 8) = w;
       }
-    if (hf == 0 && dvw == 0) {
-#pragma unroll
-      for (int i = 0; i < AE_N_ROWSCALES; i++)
-        p.partial_rs[(int64_t)i * p.batch * p.heads_q * p.num_splits + row] = frs[i];
+    } else {
+      constexpr int CPH = AE_DVW / 4;
+      float* ob = p.partial_o + (((int64_t)b * p.heads_q + hk * group + ht * AE_HEADS_PER_WG) * p.num_splits + split) * AE_DV + dvw * AE_DVW;
+#pragma unroll 8
+      for (int i = 0; i * 64 < heads_here * CPH; i++) {
+        const int hl = (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
+        const ae_f32x4 w = *(const __attribute__((address_space(3))) ae_f32x4*)(obuf + hl * (AE_DVW * 4) + ((c ^ (hl & AE_OSW)) << 4));
+        if (hl < heads_here) __builtin_nontemporal_store(w, (ae_f32x4*)(ob + (int64_t)hl * p.num_splits * AE_DV + c * 4));
+      }
     }
   }
 #if AE_CLOCK_STAMPS
