@@ -345,6 +345,11 @@ class PrefillOp:
             if self._clock_stamps():
                 cfg_src += "#define AE_CLOCK_STAMPS 1\n"
             module = rt.compile_module(self.tiles.template, {"ae_config.h": cfg_src,
+            else:
+                if self.functors.softmax is not None:
+                    cfg_src += "#define AE_PAD_GIVES_ZERO 1\n"
+                if self.functors.pad_free:
+                    cfg_src += "#define AE_PAD_FREE 1\n"
                                                           "ae_functors.h": self.functor_src},
                                        allow_spills=self.allow_spills,
                                        # the builds in which a spilled tuple came back wrong: 256 accumulator registers

@@ -128,6 +128,31 @@ AE_DEV void ae_load_lds16_burst_base(const void* base, const unsigned* off, ae_l
       : "memory");
 }
 
+// The same burst through a buffer resource whose range ends with the last row: 16-byte chunks past it arrive as zeros.
+// A tile that the end of the sequence cuts then needs no per-lane clamping (in the loop: eight address selects a tensor
+// and tile, and the registers for them), and its missing rows are zeros.  Loads 4n .. 4n + 3 go out behind one write of
+// M0; the 12-bit immediate moves the LDS and the global address, so off[i] = byte offset in the tile + 4096 -
+// (i % 4) KiB from a base that is passed 4 KiB low (offsets and range stay positive), `bytes` = the tile's valid bytes.
+template <int N>
+AE_DEV void ae_load_lds16_burst_rows(const void* base, unsigned bytes, const unsigned* off, ae_lds_u8* lds_first) {
+  static_assert(N >= 1 && N <= 8, "at most two bursts of four");
+  const unsigned long bv = (unsigned long)base;
+  const ae_u32x4 rsrc = {(unsigned)__builtin_amdgcn_readfirstlane((unsigned)bv),
+                         (unsigned)__builtin_amdgcn_readfirstlane((unsigned)(bv >> 32)) & 0xffffu,
+                         (unsigned)__builtin_amdgcn_readfirstlane(bytes + 4096u), 0x00020000u};
+  const unsigned m0a = __builtin_amdgcn_readfirstlane((unsigned)(unsigned long)lds_first);
+  asm volatile(
+      "s_mov_b32 m0, %4\n\ts_nop 0\n\t"
+      "buffer_load_dwordx4 %0, %5, 0 offen lds\n\t"
+      ".if %6 > 1\n\tbuffer_load_dwordx4 %1, %5, 0 offen offset:1024 lds\n\t.endif\n\t"
+      ".if %6 > 2\n\tbuffer_load_dwordx4 %2, %5, 0 offen offset:2048 lds\n\t.endif\n\t"
+      ".if %6 > 3\n\tbuffer_load_dwordx4 %3, %5, 0 offen offset:3072 lds\n\t.endif"
+      :
+      : "v"(off[0]), "v"(off[N > 1 ? 1 : 0]), "v"(off[N > 2 ? 2 : 0]), "v"(off[N > 3 ? 3 : 0]), "s"(m0a), "s"(rsrc), "n"(N)
+      : "memory");
+  if constexpr (N > 4) ae_load_lds16_burst_rows<N - 4>(base, bytes, off + 4, lds_first + 4096);
+}
+
 // ---- transcendentals ------------------------------------------------------------------
 AE_DEV float ae_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 AE_DEV float ae_exp(float x) { return __builtin_amdgcn_exp2f(x * AE_LOG2E); }

@@ -94,6 +94,16 @@
 #define AE_KV_PAD AE_NEG_INF
 #endif
 
+// 1: the proven online softmax - a score of -inf leaves the functor as exactly 0 (the running maximum starts at a
+// finite -1e38), so keys past the end need no second test
+#ifndef AE_PAD_GIVES_ZERO
+#define AE_PAD_GIVES_ZERO 0
+#endif
+// 1: an elementwise graph built of operations that stay finite - keys past the end arrive as rows of zeros (K and V), score
+// 0, and whatever finite weight they get multiplies a row of zeros: no test at all
+#ifndef AE_PAD_FREE
+#define AE_PAD_FREE 0
+#endif
 #ifndef AE_RB
 #define AE_RB 1
 #endif
@@ -300,48 +310,40 @@ void ae_prefill_kernel(const ae_attn_params p) {
   // (w*LOADS + i)*64 ... of the tile (whole rows when the row length is a power of two); lane L lands in LDS
   // chunk c' of row r, (w*LOADS + i)*64 + L = r*CPR + c', and fetches the permuted global chunk.
   // A lane's byte offset inside a tile never changes, so it is computed once; per tile only a
-  // wave-uniform base moves.  The K loads and the V loads of a wave each go out as one burst behind a
-  // single write of M0 (see ae_load_lds16_burst_base: bases are passed 4 KiB low and the offsets 4 KiB
-  // high, so that the offsets, which carry the compensation for the immediate offsets, stay >= 0).
-  auto k_lane_off = [&](int i, int last_row) AE_LAMBDA -> unsigned {
+  // wave-uniform base moves.  The K loads and the V loads of a wave each go out as one burst (two beyond four loads)
+  // behind a single write of M0 (ae_load_lds16_burst_rows).
+  auto k_lane_off = [&](int i) AE_LAMBDA -> unsigned {
     const int chunk = (wave * AE_K_LOADS + i) * 64 + lane;     // of the tile, in LDS order
-    int row = chunk / AE_KCPR;
+    const int row = chunk / AE_KCPR;
     const int c = ae_k_swz(chunk % AE_KCPR, row);
-    row = row < last_row ? row : last_row;
-    return (unsigned)((row * (int)p.k_stride_s + c * 8) * 2 + 4096 - (i - AE_K_LOADS / 2) * 1024);
+    return (unsigned)((row * (int)p.k_stride_s + c * 8) * 2 + 4096 - (i & 3) * 1024);
   };
-  auto v_lane_off = [&](int i, int last_row) AE_LAMBDA -> unsigned {
-    int row = (wave * AE_V_LOADS + i) * AE_V_RPI + lane / AE_VCPR;
+  auto v_lane_off = [&](int i) AE_LAMBDA -> unsigned {
+    const int row = (wave * AE_V_LOADS + i) * AE_V_RPI + lane / AE_VCPR;
     const int cp = lane % AE_VCPR;
     const int c = (((cp >> 1) ^ (row & AE_VSWM)) << 1) | (cp & 1);
-    row = row < last_row ? row : last_row;
-    return (unsigned)((row * (int)p.v_stride_s + c * 8) * 2 + 4096 - (i - AE_V_LOADS / 2) * 1024);
+    return (unsigned)((row * (int)p.v_stride_s + c * 8) * 2 + 4096 - (i & 3) * 1024);
   };
   unsigned koff[AE_K_LOADS], voff[AE_V_LOADS];
 #pragma unroll
-  for (int i = 0; i < AE_K_LOADS; i++) koff[i] = k_lane_off(i, AE_BN);
+  for (int i = 0; i < AE_K_LOADS; i++) koff[i] = k_lane_off(i);
 #pragma unroll
-  for (int i = 0; i < AE_V_LOADS; i++) voff[i] = v_lane_off(i, AE_BN);
+  for (int i = 0; i < AE_V_LOADS; i++) voff[i] = v_lane_off(i);
   auto load_tile = [&](int j, int stage) AE_LAMBDA {
     ae_lds_byte* ks = lds + stage * AE_STAGE_BYTES;
     ae_lds_byte* vs = ks + AE_K_BYTES;
     const char* gk = (const char*)kbase + (int64_t)j * AE_BN * p.k_stride_s * 2 - 4096;
     const char* gv = (const char*)vbase + (int64_t)j * AE_BN * p.v_stride_s * 2 - 4096;
-    unsigned ko[8], vo[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      ko[i] = koff[i < AE_K_LOADS ? i : 0];
-      vo[i] = voff[i < AE_V_LOADS ? i : 0];
+    int rows = AE_BN;
 #if !AE_EVEN_KV
-      // rows past the end re-read the last row (masked later)
-      if (j * AE_BN + AE_BN > p.seqlen_kv) {
-        ko[i] = k_lane_off(i < AE_K_LOADS ? i : 0, p.seqlen_kv - 1 - j * AE_BN);
-        vo[i] = v_lane_off(i < AE_V_LOADS ? i : 0, p.seqlen_kv - 1 - j * AE_BN);
-      }
+    rows = p.seqlen_kv - j * AE_BN;                            // rows past the end arrive as zeros
+    rows = __builtin_amdgcn_readfirstlane(rows < AE_BN ? rows : AE_BN);
+    asm("" : "+s"(rows));                                      // (opaque: the compiler would split the loop over it)
 #endif
-    }
-    ae_load_lds16_burst_base<AE_K_LOADS>(gk, ko, ks + (wave * AE_K_LOADS + AE_K_LOADS / 2) * 1024);
-    ae_load_lds16_burst_base<AE_V_LOADS>(gv, vo, vs + (wave * AE_V_LOADS + AE_V_LOADS / 2) * 1024);
+    ae_load_lds16_burst_rows<AE_K_LOADS>(gk, (unsigned)(((rows - 1) * (int)p.k_stride_s + AE_D) * 2), koff,
+                                         ks + wave * AE_K_LOADS * 1024);
+    ae_load_lds16_burst_rows<AE_V_LOADS>(gv, (unsigned)(((rows - 1) * (int)p.v_stride_s + AE_DV) * 2), voff,
+                                         vs + wave * AE_V_LOADS * 1024);
   };
   // next tile index >= j that has work (block table) or j itself
   auto next_tile = [&](int j) AE_LAMBDA {
@@ -548,7 +550,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
           s[e] = ae_mask_mod(b, h, qrow[rb], kvb + ae_kv_off(e)) ? s[e] : AE_NEG_INF;
       }
 #endif
-#if !AE_EVEN_KV
+#if !AE_EVEN_KV && !AE_PAD_FREE && AE_MASK_MODE != 1     // (causal over equal lengths: behind the diagonal of every row)
       if (kv0 + AE_BN > p.seqlen_kv) {
 #pragma unroll
         for (int e = 0; e < AE_NS; e++) s[e] = (kvb + ae_kv_off(e) < p.seqlen_kv) ? s[e] : AE_KV_PAD;
@@ -589,7 +591,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
       if (jn < j_end) ae_prefetch_custom(cust[rb], jn * AE_BN + 4 * hf, q0w + rb * 32, jn * AE_BN, p);
 #endif
 
-#if !AE_EVEN_KV
+#if !AE_EVEN_KV && !AE_PAD_GIVES_ZERO && !AE_PAD_FREE
       if (kv0 + AE_BN > p.seqlen_kv) {
 #pragma unroll
         for (int e = 0; e < AE_NS; e++) s[e] = (kvb + ae_kv_off(e) < p.seqlen_kv) ? s[e] : 0.f;
@@ -600,7 +602,13 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #pragma unroll
       for (int kk = 0; kk < AE_BN / 16; kk++)
 #pragma unroll
-        for (int t = 0; t < 8; t++) pf[rb][kk][t] = (ae_elem)s[kk * 8 + t];
+        for (int t = 0; t < 8; t += 2) {
+          typedef float ae_f32x2 __attribute__((ext_vector_type(2)));
+          const ae_f32x2 x2 = {s[kk * 8 + t], s[kk * 8 + t + 1]};
+          const ae_elem2 y2 = __builtin_convertvector(x2, ae_elem2);       // one packed conversion
+          pf[rb][kk][t] = y2[0];
+          pf[rb][kk][t + 1] = y2[1];
+        }
 
 #if !AE_O_SCALE_ONE
       // skip the rescale when no row of this block changed its scale (wave-uniform branch)

@@ -104,6 +104,13 @@ static_assert(AE_KV_STAGES == 2 || AE_KV_STAGES == 3, "two or three K / V stages
 #ifndef AE_TOP_PREFETCH
 #define AE_TOP_PREFETCH (AE_MASK_MODE == 0)
 #endif
+// keys past the end of the sequence are tested for on the tile that holds them: not under a causal mask over equal
+// lengths (they lie behind every row's diagonal), nor for elementwise graphs that stay finite (AE_PAD_FREE, see
+// ae_prefill.hip: the missing K and V rows are zeros)
+#ifndef AE_PAD_FREE
+#define AE_PAD_FREE 0
+#endif
+#define AE_PAD_TEST (!AE_EVEN_KV && !AE_PAD_FREE && AE_MASK_MODE != 1)
 // What turns a score into p.  0: the online softmax described above.  1: the generated functor
 // ae_online_fwd itself, two scores at a time, for graphs the lowering has shown to be ELEMENTWISE
 // (out = sum_kv f(s) v, attn_script/sigmoidattn.py, reluattn.py: no row state, no row reduction, no use of
@@ -272,7 +279,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #elif AE_HAS_MASK_MOD
     nm = true;
 #endif
-#if !AE_EVEN_KV
+#if AE_PAD_TEST
     nm = nm || (j * AE_BN + AE_BN > p.seqlen_kv);
 #endif
   };
@@ -283,56 +290,42 @@ void ae_prefill_kernel(const ae_attn_params p) {
   // Direct HBM -> LDS tile loads with the chunk swizzles of ae_prefill.hip: wave w fills the AE_K_LOADS
   // (AE_V_LOADS) consecutive 1 KiB blocks starting at block w*AE_K_LOADS of a K (V) tile.  A lane's byte
   // offset inside a tile never changes, so it is computed once; per tile only a wave-uniform base moves.
-  // A tile's loads go out as one burst behind a single write of M0 (see ae_load_lds16_burst; the offsets
-  // carry the compensation for its immediate offsets).
-  // (bases are passed 4 KiB low and the offsets 4 KiB high, so that the compensated offsets stay >= 0)
-  auto k_lane_off = [&](int i, int last_row) AE_LAMBDA -> unsigned {
-    int row = (wave * AE_K_LOADS + i) * AE_K_RPI + lane / AE_KCPR;
+  // A wave's loads of a tensor's tile go out as one burst behind a single write of M0 (ae_load_lds16_burst_rows).
+  auto k_lane_off = [&](int i) AE_LAMBDA -> unsigned {
+    const int row = (wave * AE_K_LOADS + i) * AE_K_RPI + lane / AE_KCPR;
     const int c = (lane % AE_KCPR) ^ (row & (AE_KCPR - 1));
-    row = row < last_row ? row : last_row;
-    return (unsigned)((row * (int)p.k_stride_s + c * 8) * 2 + 4096 - (i - AE_K_LOADS / 2) * 1024);
+    return (unsigned)((row * (int)p.k_stride_s + c * 8) * 2 + 4096 - (i & 3) * 1024);
   };
-  auto v_lane_off = [&](int i, int last_row) AE_LAMBDA -> unsigned {
-    int row = (wave * AE_V_LOADS + i) * AE_V_RPI + lane / AE_VCPR;
+  auto v_lane_off = [&](int i) AE_LAMBDA -> unsigned {
+    const int row = (wave * AE_V_LOADS + i) * AE_V_RPI + lane / AE_VCPR;
     const int cp = lane % AE_VCPR;
     const int c = (((cp >> 1) ^ (row & (AE_VPPR - 1))) << 1) | (cp & 1);
-    row = row < last_row ? row : last_row;
-    return (unsigned)((row * (int)p.v_stride_s + c * 8) * 2 + 4096 - (i - AE_V_LOADS / 2) * 1024);
+    return (unsigned)((row * (int)p.v_stride_s + c * 8) * 2 + 4096 - (i & 3) * 1024);
   };
   unsigned koff[AE_K_LOADS], voff[AE_V_LOADS];
 #pragma unroll
-  for (int i = 0; i < AE_K_LOADS; i++) koff[i] = k_lane_off(i, AE_BN);
+  for (int i = 0; i < AE_K_LOADS; i++) koff[i] = k_lane_off(i);
 #pragma unroll
-  for (int i = 0; i < AE_V_LOADS; i++) voff[i] = v_lane_off(i, AE_BN);
+  for (int i = 0; i < AE_V_LOADS; i++) voff[i] = v_lane_off(i);
+  // valid bytes of tile j of a tensor with these row stride and width (elements): rows past the end arrive as zeros
+  auto tile_bytes = [&](int j, int stride, int width) AE_LAMBDA -> unsigned {
+#if AE_EVEN_KV
+    const int rows = AE_BN;
+#else
+    int rows = p.seqlen_kv - j * AE_BN;
+    rows = rows < AE_BN ? rows : AE_BN;
+#endif
+    return (unsigned)(((rows - 1) * stride + width) * 2);
+  };
   auto load_k = [&](int j, int stage) AE_LAMBDA {
     const char* g = (const char*)kbase + (int64_t)j * AE_BN * p.k_stride_s * 2 - 4096;
-    unsigned gp[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int ii = i < AE_K_LOADS ? i : 0;
-      unsigned off = koff[ii];
-#if !AE_EVEN_KV
-      // rows past the end re-read the last row (masked later)
-      if (j * AE_BN + AE_BN > p.seqlen_kv) off = k_lane_off(ii, p.seqlen_kv - 1 - j * AE_BN);
-#endif
-      gp[i] = off;
-    }
-    ae_load_lds16_burst_base<AE_K_LOADS>(g, gp, lds + stage * AE_K_BYTES + (wave * AE_K_LOADS + AE_K_LOADS / 2) * 1024);
+    ae_load_lds16_burst_rows<AE_K_LOADS>(g, tile_bytes(j, (int)p.k_stride_s, AE_D), koff,
+                                         lds + stage * AE_K_BYTES + wave * AE_K_LOADS * 1024);
   };
   auto load_v = [&](int j, int stage) AE_LAMBDA {
     const char* g = (const char*)vbase + (int64_t)j * AE_BN * p.v_stride_s * 2 - 4096;
-    unsigned gp[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int ii = i < AE_V_LOADS ? i : 0;
-      unsigned off = voff[ii];
-#if !AE_EVEN_KV
-      if (j * AE_BN + AE_BN > p.seqlen_kv) off = v_lane_off(ii, p.seqlen_kv - 1 - j * AE_BN);
-#endif
-      gp[i] = off;
-    }
-    ae_load_lds16_burst_base<AE_V_LOADS>(
-        g, gp, lds + AE_KV_STAGES * AE_K_BYTES + stage * AE_V_BYTES + (wave * AE_V_LOADS + AE_V_LOADS / 2) * 1024);
+    ae_load_lds16_burst_rows<AE_V_LOADS>(g, tile_bytes(j, (int)p.v_stride_s, AE_DV), voff,
+                                         lds + AE_KV_STAGES * AE_K_BYTES + stage * AE_V_BYTES + wave * AE_V_LOADS * 1024);
   };
 
   // ---- the first tiles are requested before anything else is set up: the zeroing of the accumulators, the
@@ -493,7 +486,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
     xa[u][1] = ae_exp2(xa[u][1]);
 #endif
   };
-  auto stage_c = [&](int u) AE_LAMBDA {
+  auto stage_c = [&](int u, auto last_tag) AE_LAMBDA {
     const int qb = u & 1, e = (u >> 3) * 8 + ((u >> 1) & 3) * 2;
     typedef float ae_f32x2 __attribute__((ext_vector_type(2)));
     const ae_f32x2 x2 = {xa[u][0], xa[u][1]};
@@ -501,8 +494,9 @@ void ae_prefill_kernel(const ae_attn_params p) {
     pf[qb][e >> 3][(e & 7) >> 1] = __builtin_bit_cast(unsigned, hv);
 #if AE_PIPE_KIND == 1
     (void)rsum;
-#if !AE_EVEN_KV
-    // keys past the end: f(-inf) need not be zero
+#if AE_PAD_TEST
+    // keys past the end: f(-inf) need not be zero.  Only the last tile a wave multiplies can hold such keys.
+    if (!decltype(last_tag)::value) return;
     if (ae_kv_off(e) >= kv_lim) pf[qb][e >> 3][(e & 7) >> 1] = 0u;
     else if (ae_kv_off(e + 1) >= kv_lim) pf[qb][e >> 3][(e & 7) >> 1] &= 0xffffu;
 #endif
@@ -519,7 +513,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #pragma unroll
     for (int u = 0; u < 32; u++) {
       const int a = (u * AE_EXP_SPAN) / 32;
-      if (a + 2 == g) stage_c(u);
+      if (a + 2 == g) stage_c(u, ae_tag_false{});
       if (a + 1 == g) stage_b(u);
       if (a == g) stage_a(u);
     }
@@ -530,7 +524,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #pragma unroll
     for (int u = 0; u < 32; u++) stage_b(u);
 #pragma unroll
-    for (int u = 0; u < 32; u++) stage_c(u);
+    for (int u = 0; u < 32; u++) stage_c(u, ae_tag_true{});
   };
   // Tile j sits in sv, its lane-local maxima in mx: mask fix-up where the tile needs it, then the
   // row maxima against the (lazy) reference.  The common case ends after two exchanges and a ballot; a
@@ -560,7 +554,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #elif AE_HAS_MASK_MOD
           vis = ae_mask_mod(b, h, qrow[qb], kv);
 #endif
-#if !AE_EVEN_KV
+#if AE_PAD_TEST
           vis = vis && (kv < p.seqlen_kv);
 #endif
           const float x = vis ? sv[qb][e] : AE_NEG_INF;
