@@ -677,16 +677,20 @@ def pipelined_tiles(d: int, dv: int) -> PrefillTiles:
 
 
 def choose_prefill_tiles(d: int, dv: int, seqlen_q: int = 0, softmax=None, batch_heads: int = 0,
-                         elementwise: bool = False, seqlen_kv: int = 0) -> PrefillTiles:
+                         elementwise: bool = False, seqlen_kv: int = 0, bf16: bool = False,
+                         masked: bool = True) -> PrefillTiles:
     """The direct-to-LDS kernels handle head dims 64 and 128 (and, the generic one, 96, 160, 192, 256 and value
     head dims up to 512, with one wave per SIMD where the accumulators need it): the
     software-pipelined one (64 rows per wave, 256-row q tiles, one wave per SIMD) when the graph is
     the online softmax of scaled scores, or elementwise (out = sum f(s) v: the kernel then calls the
     generated functor), and the problem has enough q tiles to occupy the chip
     (measured on B2 H32 S4096 D128 fp16: 1.0 against 0.86 PFLOP/s non-causal) and its rows are long enough
-    for the pipeline to pay (short sequences are bound by the Q / O traffic and the start-up of a workgroup,
-    which two workgroups per CU hide better: 16k tokens fp16 H32, S256 D128 0.136 against 0.162 ms, S512
-    D64 causal 0.085 against 0.111 ms; from S1024 D128 / S2048 D64 on the pipelined kernel wins), otherwise
+    for the pipeline to pay: short sequences are bound by the Q / O traffic and the start-up of a workgroup,
+    which two workgroups per CU hide better.  16k tokens, H32, pipelined against generic, us: D128 fp16 causal S512
+    184 / 164, S1000 243 / 244, S2000 364 / 390; bf16, which keeps one more instruction per score in the pipeline,
+    S1000 251 / 239, S2000 372 / 376, S4096 588 / 617 - lines at 1024 and 1792 keys.  At head dim 64, where four generic
+    waves share a SIMD, only fp16 without a mask and from 4096 keys on: 609 / 630 (causal 370 / 360, bf16 677 / 596,
+    sigmoid 715 / 642).  Otherwise
     the generic one (32 rows per wave, two waves per SIMD, runs any functor).  Other head dims use the
     register-staged kernel with padded LDS rows (ae_prefill_simple.hip), with one wave per SIMD and a
     shorter kv tile once the accumulators outgrow 256 registers.  AE_PREFILL_KERNEL=generic|pipelined
@@ -704,11 +708,10 @@ def choose_prefill_tiles(d: int, dv: int, seqlen_q: int = 0, softmax=None, batch
     if d in DIRECT_D and dv in DIRECT_DV:
         force = os.environ.get("AE_PREFILL_KERNEL", "")
         n_tiles = batch_heads * ((seqlen_q + 255) // 256)
-        # (elementwise graphs at head dim 64 have too little matrix work per score for the pipelined kernel's
-        # one wave per SIMD to pay: relu attention B64 H6 S2048 D64 0.48 ms against 0.45 ms in the generic one)
-        fits = softmax is not None or (elementwise and max(d, dv) > 64)
-        if seqlen_kv and seqlen_kv * max(d, dv) < 1024 * 128:
-            fits = False
+        if max(d, dv) > 64:
+            fits = not seqlen_kv or seqlen_kv >= (1792 if bf16 else 1024)
+        else:
+            fits = softmax is not None and not bf16 and not masked and (not seqlen_kv or seqlen_kv >= 4096)
         if d in (64, 128) and (softmax is not None or elementwise) and force != "generic" and (
                 force == "pipelined" or (fits and n_tiles >= (3 * _MI355X_CUS) // 4)):
             return pipelined_tiles(d, dv)

@@ -62,7 +62,7 @@ class PrefillOp:
                        and not split_kv)
         if self.DV > 256 and not single_pass:
             self.DV_launch = next(c for c in (256, 192, 128, 96, 64, 32) if self.DV % c == 0)
-        self.mask_mod = mask_mod
+        self.mask_mod, self._probed = mask_mod, None
         self.elementwise_mask = mask_mod is not None and mask_value == "-inf"
         self.mask_value_zero = mask_value == "0"
         self.extern_block_mask = bool(extern_block_mask)
@@ -80,7 +80,8 @@ class PrefillOp:
                                             self._pipe_softmax,
                                             _dim(q_meta.shape[0], 1) * _dim(q_meta.shape[1], 1),
                                             elementwise=self._pipe_elementwise,
-                                            seqlen_kv=_dim(k_meta.shape[2], 0))
+                                            seqlen_kv=_dim(k_meta.shape[2], 0),
+                                            bf16=self.dtype == torch.bfloat16, masked=mask_mod is not None)
         # Masks that reach the kernel as a tile table (anything but none / exactly causal) go to the generic
         # kernel: with its 128-row q tiles fewer tiles are partly visible, and its masked path costs less than
         # the pipelined kernel's (B2 H32 S4096 D128, sliding window of 256: 0.13 against 0.31 ms; a random block
@@ -88,6 +89,12 @@ class PrefillOp:
         if self.tiles.rows_per_wave == 64 and os.environ.get("AE_PREFILL_KERNEL", "") != "pipelined" and (
                 self.extern_block_mask or (mask_mod is not None and self._probe_mask(q_meta, v_meta).mode == 2)):
             self.tiles = L.PrefillTiles()
+        # Band masks are read in 32-key tiles (B2 H32 S4096 D128, window of 256: 94.8 -> 88.4 us with them, of 1024 184 -> 180):
+        # less of the band's edges is multiplied.
+        if self.mask_mod is not None and self.tiles == L.PrefillTiles() and self.D in (64, 128) and self.DV in (64, 128):
+            band = self._probe_mask(q_meta, v_meta).band
+            if band is not None and band[1] is not None:
+                self.tiles = L.PrefillTiles(block_n=32)
         groups = self._groups = self._kv_group_choice(q_meta, v_meta, split_kv)
         if groups is not None:
             self.tiles = groups
@@ -191,8 +198,11 @@ class PrefillOp:
     def _probe_mask(self, q_meta, v_meta):
         """The mask plan at the declared sequence lengths (4096 where they are dynamic), for batch entry and head 0:
         mode 2 = the mask needs a tile table (or is a band)."""
-        sq, skv = _dim(q_meta.shape[2], 4096), _dim(v_meta.shape[2], 4096)
-        return plan_mask(self.mask_mod, self.functors.mask, 1, 1, sq, skv, 128, 64, elementwise=self.elementwise_mask)
+        if self._probed is None:
+            sq, skv = _dim(q_meta.shape[2], 4096), _dim(v_meta.shape[2], 4096)
+            self._probed = plan_mask(self.mask_mod, self.functors.mask, 1, 1, sq, skv, 128, 64,
+                                     elementwise=self.elementwise_mask)
+        return self._probed
 
     def _kv_group_choice(self, q_meta, v_meta, split_kv):
         """Tiles whose waves share the kv axis, where this engine's graph, mask and declared extents allow and want them:
@@ -335,6 +345,11 @@ class PrefillOp:
                                       exact_scale=self.exact_scale)
             if self.mask_value_zero:
                 cfg_src += "#define AE_MASK_VALUE_ZERO 1\n"
+            else:
+                if self.functors.softmax is not None:
+                    cfg_src += "#define AE_PAD_GIVES_ZERO 1\n"
+                if self.functors.pad_free:
+                    cfg_src += "#define AE_PAD_FREE 1\n"
             if mask_mode == 2:
                 cfg_src += f"#define AE_TT_ROWS {table_rows}\n#define AE_HEAVY_LAST {1 if heavy_last else 0}\n"
             if band is not None:
@@ -345,11 +360,6 @@ class PrefillOp:
             if self._clock_stamps():
                 cfg_src += "#define AE_CLOCK_STAMPS 1\n"
             module = rt.compile_module(self.tiles.template, {"ae_config.h": cfg_src,
-            else:
-                if self.functors.softmax is not None:
-                    cfg_src += "#define AE_PAD_GIVES_ZERO 1\n"
-                if self.functors.pad_free:
-                    cfg_src += "#define AE_PAD_FREE 1\n"
                                                           "ae_functors.h": self.functor_src},
                                        allow_spills=self.allow_spills,
                                        # the builds in which a spilled tuple came back wrong: 256 accumulator registers
