@@ -160,6 +160,21 @@ AE_DEV int ae_k_swz(int c, int row) {
 #endif
 }
 
+// Fragments that a wave reads from LDS ahead of the MFMA that takes them: rings with one scheduling fence per MFMA (left
+// to itself the compiler keeps one or two reads in flight and waits for each).  Not where the head is so wide that
+// the ring's registers cost a wave per SIMD (D 192, DV 128, 32-key tiles: 168 -> 180 registers, 294 -> 313 us), nor in
+// the builds that run one wave per SIMD with every register taken.  bf16, without a mask, B16 H16 S1000: D 64 90.0 ->
+// 88.2 us, D 128 160.3 -> 155.6 us (with the shorter epilogue); causal B8 H32 S1000 D128 112.3 -> 110.0 us.
+#if AE_D <= 128 && AE_DV <= 128 && AE_RB == 1
+#define AE_K_AHEAD 4
+#define AE_V_AHEAD 3
+#define AE_RING_FENCE() __builtin_amdgcn_sched_barrier(0)
+#else
+#define AE_K_AHEAD 0
+#define AE_V_AHEAD 0
+#define AE_RING_FENCE()
+#endif
+
 // Q rows on their way in and O rows on their way out pass through LDS as whole rows (16 lanes per 256-byte row).
 // A lane that loads its own row's fragments, or stores its own row's results, touches 32 rows per instruction,
 // 16 bytes of each: the workgroups of a launch start and end together and queue behind each other's requests
@@ -491,15 +506,22 @@ void ae_prefill_kernel(const ae_attn_params p) {
       for (int nb = 0; nb < AE_NB; nb++)
 #pragma unroll
         for (int r = 0; r < 16; r++) sacc[rb][nb][r] = 0.f;
+    auto k_frag = [&](int f) AE_LAMBDA -> ae_elem8 {
+      return *(__attribute__((address_space(3))) ae_elem8*)(
+          ks_ + k_row_off + f % AE_NB * 32 * AE_KSTR + (ae_k_swz(2 * (f / AE_NB) + hf, l32) << 4));
+    };
+    constexpr int NKF = (AE_D / 16) * AE_NB;
+    ae_elem8 kring[AE_K_AHEAD + 1];
 #pragma unroll
-    for (int ks = 0; ks < AE_D / 16; ks++) {
+    for (int f = 0; f < AE_K_AHEAD && f < NKF; f++) kring[f] = k_frag(f);
+    AE_RING_FENCE();
 #pragma unroll
-      for (int nb = 0; nb < AE_NB; nb++) {
-        ae_elem8 kf = *(__attribute__((address_space(3))) ae_elem8*)(
-            ks_ + k_row_off + nb * 32 * AE_KSTR + (ae_k_swz(2 * ks + hf, l32) << 4));
+    for (int f = 0; f < NKF; f++) {
+      if (f + AE_K_AHEAD < NKF) kring[(f + AE_K_AHEAD) % (AE_K_AHEAD + 1)] = k_frag(f + AE_K_AHEAD);
 #pragma unroll
-        for (int rb = 0; rb < AE_RB; rb++) sacc[rb][nb] = ae_mfma32(kf, qf[rb][ks], sacc[rb][nb]);
-      }
+      for (int rb = 0; rb < AE_RB; rb++)
+        sacc[rb][f % AE_NB] = ae_mfma32(kring[f % (AE_K_AHEAD + 1)], qf[rb][f / AE_NB], sacc[rb][f % AE_NB]);
+      AE_RING_FENCE();
     }
 
     ae_elem8 pf[AE_RB][AE_BN / 16];
@@ -635,23 +657,29 @@ void ae_prefill_kernel(const ae_attn_params p) {
     }
 
     // ---- O^T += V^T P^T: every V fragment feeds one MFMA per row block ------------------------
-#pragma unroll
-    for (int kk = 0; kk < AE_BN / 16; kk++) {
-      // slots 0..3 of this k-step are kv rows rb0+4*hf+0..3, slots 4..7 rows rb0+8+4*hf+0..3
+    auto v_frag = [&](int f) AE_LAMBDA -> ae_elem8 {
+      // slots 0..3 of k-step kk are kv rows rb0+4*hf+0..3, slots 4..7 rows rb0+8+4*hf+0..3
+      // (rb0 and +8 are multiples of 8, so they do not change the swizzle)
+      const int kk = f / AE_NDB;
       const int rb0 = (kk >> 1) * 32 + (kk & 1) * 16;
+      ae_lds_byte* a0 = vs_ + v_row_off + rb0 * AE_VSTR + (((2 * (f % AE_NDB) + v_g) ^ v_sw) << 5);
+      ae_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)a0);
+      ae_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (__attribute__((address_space(3))) ae_s16x4*)(a0 + 8 * AE_VSTR));
+      return __builtin_bit_cast(ae_elem8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    constexpr int NVF = (AE_BN / 16) * AE_NDB;
+    ae_elem8 vring[AE_V_AHEAD + 1];
 #pragma unroll
-      for (int db = 0; db < AE_NDB; db++) {
-        // (rb0 and +8 are multiples of 8, so they do not change the swizzle)
-        ae_lds_byte* a0 = vs_ + v_row_off + rb0 * AE_VSTR + (((2 * db + v_g) ^ v_sw) << 5);
-        ae_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) ae_s16x4*)a0);
-        ae_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) ae_s16x4*)(a0 + 8 * AE_VSTR));
-        ae_elem8 vf = __builtin_bit_cast(
-            ae_elem8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    for (int f = 0; f < AE_V_AHEAD && f < NVF; f++) vring[f] = v_frag(f);
+    AE_RING_FENCE();
 #pragma unroll
-        for (int rb = 0; rb < AE_RB; rb++) oacc[rb][db] = ae_mfma32(vf, pf[rb][kk], oacc[rb][db]);
-      }
+    for (int f = 0; f < NVF; f++) {
+      if (f + AE_V_AHEAD < NVF) vring[(f + AE_V_AHEAD) % (AE_V_AHEAD + 1)] = v_frag(f + AE_V_AHEAD);
+#pragma unroll
+      for (int rb = 0; rb < AE_RB; rb++)
+        oacc[rb][f % AE_NDB] = ae_mfma32(vring[f % (AE_V_AHEAD + 1)], pf[rb][f / AE_NDB], oacc[rb][f % AE_NDB]);
+      AE_RING_FENCE();
     }
     }
 
@@ -814,16 +842,18 @@ void ae_prefill_kernel(const ae_attn_params p) {
     float frs[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1];
     frs[0] = 0.f;
     const bool row_seen = ae_group_max(seen[rb]) > 0.f;     // (both lanes of a row, or neither)
-    if (any_tile && row_seen) {
-      ae_epilogue<AE_NO>(o, st[rb], frs, ctx[rb], cust[rb]);
-    } else {
-      // no visible kv block for this q-tile, or no visible key for this row: out = 0 (blockattn_tl.py:153-160),
-      // rowscales = -inf
+    // no visible kv block for this q-tile, or no visible key for this row: out = 0 (blockattn_tl.py:153-160),
+    // rowscales = -inf.  (selected after the functor and, where they are converted, on the converted pairs: as the two
+    // sides of a branch every element was a register to clear and a conversion of its own)
+    const bool live = any_tile && row_seen;
+    ae_epilogue<AE_NO>(o, st[rb], frs, ctx[rb], cust[rb]);
 #pragma unroll
-      for (int e = 0; e < AE_NO; e++) o[e] = 0.f;
-#pragma unroll
-      for (int i = 0; i < AE_N_ROWSCALES; i++) frs[i] = AE_NEG_INF;
-    }
+    for (int i = 0; i < AE_N_ROWSCALES; i++) frs[i] = live ? frs[i] : AE_NEG_INF;
+    auto out4 = [&](int e) AE_LAMBDA -> ae_elem4 {
+      typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+      const u32x2 w = __builtin_bit_cast(u32x2, (ae_elem4){(ae_elem)o[e], (ae_elem)o[e + 1], (ae_elem)o[e + 2], (ae_elem)o[e + 3]});
+      return __builtin_bit_cast(ae_elem4, (u32x2){live ? w[0] : 0u, live ? w[1] : 0u});
+    };
 #if AE_NSPLIT > 1
     // partial result of this split: fp32, rows ordered (batch, q position, head) so that the merge
     // kernel sees them as B x (Sq*Hq) "heads" of a one-token decode and writes out [B,Sq,Hq,DV]
@@ -834,7 +864,9 @@ void ae_prefill_kernel(const ae_attn_params p) {
       for (int db = 0; db < AE_NDB; db++)
 #pragma unroll
         for (int rg = 0; rg < 4; rg++) {
-          ae_f32x4 w = {o[db * 16 + rg * 4 + 0], o[db * 16 + rg * 4 + 1], o[db * 16 + rg * 4 + 2], o[db * 16 + rg * 4 + 3]};
+          ae_f32x4 w;
+#pragma unroll
+          for (int t = 0; t < 4; t++) w[t] = live ? o[db * 16 + rg * 4 + t] : 0.f;
           *(ae_f32x4*)(po + db * 32 + rg * 8 + hf * 4) = w;
         }
       if (hf == 0) {
@@ -855,10 +887,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
       for (int db = 0; db < AE_NDB; db++)
 #pragma unroll
         for (int rg = 0; rg < 4; rg++) {
-          ae_elem4 w;
-#pragma unroll
-          for (int t = 0; t < 4; t++) w[t] = (ae_elem)o[db * 16 + rg * 4 + t];
-          *(__attribute__((address_space(3))) ae_elem4*)(orow + (((db * 4 + rg) ^ osw) << 4)) = w;
+          *(__attribute__((address_space(3))) ae_elem4*)(orow + (((db * 4 + rg) ^ osw) << 4)) = out4(db * 16 + rg * 4);
         }
     }
     if (q_ok[rb] && hf == 0) {
@@ -874,10 +903,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
       for (int db = 0; db < AE_NDB; db++)
 #pragma unroll
         for (int rg = 0; rg < 4; rg++) {
-          ae_elem4 w;
-#pragma unroll
-          for (int t = 0; t < 4; t++) w[t] = (ae_elem)o[db * 16 + rg * 4 + t];
-          *(ae_elem4*)(optr + db * 32 + rg * 8 + hf * 4) = w;
+          *(ae_elem4*)(optr + db * 32 + rg * 8 + hf * 4) = out4(db * 16 + rg * 4);
         }
       if (hf == 0) {
 #pragma unroll
