@@ -259,7 +259,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 
 #if AE_BWD_ROLE == 0
   // row scales of the lane's q row: lse in log2 units (+inf for a row without a visible key: p = 0)
-  float lse2_r, delta_r;
+  float lse2_r, delta_r;              // (softmax: delta_r = -rowsum(do * o), the sign it is used with)
 #if AE_BWD_KIND == 2 && AE_BWD_NRS > 1
   float rs_more[AE_BWD_NRS - 1];      // the online function's further final row scales of the lane's row
 #endif
@@ -381,12 +381,42 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   for (int i = 0; i < AE_L1; i++) off1[i] = lane_off1(i, AE_BS, st1);
 #pragma unroll
   for (int i = 0; i < AE_L2; i++) off2[i] = lane_off2(i, AE_BS, st2);
-  // request item x (past the end: the last item again, so that every call issues AE_NLOADS loads) into `stage`
-  auto request_item = [&](int x, int stage) AE_LAMBDA {
+#if AE_MASK_MODE != 2
+  // Items are requested, and used, one after the other: what an item's position decides is carried along (a step of
+  // one tile, or on to the next head) instead of formed from the item's number, which took a division and six 64-bit
+  // products an item of one wave's issue slots.  rq_*: the next item to request; us_t, us_h: tile and head in use.
+  const int str_h = AE_BWD_ROLE == 0 ? hk : h * group;              // the first item's head in the streamed tensors
+#if AE_BWD_ROLE == 0
+  const int64_t st1h = p.k_stride_h, st2h = p.v_stride_h;
+  const char* rq_1 = (const char*)((const ae_elem*)p.k + (int64_t)b * p.k_stride_b + (int64_t)str_h * st1h + (int64_t)t_lo * AE_BS * st1);
+  const char* rq_2 = (const char*)((const ae_elem*)p.v + (int64_t)b * p.v_stride_b + (int64_t)str_h * st2h + (int64_t)t_lo * AE_BS * st2);
+#else
+  const int64_t st1h = p.q_stride_h, st2h = p.do_stride_h;
+  const char* rq_1 = (const char*)((const ae_elem*)p.q + (int64_t)b * p.q_stride_b + (int64_t)str_h * st1h + (int64_t)t_lo * AE_BS * st1);
+  const char* rq_2 = (const char*)((const ae_elem*)p.dout + (int64_t)b * p.do_stride_b + (int64_t)str_h * st2h + (int64_t)t_lo * AE_BS * st2);
+  const float* rq_d[AE_RSL];
+#pragma unroll
+  for (int i = 0; i < AE_RSL; i++) {
+    const int plane = (wave + AE_NWAVES * i) % AE_RS_PLANES;
+    rq_d[i] = p.delta + ((int64_t)plane * p.batch * p.heads_q + (int64_t)b * p.heads_q + str_h) * p.seqlen_q;
+  }
+#endif
+  const int64_t step1 = AE_BS * st1 * 2, step2 = AE_BS * st2 * 2;
+  const int64_t wrap1 = st1h * 2 - (n_t - 1) * step1, wrap2 = st2h * 2 - (n_t - 1) * step2;
+  int rq_x = 0, rq_t = t_lo, us_t = t_lo, us_h = AE_BWD_ROLE == 0 ? h : str_h;
+  (void)wrap1, (void)wrap2;
+#endif
+  // request item x (past the end: the last item again, so that every call issues AE_NLOADS loads) into the stage at byte `stage`
+  auto request_item = [&](int x, unsigned stage) AE_LAMBDA {
+    ae_lds_byte* t1 = lds + stage;
+    ae_lds_byte* t2 = t1 + AE_T1_BYTES;
+#if AE_MASK_MODE != 2
+    (void)x;
+    const int s0 = rq_t * AE_BS;
+    const char *x1 = rq_1, *x2 = rq_2;
+#else
     const int itc = x < n_items ? x : n_items - 1;
     const int s0 = item_tile(itc) * AE_BS;
-    ae_lds_byte* t1 = lds + stage * AE_STAGE_BYTES;
-    ae_lds_byte* t2 = t1 + AE_T1_BYTES;
 #if AE_BWD_ROLE == 0
     const char* x1 = (const char*)((const ae_elem*)p.k + (int64_t)b * p.k_stride_b + (int64_t)hk * p.k_stride_h + (int64_t)s0 * st1);
     const char* x2 = (const char*)((const ae_elem*)p.v + (int64_t)b * p.v_stride_b + (int64_t)hk * p.v_stride_h + (int64_t)s0 * st2);
@@ -394,6 +424,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
     const int hq = item_head(itc);
     const char* x1 = (const char*)((const ae_elem*)p.q + (int64_t)b * p.q_stride_b + (int64_t)hq * p.q_stride_h + (int64_t)s0 * st1);
     const char* x2 = (const char*)((const ae_elem*)p.dout + (int64_t)b * p.do_stride_b + (int64_t)hq * p.do_stride_h + (int64_t)s0 * st2);
+#endif
 #endif
     unsigned g1[8], g2[8];
     const bool ragged = s0 + AE_BS > n_str;           // wave-uniform
@@ -422,37 +453,71 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #pragma unroll
       for (int i = 0; i < AE_RSL; i++) {
         const int plane = (wave + AE_NWAVES * i) % AE_RS_PLANES;
+#if AE_MASK_MODE != 2
+        const float* src = rq_d[i] + row;
+#else
         const float* src = p.delta + ((int64_t)plane * p.batch * p.heads_q + (int64_t)b * p.heads_q + hq) * p.seqlen_q + row;
+#endif
         ae_load_lds4(src, t2 + AE_T2_BYTES + AE_RS_SLOT(plane) * AE_BS * 4);
       }
     }
 #endif
+#if AE_MASK_MODE != 2
+    const bool more = rq_x + 1 < n_items;
+#if AE_BWD_ROLE == 0
+    rq_1 += more ? step1 : 0;
+    rq_2 += more ? step2 : 0;
+    rq_t += more ? 1 : 0;
+#else
+    const bool next_head = rq_t + 1 == t_hi;
+    rq_1 += more ? (next_head ? wrap1 : step1) : 0;
+    rq_2 += more ? (next_head ? wrap2 : step2) : 0;
+#pragma unroll
+    for (int i = 0; i < AE_RSL; i++) rq_d[i] += more && next_head ? p.seqlen_q : 0;
+    rq_t = more ? (next_head ? t_lo : rq_t + 1) : rq_t;
+#endif
+    rq_x += more ? 1 : 0;
+#endif
   };
 
   // A operands out of a staged tile.  Row fragment: A[m = row 32*nb + lane%32][k = 16*ks + 8*hf + j].
-  auto row_frag1 = [&](const ae_lds_byte* t, int nb, int ks) AE_LAMBDA -> ae_elem8 {
-    const int r = nb * 32 + l32;
-    return *(const __attribute__((address_space(3))) ae_elem8*)(t + r * AE_STR1 + ae_bwd_chunk_pos<AE_CPR1>(r, 2 * ks + hf) * 16);
-  };
-  auto row_frag2 = [&](const ae_lds_byte* t, int nb, int ks) AE_LAMBDA -> ae_elem8 {
-    const int r = nb * 32 + l32;
-    return *(const __attribute__((address_space(3))) ae_elem8*)(t + r * AE_STR2 + ae_bwd_chunk_pos<AE_CPR2>(r, 2 * ks + hf) * 16);
-  };
   // Transposed fragment: A[m = column 32*db + ..][k = the 16 rows of k-step kk], in the row order in which
   // a lane's accumulator registers hold the rows (see the forward kernels' V^T fragment).
+  // The k-step and the column block only flip bits of the pair index, and a stage starts on a multiple of a row's
+  // bytes, so a fragment's address is (stage + lane part) ^ constant + immediate: one lane part for the row reads
+  // and one for the transposed reads, added to the stage once a tile.  (From the chunk positions as written above the
+  // compiler rebuilt the addresses with an add and a subtraction a read: 72 of the dq launch's 290 VALU
+  // instructions a tile.  With the items' positions carried along and the products started at -rowsum(do * o), a dq
+  // tile went from 468 to 357 instructions and a dk/dv tile from 658 to 558; backward of B2 H32 S4096 causal: D128
+  // 1064 -> 1047 us, where the socket's power cap takes most of it back, D64 forward + backward 885 -> 783 us.)
+  static_assert(AE_STAGE_BYTES % 256 == 0 && AE_T1_BYTES % 256 == 0, "the swizzle's bits of a stage's address are zero");
+  auto row_part = [&](int str, int cpr) AE_LAMBDA -> unsigned {
+    const int half = (hf ^ (l32 >> (cpr == 16 ? 3 : 2))) & 1;
+    return (unsigned)(l32 * str + ((l32 & (cpr / 2 - 1)) << 5) + (half << 4));
+  };
   const int t_row = 4 * hf + ((lane & 15) >> 2);
   const int t_g = l32 >> 4;
-  auto tr_frag = [&](const ae_lds_byte* t, int str, int cpr, int kk, int db) AE_LAMBDA -> ae_elem8 {
+  auto tr_part = [&](int str, int cpr) AE_LAMBDA -> unsigned {
+    const int half = (t_row >> (cpr == 16 ? 3 : 2)) & 1;
+    return (unsigned)(t_row * str + ((t_g ^ (t_row & (cpr / 2 - 1))) << 5) + (((lane & 3) * 8) ^ (half * 16)));
+  };
+  auto row_frag = [&](unsigned v, int str, int nb, int ks, int imm) AE_LAMBDA -> ae_elem8 {
+    return *(const __attribute__((address_space(3))) ae_elem8*)((const ae_lds_byte*)(v ^ (unsigned)(ks << 5)) + nb * 32 * str + imm);
+  };
+  // (8 rows further on the half flips where it is row bit 3, CPR 16; row bit 2, CPR 8, stays)
+  auto tr_frag = [&](unsigned v, int str, int cpr, int kk, int db, int imm) AE_LAMBDA -> ae_elem8 {
     const int rb0 = (kk >> 1) * 32 + (kk & 1) * 16;
-    const int r_lo = rb0 + t_row, r_hi = r_lo + 8;
-    const int sh = cpr == 16 ? 3 : 2;
-    const int pair = ((2 * db + t_g) ^ (t_row & (cpr / 2 - 1))) << 5;
-    const ae_lds_byte* a_lo = t + r_lo * str + pair + (((lane & 3) * 8) ^ (((r_lo >> sh) & 1) * 16));
-    const ae_lds_byte* a_hi = t + r_hi * str + pair + (((lane & 3) * 8) ^ (((r_hi >> sh) & 1) * 16));
+    const ae_lds_byte* a_lo = (const ae_lds_byte*)(v ^ (unsigned)(db << 6)) + rb0 * str + imm;
+    const ae_lds_byte* a_hi = (const ae_lds_byte*)(v ^ (unsigned)((db << 6) | (cpr == 16 ? 16 : 0))) + (rb0 + 8) * str + imm;
     ae_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)a_lo);
     ae_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)a_hi);
     return __builtin_bit_cast(ae_elem8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
+  const unsigned lds0 = (unsigned)(unsigned long)lds;
+  unsigned row1 = lds0 + row_part(AE_STR1, AE_CPR1), tr1 = lds0 + tr_part(AE_STR1, AE_CPR1);
+#if AE_D != AE_DV
+  unsigned row2 = lds0 + row_part(AE_STR2, AE_CPR2), tr2 = lds0 + tr_part(AE_STR2, AE_CPR2);
+#endif
 
   ae_f32x16 acc1[AE_NDB1];            // dQ^T (role 0) / dK^T (role 1): [d][resident row]
 #pragma unroll
@@ -517,7 +582,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
       for (int ks = 0; ks < AE_NKS2; ks++)
 #pragma unroll
         for (int j = 0; j < 8; j++) acc += (float)of[ks][j] * (float)rf2[ks][j];
-      delta_r = acc + __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, acc)));
+      delta_r = -(acc + __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, acc))));
       if (r_ok && hf == 0) {
         const int64_t ri = ((int64_t)b * p.heads_q + h) * p.seqlen_q + rrow;
         p.delta[ri] = delta_r;
@@ -531,23 +596,34 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
   }
   __syncthreads();       // every wave has its fragments: stages 1 and 2 go back to the ring
-  if (x0 < n_items) request_item(x1, 1);
+  if (x0 < n_items) request_item(x1, AE_STAGE_BYTES);
 #else
   if (x0 < n_items) {
     request_item(x0, 0);
-    if (AE_NSTAGE == 3) request_item(x1, 1);
+    if (AE_NSTAGE == 3) request_item(x1, AE_STAGE_BYTES);
     __builtin_amdgcn_s_waitcnt(AE_VMCNT((AE_NSTAGE - 2) * AE_NLOADS));   // the first item has landed
   }
   __syncthreads();
 #endif
 
-  for (int n = 0; x0 < n_items; n++) {
-    const int it = x0;
+  unsigned st_use = 0, st_req = (AE_NSTAGE - 1) * AE_STAGE_BYTES;      // stages of this iteration: multiplied, filled
+  while (x0 < n_items) {
     // into the stage everyone left at the last barrier
-    request_item(AE_NSTAGE == 3 ? x2 : x1, (n + AE_NSTAGE - 1) % AE_NSTAGE);
-    const ae_lds_byte* t1 = lds + (n % AE_NSTAGE) * AE_STAGE_BYTES;
-    const ae_lds_byte* t2 = t1 + AE_T1_BYTES;
-    const int s0 = item_tile(it) * AE_BS;
+    request_item(AE_NSTAGE == 3 ? x2 : x1, st_req);
+    unsigned v1 = row1 + st_use, w1 = tr1 + st_use;
+    asm("" : "+v"(v1), "+v"(w1));         // (values of their own: not rebuilt per read from their parts)
+#if AE_D != AE_DV
+    unsigned v2 = row2 + st_use, w2 = tr2 + st_use;
+    asm("" : "+v"(v2), "+v"(w2));
+#else
+    const unsigned v2 = v1, w2 = w1;
+#endif
+    (void)w2;
+#if AE_MASK_MODE != 2
+    const int s0 = us_t * AE_BS;
+#else
+    const int s0 = item_tile(x0) * AE_BS;
+#endif
 #if AE_BWD_PIN_ACC
 #pragma unroll
     for (int db = 0; db < AE_NDB1; db++) asm volatile("" : "+a"(acc1[db]));
@@ -561,8 +637,12 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
     // time; p and ds are packed as B operands: k-step kk holds the lane's elements 8*kk .. 8*kk+7
     ae_u32x4 pf[4], dsf[4];       // as packed pairs: two scores are converted by ONE packed conversion
 #if AE_BWD_ROLE == 1
-    const ae_lds_f32* rs_l = (const ae_lds_f32*)(t2 + AE_T2_BYTES);
-    const int hq = item_head(it);
+    const ae_lds_byte* rs_l = lds + (st_use + AE_T1_BYTES + AE_T2_BYTES + (unsigned)hf * 16);
+#if AE_MASK_MODE != 2
+    const int hq = us_h;
+#else
+    const int hq = item_head(x0);
+#endif
 #else
     const int hq = h;
 #endif
@@ -579,8 +659,25 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
     auto block = [&](int nb, auto masked) AE_LAMBDA {
       ae_f32x16 sacc, pacc;
+#if AE_BWD_ROLE == 1
+      // row values of the lane's 16 streamed rows, four consecutive ones a read: plane `slot` of the item
+      auto row_values = [&](int slot, int rg) AE_LAMBDA -> ae_f32x4 {
+        return *(const __attribute__((address_space(3))) ae_f32x4*)(rs_l + (slot * AE_BS + nb * 32 + 8 * rg) * 4);
+      };
+#endif
 #pragma unroll
-      for (int r = 0; r < 16; r++) sacc[r] = pacc[r] = 0.f;
+      for (int r = 0; r < 16; r++) {
+        sacc[r] = 0.f;
+        // softmax: the products start at -rowsum(do * o), so their sums are dp - rowsum(do * o) (one subtraction
+        // a score less, 32 of a tile's VALU instructions)
+#if AE_BWD_KIND == 0 && AE_BWD_ROLE == 0
+        pacc[r] = delta_r;
+#elif AE_BWD_KIND == 0
+        pacc[r] = row_values(1, r >> 2)[r & 3];
+#else
+        pacc[r] = 0.f;
+#endif
+      }
       // fragment stream of the block: S and dP k-steps alternate (two independent accumulation chains);
       // fragments are read AE_AHEAD MFMAs ahead of their use into a small ring, one fence per MFMA (left to
       // itself the scheduler either exposes the LDS latency or hoists every read and spills)
@@ -588,8 +685,9 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
       auto frag = [&](int f) AE_LAMBDA -> ae_elem8 {
         // f even and S still has k-steps: S; else dP (the dims may differ)
         const int pairs = AE_NKS1 < AE_NKS2 ? AE_NKS1 : AE_NKS2;
-        if (f < 2 * pairs) return (f & 1) ? row_frag2(t2, nb, f >> 1) : row_frag1(t1, nb, f >> 1);
-        return AE_NKS1 > AE_NKS2 ? row_frag1(t1, nb, f - pairs) : row_frag2(t2, nb, f - pairs);
+        const bool first = f < 2 * pairs ? !(f & 1) : AE_NKS1 > AE_NKS2;
+        const int ks = f < 2 * pairs ? f >> 1 : f - pairs;
+        return first ? row_frag(v1, AE_STR1, nb, ks, 0) : row_frag(v2, AE_STR2, nb, ks, AE_T1_BYTES);
       };
       ae_elem8 ring[AE_RING];
 #pragma unroll
@@ -612,19 +710,25 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
         const int srow = s0 + sl;
 #if AE_BWD_ROLE == 0
         const int qi = rrow, ki = srow;
-        const float l2 = lse2_r, dl = delta_r;
+        const float l2 = lse2_r;
+#if AE_BWD_KIND == 2
+        const float dl = delta_r;
+#endif
 #else
         const int qi = srow, ki = rrow;
-        const float l2 = rs_l[sl], dl = rs_l[AE_BS + sl];
+        const float l2 = row_values(0, r >> 2)[r & 3];
+#if AE_BWD_KIND == 2
+        const float dl = row_values(1, r >> 2)[r & 3];
+#endif
 #endif
 #if AE_BWD_KIND == 0
         float pv = ae_exp2(__builtin_fmaf(sacc[r], AE_SM_SCALE * AE_LOG2E, -l2));
-        const float dfac = pacc[r] - dl;
+        const float dfac = pacc[r];
 #elif AE_BWD_KIND == 1
         float pv, dfac;
         ae_bwd_pd(sacc[r], (float)b, (float)hq, (float)qi, (float)ki, cust, pv, dfac);
         dfac *= pacc[r];
-        (void)l2; (void)dl;
+        (void)l2;
 #else
         // traced OnlineFunc.forward / backward: l2 is the row's (first) final row scale as the forward wrote it
         float pv, dfac;
@@ -636,7 +740,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #if AE_BWD_ROLE == 0
           rsv[i] = rs_more[i - 1];
 #else
-          rsv[i] = rs_l[(1 + i) * AE_BS + sl];
+          rsv[i] = row_values(1 + i, r >> 2)[r & 3];
 #endif
 #endif
         ae_bwd_pd2(sacc[r], pacc[r], rsv, dl, b, hq, qi, ki, p, pv, dfac);
@@ -681,6 +785,15 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
       }
       __builtin_amdgcn_sched_barrier(0);
     };
+    // causal dq: the waves of a workgroup leave the diagonal at different tiles; a wave none of whose rows sees the
+    // tile leaves its SIMD to the other one (12 of the 32 (wave, tile) pairs on a 256-row tile's diagonal).  dk/dv has
+    // one wave a SIMD, all of which meet at the tile's barrier: skipping there frees nothing, and the branch makes the
+    // register allocator copy both accumulators every tile.
+    bool seen = true;
+#if AE_MASK_MODE == 1 && AE_BWD_ROLE == 0
+    seen = s0 <= r0w + 31;
+#endif
+    if (__builtin_expect(seen, 1)) {
     if (need_vis) {
       block(0, ae_bwd_true{});
       block(1, ae_bwd_true{});
@@ -696,7 +809,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
       constexpr int NF = 4 * NB_OUT;
       auto frag = [&](int f) AE_LAMBDA -> ae_elem8 {
         const int kk = f / NB_OUT, j = f % NB_OUT;
-        return j < AE_NDB1 ? tr_frag(t1, AE_STR1, AE_CPR1, kk, j) : tr_frag(t2, AE_STR2, AE_CPR2, kk, j - AE_NDB1);
+        return j < AE_NDB1 ? tr_frag(w1, AE_STR1, AE_CPR1, kk, j, 0) : tr_frag(w2, AE_STR2, AE_CPR2, kk, j - AE_NDB1, AE_T1_BYTES);
       };
       ae_elem8 ring[AE_RING];
 #pragma unroll
@@ -716,11 +829,18 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    }
     (void)pf;
 
     // the next item has landed (with three stages the one after it is still outstanding)
     __builtin_amdgcn_s_waitcnt(AE_VMCNT((AE_NSTAGE - 2) * AE_NLOADS));
     __syncthreads();
+#if AE_MASK_MODE != 2
+    us_t++;
+    if (AE_BWD_ROLE == 1 && us_t == t_hi) us_t = t_lo, us_h++;
+#endif
+    st_use = st_use == (AE_NSTAGE - 1) * AE_STAGE_BYTES ? 0 : st_use + AE_STAGE_BYTES;
+    st_req = st_req == (AE_NSTAGE - 1) * AE_STAGE_BYTES ? 0 : st_req + AE_STAGE_BYTES;
     x0 = x1, cls0 = cls1;
     x1 = x2, cls1 = cls2;
     x2 = next_item(x2 + 1, cls2);
@@ -827,7 +947,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 }
 
 #if AE_BWD_ROLE == 0
-// Work buffer fp32 [2,B,Hq,Sq]: plane 0 = rowsum(do * o), the `doosum` row scale of the reference's
+// Work buffer fp32 [2,B,Hq,Sq]: plane 0 = rowsum(do * o) (softmax: its negative), the `doosum` row scale of the reference's
 // backward (flashattn_bwd_preprocess, attn_tl.py:196-221); plane 1 = lse in log2 units, the form the two
 // other launches subtract inside exp2.  DV/8 lanes share a row, 16 bytes each.
 extern "C" __global__ __launch_bounds__(256)
@@ -858,7 +978,11 @@ void ae_bwd_delta_kernel(const ae_attn_bwd_params p) {
   if (row < n_rows && c == 0) {
     const int64_t ri = ((int64_t)b * p.heads_q + h) * p.seqlen_q + s;
     const float l = p.lse ? p.lse[ri] : 0.f;
+#if AE_BWD_KIND == 0
+    p.delta[ri] = -acc;             // (the sign in which the two launches start their dp products)
+#else
     p.delta[ri] = acc;
+#endif
 #if AE_BWD_KIND == 2
     // further planes: the online function's final row scales, as the forward wrote them
     p.delta[(int64_t)p.batch * p.heads_q * p.seqlen_q + ri] = l;
