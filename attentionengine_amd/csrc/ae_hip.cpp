@@ -647,7 +647,12 @@ int ae_prefill_bwd(ae_kernel* delta, ae_kernel* dkv, ae_kernel* dq, const ae_att
         return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: a stride of %lld elements is not a multiple of 8 (rows are moved 16 bytes at a time)",
                     (long long)st);
   }
-  // block_m / threads describe the dq launch (4 or 8 waves of 32 resident rows); dk/dv always runs 4 waves
+  // block_m / threads describe the dq launch (4 or 8 waves of 32 resident rows); dk/dv owns 128 rows, with 4 waves or 8
+  // in pairs, whose p and ds take 8 KiB of LDS a pair behind the tile ring
+  const uint32_t dkv_waves = cfg->table_rows ? (uint32_t)cfg->table_rows : 4u;
+  if (dkv_waves != 4 && (dkv_waves != 8 || cfg->head_dim <= 0 ||
+                         cfg->lds_bytes < 3 * (128 * (cfg->head_dim + cfg->head_dim_v) + 512) + 4 * 8192))
+    return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: dk/dv launch of %u waves with %d bytes of LDS", dkv_waves, cfg->lds_bytes);
   if ((cfg->block_m != 128 && cfg->block_m != 256) || cfg->block_n != 64 || cfg->threads != 2 * cfg->block_m || cfg->lds_bytes <= 0 ||
       cfg->lds_bytes > 160 * 1024 || cfg->head_dim_v <= 0 || cfg->head_dim_v % 8 != 0)
     return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: bad tile configuration (bm=%d bn=%d threads=%d lds=%d dv=%d)",
@@ -685,12 +690,13 @@ int ae_prefill_bwd(ae_kernel* delta, ae_kernel* dkv, ae_kernel* dq, const ae_att
     rc = ae_launch(dq, p, sizeof *p, grid, block, (uint32_t)cfg->lds_bytes, stream);
     if (rc) return rc;
     grid[0] = (uint32_t)g_dkv;
-    block[0] = 256;
+    block[0] = dkv_waves * 64;
     return ae_launch(dkv, p, sizeof *p, grid, block, (uint32_t)cfg->lds_bytes, stream);
   }
   rc = ae_launch(delta, p, sizeof *p, grid, block, 0, stream);
   if (rc) return rc;
   grid[0] = (uint32_t)g_dkv;
+  block[0] = dkv_waves * 64;
   rc = ae_launch(dkv, p, sizeof *p, grid, block, (uint32_t)cfg->lds_bytes, stream);
   if (rc) return rc;
   grid[0] = (uint32_t)g_dq;

@@ -33,7 +33,8 @@
 // straddles blocks of both kinds - looks every element up in the user's mask (ae_attn_bwd_params.block_mask).
 //
 // Waves per workgroup (AE_BWD_NWAVES, 32 resident rows each): dk/dv runs four, one per SIMD with the
-// whole register file (two accumulators). dq has one accumulator and fits 256 registers, so it runs
+// whole register file (two accumulators), or, softmax attention without a tile table, eight in pairs at head dims 128
+// (AE_BWD_PAIRS) and two workgroups a CU at head dims 64. dq has one accumulator and fits 256 registers, so it runs
 // eight, two per SIMD (AE_BWD_WAVES_PER_EU 2, AE_AHEAD 2): a wave spends about half of its time waiting
 // (LDS fragments, MFMA results, the p/ds arithmetic between two sets of MFMAs) and the second wave
 // fills it - 0.59 -> 0.44 ms for B2 H32 S4096 D128 causal.
@@ -68,7 +69,13 @@
 #endif
 #define AE_NWAVES AE_BWD_NWAVES
 #define AE_NT (AE_NWAVES * 64)
-#define AE_BR (AE_NWAVES * 32)     // resident rows per workgroup
+// 1 (dk/dv launch of softmax attention at head dim 128, eight waves): waves in pairs that share 32 kv rows, see
+// "two waves a pair" below.
+#ifndef AE_BWD_PAIRS
+#define AE_BWD_PAIRS 0
+#endif
+#define AE_NRW (AE_BWD_PAIRS ? AE_NWAVES / 2 : AE_NWAVES)      // waves that hold resident rows
+#define AE_BR (AE_NRW * 32)        // resident rows per workgroup
 #define AE_BS 64                   // streamed rows per tile
 #define AE_STR1 (AE_D * 2)         // LDS row pitch of the first streamed tensor (K or Q), bytes
 #define AE_STR2 (AE_DV * 2)        // ... of the second (V or dO)
@@ -143,11 +150,11 @@ AE_DEV int ae_bwd_chunk_pos(int r, int c) {
 // fit, else one after the other; the results use the ring after the last item.
 #define AE_R1B (32 * AE_STR1)      // bytes of a wave's resident rows, first tensor
 #define AE_R2B (32 * AE_STR2)
-#define AE_RES_ONEPASS (AE_NWAVES * (AE_R1B + AE_R2B) <= 2 * AE_STAGE_BYTES)
-#define AE_RES_TWOPASS (AE_NWAVES * (AE_R1B > AE_R2B ? AE_R1B : AE_R2B) <= 2 * AE_STAGE_BYTES)
+#define AE_RES_ONEPASS (AE_NRW * (AE_R1B + AE_R2B) <= 2 * AE_STAGE_BYTES)
+#define AE_RES_TWOPASS (AE_NRW * (AE_R1B > AE_R2B ? AE_R1B : AE_R2B) <= 2 * AE_STAGE_BYTES)
 #define AE_RES_VIA_LDS (AE_NSTAGE == 3 && (AE_RES_ONEPASS || AE_RES_TWOPASS))
 #define AE_OUT_BYTES (AE_R1B + (AE_BWD_ROLE == 1 ? AE_R2B : 0))   // a wave's results
-#define AE_OUT_VIA_LDS (AE_NWAVES * AE_OUT_BYTES <= AE_NSTAGE * AE_STAGE_BYTES)
+#define AE_OUT_VIA_LDS (AE_NRW * AE_OUT_BYTES <= AE_NSTAGE * AE_STAGE_BYTES)
 // 1 (softmax attention, set by the host with both launches): there is no ae_bwd_delta_kernel launch.  The dq
 // launch, which holds the dO rows anyway, fetches its O rows behind them, forms rowsum(dO * O) and writes both
 // planes of the work buffer; the dk/dv launch runs after it.  (The separate launch read O and dO once more:
@@ -155,6 +162,7 @@ AE_DEV int ae_bwd_chunk_pos(int r, int c) {
 #ifndef AE_BWD_FUSE_DELTA
 #define AE_BWD_FUSE_DELTA 0
 #endif
+static_assert(!AE_BWD_PAIRS || (AE_BWD_ROLE == 1 && AE_BWD_KIND == 0 && AE_NWAVES == 8 && AE_RES_VIA_LDS && AE_OUT_VIA_LDS), "pairs");
 static_assert(!AE_BWD_FUSE_DELTA || (AE_RES_VIA_LDS && AE_BWD_KIND == 0), "the fused row sums need the staged resident rows");
 
 // 32 rows of CPR 16-byte chunks, HBM -> dst, one burst; LDS chunk c' of row r holds global chunk c' ^ (r mod CPR).
@@ -199,6 +207,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rw = AE_BWD_PAIRS ? wave % AE_NRW : wave;      // the wave's 32 resident rows
   const int l32 = lane & 31;
   const int hf = lane >> 5;
   const int group = p.heads_q / p.heads_kv;
@@ -229,7 +238,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   const int h = bh % heads;            // role 0: q head; role 1: kv head
   const int b = bh / heads;
   const int r0 = rt * AE_BR;
-  const int rrow = r0 + wave * 32 + l32;            // this lane's resident row
+  const int rrow = r0 + rw * 32 + l32;            // this lane's resident row
   const bool r_ok = rrow < n_res;
   const int rrow_c = r_ok ? rrow : n_res - 1;
 
@@ -357,18 +366,16 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   // one burst behind a single write of M0 (wave-uniform base + per-lane offset + immediate, see
   // ae_load_lds16_burst_base: bases are passed 4 KiB low and offsets 4 KiB high).  Rows past the end of
   // the sequence re-read its last row (they are masked).
-  auto lane_off1 = [&](int i, int last_row, int64_t st) AE_LAMBDA -> unsigned {
+  auto lane_off1 = [&](int i, int64_t st) AE_LAMBDA -> unsigned {
     const int sidx = (wave * AE_L1 + i) * 64 + lane;
-    int r = sidx / AE_CPR1;
+    const int r = sidx / AE_CPR1;
     const int c = ae_bwd_chunk_pos<AE_CPR1>(r, sidx % AE_CPR1);
-    r = r < last_row ? r : last_row;
     return (unsigned)((r * (int)st + c * 8) * 2 + 4096 - (i - AE_L1 / 2) * 1024);
   };
-  auto lane_off2 = [&](int i, int last_row, int64_t st) AE_LAMBDA -> unsigned {
+  auto lane_off2 = [&](int i, int64_t st) AE_LAMBDA -> unsigned {
     const int sidx = (wave * AE_L2 + i) * 64 + lane;
-    int r = sidx / AE_CPR2;
+    const int r = sidx / AE_CPR2;
     const int c = ae_bwd_chunk_pos<AE_CPR2>(r, sidx % AE_CPR2);
-    r = r < last_row ? r : last_row;
     return (unsigned)((r * (int)st + c * 8) * 2 + 4096 - (i - AE_L2 / 2) * 1024);
   };
 #if AE_BWD_ROLE == 0
@@ -378,9 +385,9 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
   unsigned off1[AE_L1], off2[AE_L2];
 #pragma unroll
-  for (int i = 0; i < AE_L1; i++) off1[i] = lane_off1(i, AE_BS, st1);
+  for (int i = 0; i < AE_L1; i++) off1[i] = lane_off1(i, st1);
 #pragma unroll
-  for (int i = 0; i < AE_L2; i++) off2[i] = lane_off2(i, AE_BS, st2);
+  for (int i = 0; i < AE_L2; i++) off2[i] = lane_off2(i, st2);
 #if AE_MASK_MODE != 2
   // Items are requested, and used, one after the other: what an item's position decides is carried along (a step of
   // one tile, or on to the next head) instead of formed from the item's number, which took a division and six 64-bit
@@ -434,11 +441,17 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
       g2[i] = off2[i < AE_L2 ? i : 0];
     }
     if (__builtin_expect(ragged, 0)) {
-      asm volatile("" ::: "memory");                   // (keeps this one branch, out of the common path)
+      // the rows past the last one step back onto it (from a copy of the lane id that the compiler cannot trace: the
+      // lane's rows and chunks would otherwise be kept in registers, or scratch memory, all through the loop)
+      int le = lane;
+      asm volatile("" : "+v"(le) :: "memory");         // (keeps this one branch, out of the common path)
+      const int last = n_str - 1 - s0;
 #pragma unroll
       for (int i = 0; i < 8; i++) {
-        g1[i] = lane_off1(i < AE_L1 ? i : 0, n_str - 1 - s0, st1);
-        g2[i] = lane_off2(i < AE_L2 ? i : 0, n_str - 1 - s0, st2);
+        const int over1 = ((wave * AE_L1 + (i < AE_L1 ? i : 0)) * 64 + le) / AE_CPR1 - last;
+        const int over2 = ((wave * AE_L2 + (i < AE_L2 ? i : 0)) * 64 + le) / AE_CPR2 - last;
+        g1[i] -= (unsigned)((over1 > 0 ? over1 : 0) * (int)st1 * 2);
+        g2[i] -= (unsigned)((over2 > 0 ? over2 : 0) * (int)st2 * 2);
       }
     }
     ae_load_lds16_burst_base<AE_L1>(x1 - 4096, g1, t1 + (wave * AE_L1 + AE_L1 / 2) * 1024);
@@ -519,17 +532,18 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   unsigned row2 = lds0 + row_part(AE_STR2, AE_CPR2), tr2 = lds0 + tr_part(AE_STR2, AE_CPR2);
 #endif
 
+  // (pairs: the waves that hold them clear them, behind the other waves' loop)
+  auto clear = [](auto& acc) AE_LAMBDA {
+#pragma unroll
+    for (int db = 0; db < (int)(sizeof(acc) / sizeof(acc[0])); db++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[db][r] = 0.f;
+  };
   ae_f32x16 acc1[AE_NDB1];            // dQ^T (role 0) / dK^T (role 1): [d][resident row]
-#pragma unroll
-  for (int db = 0; db < AE_NDB1; db++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) acc1[db][r] = 0.f;
+  if (!AE_BWD_PAIRS) clear(acc1);
 #if AE_BWD_ROLE == 1
   ae_f32x16 acc2[AE_NDB2];            // dV^T
-#pragma unroll
-  for (int db = 0; db < AE_NDB2; db++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) acc2[db][r] = 0.f;
+  if (!AE_BWD_PAIRS) clear(acc2);
 #endif
 
   // the n-th visited item is multiplied out of stage n % NSTAGE while the next two are on their way
@@ -537,9 +551,11 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   int x0 = next_item(0, cls0), x1 = next_item(x0 + 1, cls1), x2 = next_item(x1 + 1, cls2);
 #if AE_RES_VIA_LDS
   if (x0 < n_items) request_item(x0, 0);
-  {
+  if (AE_BWD_PAIRS && wave >= AE_NRW) {
+    __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
+  } else {
     // the wave's 32 resident rows of both tensors travel together with the first item
-    const int rw0 = r0 + wave * 32;
+    const int rw0 = r0 + rw * 32;
     const int rw0c = rw0 < n_res ? rw0 : n_res - 1;
 #if AE_BWD_ROLE == 0
     const char* g1 = (const char*)((const ae_elem*)p.q + (int64_t)b * p.q_stride_b + (int64_t)rw0c * p.q_stride_s + (int64_t)h * p.q_stride_h);
@@ -551,14 +567,14 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
     const int rs1 = (int)p.k_stride_s, rs2 = (int)p.v_stride_s;
 #endif
 #if AE_RES_ONEPASS
-    ae_lds_byte* rs = lds + AE_STAGE_BYTES + wave * (AE_R1B + AE_R2B);
+    ae_lds_byte* rs = lds + AE_STAGE_BYTES + rw * (AE_R1B + AE_R2B);
     ae_bwd_rows_to_lds<AE_CPR1>(g1 - 4096, rs, lane, rw0 - rw0c, n_res - 1 - rw0c, rs1);
     ae_bwd_rows_to_lds<AE_CPR2>(g2 - 4096, rs + AE_R1B, lane, rw0 - rw0c, n_res - 1 - rw0c, rs2);
     __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
     ae_bwd_frags_from_lds<AE_NKS1, AE_CPR1>(rf1, rs, l32, hf);
     ae_bwd_frags_from_lds<AE_NKS2, AE_CPR2>(rf2, rs + AE_R1B, l32, hf);
 #else
-    ae_lds_byte* rs = lds + AE_STAGE_BYTES + wave * (AE_R1B > AE_R2B ? AE_R1B : AE_R2B);
+    ae_lds_byte* rs = lds + AE_STAGE_BYTES + rw * (AE_R1B > AE_R2B ? AE_R1B : AE_R2B);
     ae_bwd_rows_to_lds<AE_CPR1>(g1 - 4096, rs, lane, rw0 - rw0c, n_res - 1 - rw0c, rs1);
     __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
     ae_bwd_frags_from_lds<AE_NKS1, AE_CPR1>(rf1, rs, l32, hf);
@@ -596,7 +612,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
   }
   __syncthreads();       // every wave has its fragments: stages 1 and 2 go back to the ring
-  if (x0 < n_items) request_item(x1, AE_STAGE_BYTES);
+  if (!AE_BWD_PAIRS && x0 < n_items) request_item(x1, AE_STAGE_BYTES);
 #else
   if (x0 < n_items) {
     request_item(x0, 0);
@@ -606,24 +622,312 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   __syncthreads();
 #endif
 
+  // A tile in LDS, as the fragments of S and dP are read from it: lane parts (see row_part) of the two tensors, its first
+  // row, the byte of its row values that this half of the wave reads first, and its q head.
+  struct tile_at { unsigned v1, v2; int s0; unsigned rows; int hq; };
+  auto tile_in_use = [&](unsigned stage) AE_LAMBDA -> tile_at {
+    tile_at at;
+    at.v1 = row1 + stage;
+    asm("" : "+v"(at.v1));                // (a value of its own: not rebuilt per read from its parts)
+#if AE_D != AE_DV
+    at.v2 = row2 + stage;
+    asm("" : "+v"(at.v2));
+#else
+    at.v2 = at.v1;
+#endif
+    at.rows = stage + AE_T1_BYTES + AE_T2_BYTES + (unsigned)hf * 16;
+#if AE_MASK_MODE != 2
+    at.s0 = us_t * AE_BS, at.hq = us_h;
+#else
+    at.s0 = item_tile(x0) * AE_BS, at.hq = item_head(x0);
+#endif
+    return at;
+  };
+  // only tiles that touch the diagonal, the end of a sequence or an elementwise mask test visibility
+  const int r0w = r0 + rw * 32;
+  auto tests_visibility = [&](int s0) AE_LAMBDA {
+#if AE_MASK_MODE == 2
+    bool need_vis = cls0 != 2 || s0 + AE_BS > n_str || r0w + 32 > n_res;
+#else
+    bool need_vis = (AE_HAS_MASK_MOD != 0) || (AE_EXT_BLOCK_MASK != 0) || s0 + AE_BS > n_str || r0w + 32 > n_res;
+#endif
+#if AE_MASK_MODE == 1
+    need_vis = need_vis || (AE_BWD_ROLE == 0 ? s0 + AE_BS - 1 > r0w : s0 < r0w + 31);
+#endif
+    return need_vis;
+  };
+  // S = X1 R1^T and dP = X2 R2^T, [streamed row][resident row], one 32-row block of the tile at a time; p and ds are
+  // packed as B operands: k-step kk holds the lane's elements 8*kk .. 8*kk+7 (as packed pairs: two scores are converted
+  // by ONE packed conversion)
+  auto block = [&](int nb, auto masked, const tile_at& at, ae_u32x4* pf, ae_u32x4* dsf) AE_LAMBDA {
+    const int s0 = at.s0, hq = at.hq;
+    (void)hq;
+    ae_f32x16 sacc, pacc;
+#if AE_BWD_ROLE == 1
+    // row values of the lane's 16 streamed rows, four consecutive ones a read: plane `slot` of the item
+    auto row_values = [&](int slot, int rg) AE_LAMBDA -> ae_f32x4 {
+      return *(const __attribute__((address_space(3))) ae_f32x4*)(lds + at.rows + (slot * AE_BS + nb * 32 + 8 * rg) * 4);
+    };
+#endif
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      sacc[r] = 0.f;
+      // softmax: the products start at -rowsum(do * o), so their sums are dp - rowsum(do * o) (one subtraction
+      // a score less, 32 of a tile's VALU instructions)
+#if AE_BWD_KIND == 0 && AE_BWD_ROLE == 0
+      pacc[r] = delta_r;
+#elif AE_BWD_KIND == 0
+      pacc[r] = row_values(1, r >> 2)[r & 3];
+#else
+      pacc[r] = 0.f;
+#endif
+    }
+    // fragment stream of the block: S and dP k-steps alternate (two independent accumulation chains);
+    // fragments are read AE_AHEAD MFMAs ahead of their use into a small ring, one fence per MFMA (left to
+    // itself the scheduler either exposes the LDS latency or hoists every read and spills)
+    constexpr int NF = AE_NKS1 + AE_NKS2;
+    auto frag = [&](int f) AE_LAMBDA -> ae_elem8 {
+      // f even and S still has k-steps: S; else dP (the dims may differ)
+      const int pairs = AE_NKS1 < AE_NKS2 ? AE_NKS1 : AE_NKS2;
+      const bool first = f < 2 * pairs ? !(f & 1) : AE_NKS1 > AE_NKS2;
+      const int ks = f < 2 * pairs ? f >> 1 : f - pairs;
+      return first ? row_frag(at.v1, AE_STR1, nb, ks, 0) : row_frag(at.v2, AE_STR2, nb, ks, AE_T1_BYTES);
+    };
+    ae_elem8 ring[AE_RING];
+#pragma unroll
+    for (int f = 0; f < AE_AHEAD && f < NF; f++) ring[f] = frag(f);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+      if (f + AE_AHEAD < NF) ring[(f + AE_AHEAD) % AE_RING] = frag(f + AE_AHEAD);
+      const int pairs = AE_NKS1 < AE_NKS2 ? AE_NKS1 : AE_NKS2;
+      const bool is_s = f < 2 * pairs ? !(f & 1) : AE_NKS1 > AE_NKS2;
+      const int ks = f < 2 * pairs ? f >> 1 : f - pairs;
+      if (is_s) sacc = ae_mfma32(ring[f % AE_RING], rf1[ks], sacc);
+      else pacc = ae_mfma32(ring[f % AE_RING], rf2[ks], pacc);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // masked tiles: the streamed rows a lane's resident row sees by position - inside the sequence and, causal, on
+    // its side of the diagonal - are one interval, tested with one comparison a score
+    int vis_lo = 0;
+    unsigned vis_span = 0;
+    if (decltype(masked)::value) {
+      int lo = 0, hi = r_ok ? n_str : 0;
+#if AE_MASK_MODE == 1 && AE_BWD_ROLE == 0
+      hi = hi < rrow + 1 ? hi : rrow + 1;
+#elif AE_MASK_MODE == 1
+      lo = rrow;
+#endif
+      vis_lo = lo - s0 - 4 * hf;
+      vis_span = hi > lo ? (unsigned)(hi - lo) : 0u;
+    }
+    (void)vis_lo, (void)vis_span;
+    float pvs[16], dss[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int sl = nb * 32 + 8 * (r >> 2) + 4 * hf + (r & 3);     // streamed row inside the tile
+      const int srow = s0 + sl;
+#if AE_BWD_ROLE == 0
+      const int qi = rrow, ki = srow;
+      const float l2 = lse2_r;
+#if AE_BWD_KIND == 2
+      const float dl = delta_r;
+#endif
+#else
+      const int qi = srow, ki = rrow;
+      const float l2 = row_values(0, r >> 2)[r & 3];
+#if AE_BWD_KIND == 2
+      const float dl = row_values(1, r >> 2)[r & 3];
+#endif
+#endif
+#if AE_BWD_KIND == 0
+      float pv = ae_exp2(__builtin_fmaf(sacc[r], AE_SM_SCALE * AE_LOG2E, -l2));
+      const float dfac = pacc[r];
+#elif AE_BWD_KIND == 1
+      float pv, dfac;
+      ae_bwd_pd(sacc[r], (float)b, (float)hq, (float)qi, (float)ki, cust, pv, dfac);
+      dfac *= pacc[r];
+      (void)l2;
+#else
+      // traced OnlineFunc.forward / backward: l2 is the row's (first) final row scale as the forward wrote it
+      float pv, dfac;
+      float rsv[AE_BWD_NRS];
+      rsv[0] = l2;
+#if AE_BWD_NRS > 1
+#pragma unroll
+      for (int i = 1; i < AE_BWD_NRS; i++)
+#if AE_BWD_ROLE == 0
+        rsv[i] = rs_more[i - 1];
+#else
+        rsv[i] = row_values(1 + i, r >> 2)[r & 3];
+#endif
+#endif
+      ae_bwd_pd2(sacc[r], pacc[r], rsv, dl, b, hq, qi, ki, p, pv, dfac);
+#endif
+      bool vis = true;
+      if (decltype(masked)::value) {
+        vis = (unsigned)(nb * 32 + 8 * (r >> 2) + (r & 3) - vis_lo) < vis_span;
+#if AE_HAS_MASK_MOD
+        vis = vis && ae_mask_mod(b, hq, qi, ki);
+#endif
+#if AE_EXT_BLOCK_MASK
+        {
+          // the user's block of this (q, kv) position (positions past the end are invisible anyway: clamped)
+          int mr = qi / p.mask_block_m, mc = ki / p.mask_block_n;
+          mr = mr < p.mask_nq ? mr : p.mask_nq - 1;
+          mc = mc < p.mask_nkv ? mc : p.mask_nkv - 1;
+          const int64_t mbh = (int64_t)(p.mask_b == 1 ? 0 : b) * p.mask_h + (p.mask_h == 1 ? 0 : hq);
+          vis = vis && p.block_mask[(mbh * p.mask_nq + mr) * p.mask_nkv + mc] != 0;
+        }
+#endif
+        pv = vis ? pv : 0.f;
+      }
+      (void)qi; (void)ki;
+#if AE_BWD_KIND == 0
+      const float dsv = pv * dfac;                           // score_mod's derivative (the scale) is applied to the sums
+#else
+      const float dsv = vis ? dfac : 0.f;                    // an invisible score contributes nothing and moves nothing
+#endif
+      pvs[r] = pv;
+      dss[r] = dsv;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r += 2) {
+      typedef float ae_f32x2 __attribute__((ext_vector_type(2)));
+      const int e = nb * 16 + r;
+      const ae_f32x2 p2 = {pvs[r], pvs[r + 1]}, d2 = {dss[r], dss[r + 1]};
+      pf[e >> 3][(e & 7) >> 1] = __builtin_bit_cast(unsigned, __builtin_convertvector(p2, ae_elem2));
+      dsf[e >> 3][(e & 7) >> 1] = __builtin_bit_cast(unsigned, __builtin_convertvector(d2, ae_elem2));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // OUT^T[d][resident] += X^T[d][streamed] ds[streamed][resident] of the tile in the stage at byte `stage`; half_way runs
+  // when half of it is done
+  auto add_products = [&](unsigned stage, const ae_u32x4* pf, const ae_u32x4* dsf, auto half_way) AE_LAMBDA {
+    unsigned w1 = tr1 + stage;
+    asm("" : "+v"(w1));
+#if AE_D != AE_DV
+    unsigned w2 = tr2 + stage;
+    asm("" : "+v"(w2));
+#else
+    const unsigned w2 = w1;
+#endif
+    (void)w2;
+    (void)pf;
+    // fragment f = (k-step kk, output block j of dQ/dK, then of dV), read ahead through the same kind of ring
+    constexpr int NB_OUT = AE_NDB1 + (AE_BWD_ROLE == 1 ? AE_NDB2 : 0);
+    constexpr int NF = 4 * NB_OUT;
+    auto frag = [&](int f) AE_LAMBDA -> ae_elem8 {
+      const int kk = f / NB_OUT, j = f % NB_OUT;
+      return j < AE_NDB1 ? tr_frag(w1, AE_STR1, AE_CPR1, kk, j, 0) : tr_frag(w2, AE_STR2, AE_CPR2, kk, j - AE_NDB1, AE_T1_BYTES);
+    };
+    ae_elem8 ring[AE_RING];
+#pragma unroll
+    for (int f = 0; f < AE_AHEAD && f < NF; f++) ring[f] = frag(f);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+      if (f + AE_AHEAD < NF) ring[(f + AE_AHEAD) % AE_RING] = frag(f + AE_AHEAD);
+      const int kk = f / NB_OUT, j = f % NB_OUT;
+      if (f == NF / 2) half_way();
+      if (j < AE_NDB1) {
+        acc1[j] = ae_mfma32(ring[f % AE_RING], __builtin_bit_cast(ae_elem8, dsf[kk]), acc1[j]);
+      } else {
+#if AE_BWD_ROLE == 1
+        acc2[j - AE_NDB1] = ae_mfma32(ring[f % AE_RING], __builtin_bit_cast(ae_elem8, pf[kk]), acc2[j - AE_NDB1]);
+#endif
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+#if AE_BWD_PAIRS
+  // Two waves a pair.  dk and dv of 32 rows are 128 accumulators, the resident operands 64 registers, the scores 64: one
+  // wave a SIMD with the whole file, which issues its LDS reads, its p / ds arithmetic and its MFMAs one after the other
+  // and moves every score out of the accumulator file.  Here wave w (w < 4) holds K and V of the pair's rows and forms p
+  // and ds of tile n, and wave w + 4, on the same SIMD, holds dk and dv and adds tile n - 1's products: 32 MFMAs a tile
+  // each, 256 registers suffice, and one's arithmetic runs under the other's MFMAs.  p and ds go over through 8 KiB of
+  // LDS a pair, in the operand layout.  A tile's two barriers: A, half-way, the second wave has p and ds of n - 1 in its
+  // registers (the first may write those of n); B, at the end, tile n + 1 has landed and p and ds of n are written.
+  // Tile n + 1 goes into the stage of tile n - 2, which the second wave left at the last B.
+  // Against one wave a SIMD: causal backward of B2 H32 S4096 fp16 1047 -> 1005 us, B4 H32 S2048 bf16 594 -> 558, B2 H16
+  // S1000 88.5 -> 77.
+  ae_lds_byte* ho = lds + 3 * AE_STAGE_BYTES + rw * 8192 + lane * 16;      // fragment i (p: 0..3, ds: 4..7) at + 1024 * i
+  typedef __attribute__((address_space(3))) ae_u32x4 ae_lds_u32x4;
+  unsigned st_use = 0, st_req = AE_STAGE_BYTES;
+  if (wave < AE_NRW) {
+    while (x0 < n_items) {
+      request_item(x1, st_req);
+      const tile_at at = tile_in_use(st_use);
+      const bool need_vis = tests_visibility(at.s0);
+      ae_u32x4 pf[4], dsf[4];
+      auto hand_over = [&](int nb) AE_LAMBDA {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          *(ae_lds_u32x4*)(ho + (2 * nb + i) * 1024) = pf[2 * nb + i];
+          *(ae_lds_u32x4*)(ho + (4 + 2 * nb + i) * 1024) = dsf[2 * nb + i];
+        }
+      };
+      if (need_vis) block(0, ae_bwd_true{}, at, pf, dsf);
+      else block(0, ae_bwd_false{}, at, pf, dsf);
+      __syncthreads();                                         // A
+      hand_over(0);
+      if (need_vis) block(1, ae_bwd_true{}, at, pf, dsf);
+      else block(1, ae_bwd_false{}, at, pf, dsf);
+      hand_over(1);
+      __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
+      __syncthreads();                                         // B
+#if AE_MASK_MODE != 2
+      us_t++;
+      if (us_t == t_hi) us_t = t_lo, us_h++;
+#endif
+      st_use = st_use == 2 * AE_STAGE_BYTES ? 0 : st_use + AE_STAGE_BYTES;
+      st_req = st_req == 2 * AE_STAGE_BYTES ? 0 : st_req + AE_STAGE_BYTES;
+      x0 = x1, cls0 = cls1;
+      x1 = next_item(x1 + 1, cls1);
+    }
+    __syncthreads();                                           // the ring goes to the results
+    return;
+  }
+  clear(acc1);
+  clear(acc2);
+  // the tile's products with p and ds as they were handed over
+  auto add_handed_over = [&](unsigned stage, auto all_read) AE_LAMBDA {
+    ae_u32x4 pf[4], dsf[4];
+    auto take = [&](int i0) AE_LAMBDA {
+#pragma unroll
+      for (int i = i0; i < i0 + 2; i++) {
+        pf[i] = *(const ae_lds_u32x4*)(ho + i * 1024);
+        dsf[i] = *(const ae_lds_u32x4*)(ho + (4 + i) * 1024);
+      }
+    };
+    take(0);
+    add_products(stage, pf, dsf, [&]() AE_LAMBDA {
+      take(2);
+      all_read();
+    });
+  };
+  unsigned st_prev = 2 * AE_STAGE_BYTES;
+  bool first = true;
+  while (x0 < n_items) {
+    request_item(x1, st_req);
+    if (first) __syncthreads();                                // A (nothing is handed over yet)
+    else add_handed_over(st_prev, [&]() AE_LAMBDA { __syncthreads(); });
+    first = false;
+    __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
+    __syncthreads();                                           // B
+    st_prev = st_prev == 2 * AE_STAGE_BYTES ? 0 : st_prev + AE_STAGE_BYTES;
+    st_req = st_req == 2 * AE_STAGE_BYTES ? 0 : st_req + AE_STAGE_BYTES;
+    x0 = x1;
+    x1 = next_item(x1 + 1, cls1);
+  }
+  if (!first) add_handed_over(st_prev, []() AE_LAMBDA {});
+  (void)st_use;
+#else
   unsigned st_use = 0, st_req = (AE_NSTAGE - 1) * AE_STAGE_BYTES;      // stages of this iteration: multiplied, filled
   while (x0 < n_items) {
     // into the stage everyone left at the last barrier
     request_item(AE_NSTAGE == 3 ? x2 : x1, st_req);
-    unsigned v1 = row1 + st_use, w1 = tr1 + st_use;
-    asm("" : "+v"(v1), "+v"(w1));         // (values of their own: not rebuilt per read from their parts)
-#if AE_D != AE_DV
-    unsigned v2 = row2 + st_use, w2 = tr2 + st_use;
-    asm("" : "+v"(v2), "+v"(w2));
-#else
-    const unsigned v2 = v1, w2 = w1;
-#endif
-    (void)w2;
-#if AE_MASK_MODE != 2
-    const int s0 = us_t * AE_BS;
-#else
-    const int s0 = item_tile(x0) * AE_BS;
-#endif
+    const tile_at at = tile_in_use(st_use);
 #if AE_BWD_PIN_ACC
 #pragma unroll
     for (int db = 0; db < AE_NDB1; db++) asm volatile("" : "+a"(acc1[db]));
@@ -633,204 +937,26 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
 #endif
 
-    // S = X1 R1^T and dP = X2 R2^T, [streamed row][resident row], one 32-row block of the tile at a
-    // time; p and ds are packed as B operands: k-step kk holds the lane's elements 8*kk .. 8*kk+7
-    ae_u32x4 pf[4], dsf[4];       // as packed pairs: two scores are converted by ONE packed conversion
-#if AE_BWD_ROLE == 1
-    const ae_lds_byte* rs_l = lds + (st_use + AE_T1_BYTES + AE_T2_BYTES + (unsigned)hf * 16);
-#if AE_MASK_MODE != 2
-    const int hq = us_h;
-#else
-    const int hq = item_head(x0);
-#endif
-#else
-    const int hq = h;
-#endif
-    (void)hq;
-    // only tiles that touch the diagonal, the end of a sequence or an elementwise mask test visibility
-    const int r0w = r0 + wave * 32;
-#if AE_MASK_MODE == 2
-    bool need_vis = cls0 != 2 || s0 + AE_BS > n_str || r0w + 32 > n_res;
-#else
-    bool need_vis = (AE_HAS_MASK_MOD != 0) || (AE_EXT_BLOCK_MASK != 0) || s0 + AE_BS > n_str || r0w + 32 > n_res;
-#endif
-#if AE_MASK_MODE == 1
-    need_vis = need_vis || (AE_BWD_ROLE == 0 ? s0 + AE_BS - 1 > r0w : s0 < r0w + 31);
-#endif
-    auto block = [&](int nb, auto masked) AE_LAMBDA {
-      ae_f32x16 sacc, pacc;
-#if AE_BWD_ROLE == 1
-      // row values of the lane's 16 streamed rows, four consecutive ones a read: plane `slot` of the item
-      auto row_values = [&](int slot, int rg) AE_LAMBDA -> ae_f32x4 {
-        return *(const __attribute__((address_space(3))) ae_f32x4*)(rs_l + (slot * AE_BS + nb * 32 + 8 * rg) * 4);
-      };
-#endif
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        sacc[r] = 0.f;
-        // softmax: the products start at -rowsum(do * o), so their sums are dp - rowsum(do * o) (one subtraction
-        // a score less, 32 of a tile's VALU instructions)
-#if AE_BWD_KIND == 0 && AE_BWD_ROLE == 0
-        pacc[r] = delta_r;
-#elif AE_BWD_KIND == 0
-        pacc[r] = row_values(1, r >> 2)[r & 3];
-#else
-        pacc[r] = 0.f;
-#endif
-      }
-      // fragment stream of the block: S and dP k-steps alternate (two independent accumulation chains);
-      // fragments are read AE_AHEAD MFMAs ahead of their use into a small ring, one fence per MFMA (left to
-      // itself the scheduler either exposes the LDS latency or hoists every read and spills)
-      constexpr int NF = AE_NKS1 + AE_NKS2;
-      auto frag = [&](int f) AE_LAMBDA -> ae_elem8 {
-        // f even and S still has k-steps: S; else dP (the dims may differ)
-        const int pairs = AE_NKS1 < AE_NKS2 ? AE_NKS1 : AE_NKS2;
-        const bool first = f < 2 * pairs ? !(f & 1) : AE_NKS1 > AE_NKS2;
-        const int ks = f < 2 * pairs ? f >> 1 : f - pairs;
-        return first ? row_frag(v1, AE_STR1, nb, ks, 0) : row_frag(v2, AE_STR2, nb, ks, AE_T1_BYTES);
-      };
-      ae_elem8 ring[AE_RING];
-#pragma unroll
-      for (int f = 0; f < AE_AHEAD && f < NF; f++) ring[f] = frag(f);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int f = 0; f < NF; f++) {
-        if (f + AE_AHEAD < NF) ring[(f + AE_AHEAD) % AE_RING] = frag(f + AE_AHEAD);
-        const int pairs = AE_NKS1 < AE_NKS2 ? AE_NKS1 : AE_NKS2;
-        const bool is_s = f < 2 * pairs ? !(f & 1) : AE_NKS1 > AE_NKS2;
-        const int ks = f < 2 * pairs ? f >> 1 : f - pairs;
-        if (is_s) sacc = ae_mfma32(ring[f % AE_RING], rf1[ks], sacc);
-        else pacc = ae_mfma32(ring[f % AE_RING], rf2[ks], pacc);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      float pvs[16], dss[16];
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int sl = nb * 32 + 8 * (r >> 2) + 4 * hf + (r & 3);     // streamed row inside the tile
-        const int srow = s0 + sl;
-#if AE_BWD_ROLE == 0
-        const int qi = rrow, ki = srow;
-        const float l2 = lse2_r;
-#if AE_BWD_KIND == 2
-        const float dl = delta_r;
-#endif
-#else
-        const int qi = srow, ki = rrow;
-        const float l2 = row_values(0, r >> 2)[r & 3];
-#if AE_BWD_KIND == 2
-        const float dl = row_values(1, r >> 2)[r & 3];
-#endif
-#endif
-#if AE_BWD_KIND == 0
-        float pv = ae_exp2(__builtin_fmaf(sacc[r], AE_SM_SCALE * AE_LOG2E, -l2));
-        const float dfac = pacc[r];
-#elif AE_BWD_KIND == 1
-        float pv, dfac;
-        ae_bwd_pd(sacc[r], (float)b, (float)hq, (float)qi, (float)ki, cust, pv, dfac);
-        dfac *= pacc[r];
-        (void)l2;
-#else
-        // traced OnlineFunc.forward / backward: l2 is the row's (first) final row scale as the forward wrote it
-        float pv, dfac;
-        float rsv[AE_BWD_NRS];
-        rsv[0] = l2;
-#if AE_BWD_NRS > 1
-#pragma unroll
-        for (int i = 1; i < AE_BWD_NRS; i++)
-#if AE_BWD_ROLE == 0
-          rsv[i] = rs_more[i - 1];
-#else
-          rsv[i] = row_values(1 + i, r >> 2)[r & 3];
-#endif
-#endif
-        ae_bwd_pd2(sacc[r], pacc[r], rsv, dl, b, hq, qi, ki, p, pv, dfac);
-#endif
-        bool vis = true;
-        if (decltype(masked)::value) {
-          vis = r_ok && srow < n_str;
-#if AE_MASK_MODE == 1
-          vis = vis && qi >= ki;
-#endif
-#if AE_HAS_MASK_MOD
-          vis = vis && ae_mask_mod(b, hq, qi, ki);
-#endif
-#if AE_EXT_BLOCK_MASK
-          {
-            // the user's block of this (q, kv) position (positions past the end are invisible anyway: clamped)
-            int mr = qi / p.mask_block_m, mc = ki / p.mask_block_n;
-            mr = mr < p.mask_nq ? mr : p.mask_nq - 1;
-            mc = mc < p.mask_nkv ? mc : p.mask_nkv - 1;
-            const int64_t mbh = (int64_t)(p.mask_b == 1 ? 0 : b) * p.mask_h + (p.mask_h == 1 ? 0 : hq);
-            vis = vis && p.block_mask[(mbh * p.mask_nq + mr) * p.mask_nkv + mc] != 0;
-          }
-#endif
-          pv = vis ? pv : 0.f;
-        }
-        (void)qi; (void)ki;
-#if AE_BWD_KIND == 0
-        const float dsv = pv * dfac;                           // score_mod's derivative (the scale) is applied to the sums
-#else
-        const float dsv = vis ? dfac : 0.f;                    // an invisible score contributes nothing and moves nothing
-#endif
-        pvs[r] = pv;
-        dss[r] = dsv;
-      }
-#pragma unroll
-      for (int r = 0; r < 16; r += 2) {
-        typedef float ae_f32x2 __attribute__((ext_vector_type(2)));
-        const int e = nb * 16 + r;
-        const ae_f32x2 p2 = {pvs[r], pvs[r + 1]}, d2 = {dss[r], dss[r + 1]};
-        pf[e >> 3][(e & 7) >> 1] = __builtin_bit_cast(unsigned, __builtin_convertvector(p2, ae_elem2));
-        dsf[e >> 3][(e & 7) >> 1] = __builtin_bit_cast(unsigned, __builtin_convertvector(d2, ae_elem2));
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    };
+    ae_u32x4 pf[4], dsf[4];
     // causal dq: the waves of a workgroup leave the diagonal at different tiles; a wave none of whose rows sees the
     // tile leaves its SIMD to the other one (12 of the 32 (wave, tile) pairs on a 256-row tile's diagonal).  dk/dv has
     // one wave a SIMD, all of which meet at the tile's barrier: skipping there frees nothing, and the branch makes the
     // register allocator copy both accumulators every tile.
     bool seen = true;
 #if AE_MASK_MODE == 1 && AE_BWD_ROLE == 0
-    seen = s0 <= r0w + 31;
+    seen = at.s0 <= r0w + 31;
 #endif
     if (__builtin_expect(seen, 1)) {
-    if (need_vis) {
-      block(0, ae_bwd_true{});
-      block(1, ae_bwd_true{});
+    if (tests_visibility(at.s0)) {
+      block(0, ae_bwd_true{}, at, pf, dsf);
+      block(1, ae_bwd_true{}, at, pf, dsf);
     } else {
-      block(0, ae_bwd_false{});
-      block(1, ae_bwd_false{});
+      block(0, ae_bwd_false{}, at, pf, dsf);
+      block(1, ae_bwd_false{}, at, pf, dsf);
     }
 
-    // OUT^T[d][resident] += X^T[d][streamed] ds[streamed][resident]: fragment f = (k-step kk, output block
-    // j of dQ/dK, then of dV), read ahead through the same kind of ring
-    {
-      constexpr int NB_OUT = AE_NDB1 + (AE_BWD_ROLE == 1 ? AE_NDB2 : 0);
-      constexpr int NF = 4 * NB_OUT;
-      auto frag = [&](int f) AE_LAMBDA -> ae_elem8 {
-        const int kk = f / NB_OUT, j = f % NB_OUT;
-        return j < AE_NDB1 ? tr_frag(w1, AE_STR1, AE_CPR1, kk, j, 0) : tr_frag(w2, AE_STR2, AE_CPR2, kk, j - AE_NDB1, AE_T1_BYTES);
-      };
-      ae_elem8 ring[AE_RING];
-#pragma unroll
-      for (int f = 0; f < AE_AHEAD && f < NF; f++) ring[f] = frag(f);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int f = 0; f < NF; f++) {
-        if (f + AE_AHEAD < NF) ring[(f + AE_AHEAD) % AE_RING] = frag(f + AE_AHEAD);
-        const int kk = f / NB_OUT, j = f % NB_OUT;
-        if (j < AE_NDB1) {
-          acc1[j] = ae_mfma32(ring[f % AE_RING], __builtin_bit_cast(ae_elem8, dsf[kk]), acc1[j]);
-        } else {
-#if AE_BWD_ROLE == 1
-          acc2[j - AE_NDB1] = ae_mfma32(ring[f % AE_RING], __builtin_bit_cast(ae_elem8, pf[kk]), acc2[j - AE_NDB1]);
-#endif
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
+    add_products(st_use, pf, dsf, []() AE_LAMBDA {});
     }
-    }
-    (void)pf;
 
     // the next item has landed (with three stages the one after it is still outstanding)
     __builtin_amdgcn_s_waitcnt(AE_VMCNT((AE_NSTAGE - 2) * AE_NLOADS));
@@ -845,6 +971,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
     x1 = x2, cls1 = cls2;
     x2 = next_item(x2 + 1, cls2);
   }
+#endif
   __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));             // nothing may land in LDS after the workgroup has gone
 
   // ---- results: lane owns its resident row, columns 32*db + 8*(r/4) + 4*hf + r%4 ------------------
@@ -854,7 +981,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
     // (addresses from a copy of the lane id that the compiler cannot trace back to the prologue's)
     int le = lane;
     asm volatile("" : "+v"(le));
-    ae_lds_byte* os1 = lds + wave * AE_OUT_BYTES;
+    ae_lds_byte* os1 = lds + rw * AE_OUT_BYTES;
     {
       ae_lds_byte* orow = os1 + (le & 31) * AE_STR1 + (le >> 5) * 8;
       const int osw = le & (AE_CPR1 - 1);
@@ -885,7 +1012,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
     // (the rows were written by other lanes of this wave: LDS instructions of a wave complete in order)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    const int rw0 = r0 + wave * 32;
+    const int rw0 = r0 + rw * 32;
 #if AE_BWD_ROLE == 0
     ae_elem* o1 = (ae_elem*)p.dq + (int64_t)b * p.dq_stride_b + (int64_t)h * p.dq_stride_h;
     const int64_t os1s = p.dq_stride_s;

@@ -138,7 +138,9 @@ typedef struct ae_tile_cfg {
                           AE_MERGE_LAST 1 (the workgroup that finishes last merges: no combine kernel, work
                           buffers with arrival counters, see ae_decode_fwd); else 0                        */
   int32_t table_rows;  /* mask_mode 2: block-mask rows one q tile may span, the AE_TT_ROWS the kernel was
-                          compiled with (1, 2, 4 or 8); 0 stands for the kernels' default of 8             */
+                          compiled with (1, 2, 4 or 8); 0 stands for the kernels' default of 8.
+                          ae_prefill_bwd: waves of the dk/dv launch, 4 (also 0) or, kernels compiled with
+                          AE_BWD_PAIRS 1, 8                                                                */
 } ae_tile_cfg;
 
 /*

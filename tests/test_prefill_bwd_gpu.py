@@ -91,6 +91,26 @@ def test_softmax_backward(cuda_device, B, H, Hkv, S, D, dtype, causal):
     _run(B, H, Hkv, S, S, D, D, dtype, C.causal_mask if causal else None, causal)
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,Hkv,Sq,Skv", [
+    (1, 1, 1, 1, 1),           # one item, one row
+    (1, 2, 1, 64, 64),         # one tile per head of the group: every step is on to the next head
+    (1, 6, 2, 65, 65),         # ... a last tile of one row
+    (2, 3, 3, 129, 129),       # three items: as many as stages; a second kv tile of one row
+    (1, 4, 1, 193, 300),       # kv rows past the last query
+    (1, 9, 9, 257, 100),       # more heads than XCDs, queries past the last key
+])
+def test_softmax_backward_item_walk(cuda_device, B, H, Hkv, Sq, Skv, D, causal):
+    """Ends of the walk over a kv tile's streamed items (few items, one tile a head, a ragged last tile, rows without a
+    partner), which the dk/dv launch's two halves of a wave pair go through one tile apart.  _check's tolerance: p, ds
+    and the results are rounded to the input type as at every other shape."""
+    if causal and Sq != Skv:
+        pytest.skip("the oracle's causal mask is square")
+    print(f"case bwd walk B{B} H{H} Hkv{Hkv} Sq{Sq} Skv{Skv} D{D} causal={causal}", flush=True)
+    _run(B, H, Hkv, Sq, Skv, D, D, torch.float16, C.causal_mask if causal else None, causal)
+
+
 def test_softmax_backward_headline_shape(cuda_device):
     """The shape bench.py times the backward on (B2 H32 S4096 D128 fp16, causal): every gradient finite,
     and dq, dk, dv of two (batch, head) slices -- which depend on that slice's tensors only -- against the
