@@ -924,7 +924,30 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   (void)st_use;
 #else
   unsigned st_use = 0, st_req = (AE_NSTAGE - 1) * AE_STAGE_BYTES;      // stages of this iteration: multiplied, filled
-  while (x0 < n_items) {
+  auto next_step = [&]() AE_LAMBDA {
+    // the next item has landed (with three stages the one after it is still outstanding)
+    __builtin_amdgcn_s_waitcnt(AE_VMCNT((AE_NSTAGE - 2) * AE_NLOADS));
+    __syncthreads();
+#if AE_MASK_MODE != 2
+    us_t++;
+    if (AE_BWD_ROLE == 1 && us_t == t_hi) us_t = t_lo, us_h++;
+#endif
+    st_use = st_use == (AE_NSTAGE - 1) * AE_STAGE_BYTES ? 0 : st_use + AE_STAGE_BYTES;
+    st_req = st_req == (AE_NSTAGE - 1) * AE_STAGE_BYTES ? 0 : st_req + AE_STAGE_BYTES;
+    x0 = x1, cls0 = cls1;
+    x1 = x2, cls1 = cls2;
+    x2 = next_item(x2 + 1, cls2);
+  };
+  // causal dq: the waves of a workgroup leave the diagonal at different tiles; one none of whose rows sees a tile sees
+  // none after it either, and only keeps up requests and barriers, leaving its SIMD to the other wave (12 of the 32
+  // (wave, tile) pairs on a 256-row tile's diagonal).  A loop of its own: a test inside the first one makes the register
+  // allocator copy the accumulators every tile (442 instructions a tile instead of 346; backward of B2 H16 S1000 D128 77 ->
+  // 73 us, B2 H32/8 S4096 bf16 937 -> 916).  (dk/dv has one wave a SIMD, which would only wait at the barrier.)
+  int n_mine = n_items;
+#if AE_MASK_MODE == 1 && AE_BWD_ROLE == 0
+  n_mine = (r0w + 31) / AE_BS + 1 < n_items ? (r0w + 31) / AE_BS + 1 : n_items;
+#endif
+  while (x0 < n_mine) {
     // into the stage everyone left at the last barrier
     request_item(AE_NSTAGE == 3 ? x2 : x1, st_req);
     const tile_at at = tile_in_use(st_use);
@@ -938,15 +961,6 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
 
     ae_u32x4 pf[4], dsf[4];
-    // causal dq: the waves of a workgroup leave the diagonal at different tiles; a wave none of whose rows sees the
-    // tile leaves its SIMD to the other one (12 of the 32 (wave, tile) pairs on a 256-row tile's diagonal).  dk/dv has
-    // one wave a SIMD, all of which meet at the tile's barrier: skipping there frees nothing, and the branch makes the
-    // register allocator copy both accumulators every tile.
-    bool seen = true;
-#if AE_MASK_MODE == 1 && AE_BWD_ROLE == 0
-    seen = at.s0 <= r0w + 31;
-#endif
-    if (__builtin_expect(seen, 1)) {
     if (tests_visibility(at.s0)) {
       block(0, ae_bwd_true{}, at, pf, dsf);
       block(1, ae_bwd_true{}, at, pf, dsf);
@@ -956,21 +970,9 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
     }
 
     add_products(st_use, pf, dsf, []() AE_LAMBDA {});
-    }
-
-    // the next item has landed (with three stages the one after it is still outstanding)
-    __builtin_amdgcn_s_waitcnt(AE_VMCNT((AE_NSTAGE - 2) * AE_NLOADS));
-    __syncthreads();
-#if AE_MASK_MODE != 2
-    us_t++;
-    if (AE_BWD_ROLE == 1 && us_t == t_hi) us_t = t_lo, us_h++;
-#endif
-    st_use = st_use == (AE_NSTAGE - 1) * AE_STAGE_BYTES ? 0 : st_use + AE_STAGE_BYTES;
-    st_req = st_req == (AE_NSTAGE - 1) * AE_STAGE_BYTES ? 0 : st_req + AE_STAGE_BYTES;
-    x0 = x1, cls0 = cls1;
-    x1 = x2, cls1 = cls2;
-    x2 = next_item(x2 + 1, cls2);
+    next_step();
   }
+  for (; x0 < n_items; next_step()) request_item(AE_NSTAGE == 3 ? x2 : x1, st_req);
 #endif
   __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));             // nothing may land in LDS after the workgroup has gone
 
