@@ -35,7 +35,7 @@
 // Waves per workgroup (AE_BWD_NWAVES, 32 resident rows each): dk/dv runs four, one per SIMD with the
 // whole register file (two accumulators), or, softmax attention without a tile table, eight in pairs at head dims 128
 // (AE_BWD_PAIRS) and two workgroups a CU at head dims 64. dq has one accumulator and fits 256 registers, so it runs
-// eight, two per SIMD (AE_BWD_WAVES_PER_EU 2, AE_AHEAD 2): a wave spends about half of its time waiting
+// eight, two per SIMD (AE_BWD_WAVES_PER_EU 2, AE_AHEAD 3): a wave spends about half of its time waiting
 // (LDS fragments, MFMA results, the p/ds arithmetic between two sets of MFMAs) and the second wave
 // fills it - 0.59 -> 0.44 ms for B2 H32 S4096 D128 causal.
 //
@@ -501,7 +501,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   // and one for the transposed reads, added to the stage once a tile.  (From the chunk positions as written above the
   // compiler rebuilt the addresses with an add and a subtraction a read: 72 of the dq launch's 290 VALU
   // instructions a tile.  With the items' positions carried along and the products started at -rowsum(do * o), a dq
-  // tile went from 468 to 357 instructions and a dk/dv tile from 658 to 558; backward of B2 H32 S4096 causal: D128
+  // tile went from 448 to 346 instructions and a dk/dv tile from 652 to 558; backward of B2 H32 S4096 causal: D128
   // 1064 -> 1047 us, where the socket's power cap takes most of it back, D64 forward + backward 885 -> 783 us.)
   static_assert(AE_STAGE_BYTES % 256 == 0 && AE_T1_BYTES % 256 == 0, "the swizzle's bits of a stage's address are zero");
   auto row_part = [&](int str, int cpr) AE_LAMBDA -> unsigned {
