@@ -649,9 +649,9 @@ int ae_prefill_bwd(ae_kernel* delta, ae_kernel* dkv, ae_kernel* dq, const ae_att
   }
   // block_m / threads describe the dq launch (4 or 8 waves of 32 resident rows); dk/dv owns 128 rows, with 4 waves or 8
   // in pairs, whose p and ds take 8 KiB of LDS a pair behind the tile ring
-  const uint32_t dkv_waves = cfg->table_rows ? (uint32_t)cfg->table_rows : 4u;
-  if (dkv_waves != 4 && (dkv_waves != 8 || cfg->head_dim <= 0 ||
-                         cfg->lds_bytes < 3 * (128 * (cfg->head_dim + cfg->head_dim_v) + 512) + 4 * 8192))
+  // (table_rows 16: a value that no forward configuration has)
+  const uint32_t dkv_waves = cfg->table_rows == 16 ? 8u : 4u;
+  if (dkv_waves == 8 && (cfg->head_dim <= 0 || cfg->lds_bytes < 3 * (128 * (cfg->head_dim + cfg->head_dim_v) + 512) + 4 * 8192))
     return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: dk/dv launch of %u waves with %d bytes of LDS", dkv_waves, cfg->lds_bytes);
   if ((cfg->block_m != 128 && cfg->block_m != 256) || cfg->block_n != 64 || cfg->threads != 2 * cfg->block_m || cfg->lds_bytes <= 0 ||
       cfg->lds_bytes > 160 * 1024 || cfg->head_dim_v <= 0 || cfg->head_dim_v % 8 != 0)

@@ -139,8 +139,8 @@ typedef struct ae_tile_cfg {
                           buffers with arrival counters, see ae_decode_fwd); else 0                        */
   int32_t table_rows;  /* mask_mode 2: block-mask rows one q tile may span, the AE_TT_ROWS the kernel was
                           compiled with (1, 2, 4 or 8); 0 stands for the kernels' default of 8.
-                          ae_prefill_bwd: waves of the dk/dv launch, 4 (also 0) or, kernels compiled with
-                          AE_BWD_PAIRS 1, 8                                                                */
+                          ae_prefill_bwd: 16 when the dk/dv kernel was compiled with AE_BWD_PAIRS 1 (its
+                          launch has eight waves instead of four), else not read                           */
 } ae_tile_cfg;
 
 /*
