@@ -55,8 +55,6 @@ class LoweredFunctors:
     # no final row scales (sigmoid / relu attention) - ae_online_fwd<N> may then be called on any subset
     # of a tile's scores, which is how the software-pipelined prefill kernel calls it
     elementwise: bool = False
-    # ... and built of operations that are finite for finite operands: a key of zeros gets some finite weight
-    pad_free: bool = False
 
 
 def _custom_leaves(custom_fwd_inputs: CustomIO, in_dtype, slot_offset: int = 0):
@@ -346,26 +344,6 @@ def _no_tile_reduction(node) -> bool:
     return True
 
 
-def _stays_finite(node) -> bool:
-    """True when the graph holds only operations whose result is finite for finite operands (a division only by a
-    non-zero number)."""
-    seen, stack = set(), [node]
-    while stack:
-        n = stack.pop()
-        if id(n) in seen or not isinstance(n, SymbolScalar):
-            continue
-        seen.add(id(n))
-        prev = list(n.prev or [])
-        if prev and n.code.type == "Div":
-            c = getattr(prev[1], "code", None)
-            if c is None or c.type != "Const" or float(c.value) == 0.0:
-                return False
-        elif prev and n.code.type not in ("Add", "Sub", "Mul", "Neg", "Tanh", "Abs", "Max"):
-            return False
-        stack.extend(prev)
-    return True
-
-
 def _depends_on(node, target) -> bool:
     seen, stack = set(), [node]
     while stack:
@@ -533,7 +511,6 @@ def trace_functors(score_mod, mask_mod, online_func, custom_fwd_inputs: CustomIO
     lf.custom_stage = cust_stage
     lf.softmax = softmax
     lf.elementwise = bool(elementwise and not fvals)
-    lf.pad_free = lf.elementwise and _stays_finite(new_scores)
     lf.deferred_norm = deferred[0] if deferred is not None else None
     return lf
 

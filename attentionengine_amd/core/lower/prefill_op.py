@@ -348,8 +348,8 @@ class PrefillOp:
             else:
                 if self.functors.softmax is not None:
                     cfg_src += "#define AE_PAD_GIVES_ZERO 1\n"
-                if self.functors.pad_free:
-                    cfg_src += "#define AE_PAD_FREE 1\n"
+                if self.functors.elementwise:
+                    cfg_src += "#define AE_ELEMENTWISE 1\n"
             if mask_mode == 2:
                 cfg_src += f"#define AE_TT_ROWS {table_rows}\n#define AE_HEAVY_LAST {1 if heavy_last else 0}\n"
             if band is not None:

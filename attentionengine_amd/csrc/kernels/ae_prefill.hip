@@ -99,11 +99,15 @@
 #ifndef AE_PAD_GIVES_ZERO
 #define AE_PAD_GIVES_ZERO 0
 #endif
-// 1: an elementwise graph built of operations that stay finite - keys past the end arrive as rows of zeros (K and V), score
-// 0, and whatever finite weight they get multiplies a row of zeros: no test at all
-#ifndef AE_PAD_FREE
-#define AE_PAD_FREE 0
+// 1: an elementwise graph (out = sum_kv f(s) v: no row state, no use of the kv index).  The weight of a key past the end is
+// set to 0 whatever its score was - f(0) of a row of zeros need not be finite once it is in the input type, an infinite
+// query times a row of zeros is NaN, and a V whose rows overlap (expanded along the sequence) has no rows of zeros -, so
+// its score needs no test, except where the mask's own test decides whether the row has seen a key
+#ifndef AE_ELEMENTWISE
+#define AE_ELEMENTWISE 0
 #endif
+#define AE_PAD_SCORES (!AE_EVEN_KV && AE_MASK_MODE != 1 && !(AE_ELEMENTWISE && (AE_ANALYTIC || !AE_HAS_MASK_MOD)))
+#define AE_PAD_WEIGHTS (!AE_EVEN_KV && !AE_PAD_GIVES_ZERO)
 #ifndef AE_RB
 #define AE_RB 1
 #endif
@@ -572,7 +576,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
           s[e] = ae_mask_mod(b, h, qrow[rb], kvb + ae_kv_off(e)) ? s[e] : AE_NEG_INF;
       }
 #endif
-#if !AE_EVEN_KV && !AE_PAD_FREE && AE_MASK_MODE != 1     // (causal over equal lengths: behind the diagonal of every row)
+#if AE_PAD_SCORES          // (not causal over equal lengths: behind the diagonal of every row)
       if (kv0 + AE_BN > p.seqlen_kv) {
 #pragma unroll
         for (int e = 0; e < AE_NS; e++) s[e] = (kvb + ae_kv_off(e) < p.seqlen_kv) ? s[e] : AE_KV_PAD;
@@ -613,7 +617,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
       if (jn < j_end) ae_prefetch_custom(cust[rb], jn * AE_BN + 4 * hf, q0w + rb * 32, jn * AE_BN, p);
 #endif
 
-#if !AE_EVEN_KV && !AE_PAD_GIVES_ZERO && !AE_PAD_FREE
+#if AE_PAD_WEIGHTS
       if (kv0 + AE_BN > p.seqlen_kv) {
 #pragma unroll
         for (int e = 0; e < AE_NS; e++) s[e] = (kvb + ae_kv_off(e) < p.seqlen_kv) ? s[e] : 0.f;

@@ -104,13 +104,10 @@ static_assert(AE_KV_STAGES == 2 || AE_KV_STAGES == 3, "two or three K / V stages
 #ifndef AE_TOP_PREFETCH
 #define AE_TOP_PREFETCH (AE_MASK_MODE == 0)
 #endif
-// keys past the end of the sequence are tested for on the tile that holds them: not under a causal mask over equal
-// lengths (they lie behind every row's diagonal), nor for elementwise graphs that stay finite (AE_PAD_FREE, see
-// ae_prefill.hip: the missing K and V rows are zeros)
-#ifndef AE_PAD_FREE
-#define AE_PAD_FREE 0
-#endif
-#define AE_PAD_TEST (!AE_EVEN_KV && !AE_PAD_FREE && AE_MASK_MODE != 1)
+// keys past the end of the sequence are tested for on the tile that holds them: the scores of the softmax not under a
+// causal mask over equal lengths (they lie behind every row's diagonal); an elementwise graph's weights always (see
+// AE_PAD_WEIGHTS of ae_prefill.hip: the missing K and V rows are not always rows of zeros, and f(0) is not always finite)
+#define AE_PAD_TEST (AE_PIPE_KIND == 0 && !AE_EVEN_KV && AE_MASK_MODE != 1)
 // What turns a score into p.  0: the online softmax described above.  1: the generated functor
 // ae_online_fwd itself, two scores at a time, for graphs the lowering has shown to be ELEMENTWISE
 // (out = sum_kv f(s) v, attn_script/sigmoidattn.py, reluattn.py: no row state, no row reduction, no use of
@@ -510,8 +507,8 @@ void ae_prefill_kernel(const ae_attn_params p) {
     pf[qb][e >> 3][(e & 7) >> 1] = __builtin_bit_cast(unsigned, hv);
 #if AE_PIPE_KIND == 1
     (void)rsum;
-#if AE_PAD_TEST
-    // keys past the end: f(-inf) need not be zero.  Only the last tile a wave multiplies can hold such keys.
+#if !AE_EVEN_KV
+    // keys past the end: their weight need not be zero.  Only the last tile a wave multiplies can hold such keys.
     if (!decltype(last_tag)::value) return;
     if (ae_kv_off(e) >= kv_lim) pf[qb][e >> 3][(e & 7) >> 1] = 0u;
     else if (ae_kv_off(e + 1) >= kv_lim) pf[qb][e >> 3][(e & 7) >> 1] &= 0xffffu;
