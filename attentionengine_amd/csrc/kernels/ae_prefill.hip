@@ -720,6 +720,9 @@ void ae_prefill_kernel(const ae_attn_params p) {
     xs[(wave_wg * 3 + 2) * 64 + lane] = seen[0];
     __syncthreads();
     float w[AE_KW];
+    // a group that met a visible key of the row counts, whatever its weight is: one whose visible scores are all NaN
+    // keeps the reference it started with (weight 0) and its NaN has to reach the row all the same
+    bool live[AE_KW];
     bool row_seen = false;
 #if AE_KW_SOFTMAX
     float mg[AE_KW], top = AE_NEG_INF, r_sum = 0.f;
@@ -727,20 +730,19 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #pragma unroll
     for (int k = 0; k < AE_KW; k++) {
       const int wk = (k * AE_NWAVES + wave) * 3;
-      const float sk = xs[(wk + 2) * 64 + lane];
-      row_seen = row_seen || ae_group_max(sk) > 0.f;
+      live[k] = ae_group_max(xs[(wk + 2) * 64 + lane]) > 0.f;
+      row_seen = row_seen || live[k];
       w[k] = 1.f;
 #if AE_KW_SOFTMAX
-      // (a group that met no visible key of the row has r = 0 and O = 0: its reference does not count)
-      mg[k] = sk > 0.f ? xs[wk * 64 + lane] : AE_NEG_INF;
-      top = __builtin_fmaxf(top, mg[k]);
+      mg[k] = xs[wk * 64 + lane];
+      top = live[k] ? __builtin_fmaxf(top, mg[k]) : top;
 #endif
     }
 #if AE_KW_SOFTMAX
 #pragma unroll
     for (int k = 0; k < AE_KW; k++) {
-      w[k] = mg[k] > AE_NEG_INF ? ae_exp(mg[k] - top) : 0.f;
-      r_sum += w[k] > 0.f ? xs[((k * AE_NWAVES + wave) * 3 + 1) * 64 + lane] * w[k] : 0.f;
+      w[k] = ae_exp(mg[k] - top);
+      r_sum += live[k] ? xs[((k * AE_NWAVES + wave) * 3 + 1) * 64 + lane] * w[k] : 0.f;
     }
     st[0].AE_SM_M = top;
     st[0].AE_SM_R = r_sum;
@@ -754,7 +756,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
       for (int e = 0; e < AE_NE; e += 4) {
         const ae_f32x4 v = *(const lds_f4*)(xo + (k * AE_NWAVES + wave) * (AE_NO * 256) + ((kg * AE_NE + e) >> 2) * 1024 + lane * 16);
 #pragma unroll
-        for (int t = 0; t < 4; t++) o[e + t] += w[k] > 0.f ? v[t] * w[k] : 0.f;
+        for (int t = 0; t < 4; t++) o[e + t] += live[k] ? v[t] * w[k] : 0.f;
       }
     float frs[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1];
     frs[0] = 0.f;

@@ -81,3 +81,30 @@ def test_kv_groups_of_graphs_without_row_state(cuda_device):
     out = mod(q.cuda(), k.cuda(), v.cuda(), torch.tensor([-2.0], device="cuda"))
     ref = R.sigmoid_attention(q, k, v, bias=-2.0)
     assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tiles", TILES, ids=lambda t: f"{t.block_m}x{t.kv_groups}x{t.block_n}")
+@pytest.mark.parametrize("what", ["key", "tile", "value", "infinite_key"])
+@pytest.mark.parametrize("causal", [False, True])
+def test_a_nan_reaches_every_row_that_sees_it(cuda_device, tiles, what, causal):
+    """... also where it is all that a kv group sees of a row; rows that do not see it are as without it.  (An infinite
+    score makes its row NaN: inf - inf.)"""
+    B, H, S, D, dtype = 1, 2, 200, 64, torch.float16
+    print(f"case nan {tiles.block_m}x{tiles.kv_groups}x{tiles.block_n} {what} causal={causal}", flush=True)
+    q, k, v = C.make_inputs(B, S, S, H, H, D, D, dtype, seed=13)
+    q = q.abs() + 2 ** -6                                         # (an infinite key scores +inf with every row)
+    meta = (meta_tensor(B, H, S, D, dtype=dtype),) * 3
+    op = PrefillOp(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), C.causal_mask if causal else None,
+                   C.OnlineSoftmax(), "-inf", tiles=tiles)
+    ref, _ = R.softmax_attention(q, k, v, causal=causal)
+    lo, hi = (64, 96) if what == "tile" else (70, 71)
+    bad = (v if what == "value" else k).clone()
+    bad[:, lo:hi] = math.nan if what != "infinite_key" else 0.0
+    if what == "infinite_key":
+        bad[:, lo:hi, :, 0] = math.inf
+    out = op(q.cuda(), (k if what == "value" else bad).cuda(), (bad if what == "value" else v).cuda()).float().cpu()
+    sees = torch.arange(S) >= lo if causal else torch.ones(S, dtype=torch.bool)
+    assert torch.isnan(out[:, sees]).all()
+    if causal and what != "value":                                # (0 * NaN: a masked key's value still spoils its tile)
+        assert (out[:, ~sees] - ref[:, ~sees]).abs().max().item() <= 2e-2
