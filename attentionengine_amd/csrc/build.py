@@ -27,6 +27,7 @@ HOST = osp.join(CSRC, "_ae_host.so")
 DEVICE_FLAGS = ["-O3", "-std=c++17", "-fno-math-errno", "-fno-trapping-math", "-fno-signed-zeros",
                 "-freciprocal-math", "-ffp-contract=fast",
                 "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+TEMPLATE_FLAGS = {"ae_prefill_pipe.hip": ["-mllvm", "-align-all-nofallthru-blocks=6"]}      # (TEMPLATE_OPTS there)
 
 
 def _run(cmd):
@@ -83,7 +84,7 @@ def check_templates(header_sets, verbose=False):
                 with open(osp.join(d, name), "w") as f:
                     f.write(text)
             obj = osp.join(d, "k.o")
-            cmd = [hipcc, "--offload-arch=gfx950", "--cuda-device-only", "-c", *DEVICE_FLAGS,
+            cmd = [hipcc, "--offload-arch=gfx950", "--cuda-device-only", "-c", *DEVICE_FLAGS, *TEMPLATE_FLAGS.get(template, []),
                    f"-I{INCLUDE}", f"-I{d}", f"-I{osp.join(CSRC, 'kernels')}",
                    osp.join(CSRC, "kernels", template), "-o", obj]
             _run(cmd)

@@ -739,3 +739,30 @@ def test_tile_classes_of_a_user_block_mask():
                     some, every = t.any(-1).any(-1), t.all(-1).all(-1)
                     want = some.to(torch.int8) + (some & every).to(torch.int8)
                     assert torch.equal(got[:, :, i, j], want), (bm, bn, Sq, Skv, tm, tn, i, j)
+
+
+def test_options_of_one_template_stay_with_it(monkeypatch):
+    """Compiler options that a single template adds (hip_rt.TEMPLATE_OPTS) do not change what is compiled after it in the
+    same process, and are part of the key of its code objects."""
+    import ctypes
+    from core.runtime import hip_rt as rt
+    headers = {}
+    compiled = rt._compile_module
+    monkeypatch.setattr(rt, "_compile_module", lambda t, h, *a: headers.setdefault(t, h) and compiled(t, h, *a))
+    for kernel in ("generic", "pipelined"):
+        monkeypatch.setenv("AE_PREFILL_KERNEL", kernel)
+        AttentionEngine((meta_tensor(1, 2, 256, 128, dtype=torch.float16),) * 3, CustomIO({}),
+                        C.make_scale_score_mod(0.1), C.causal_mask, C.OnlineSoftmax())
+
+    def code(template):
+        monkeypatch.setattr(rt, "_modules", {})
+        m = compiled(template, headers[template], None, False)
+        data, n = ctypes.c_void_p(), ctypes.c_size_t()
+        assert rt.lib().ae_module_code(m.handle, ctypes.byref(data), ctypes.byref(n)) == 0
+        return m.key, ctypes.string_at(data, n.value)
+    assert set(headers) == {"ae_prefill.hip", "ae_prefill_pipe.hip"} and "ae_prefill_pipe.hip" in rt.TEMPLATE_OPTS
+    first = code("ae_prefill.hip")
+    with_opts = code("ae_prefill_pipe.hip")
+    assert code("ae_prefill.hip") == first
+    monkeypatch.setattr(rt, "TEMPLATE_OPTS", {})
+    assert code("ae_prefill_pipe.hip")[0] != with_opts[0] and code("ae_prefill.hip") == first
