@@ -766,3 +766,37 @@ def test_options_of_one_template_stay_with_it(monkeypatch):
     assert code("ae_prefill.hip") == first
     monkeypatch.setattr(rt, "TEMPLATE_OPTS", {})
     assert code("ae_prefill_pipe.hip")[0] != with_opts[0] and code("ae_prefill.hip") == first
+
+
+@pytest.mark.parametrize("kind", ["gqa", "mla"])
+def test_every_split_count_that_is_tuned_is_launched(monkeypatch, tmp_path, kind):
+    """tune=True measures through the operator's own calls, which the native host path serves from the plan that the last
+    Python call of the shape left: no candidate may be served by another one's plan."""
+    from core.lower import tuner
+    if kind == "gqa":
+        meta, more, key = (meta_tensor(1, 8, 1, 128, dtype=torch.float16),) + (meta_tensor(1, 2, 2048, 128, dtype=torch.float16),) * 2, {}, (1, 8, 2, 2048)
+    else:
+        meta = (meta_tensor(1, 16, 1, 576, dtype=torch.float16), meta_tensor(1, 1, 2048, 576, dtype=torch.float16),
+                meta_tensor(1, 1, 2048, 512, dtype=torch.float16))
+        more, key = {"kv_shared": True}, (1, 16, 1, 2048)
+    op = AttentionEngine(meta, CustomIO({}), C.make_scale_score_mod(0.1), None, C.OnlineSoftmax(), tune=True,
+                         tune_file=str(tmp_path / "tuned.json"), **more).attention
+
+    class Host:
+        plan = None
+
+        def clear(self):
+            self.plan = None
+    op._host = Host()
+    launched = []
+
+    def run():
+        if op._host.plan is None:                    # the Python path: plans, launches and leaves its plan behind
+            op._host.plan = op.plan_splits(*key)[0]
+        launched.append(op._host.plan)
+    ms = iter((3.0, 1.0, 2.0))
+    monkeypatch.setattr(tuner, "time_call", lambda f: (f(), next(ms))[1])
+    op._tune_splits(key, [2, 4, 8], run)
+    assert len(set(launched)) == 3 and op._tuned[key] == 4
+    run()
+    assert launched[-1] == launched[1]               # ... and the calls that follow run the one that was fastest
