@@ -29,10 +29,12 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
 
 #include <cstdlib>
 #include <memory>
 #include <string>
+#include <tuple>
 #include <utility>
 #include <vector>
 
@@ -41,7 +43,7 @@
 namespace {
 
 constexpr size_t kMaxPlans = 64;       // plans a Host keeps; the oldest goes
-constexpr size_t kMaxWork = 16;        // (plan, stream) pairs whose split-KV work buffers a plan keeps
+constexpr size_t kMaxWork = 16;        // work buffers a Host keeps, beyond those that a captured graph replays on
 
 // Python objects that own the plan's code objects: released under the GIL whichever thread drops the last reference
 struct Keep {
@@ -82,11 +84,19 @@ struct Plan {
   std::vector<std::pair<std::string, std::string>> env;   // switches this plan was made under
   std::shared_ptr<Keep> keep;
   std::shared_ptr<BwdPlan> bwd;
-  struct Work {
-    void* stream;
-    at::Tensor partial_o, partial_rs;
-  };
-  std::vector<Work> work;   // merge in the last workgroup: buffers whose arrival counters stay zero between launches
+  int64_t o_rows = 0, counters = 0;   // partial results a split launch writes; arrival counters behind the row scales
+};
+
+// Work buffers of launches whose last workgroup merges: the arrival counters behind the row scales are zero when a
+// launch starts, and every launch leaves them at zero (ae_decode_fwd).  Kept by the Host, per size and stream - launches
+// on one stream run one after the other and may share them -, not by a plan: plans come and go with the shapes and
+// settings of the calls, while a graph captured on the stream goes on using the addresses.
+struct Work {
+  int device;
+  void* stream;
+  int64_t o_rows, rs_floats, counters;
+  bool captured;            // recorded into a graph: kept as long as the Host
+  at::Tensor partial_o, partial_rs;
 };
 
 struct Host {
@@ -96,6 +106,7 @@ struct Host {
   int n_custom, n_rs;
   int custom_in_dtype;      // bit i: custom input i is read in the input dtype (else fp32)
   std::vector<std::shared_ptr<Plan>>* plans;
+  std::vector<Work>* work;
 };
 
 bool env_matches(const Plan& pl) {
@@ -123,6 +134,35 @@ bool readable(const at::Tensor& t) {
 
 at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dt, int device) {
   return at::Tensor(at::detail::empty_cuda(sizes, dt, c10::Device(c10::kCUDA, (c10::DeviceIndex)device), std::nullopt));
+}
+
+// The work buffers of a launch on `stream` (see Work).  A capture that finds none kept gets buffers of its own, which live
+// in the graph's memory, and records the clearing of their counters: what a capture allocates and clears is only there
+// when that graph has been replayed, so no other call may be given it.
+std::pair<at::Tensor, at::Tensor> get_work(Host* h, int64_t o_rows, int64_t rs_floats, int64_t counters, int device, void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  bool capturing = true;
+  if (hipStreamIsCapturing((hipStream_t)stream, &status) == hipSuccess) capturing = status != hipStreamCaptureStatusNone;
+  else (void)hipGetLastError();         // (the default stream while another one captures)
+  for (auto& w : *h->work)
+    if (w.device == device && w.stream == stream && w.o_rows == o_rows && w.rs_floats == rs_floats && w.counters == counters) {
+      w.captured = w.captured || capturing;
+      return {w.partial_o, w.partial_rs};
+    }
+  at::Tensor po = empty({o_rows, h->DV}, at::kFloat, device), prs = empty({rs_floats + counters}, at::kFloat, device);
+  prs.narrow(0, rs_floats, counters).zero_();
+  if (!capturing) {
+    size_t n = 0;
+    for (const auto& w : *h->work) n += !w.captured;
+    if (n >= kMaxWork)
+      for (auto it = h->work->begin(); it != h->work->end(); ++it)
+        if (!it->captured) {
+          h->work->erase(it);
+          break;
+        }
+    h->work->push_back({device, stream, o_rows, rs_floats, counters, false, po, prs});
+  }
+  return {po, prs};
 }
 
 void set_strides(const at::Tensor& t, int64_t& b, int64_t& s, int64_t& h) {
@@ -352,29 +392,14 @@ PyObject* run(Host* h, PyObject* const* args, Py_ssize_t nargs, bool mla) {
     p.mask_nq = (int)pl.table.size(2), p.mask_nkv = (int)pl.table.size(3);
     p.mask_block_m = pl.mask_bm, p.mask_block_n = pl.mask_bn;
   }
-  const int64_t n_rs1 = h->n_rs > 0 ? h->n_rs : 1;
+  const int64_t rs_floats = (h->n_rs > 0 ? h->n_rs : 1) * B * Sq * Hq * pl.n_split;
   at::Tensor po, prs;
   if (pl.kind != kPrefill) p.num_splits = pl.n_split, p.kv_per_split = pl.kv_per_split;
   if (pl.cfg.merge_in_wg == 2) {
-    // work buffers kept per (plan, stream): launches on one stream run one after the other and may share them, and
-    // every launch leaves the arrival counters behind the row scales at zero (ae_decode_fwd)
-    Plan::Work* w = nullptr;
-    for (auto& x : pl.work)
-      if (x.stream == stream) w = &x;
-    if (!w) {
-      if (pl.work.size() >= kMaxWork) pl.work.erase(pl.work.begin());
-      const int64_t rows = B * Sq * Hq * pl.n_split;
-      const int64_t counters = pl.kind == kDecode
-          ? B * c.Hkv * ((Hq / c.Hkv + pl.cfg.block_m - 1) / pl.cfg.block_m)
-          : B * Hq * ((Sq + pl.cfg.block_m - 1) / pl.cfg.block_m);
-      pl.work.push_back({stream, empty({rows, h->DV}, at::kFloat, dev),
-                         at::zeros({n_rs1 * rows + counters}, at::TensorOptions().dtype(at::kFloat).device(c.q.device()))});
-      w = &pl.work.back();
-    }
-    po = w->partial_o, prs = w->partial_rs;
+    std::tie(po, prs) = get_work(h, pl.o_rows, rs_floats, pl.counters, dev, stream);
   } else if (pl.n_split > 1 && pl.cfg.merge_in_wg == 0) {
-    po = empty({B * Sq * Hq * pl.n_split, h->DV}, at::kFloat, dev);
-    prs = empty({n_rs1 * B * Sq * Hq * pl.n_split}, at::kFloat, dev);
+    po = empty({pl.o_rows, h->DV}, at::kFloat, dev);
+    prs = empty({rs_floats}, at::kFloat, dev);
   }
   if (po.defined()) p.partial_o = (float*)po.mutable_data_ptr(), p.partial_rs = (float*)prs.mutable_data_ptr();
 
@@ -452,6 +477,8 @@ PyObject* host_add(PyObject* self, PyObject* d) {
   TORCH_CHECK(pl->k0 && get_cfg(d, "cfg", pl->cfg), "a plan needs a kernel and its tile configuration");
   pl->has_ccfg = get_cfg(d, "ccfg", pl->ccfg);
   pl->n_split = (int)get_int(d, "n_split", 1), pl->kv_per_split = (int)get_int(d, "kv_per_split");
+  pl->o_rows = get_int(d, "o_rows", pl->B * pl->Sq * pl->Hq * pl->n_split), pl->counters = get_int(d, "counters");
+  TORCH_CHECK(pl->cfg.merge_in_wg != 2 || pl->counters > 0, "a launch whose last workgroup merges needs arrival counters");
   pl->table = get_tensor(d, "table");
   pl->mask_bm = (int)get_int(d, "mask_bm"), pl->mask_bn = (int)get_int(d, "mask_bn");
   if (PyObject* env = PyDict_GetItemString(d, "env")) {
@@ -494,6 +521,22 @@ PyObject* host_add_backward(PyObject* self, PyObject* d) {
   END_HANDLE_TH_ERRORS
 }
 
+// work(o_rows, rs_floats, counters, device, stream) -> (partial_o, partial_rs)
+PyObject* host_work(PyObject* self, PyObject* args) {
+  HANDLE_TH_ERRORS
+  long long o_rows, rs_floats, counters, stream;
+  int device;
+  if (!PyArg_ParseTuple(args, "LLLiL", &o_rows, &rs_floats, &counters, &device, &stream)) return nullptr;
+  TORCH_CHECK(o_rows > 0 && rs_floats > 0 && counters > 0, "work(): sizes must be positive");
+  auto w = get_work((Host*)self, o_rows, rs_floats, counters, device, (void*)(uintptr_t)stream);
+  PyObject* res = PyTuple_New(2);
+  if (!res) return nullptr;
+  PyTuple_SET_ITEM(res, 0, THPVariable_Wrap(w.first));
+  PyTuple_SET_ITEM(res, 1, THPVariable_Wrap(w.second));
+  return res;
+  END_HANDLE_TH_ERRORS
+}
+
 PyObject* host_clear(PyObject* self, PyObject*) {
   ((Host*)self)->plans->clear();
   Py_RETURN_NONE;
@@ -513,10 +556,12 @@ PyObject* host_new(PyTypeObject* type, PyObject* args, PyObject*) {
   h->D = D, h->DV = DV, h->dtype = bf16 ? at::kBFloat16 : at::kHalf, h->n_custom = n_custom, h->n_rs = n_rs;
   h->custom_in_dtype = in_dtype;
   h->plans = new std::vector<std::shared_ptr<Plan>>();
+  h->work = new std::vector<Work>();
   return (PyObject*)h;
 }
 void host_dealloc(PyObject* self) {
   delete ((Host*)self)->plans;
+  delete ((Host*)self)->work;
   PyTypeObject* tp = Py_TYPE(self);
   tp->tp_free(self);
   Py_DECREF(tp);
@@ -528,6 +573,7 @@ PyMethodDef host_methods[] = {
      "run_mla(q, q_pe, kv, k_pe) or run_mla(q, cache[, block_table, cache_seqlens]) -> (out, *row scales) or None"},
     {"add", host_add, METH_O, "add(plan dict)"},
     {"add_backward", host_add_backward, METH_O, "add_backward(plan dict)"},
+    {"work", host_work, METH_VARARGS, "work(o_rows, rs_floats, counters, device, stream) -> (partial_o, partial_rs) with zero counters"},
     {"clear", host_clear, METH_NOARGS, "drop every plan"},
     {nullptr, nullptr, 0, nullptr}};
 PyType_Slot host_slots[] = {{Py_tp_new, (void*)host_new}, {Py_tp_dealloc, (void*)host_dealloc}, {Py_tp_methods, host_methods},

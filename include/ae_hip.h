@@ -266,7 +266,9 @@ int ae_launch(ae_kernel* k, const void* params, size_t params_bytes,
  *   kv head, head tile) that finishes last merges all partial results and writes out (one launch).  Its arrival
  *   counters are 32-bit integers BEHIND the row scales in partial_rs -- after max(1, n_rowscales) * batch * heads_q *
  *   num_splits floats, batch * ceil(Hq/Hkv / block_m) * Hkv of them -- which must be zero before the first launch
- *   and which every launch leaves at zero; launches that share these buffers must not overlap.  With
+ *   and which every launch leaves at zero; launches that share these buffers must not overlap.  A split kernel
+ *   compiled with AE_WG_FIRST 1 writes one partial per workgroup: the first batch * heads_q * num_splits / (threads/64)
+ *   rows of partial_o are all it touches.  With
  *   cfg->merge_in_wg = 0 the combine kernel, its configuration and both work buffers are required; a launch that
  *   lacks any of them is refused, nothing runs.
  */

@@ -93,3 +93,65 @@ def test_repeated_training_steps_run_natively_and_agree(cuda_device, kind):
     out.backward(do)
     with pytest.raises(RuntimeError, match="second time"):
         out.backward(do)
+
+
+def _split_decode(cuda_device, Skv=3001, B=1, Hq=8, Hkv=2, D=128):
+    mod = _engine(B, Hq, Hkv, 1, Skv, D)
+    q, k, v = (t.to(cuda_device) for t in C.make_inputs(B, 1, Skv, Hq, Hkv, D, D, torch.float16))
+    op = mod._op
+    n_split, _ = op.plan_splits(B, Hq, Hkv, Skv)
+    assert op.merges_in_last_workgroup(n_split) and op.grouped_merge
+
+    def work(stream):      # the buffers of this call on a stream
+        return op._host.work(B * Hq * n_split // op.N_WAVES, B * Hq * n_split, B * Hkv, cuda_device.index or 0, stream.cuda_stream)
+    return mod, q, k, v, work
+
+
+@pytest.mark.gpu
+def test_kept_work_buffers_outlive_the_plans(cuda_device):
+    """A graph captured on a warmed-up stream replays on the buffers that were kept for it, whatever shapes, strides and
+    settings the operator has been called with since."""
+    mod, q, k, v, work = _split_decode(cuda_device)
+    want, s = mod(q, k, v).clone(), torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        for _ in range(2):
+            assert torch.equal(mod(q, k, v), want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        out = mod(q, k, v)
+    kept = [t.data_ptr() for t in work(s)]
+    assert work(s)[0].shape[0] == mod._op.plan_splits(1, 8, 2, 3001)[0] * 8 // mod._op.N_WAVES
+    odd = torch.empty(*k.shape[:3], k.shape[3] + 4, dtype=k.dtype, device=k.device)[..., 4:].copy_(k)
+    for r in range(3):
+        with torch.cuda.stream(s):
+            for n in range(100, 3001, 41):               # more shapes than plans are kept
+                mod(q, k[:, :n], v[:, :n])
+            assert torch.equal(mod(q, odd, v), want)     # the Python path: its plan replaces the shape's
+            mod._op.target_workgroups = 256              # drops every plan
+            assert torch.equal(mod(q, k, v), want)
+            out.zero_()
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), r
+    assert [t.data_ptr() for t in work(s)] == kept
+
+
+@pytest.mark.gpu
+def test_a_capture_on_a_new_stream_has_its_own_work_buffers(cuda_device):
+    """Counters that a capture clears are zero only once that graph has been replayed."""
+    mod, q, k, v, work = _split_decode(cuda_device)
+    want, s = mod(q, k, v).clone(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graphs, outs = [torch.cuda.CUDAGraph() for _ in range(2)], []
+    for g in graphs:
+        with torch.cuda.graph(g, stream=s):
+            outs.append(mod(q, k, v))
+    for i in (1, 1, 0, 1, 0):
+        with torch.cuda.stream(s):
+            outs[i].zero_()
+            graphs[i].replay()
+            assert torch.equal(outs[i], want), i
+            assert torch.equal(mod(q, k, v), want)       # an eager call on the stream the graphs were captured on
+        torch.cuda.synchronize()
