@@ -245,8 +245,9 @@ std::shared_ptr<Plan> find(Host* h, const Call& c, int device) {
   return nullptr;
 }
 
+// (torch.Tensor and torch.nn.Parameter themselves: a subclass may override what its calls do, __torch_function__)
 const at::Tensor* tensor_arg(PyObject* o) {
-  return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr;
+  return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr;
 }
 
 // The call's tensors as the plan's kernel takes them; false: not a call for this path

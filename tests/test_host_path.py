@@ -155,3 +155,25 @@ def test_a_capture_on_a_new_stream_has_its_own_work_buffers(cuda_device):
             assert torch.equal(outs[i], want), i
             assert torch.equal(mod(q, k, v), want)       # an eager call on the stream the graphs were captured on
         torch.cuda.synchronize()
+
+
+class _Labelled(torch.Tensor):
+    """A subclass that only overrides what happens to its calls (no dispatch key of its own)."""
+    calls = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.calls.append(getattr(func, "__name__", str(func)))
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+@pytest.mark.gpu
+def test_tensor_subclasses_go_to_python(cuda_device):
+    mod = _engine(1, 2, 2, 70, 70, 64, mask=C.causal_mask)
+    q, k, v = (t.to(cuda_device) for t in C.make_inputs(1, 70, 70, 2, 2, 64, 64, torch.float16))
+    want = mod(q, k, v)
+    host = mod._op._host
+    assert len(host) == 1 and host.run(q, k, v) is not None and host.run(torch.nn.Parameter(q, False), k, v) is not None
+    assert host.run(q.as_subclass(_Labelled), k, v) is None and host.run(q, k, v.as_subclass(_Labelled)) is None
+    _Labelled.calls.clear()
+    assert torch.equal(mod(q.as_subclass(_Labelled), k, v).as_subclass(torch.Tensor), want) and _Labelled.calls
