@@ -119,7 +119,7 @@ bool env_matches(const Plan& pl) {
 
 bool plain(const at::Tensor& t) {
   return t.defined() && t.is_cuda() && !t.unsafeGetTensorImpl()->is_python_dispatch() && t.layout() == at::kStrided &&
-         !t.is_conj() && !t.is_neg();
+         !t.is_conj() && !t.is_neg() && !t._fw_grad(0).defined();      // (forward mode: autograd.Function says it has no rule)
 }
 
 // a tensor the kernels read as it is: dense last dimension, 16-byte start, other strides multiples of 8 elements

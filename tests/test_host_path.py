@@ -177,3 +177,16 @@ def test_tensor_subclasses_go_to_python(cuda_device):
     assert host.run(q.as_subclass(_Labelled), k, v) is None and host.run(q, k, v.as_subclass(_Labelled)) is None
     _Labelled.calls.clear()
     assert torch.equal(mod(q.as_subclass(_Labelled), k, v).as_subclass(torch.Tensor), want) and _Labelled.calls
+
+
+@pytest.mark.gpu
+def test_forward_mode_is_refused_on_every_call(cuda_device):
+    import torch.autograd.forward_ad as fw
+    mod = _engine(1, 2, 2, 70, 70, 64, mask=C.causal_mask)
+    q, k, v = (t.to(cuda_device).requires_grad_(True) for t in C.make_inputs(1, 70, 70, 2, 2, 64, 64, torch.float16))
+    for i in range(3):
+        out = mod(q, k, v)
+        assert ("AttentionEngineBackward" in out.grad_fn.name()) == (i > 0)
+        torch.autograd.grad(out, (q, k, v), torch.ones_like(out))
+        with fw.dual_level(), pytest.raises(NotImplementedError, match="jvp"):
+            mod(fw.make_dual(q, torch.ones_like(q)), k, v)
