@@ -14,8 +14,9 @@
 // 77 -> 36 us of host time.  The reference's generated torch.autograd.Function and its TileLang / pybind11 callables
 // do this work per call in Python as well (core/template/tl_template/attn/attn_tl.py:567-640).
 //
-// Threads: calls come from Python with the GIL held, which also guards the plans and the kept work buffers; the
-// backward node runs on autograd's own threads without it and touches only what it holds itself.
+// Threads: calls come from Python with the GIL held, which also guards the plans and the kept work buffers.  A launch
+// runs without it - a full launch queue makes the caller wait, not the process - on what the call holds itself; so does
+// the backward node, on autograd's own threads.
 
 #include <torch/csrc/autograd/edge.h>
 #include <torch/csrc/autograd/function.h>
@@ -405,12 +406,14 @@ PyObject* run(Host* h, PyObject* const* args, Py_ssize_t nargs, bool mla) {
   if (po.defined()) p.partial_o = (float*)po.mutable_data_ptr(), p.partial_rs = (float*)prs.mutable_data_ptr();
 
   int rc;
+  PyThreadState* thread = PyEval_SaveThread();
   switch (pl.kind) {
     case kPrefill: rc = ae_prefill_fwd(pl.k0, &p, &pl.cfg, stream); break;
     case kPrefillSplit: rc = ae_prefill_split_fwd(pl.k0, pl.k1, &p, &pl.cfg, &pl.ccfg, stream); break;
     case kDecode: rc = ae_decode_fwd(pl.k0, pl.k1, &p, &pl.cfg, pl.has_ccfg ? &pl.ccfg : nullptr, stream); break;
     default: rc = ae_mla_decode_fwd(pl.k0, pl.k1, &p, &pl.cfg, &pl.ccfg, stream); break;
   }
+  PyEval_RestoreThread(thread);
   if (rc) return raise_status(rc);
 
   if (wants_grad) {

@@ -1,6 +1,9 @@
 """The native host path of repeated calls (csrc/ae_host.cpp): a second call of a shape runs there, gives what the first
 one gave, and calls that its plans do not cover go back to the operators' Python code."""
 import math
+import sys
+import threading
+import time
 
 import pytest
 import torch
@@ -190,3 +193,31 @@ def test_forward_mode_is_refused_on_every_call(cuda_device):
         torch.autograd.grad(out, (q, k, v), torch.ones_like(out))
         with fw.dual_level(), pytest.raises(NotImplementedError, match="jvp"):
             mod(fw.make_dual(q, torch.ones_like(q)), k, v)
+
+
+@pytest.mark.gpu
+def test_other_threads_run_while_a_call_launches(cuda_device):
+    mod = _engine(1, 2, 2, 70, 70, 64, mask=C.causal_mask)
+    q, k, v = (t.to(cuda_device) for t in C.make_inputs(1, 70, 70, 2, 2, 64, 64, torch.float16))
+    mod(q, k, v)
+    run, turns, stop, old = mod._op._host.run, [0], [], sys.getswitchinterval()
+
+    def other():
+        while not stop:
+            turns[0] += 1
+            time.sleep(0)                   # gives the interpreter lock back
+    t = threading.Thread(target=other)
+    t.start()
+    try:
+        sys.setswitchinterval(60.0)         # this thread gives it up of its own accord only
+        time.sleep(0.1)                     # (the other one no longer waits by the old interval)
+        before = turns[0]
+        for i in range(5000):
+            run(q, k, v)
+        # (50,000 and more where the launches give the lock back; 4 to 400 where they kept it: other parts of a call,
+        # the freeing of its results for one, give it back now and then)
+        assert turns[0] - before > 2500
+    finally:
+        sys.setswitchinterval(old)
+        stop.append(True)
+        t.join()
