@@ -9,6 +9,7 @@ rowscales, launches on torch's current stream, returns ``o``.
 from __future__ import annotations
 
 import os
+from dataclasses import astuple
 
 import torch
 
@@ -89,19 +90,29 @@ class PrefillOp:
         if self.tiles.rows_per_wave == 64 and os.environ.get("AE_PREFILL_KERNEL", "") != "pipelined" and (
                 self.extern_block_mask or (mask_mod is not None and self._probe_mask(q_meta, v_meta).mode == 2)):
             self.tiles = L.PrefillTiles()
+        self._table_tiles = L.PrefillTiles() if split_kv else self.tiles     # ... of a call that brings a block mask
         # Band masks are read in 32-key tiles (B2 H32 S4096 D128, window of 256: 94.8 -> 88.4 us with them, of 1024 184 -> 180):
         # less of the band's edges is multiplied.
         if self.mask_mod is not None and self.tiles == L.PrefillTiles() and self.D in (64, 128) and self.DV in (64, 128):
             band = self._probe_mask(q_meta, v_meta).band
             if band is not None and band[1] is not None:
                 self.tiles = L.PrefillTiles(block_n=32)
-        groups = self._groups = self._kv_group_choice(q_meta, v_meta, split_kv)
+        # Launches that leave the chip idle with these tiles: waves that share the kv axis.  That depends on the extents
+        # of a call, so an engine declared at such extents decides again for every shape it is called with (tiles_for);
+        # self.tiles are the declared shape's, self._base what the other shapes use where the kv axis is not shared.
+        self.split_kv = bool(split_kv)
+        self._base = L.PrefillTiles() if self.split_kv else self.tiles
+        shape = (q_meta.shape[0], q_meta.shape[1], q_meta.shape[2], v_meta.shape[2])
+        self._declared = None if any(isinstance(x, str) for x in shape) else tuple(int(x) for x in shape)
+        groups = self._groups = self._kv_group_choice(
+            *self._declared, lambda found: self._probe_mask(q_meta, v_meta)) if self._declared else None
         if groups is not None:
             self.tiles = groups
+        self._call_tiles = {}      # (B, H, Sq, Skv) other than the declared ones -> tiles_for()
         # tune=True (attn_tl.py:465-521 of the reference): the tile configuration comes from the record of
         # this problem in tune_file, or is measured at the first call and recorded there.  Launches whose
         # tiles are bound to something else (split-KV, an external block mask) keep the fixed choice.
-        self._tune_file, self._tune_pending, self.tune_times = "", False, None
+        self._tune_file, self._tune_pending, self._tune_found, self.tune_times = "", False, False, None
         self._tune_bwd = (bool(tune_bwd), tune_file_bwd)
         if tiles is not None:
             self.tiles = tiles
@@ -111,13 +122,12 @@ class PrefillOp:
             self._tune_keys = tuner.problem_keys(q_meta.shape, self.D, self.DV)
             found = tuner.decode_tiles(tuner.lookup(tune_file, self._tune_keys), self._tune_candidates())
             if found is not None:
-                self.tiles = found
+                self.tiles, self._tune_found = found, True
             else:
                 self._tune_pending = True
         # Split-KV ("MHA decode": a few query tokens against a long KV, attn_engine.py:273-290 and
         # core/lower/lower_decode.py:287-313 of the reference): the kv axis is shared out over several
         # workgroups per q tile and the partial results are merged with the user's combine().
-        self.split_kv = bool(split_kv)
         self.target_workgroups = int(target_workgroups)
         if self.split_kv:
             if self.tiles.template == "ae_prefill_simple.hip" or max(self.D, self.DV) > 128:
@@ -144,6 +154,10 @@ class PrefillOp:
                     self.mask_block[1] % self.tiles.block_n or \
                     self.tiles.block_m > self.MASK_ROWS_PER_TILE * self.mask_block[0]:
                 raise NotImplementedError(f"block mask granularity {self.mask_block} does not fit the tiles")
+        if self.tiles.kv_groups == 1:
+            self._base = self.tiles
+        if self._tiles_given or self.extern_block_mask or self._tune_found:
+            self._table_tiles = self._base
         self.n_rowscales = len(self.functors.final_rowscale_names)
         if self.n_rowscales > rt.AE_MAX_ROWSCALES or len(self.functors.customs) > rt.AE_MAX_CUSTOM:
             raise NotImplementedError("too many rowscales / custom inputs")
@@ -173,9 +187,12 @@ class PrefillOp:
         switches to the generic kernel, whose two waves per SIMD leave the compiler room, for every later launch:
         True if it did.  (The pipelined kernel holds 64 query rows per wave in one wave per SIMD and fills the
         register file; its fp16 builds fit, some bf16 builds at head dim 128 spill a few values.)"""
-        if self._tiles_given or self.tiles.template != "ae_prefill_pipe.hip":
+        if self._tiles_given or self._base.template != "ae_prefill_pipe.hip":
             return False
-        self.tiles = L.PrefillTiles()
+        if self.tiles == self._base:
+            self.tiles = L.PrefillTiles()
+        self._base = self._table_tiles = L.PrefillTiles()
+        self._call_tiles.clear()
         self._variants.clear()
         self._plans.clear()
         self._host.clear()
@@ -184,13 +201,14 @@ class PrefillOp:
         return True
 
     def _compile_declared_shape(self, B, H, Sq, Skv, infer_mask, mask_mod):
-        plan = self._plan(B, H, Sq, Skv, device=None)
+        tiles = self.tiles_for(B, H, Sq, Skv)
+        plan = self._plan(B, H, Sq, Skv, device=None, tiles=tiles)
         mode = 2 if self.extern_block_mask else plan.mode
-        n_split, _ = self.plan_splits(B, H, Sq, Skv)
-        _, _, cfg_src = self._variant(mode, Sq % self.tiles.block_m == 0, Skv % self.tiles.block_n == 0, n_split,
-                                      self._table_rows(self.mask_block[0] if self.extern_block_mask else plan.block_m),
+        n_split, _ = self.plan_splits(B, H, Sq, Skv, tiles)
+        _, _, cfg_src = self._variant(tiles, mode, Sq, Skv, n_split,
+                                      self._table_rows(self.mask_block[0] if self.extern_block_mask else plan.block_m, tiles),
                                       plan.heavy_last and not self.extern_block_mask,
-                                      None if self.extern_block_mask else self._band(plan))
+                                      None if self.extern_block_mask else self._band(plan, tiles))
         self.source = cfg_src + "\n" + self.functor_src
         if infer_mask and mask_mod is not None and not self.extern_block_mask:
             self.block_mask = self._reference_block_mask(B, H, Sq, Skv)
@@ -204,24 +222,36 @@ class PrefillOp:
                                      elementwise=self.elementwise_mask)
         return self._probed
 
-    def _kv_group_choice(self, q_meta, v_meta, split_kv):
-        """Tiles whose waves share the kv axis, where this engine's graph, mask and declared extents allow and want them:
-        a merge the kernel knows (the proven online softmax, or no row state), no mask table, no tensor read per score."""
-        sq, skv = _dim(q_meta.shape[2], 0), _dim(v_meta.shape[2], 0)
-        bh = _dim(q_meta.shape[0], 0) * _dim(q_meta.shape[1], 0)
-        if (not sq or not skv or not bh or self.extern_block_mask or self.D not in (64, 128) or self.DV not in (64, 128)
+    def _kv_group_choice(self, B, H, Sq, Skv, mask_plan):
+        """Tiles whose waves share the kv axis, where this engine's graph, its mask (``mask_plan(tiles)``) and the extents
+        allow and want them: a merge the kernel knows (the proven online softmax, or no row state), no mask table, no
+        tensor read per score."""
+        if (not (B and H and Sq and Skv) or self.extern_block_mask or self.D not in (64, 128) or self.DV not in (64, 128)
                 or not (self._pipe_softmax is not None or self._pipe_elementwise)
                 or any(c.per_kv for c in self.functors.customs) or os.environ.get("AE_PREFILL_KERNEL", "")):
             return None
-        if split_kv:
-            return L.kv_group_tiles_split(sq) if self.mask_mod is None else None
-        found = L.kv_group_tiles(self.D, self.DV, bh, sq, skv, self.mask_mod is not None)
+        if self.split_kv:
+            return L.kv_group_tiles_split(Sq) if self.mask_mod is None else None
+        found = L.kv_group_tiles(self.D, self.DV, B * H, Sq, Skv, self.mask_mod is not None)
         if found is not None and self.mask_mod is not None:
-            plan = self._probe_mask(q_meta, v_meta)
             lm = self.functors.mask
-            if lm.uses_b or lm.uses_h or not (plan.mode == 1 or plan.band is not None):
+            if lm.uses_b or lm.uses_h:
+                return None
+            plan = mask_plan(found)
+            if not (plan.mode == 1 or plan.band is not None):
                 return None
         return found
+
+    def tiles_for(self, B, H, Sq, Skv):
+        """The tile configuration of a call with these extents."""
+        key = (B, H, Sq, Skv)
+        if self.tiles.kv_groups == 1 or key == self._declared:
+            return self.tiles
+        tiles = self._call_tiles.get(key)
+        if tiles is None:
+            tiles = self._call_tiles[key] = self._kv_group_choice(
+                *key, lambda found: self._plan(*key, device=None, tiles=found)) or self._base
+        return tiles
 
     # ---- tuning ------------------------------------------------------------------------
     def _tune_candidates(self):
@@ -253,14 +283,15 @@ class PrefillOp:
         tuner.store(self._tune_file, self._tune_keys, tuner.encode_tiles(best))
 
     # ---- mask --------------------------------------------------------------------------
-    def _plan(self, B, H, Sq, Skv, device):
-        key = (B, H, Sq, Skv)
+    def _plan(self, B, H, Sq, Skv, device, tiles=None):
+        tiles = tiles or self.tiles_for(B, H, Sq, Skv)
+        key = (B, H, Sq, Skv, tiles.block_m, tiles.block_n)
         plan = self._plans.get(key)
         if plan is None:
-            plan = plan_mask(self.mask_mod, self.functors.mask, B, H, Sq, Skv, self.tiles.block_m,
-                             self.tiles.block_n, elementwise=self.elementwise_mask)
+            plan = plan_mask(self.mask_mod, self.functors.mask, B, H, Sq, Skv, tiles.block_m, tiles.block_n,
+                             elementwise=self.elementwise_mask)
             self._plans[key] = plan
-        if device is not None and plan.table is not None and plan.table.device != device and self._band(plan) is None:
+        if device is not None and plan.table is not None and plan.table.device != device and self._band(plan, tiles) is None:
             plan.table = plan.table.to(device)
         return plan
 
@@ -289,59 +320,61 @@ class PrefillOp:
     # ---- kernels -------------------------------------------------------------------------
     COMBINE_THREADS = 128
 
-    def plan_splits(self, B, Hq, Sq, Skv):
+    def plan_splits(self, B, Hq, Sq, Skv, tiles=None):
         """(number of KV splits, kv positions per split): a workgroup for every CU of the chip (more splits cost
         more in partial results and their merge than they gain: B1 H32 Sq128 Skv8192, the shape of
         attn_script/mha_inference.py, 43 us with 8 splits, 44 with 16, 75 with 32), whole kv tiles per split, no
         empty split."""
         if not self.split_kv:
             return 1, Skv
-        bn = self.tiles.block_n
+        tiles = tiles or self.tiles_for(B, Hq, Sq, Skv)
+        bn = tiles.block_n
         kv_tiles = -(-Skv // bn)
-        wgs = -(-Sq // self.tiles.block_m) * (-(-(B * Hq) // 8) * 8)
+        wgs = -(-Sq // tiles.block_m) * (-(-(B * Hq) // 8) * 8)
         want = max(1, min(kv_tiles, -(-self.target_workgroups // wgs)))
         per = -(-kv_tiles // want)
         return -(-kv_tiles // per), per * bn
 
-    def _kv_custom_scratch(self) -> int:
+    def _kv_custom_scratch(self, tiles) -> int:
         """LDS a launch needs beyond its K / V stages: the direct-to-LDS kernel redistributes the tiles of custom
         inputs with a kv dimension (fetched in a coalesced layout) through 2560 bytes per wave and 32-row block
         (AE_KV_SCRATCH of ae_prefill.hip; its builds with two waves per SIMD)."""
-        if (self.tiles.template != "ae_prefill.hip" or self.tiles.waves_per_eu < 2
+        if (tiles.template != "ae_prefill.hip" or tiles.waves_per_eu < 2
                 or not any(c.per_kv for c in self.functors.customs)):
             return 0
-        return self.tiles.n_waves * (self.tiles.rows_per_wave // 32) * 2560
+        return tiles.n_waves * (tiles.rows_per_wave // 32) * 2560
 
-    def _clock_stamps(self):
+    def _clock_stamps(self, tiles):
         """AE_CLOCK_STAMPS=1 (a measurement switch, read by ``bench.py --mfma-probe``): the pipelined kernel is
         built so that every workgroup reports the shader-clock cycles and the 100 MHz ticks it ran for; the
         pairs of the last launch are kept on ``self.clock_stamps`` (int64 [workgroups, 2])."""
-        return os.environ.get("AE_CLOCK_STAMPS", "") == "1" and self.tiles.template == "ae_prefill_pipe.hip"
+        return os.environ.get("AE_CLOCK_STAMPS", "") == "1" and tiles.template == "ae_prefill_pipe.hip"
 
-    def _table_rows(self, mask_block_m):
+    def _table_rows(self, mask_block_m, tiles):
         """Block-table rows a q tile spans (1, 2, 4 or 8): the kernels keep that many pairs of 64-bit masks."""
         if not mask_block_m:
             return 1
-        rows = max(1, -(-self.tiles.block_m // int(mask_block_m)))
+        rows = max(1, -(-tiles.block_m // int(mask_block_m)))
         return next(r for r in (1, 2, 4, 8) if r >= min(rows, 8))
 
-    def _band(self, plan):
+    def _band(self, plan, tiles):
         """The mask's band (MaskPlan.band) where the kernel takes one instead of the tile table."""
-        return plan.band if self.tiles.template == "ae_prefill.hip" else None
+        return plan.band if tiles.template == "ae_prefill.hip" else None
 
-    def _variant(self, mask_mode, even_q, even_kv, n_split=1, table_rows=1, heavy_last=False, band=None):
+    def _variant(self, tiles, mask_mode, Sq, Skv, n_split=1, table_rows=1, heavy_last=False, band=None):
+        even_q, even_kv = Sq % tiles.block_m == 0, Skv % tiles.block_n == 0
         if mask_mode != 2 or band is not None:
             table_rows = 1
         if mask_mode != 2:
             heavy_last = False
-        key = (mask_mode, even_q, even_kv, n_split, table_rows, bool(heavy_last), band)
+        key = (mask_mode, even_q, even_kv, n_split, table_rows, bool(heavy_last), band, astuple(tiles))
         v = self._variants.get(key)
         if v is None:
             has_mask_mod = self.elementwise_mask and mask_mode != 1
-            cfg_src = L.render_config(self.D, self.DV_launch, self.dtype, self.tiles, mask_mode, has_mask_mod,
+            cfg_src = L.render_config(self.D, self.DV_launch, self.dtype, tiles, mask_mode, has_mask_mod,
                                       self.n_rowscales, self.functors.o_scale_one, even_q, even_kv,
-                                      self._pipe_softmax if (self.tiles.rows_per_wave == 64 or self.tiles.kv_groups > 1) else None,
-                                      elementwise=self._pipe_elementwise and self.tiles.rows_per_wave == 64,
+                                      self._pipe_softmax if (tiles.rows_per_wave == 64 or tiles.kv_groups > 1) else None,
+                                      elementwise=self._pipe_elementwise and tiles.rows_per_wave == 64,
                                       exact_scale=self.exact_scale)
             if self.mask_value_zero:
                 cfg_src += "#define AE_MASK_VALUE_ZERO 1\n"
@@ -357,16 +390,16 @@ class PrefillOp:
                             f"#define AE_BAND_HI {'0x7fffffff' if band[1] is None else f'({band[1]})'}\n")
             if n_split > 1:
                 cfg_src += f"#define AE_NSPLIT {n_split}\n#define AE_COMBINE_THREADS {self.COMBINE_THREADS}\n"
-            if self._clock_stamps():
+            if self._clock_stamps(tiles):
                 cfg_src += "#define AE_CLOCK_STAMPS 1\n"
-            module = rt.compile_module(self.tiles.template, {"ae_config.h": cfg_src,
+            module = rt.compile_module(tiles.template, {"ae_config.h": cfg_src,
                                                           "ae_functors.h": self.functor_src},
                                        allow_spills=self.allow_spills,
                                        # the builds in which a spilled tuple came back wrong: 256 accumulator registers
-                                       strict_spills=self.tiles.template == "ae_prefill.hip" and self.DV_launch > 256)
-            cfg = rt.TileCfg(block_m=self.tiles.block_m, block_n=self.tiles.block_n,
-                             threads=self.tiles.threads,
-                             lds_bytes=self.tiles.lds_bytes(self.D, self.DV_launch) + self._kv_custom_scratch(), head_dim=self.D,
+                                       strict_spills=tiles.template == "ae_prefill.hip" and self.DV_launch > 256)
+            cfg = rt.TileCfg(block_m=tiles.block_m, block_n=tiles.block_n,
+                             threads=tiles.threads,
+                             lds_bytes=tiles.lds_bytes(self.D, self.DV_launch) + self._kv_custom_scratch(tiles), head_dim=self.D,
                              head_dim_v=self.DV_launch, elem_bytes=2, n_rowscales=self.n_rowscales,
                              mask_mode=mask_mode if band is None else 1,      # (a band is analytic: no table comes with the call)
                              table_rows=table_rows if mask_mode == 2 and band is None else 0)
@@ -436,13 +469,15 @@ class PrefillOp:
             # call, attn_engine.py:391-392 of the reference): the tile-class table planned from the same
             # mask_mod says the same at the kernel's own tile granularity, whatever infer_mask_block_M/N are
             extern_mask = None
+        tiles = self.tiles_for(B, Hq, Sq, Skv)
         if extern_mask is not None:
+            tiles = self._table_tiles
             bm, bn = self.mask_block
-            if bn % self.tiles.block_n or (self.tiles.block_m % bm and bm % self.tiles.block_m) or \
-                    self.tiles.block_m > self.MASK_ROWS_PER_TILE * bm:
+            if bn % tiles.block_n or (tiles.block_m % bm and bm % tiles.block_m) or \
+                    tiles.block_m > self.MASK_ROWS_PER_TILE * bm:
                 raise NotImplementedError(
-                    f"a block mask of {bm}x{bn} blocks does not fit the kernel's {self.tiles.block_m}x"
-                    f"{self.tiles.block_n} tiles (construct the engine with extern_block_mask=True)")
+                    f"a block mask of {bm}x{bn} blocks does not fit the kernel's {tiles.block_m}x"
+                    f"{tiles.block_n} tiles (construct the engine with extern_block_mask=True)")
             table = extern_mask
             if table.dim() != 4:
                 raise ValueError("block_mask must be [B|1, H|1, Sq/bm, Skv/bn]")
@@ -451,18 +486,10 @@ class PrefillOp:
             table = table.to(dev).contiguous()
             mode, mbm, mbn, band = 2, bm, bn, None
         else:
-            plan = self._plan(B, Hq, Sq, Skv, dev)
-            mode, table, mbm, mbn, band = plan.mode, plan.table, plan.block_m, plan.block_n, self._band(plan)
-        if mode == 2 and band is None and self.tiles.kv_groups > 1:
-            # (a shape other than the declared one whose mask needs a table, or a block mask of the caller's)
-            self.tiles = L.PrefillTiles()
-            self._variants.clear()
-            self._plans.clear()
-            self._host.clear()
-            return self._forward_once(q, k, v, *extra, *(() if extern_mask is None else (extern_mask,)))
-        n_split, kv_per_split = self.plan_splits(B, Hq, Sq, Skv)
-        module, cfg, _ = self._variant(mode, Sq % self.tiles.block_m == 0, Skv % self.tiles.block_n == 0, n_split,
-                                       self._table_rows(mbm) if mode == 2 else 1,
+            plan = self._plan(B, Hq, Sq, Skv, dev, tiles)
+            mode, table, mbm, mbn, band = plan.mode, plan.table, plan.block_m, plan.block_n, self._band(plan, tiles)
+        n_split, kv_per_split = self.plan_splits(B, Hq, Sq, Skv, tiles)
+        module, cfg, _ = self._variant(tiles, mode, Sq, Skv, n_split, self._table_rows(mbm, tiles) if mode == 2 else 1,
                                        extern_mask is None and plan.heavy_last, band)
         kern = module.kernel("ae_prefill_kernel")
 
@@ -499,8 +526,8 @@ class PrefillOp:
                               n_rowscales=self.n_rowscales, mask_mode=0)
             rt.prefill_split_fwd(kern, module.kernel("ae_decode_combine_kernel"), p, cfg, ccfg, stream)
         else:
-            if self._clock_stamps():
-                n_wg = -(-Sq // self.tiles.block_m) * (-(-(B * Hq) // 8) * 8)
+            if self._clock_stamps(tiles):
+                n_wg = -(-Sq // tiles.block_m) * (-(-(B * Hq) // 8) * 8)
                 self.clock_stamps = torch.zeros((n_wg, 2), dtype=torch.int64, device=dev)
                 p.partial_o = self.clock_stamps.data_ptr()
             # one launch per slice of DV_launch value columns (a single one unless DV > 256)
@@ -511,7 +538,7 @@ class PrefillOp:
                 rt.prefill_fwd(kern, p, cfg, stream)
         self.final_rowscales = dict(zip(self.functors.final_rowscale_names, rowscales))
         self._keepalive = keep
-        if extern_mask is None and self.DV_launch == self.DV and not self._clock_stamps():
+        if extern_mask is None and self.DV_launch == self.DV and not self._clock_stamps(tiles):
             host.add_forward(self._host, host.PREFILL_SPLIT if n_split > 1 else host.PREFILL, B, Sq, Hq, Hkv, Skv, dev, module,
                              kern, cfg, combine=module.kernel("ae_decode_combine_kernel") if n_split > 1 else None,
                              ccfg=ccfg if n_split > 1 else None, n_split=n_split, kv_per_split=kv_per_split,

@@ -108,3 +108,55 @@ def test_a_nan_reaches_every_row_that_sees_it(cuda_device, tiles, what, causal):
     assert torch.isnan(out[:, sees]).all()
     if causal and what != "value":                                # (0 * NaN: a masked key's value still spoils its tile)
         assert (out[:, ~sees] - ref[:, ~sees]).abs().max().item() <= 2e-2
+
+
+def _engine(S, mask, split=False, H=32, Hkv=8, D=128, B=1, Skv=None, dtype=torch.bfloat16):
+    meta = (meta_tensor(B, H, S, D, dtype=dtype),) + (meta_tensor(B, Hkv, Skv or S, D, dtype=dtype),) * 2
+    return AttentionEngine(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), mask, C.OnlineSoftmax())
+
+
+def test_the_tiles_follow_the_shape_of_the_call():
+    """An engine declared for a short prompt keeps nothing of it at other lengths; one declared large does not change."""
+    op = _engine(333, C.causal_mask)._op
+    assert op.tiles == TILES[1] and op.tiles_for(1, 32, 333, 333) == TILES[1]
+    assert op.tiles_for(1, 32, 4096, 4096) == PrefillTiles() == op.tiles_for(8, 32, 333, 333)
+    assert op.tiles_for(1, 32, 1000, 1000) == kv_group_tiles(128, 128, 32, 1000, 1000, True) == TILES[2]
+    assert op._plan(1, 32, 4096, 4096, None).block_m == 128 and op.tiles == TILES[1]
+    # no table reaches the tiles that share the kv axis: a mask that is a band at the declared length only
+    odd = _engine(333, lambda b, h, q, kv: (q >= kv) & ((q < 400) | (kv % 2 == 0)))._op
+    assert odd.tiles == TILES[1] and odd.tiles_for(1, 32, 500, 500) == PrefillTiles()
+    large = _engine(4096, C.causal_mask, H=16)._op
+    assert large.tiles.kv_groups == 1 and large.tiles_for(1, 16, 100, 100) == large.tiles
+    few = _engine(8, None, H=8, Hkv=8, Skv=4096)._op
+    assert few.split_kv and few.tiles == TILES[0] and few.tiles_for(1, 8, 64, 4096) == TILES[2]
+    assert few.tiles_for(1, 8, 128, 4096) == PrefillTiles() and few.plan_splits(1, 8, 128, 4096)[1] % 64 == 0
+
+
+@pytest.mark.gpu
+def test_an_engine_for_short_prompts_at_other_lengths(cuda_device):
+    H, Hkv, D = 32, 8, 128
+    mod = _engine(333, C.causal_mask)
+    op = mod._op
+
+    def check(S, B=1):
+        print(f"case B{B} S{S}", flush=True)
+        q, k, v = C.make_inputs(B, S, S, H, Hkv, D, D, torch.bfloat16, seed=S)
+        ref, rlse = R.softmax_attention(q, k, v, causal=True)
+        for _ in range(2):                       # through Python, then natively
+            out = mod(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+            assert (out - ref).abs().max().item() <= 2e-2
+            assert (mod.final_rowscales["lse"].cpu() - rlse).abs().max().item() <= 1e-3
+    for S, B in ((333, 1), (1100, 1), (333, 4), (70, 1), (333, 1)):
+        check(S, B)
+    built = {src.count("#define AE_KW ") for _, _, src in op._variants.values()}
+    assert built == {0, 1} and op.tiles == TILES[1]
+    # a block mask of the caller's, once: it takes the tiles that read tables, the declared shape keeps its own
+    q, k, v = C.make_inputs(1, 333, 333, H, Hkv, D, D, torch.bfloat16, seed=1)
+    blocks = torch.zeros(1, 1, 3, 3, dtype=torch.int8)
+    blocks[..., 0] = 1
+    out = mod(q.cuda(), k.cuda(), v.cuda(), blocks.cuda()).float().cpu()
+    ref, _ = R.softmax_attention(q, k, v, causal=False, mask=torch.from_numpy(
+        OM.dense_mask_grid(lambda b, h, qi, ki: (qi >= ki) & (ki < 128), 1, H, 333, 333)))
+    assert (out - ref).abs().max().item() <= 2e-2
+    assert op.tiles == TILES[1]
+    check(333)
