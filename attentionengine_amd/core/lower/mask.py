@@ -125,22 +125,38 @@ class MaskPlan:
             self.heavy_last = bool(work[-third:].mean() >= 1.25 * work[:third].mean())
 
 
-def plan_mask(mask_mod, lowered: LoweredMask, B: int, H: int, Sq: int, Skv: int, tile_m: int,
-              tile_n: int, elementwise: bool = True, chunk_rows: int = 4096) -> MaskPlan:
-    """Classify the mask on the host.  The mask is evaluated with batch/head extent 1 when the
-    traced graph does not read b / h, and in row chunks so the full [Sq, Skv] grid is never
-    resident at once."""
-    if mask_mod is None:
-        return MaskPlan(0)
+class MaskSurvey:
+    """A mask evaluated once over the whole [Sq, Skv] grid, in blocks of ``step_m`` x ``step_n`` positions that tables of
+    any coarser tile are put together from (``table``)."""
+
+    def __init__(self, classes, causal, band, Sq, Skv, step_m, step_n):
+        self.classes = classes        # int8 [b|1, h|1, blocks, blocks]: 0 empty, 1 partly, 2 fully visible
+        self.causal = causal          # exactly q_idx >= kv_idx, over equal lengths
+        self.band = band              # see MaskPlan; None for masks that read b or h
+        self.Sq, self.Skv, self.step_m, self.step_n = Sq, Skv, step_m, step_n
+
+    def table(self, tile_m, tile_n):
+        """int8 [b|1, h|1, n_q_tiles, n_kv_tiles] (see MaskPlan)."""
+        c = self.classes
+        rm, rn = tile_m // self.step_m, tile_n // self.step_n
+        if (rm, rn) == (1, 1):
+            return c
+        some, every = (c > 0), (c == 2)
+        for dim, r in ((3, rn), (2, rm)):
+            some, every = _blocks(some, dim, r, torch.any), _blocks(every, dim, r, torch.all)
+        return some.to(torch.int8) + every.to(torch.int8)
+
+
+def survey_mask(mask_mod, lowered: LoweredMask, B: int, H: int, Sq: int, Skv: int, step_m: int = 32, step_n: int = 32,
+                chunk_rows: int = 4096) -> MaskSurvey:
+    """Evaluates the mask on the host: with batch/head extent 1 when the traced graph does not read b / h, and in row
+    chunks so the full [Sq, Skv] grid is never resident at once."""
     mb = B if lowered.uses_b else 1
     mh = H if lowered.uses_h else 1
-    n_qt = (Sq + tile_m - 1) // tile_m
-    n_kt = (Skv + tile_n - 1) // tile_n
-    table = torch.zeros(mb, mh, n_qt, n_kt, dtype=torch.int8)
-    exactly_causal = True
-    band = (mb, mh) == (1, 1) and elementwise
+    parts = []
+    causal, one = True, (mb, mh) == (1, 1)
     d_lo, d_hi, seen = Sq + Skv, -(Sq + Skv), 0       # extremes of q - kv over the visible positions, and their number
-    chunk_rows = max(tile_m, (chunk_rows // tile_m) * tile_m)
+    chunk_rows = max(step_m, (chunk_rows // step_m) * step_m)
     kv = torch.arange(Skv).view(1, 1, 1, Skv)
     bb = torch.arange(mb).view(mb, 1, 1, 1)
     hh = torch.arange(mh).view(1, mh, 1, 1)
@@ -151,9 +167,12 @@ def plan_mask(mask_mod, lowered: LoweredMask, B: int, H: int, Sq: int, Skv: int,
         if not isinstance(m, torch.Tensor):
             m = torch.tensor(bool(m))
         m = m.to(torch.bool).expand(mb, mh, r1 - r0, Skv)
-        if exactly_causal:
-            exactly_causal = bool(torch.equal(m, (q >= kv).expand_as(m)))
-        if band:
+        here = (causal or one) and bool(torch.equal(m, (q >= kv).expand_as(m)))
+        causal = causal and here
+        if one and here:              # (the extremes and the number of a causal chunk are known)
+            d_lo, d_hi = min(d_lo, max(0, r0 - Skv + 1)), max(d_hi, r1 - 1)
+            seen += int(torch.arange(r0 + 1, r1 + 1).clamp(max=Skv).sum())
+        elif one:
             rows = m[0, 0]
             any_row = rows.any(dim=1)
             if bool(any_row.any()):
@@ -163,22 +182,31 @@ def plan_mask(mask_mod, lowered: LoweredMask, B: int, H: int, Sq: int, Skv: int,
                 d_lo, d_hi = min(d_lo, int((qr - last).min())), max(d_hi, int((qr - first).max()))
             seen += int(rows.sum())
         # a block cut by the sequence end is "full" when every in-range element is visible
-        vis = _count_blocks(m, tile_m, tile_n)
-        tot = _count_blocks(torch.ones(1, 1, r1 - r0, Skv, dtype=torch.bool), tile_m, tile_n)
-        full = ((vis == tot) & (vis > 0)).to(torch.int8)
-        partial = ((vis > 0) & (vis < tot)).to(torch.int8)
-        cls = partial + 2 * full
-        t0 = r0 // tile_m
-        table[:, :, t0:t0 + cls.shape[2], :] = cls
-    if exactly_causal and Sq == Skv and elementwise:
+        some = _blocks(_blocks(m, 3, step_n, torch.any), 2, step_m, torch.any)
+        every = _blocks(_blocks(m, 3, step_n, torch.all), 2, step_m, torch.all)
+        parts.append(some.to(torch.int8) + every.to(torch.int8))
+    band = None
+    if one and seen and seen == band_size(Sq, Skv, d_lo, d_hi):
+        band = (d_lo, None if d_hi >= Sq - 1 else d_hi)
+    return MaskSurvey(torch.cat(parts, dim=2), causal and Sq == Skv, band, Sq, Skv, step_m, step_n)
+
+
+def plan_mask(mask_mod, lowered: LoweredMask, B: int, H: int, Sq: int, Skv: int, tile_m: int,
+              tile_n: int, elementwise: bool = True, chunk_rows: int = 4096, survey=None) -> MaskPlan:
+    """Classify the mask on the host for tiles of ``tile_m`` x ``tile_n`` positions, from a ``survey`` of the same mask
+    and extents if there is one."""
+    if mask_mod is None:
+        return MaskPlan(0)
+    if survey is None or tile_m % survey.step_m or tile_n % survey.step_n:
+        survey = survey_mask(mask_mod, lowered, B, H, Sq, Skv, tile_m, tile_n, chunk_rows)
+    if survey.causal and elementwise:
         return MaskPlan(1, None, tile_m, tile_n, True)
+    table = survey.table(tile_m, tile_n)
     if not elementwise:
         # mask_value != "-inf": the forward only skips tiles (attn_tl.py:124-137 guards the
         # elementwise test with is_inf_mask); visited tiles are treated as fully visible.
         table = torch.where(table > 0, torch.full_like(table, 2), table)
-    if band and seen and seen == band_size(Sq, Skv, d_lo, d_hi):
-        return MaskPlan(2, table.contiguous(), tile_m, tile_n, elementwise, (d_lo, None if d_hi >= Sq - 1 else d_hi))
-    return MaskPlan(2, table.contiguous(), tile_m, tile_n, elementwise)
+    return MaskPlan(2, table.contiguous(), tile_m, tile_n, elementwise, survey.band if elementwise else None)
 
 
 def band_size(Sq: int, Skv: int, lo: int, hi: int) -> int:
@@ -188,10 +216,15 @@ def band_size(Sq: int, Skv: int, lo: int, hi: int) -> int:
     return int(((q - lo).clamp(max=Skv - 1) - (q - hi).clamp(min=0) + 1).clamp(min=0).sum())
 
 
-def _count_blocks(mask: torch.Tensor, bm: int, bn: int) -> torch.Tensor:
-    """Number of True elements per (bm x bn) block of a bool [B,H,Q,KV] tensor (zero padded)."""
-    B, H, Q, KV = mask.shape
-    Qp, KVp = (Q + bm - 1) // bm * bm, (KV + bn - 1) // bn * bn
-    if (Qp, KVp) != (Q, KV):
-        mask = torch.nn.functional.pad(mask, (0, KVp - KV, 0, Qp - Q))
-    return mask.reshape(B, H, Qp // bm, bm, KVp // bn, bn).sum(dim=(3, 5), dtype=torch.int64)
+def _blocks(x: torch.Tensor, dim: int, n: int, reduce) -> torch.Tensor:
+    """``reduce`` (torch.any / torch.all) over runs of n elements of dimension ``dim``; a last run that the end cuts is
+    reduced over what it has."""
+    if n == 1:
+        return x
+    whole = x.shape[dim] // n * n
+    parts = []
+    if whole:
+        parts.append(reduce(x.narrow(dim, 0, whole).unflatten(dim, (whole // n, n)), dim=dim + 1))
+    if whole < x.shape[dim]:
+        parts.append(reduce(x.narrow(dim, whole, x.shape[dim] - whole), dim=dim, keepdim=True))
+    return parts[0] if len(parts) == 1 else torch.cat(parts, dim=dim)

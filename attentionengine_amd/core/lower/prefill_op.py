@@ -18,7 +18,7 @@ from ..runtime import host
 from ..transform.core import _convert_mask_to_block_mask, is_causal_mask
 from . import lower as L
 from .lower_decode import combine_rows
-from .mask import plan_mask
+from .mask import plan_mask, survey_mask
 
 
 def _dim(x, default):
@@ -63,7 +63,7 @@ class PrefillOp:
                        and not split_kv)
         if self.DV > 256 and not single_pass:
             self.DV_launch = next(c for c in (256, 192, 128, 96, 64, 32) if self.DV % c == 0)
-        self.mask_mod, self._probed = mask_mod, None
+        self.mask_mod, self._probed, self._surveys = mask_mod, None, {}
         self.elementwise_mask = mask_mod is not None and mask_value == "-inf"
         self.mask_value_zero = mask_value == "0"
         self.extern_block_mask = bool(extern_block_mask)
@@ -219,8 +219,19 @@ class PrefillOp:
         if self._probed is None:
             sq, skv = _dim(q_meta.shape[2], 4096), _dim(v_meta.shape[2], 4096)
             self._probed = plan_mask(self.mask_mod, self.functors.mask, 1, 1, sq, skv, 128, 64,
-                                     elementwise=self.elementwise_mask)
+                                     elementwise=self.elementwise_mask, survey=self._mask_survey(1, 1, sq, skv))
         return self._probed
+
+    def _mask_survey(self, B, H, Sq, Skv):
+        """The mask evaluated at these extents: once for all tile shapes that are tried there (the last few are kept)."""
+        lm = self.functors.mask
+        key = (B if lm.uses_b else 1, H if lm.uses_h else 1, Sq, Skv)
+        found = self._surveys.get(key)
+        if found is None:
+            if len(self._surveys) >= 4:
+                self._surveys.pop(next(iter(self._surveys)))
+            found = self._surveys[key] = survey_mask(self.mask_mod, lm, B, H, Sq, Skv)
+        return found
 
     def _kv_group_choice(self, B, H, Sq, Skv, mask_plan):
         """Tiles whose waves share the kv axis, where this engine's graph, its mask (``mask_plan(tiles)``) and the extents
@@ -289,7 +300,8 @@ class PrefillOp:
         plan = self._plans.get(key)
         if plan is None:
             plan = plan_mask(self.mask_mod, self.functors.mask, B, H, Sq, Skv, tiles.block_m, tiles.block_n,
-                             elementwise=self.elementwise_mask)
+                             elementwise=self.elementwise_mask,
+                             survey=self._mask_survey(B, H, Sq, Skv) if self.mask_mod is not None else None)
             self._plans[key] = plan
         if device is not None and plan.table is not None and plan.table.device != device and self._band(plan, tiles) is None:
             plan.table = plan.table.to(device)

@@ -9,7 +9,7 @@ import attn_cases as C
 from attn_engine import AttentionEngine
 from core import CustomIO, meta_tensor
 from core.lower.lower_decode import merges_in_any_order
-from core.lower.mask import lower_mask_mod, plan_mask
+from core.lower.mask import lower_mask_mod, plan_mask, survey_mask
 from oracle import attention_ref as R
 from oracle import masks as OM
 
@@ -68,3 +68,42 @@ def test_banded_masks_against_the_oracle(cuda_device, name, Sq, Skv, D):
     seen = torch.isfinite(rlse)
     assert (out[b] - ref.nan_to_num(0.0)).abs().max().item() <= 2e-2
     assert torch.equal(torch.isfinite(lse[b]), seen) and (lse[b][seen] - rlse[seen]).abs().max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("Sq,Skv", [(1, 1), (31, 33), (300, 300), (130, 517), (517, 130), (256, 64)])
+@pytest.mark.parametrize("name", ["causal", "plus_one", "window", "head", "holes", "all", "none"])
+def test_tables_put_together_from_one_survey(name, Sq, Skv):
+    """One evaluation of a mask serves every tile shape: the tables are the oracle's, and band and mode do not depend on
+    how it was cut into rows and blocks."""
+    mod = {"causal": C.causal_mask, "plus_one": C.causal_plus_one_mask, "window": C.make_sliding_window_mask(70),
+           "head": C.head_dependent_mask, "holes": lambda b, h, q, kv: (q >= kv) & (kv % 40 != 5),
+           "all": lambda b, h, q, kv: q + kv >= 0, "none": lambda b, h, q, kv: q + kv < 0}[name]
+    lm = lower_mask_mod(mod)
+    survey = survey_mask(mod, lm, 2, 3, Sq, Skv, chunk_rows=64)
+    dense = OM.dense_mask_grid(mod, 2 if lm.uses_b else 1, 3 if lm.uses_h else 1, Sq, Skv)
+    for tm, tn in ((32, 32), (64, 32), (128, 32), (128, 64), (256, 64), (64, 128)):
+        plan = plan_mask(mod, lm, 2, 3, Sq, Skv, tm, tn, survey=survey)
+        alone = plan_mask(mod, lm, 2, 3, Sq, Skv, tm, tn)
+        assert (plan.mode, plan.band) == (alone.mode, alone.band)
+        assert (plan.mode == 1) == (Sq == Skv and bool((torch.from_numpy(dense)[0, 0] == torch.ones(Sq, Skv).tril().bool()).all()))
+        if plan.mode == 2:
+            assert torch.equal(plan.table, alone.table)
+            assert torch.equal(plan.table, torch.from_numpy(OM.block_classes(dense, tm, tn)).to(torch.int8))
+        if plan.band is not None:
+            lo, hi = plan.band
+            d = torch.arange(Sq).view(-1, 1) - torch.arange(Skv).view(1, -1)
+            assert torch.equal((d >= lo) & (d <= (Sq if hi is None else hi)), torch.from_numpy(dense)[0, 0])
+
+
+def test_construction_evaluates_a_mask_once(monkeypatch):
+    """... whatever tiles are tried on the way (bands, waves that share the kv axis)."""
+    from core.lower import mask
+    seen = []
+    real = mask.survey_mask
+    monkeypatch.setattr("core.lower.prefill_op.survey_mask", lambda *a, **k: seen.append(a[4:6]) or real(*a, **k))
+    monkeypatch.setattr(mask, "survey_mask", lambda *a, **k: seen.append(a[4:6]) or real(*a, **k))
+    for mod, S in ((C.causal_mask, 333), (C.causal_mask, 4096), (C.make_sliding_window_mask(256), 4096)):
+        seen.clear()
+        AttentionEngine((meta_tensor(1, 32, S, 128, dtype=torch.float16),) * 3, CustomIO({}), C.make_scale_score_mod(0.1), mod,
+                        C.OnlineSoftmax())
+        assert seen == [(S, S)]
