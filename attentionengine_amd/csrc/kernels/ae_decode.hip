@@ -296,7 +296,6 @@ void ae_decode_split_kernel(const ae_attn_params p) {
     __amdgpu_buffer_rsrc_t po_buf = __builtin_amdgcn_make_buffer_rsrc(
         p.partial_o + tile_row0 * AE_DV, 0, tile_heads * AE_NSPLIT * AE_DV * 4, 0x00020000);
 #endif
-    const bool no_keys = wg_base >= p.seqlen_kv;        // (else the workgroup's first wave has some)
     for (int idx = tid; idx < tile_heads * (AE_DV / 4); idx += AE_NT) {
       const int hl = idx / (AE_DV / 4), dv = (idx % (AE_DV / 4)) * 4;
       float rs[AE_NWAVES];
@@ -306,19 +305,19 @@ void ae_decode_split_kernel(const ae_attn_params p) {
       float w[AE_NWAVES];
 #pragma unroll
       for (int k = 0; k < AE_NWAVES; k++) w[k] = ae_exp(rs[k] - top);
-      float merged = ae_log(ae_arr_sum<AE_NWAVES>(w)) + top;
+      // a workgroup without keys, or whose scores are all -inf: -inf - -inf would make it NaN, its partial result weighs
+      // nothing in the merge that follows (a wave's NaN stays one)
+      const bool some = top > AE_NEG_INF;
+      const float merged = some ? ae_log(ae_arr_sum<AE_NWAVES>(w)) + top : ae_arr_sum<AE_NWAVES>(rs);
+      const float ref = some ? merged : 0.f;
       ae_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < AE_NWAVES; k++) {
         const ae_f32x4 v = *(__attribute__((address_space(3))) ae_f32x4*)(
             (__attribute__((address_space(3))) float*)((ae_lds_byte*)ae_smem + k * AE_V_WAVE_BYTES) + hl * AE_DV + dv);
-        const float wk = ae_exp(rs[k] - merged);
+        const float wk = ae_exp(rs[k] - ref);
 #pragma unroll
         for (int r = 0; r < 4; r++) acc[r] += v[r] * wk;
-      }
-      if (no_keys) {
-        acc = (ae_f32x4){0.f, 0.f, 0.f, 0.f};
-        merged = AE_NEG_INF;
       }
       const int row_in_tile = hl * AE_NSPLIT + blockIdx.x;
 #if AE_MERGE_LAST

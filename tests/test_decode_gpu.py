@@ -577,3 +577,31 @@ def test_decode_and_prefill_replay_from_a_hip_graph(cuda_device):
         assert torch.equal(got_p, ref_p), step
     ref, _ = R.softmax_attention(q.cpu(), k.cpu(), v.cpu(), causal=False)
     assert (got_d.float().cpu() - ref).abs().max().item() <= OUT_TOL
+
+
+@pytest.mark.parametrize("Skv,used", [(3001, 700), (8192, 33), (3001, 3001)])
+@pytest.mark.parametrize("merge_last", ["1", "0"])
+def test_a_workgroup_whose_keys_are_all_masked_adds_nothing(cuda_device, monkeypatch, Skv, used, merge_last):
+    """A score_mod that gives every key past the first ``used`` a score of -inf, with the guarded division of
+    attn_script/sparseattn.py:68: whole workgroups see nothing else, and the partial results that their waves merge first
+    must weigh nothing in the merge over the workgroups."""
+    monkeypatch.setenv("AE_DECODE_MERGE_LAST", merge_last)
+    B, Hq, Hkv, D, dtype = 1, 8, 2, 128, torch.float16
+
+    class Guarded(C.OnlineSoftmax):
+        @staticmethod
+        def online_fwd_epilogue(o, online_rowscales, b, h, q_idx):
+            return o / (online_rowscales["r"] + 1e-20), {"lse": online_rowscales["r"].log() + online_rowscales["m"]}
+
+    def score_mod(score, custom_fwd_inputs, b, h, q_idx, kv_idx):
+        return score * (1 / math.sqrt(D)) - (kv_idx - (used - 1)).max(0) * 1e37 * 100.0      # (1e39 a key: -inf)
+    meta = (meta_tensor(B, Hq, 1, D, dtype=dtype),) + (meta_tensor(B, Hkv, Skv, D, dtype=dtype),) * 2
+    mod = AttentionEngine(meta, CustomIO({}), score_mod, None, Guarded())
+    op = mod.attention
+    assert op.grouped_merge and op.plan_splits(B, Hq, Hkv, Skv)[0] > op.N_WAVES
+    q, k, v = C.make_inputs(B, 1, Skv, Hq, Hkv, D, D, dtype, seed=used)
+    ref, rlse = R.softmax_attention(q, k[:, :used], v[:, :used], causal=False)
+    for _ in range(2):
+        out = mod(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+        assert torch.isfinite(out).all() and (out - ref).abs().max().item() <= 2e-2
+        assert (mod.final_rowscales["lse"].cpu().view(-1) - rlse.view(-1)).abs().max().item() <= 1e-3
