@@ -8,6 +8,7 @@ import torch
 import attn_cases as C
 from attn_engine import AttentionEngine
 from core import CustomIO, meta_tensor
+from oracle import attention_ref as R
 
 pytestmark = pytest.mark.gpu
 
@@ -93,3 +94,44 @@ def test_the_weight_of_a_zero_score_may_overflow_the_input_type(cuda_device, mon
     out = mod(q.cuda(), k.cuda(), v.cuda(), torch.tensor([70000.0], device="cuda")).double().cpu()
     ref = 4464.0 * v.double().sum(dim=1, keepdim=True).expand_as(out)      # (4464 is a value of fp16: the weights are exact)
     assert ((out - ref).abs() <= 2.0 ** -10 * ref.abs() + 1e-3).all()
+
+
+def _softmax_engine(monkeypatch, kernel, S, D, dtype, mask=None):
+    monkeypatch.setenv("AE_PREFILL_KERNEL", KERNELS[kernel])
+    meta = (meta_tensor(1, 2, S, D, dtype=dtype),) * 3
+    mod = AttentionEngine(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), mask, C.OnlineSoftmax())
+    assert (mod._op.tiles.kv_groups > 1) == (kernel == "groups")
+    assert (mod._op.tiles.rows_per_wave == 64) == (kernel == "pipelined")
+    return mod
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("kl,vl", [("own", "expanded"), ("expanded", "own"), ("near", "near")])
+def test_rows_may_overlap_under_the_softmax(cuda_device, monkeypatch, kernel, causal, kl, vl):
+    S, D, dtype = 130, 128, torch.float16
+    mod = _softmax_engine(monkeypatch, kernel, S, D, dtype, C.causal_mask if causal else None)
+    q, k, v = (t.cuda() for t in C.make_inputs(1, S, S, 2, 2, D, D, dtype, seed=15))
+    k, v = _layout(k, kl), _layout(v, vl)
+    ref, rlse = R.softmax_attention(q.cpu(), k.cpu(), v.cpu(), causal=causal)
+    for _ in range(2):
+        out = mod(q, k, v).float().cpu()
+        assert (out - ref).abs().max().item() <= 2e-2
+        assert (mod.final_rowscales["lse"].cpu() - rlse).abs().max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+@pytest.mark.parametrize("where", [3, 70, 129])
+@pytest.mark.parametrize("value", [math.nan, math.inf])
+@pytest.mark.parametrize("causal", [False, True])
+def test_a_key_that_is_not_finite_spoils_the_rows_that_see_it(cuda_device, monkeypatch, kernel, where, value, causal):
+    S, D, dtype = 130, 64, torch.bfloat16
+    mod = _softmax_engine(monkeypatch, kernel, S, D, dtype, C.causal_mask if causal else None)
+    q, k, v = C.make_inputs(1, S, S, 2, 2, D, D, dtype, seed=16)
+    q = q.abs() + 2 ** -6                        # (an infinite key scores +inf with every row, and inf - inf is NaN)
+    ref, _ = R.softmax_attention(q, k, v, causal=causal)
+    k[:, where], k[:, where, :, 1] = 0.0, value
+    out = mod(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+    sees = torch.arange(S) >= where if causal else torch.ones(S, dtype=torch.bool)
+    assert torch.isnan(out[:, sees]).all()
+    assert not causal or (out[:, ~sees] - ref[:, ~sees]).abs().max().item() <= 2e-2
