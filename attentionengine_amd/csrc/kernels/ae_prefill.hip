@@ -733,7 +733,9 @@ void ae_prefill_kernel(const ae_attn_params p) {
       live[k] = ae_group_max(xs[(wk + 2) * 64 + lane]) > 0.f;
       row_seen = row_seen || live[k];
       w[k] = 1.f;
-#if AE_KW_SOFTMAX
+#if !AE_KW_SOFTMAX
+      live[k] = true;      // (no row state: what a group's tiles gave is the row's, the weights of masked keys included)
+#else
       mg[k] = xs[wk * 64 + lane];
       top = live[k] ? __builtin_fmaxf(top, mg[k]) : top;
 #endif
