@@ -289,7 +289,8 @@ void ae_prefill_kernel(const ae_attn_params p) {
   // offset inside a tile never changes, so it is computed once; per tile only a wave-uniform base moves.
   // A wave's loads of a tensor's tile go out as one burst behind a single write of M0: through a buffer resource that
   // ends with the last row (ae_load_lds16_burst_rows), or, where every tile is whole, from the plain address, which
-  // saves forming the resource in the pinned slots (causal B2 H32 S4096 D128 282.7 -> 281.5 us).
+  // saves forming the resource in the pinned slots (B2 H32 S4096 D128 fp16, medians of three runs a side: sigmoid 510.9 ->
+  // 507.6 us, softmax without a mask 477.8 -> 475.1; causal no difference).
 #define AE_LOAD_COMP(i, n) (AE_EVEN_KV ? ((i) - (n) / 2) * 1024 : ((i) & 3) * 1024)
   auto k_lane_off = [&](int i) AE_LAMBDA -> unsigned {
     const int row = (wave * AE_K_LOADS + i) * AE_K_RPI + lane / AE_KCPR;
