@@ -82,6 +82,7 @@ static_assert(AE_L1 <= 8 && AE_L2 >= 1 && AE_BLOCKS >= AE_LOADS, "two bursts of 
 #define AE_OSW1 ((AE_DVW / 8) & -(AE_DVW / 8))
 #define AE_OSW (AE_OSW1 < 16 ? AE_OSW1 - 1 : 15)
 static_assert(AE_DV * AE_HEADS_PER_WG * 4 <= AE_NSTAGE * AE_STAGE_BYTES, "the results of 64 heads fit the tile stages");
+static_assert(AE_DVW % 32 == 0, "a block of 32 heads leaves in whole instructions of 64 lanes x 16 bytes");
 static_assert(AE_NSTAGE >= 3, "a tile is multiplied by K one trip before it is multiplied as V");
 
 #ifndef AE_PAGED
@@ -126,32 +127,69 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #endif
 
   // ---- which (head tile, split, kv head, batch): 1-D grid, ids 8 apart share their KV range ---------
-  const int group = p.heads_q / p.heads_kv;
-  const int n_ht = (group + AE_HEADS_PER_WG - 1) / AE_HEADS_PER_WG;
+  // (What a workgroup does before its first tile is requested is a serial chain that a short launch pays in full: the
+  // integer divisions are left out where a shift does - one latent head, a power of two of head tiles, of tokens a page.
+  // The launch is planned with AE_NSPLIT splits.)
+  int group = p.heads_q;
+  if (__builtin_expect(p.heads_kv != 1, 0)) group /= p.heads_kv;
+  const int n_ht = (int)((unsigned)(group + AE_HEADS_PER_WG - 1) / AE_HEADS_PER_WG);
   const int wg = blockIdx.x;
-  const int ht = (wg >> 3) % n_ht;
-  const int u = (wg / (8 * n_ht)) * 8 + (wg & 7);        // flattened (batch, kv head, split)
-  if (u >= p.batch * p.heads_kv * p.num_splits) return;  // grid padding (whole workgroup exits)
-  const int split = u % p.num_splits;
-  const int hk = (u / p.num_splits) % p.heads_kv;
-  const int b = u / (p.num_splits * p.heads_kv);
+  int ht, u8;
+  if (__builtin_expect((n_ht & (n_ht - 1)) != 0, 0)) {
+    ht = (wg >> 3) % n_ht;
+    u8 = (wg >> 3) / n_ht;
+  } else {
+    ht = (wg >> 3) & (n_ht - 1);
+    u8 = (wg >> 3) >> __builtin_ctz(n_ht);
+  }
+  const unsigned u = (unsigned)(u8 * 8 + (wg & 7));      // flattened (batch, kv head, split)
+  if (u >= (unsigned)(p.batch * p.heads_kv * AE_NSPLIT)) return;  // grid padding (whole workgroup exits)
+  const int split = u % AE_NSPLIT;
+  int b = u / AE_NSPLIT, hk = 0;
+  if (__builtin_expect(p.heads_kv != 1, 0)) {
+    hk = b % p.heads_kv;
+    b /= p.heads_kv;
+  }
 
+  // (wave-uniform values are pinned to scalar registers: a copy in a vector register that gets spilled is
+  // reloaded with a scratch load, which the tile loads' vmcnt bookkeeping would have to wait for)
+  const int kv_begin = __builtin_amdgcn_readfirstlane(split * p.kv_per_split);
 #if AE_PAGED
   const ae_elem* k1 = (const ae_elem*)p.k + (int64_t)hk * p.k_stride_h;
   const ae_elem* k2 = (const ae_elem*)p.k2 + (int64_t)hk * p.k2_stride_h;
   const int32_t* pages = p.block_table + (int64_t)b * p.block_table_stride;
+  const int page_size = p.page_block_size;
+  int rq_slot0, top_slot;          // table slots of the split's first token and of the last one that it could hold
+  {
+    int top = kv_begin + p.kv_per_split;
+    top = (top < p.seqlen_kv ? top : p.seqlen_kv) - 1;
+    top = top > 0 ? top : 0;
+    if (__builtin_expect((page_size & (page_size - 1)) != 0, 0)) {
+      rq_slot0 = kv_begin / page_size;
+      top_slot = top / page_size;
+    } else {
+      rq_slot0 = kv_begin >> __builtin_ctz(page_size);
+      top_slot = top >> __builtin_ctz(page_size);
+    }
+  }
+  // The entry's length and the split's first 64 table entries are requested together (one after the other they held the
+  // first tile back by another trip to memory).  So the entries are those that the split COULD hold: inside the table's
+  // row; what an entry shorter than that left unset is read, but never followed.
   int seqlen_b = p.seqlens_k[b];
-  seqlen_b = seqlen_b < p.seqlen_kv ? seqlen_b : p.seqlen_kv;
-  seqlen_b = __builtin_amdgcn_readfirstlane(seqlen_b > 0 ? seqlen_b : 0);
+  int table0 = 0;
+  if (!score_wave && rq_slot0 + lane <= top_slot) table0 = pages[rq_slot0 + lane];
 #else
   const ae_elem* k1 = (const ae_elem*)p.k + (int64_t)b * p.k_stride_b + (int64_t)hk * p.k_stride_h;
   const ae_elem* k2 = (const ae_elem*)p.k2 + (int64_t)b * p.k2_stride_b + (int64_t)hk * p.k2_stride_h;
   const int seqlen_b = p.seqlen_kv;
 #endif
 
-  // (wave-uniform values are pinned to scalar registers: a copy in a vector register that gets spilled is
-  // reloaded with a scratch load, which the tile loads' vmcnt bookkeeping would have to wait for)
-  const int kv_begin = __builtin_amdgcn_readfirstlane(split * p.kv_per_split);
+#if AE_PAGED
+  asm volatile("" ::: "memory");   // (both requests stay in front of the first wait and of the exits below)
+  seqlen_b = seqlen_b < p.seqlen_kv ? seqlen_b : p.seqlen_kv;
+  seqlen_b = __builtin_amdgcn_readfirstlane(seqlen_b > 0 ? seqlen_b : 0);
+#endif
+
   int kv_end_ = kv_begin + p.kv_per_split;
   kv_end_ = kv_end_ < seqlen_b ? kv_end_ : seqlen_b;
   const int kv_end = __builtin_amdgcn_readfirstlane(kv_end_);
@@ -169,7 +207,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #if AE_NSPLIT == 1
   constexpr bool direct = true;
 #elif AE_PAGED
-  const bool direct = ae_mla_splits_used(p, seqlen_b) <= 1;
+  const bool direct = seqlen_b <= p.kv_per_split;      // ae_mla_splits_used() <= 1
 #else
   constexpr bool direct = false;
 #endif
@@ -180,8 +218,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     const int l32s = lane & 31;
     const int hfs = lane >> 5;
     const int head_in_group = ht * AE_HEADS_PER_WG + wave * 32 + l32s;
-    const bool head_ok = head_in_group < group;
-    const int hq = hk * group + (head_ok ? head_in_group : 0);
+    const int hq = hk * group + (head_in_group < group ? head_in_group : 0);
     // Q^T fragments: B operand (n = head = lane%32, k = d = 16*ks + 8*(lane/32) + j)
     const ae_elem* q1 = (const ae_elem*)p.q + (int64_t)b * p.q_stride_b + (int64_t)hq * p.q_stride_h;
     const ae_elem* q2 = (const ae_elem*)p.q2 + (int64_t)b * p.q2_stride_b + (int64_t)hq * p.q2_stride_h;
@@ -336,34 +373,19 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   // end re-read the last tile, so every trip issues the same number of loads; rows past the end re-read
   // the last row.
   const int blk0 = dvw * AE_LOADS < AE_BLOCKS - AE_LOADS ? dvw * AE_LOADS : AE_BLOCKS - AE_LOADS;
-  int ld_off[AE_LOADS];           // this lane's byte offset of load i inside a tile (may be negative)
-  unsigned ld_rope = 0;           // bit i: load i reads from the rope tensor (k2), else from the latent (k1)
-  const unsigned stride1 = (unsigned)p.k_stride_s * 2, stride2 = (unsigned)p.k2_stride_s * 2;   // bytes per kv row
-#pragma unroll
-  for (int i = 0; i < AE_LOADS; i++) {
-    const int sidx = (blk0 + i) * 64 + lane;
-    const int row = sidx / AE_CPR, cp = sidx % AE_CPR;
-    const int c = cp ^ AE_SWZ(row);
-    if (c < AE_CPR1) {
-      ld_off[i] = c * 16 + row * (int)stride1;
-    } else {
-      ld_off[i] = (c - AE_CPR1) * 16 + row * (int)stride2;
-      ld_rope |= 1u << i;
-    }
-    // immediate offset of load i inside its burst
-    ld_off[i] -= i < AE_L1 ? (i - AE_L1 / 2) * 1024 : (i - AE_L1 - AE_L2 / 2) * 1024;
-  }
+  // (the row and chunk of load i are carried along, and their row's offset with them: a division and a multiplication
+  // per load were a third of the instructions in front of the first request)
+  const int stride1 = (int)p.k_stride_s * 2, stride2 = (int)p.k2_stride_s * 2;   // bytes per kv row
+  int ld_row = (blk0 * 64 + lane) / AE_CPR, ld_cp = (blk0 * 64 + lane) % AE_CPR;
 #if AE_PAGED
   // Paged cache: the latent and the rope part are column ranges of ONE cache tensor (equal strides, the rope
   // columns rope_delta bytes behind the latent ones: checked by ae_mla_decode_fwd), so every load of a tile is
   // (the tile's wave-uniform address) + (an offset of the lane that never changes): scalar base + 32-bit offset
   // loads, no address arithmetic per tile at all.  Bases are passed 4 KiB low and the offsets 4 KiB high, so
   // that the offsets, which carry the compensation for the immediate offsets, stay >= 0.
-  const unsigned rope_delta = (unsigned)((const char*)k2 - (const char*)k1);
+  const int rope_off = (int)((const char*)k2 - (const char*)k1) - AE_CPR1 * 16;
   unsigned ld_uoff[AE_LOADS];
-#pragma unroll
-  for (int i = 0; i < AE_LOADS; i++)
-    ld_uoff[i] = (unsigned)(ld_off[i] + 4096) + (((ld_rope >> i) & 1u) ? rope_delta : 0u);
+  int ld_roff = ld_row * stride1 + 4096;
 #else
   // Dense cache: the requests go tile by tile, so a lane keeps the source address of each of its loads for the
   // NEXT tile to request and adds the tile pitch after every request - two instructions per load and tile.
@@ -371,15 +393,34 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   // form needs, made these waves, not the matrix pipe, set the pace of the whole workgroup.)
   const char* ld_ptr[AE_LOADS];
   unsigned ld_adv[AE_LOADS];
+  const char* const ld_base1 = (const char*)k1 + (uint64_t)((unsigned)kv_begin * (uint64_t)(unsigned)stride1);
+  const char* const ld_base2 = (const char*)k2 + (uint64_t)((unsigned)kv_begin * (uint64_t)(unsigned)stride2);
+  int ld_roff1 = ld_row * stride1, ld_roff2 = ld_row * stride2 - AE_CPR1 * 16;
+#endif
 #pragma unroll
   for (int i = 0; i < AE_LOADS; i++) {
-    const bool rope = (ld_rope >> i) & 1u;
-    const unsigned stride = rope ? stride2 : stride1;
-    ld_ptr[i] = (const char*)(rope ? (const void*)k2 : (const void*)k1) + (uint64_t)((unsigned)kv_begin * (uint64_t)stride) +
-                (int64_t)ld_off[i];
-    ld_adv[i] = AE_BN * stride;
-  }
+    const int c = ld_cp ^ AE_SWZ(ld_row);
+    const bool rope = c >= AE_CPR1;
+    // immediate offset of load i inside its burst
+    const int imm = i < AE_L1 ? (i - AE_L1 / 2) * 1024 : (i - AE_L1 - AE_L2 / 2) * 1024;
+#if AE_PAGED
+    ld_uoff[i] = (unsigned)(c * 16 + ld_roff + (rope ? rope_off : 0) - imm);
+#else
+    ld_ptr[i] = (rope ? ld_base2 : ld_base1) + (int64_t)(c * 16 + (rope ? ld_roff2 : ld_roff1) - imm);
+    ld_adv[i] = AE_BN * (unsigned)(rope ? stride2 : stride1);
 #endif
+    ld_cp += 64 % AE_CPR;
+    const bool wrap = ld_cp >= AE_CPR;
+    const int rows = 64 / AE_CPR + (wrap ? 1 : 0);
+    ld_cp -= wrap ? AE_CPR : 0;
+    ld_row += rows;
+#if AE_PAGED
+    ld_roff += 64 / AE_CPR * stride1 + (wrap ? stride1 : 0);
+#else
+    ld_roff1 += 64 / AE_CPR * stride1 + (wrap ? stride1 : 0);
+    ld_roff2 += 64 / AE_CPR * stride2 + (wrap ? stride2 : 0);
+#endif
+  }
 #if AE_PAGED
   // Paged cache: page, and row inside it, of the tile the NEXT request reads (wave-uniform; requests go tile by
   // tile, so no division per tile).  The split's part of the block table is copied into LDS first and looked up
@@ -388,14 +429,11 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   // waiting for every tile requested so far - 0.190 against 0.170 ms for the dense cache at B128 H128 S4096,
   // 0.166 ms with the table in LDS.  Every value wave writes the same entries and reads them back itself (a wave's
   // LDS operations complete in order), so no barrier is needed.
-  const int rq_slot0 = kv_begin / p.page_block_size;
-  {
-    const int n_ent = (kv_end - 1) / p.page_block_size - rq_slot0 + 1;     // <= AE_PTAB: checked by ae_mla_decode_fwd
-    for (int i = lane; i < n_ent && i < AE_PTAB; i += 64) ptab[i] = pages[rq_slot0 + i];
-  }
+  if (rq_slot0 + lane <= top_slot) ptab[lane] = table0;
+  for (int i = 64 + lane; i < AE_PTAB && rq_slot0 + i <= top_slot; i += 64) ptab[i] = pages[rq_slot0 + i];   // (<= AE_PTAB: checked by ae_mla_decode_fwd)
   int rq_idx = 0;
-  int rq_in_page = kv_begin - rq_slot0 * p.page_block_size;
-  int rq_page = pages[rq_slot0];
+  int rq_in_page = kv_begin - rq_slot0 * page_size;
+  int rq_page = __builtin_amdgcn_readfirstlane(table0);
 #endif
   // requests are made for t = 0, 1, 2, ... in this order
   auto load_tile = [&](int t_) AE_LAMBDA {
@@ -418,14 +456,15 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
       o2[i] = ld_uoff[i < AE_L2 ? AE_L1 + i : AE_L1];
     }
     if (__builtin_expect(ragged, 0)) {                        // rows past the end re-read the last row
-      asm volatile("" ::: "memory");                          // (keeps this ONE branch, out of the common path)
+      int ln = lane;
+      asm volatile("" : "+v"(ln)::"memory");                  // (keeps this ONE branch, out of the common path, rows and all)
 #pragma unroll
       for (int i = 0; i < 16; i++) {
         const int j = i < 8 ? (i < AE_L1 ? i : 0) : (i - 8 < AE_L2 ? AE_L1 + i - 8 : AE_L1);
-        const int row = ((blk0 + j) * 64 + lane) / AE_CPR;
+        const int row = ((blk0 + j) * 64 + ln) / AE_CPR;
         int over = kv0 + row - (seqlen_b - 1);
         over = over > 0 ? over : 0;                           // <= row: the offset stays >= 0
-        const unsigned back = (unsigned)over * stride1;
+        const unsigned back = (unsigned)(over * stride1);
         if (i < 8) o1[i] -= back;
         else o2[i - 8] -= back;
       }
@@ -441,14 +480,15 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
       g2[i] = ld_ptr[i < AE_L2 ? AE_L1 + i : AE_L1];
     }
     if (__builtin_expect(ragged, 0)) {                        // rows past the end re-read the last row
-      asm volatile("" ::: "memory");                          // (keeps this ONE branch, out of the common path)
+      int ln = lane;
+      asm volatile("" : "+v"(ln)::"memory");                  // (keeps this ONE branch, out of the common path, rows and all)
 #pragma unroll
       for (int i = 0; i < 16; i++) {
         const int j = i < 8 ? (i < AE_L1 ? i : 0) : (i - 8 < AE_L2 ? AE_L1 + i - 8 : AE_L1);
-        const int row = ((blk0 + j) * 64 + lane) / AE_CPR;
+        const int row = ((blk0 + j) * 64 + ln) / AE_CPR, cp = ((blk0 + j) * 64 + ln) % AE_CPR;
         int over = kv0 + row - (seqlen_b - 1);
         over = over > 0 ? over : 0;
-        const int back = over * (int)(((ld_rope >> j) & 1u) ? stride2 : stride1);
+        const int back = over * ((cp ^ AE_SWZ(row)) >= AE_CPR1 ? stride2 : stride1);
         if (i < 8) g1[i] -= back;
         else g2[i - 8] -= back;
       }
@@ -464,7 +504,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #else
     if (t + 1 < n_tiles) {                                    // where the next request reads: an LDS lookup per new
       rq_in_page += AE_BN;                                    // page, a whole trip before its result is used
-      if (rq_in_page >= p.page_block_size) {
+      if (rq_in_page >= page_size) {
         rq_in_page = 0;
         rq_idx++;
         rq_page = ptab[rq_idx];
@@ -480,6 +520,9 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     load_tile(t + AE_NSTAGE);
   };
 
+  __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
+#pragma unroll
+  for (int t = 0; t < AE_NSTAGE - 1; t++) load_tile(t);
   ae_f32x16 oacc[2][AE_NDB];     // [head block][dv block]: O^T
 #pragma unroll
   for (int hb = 0; hb < 2; hb++)
@@ -487,10 +530,6 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     for (int db = 0; db < AE_NDB; db++)
 #pragma unroll
       for (int r = 0; r < 16; r++) oacc[hb][db][r] = 0.f;
-
-  __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
-#pragma unroll
-  for (int t = 0; t < AE_NSTAGE - 1; t++) load_tile(t);
   __builtin_amdgcn_s_waitcnt(AE_VMCNT((AE_NSTAGE - 2) * AE_LOADS));
   __syncthreads();
 #if AE_CLOCK_STAMPS
@@ -628,10 +667,10 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     }
     // row scales: this lane's own head
     if (head_ok && hf == 0 && dvw == 0) {
-      const int64_t row = ((int64_t)b * p.heads_q + hq) * p.num_splits + split;
+      const int64_t row = ((int64_t)b * p.heads_q + hq) * AE_NSPLIT + split;
 #pragma unroll
       for (int i = 0; i < AE_N_ROWSCALES; i++) {
-        if (!direct) p.partial_rs[(int64_t)i * p.batch * p.heads_q * p.num_splits + row] = frs[i];
+        if (!direct) p.partial_rs[(int64_t)i * p.batch * p.heads_q * AE_NSPLIT + row] = frs[i];
         else if (p.rowscale_out[i]) p.rowscale_out[i][(int64_t)b * p.heads_q + hq] = frs[i];
       }
     }
@@ -661,26 +700,25 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
           *(__attribute__((address_space(3))) ae_f32x4*)(obuf + hl * (AE_DVW * 4) + (((db * 8 + rg * 2 + hf) ^ (hl & AE_OSW)) << 4)) = w;
         }
     }
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the wave's own region: its LDS writes have been made)
-  {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the wave's own region: its LDS writes have been made)
+    // (the 32 heads of a block leave while the next block's results are scaled and written)
     if (direct) {
-      constexpr int CPH = AE_DVW / 8;                         // 16-byte chunks of a head's piece
+      constexpr int CPH = AE_DVW / 8, N = 32 * CPH / 64;      // 16-byte chunks of a head's piece, of the block
       ae_elem* ob = (ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)(hk * group + ht * AE_HEADS_PER_WG) * p.o_stride_h + dvw * AE_DVW;
 #pragma unroll 4
-      for (int i = 0; i * 64 < heads_here * CPH; i++) {
-        const int hl = (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
-        const ae_elem8 w = *(const __attribute__((address_space(3))) ae_elem8*)(obuf + hl * (AE_DVW * 2) + ((c ^ (hl & AE_OSW)) << 4));
-        if (hl < heads_here) *(ae_elem8*)(ob + (int64_t)hl * p.o_stride_h + c * 8) = w;
+      for (int i = 0; i < N; i++) {
+        const int hs = hb * 32 + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
+        const ae_elem8 w = *(const __attribute__((address_space(3))) ae_elem8*)(obuf + hs * (AE_DVW * 2) + ((c ^ (hs & AE_OSW)) << 4));
+        if (hs < heads_here) *(ae_elem8*)(ob + (int64_t)hs * p.o_stride_h + c * 8) = w;
       }
     } else {
-      constexpr int CPH = AE_DVW / 4;
-      float* ob = p.partial_o + (((int64_t)b * p.heads_q + hk * group + ht * AE_HEADS_PER_WG) * p.num_splits + split) * AE_DV + dvw * AE_DVW;
+      constexpr int CPH = AE_DVW / 4, N = 32 * CPH / 64;
+      float* ob = p.partial_o + (((int64_t)b * p.heads_q + hk * group + ht * AE_HEADS_PER_WG) * AE_NSPLIT + split) * AE_DV + dvw * AE_DVW;
 #pragma unroll 8
-      for (int i = 0; i * 64 < heads_here * CPH; i++) {
-        const int hl = (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
-        const ae_f32x4 w = *(const __attribute__((address_space(3))) ae_f32x4*)(obuf + hl * (AE_DVW * 4) + ((c ^ (hl & AE_OSW)) << 4));
-        if (hl < heads_here) __builtin_nontemporal_store(w, (ae_f32x4*)(ob + (int64_t)hl * p.num_splits * AE_DV + c * 4));
+      for (int i = 0; i < N; i++) {
+        const int hs = hb * 32 + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
+        const ae_f32x4 w = *(const __attribute__((address_space(3))) ae_f32x4*)(obuf + hs * (AE_DVW * 4) + ((c ^ (hs & AE_OSW)) << 4));
+        if (hs < heads_here) __builtin_nontemporal_store(w, (ae_f32x4*)(ob + (int64_t)hs * AE_NSPLIT * AE_DV + c * 4));
       }
     }
   }
