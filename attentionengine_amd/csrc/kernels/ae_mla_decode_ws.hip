@@ -369,9 +369,9 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   // Which row and chunk a lane fetches never changes: its byte offset inside a tile is computed once (one
   // register per load) and added per tile to the tile's wave-uniform address in the latent or in the rope
   // tensor.  The loads of a wave go out as two bursts, each behind a single write of M0 (see
-  // ae_load_lds16_burst; the offsets carry the compensation for its immediate offsets).  Tiles past the
-  // end re-read the last tile, so every trip issues the same number of loads; rows past the end re-read
-  // the last row.
+  // ae_load_lds16_burst; the offsets carry the compensation for its immediate offsets).  Rows past the
+  // end re-read the last row.  Tiles past the end are not requested, so the waits for a tile ask whether a newer one
+  // is on its way (a split of four tiles asked for nine when every trip requested one, and waited for them at its end).
   const int blk0 = dvw * AE_LOADS < AE_BLOCKS - AE_LOADS ? dvw * AE_LOADS : AE_BLOCKS - AE_LOADS;
   // (the row and chunk of load i are carried along, and their row's offset with them: a division and a multiplication
   // per load were a third of the instructions in front of the first request)
@@ -438,9 +438,8 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   // requests are made for t = 0, 1, 2, ... in this order
   auto load_tile = [&](int t_) AE_LAMBDA {
     const int t = __builtin_amdgcn_readfirstlane(t_);
-    int tt = t < n_tiles ? t : n_tiles - 1;
-    tt = tt < 0 ? 0 : tt;
-    const int kv0 = kv_begin + tt * AE_BN;
+    if (t >= n_tiles) return;                       // (wave-uniform)
+    const int kv0 = kv_begin + t * AE_BN;
     ae_lds_byte* dst = lds + (t % AE_NSTAGE) * AE_STAGE_BYTES;
     const bool ragged = kv0 + AE_BN > seqlen_b;     // wave-uniform
 #if AE_PAGED
@@ -497,25 +496,22 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     ae_load_lds16_burst<AE_L2>((const void* const*)g2, dst + (blk0 + AE_L1 + AE_L2 / 2) * 1024);
 #endif
 #if !AE_PAGED
-    if (t + 1 < n_tiles) {                                    // (requests past the end repeat the last tile)
 #pragma unroll
-      for (int i = 0; i < AE_LOADS; i++) ld_ptr[i] += ld_adv[i];
-    }
+    for (int i = 0; i < AE_LOADS; i++) ld_ptr[i] += ld_adv[i];
 #else
-    if (t + 1 < n_tiles) {                                    // where the next request reads: an LDS lookup per new
-      rq_in_page += AE_BN;                                    // page, a whole trip before its result is used
-      if (rq_in_page >= page_size) {
-        rq_in_page = 0;
-        rq_idx++;
-        rq_page = ptab[rq_idx];
-      }
+    rq_in_page += AE_BN;                                      // where the next request reads: an LDS lookup per new
+    if (rq_in_page >= page_size) {                            // page, a whole trip before its result is used
+      rq_in_page = 0;
+      rq_idx++;
+      if (t + 1 < n_tiles) rq_page = ptab[rq_idx];
     }
 #endif
   };
-  // end of a trip: tile t+2 has landed when only the newest request is outstanding; after the barrier
+  // end of a trip: tile t+2 has landed when only the newest request (tile t+3) is outstanding; after the barrier
   // everyone is done with tile t, whose stage takes the next request
   auto end_trip = [&](int t) AE_LAMBDA {
-    __builtin_amdgcn_s_waitcnt(AE_VMCNT_LGKM0(AE_LOADS));   // ... and this trip's LDS reads have returned
+    if (t + AE_NSTAGE - 1 < n_tiles) __builtin_amdgcn_s_waitcnt(AE_VMCNT_LGKM0(AE_LOADS));   // ... and this trip's LDS reads have returned
+    else __builtin_amdgcn_s_waitcnt(AE_VMCNT_LGKM0(0));     // (the last tile has been requested: nothing is newer)
     __syncthreads();
     load_tile(t + AE_NSTAGE);
   };
@@ -530,7 +526,9 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     for (int db = 0; db < AE_NDB; db++)
 #pragma unroll
       for (int r = 0; r < 16; r++) oacc[hb][db][r] = 0.f;
-  __builtin_amdgcn_s_waitcnt(AE_VMCNT((AE_NSTAGE - 2) * AE_LOADS));
+  if (n_tiles >= AE_NSTAGE - 1) __builtin_amdgcn_s_waitcnt(AE_VMCNT((AE_NSTAGE - 2) * AE_LOADS));
+  else if (n_tiles == 2) __builtin_amdgcn_s_waitcnt(AE_VMCNT(AE_LOADS));
+  else __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
   __syncthreads();
 #if AE_CLOCK_STAMPS
   const unsigned long long ae_w1 = __builtin_amdgcn_s_memrealtime();     // tile 0 (and Q) have landed
@@ -706,7 +704,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
       constexpr int CPH = AE_DVW / 8, N = 32 * CPH / 64;      // 16-byte chunks of a head's piece, of the block
       ae_elem* ob = (ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)(hk * group + ht * AE_HEADS_PER_WG) * p.o_stride_h + dvw * AE_DVW;
 #pragma unroll 4
-      for (int i = 0; i < N; i++) {
+      for (int i = 0; i < N && i * 64 < (heads_here - hb * 32) * CPH; i++) {
         const int hs = hb * 32 + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
         const ae_elem8 w = *(const __attribute__((address_space(3))) ae_elem8*)(obuf + hs * (AE_DVW * 2) + ((c ^ (hs & AE_OSW)) << 4));
         if (hs < heads_here) *(ae_elem8*)(ob + (int64_t)hs * p.o_stride_h + c * 8) = w;
@@ -715,7 +713,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
       constexpr int CPH = AE_DVW / 4, N = 32 * CPH / 64;
       float* ob = p.partial_o + (((int64_t)b * p.heads_q + hk * group + ht * AE_HEADS_PER_WG) * AE_NSPLIT + split) * AE_DV + dvw * AE_DVW;
 #pragma unroll 8
-      for (int i = 0; i < N; i++) {
+      for (int i = 0; i < N && i * 64 < (heads_here - hb * 32) * CPH; i++) {
         const int hs = hb * 32 + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
         const ae_f32x4 w = *(const __attribute__((address_space(3))) ae_f32x4*)(obuf + hs * (AE_DVW * 4) + ((c ^ (hs & AE_OSW)) << 4));
         if (hs < heads_here) __builtin_nontemporal_store(w, (ae_f32x4*)(ob + (int64_t)hs * AE_NSPLIT * AE_DV + c * 4));
