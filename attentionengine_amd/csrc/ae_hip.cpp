@@ -605,10 +605,12 @@ int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params
     if (!p->rowscale_out[i])
       return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: rowscale_out[%d] is NULL", i);
   // 1-D grid: head tiles of one (batch, kv head, split) sit 8 ids apart (same XCD); the
-  // (batch, kv head, split) count is padded to a multiple of 8, surplus workgroups exit at once.
+  // (batch, kv head, split) count is padded to a multiple of 8, surplus workgroups exit at once.  A large
+  // paged launch counts an odd number of splits per entry (ae_mla_units in ae_mla_paged.h).
   int group = p->heads_q / p->heads_kv;
   int64_t n_ht = (group + cfg->block_m - 1) / cfg->block_m;
   int64_t units = (int64_t)p->batch * p->heads_kv * p->num_splits;
+  if (cfg->paged && units * n_ht > 128) units = (int64_t)p->batch * p->heads_kv * (p->num_splits | 1);
   int64_t total = ((units + 7) / 8) * 8 * n_ht;
   if (total > 0x7fffffffll) return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: grid too large");
   uint32_t grid[3] = {(uint32_t)total, 1, 1};

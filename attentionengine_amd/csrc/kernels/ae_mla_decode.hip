@@ -86,10 +86,15 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   const int wg = blockIdx.x;
   const int ht = (wg >> 3) % n_ht;
   const int u = (wg / (8 * n_ht)) * 8 + (wg & 7);        // flattened (batch, kv head, split)
-  if (u >= p.batch * p.heads_kv * p.num_splits) return;  // grid padding (whole workgroup exits)
-  const int split = u % p.num_splits;
-  const int hk = (u / p.num_splits) % p.heads_kv;
-  const int b = u / (p.num_splits * p.heads_kv);
+#if AE_PAGED
+  const int units = ae_mla_odd_units(p, n_ht) ? p.num_splits | 1 : p.num_splits;
+#else
+  const int units = p.num_splits;
+#endif
+  const int split = u % units;
+  if (u >= p.batch * p.heads_kv * units || split >= p.num_splits) return;  // grid padding (whole workgroup exits)
+  const int hk = (u / units) % p.heads_kv;
+  const int b = u / (units * p.heads_kv);
   const int hblk = wave >> 1;     // which 16 heads of the workgroup
   const int dvh = wave & 1;       // which half of the value dimension
   const int head_in_group = ht * AE_HEADS_PER_WG + hblk * 16 + l16;

@@ -25,7 +25,16 @@
 // directly (16 B per lane, chunk-swizzled as in ae_mla_decode.hip), AE_NSTAGE tiles deep; a trip ends by
 // waiting until only the newest tile request is outstanding.
 //
-// Configuration ("ae_config.h"): AE_D1 AE_D2 AE_DV AE_DTYPE_BF16 AE_N_ROWSCALES AE_NSPLIT
+// AE_HPW (heads per workgroup): 64 is the form above.  32 and 16 are for launches that 64-head workgroups spread thin -
+// few query heads, or so few sequences that the kv axis is split over many workgroups and every one of them pays for the
+// fp32 partial results of 64 heads.  A trip of the 64-head form is one score wave's instruction stream (36 MFMAs, 36
+// fragment reads, the softmax of 16 scores a lane: 0.92 us); here 16 heads and 16 of the tile's 32 keys make up a score
+// wave's share (v_mfma_f32_16x16x32: 18 MFMAs, 18 reads, 4 scores a lane), two waves per 16 heads, which exchange their
+// maxima through LDS at the end of a trip and so keep one reference.  The value waves take 16x16x32 too: 128 columns x
+// 16 or 32 heads.  Per head the tile is fetched and read two or four times as often as with 64 heads, which is why the
+// large launches keep that form.
+//
+// Configuration ("ae_config.h"): AE_HPW AE_D1 AE_D2 AE_DV AE_DTYPE_BF16 AE_N_ROWSCALES AE_NSPLIT
 // AE_COMBINE_THREADS AE_PAGED (1: the cache is paged, rows are found through ae_attn_params.block_table and
 // every batch entry has its own length seqlens_k[b], as in the reference's
 // cute_template_kvshared/kernels/params.h:33-36; a kv tile never straddles two pages), plus AE_SM_SCALE (the constant c > 0) and AE_SM_M / AE_SM_R (names of the
@@ -41,13 +50,27 @@
 #define AE_D (AE_D1 + AE_D2)
 #define AE_NWAVES 8
 #define AE_NT (AE_NWAVES * 64)
-#define AE_HEADS_PER_WG 64
+#ifndef AE_HPW
+#define AE_HPW 64
+#endif
+#define AE_HEADS_PER_WG AE_HPW
+#define AE_NHB (AE_HPW == 64 ? 2 : AE_HPW / 16)      // head blocks: of 32 heads, or of 16
+#define AE_HB (AE_HPW / AE_NHB)
 #define AE_BN 32                          // kv rows per tile
+#if AE_HPW == 64
 #define AE_NKS (AE_D / 16)                // 16-deep k-steps of S^T = K Q^T
+#else
+#define AE_NKS (AE_D / 32)                // 32-deep ones
+#endif
 #define AE_NLOADERS 4                     // the value waves also request the KV tiles
 #define AE_DVW (AE_DV / 4)                // value columns of one value wave
+#if AE_HPW == 64
 #define AE_NDB (AE_DVW / 32)              // 32-wide dv blocks of a value wave
 #define AE_NO (AE_NDB * 16)               // output elements per lane and head block
+#else
+#define AE_NDB (AE_DVW / 16)
+#define AE_NO (AE_NDB * 4)
+#endif
 #define AE_KSTR (AE_D * 2)                // LDS row pitch, bytes (unpadded: swizzled)
 #define AE_STAGE_BYTES (AE_BN * AE_KSTR)
 #define AE_CPR (AE_D / 8)                 // 16-byte chunks per K row
@@ -62,18 +85,21 @@
 #endif
 #define AE_PSTR 80                        // LDS pitch of one head's P row (32 kv * 2 B, padded against bank conflicts)
 #define AE_P_BYTES (AE_HEADS_PER_WG * AE_PSTR)
-#define AE_X_BYTES (AE_HEADS_PER_WG * 4 + 16)   // per-head rescale factors + one flag word per score wave (2 used)
+#define AE_X_BYTES (AE_HEADS_PER_WG * 4 + 16)   // per-head rescale factors + one flag word per head block
+#define AE_XMAX_BYTES (AE_HPW == 64 ? 0 : AE_HPW * 8)   // the row maxima of a tile's two halves
+#define AE_FIN (AE_HPW == 64 ? 2 : 3)                   // final row state per head: m, r (of each half)
 #define AE_TAU2 8.0f                      // the running maximum (log2 units) is refreshed only when it moved by more
 #define AE_SWZ(r) ((((r) >> 1) & 3) * 2 + (((r) >> 3) & 1))
 #define AE_VMCNT(n) (0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
 #define AE_VMCNT_LGKM0(n) (0x0070 | ((n) & 15) | (((n) >> 4) << 14))
 #ifndef AE_AHEAD
-#define AE_AHEAD 4
+#define AE_AHEAD (AE_HPW == 64 ? 4 : 6)
 #endif
 #define AE_RING (AE_AHEAD + 1)
 
 static_assert(AE_D1 % 32 == 0 && AE_D2 % 32 == 0, "latent / rope dims must be multiples of 32");
-static_assert(AE_NKS % 2 == 0, "two accumulation chains over the k-steps");
+static_assert(AE_HPW == 64 || AE_HPW == 32 || AE_HPW == 16, "two blocks of 32 heads, or one or two of 16");
+static_assert(AE_D % 64 == 0, "two accumulation chains over the k-steps");
 static_assert(AE_DV % 128 == 0 && AE_DV <= AE_D1, "V must be a prefix of the latent part, four 32-column blocks wide");
 static_assert(AE_CPR % 8 == 0 && AE_CPR1 % 8 == 0, "chunk groups of eight must not straddle the two K tensors");
 static_assert((AE_BN * AE_CPR) % 64 == 0, "tile must be a whole number of 1 KiB blocks");
@@ -82,7 +108,7 @@ static_assert(AE_L1 <= 8 && AE_L2 >= 1 && AE_BLOCKS >= AE_LOADS, "two bursts of 
 #define AE_OSW1 ((AE_DVW / 8) & -(AE_DVW / 8))
 #define AE_OSW (AE_OSW1 < 16 ? AE_OSW1 - 1 : 15)
 static_assert(AE_DV * AE_HEADS_PER_WG * 4 <= AE_NSTAGE * AE_STAGE_BYTES, "the results of 64 heads fit the tile stages");
-static_assert(AE_DVW % 32 == 0, "a block of 32 heads leaves in whole instructions of 64 lanes x 16 bytes");
+static_assert(AE_DVW % 64 == 0, "a value wave's first chunk is a multiple of eight, a block of heads leaves in whole instructions");
 static_assert(AE_NSTAGE >= 3, "a tile is multiplied by K one trip before it is multiplied as V");
 
 #ifndef AE_PAGED
@@ -112,15 +138,16 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   ae_lds_byte* lds = (ae_lds_byte*)ae_smem;                     // AE_NSTAGE kv tiles
   ae_lds_byte* pbuf = lds + AE_NSTAGE * AE_STAGE_BYTES;         // 2 x P^T [head][kv]
   ae_lds_byte* xbuf = pbuf + 2 * AE_P_BYTES;                    // 2 x (rescale factors, flags)
-  ae_lds_f32* fin = (ae_lds_f32*)(xbuf + 2 * AE_X_BYTES);       // final (m, r) per head
+  ae_lds_f32* xmax = (ae_lds_f32*)(xbuf + 2 * AE_X_BYTES);      // 2 x row maxima [half][head]
+  ae_lds_f32* fin = xmax + 2 * (AE_XMAX_BYTES / 4);             // final (m, r) per head
 #if AE_PAGED
-  ae_lds_i32* ptab = (ae_lds_i32*)(fin + 2 * AE_HEADS_PER_WG);  // AE_PTAB page numbers: this split's part of the block table
+  ae_lds_i32* ptab = (ae_lds_i32*)(fin + AE_FIN * AE_HEADS_PER_WG);  // AE_PTAB page numbers: this split's part of the block table
 #endif
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool score_wave = wave < 2;
+  const bool score_wave = wave < 2 || (AE_HPW == 32 && (wave == 4 || wave == 5));
 #if AE_CLOCK_STAMPS
   const unsigned long long ae_t0 = __builtin_amdgcn_s_memtime();
   const unsigned long long ae_w0 = __builtin_amdgcn_s_memrealtime();
@@ -143,9 +170,11 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     u8 = (wg >> 3) >> __builtin_ctz(n_ht);
   }
   const unsigned u = (unsigned)(u8 * 8 + (wg & 7));      // flattened (batch, kv head, split)
-  if (u >= (unsigned)(p.batch * p.heads_kv * AE_NSPLIT)) return;  // grid padding (whole workgroup exits)
-  const int split = u % AE_NSPLIT;
-  int b = u / AE_NSPLIT, hk = 0;
+  int split = u % AE_NSPLIT, b = u / AE_NSPLIT, hk = 0;
+#if AE_PAGED
+  if (ae_mla_odd_units(p, n_ht)) split = u % (AE_NSPLIT | 1), b = u / (AE_NSPLIT | 1);
+#endif
+  if (b >= p.batch * p.heads_kv || split >= AE_NSPLIT) return;  // grid padding (whole workgroup exits)
   if (__builtin_expect(p.heads_kv != 1, 0)) {
     hk = b % p.heads_kv;
     b /= p.heads_kv;
@@ -211,8 +240,132 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #else
   constexpr bool direct = false;
 #endif
-  if (wave == 4 || wave == 5) return;      // placeholders: they only steer the value waves onto SIMD 2, 3
+  if (!score_wave && (wave == 4 || wave == 5)) return;      // placeholders: they only steer the value waves onto SIMD 2, 3
 
+#if AE_HPW != 64
+  if (score_wave) {
+    // ======================= score wave: 16 heads, 16 of the tile's 32 keys ==============================
+    const int half = wave & 1;                 // which keys; waves 4, 5: the second 16 heads
+    const int l16 = lane & 15;
+    const int g = lane >> 4;
+    const int hl = (wave >> 2) * 16 + l16;     // head in the workgroup
+    const int head_in_group = ht * AE_HEADS_PER_WG + hl;
+    const int hq = hk * group + (head_in_group < group ? head_in_group : 0);
+    // Q^T fragments: B operand (n = head = lane%16, k = d = 32*ks + 8*(lane/16) + j)
+    const ae_elem* q1 = (const ae_elem*)p.q + (int64_t)b * p.q_stride_b + (int64_t)hq * p.q_stride_h;
+    const ae_elem* q2 = (const ae_elem*)p.q2 + (int64_t)b * p.q2_stride_b + (int64_t)hq * p.q2_stride_h;
+    ae_elem8 qf[AE_NKS];
+#pragma unroll
+    for (int ks = 0; ks < AE_D1 / 32; ks++) qf[ks] = *(const ae_elem8*)(q1 + ks * 32 + g * 8);
+#pragma unroll
+    for (int ks = 0; ks < AE_D2 / 32; ks++) qf[AE_D1 / 32 + ks] = *(const ae_elem8*)(q2 + ks * 32 + g * 8);
+
+    ae_rowstate st;
+    ae_rowstate_init(st);
+    float m2 = st.AE_SM_M * AE_LOG2E;   // running reference, log2 units: the same in both halves' waves
+    float r_run = half == 0 && g == 0 ? st.AE_SM_R : 0.f;      // this lane's part of the row sum
+    __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));   // Q has landed
+    __syncthreads();                           // tile 0 has landed
+
+    // K fragment of k-step ks: row 16*half + lane%16, global chunk 4*ks + lane/16 (swizzled in its three low bits)
+    const int k_row = half * 16 + l16;
+    int k_base[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) k_base[i] = k_row * AE_KSTR + (((4 * i + g) ^ AE_SWZ(k_row)) << 4);
+    // A trip multiplies tile n by Q^T, with the softmax of tile n - 1 between those MFMAs, and leaves the row maxima of
+    // tile n for the other half's wave.  A lane's scores: head lane%16, keys 16*half + 4*(lane/16) + e.
+    float xs[4], mx;
+    ae_lds_f32* const mine = xmax + half * AE_HPW + hl;
+    const ae_lds_f32* const other = xmax + (1 - half) * AE_HPW + hl;
+    float mn, osc, rs;
+    bool need;
+    // the softmax of tile tp in pieces, piece f issued behind the MFMA of k-step f
+    auto soft_slot = [&](int f, int tp, float mo) AE_LAMBDA {
+      if (f == 4) {
+        mx = __builtin_fmaxf(mx, mo) * (AE_SM_SCALE * AE_LOG2E);   // the scale is positive
+        need = (mx - m2) > AE_TAU2;
+        mn = need ? mx : m2;
+        osc = need ? ae_exp2(m2 - mn) : 1.0f;
+        m2 = mn;
+        rs = 0.f;
+      } else if (f >= 5 && f < 9) {
+        xs[f - 5] = ae_exp2(__builtin_fmaf(xs[f - 5], AE_SM_SCALE * AE_LOG2E, -mn));
+        rs += xs[f - 5];
+      } else if (f == 9) {
+        // P^T [head][slot]: a value wave's lane takes slots 8*(lane/16) .. +7, the keys 4*(lane/16) .. +3 of both halves
+        ae_elem4 w;
+#pragma unroll
+        for (int i = 0; i < 4; i++) w[i] = (ae_elem)xs[i];
+        *(__attribute__((address_space(3))) ae_elem4*)(pbuf + (tp & 1) * AE_P_BYTES + hl * AE_PSTR + 16 * g + 8 * half) = w;
+      } else if (f == 10) {
+        r_run = r_run * osc + rs;
+        ae_lds_byte* xb = xbuf + (tp & 1) * AE_X_BYTES;
+        if (half == 0) {
+          if (g == 0) ((ae_lds_f32*)xb)[hl] = osc;
+          const bool any = __builtin_amdgcn_ballot_w64(need) != 0;
+          if (lane == 0) ((ae_lds_i32*)(xb + AE_HEADS_PER_WG * 4))[wave >> 2] = any ? 1 : 0;
+        }
+      }
+    };
+    static_assert(AE_NKS >= 11, "the softmax of a tile is spread over 11 k-steps");
+    auto score_trip = [&](int tn, auto with_soft) AE_LAMBDA {
+      constexpr bool SOFT = decltype(with_soft)::value;
+      int ka[2];
+#pragma unroll
+      for (int i = 0; i < 2; i++) ka[i] = k_base[i] + (tn % AE_NSTAGE) * AE_STAGE_BYTES;
+      auto read_kfrag = [&](int ks) AE_LAMBDA -> ae_elem8 {
+        return *(const __attribute__((address_space(3))) ae_elem8*)(lds + ka[ks & 1] + (ks >> 1) * 128);
+      };
+      float mo = 0.f;
+      if (SOFT) mo = other[((tn - 1) & 1) * (AE_XMAX_BYTES / 4)];
+      ae_elem8 ring[AE_RING];
+#pragma unroll
+      for (int f = 0; f < AE_AHEAD; f++) ring[f] = read_kfrag(f);
+      ae_f32x4 sacc[2];
+#pragma unroll
+      for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) sacc[c][r] = 0.f;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int f = 0; f < AE_NKS; f++) {
+        if (f + AE_AHEAD < AE_NKS) ring[(f + AE_AHEAD) % AE_RING] = read_kfrag(f + AE_AHEAD);
+        sacc[f & 1] = ae_mfma16(ring[f % AE_RING], qf[f], sacc[f & 1]);
+        if (SOFT) soft_slot(f, tn - 1, mo);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++) xs[r] = sacc[0][r] + sacc[1][r];
+      if (__builtin_expect(kv_begin + tn * AE_BN + AE_BN > kv_end, 0)) {     // keys beyond the end of the range
+        asm volatile("" ::: "memory");
+        const int kvb = kv_begin + tn * AE_BN + 16 * half + 4 * g;
+#pragma unroll
+        for (int e = 0; e < 4; e++) xs[e] = kvb + e < kv_end ? xs[e] : AE_NEG_INF;
+      }
+      mx = ae_group_max(__builtin_fmaxf(__builtin_fmaxf(xs[0], xs[1]), __builtin_fmaxf(xs[2], xs[3])));
+      if (g == 0) mine[(tn & 1) * (AE_XMAX_BYTES / 4)] = mx;
+    };
+    if (n_tiles > 0) score_trip(0, ae_const_bool<false>());
+    __syncthreads();                             // end of trip 0: tile 1 has landed
+    for (int tn = 1; tn < n_tiles; tn++) {
+      score_trip(tn, ae_const_bool<true>());
+      __syncthreads();                           // end of the trip: P of tile tn - 1 is handed over, tile tn + 1 has landed
+    }
+    if (n_tiles > 0) {                           // the last tile's softmax has no MFMAs to hide behind
+      const float mo = other[((n_tiles - 1) & 1) * (AE_XMAX_BYTES / 4)];
+#pragma unroll
+      for (int f = 4; f < 11; f++) soft_slot(f, n_tiles - 1, mo);
+      __syncthreads();
+    }
+    const float r_row = ae_group_sum(r_run);
+    if (g == 0) {                                // final row state for the value waves
+      fin[hl * AE_FIN + 1 + half] = r_row;
+      if (half == 0) fin[hl * AE_FIN] = m2 * AE_LN2;
+    }
+    __syncthreads();
+    return;
+  }
+#else
   if (score_wave) {
     // =============================== score wave: 32 heads ==============================================
     const int l32s = lane & 31;
@@ -351,17 +504,23 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
       float hi;
       const float lo = ae_swap32_lo_hi(r_run, hi);
       if (hfs == 0) {
-        fin[(wave * 32 + l32s) * 2] = m2 * AE_LN2;
-        fin[(wave * 32 + l32s) * 2 + 1] = lo + hi;
+        fin[(wave * 32 + l32s) * AE_FIN] = m2 * AE_LN2;
+        fin[(wave * 32 + l32s) * AE_FIN + 1] = lo + hi;
       }
     }
     __syncthreads();
     return;
   }
+#endif
 
-  // ================================= value wave: AE_DVW value columns, 64 heads ========================
-  const int l32 = lane & 31;
-  const int hf = lane >> 5;
+  // ============================== value wave: AE_DVW value columns, AE_HPW heads =======================
+#if AE_HPW == 64
+  const int lhd = lane & 31;       // the lane's head in a block of heads
+  const int hf = lane >> 5;        // ... and which part of the block's rows
+#else
+  const int lhd = lane & 15;
+  const int hf = lane >> 4;
+#endif
   const int dvw = wave < 4 ? wave - 2 : wave - 4;   // waves 2, 3, 6, 7
   // Direct HBM -> LDS tile load, by the four value waves: wave w fills AE_LOADS consecutive 1 KiB blocks of
   // the tile, starting at block min(w*AE_LOADS, AE_BLOCKS-AE_LOADS) (the last wave overlaps its neighbour, so
@@ -519,13 +678,19 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
 #pragma unroll
   for (int t = 0; t < AE_NSTAGE - 1; t++) load_tile(t);
-  ae_f32x16 oacc[2][AE_NDB];     // [head block][dv block]: O^T
+#if AE_HPW == 64
+  typedef ae_f32x16 ae_acc;
+#else
+  typedef ae_f32x4 ae_acc;
+#endif
+  constexpr int NR = sizeof(ae_acc) / 4;
+  ae_acc oacc[AE_NHB][AE_NDB];     // [head block][dv block]: O^T
 #pragma unroll
-  for (int hb = 0; hb < 2; hb++)
+  for (int hb = 0; hb < AE_NHB; hb++)
 #pragma unroll
     for (int db = 0; db < AE_NDB; db++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) oacc[hb][db][r] = 0.f;
+      for (int r = 0; r < NR; r++) oacc[hb][db][r] = 0.f;
   if (n_tiles >= AE_NSTAGE - 1) __builtin_amdgcn_s_waitcnt(AE_VMCNT((AE_NSTAGE - 2) * AE_LOADS));
   else if (n_tiles == 2) __builtin_amdgcn_s_waitcnt(AE_VMCNT(AE_LOADS));
   else __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
@@ -534,13 +699,14 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   const unsigned long long ae_w1 = __builtin_amdgcn_s_memrealtime();     // tile 0 (and Q) have landed
 #endif
 
+#if AE_HPW == 64
   // V^T fragment (k-step kk, dv block db): A[m = dv][k = kv]: lane i of a 16-lane group supplies the
   // address of row 16*kk + 8*hf + i/4 (+4 for slots 4..7), 8 bytes at value column
   // 32*db + 16*((lane%32)/16) + 4*(i%4), and receives column i of those four rows.  The swizzle of a
   // row's chunks touches the three low bits of the chunk number only, so a lane has four distinct
   // offsets (parity of db, first / second group of four rows) and everything else is an immediate.
   const int v_row = 8 * hf + ((lane & 15) >> 2);
-  const int v_c0 = 2 * (l32 >> 4) + ((lane & 3) >> 1);
+  const int v_c0 = 2 * (lhd >> 4) + ((lane & 3) >> 1);
   const int v_half = (lane & 1) * 8;
   int v_base[2][2];     // [db & 1][row group]
 #pragma unroll
@@ -550,7 +716,6 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
       const int r = v_row + 4 * rg;
       v_base[par][rg] = r * AE_KSTR + ((((4 * par + v_c0) ^ AE_SWZ(r)) + 4 * AE_NDB * dvw) << 4) + v_half;
     }
-  static_assert(AE_NDB % 2 == 0, "a value wave's first chunk must be a multiple of eight");
   auto read_vfrag = [&](const int (&va)[2][2], int kk, int db) AE_LAMBDA -> ae_elem8 {
     const int imm = 16 * kk * AE_KSTR + (db >> 1) * 128;
     ae_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)(
@@ -560,50 +725,81 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     return __builtin_bit_cast(ae_elem8, __builtin_shufflevector(lo, hi2, 0, 1, 2, 3, 4, 5, 6, 7));
   };
 
+#else
+  // V^T fragment of dv block db (16 columns, all 32 keys): A[m = dv][k]: k = 8*(lane/16) + j is key 4*(lane/16) + j of the
+  // tile's first half (j < 4) or second half (the order in which the score waves leave P): the 16 rows of one transposed
+  // read then lie in 16 different places of the swizzle, where rows 0-3 and 8-11 would share theirs.
+  const int v_row = 4 * hf + (lhd >> 2);
+  int v_base[4];        // [db & 3]; rows 16 apart share a permutation
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    v_base[i] = v_row * AE_KSTR + ((((2 * i + ((lane & 3) >> 1)) ^ AE_SWZ(v_row)) + (AE_DVW / 8) * dvw) << 4) + (lane & 1) * 8;
+  auto read_vfrag = [&](const int (&va)[4], int, int db) AE_LAMBDA -> ae_elem8 {
+    const int imm = (db >> 2) * 128;
+    ae_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)(
+        lds + va[db & 3] + imm));
+    ae_s16x4 hi2 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)(
+        lds + va[db & 3] + imm + 16 * AE_KSTR));
+    return __builtin_bit_cast(ae_elem8, __builtin_shufflevector(lo, hi2, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+#endif
+
   // A trip of a value wave: O^T += V^T P^T for tile n - 2 with the V^T fragments it holds in registers (PV),
   // and the fragments of tile n - 1 read from LDS into those registers as they fall free (RD) - the read
   // has a whole trip to complete, and tile n - 1's stage can take the next request when the trip ends.
-  ae_elem8 vreg[2 * AE_NDB];     // fragment f = (k-step f / AE_NDB, dv block f % AE_NDB)
+  constexpr int NKK = AE_HPW == 64 ? 2 : 1;      // k-steps over the tile's keys
+  ae_elem8 vreg[NKK * AE_NDB];     // fragment f = (k-step f / AE_NDB, dv block f % AE_NDB)
 #pragma unroll
-  for (int f = 0; f < 2 * AE_NDB; f++) vreg[f] = (ae_elem8){};
+  for (int f = 0; f < NKK * AE_NDB; f++) vreg[f] = (ae_elem8){};
   auto value_trip = [&](int n, auto with_pv, auto with_rd) AE_LAMBDA {
     constexpr bool PV = decltype(with_pv)::value;
     constexpr bool RD = decltype(with_rd)::value;
-    int va[2][2];          // the lane's four fragment offsets inside tile n - 1's stage
+    // the lane's four fragment offsets inside tile n - 1's stage
+#if AE_HPW == 64
+    int va[2][2];
 #pragma unroll
     for (int i = 0; i < 4; i++) va[i >> 1][i & 1] = v_base[i >> 1][i & 1] + ((n - 1) % AE_NSTAGE) * AE_STAGE_BYTES;
-    ae_elem8 pf[2][2];
+#else
+    int va[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) va[i] = v_base[i] + ((n - 1) % AE_NSTAGE) * AE_STAGE_BYTES;
+#endif
+    ae_elem8 pf[AE_NHB][NKK];
     if (PV) {
       const int t = n - 2;
       const ae_lds_byte* pb = pbuf + (t & 1) * AE_P_BYTES;
       const ae_lds_byte* xb = xbuf + (t & 1) * AE_X_BYTES;
       // rescale O for the heads whose reference moved (rare once the maxima have settled)
       const ae_lds_i32* flags = (const ae_lds_i32*)(xb + AE_HEADS_PER_WG * 4);
-      if (__builtin_amdgcn_readfirstlane(flags[0] | flags[1]) != 0) {
+      if (__builtin_amdgcn_readfirstlane(flags[0] | flags[AE_NHB - 1]) != 0) {
 #pragma unroll
-        for (int hb = 0; hb < 2; hb++) {
-          const float osc = ((const ae_lds_f32*)xb)[hb * 32 + l32];
+        for (int hb = 0; hb < AE_NHB; hb++) {
+          const float osc = ((const ae_lds_f32*)xb)[hb * AE_HB + lhd];
 #pragma unroll
           for (int db = 0; db < AE_NDB; db++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) oacc[hb][db][r] *= osc;
+            for (int r = 0; r < NR; r++) oacc[hb][db][r] *= osc;
         }
       }
-      // P^T fragments: B[k = kv = 16*kk + 8*hf + j][n = head = 32*hb + l32]
+      // P^T fragments: B[k = kv = 16*kk + 8*hf + j][n = head = 32*hb + lhd] (16 heads a block: all 32 kv, k = 8*hf + j)
 #pragma unroll
-      for (int hb = 0; hb < 2; hb++)
+      for (int hb = 0; hb < AE_NHB; hb++)
 #pragma unroll
-        for (int kk = 0; kk < 2; kk++)
+        for (int kk = 0; kk < NKK; kk++)
           pf[hb][kk] = *(const __attribute__((address_space(3))) ae_elem8*)(
-              pb + (hb * 32 + l32) * AE_PSTR + 32 * kk + 16 * hf);
+              pb + (hb * AE_HB + lhd) * AE_PSTR + 32 * kk + 16 * hf);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int f = 0; f < 2 * AE_NDB; f++) {
+    for (int f = 0; f < NKK * AE_NDB; f++) {
       if (PV) {
 #pragma unroll
-        for (int hb = 0; hb < 2; hb++)
+        for (int hb = 0; hb < AE_NHB; hb++)
+#if AE_HPW == 64
           oacc[hb][f % AE_NDB] = ae_mfma32(vreg[f], pf[hb][f / AE_NDB], oacc[hb][f % AE_NDB]);
+#else
+          oacc[hb][f] = ae_mfma16(vreg[f], pf[hb][0], oacc[hb][f]);
+#endif
       }
       if (RD) vreg[f] = read_vfrag(va, f / AE_NDB, f % AE_NDB);
       __builtin_amdgcn_sched_barrier(0);
@@ -630,11 +826,13 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   ae_lds_byte* obuf = lds + dvw * (AE_HEADS_PER_WG * AE_DVW * 4);
   const int heads_left = group - ht * AE_HEADS_PER_WG;          // heads of the tile that exist
   const int heads_here = heads_left < AE_HEADS_PER_WG ? heads_left : AE_HEADS_PER_WG;
-  // ---- per-split epilogue: lane owns head 32*hb + l32, value columns AE_DVW*dvw + 32*db + 8*(r/4) + 4*hf + r%4
+  // ---- per-split epilogue: lane owns head 32*hb + lhd, value columns AE_DVW*dvw + 32*db + 8*(r/4) + 4*hf + r%4
+  //      (16 heads a block: head 16*hb + lhd, columns AE_DVW*dvw + 16*db + 4*hf + r)
 #pragma unroll
-  for (int hb = 0; hb < 2; hb++) {
-    if (hb * 32 >= heads_here) break;                           // (wave uniform)
-    const int head_in_group = ht * AE_HEADS_PER_WG + hb * 32 + l32;
+  for (int hb = 0; hb < AE_NHB; hb++) {
+    if (hb * AE_HB >= heads_here) break;                        // (wave uniform)
+    const int hl = hb * AE_HB + lhd;
+    const int head_in_group = ht * AE_HEADS_PER_WG + hl;
     const bool head_ok = head_in_group < group;
     const int hq = hk * group + (head_ok ? head_in_group : 0);
     ae_ctx ctx;
@@ -650,12 +848,13 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #pragma unroll
     for (int db = 0; db < AE_NDB; db++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) o[db * 16 + r] = oacc[hb][db][r];
+      for (int r = 0; r < NR; r++) o[db * NR + r] = oacc[hb][db][r];
     float frs[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1];
     frs[0] = 0.f;
     if (n_tiles > 0) {
-      st.AE_SM_M = fin[(hb * 32 + l32) * 2];
-      st.AE_SM_R = fin[(hb * 32 + l32) * 2 + 1];
+      st.AE_SM_M = fin[hl * AE_FIN];
+      st.AE_SM_R = fin[hl * AE_FIN + 1];
+      if (AE_FIN == 3) st.AE_SM_R += fin[hl * AE_FIN + 2];
       ae_epilogue<AE_NO>(o, st, frs, ctx, cust);
     } else {
 #pragma unroll
@@ -678,43 +877,41 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     // workgroup).  The partial results are stored past the cache (nontemporal, and read so by the merge kernel): their
     // lines are read once, on another XCD; left dirty they are written back between the two launches and again when the
     // next call's stores meet them.  B4 H128 Skv2048: call 24.7 -> 20.2 us.  16-byte chunks of a row are exchanged by the head number, so neither side meets a bank twice.
-    const int hl = hb * 32 + l32;
-    if (direct) {
+    // (piece e of a lane, four columns: fp32 chunk at4, in the output type half at4 % 2 of chunk at4 / 2)
 #pragma unroll
-      for (int db = 0; db < AE_NDB; db++)
+    for (int e = 0; e < AE_NO / 4; e++) {
+#if AE_HPW == 64
+      const int at4 = e * 2 + hf;                   // (dv block e / 4)
+#else
+      const int at4 = e * 4 + hf;
+#endif
+      if (direct) {
+        ae_elem4 w;
 #pragma unroll
-        for (int rg = 0; rg < 4; rg++) {
-          ae_elem4 w;
-#pragma unroll
-          for (int i = 0; i < 4; i++) w[i] = (ae_elem)o[db * 16 + rg * 4 + i];
-          *(__attribute__((address_space(3))) ae_elem4*)(obuf + hl * (AE_DVW * 2) + (((db * 4 + rg) ^ (hl & AE_OSW)) << 4) + hf * 8) = w;
-        }
-    } else {
-#pragma unroll
-      for (int db = 0; db < AE_NDB; db++)
-#pragma unroll
-        for (int rg = 0; rg < 4; rg++) {
-          const ae_f32x4 w = {o[db * 16 + rg * 4 + 0], o[db * 16 + rg * 4 + 1], o[db * 16 + rg * 4 + 2], o[db * 16 + rg * 4 + 3]};
-          *(__attribute__((address_space(3))) ae_f32x4*)(obuf + hl * (AE_DVW * 4) + (((db * 8 + rg * 2 + hf) ^ (hl & AE_OSW)) << 4)) = w;
-        }
+        for (int i = 0; i < 4; i++) w[i] = (ae_elem)o[e * 4 + i];
+        *(__attribute__((address_space(3))) ae_elem4*)(obuf + hl * (AE_DVW * 2) + (((at4 >> 1) ^ (hl & AE_OSW)) << 4) + (at4 & 1) * 8) = w;
+      } else {
+        const ae_f32x4 w = {o[e * 4 + 0], o[e * 4 + 1], o[e * 4 + 2], o[e * 4 + 3]};
+        *(__attribute__((address_space(3))) ae_f32x4*)(obuf + hl * (AE_DVW * 4) + ((at4 ^ (hl & AE_OSW)) << 4)) = w;
+      }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the wave's own region: its LDS writes have been made)
-    // (the 32 heads of a block leave while the next block's results are scaled and written)
+    // (the heads of a block leave while the next block's results are scaled and written)
     if (direct) {
-      constexpr int CPH = AE_DVW / 8, N = 32 * CPH / 64;      // 16-byte chunks of a head's piece, of the block
+      constexpr int CPH = AE_DVW / 8, N = AE_HB * CPH / 64;      // 16-byte chunks of a head's piece, instructions of the block
       ae_elem* ob = (ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)(hk * group + ht * AE_HEADS_PER_WG) * p.o_stride_h + dvw * AE_DVW;
 #pragma unroll 4
-      for (int i = 0; i < N && i * 64 < (heads_here - hb * 32) * CPH; i++) {
-        const int hs = hb * 32 + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
+      for (int i = 0; i < N && i * 64 < (heads_here - hb * AE_HB) * CPH; i++) {
+        const int hs = hb * AE_HB + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
         const ae_elem8 w = *(const __attribute__((address_space(3))) ae_elem8*)(obuf + hs * (AE_DVW * 2) + ((c ^ (hs & AE_OSW)) << 4));
         if (hs < heads_here) *(ae_elem8*)(ob + (int64_t)hs * p.o_stride_h + c * 8) = w;
       }
     } else {
-      constexpr int CPH = AE_DVW / 4, N = 32 * CPH / 64;
+      constexpr int CPH = AE_DVW / 4, N = AE_HB * CPH / 64;
       float* ob = p.partial_o + (((int64_t)b * p.heads_q + hk * group + ht * AE_HEADS_PER_WG) * AE_NSPLIT + split) * AE_DV + dvw * AE_DVW;
 #pragma unroll 8
-      for (int i = 0; i < N && i * 64 < (heads_here - hb * 32) * CPH; i++) {
-        const int hs = hb * 32 + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
+      for (int i = 0; i < N && i * 64 < (heads_here - hb * AE_HB) * CPH; i++) {
+        const int hs = hb * AE_HB + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
         const ae_f32x4 w = *(const __attribute__((address_space(3))) ae_f32x4*)(obuf + hs * (AE_DVW * 4) + ((c ^ (hs & AE_OSW)) << 4));
         if (hs < heads_here) __builtin_nontemporal_store(w, (ae_f32x4*)(ob + (int64_t)hs * AE_NSPLIT * AE_DV + c * 4));
       }

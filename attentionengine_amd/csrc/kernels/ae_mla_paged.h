@@ -10,6 +10,16 @@
 // output and -inf row scales, the values the kernels' epilogues produce for an empty range.
 #pragma once
 
+// Workgroup ids per (batch entry, kv head): the splits, in a launch of more than half as many workgroups as there are CUs
+// made an odd number (as ae_mla_decode_fwd counts them).  Ids are dealt to the eight XCDs in turn and the first splits of
+// every entry are the ones that hold keys: with an even number of ids per entry the live ones of all entries gather on some
+// XCDs, which then take a second round.  Entries of 1/B ... all of the table, 16 heads a workgroup: B40 H64, 16 pages, 2
+// splits 29.3 -> 21.9 us; B6 H128, 37 pages, 8 splits 25.8 -> 19.5; the small launch pays 0.4 us for the surplus ids (B2
+// H128, 8 splits 11.6 -> 12.5).
+__device__ __forceinline__ bool ae_mla_odd_units(const ae_attn_params& p, int n_ht) {
+  return p.batch * p.heads_kv * p.num_splits * n_ht > 128;
+}
+
 __device__ __forceinline__ int ae_mla_splits_used(const ae_attn_params& p, int seqlen_b) {
   const int n = (seqlen_b + p.kv_per_split - 1) / p.kv_per_split;
   return n < p.num_splits ? n : p.num_splits;
