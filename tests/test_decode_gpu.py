@@ -293,6 +293,37 @@ def test_mla_decode_long_single_split_loop(cuda_device, monkeypatch, kernel, tem
     assert ((got - lse).abs() <= LSE_TOL + 2e-6 * lse.abs()).all()
 
 
+@pytest.mark.parametrize("heads", [16, 32, 64])
+@pytest.mark.parametrize("B,H,G,S,n_split,dtype", [
+    (1, 1, 1, 1, 1, torch.bfloat16),         # one head, one key: fifteen dead heads, half a tile without keys
+    (2, 40, 2, 97, 2, torch.float16),        # 20 heads a latent head (a block and a quarter); the second split ends in a
+                                             # tile of one key, whose second half has none
+    (1, 100, 1, 530, 3, torch.bfloat16),     # seven / four / two head tiles; 6 + 6 + 5 tiles
+    (3, 33, 1, 1100, 1, torch.float16),      # unsplit: 35 tiles through the stage ring
+])
+def test_mla_decode_heads_per_workgroup(cuda_device, B, H, G, S, n_split, dtype, heads):
+    """Every form of the wave-specialised kernel (AE_HPW) on every shape, also where the plan would take another.  Keys
+    late in the sequence score far above everything before them, so the lazy reference moves with O in flight."""
+    D, DV = 576, 512
+    scale = 1 / math.sqrt(192)
+    print(f"case mla heads per workgroup {heads} B{B} H{H} G{G} S{S} splits {n_split} {dtype}", flush=True)
+    q, q_pe, kv, k_pe = _mla_inputs(B, H, G, S, DV, D - DV, dtype, seed=23)
+    k_pe = k_pe.float()
+    k_pe[:, S // 2:] *= 6.0
+    k_pe[:, -3:] *= 2.0
+    k_pe = k_pe.to(dtype)
+    mod = _mla_engine(B, H, G, S, D, DV, dtype, scale)
+    tiles = -(-S // 32)
+    mod.attention.plan = lambda *a, **k: (heads, n_split, -(-tiles // n_split) * 32)
+    ref, lse = R.mla_decode(q[:, 0], q_pe[:, 0], kv, k_pe, scale=scale)
+    for _ in range(2):                        # through Python, then through the native host path
+        out = mod(q.cuda(), q_pe.cuda(), kv.cuda(), k_pe.cuda())
+        assert torch.isfinite(out).all()
+        assert (out[:, 0].float().cpu() - ref).abs().max().item() <= OUT_TOL
+        got = mod.final_rowscales["lse"][:, :, 0].cpu()
+        assert ((got - lse).abs() <= LSE_TOL + 2e-6 * lse.abs()).all()
+
+
 def test_mla_decode_full_size(cuda_device):
     """BASELINE config 5 at full size (B128 H128 one latent head, D576 DV512, Skv4096, bf16, scale
     1/sqrt(192)) with the plan the benchmark times: one split, 128 tiles per workgroup.  Oracle on batch

@@ -800,3 +800,25 @@ def test_every_split_count_that_is_tuned_is_launched(monkeypatch, tmp_path, kind
     assert len(set(launched)) == 3 and op._tuned[key] == 4
     run()
     assert launched[-1] == launched[1]               # ... and the calls that follow run the one that was fastest
+
+
+def test_mla_plan():
+    """Splits cover the cache with none empty, whatever the shape; small batches take few heads a workgroup, the full one
+    64; a paged split holds no more pages than the kernel keeps table entries for; target_workgroups = 1 means no splits."""
+    from core.lower.lower_decode import MLADecodeOp
+    dt = torch.bfloat16
+    meta = (meta_tensor(1, 16, 1, 576, dtype=dt), meta_tensor(1, 1, 64, 576, dtype=dt), meta_tensor(1, 1, 64, 512, dtype=dt))
+    op = MLADecodeOp(meta, CustomIO({}), C.make_scale_score_mod(192 ** -0.5), None, C.OnlineSoftmax(), "-inf")
+    for B in (1, 3, 17, 128):
+        for Hq, Hkv in ((1, 1), (16, 1), (40, 2), (128, 1)):
+            for Skv in (1, 31, 33, 1000, 8192):
+                heads, n_split, per = op.plan(B, Hq, Hkv, Skv)
+                assert heads in (16, 32, 64) and per % op.BLOCK_N == 0
+                assert n_split * per >= Skv > (n_split - 1) * per and 1 <= n_split <= op.MAX_SPLITS
+                assert heads == 16 or Hq // Hkv > heads // 2
+    assert op.plan(128, 128, 1, 4096) == (64, 1, 4096)
+    assert op.plan(4, 128, 1, 2048)[0] == 16 and op.plan(4, 128, 1, 2048)[1] > 1
+    _, n_split, per = op.plan(1, 16, 1, 300000, 64)
+    assert per // 64 + 2 <= op.PAGE_TABLE_ENTRIES and n_split * per >= 300000
+    op.target_workgroups = 1
+    assert op.plan(2, 128, 1, 1000) == (64, 1, 1024)
