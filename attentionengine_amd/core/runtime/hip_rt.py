@@ -84,7 +84,7 @@ class AttnBwdParams(C.Structure):
         + [("batch", C.c_int32), ("heads_q", C.c_int32), ("heads_kv", C.c_int32),
            ("seqlen_q", C.c_int32), ("seqlen_kv", C.c_int32), ("mask_b", C.c_int32), ("mask_h", C.c_int32),
            ("mask_nq", C.c_int32), ("mask_nkv", C.c_int32), ("mask_block_m", C.c_int32), ("mask_block_n", C.c_int32),
-           ("reserved", C.c_int32 * 1)]
+           ("dkv_parts", C.c_int32)]
     )
 
 

@@ -678,7 +678,18 @@ int ae_prefill_bwd(ae_kernel* delta, ae_kernel* dkv, ae_kernel* dq, const ae_att
   const uint64_t rows_per_wg = 256u / (uint32_t)(cfg->head_dim_v / 8);
   const uint64_t g_delta = (rows + rows_per_wg - 1) / rows_per_wg;
   // ids are 8*slot + xcd, slot = tile*ceil(batch*heads/8) + head group (see ae_prefill_bwd.hip)
-  const uint64_t g_dkv = (((uint64_t)p->seqlen_kv + 127) / 128) * ((((uint64_t)p->batch * p->heads_kv) + 7) / 8) * 8;
+  uint64_t g_dkv = (((uint64_t)p->seqlen_kv + 127) / 128) * ((((uint64_t)p->batch * p->heads_kv) + 7) / 8) * 8;
+  if (cfg->merge_in_wg == 2) {         // kernels that share a kv tile out over several workgroups
+    if (delta || cfg->mask_mode == 2)
+      return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: shared kv tiles need the dq launch first and no tile tables");
+    if (p->dkv_parts < 2 || p->dkv_parts > 64)
+      return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: dkv_parts=%d", p->dkv_parts);
+    if (((uintptr_t)p->delta & 15) != 0)
+      return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: the work buffer must start on a 16-byte boundary");
+    g_dkv *= (uint64_t)p->dkv_parts;
+  } else if (cfg->merge_in_wg != 0) {
+    return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: merge_in_wg=%d", cfg->merge_in_wg);
+  }
   const uint64_t g_dq = (((uint64_t)p->seqlen_q + cfg->block_m - 1) / cfg->block_m) * ((((uint64_t)p->batch * p->heads_q) + 7) / 8) * 8;
   if (g_delta > 0x7fffffffull || g_dkv > 0x7fffffffull || g_dq > 0x7fffffffull)
     return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: grid too large");

@@ -68,6 +68,8 @@ struct BwdPlan {
   ae_tile_cfg cfg{};
   int n_rs = 0;             // final row scales the kernels read (0: none)
   int planes = 2;           // fp32 planes of the work buffer
+  int dkv_parts = 0;        // workgroups per kv tile of the dk/dv launch (0: kernels that do not share one out)
+  int64_t work_more = 0;    // fp32 values of the work buffer behind its planes
   at::Tensor table_dq, table_dkv;     // tile classes of the two launches (mask mode 2)
   std::shared_ptr<Keep> keep;
 };
@@ -196,7 +198,7 @@ struct AeBackward : public torch::autograd::Node {
     const int dev = q.get_device();
     const int64_t B = q.size(0), Sq = q.size(1), Hq = q.size(2), Skv = k.size(1), Hkv = k.size(2);
     at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
-    at::Tensor work = empty({pl.planes, B, Hq, Sq}, at::kFloat, dev);
+    at::Tensor work = empty({pl.planes * B * Hq * Sq + pl.work_more}, at::kFloat, dev);
     ae_attn_bwd_params p{};
     p.q = q.const_data_ptr(), p.k = k.const_data_ptr(), p.v = v.const_data_ptr(), p.out = out.const_data_ptr();
     p.dout = dout.const_data_ptr();
@@ -214,6 +216,7 @@ struct AeBackward : public torch::autograd::Node {
     set_strides(dk, p.dk_stride_b, p.dk_stride_s, p.dk_stride_h);
     set_strides(dv, p.dv_stride_b, p.dv_stride_s, p.dv_stride_h);
     p.batch = (int)B, p.heads_q = (int)Hq, p.heads_kv = (int)Hkv, p.seqlen_q = (int)Sq, p.seqlen_kv = (int)Skv;
+    p.dkv_parts = pl.dkv_parts;
     if (pl.table_dq.defined()) {
       p.mask_dq = (const int8_t*)pl.table_dq.const_data_ptr(), p.mask_dkv = (const int8_t*)pl.table_dkv.const_data_ptr();
       p.mask_b = (int)pl.table_dq.size(0), p.mask_h = (int)pl.table_dq.size(1);
@@ -515,6 +518,7 @@ PyObject* host_add_backward(PyObject* self, PyObject* d) {
   bw->dq = (ae_kernel*)(uintptr_t)get_int(d, "dq");
   TORCH_CHECK(bw->dkv && bw->dq && get_cfg(d, "cfg", bw->cfg), "a backward plan needs its kernels and their tile configuration");
   bw->n_rs = (int)get_int(d, "n_rs"), bw->planes = (int)get_int(d, "planes", 2);
+  bw->dkv_parts = (int)get_int(d, "dkv_parts"), bw->work_more = get_int(d, "work_more");
   bw->table_dq = get_tensor(d, "table_dq"), bw->table_dkv = get_tensor(d, "table_dkv");
   bw->keep = std::make_shared<Keep>(PyDict_GetItemString(d, "keep"));
   for (auto& pl : *h->plans)

@@ -162,6 +162,16 @@ AE_DEV int ae_bwd_chunk_pos(int r, int c) {
 #ifndef AE_BWD_FUSE_DELTA
 #define AE_BWD_FUSE_DELTA 0
 #endif
+// 1 (softmax attention, both launches): the items of a kv tile are shared out over p.dkv_parts workgroups of the dk/dv
+// launch, which leave fp32 partial sums in the work buffer; the last one to finish adds them up in the order of the parts
+// (bit-reproducible) and writes dk and dv.  For launches whose kv tiles do not fill the chip or whose longest tile sets the
+// time: grouped heads (a tile's items are those of all its q heads) at small batch.  Behind the two planes of the work
+// buffer: one arrival counter per kv tile, cleared by the dq launch, then the partial sums [tile][part][wave][register][lane].
+// Backward of B2 Hq32 Hkv8 S1389 D64 causal bf16: 176 workgroups, the longest 88 items; see dkv_parts() on the host.
+#ifndef AE_BWD_SPLIT
+#define AE_BWD_SPLIT 0
+#endif
+static_assert(!AE_BWD_SPLIT || (AE_BWD_FUSE_DELTA && AE_MASK_MODE != 2), "shared kv tiles: softmax without a tile table");
 static_assert(!AE_BWD_PAIRS || (AE_BWD_ROLE == 1 && AE_BWD_KIND == 0 && AE_NWAVES == 8 && AE_RES_VIA_LDS && AE_OUT_VIA_LDS), "pairs");
 static_assert(!AE_BWD_FUSE_DELTA || (AE_RES_VIA_LDS && AE_BWD_KIND == 0), "the fused row sums need the staged resident rows");
 
@@ -225,7 +235,18 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   const int n_rt = (n_res + AE_BR - 1) / AE_BR;
   const int n_bh = p.batch * heads;
   const int n_bg = (n_bh + 7) >> 3;
+#if AE_BWD_SPLIT
+  const int64_t counters_at = ((int64_t)2 * p.batch * p.heads_q * p.seqlen_q + 3) & ~(int64_t)3;
+  const int n_kv_tiles = (p.seqlen_kv + 127) / 128 * p.batch * p.heads_kv;
+#if AE_BWD_ROLE == 0
+  for (int i = blockIdx.x * AE_NT + tid; i < n_kv_tiles; i += gridDim.x * AE_NT) ((int*)(p.delta + counters_at))[i] = 0;
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+#else
+  const int xcd = blockIdx.x & 7, slot = (blockIdx.x >> 3) / p.dkv_parts, part = (blockIdx.x >> 3) % p.dkv_parts;
+#endif
+#else
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+#endif
   const int bh = (slot % n_bg) * 8 + xcd;
 #if AE_BWD_ROLE == 0 && (AE_MASK_MODE == 1 || (AE_MASK_MODE == 2 && AE_HEAVY_LAST))
   // (the q tiles with the most visible keys first: the last ones under a causal mask, and under a tile table
@@ -311,9 +332,12 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   const int n_t = t_hi - t_lo;
   // item x: tile t_lo + x % n_t of q head x / n_t of the group (role 0: one head)
 #if AE_BWD_ROLE == 0
-  const int n_items = n_t;
+  const int x_first = 0, n_items = n_t;
+#elif AE_BWD_SPLIT
+  // (this part's share; n_items: the end of it)
+  const int x_first = (int)((int64_t)n_t * group * part / p.dkv_parts), n_items = (int)((int64_t)n_t * group * (part + 1) / p.dkv_parts);
 #else
-  const int n_items = n_t * group;
+  const int x_first = 0, n_items = n_t * group;
 #endif
   auto item_tile = [&](int x) AE_LAMBDA { return t_lo + (AE_BWD_ROLE == 0 ? x : x % n_t); };
   auto item_head = [&](int x) AE_LAMBDA { return AE_BWD_ROLE == 0 ? h : h * group + x / n_t; };   // q head of the item
@@ -392,15 +416,18 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   // Items are requested, and used, one after the other: what an item's position decides is carried along (a step of
   // one tile, or on to the next head) instead of formed from the item's number, which took a division and six 64-bit
   // products an item of one wave's issue slots.  rq_*: the next item to request; us_t, us_h: tile and head in use.
-  const int str_h = AE_BWD_ROLE == 0 ? hk : h * group;              // the first item's head in the streamed tensors
+  int str_h = AE_BWD_ROLE == 0 ? hk : h * group, str_t = t_lo;      // the first item's head and tile in the streamed tensors
+#if AE_BWD_SPLIT && AE_BWD_ROLE == 1
+  if (x_first < n_items) str_h += x_first / n_t, str_t += x_first % n_t;
+#endif
 #if AE_BWD_ROLE == 0
   const int64_t st1h = p.k_stride_h, st2h = p.v_stride_h;
-  const char* rq_1 = (const char*)((const ae_elem*)p.k + (int64_t)b * p.k_stride_b + (int64_t)str_h * st1h + (int64_t)t_lo * AE_BS * st1);
-  const char* rq_2 = (const char*)((const ae_elem*)p.v + (int64_t)b * p.v_stride_b + (int64_t)str_h * st2h + (int64_t)t_lo * AE_BS * st2);
+  const char* rq_1 = (const char*)((const ae_elem*)p.k + (int64_t)b * p.k_stride_b + (int64_t)str_h * st1h + (int64_t)str_t * AE_BS * st1);
+  const char* rq_2 = (const char*)((const ae_elem*)p.v + (int64_t)b * p.v_stride_b + (int64_t)str_h * st2h + (int64_t)str_t * AE_BS * st2);
 #else
   const int64_t st1h = p.q_stride_h, st2h = p.do_stride_h;
-  const char* rq_1 = (const char*)((const ae_elem*)p.q + (int64_t)b * p.q_stride_b + (int64_t)str_h * st1h + (int64_t)t_lo * AE_BS * st1);
-  const char* rq_2 = (const char*)((const ae_elem*)p.dout + (int64_t)b * p.do_stride_b + (int64_t)str_h * st2h + (int64_t)t_lo * AE_BS * st2);
+  const char* rq_1 = (const char*)((const ae_elem*)p.q + (int64_t)b * p.q_stride_b + (int64_t)str_h * st1h + (int64_t)str_t * AE_BS * st1);
+  const char* rq_2 = (const char*)((const ae_elem*)p.dout + (int64_t)b * p.do_stride_b + (int64_t)str_h * st2h + (int64_t)str_t * AE_BS * st2);
   const float* rq_d[AE_RSL];
 #pragma unroll
   for (int i = 0; i < AE_RSL; i++) {
@@ -410,7 +437,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
   const int64_t step1 = AE_BS * st1 * 2, step2 = AE_BS * st2 * 2;
   const int64_t wrap1 = st1h * 2 - (n_t - 1) * step1, wrap2 = st2h * 2 - (n_t - 1) * step2;
-  int rq_x = 0, rq_t = t_lo, us_t = t_lo, us_h = AE_BWD_ROLE == 0 ? h : str_h;
+  int rq_x = x_first, rq_t = str_t, us_t = str_t, us_h = AE_BWD_ROLE == 0 ? h : str_h;
   (void)wrap1, (void)wrap2;
 #endif
   // request item x (past the end: the last item again, so that every call issues AE_NLOADS loads) into the stage at byte `stage`
@@ -548,7 +575,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 
   // the n-th visited item is multiplied out of stage n % NSTAGE while the next two are on their way
   int cls0, cls1, cls2;                 // ... and the classes of those three items
-  int x0 = next_item(0, cls0), x1 = next_item(x0 + 1, cls1), x2 = next_item(x1 + 1, cls2);
+  int x0 = next_item(x_first, cls0), x1 = next_item(x0 + 1, cls1), x2 = next_item(x1 + 1, cls2);
 #if AE_RES_VIA_LDS
   if (x0 < n_items) request_item(x0, 0);
   if (AE_BWD_PAIRS && wave >= AE_NRW) {
@@ -976,6 +1003,53 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
   __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));             // nothing may land in LDS after the workgroup has gone
 
+#if AE_BWD_SPLIT && AE_BWD_ROLE == 1
+  // Device-scope accesses (sc1): another part's workgroup may sit on another XCD, with its own L2.  Every wave waits for its
+  // stores to be acknowledged before the workgroup counts itself in.
+  constexpr int kDeviceScope = 16;
+  constexpr int NB = AE_NDB1 + AE_NDB2, kPartBytes = AE_NRW * NB * 4096;
+  const int part_tile = rt * n_bh + bh;
+  __amdgpu_buffer_rsrc_t part_buf = __builtin_amdgcn_make_buffer_rsrc(
+      p.delta + counters_at + ((n_kv_tiles + 3) & ~3) + (int64_t)part_tile * p.dkv_parts * (kPartBytes / 4), 0,
+      p.dkv_parts * kPartBytes, 0x00020000);
+  int part_at = lane;
+  asm volatile("" : "+v"(part_at));
+  part_at = rw * NB * 4096 + part_at * 16;
+  {
+    auto quad = [&](int j) AE_LAMBDA -> ae_f32x4 {          // registers 4 (j % 4) .. + 3 of block j / 4: dk's blocks, then dv's
+      const ae_f32x16& a = j / 4 < AE_NDB1 ? acc1[j / 4 < AE_NDB1 ? j / 4 : 0] : acc2[j / 4 < AE_NDB1 ? 0 : j / 4 - AE_NDB1];
+      return ae_f32x4{a[j % 4 * 4], a[j % 4 * 4 + 1], a[j % 4 * 4 + 2], a[j % 4 * 4 + 3]};
+    };
+#pragma unroll
+    for (int j = 0; j < NB * 4; j++)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(ae_u32x4, quad(j)), part_buf, part_at + j * 1024, part * kPartBytes, kDeviceScope);
+    __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
+    __syncthreads();                                        // (and every wave has left the ring)
+    ae_lds_byte* const flag = lds;
+    if (rw == 0 && lane == 0) {
+      const int seen = __hip_atomic_fetch_add((int*)(p.delta + counters_at) + part_tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *(__attribute__((address_space(3))) int*)flag = seen == p.dkv_parts - 1;
+    }
+    __syncthreads();
+    if (*(__attribute__((address_space(3))) int*)flag == 0) return;
+  }
+  // the sum of the parts, one output's registers at a time; the own part comes back from memory too: the order of the sum
+  // does not depend on who was last
+  auto merge_parts = [&](auto& acc, int j_first) AE_LAMBDA {
+    constexpr int N = (int)(sizeof(acc) / sizeof(acc[0])) * 4;
+    clear(acc);
+    for (int k = 0; k < p.dkv_parts; k++) {
+      ae_f32x4 w[N];
+#pragma unroll
+      for (int j = 0; j < N; j++)
+        w[j] = __builtin_bit_cast(ae_f32x4, __builtin_amdgcn_raw_buffer_load_b128(part_buf, part_at + (j_first + j) * 1024, k * kPartBytes, kDeviceScope));
+#pragma unroll
+      for (int j = 0; j < N; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[j / 4][j % 4 * 4 + r] += w[j][r];
+    }
+  };
+#endif
   // ---- results: lane owns its resident row, columns 32*db + 8*(r/4) + 4*hf + r%4 ------------------
 #if AE_OUT_VIA_LDS
   __syncthreads();       // ... of any wave: the ring becomes the staging area of the results
@@ -984,6 +1058,9 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
     int le = lane;
     asm volatile("" : "+v"(le));
     ae_lds_byte* os1 = lds + rw * AE_OUT_BYTES;
+#if AE_BWD_SPLIT && AE_BWD_ROLE == 1
+    merge_parts(acc1, 0);
+#endif
     {
       ae_lds_byte* orow = os1 + (le & 31) * AE_STR1 + (le >> 5) * 8;
       const int osw = le & (AE_CPR1 - 1);
@@ -998,6 +1075,9 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
         }
     }
 #if AE_BWD_ROLE == 1
+#if AE_BWD_SPLIT
+    merge_parts(acc2, 4 * AE_NDB1);
+#endif
     {
       ae_lds_byte* orow = os1 + AE_R1B + (le & 31) * AE_STR2 + (le >> 5) * 8;
       const int osw = le & (AE_CPR2 - 1);
@@ -1044,6 +1124,10 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   }
   (void)r_ok;
 #else
+#if AE_BWD_SPLIT && AE_BWD_ROLE == 1
+  merge_parts(acc1, 0);
+  merge_parts(acc2, 4 * AE_NDB1);
+#endif
   if (r_ok) {
 #if AE_BWD_ROLE == 0
     ae_elem* o1 = (ae_elem*)p.dq + (int64_t)b * p.dq_stride_b + (int64_t)rrow * p.dq_stride_s + (int64_t)h * p.dq_stride_h;

@@ -186,7 +186,11 @@ typedef struct ae_attn_bwd_params {
   int32_t batch, heads_q, heads_kv, seqlen_q, seqlen_kv;
   int32_t mask_b, mask_h;  /* batch / head extents of the two tables (and of block_mask): 1 or (B, Hq) */
   int32_t mask_nq, mask_nkv, mask_block_m, mask_block_n;  /* geometry of block_mask (0 without one)   */
-  int32_t reserved[1];
+  /* kernels compiled with AE_BWD_SPLIT 1 (announced by cfg->merge_in_wg = 2): workgroups per kv tile of the dk/dv launch,
+   * 2 .. 64.  `delta` then has, behind its two planes (their length rounded up to a multiple of 4), ceil(Skv/128) * B * Hkv
+   * arrival counters (rounded up likewise; the dq launch clears them) and, per kv tile, dkv_parts * 128 * (D + DV) floats
+   * of partial sums.  Ignored otherwise. */
+  int32_t dkv_parts;
 } ae_attn_bwd_params;
 
 typedef struct ae_devinfo {

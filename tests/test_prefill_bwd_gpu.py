@@ -402,3 +402,63 @@ def test_backward_of_other_graphs_is_refused(cuda_device):
     with pytest.raises(NotImplementedError, match="no backward for this engine"):
         out.sum().backward()
     assert qg.grad is None
+
+
+@pytest.mark.parametrize("B,H,Hkv,Sq,Skv,D,dtype,causal,parts", [
+    (1, 8, 2, 333, 333, 128, torch.bfloat16, True, 3),      # ragged; the last kv tile has 4 heads x 2 items
+    (2, 4, 1, 700, 700, 64, torch.float16, True, 6),
+    (1, 2, 2, 130, 130, 128, torch.float16, True, 4),       # the second kv tile has one item: three parts without any
+    (1, 4, 2, 200, 520, 64, torch.bfloat16, False, 2),      # no mask, unequal lengths
+    (1, 4, 4, 65, 1, 128, torch.bfloat16, False, 2),        # one key
+])
+def test_backward_kv_tiles_shared_by_workgroups(cuda_device, monkeypatch, B, H, Hkv, Sq, Skv, D, dtype, causal, parts):
+    """dk/dv launches that share a kv tile out (AE_BWD_SPLIT): gradients as the oracle's, the same bits on every call (the
+    parts are added in their order, whoever finishes last) and on every replay of a graph, with eager calls in between."""
+    scale = 1 / math.sqrt(D)
+    print(f"case shared kv tiles B{B} H{H}/{Hkv} {Sq}x{Skv} D{D} {dtype} causal={causal} parts={parts}", flush=True)
+    q, k, v = C.make_inputs(B, Sq, Skv, H, Hkv, D, D, dtype, seed=31)
+    dout = torch.randn(B, Sq, H, D, generator=torch.Generator().manual_seed(32)).to(dtype)
+    mod = _engine(B, H, Hkv, Sq, D, D, dtype, C.causal_mask if causal else None, scale)
+    op = mod._op.backward_op()
+    monkeypatch.setattr(op, "dkv_parts", lambda *a: parts)
+    ref = R.softmax_attention_grads(q, k, v, dout, scale=scale, causal=causal)
+    leaves = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    do = dout.cuda()
+
+    def step():
+        return torch.autograd.grad(mod(*leaves), leaves, do)
+    first = step()                                   # through Python
+    for got, want, what in zip(first, ref, ("dq", "dk", "dv")):
+        _check(got, want, what, (B, H, Hkv, Sq, Skv, D, parts))
+    for _ in range(3):                               # through the native host path
+        assert all(torch.equal(a, b) for a, b in zip(step(), first))
+    torch.cuda.synchronize()
+    qd, kd, vd = (t.detach() for t in leaves)
+    out, rs = mod.forward_with_rowscales(qd, kd, vd)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        grads = op(qd, kd, vd, out, rs["lse"], do)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(grads, first))
+        step()
+
+
+@pytest.mark.parametrize("S,rows", [(1000, 128), (4097, 256)])
+def test_backward_rows_of_the_dq_launch_follow_the_problem(cuda_device, S, rows):
+    """Few 256-row q tiles are halved; an engine whose caller chose keeps that choice."""
+    B, H, D, dtype = 1, 16, 128, torch.bfloat16
+    mod = _engine(B, H, H, S, D, D, dtype, C.causal_mask, 1 / math.sqrt(D))
+    op = mod._op.backward_op()
+    assert op.rows_of_dq(B, H, S, True, True) == rows
+    from core.lower.prefill_bwd_op import PrefillBwdOp
+    assert PrefillBwdOp(mod._op, *op._graph, dq_rows=256).rows_of_dq(B, H, S, True, True) == 256
+    q, k, v = C.make_inputs(B, S, S, H, H, D, D, dtype, seed=5)
+    dout = torch.randn(B, S, H, D, generator=torch.Generator().manual_seed(6)).to(dtype)
+    leaves = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    got = torch.autograd.grad(mod(*leaves), leaves, dout.cuda())
+    one = [t[:, :, 3:4] for t in (q, k, v, dout)]
+    ref = R.softmax_attention_grads(*one, scale=1 / math.sqrt(D), causal=True)
+    for g, want, what in zip(got, ref, ("dq", "dk", "dv")):
+        _check(g[:, :, 3:4], want, what, (S, rows))
