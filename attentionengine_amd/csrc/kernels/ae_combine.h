@@ -32,7 +32,7 @@ void ae_decode_combine_kernel(const ae_attn_params p) {
   // The partial results are read 16 splits at a time, unconditionally, so that the loads of a group all go
   // out before the first one is waited for (one memory round trip per group instead of one per split: the
   // merge of 32 splits 18 -> 4 us).  Splits that wrote nothing re-read the last one that did, with weight 0.  The row
-  // scales are read the same way, behind the first group, whose weights they are: one trip to memory for both (B8 H128,
+  // scales are read the same way, in front of the first group, whose weights they are: one trip to memory for both (B8 H128,
   // paged, 16 splits: the call 22.2 -> 21.5 us).
   constexpr int G = AE_NSPLIT < 16 ? AE_NSPLIT : 16;
   const float* part = p.partial_o + row * AE_DV;
@@ -46,16 +46,19 @@ void ae_decode_combine_kernel(const ae_attn_params p) {
     }
   };
   const int dv0 = (threadIdx.x % TPR) * 4;
-  ae_f32x4 val[G];
-  load_group(val, 0, dv0);
   float rs[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1][AE_NSPLIT];
 #pragma unroll
   for (int i = 0; i < AE_N_ROWSCALES; i++)
 #pragma unroll
-    for (int k = 0; k < AE_NSPLIT; k++) {
-      const float r = p.partial_rs[(int64_t)i * p.batch * p.heads_q * AE_NSPLIT + row + (k < n_used ? k : n_used - 1)];
-      rs[i][k] = k < n_used ? r : AE_NEG_INF;
-    }
+    for (int k = 0; k < AE_NSPLIT; k++)
+      rs[i][k] = p.partial_rs[(int64_t)i * p.batch * p.heads_q * AE_NSPLIT + row + (k < n_used ? k : n_used - 1)];
+  ae_f32x4 val[G];
+  load_group(val, 0, dv0);
+  __builtin_amdgcn_sched_barrier(0);             // (left alone the compiler moves the loads behind the weights)
+#pragma unroll
+  for (int i = 0; i < AE_N_ROWSCALES; i++)
+#pragma unroll
+    for (int k = 0; k < AE_NSPLIT; k++) rs[i][k] = k < n_used ? rs[i][k] : AE_NEG_INF;
   float w[AE_NSPLIT];
   float merged[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1];
   ae_combine(rs, w, merged);

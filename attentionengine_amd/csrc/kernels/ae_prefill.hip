@@ -147,6 +147,7 @@ static_assert(AE_KCPR == 8 || AE_KCPR == 16 || AE_KCPR == 32 || AE_KCPR % 8 == 4
 static_assert(AE_VCPR == 8 || AE_VCPR == 16 || AE_VCPR == 32 || AE_VCPR == 64, "swizzle is written for 128- to 1024-byte V rows");
 
 typedef __attribute__((address_space(3))) unsigned char ae_lds_byte;
+template <bool B> struct ae_const_bool { static constexpr bool value = B; };
 
 // LDS chunk of K row `row` that holds global chunk c (and the other way round: an involution).  A fragment read
 // (ds_read_b128) takes one chunk index of 16 consecutive rows; they must fall into 16 different groups of four
@@ -864,24 +865,63 @@ void ae_prefill_kernel(const ae_attn_params p) {
     };
 #if AE_NSPLIT > 1
     // partial result of this split: fp32, rows ordered (batch, q position, head) so that the merge
-    // kernel sees them as B x (Sq*Hq) "heads" of a one-token decode and writes out [B,Sq,Hq,DV]
-    if (q_ok[rb]) {
-      const int64_t prow = ((((int64_t)b * p.seqlen_q + qrow[rb]) * p.heads_q + h) * AE_NSPLIT) + split;
-      float* po = p.partial_o + prow * AE_DV;
+    // kernel sees them as B x (Sq*Hq) "heads" of a one-token decode and writes out [B,Sq,Hq,DV].  O leaves through the
+    // wave's share of the tile ring, a row's columns as one contiguous piece: straight from the accumulators a
+    // store instruction writes 16 bytes of each of 64 rows, lines that the L2 has to put together out of eight pieces.  Up
+    // to 12 MB of them go past the caches, which have less to write back when the launch ends; more of them wait for
+    // memory beside the cache's reads.  B5 H8 Sq77 Skv842 D128 (8 MB): the call 16.9 us, 17.3 through the caches, 15.0 past
+    // them; B1 H32 Sq128 Skv8192 (17 MB): 42.7, 42.2, 43.4.
+    {
+      constexpr int REGION = 2 * AE_STAGE_BYTES / AE_NWAVES;                            // bytes of LDS a wave may use
+      constexpr int NP = 32 * AE_DV * 4 <= REGION ? 1 : (16 * AE_DV * 4 <= REGION ? 2 : 4);   // passes over the columns
+      constexpr int CPR = AE_DV / 4 / NP;                                               // 16-byte chunks of a row and pass
+      constexpr int SW = (CPR & -CPR) < 32 ? (CPR & -CPR) - 1 : 31;
+      static_assert(AE_RB == 1 && 32 * CPR * 16 <= REGION && AE_NDB % NP == 0 && 32 * CPR % 64 == 0, "the rows fit the wave's share of the tile ring");
+      typedef __attribute__((address_space(3))) ae_f32x4 lds_f4;
+      int le = lane;
+      asm volatile("" : "+v"(le));
+      ae_lds_byte* os = lds + wave * REGION;
+      const int64_t row0 = ((int64_t)b * p.seqlen_q + q0w) * p.heads_q + h;
+      const bool past = (int64_t)p.batch * p.seqlen_q * p.heads_q * (AE_NSPLIT * AE_DV * 4) <= 12 << 20;
 #pragma unroll
-      for (int db = 0; db < AE_NDB; db++)
+      for (int ps = 0; ps < NP; ps++) {
+        ae_lds_byte* orow = os + (le & 31) * (CPR * 16);
 #pragma unroll
-        for (int rg = 0; rg < 4; rg++) {
-          ae_f32x4 w;
+        for (int db = 0; db < AE_NDB / NP; db++)
 #pragma unroll
-          for (int t = 0; t < 4; t++) w[t] = live ? o[db * 16 + rg * 4 + t] : 0.f;
-          *(ae_f32x4*)(po + db * 32 + rg * 8 + hf * 4) = w;
+          for (int rg = 0; rg < 4; rg++) {
+            ae_f32x4 w;
+#pragma unroll
+            for (int t = 0; t < 4; t++) w[t] = live ? o[(ps * (AE_NDB / NP) + db) * 16 + rg * 4 + t] : 0.f;
+            *(lds_f4*)(orow + (((db * 8 + rg * 2 + (le >> 5)) ^ (le & SW)) << 4)) = w;
+          }
+        // (the rows were written by other lanes of this wave: LDS instructions of a wave complete in order)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        auto leave = [&](auto past_tag) AE_LAMBDA {
+#pragma unroll 8
+          for (int i = 0; i < 32 * CPR / 64; i++) {
+            const int row = (i * 64 + le) / CPR, c = (i * 64 + le) % CPR;
+            const ae_f32x4 w = *(const lds_f4*)(os + row * (CPR * 16) + ((c ^ (row & SW)) << 4));
+            ae_f32x4* at = (ae_f32x4*)(p.partial_o + ((row0 + (int64_t)row * p.heads_q) * AE_NSPLIT + split) * AE_DV + (ps * CPR + c) * 4);
+            if (AE_EVEN_Q || q0w + row < p.seqlen_q) {
+              if (decltype(past_tag)::value) __builtin_nontemporal_store(w, at);
+              else *at = w;
+            }
+          }
+        };
+        if (past) {
+          asm volatile("" ::: "memory");                 // (else the two loops become one, of plain stores)
+          leave(ae_const_bool<true>());
+        } else {
+          leave(ae_const_bool<false>());
         }
-      if (hf == 0) {
-#pragma unroll
-        for (int i = 0; i < AE_N_ROWSCALES; i++)
-          p.partial_rs[(int64_t)i * p.batch * p.seqlen_q * p.heads_q * AE_NSPLIT + prow] = frs[i];
       }
+    }
+    if (q_ok[rb] && hf == 0) {
+      const int64_t prow = ((((int64_t)b * p.seqlen_q + qrow[rb]) * p.heads_q + h) * AE_NSPLIT) + split;
+#pragma unroll
+      for (int i = 0; i < AE_N_ROWSCALES; i++)
+        p.partial_rs[(int64_t)i * p.batch * p.seqlen_q * p.heads_q * AE_NSPLIT + prow] = frs[i];
     }
 #elif AE_O_VIA_LDS
     {
