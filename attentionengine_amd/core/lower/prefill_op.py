@@ -154,7 +154,7 @@ class PrefillOp:
                     self.mask_block[1] % self.tiles.block_n or \
                     self.tiles.block_m > self.MASK_ROWS_PER_TILE * self.mask_block[0]:
                 raise NotImplementedError(f"block mask granularity {self.mask_block} does not fit the tiles")
-        if self.tiles.kv_groups == 1:
+        if self.tiles.kv_groups == 1 and self.tiles is not groups:
             self._base = self.tiles
         if self._tiles_given or self.extern_block_mask or self._tune_found:
             self._table_tiles = self._base
@@ -242,7 +242,7 @@ class PrefillOp:
                 or any(c.per_kv for c in self.functors.customs) or os.environ.get("AE_PREFILL_KERNEL", "")):
             return None
         if self.split_kv:
-            return L.kv_group_tiles_split(Sq) if self.mask_mod is None else None
+            return L.kv_group_tiles_split(Sq, B * H) if self.mask_mod is None else None
         found = L.kv_group_tiles(self.D, self.DV, B * H, Sq, Skv, self.mask_mod is not None)
         if found is not None and self.mask_mod is not None:
             lm = self.functors.mask
@@ -256,7 +256,7 @@ class PrefillOp:
     def tiles_for(self, B, H, Sq, Skv):
         """The tile configuration of a call with these extents."""
         key = (B, H, Sq, Skv)
-        if self.tiles.kv_groups == 1 or key == self._declared:
+        if key == self._declared or (self.tiles.kv_groups == 1 and self.tiles is not self._groups):
             return self.tiles
         tiles = self._call_tiles.get(key)
         if tiles is None:

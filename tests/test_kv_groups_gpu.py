@@ -71,6 +71,26 @@ def test_kv_groups_of_split_launches(cuda_device, Sq, Skv):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,Sq,Skv", [(1, 3, 65, 700), (2, 5, 127, 1000), (1, 2, 193, 2100), (1, 3, 256, 1030), (8, 16, 200, 500), (1, 1, 300, 2000)])
+def test_partial_results_of_split_launches(cuda_device, B, H, Sq, Skv, D):
+    """Rows that end inside a wave, a wave without rows, 256-row workgroups (two passes over the columns), a row's columns
+    of 64 and 128; through Python, then natively."""
+    dtype = torch.float16
+    print(f"case partial results B{B} H{H} {Sq}x{Skv} D{D}", flush=True)
+    q, k, v = C.make_inputs(B, Sq, Skv, H, H, D, D, dtype, seed=9)
+    meta = (meta_tensor(B, H, Sq, D, dtype=dtype), meta_tensor(B, H, Skv, D, dtype=dtype), meta_tensor(B, H, Skv, D, dtype=dtype))
+    mod = AttentionEngine(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), None, C.OnlineSoftmax())
+    assert mod._op.tiles.block_m == (256 if 192 < Sq <= 256 and B * H <= 64 else 128)
+    assert mod._op.tiles_for(B, H, 100, Skv) == PrefillTiles()
+    ref, lse = R.softmax_attention(q, k, v, causal=False)
+    for _ in range(2):
+        out = mod(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+        assert (out - ref).abs().max().item() <= 2e-2
+        assert (mod.final_rowscales["lse"].cpu() - lse).abs().max().item() <= 1e-3
+
+
+@pytest.mark.gpu
 def test_kv_groups_of_graphs_without_row_state(cuda_device):
     B, H, S, D, dtype = 1, 2, 200, 64, torch.float16
     q, k, v = C.make_inputs(B, S, S, H, H, D, D, dtype, seed=3)
