@@ -89,10 +89,11 @@ void ae_decode_split_kernel(const ae_attn_params p) {
   ae_lds_byte* vs = (ae_lds_byte*)ae_smem + wave * AE_V_WAVE_BYTES;
 
   // ---- which (batch, kv head, head tile, split) ------------------------------------------------
-  const int group = p.heads_q / p.heads_kv;
+  // (one head tile a kv head, a power of two of kv heads: no integer division in front of the first request)
+  const int group = (p.heads_kv & (p.heads_kv - 1)) == 0 ? p.heads_q >> __builtin_ctz(p.heads_kv) : p.heads_q / p.heads_kv;
   const int b = blockIdx.z;
-  const int hk = blockIdx.y % p.heads_kv;
-  const int ht = blockIdx.y / p.heads_kv;
+  int hk = blockIdx.y, ht = 0;
+  if (__builtin_expect((int)gridDim.y != p.heads_kv, 0)) hk = blockIdx.y % p.heads_kv, ht = blockIdx.y / p.heads_kv;
   const int split = blockIdx.x * AE_NWAVES + wave;       // index of this wave's partial
   const int head_in_group = ht * 16 + l16;
   const bool head_ok = head_in_group < group;
@@ -163,9 +164,9 @@ void ae_decode_split_kernel(const ae_attn_params p) {
   for (int db = 0; db < AE_NDB; db++) oacc[db] = (ae_f32x4){0.f, 0.f, 0.f, 0.f};
 
   // tiles of this wave that start inside the sequence
-  int my_tiles = 0;
-  for (int i = 0; i < n_tiles; i++)
-    if (tile_kv0(i) < p.seqlen_kv) my_tiles = i + 1;
+  int my_tiles = p.seqlen_kv - wg_base - wave * AE_TILE;
+  my_tiles = my_tiles > 0 ? (my_tiles + AE_NWAVES * AE_TILE - 1) / (AE_NWAVES * AE_TILE) : 0;
+  my_tiles = __builtin_amdgcn_readfirstlane(my_tiles < n_tiles ? my_tiles : n_tiles);
 
   if (my_tiles > 0) {
     load_k(tile_kv0(0), kf);
