@@ -36,6 +36,26 @@ typedef unsigned int ae_u32x2 __attribute__((ext_vector_type(2)));
 #define AE_LOG2E 1.4426950408889634f
 #define AE_LN2 0.6931471805599453f
 
+// Quotient and remainder of wave-uniform numbers, a >= 0 and d > 0.  The compiler's division is a chain of some thirty
+// dependent instructions, and which tile a workgroup has takes four of them in front of its first request: a shift where d
+// is a power of two, else a reciprocal whose quotient is off by at most one below 2^22.
+AE_DEV int ae_divide(int a, int d, int& rem) {
+  int q;
+  if ((d & (d - 1)) == 0) {
+    q = a >> __builtin_ctz(d);
+    rem = a & (d - 1);
+  } else if (__builtin_expect(a < 1 << 22, 1)) {
+    q = __builtin_amdgcn_readfirstlane((int)((float)a * __builtin_amdgcn_rcpf((float)d)));
+    rem = a - q * d;
+    if (rem < 0) q--, rem += d;
+    if (rem >= d) q++, rem -= d;
+  } else {
+    q = a / d;
+    rem = a - q * d;
+  }
+  return q;
+}
+
 // D[m][n] += sum_k A[m][k] B[k][n], 32x32 output, 16-deep. Lane l supplies A[l%32][8*(l/32)+j]
 // and B[8*(l/32)+j][l%32], j=0..7, and owns D[8*(r/4) + 4*(l/32) + r%4][l%32], r=0..15.
 AE_DEV ae_f32x16 ae_mfma32(ae_elem8 a, ae_elem8 b, ae_f32x16 c) {

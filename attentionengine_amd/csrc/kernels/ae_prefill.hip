@@ -254,16 +254,17 @@ void ae_prefill_kernel(const ae_attn_params p) {
   // late q tiles are the long ones (AE_HEAVY_LAST, found on the host: causal variants, long sliding windows)
   // takes the same order: B2 H32 S4096, "kv <= q + 1": 0.40 -> 0.35 ms.
   const int n_bg = (n_bh + 7) >> 3;
-  const int qt = n_qt - 1 - slot / n_bg;
-  const int bh = (slot % n_bg) * 8 + xcd;
+  int bh;
+  const int qt = n_qt - 1 - ae_divide(slot, n_bg, bh);
+  bh = bh * 8 + xcd;
 #else
-  const int qt = slot % n_qt;
-  const int bh = (slot / n_qt) * 8 + xcd;
+  int qt;
+  const int bh = ae_divide(slot, n_qt, qt) * 8 + xcd;
 #endif
   if (bh >= n_bh) return;
-  const int h = bh % p.heads_q;
-  const int b = bh / p.heads_q;
-  const int hk = h / (p.heads_q / p.heads_kv);
+  int h, rest;
+  const int b = ae_divide(bh, p.heads_q, h);
+  const int hk = p.heads_q == p.heads_kv ? h : ae_divide(h, ae_divide(p.heads_q, p.heads_kv, rest), rest);
   const int q0 = qt * AE_BM;
   const int q0w = q0 + wave * AE_WROWS;       // first row of this wave
   int qrow[AE_RB];                             // this lane's row in each row block
