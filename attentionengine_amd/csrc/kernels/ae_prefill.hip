@@ -237,6 +237,12 @@ void ae_prefill_kernel(const ae_attn_params p) {
   // concurrently, walk the kv axis roughly in step and share K/V through that XCD's L2.
   // With a causal mask the tiles with the most kv work (last q-tiles) are issued first.
   // The grid is padded to 8*ceil(n_bh/8)*n_qt ids; surplus workgroups exit immediately.
+  // (All arguments that the requests of the first tile need are read here, in one trip to memory: where they are first
+  // used the compiler reads them in three, each waited for, with the arithmetic of the ids between them.)
+  asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.batch), "s"(p.heads_q), "s"(p.heads_kv), "s"(p.seqlen_q),
+               "s"(p.seqlen_kv), "s"(p.q_stride_b), "s"(p.q_stride_s), "s"(p.q_stride_h));
+  asm volatile("" ::"s"(p.k_stride_b), "s"(p.k_stride_s), "s"(p.k_stride_h), "s"(p.v_stride_b), "s"(p.v_stride_s),
+               "s"(p.v_stride_h));
   const int n_qt = (p.seqlen_q + AE_BM - 1) / AE_BM;
   const int n_bh = p.batch * p.heads_q;
 #if AE_NSPLIT > 1
