@@ -610,6 +610,34 @@ def test_decode_and_prefill_replay_from_a_hip_graph(cuda_device):
     assert (got_d.float().cpu() - ref).abs().max().item() <= OUT_TOL
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Skv,D,x,dtype", [
+    (2, 8, 2, 1001, 128, 3, torch.float16),     # no power of two; the last workgroup's last tile is cut
+    (1, 40, 2, 1500, 128, 5, torch.bfloat16),   # two head tiles a kv head; the fifth workgroup has no keys
+    (3, 16, 4, 2050, 64, 10, torch.float16),
+    (1, 8, 2, 8200, 128, 20, torch.bfloat16),   # the merge's second group of partial results is not full; three are empty
+])
+def test_gqa_decode_any_number_of_workgroups(cuda_device, monkeypatch, B, Hq, Hkv, Skv, D, x, dtype):
+    """Kv axes shared by a number of workgroups that is no power of two, merged by the last of them and by the merge
+    kernel: the same result to the last bit, and the oracle's."""
+    print(f"case gqa decode B{B} Hq{Hq} Hkv{Hkv} Skv{Skv} D{D} workgroups {x} {dtype}", flush=True)
+    q, k, v = C.make_inputs(B, 1, Skv, Hq, Hkv, D, D, dtype, seed=x)
+    ref, rlse = R.softmax_attention(q, k, v, causal=False)
+    got = []
+    for last in ("1", "0"):
+        monkeypatch.setenv("AE_DECODE_MERGE_LAST", last)
+        mod = _decode_engine(B, Hq, Hkv, Skv, D, D, dtype, C.make_scale_score_mod(1 / math.sqrt(D)), C.OnlineSoftmax())
+        op = mod.attention
+        op._workgroups = lambda *a: x
+        assert op.plan_splits(B, Hq, Hkv, Skv)[0] == x * op.N_WAVES
+        for _ in range(2):                       # through Python, then through the native host path
+            out = mod(q.cuda(), k.cuda(), v.cuda())
+            lse = mod.final_rowscales["lse"]
+            assert (out.float().cpu() - ref).abs().max().item() <= OUT_TOL
+            assert (lse.cpu().view(-1) - rlse.view(-1)).abs().max().item() <= LSE_TOL
+            got.append((out.clone(), lse.clone()))
+    assert all(torch.equal(a, b) for g in got[1:] for a, b in zip(got[0], g))
+
+
 @pytest.mark.parametrize("Skv,used", [(3001, 700), (8192, 33), (3001, 3001)])
 @pytest.mark.parametrize("merge_last", ["1", "0"])
 def test_a_workgroup_whose_keys_are_all_masked_adds_nothing(cuda_device, monkeypatch, Skv, used, merge_last):

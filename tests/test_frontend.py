@@ -822,3 +822,32 @@ def test_mla_plan():
     assert per // 64 + 2 <= op.PAGE_TABLE_ENTRIES and n_split * per >= 300000
     op.target_workgroups = 1
     assert op.plan(2, 128, 1, 1000) == (64, 1, 1024)
+
+
+def test_gqa_plan():
+    """Any number of workgroups of a kv axis is one that a kernel is built for, with a tile for every wave, and fits the
+    built-in work buffer; keys are covered; a combine() that wants every partial result keeps a power of two."""
+    from core.lower.lower_decode import GQADecodeOp
+    from core.runtime import hip_rt as rt
+    dt = torch.float16
+    meta = (meta_tensor(1, 8, 1, 128, dtype=dt), meta_tensor(1, 2, 64, 128, dtype=dt), meta_tensor(1, 2, 64, 128, dtype=dt))
+    op = GQADecodeOp(meta, CustomIO({}), C.make_scale_score_mod(0.1), None, C.OnlineSoftmax(), "-inf")
+    assert op.grouped_merge
+    for B in (1, 3, 17, 128):
+        for Hq, Hkv in ((8, 2), (32, 4), (40, 2), (64, 8)):
+            for Skv in (1, 33, 300, 2204, 13634, 32768):
+                n_split, per = op.plan_splits(B, Hq, Hkv, Skv)
+                x = n_split // op.N_WAVES
+                assert x in op.GROUPED_WGS_PER_KV_HEAD and n_split % op.N_WAVES == 0 and per % op.TILE == 0
+                assert n_split * per >= Skv and x <= max(1, -(-Skv // op.TILE) // op.N_WAVES)
+                assert x == 1 or B * Hq * n_split * (op.DV + 1) * 4 <= rt.NOALLOC_SCRATCH_BYTES
+    assert op.plan_splits(67, 32, 4, 13634)[0] // op.N_WAVES == 3      # 804 workgroups of a third, not 268 of all keys
+    assert op.plan_splits(64, 32, 8, 8001)[0] == op.N_WAVES            # 512 workgroups: two a CU
+    op._tuned[(1, 8, 2, 8192)] = 16
+    assert op.plan_splits(1, 8, 2, 8192)[0] == 16 * op.N_WAVES
+    op.grouped_merge = False
+    for B in (1, 5, 33):
+        x = op.plan_splits(B, 32, 4, 9000)[0] // op.N_WAVES
+        assert x & (x - 1) == 0
+    op.grouped_merge, op.target_workgroups = True, 1
+    assert op.plan_splits(2, 8, 2, 4096)[0] == op.N_WAVES
