@@ -8,6 +8,7 @@ rowscales, launches on torch's current stream, returns ``o``.
 """
 from __future__ import annotations
 
+import functools
 import os
 from dataclasses import astuple
 
@@ -332,11 +333,44 @@ class PrefillOp:
     # ---- kernels -------------------------------------------------------------------------
     COMBINE_THREADS = 128
 
+    # microseconds of a workgroup's start and end, and of a trip over its kv groups' next tiles, by the rows of its q tile
+    SPLIT_COST = {32: (3.0, 0.92), 64: (1.8, 0.66), 128: (1.3, 0.91), 256: (5.2, 1.39)}
+
+    @classmethod
+    @functools.lru_cache(maxsize=1024)
+    def _cheapest_splits(cls, wgs, rows, kv_tiles, block_m, block_n, kv_groups, width, cus, heads):
+        """Kv tiles of a split, for launches that one split for every CU would leave with two workgroups on some CUs and
+        one on the others: two share a CU's issue slots and its lines on the way, so that the launch takes as long as two
+        rounds.  A call takes its rounds of starts and trips (half rounds beyond the second, where workgroups no longer
+        end together), at least what memory needs for the cache (8.4 TB/s while the memory-side cache holds it, else 6.2),
+        and the partial results: written and merged.  Fitted to 1926 timings (150 shapes, batch 1 to 8, 8 to 32 heads, 1
+        to 256 rows, 512 to 16384 keys, D128): 1 % above the best count on average.  Measured, one split for every CU ->
+        this: B7 H16 Sq31 Skv522 17.6 -> 9.2 us, B6 H16 Sq25 Skv1118 22.0 -> 15.3, B6 H8 Sq78 Skv2854 26.1 -> 21.6,
+        B3 H32 Sq2 Skv9161 109 -> 88.  ``width``: bytes of a key and a value row in units of 512."""
+        start, trip = cls.SPLIT_COST[block_m]
+        read = heads * kv_tiles * block_n * 512e-6 * width
+        read /= 8.4 if read <= 300 else 6.2
+        best = []
+        for x in range(1, min(64, kv_tiles) + 1):
+            per = -(-kv_tiles // x)
+            if -(-kv_tiles // per) != x:
+                continue
+            rounds, r = -(-wgs * x // cus), wgs * x / cus
+            if r > 8 and x > 1:
+                break
+            if r > 2:
+                rounds = 0.5 * (rounds + r) + 0.26
+            body = rounds * (start + trip * width * -(-per // kv_groups))
+            merge = 2.7 + 0.056 * x + 0.285 * rows * x * 512e-6 * width if x > 1 else 0.0
+            best.append((2.3 + (body ** 1.85 + read ** 1.85) ** (1 / 1.85) + merge, per))
+        least = min(best)[0]
+        return next(per for us, per in best if us <= 1.01 * least)
+
     def plan_splits(self, B, Hq, Sq, Skv, tiles=None):
         """(number of KV splits, kv positions per split): a workgroup for every CU of the chip (more splits cost
         more in partial results and their merge than they gain: B1 H32 Sq128 Skv8192, the shape of
         attn_script/mha_inference.py, 43 us with 8 splits, 44 with 16, 75 with 32), whole kv tiles per split, no
-        empty split."""
+        empty split.  Where that leaves some CUs with two workgroups the cheapest count is taken (``_cheapest_splits``)."""
         if not self.split_kv:
             return 1, Skv
         tiles = tiles or self.tiles_for(B, Hq, Sq, Skv)
@@ -345,6 +379,9 @@ class PrefillOp:
         wgs = -(-Sq // tiles.block_m) * (-(-(B * Hq) // 8) * 8)
         want = max(1, min(kv_tiles, -(-self.target_workgroups // wgs)))
         per = -(-kv_tiles // want)
+        if wgs * -(-kv_tiles // per) > self.target_workgroups and tiles.block_m in self.SPLIT_COST:
+            per = self._cheapest_splits(wgs, B * Hq * Sq, kv_tiles, tiles.block_m, bn, tiles.kv_groups,
+                                        (self.D + self.DV) / 256, self.target_workgroups, B * Hq)
         return -(-kv_tiles // per), per * bn
 
     def _kv_custom_scratch(self, tiles) -> int:

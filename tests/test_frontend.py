@@ -851,3 +851,20 @@ def test_gqa_plan():
         assert x & (x - 1) == 0
     op.grouped_merge, op.target_workgroups = True, 1
     assert op.plan_splits(2, 8, 2, 4096)[0] == op.N_WAVES
+
+
+def test_split_prefill_plan():
+    """Splits cover the cache with none empty and whole tiles, also where the count is chosen by cost; a count that gives
+    no CU two workgroups stays."""
+    op = AttentionEngine(_meta(1, 16, 16, 4, 512, 128, 128, torch.float16), CustomIO({}), C.make_scale_score_mod(0.1), None,
+                         C.OnlineSoftmax())._op
+    assert op.split_kv
+    for B, H in ((1, 8), (3, 16), (7, 16), (6, 32), (40, 32)):
+        for Sq in (1, 31, 64, 90, 230):
+            tiles = op.tiles_for(B, H, Sq, 4000)
+            for Skv in (1, 300, 522, 9161):
+                n_split, per = op.plan_splits(B, H, Sq, Skv, tiles)
+                assert per % tiles.block_n == 0 and n_split * per >= Skv > (n_split - 1) * per and n_split >= 1
+    tiles = op.tiles_for(7, 16, 31, 522)
+    assert op.plan_splits(7, 16, 31, 522, tiles)[0] == 1             # 112 workgroups, not 336 on 256 CUs
+    assert op.plan_splits(4, 8, 15, 9539, op.tiles_for(4, 8, 15, 9539))[0] == 8      # 256 workgroups
