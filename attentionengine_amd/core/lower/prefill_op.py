@@ -384,6 +384,42 @@ class PrefillOp:
                                         (self.D + self.DV) / 256, self.target_workgroups, B * Hq)
         return -(-kv_tiles // per), per * bn
 
+    MAX_TAIL_PARTS = 8        # kMaxParts of ae_prefill_pipe.hip
+
+    @classmethod
+    @functools.lru_cache(maxsize=1024)
+    def _tail_plan(cls, slots, kv_tiles, cus_per_xcd, width):
+        """(q tiles of an XCD, workgroups of each, kv tiles of a workgroup) that share their kv axes in an unmasked launch of the
+        pipelined kernel with ``slots`` q tiles an XCD (AE_TAIL of ae_prefill_pipe.hip), or None: what is left over when the
+        CUs have been filled as often as possible would take a round of its own.  A workgroup takes 7 us to start and end
+        and 2.0 us a kv tile (D128); shares are few (the last workgroup reads all of them, about 1.2 us each), and taken
+        where the call gains 6 % by this count - what it says is 3 % turned out between -7 and +2.  Measured: softmax B3 H8
+        S2944 D128 fp16 162 -> 117 us, bf16 174 -> 120, B1 H32 S2560 sigmoid bf16 155 -> 115 (40 tiles an XCD), B1 H40 S3584
+        (70) 301 -> 250, D64 B2 H16 S4200 231 -> 178, sigmoid fp16 B3 H16 S1325 83 -> 68; 56 of 64 tiles: 232 -> 230."""
+        rounds, rest = divmod(slots, cus_per_xcd)
+        if not rest:
+            return None
+        start, trip = 7.0, 2.0 * width
+        whole = start + trip * kv_tiles
+        best = None
+        for n in range(2, cls.MAX_TAIL_PARTS + 1):
+            per = -(-kv_tiles // n)
+            if -(-kv_tiles // per) != n:
+                continue
+            us = -(-rest * n // cus_per_xcd) * (start + trip * per) + 3.0 + 1.2 * n * width
+            if best is None or us < best[0]:
+                best = us, n, per
+        if best is None or (rounds * whole + best[0]) > 0.94 * (rounds + 1) * whole:
+            return None
+        return rest, best[1], best[2]
+
+    def _tail(self, B, H, Sq, Skv, tiles, mode, n_split):
+        if (tiles.template != "ae_prefill_pipe.hip" or mode != 0 or n_split > 1 or self.DV_launch != self.DV
+                or self._clock_stamps(tiles)):
+            return None
+        return self._tail_plan(-(-Sq // tiles.block_m) * -(-(B * H) // 8), -(-Skv // tiles.block_n),
+                               L._MI355X_CUS // 8, (self.D + self.DV) / 256)
+
     def _kv_custom_scratch(self, tiles) -> int:
         """LDS a launch needs beyond its K / V stages: the direct-to-LDS kernel redistributes the tiles of custom
         inputs with a kv dimension (fetched in a coalesced layout) through 2560 bytes per wave and 32-row block
@@ -410,13 +446,14 @@ class PrefillOp:
         """The mask's band (MaskPlan.band) where the kernel takes one instead of the tile table."""
         return plan.band if tiles.template == "ae_prefill.hip" else None
 
-    def _variant(self, tiles, mask_mode, Sq, Skv, n_split=1, table_rows=1, heavy_last=False, band=None):
+    def _variant(self, tiles, mask_mode, Sq, Skv, n_split=1, table_rows=1, heavy_last=False, band=None,
+                 tail=False):
         even_q, even_kv = Sq % tiles.block_m == 0, Skv % tiles.block_n == 0
         if mask_mode != 2 or band is not None:
             table_rows = 1
         if mask_mode != 2:
             heavy_last = False
-        key = (mask_mode, even_q, even_kv, n_split, table_rows, bool(heavy_last), band, astuple(tiles))
+        key = (mask_mode, even_q, even_kv, n_split, table_rows, bool(heavy_last), band, astuple(tiles), tail)
         v = self._variants.get(key)
         if v is None:
             has_mask_mod = self.elementwise_mask and mask_mode != 1
@@ -441,6 +478,8 @@ class PrefillOp:
                 cfg_src += f"#define AE_NSPLIT {n_split}\n#define AE_COMBINE_THREADS {self.COMBINE_THREADS}\n"
             if self._clock_stamps(tiles):
                 cfg_src += "#define AE_CLOCK_STAMPS 1\n"
+            if tail:
+                cfg_src += "#define AE_TAIL 1\n"
             module = rt.compile_module(tiles.template, {"ae_config.h": cfg_src,
                                                           "ae_functors.h": self.functor_src},
                                        allow_spills=self.allow_spills,
@@ -451,7 +490,8 @@ class PrefillOp:
                              lds_bytes=tiles.lds_bytes(self.D, self.DV_launch) + self._kv_custom_scratch(tiles), head_dim=self.D,
                              head_dim_v=self.DV_launch, elem_bytes=2, n_rowscales=self.n_rowscales,
                              mask_mode=mask_mode if band is None else 1,      # (a band is analytic: no table comes with the call)
-                             table_rows=table_rows if mask_mode == 2 and band is None else 0)
+                             table_rows=table_rows if mask_mode == 2 and band is None else 0,
+                             merge_in_wg=2 if tail else 0)
             v = self._variants[key] = (module, cfg, cfg_src)
         return v
 
@@ -538,8 +578,9 @@ class PrefillOp:
             plan = self._plan(B, Hq, Sq, Skv, dev, tiles)
             mode, table, mbm, mbn, band = plan.mode, plan.table, plan.block_m, plan.block_n, self._band(plan, tiles)
         n_split, kv_per_split = self.plan_splits(B, Hq, Sq, Skv, tiles)
+        tail = self._tail(B, Hq, Sq, Skv, tiles, mode, n_split)
         module, cfg, _ = self._variant(tiles, mode, Sq, Skv, n_split, self._table_rows(mbm, tiles) if mode == 2 else 1,
-                                       extern_mask is None and plan.heavy_last, band)
+                                       extern_mask is None and plan.heavy_last, band, tail is not None)
         kern = module.kernel("ae_prefill_kernel")
 
         out = torch.empty((B, Sq, Hq, self.DV), dtype=self.dtype, device=dev)
@@ -575,6 +616,15 @@ class PrefillOp:
                               n_rowscales=self.n_rowscales, mask_mode=0)
             rt.prefill_split_fwd(kern, module.kernel("ae_decode_combine_kernel"), p, cfg, ccfg, stream)
         else:
+            shared = {}
+            if tail is not None:
+                p.tail_slots, p.num_splits, p.kv_per_split = tail[0], tail[1], tail[2] * tiles.block_n
+                shared = {"n_split": tail[1], "kv_per_split": p.kv_per_split, "tail_slots": tail[0], "counters": 8 * tail[0],
+                          "o_rows": 8 * tail[0] * tail[1] * (tiles.block_m + 4 * tiles.threads // self.DV)}
+                partial_o = torch.empty((shared["o_rows"], self.DV), dtype=torch.float32, device=dev)
+                counters = self._host.work(1, 1, shared["counters"], dev.index, stream)[1]
+                p.partial_o, p.partial_rs = partial_o.data_ptr(), counters.data_ptr() + 4
+                keep += [partial_o, counters]
             if self._clock_stamps(tiles):
                 n_wg = -(-Sq // tiles.block_m) * (-(-(B * Hq) // 8) * 8)
                 self.clock_stamps = torch.zeros((n_wg, 2), dtype=torch.int64, device=dev)
@@ -588,9 +638,11 @@ class PrefillOp:
         self.final_rowscales = dict(zip(self.functors.final_rowscale_names, rowscales))
         self._keepalive = keep
         if extern_mask is None and self.DV_launch == self.DV and not self._clock_stamps(tiles):
+            if n_split > 1:
+                shared = {"n_split": n_split, "kv_per_split": kv_per_split}
             host.add_forward(self._host, host.PREFILL_SPLIT if n_split > 1 else host.PREFILL, B, Sq, Hq, Hkv, Skv, dev, module,
                              kern, cfg, combine=module.kernel("ae_decode_combine_kernel") if n_split > 1 else None,
-                             ccfg=ccfg if n_split > 1 else None, n_split=n_split, kv_per_split=kv_per_split,
+                             ccfg=ccfg if n_split > 1 else None, **shared,
                              table=table if mode == 2 and band is None else None, mask_block=(mbm, mbn), env=("AE_CLOCK_STAMPS",))
         return out
 

@@ -389,7 +389,24 @@ int ae_prefill_fwd(ae_kernel* k, const ae_attn_params* p, const ae_tile_cfg* cfg
   // ids are 8*slot + xcd with slot = (batch*head / 8)*q_tiles + q_tile, see ae_prefill.hip
   uint64_t q_tiles = ((uint64_t)p->seqlen_q + cfg->block_m - 1) / cfg->block_m;
   uint64_t bh = (uint64_t)p->heads_q * (uint64_t)p->batch;
-  uint64_t total = q_tiles * ((bh + 7) / 8) * 8;
+  uint64_t slots = q_tiles * ((bh + 7) / 8);
+  // cfg->merge_in_wg = 2: the last tail_slots slots are num_splits workgroups each (AE_TAIL of ae_prefill_pipe.hip)
+  if (cfg->merge_in_wg != 0 && cfg->merge_in_wg != 2)
+    return fail(AE_ERR_INVALID_ARG, "ae_prefill_fwd: merge_in_wg=%d", cfg->merge_in_wg);
+  if (cfg->merge_in_wg == 2) {
+    if (cfg->mask_mode != 0 || !p->partial_o || !p->partial_rs)
+      return fail(AE_ERR_INVALID_ARG, "ae_prefill_fwd: shared q tiles need work buffers and no mask");
+    if (p->tail_slots <= 0 || (uint64_t)p->tail_slots > slots || p->num_splits < 2 || p->num_splits > 8)
+      return fail(AE_ERR_INVALID_ARG, "ae_prefill_fwd: %d of %llu slots shared by %d workgroups", p->tail_slots,
+                  (unsigned long long)slots, p->num_splits);
+    if (p->kv_per_split <= 0 || p->kv_per_split % cfg->block_n != 0 ||
+        (int64_t)p->num_splits * p->kv_per_split < p->seqlen_kv ||
+        (int64_t)(p->num_splits - 1) * p->kv_per_split >= p->seqlen_kv)
+      return fail(AE_ERR_INVALID_ARG, "ae_prefill_fwd: %d shares of %d positions for Skv=%d", p->num_splits, p->kv_per_split,
+                  p->seqlen_kv);
+    slots += (uint64_t)p->tail_slots * (uint64_t)(p->num_splits - 1);
+  }
+  uint64_t total = slots * 8;
   if (total == 0 || total > 0x7fffffffull)
     return fail(AE_ERR_INVALID_ARG, "ae_prefill_fwd: grid of %llu workgroups",
                 (unsigned long long)total);

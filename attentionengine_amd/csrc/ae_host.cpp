@@ -88,6 +88,7 @@ struct Plan {
   std::shared_ptr<Keep> keep;
   std::shared_ptr<BwdPlan> bwd;
   int64_t o_rows = 0, counters = 0;   // partial results a split launch writes; arrival counters behind the row scales
+  int tail_slots = 0;                 // prefill: q-tile slots of an XCD that several workgroups share
 };
 
 // Work buffers of launches whose last workgroup merges: the arrival counters behind the row scales are zero when a
@@ -399,8 +400,12 @@ PyObject* run(Host* h, PyObject* const* args, Py_ssize_t nargs, bool mla) {
   }
   const int64_t rs_floats = (h->n_rs > 0 ? h->n_rs : 1) * B * Sq * Hq * pl.n_split;
   at::Tensor po, prs;
-  if (pl.kind != kPrefill) p.num_splits = pl.n_split, p.kv_per_split = pl.kv_per_split;
-  if (pl.cfg.merge_in_wg == 2) {
+  if (pl.kind != kPrefill || pl.tail_slots) p.num_splits = pl.n_split, p.kv_per_split = pl.kv_per_split;
+  if (pl.tail_slots) {      // (only the counters are kept: the partial results are the size of a few thousand rows)
+    p.tail_slots = pl.tail_slots;
+    po = empty({pl.o_rows, h->DV}, at::kFloat, dev);
+    prs = get_work(h, 1, 1, pl.counters, dev, stream).second.narrow(0, 1, pl.counters);
+  } else if (pl.cfg.merge_in_wg == 2) {
     std::tie(po, prs) = get_work(h, pl.o_rows, rs_floats, pl.counters, dev, stream);
   } else if (pl.n_split > 1 && pl.cfg.merge_in_wg == 0) {
     po = empty({pl.o_rows, h->DV}, at::kFloat, dev);
@@ -485,6 +490,7 @@ PyObject* host_add(PyObject* self, PyObject* d) {
   pl->has_ccfg = get_cfg(d, "ccfg", pl->ccfg);
   pl->n_split = (int)get_int(d, "n_split", 1), pl->kv_per_split = (int)get_int(d, "kv_per_split");
   pl->o_rows = get_int(d, "o_rows", pl->B * pl->Sq * pl->Hq * pl->n_split), pl->counters = get_int(d, "counters");
+  pl->tail_slots = (int)get_int(d, "tail_slots");
   TORCH_CHECK(pl->cfg.merge_in_wg != 2 || pl->counters > 0, "a launch whose last workgroup merges needs arrival counters");
   pl->table = get_tensor(d, "table");
   pl->mask_bm = (int)get_int(d, "mask_bm"), pl->mask_bn = (int)get_int(d, "mask_bn");

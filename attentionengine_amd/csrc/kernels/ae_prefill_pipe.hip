@@ -123,10 +123,19 @@ static_assert(AE_KV_STAGES == 2 || AE_KV_STAGES == 3, "two or three K / V stages
 #ifndef AE_CLOCK_STAMPS
 #define AE_CLOCK_STAMPS 0
 #endif
+// 1: the last p.tail_slots q tiles of every XCD are shared by p.num_splits workgroups each, which take a share of the kv
+// axis and leave O and the row state in memory; the one that finishes last adds them up and goes on to the epilogue.  A
+// launch takes as many rounds as an XCD has q tiles for its 32 CUs: 36 tiles used to take two, the second with 28 idle CUs
+// (softmax B3 H8 S2944 D128 fp16: 162 us; the four shared by eight workgroups each, 117).
+#ifndef AE_TAIL
+#define AE_TAIL 0
+#endif
 // 1: Q carries c*log2e and the reference is the C operand of the first k-step (see above)
 #ifndef AE_PRESCALE
 #define AE_PRESCALE (!AE_DTYPE_BF16 && AE_PIPE_KIND == 0)
 #endif
+
+static_assert(!AE_TAIL || (AE_MASK_MODE == 0 && !AE_CLOCK_STAMPS), "shared q tiles: every tile of the kv axis is visited");
 
 typedef __attribute__((address_space(3))) unsigned char ae_lds_byte;
 #define AE_SB() __builtin_amdgcn_sched_barrier(0)
@@ -161,7 +170,14 @@ void ae_prefill_kernel(const ae_attn_params p) {
   const int n_bh = p.batch * p.heads_q;
   const int wg = blockIdx.x;
   const int xcd = wg & 7;
+#if AE_TAIL
+  int slot = wg >> 3, part = 0;
+  const int tail0 = n_qt * ((n_bh + 7) >> 3) - p.tail_slots;      // first shared tile of the XCD
+  const bool shared = slot >= tail0;
+  if (shared) slot = tail0 + ae_divide(slot - tail0, p.num_splits, part);
+#else
   const int slot = wg >> 3;
+#endif
 #if AE_MASK_MODE == 1 || (AE_MASK_MODE == 2 && AE_HEAVY_LAST)
   // causal: q tiles differ in work by up to n_qt : 1, so ids go heaviest tile first across ALL heads
   // (longest-job-first keeps the tail short); the heads of one XCD still meet in its L2.  A tile table whose
@@ -230,6 +246,14 @@ void ae_prefill_kernel(const ae_attn_params p) {
   // ---- KV tile range and tile classes --------------------------------------------------------
   const int n_kvt = (p.seqlen_kv + AE_BN - 1) / AE_BN;
   int j_end = n_kvt;
+  int j_first = 0;
+#if AE_TAIL
+  if (shared) {
+    j_first = part * (p.kv_per_split / AE_BN);
+    const int lim = j_first + p.kv_per_split / AE_BN;
+    j_end = lim < n_kvt ? lim : n_kvt;
+  }
+#endif
 #if AE_MASK_MODE == 1
   {
     int lim = (q0 + AE_BM + AE_BN - 1) / AE_BN;   // attn_tl.py:113-115
@@ -345,7 +369,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
   // ---- the first tiles are requested before anything else is set up: the zeroing of the accumulators, the
   // constants and the address arithmetic below (about a thousand instructions of one wave per SIMD) then run
   // while they and the Q rows travel ----
-  int j0 = next_tile(0);                  // tile whose scores are in sv (exp + PV next)
+  int j0 = next_tile(j_first);            // tile whose scores are in sv (exp + PV next)
   int tc0[2], tc1[2], tc2[2], tcn[2];     // ... and what tiles j0, j1, j2, jn mean to this wave (tile_info)
   bool tnm0, tnm1, tnm2 = false, tnmn = false;
   tile_info(j0, tc0, tnm0);
@@ -865,6 +889,125 @@ void ae_prefill_kernel(const ae_attn_params p) {
       break;
     }
     iteration(ae_tag_false{}, ae_tag_false{});
+  }
+#endif
+
+#if AE_TAIL
+  // ---- a shared q tile: O and the row state of this share -> memory; the last of the tile's workgroups adds them up -----
+  // The partial results travel as in the dk/dv launch of ae_prefill_bwd.hip: stores that are written through this XCD's L2
+  // and acknowledged before the counter moves, loads that take no line the L2 may still hold.  The own share comes back
+  // from memory as well: the order of the sums does not depend on who was last.  A share costs the last workgroup
+  // about a trip to memory (128 KiB a workgroup), so they are few: eight at most.
+  if (shared) {
+    constexpr int kDeviceScope = 16;     // the sc1 bit of a buffer instruction's cache policy
+    constexpr int kPartBytes = AE_BM * AE_DV * 4 + AE_NT * 16, kMaxParts = 8;
+    const int n_parts = p.num_splits;
+    const int tile_id = (blockIdx.x & 7) * p.tail_slots + ((int)(blockIdx.x >> 3) - tail0) / n_parts;
+    __amdgpu_buffer_rsrc_t part_buf = __builtin_amdgcn_make_buffer_rsrc(
+        p.partial_o + (int64_t)tile_id * n_parts * (kPartBytes / 4), 0, n_parts * kPartBytes, 0x00020000);
+    int part_at = lane;
+    asm volatile("" : "+v"(part_at));
+    const int state_at = AE_BM * AE_DV * 4 + (wave * 64 + part_at) * 16;
+    part_at = wave * (2 * AE_NDB * 4096) + part_at * 16;
+    auto load_part = [&](int at, int k) AE_LAMBDA -> ae_f32x4 {
+      return __builtin_bit_cast(ae_f32x4, __builtin_amdgcn_raw_buffer_load_b128(part_buf, at, k * kPartBytes, kDeviceScope));
+    };
+#pragma unroll
+    for (int qb = 0; qb < 2; qb++)
+#pragma unroll
+      for (int db = 0; db < AE_NDB; db++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          const ae_f32x16& a = oacc[qb][db];
+          const ae_f32x4 w = {a[g * 4], a[g * 4 + 1], a[g * 4 + 2], a[g * 4 + 3]};
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(ae_u32x4, w), part_buf,
+                                                 part_at + ((qb * AE_NDB + db) * 4 + g) * 1024, part * kPartBytes, kDeviceScope);
+        }
+#if AE_PIPE_KIND == 0
+    {
+      // (a row whose scores are all -inf has no reference yet: it says so, and weighs nothing)
+      const ae_f32x4 w = {ae_group_sum(r_run[0]) == 0.f ? AE_NEG_INF : m2[0], ae_group_sum(r_run[1]) == 0.f ? AE_NEG_INF : m2[1],
+                          r_run[0], r_run[1]};
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(ae_u32x4, w), part_buf, state_at, part * kPartBytes, kDeviceScope);
+    }
+#endif
+    __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
+    __syncthreads();                     // (and every wave is past its last tile: the stages are free)
+    __attribute__((address_space(3))) int* flag = (__attribute__((address_space(3))) int*)lds;
+    if (wave == 0 && lane == 0) {
+      int* counter = (int*)p.partial_rs + tile_id;
+      const int seen = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (seen == n_parts - 1) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *flag = seen == n_parts - 1;
+    }
+    __syncthreads();
+    if (*flag == 0) return;
+    float weight[kMaxParts][2];
+#if AE_PIPE_KIND == 0
+    {
+      ae_f32x4 state[kMaxParts];
+#pragma unroll
+      for (int k = 0; k < kMaxParts; k++) state[k] = load_part(state_at, k < n_parts ? k : n_parts - 1);
+#pragma unroll
+      for (int qb = 0; qb < 2; qb++) {
+        float top = AE_NEG_INF, sum = 0.f;
+#pragma unroll
+        for (int k = 0; k < kMaxParts; k++) top = __builtin_fmaxf(top, state[k][qb]);
+#pragma unroll
+        for (int k = 0; k < kMaxParts; k++) {
+          weight[k][qb] = state[k][qb] == AE_NEG_INF ? 0.f : ae_exp2(state[k][qb] - top);
+          if (k < n_parts) sum += state[k][2 + qb] * weight[k][qb];
+        }
+        m2[qb] = top == AE_NEG_INF ? 0.f : top;
+        r_run[qb] = sum;
+      }
+    }
+#else
+#pragma unroll
+    for (int k = 0; k < kMaxParts; k++) weight[k][0] = weight[k][1] = 1.f;
+#endif
+#pragma unroll
+    for (int qb = 0; qb < 2; qb++) {
+      ae_f32x16 acc[AE_NDB];
+#pragma unroll
+      for (int db = 0; db < AE_NDB; db++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[db][r] = 0.f;
+#pragma unroll
+      for (int k0 = 0; k0 < kMaxParts; k0 += 2) {         // two shares on the way at a time
+        if (k0 >= n_parts) break;
+        const bool two = k0 + 1 < n_parts;
+        ae_f32x4 w0[AE_NDB * 4], w1[AE_NDB * 4];
+#pragma unroll
+        for (int j = 0; j < AE_NDB * 4; j++) w0[j] = load_part(part_at + (qb * AE_NDB * 4 + j) * 1024, k0);
+        if (two) {
+#pragma unroll
+          for (int j = 0; j < AE_NDB * 4; j++) w1[j] = load_part(part_at + (qb * AE_NDB * 4 + j) * 1024, k0 + 1);
+        }
+#pragma unroll
+        for (int j = 0; j < AE_NDB * 4; j++)
+#pragma unroll
+          for (int t = 0; t < 4; t++) acc[j / 4][j % 4 * 4 + t] += w0[j][t] * weight[k0][qb];
+        if (two) {
+#pragma unroll
+          for (int j = 0; j < AE_NDB * 4; j++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) acc[j / 4][j % 4 * 4 + t] += w1[j][t] * weight[k0 + 1][qb];
+        }
+      }
+#pragma unroll
+      for (int db = 0; db < AE_NDB; db++) oacc[qb][db] = acc[db];
+    }
+  }
+  {
+    // (the rows once more, from a copy of the lane id: one register less across the loop, which has none to spare)
+    int le = lane;
+    asm volatile("" : "+v"(le));
+#pragma unroll
+    for (int qb = 0; qb < 2; qb++) {
+      qrow[qb] = q0w + qb * 32 + (le & 31);
+      q_ok[qb] = AE_EVEN_Q || qrow[qb] < p.seqlen_q;
+    }
   }
 #endif
 

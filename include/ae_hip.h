@@ -100,7 +100,12 @@ typedef struct ae_attn_params {
   int32_t mask_block_m, mask_block_n;        /* rows/cols one block-mask entry covers     */
   int32_t num_splits;                        /* decode: KV splits per (batch, q-head)     */
   int32_t kv_per_split;                      /* decode: KV positions per split            */
-  int32_t reserved[3];
+  /* prefill kernels compiled with AE_TAIL 1 (announced by cfg->merge_in_wg = 2): of the q-tile slots of every XCD (see
+   * ae_prefill_fwd) the last tail_slots are shared by num_splits workgroups each, kv_per_split positions a workgroup;
+   * the one that finishes last merges.  partial_o: 8 * tail_slots * num_splits * (block_m * DV + 4 * threads) floats;
+   * partial_rs: 8 * tail_slots int32 arrival counters, zero when the launch starts and when it ends.  Else 0. */
+  int32_t tail_slots;
+  int32_t reserved[2];
   /* MLA decode on a paged cache (kernels whose ae_tile_cfg.paged is 1; NULL / 0 otherwise): the cache is
    * [num_pages, page_block_size, Hkv, D] (k_stride_b = elements between pages, k_stride_s between the
    * rows of a page), token t of batch entry b is row t % page_block_size of page

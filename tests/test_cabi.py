@@ -303,6 +303,33 @@ def test_block_table_geometry_is_checked_before_any_launch():
         assert rc == 1 and "table_rows=-1" in msg, msg
 
 
+def test_shared_q_tiles_are_checked_before_any_launch():
+    """merge_in_wg = 2: shares of a kv axis must cover it with none empty, two to eight of them, of q tiles that exist,
+    with work buffers and without a mask."""
+    lib = rt.lib()
+    fake = ctypes.c_void_p(8)
+    buf = ctypes.create_string_buffer(64)
+    addr = ctypes.addressof(buf)
+
+    def refused(cfg_kw=None, **kw):
+        p = rt.AttnParams()
+        p.q = p.k = p.v = p.out = p.partial_o = p.partial_rs = addr
+        p.batch, p.heads_q, p.heads_kv, p.seqlen_q, p.seqlen_kv = 1, 8, 8, 1000, 1000
+        p.tail_slots, p.num_splits, p.kv_per_split = 3, 2, 512
+        for k, v in kw.items():
+            setattr(p, k, v)
+        c = rt.TileCfg(block_m=256, block_n=64, threads=256, lds_bytes=1024, head_dim=64, head_dim_v=64, elem_bytes=2,
+                       merge_in_wg=2, **(cfg_kw or {}))
+        assert lib.ae_prefill_fwd(fake, ctypes.byref(p), ctypes.byref(c), None) == 1
+        return lib.ae_last_error().decode()
+    assert "work buffers" in refused(partial_o=None) and "work buffers" in refused(partial_rs=None)
+    assert "0 of 4 slots" in refused(tail_slots=0) and "5 of 4 slots" in refused(tail_slots=5)
+    assert "by 1 workgroups" in refused(num_splits=1) and "by 9 workgroups" in refused(num_splits=9, kv_per_split=128)
+    assert "2 shares of 448" in refused(kv_per_split=448) and "2 shares of 1024" in refused(kv_per_split=1024)
+    assert "2 shares of 500" in refused(kv_per_split=500) and "2 shares of 0" in refused(kv_per_split=0)
+    assert "no mask" in refused({"mask_mode": 1})
+
+
 def test_misaligned_tensors_are_refused_before_any_launch():
     """The kernels move rows 16 bytes at a time: a tensor that does not start on a 16-byte boundary, or whose
     strides are not multiples of 8 elements, is refused by the argument checks (the Python operators copy such

@@ -868,3 +868,16 @@ def test_split_prefill_plan():
     tiles = op.tiles_for(7, 16, 31, 522)
     assert op.plan_splits(7, 16, 31, 522, tiles)[0] == 1             # 112 workgroups, not 336 on 256 CUs
     assert op.plan_splits(4, 8, 15, 9539, op.tiles_for(4, 8, 15, 9539))[0] == 8      # 256 workgroups
+
+
+def test_tail_plan():
+    """Shares of what is left over after whole rounds: only where they save time, at least two and at most eight, none empty."""
+    from core.lower.prefill_op import PrefillOp
+    for slots in range(1, 200):
+        for tiles in (16, 46, 110):
+            plan = PrefillOp._tail_plan(slots, tiles, 32, 1.0)
+            if plan is not None:
+                rest, n, per = plan
+                assert rest == slots % 32 and 2 <= n <= PrefillOp.MAX_TAIL_PARTS and (n - 1) * per < tiles <= n * per
+    assert PrefillOp._tail_plan(64, 46, 32, 1.0) is None and PrefillOp._tail_plan(56, 56, 32, 1.0) is None
+    assert PrefillOp._tail_plan(36, 46, 32, 1.0)[0] == 4

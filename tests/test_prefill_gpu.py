@@ -1086,3 +1086,81 @@ def test_very_long_sequences(cuda_device, H, Hkv, S, D, dtype, causal):
         ref = torch.einsum("hqk,khd->qhd", torch.softmax(s, -1), vv)
         assert (out[0, rows].float().cpu() - ref).abs().max().item() <= 2e-2, r0
         assert (lse[0, :, rows].cpu() - torch.logsumexp(s, -1)).abs().max().item() <= 1e-3, r0
+
+
+@pytest.mark.parametrize("kind,B,H,S,D,tail,dtype", [
+    ("softmax", 1, 3, 700, 128, (3, 2, 6), torch.float16),      # every q tile shared; five surplus heads; ragged rows and keys
+    ("softmax", 3, 4, 512, 128, (1, 8, 1), torch.bfloat16),     # one of four tiles an XCD, a kv tile a workgroup
+    ("softmax", 1, 16, 520, 64, (4, 3, 3), torch.float16),      # the last share: three tiles, the third of eight keys
+    ("softmax", 1, 9, 577, 128, (1, 5, 2), torch.bfloat16),     # an odd number of shares; one key in the last tile
+    ("sigmoid", 2, 5, 640, 128, (5, 5, 2), torch.float16),      # no row state
+    ("sigmoid", 1, 8, 333, 64, (2, 6, 1), torch.bfloat16),
+])
+def test_q_tiles_shared_by_several_workgroups(cuda_device, monkeypatch, kind, B, H, S, D, tail, dtype):
+    """The pipelined kernel with some q tiles' kv axes shared out (AE_TAIL): the oracle's result, the same bits on every
+    call, through Python, through the native host path and as replays of a graph.  Keys of the second share score far
+    above the others, so the shares' references differ."""
+    print(f"case shared q tiles {kind} B{B} H{H} S{S} D{D} {tail} {dtype}", flush=True)
+    monkeypatch.setenv("AE_PREFILL_KERNEL", "pipelined")
+    q, k, v = C.make_inputs(B, S, S, H, H, D, D, dtype, seed=S)
+    if kind == "softmax":
+        # (fp16 folds the score scale into Q: a score is off by up to 2^-11 of the products it sums, 4 x the keys would
+        # move an lse of 14 by 0.003; the bound of LSE_TOL is for scores of the size that unit inputs have)
+        k[:, tail[2] * 64:2 * tail[2] * 64] *= 4 if dtype == torch.bfloat16 else 1.5
+        mod = _engine(B, H, S, D, D, dtype, C.make_scale_score_mod(1 / math.sqrt(D)), None, C.OnlineSoftmax())
+        ref, rlse = R.softmax_attention(q, k, v, causal=False)
+        more = ()
+    else:
+        bias = torch.tensor([-math.log(S)])
+        mod = _engine(B, H, S, D, D, dtype, C.make_sigmoid_score_mod(1 / math.sqrt(D)), None, C.OnlineIdentity(),
+                      customs=CustomIO({"softmax_bias": (1,)}))
+        ref = R.sigmoid_attention(q, k, v, bias=bias.item(), causal=False)
+        more = (bias.cuda(),)
+    op = mod.attention
+    assert op.tiles.template == "ae_prefill_pipe.hip"
+    assert -(-S // 64) <= tail[1] * tail[2] and (tail[1] - 1) * tail[2] < -(-S // 64)
+    op._tail_plan = lambda *a: tail
+    args = tuple(t.cuda() for t in (q, k, v)) + more
+    got = []
+    for _ in range(3):
+        out = mod(*args)
+        got.append([out.clone()] + [r.clone() for r in mod.final_rowscales.values()])
+    assert (got[0][0].float().cpu() - ref).abs().max().item() <= OUT_TOL
+    if kind == "softmax":
+        assert (got[0][1].cpu() - rlse).abs().max().item() <= LSE_TOL
+    assert all(torch.equal(a, b) for g in got[1:] for a, b in zip(got[0], g))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = mod(*args)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, got[0][0])
+        mod(*args)
+        torch.cuda.synchronize()
+
+
+def test_a_share_without_visible_keys_weighs_nothing(cuda_device, monkeypatch):
+    """A share whose scores are all -inf has no reference and adds nothing, also where the others' references are far
+    below zero."""
+    monkeypatch.setenv("AE_PREFILL_KERNEL", "pipelined")
+    B, H, S, D, dtype = 1, 2, 384, 128, torch.bfloat16
+    q, k, v = C.make_inputs(B, S, S, H, H, D, D, dtype, seed=1)
+    q = q.abs() + 0.125
+    k = -(k.abs() + 4)                          # every score about -50
+    k[:, 128:256] = float("-inf")
+    mod = _engine(B, H, S, D, D, dtype, C.make_scale_score_mod(1 / math.sqrt(D)), None, C.OnlineSoftmax())
+    op = mod.attention
+    outs = {}
+    for tail in (None, (2, 3, 2)):
+        op._tail_plan = lambda *a: tail
+        op._host.clear()
+        outs[tail] = mod(q.cuda(), k.cuda(), v.cuda()).float().cpu(), mod.final_rowscales["lse"].cpu()
+    seen = torch.cat((torch.arange(128), torch.arange(256, 384)))
+    ref, rlse = R.softmax_attention(q, k[:, seen], v[:, seen], causal=False)
+    for out, lse in outs.values():
+        assert (out - ref).abs().max().item() <= OUT_TOL
+        assert ((lse - rlse).abs() <= LSE_TOL + 2e-6 * rlse.abs()).all()
