@@ -9,6 +9,7 @@ host needs at launch time.
 """
 from __future__ import annotations
 
+import functools
 import math
 import os
 from dataclasses import dataclass, field
@@ -710,6 +711,33 @@ def choose_prefill_tiles(d: int, dv: int, seqlen_q: int = 0, softmax=None, batch
     if t.v_pad == 0:
         t.v_pad = 256
     return t
+
+
+# Causal softmax, head dim 128, microseconds: (call, workgroup's start and end, trip of a workgroup that has to finish,
+# trip where the CUs' sum counts, exponent of the norm that joins the two) of the pipelined kernel's 256-row tiles and the
+# generic one's 128-row tiles, by whether the type is bf16
+_CAUSAL_COST = {False: ((3.2, 7.6, 1.61, 1.83, 12.0), (0.8, 3.3, 1.28, 1.03, 4.6)),
+                True: ((3.2, 8.6, 1.70, 1.87, 12.0), (0.0, 3.9, 1.26, 0.965, 4.9))}
+
+
+@functools.lru_cache(maxsize=1024)
+def pipelined_pays(bf16: bool, batch_heads: int, seqlen: int) -> bool:
+    """Whether a causal softmax over equal lengths (head dim 128) takes less time in the pipelined kernel than in the generic
+    one.  Under the mask the q tiles differ in work, and a launch takes as long as its longest tile or as its share of all
+    tiles and their starts, whichever is more: 256-row tiles are longer, fewer and waste more rows at the end of a ragged
+    sequence, but multiply faster.  Fitted to both kernels' times of 170 shapes (22 to 400 of the larger tiles an XCD, 1024 to
+    12000 positions; windows of 60 ms, since the first 20 favour the generic one), where the choice (a tie
+    goes to the pipelined kernel) is 0.3 % slower than the better one on average; the lengths of choose_prefill_tiles alone: 7 %.  Pipelined -> generic where it now goes there,
+    us: fp16 B3 H32 S1400 76 -> 64, B1 H32 S2009 56 -> 49, bf16 B4 H16 S2680 146 -> 127, B2 H32 S2867 166 -> 149; the other
+    way it is 270 against 290 for fp16 B2 H32 S4096 and 257 against 280 for bf16 B1 H16 S8192."""
+    heads, kv_tiles = -(-batch_heads // 8), -(-seqlen // 64)
+    us = []
+    for rows, (call, start, longest, shared, p) in zip((256, 128), _CAUSAL_COST[bf16]):
+        n = -(-seqlen // rows)
+        trips = (rows // 64) * n * (n + 1) // 2                    # of a head: q tile i sees (i + 1) * rows / 64 kv tiles
+        trips -= (rows // 64) * n - kv_tiles                        # (the last one no more than there are)
+        us.append(call + ((longest * kv_tiles) ** p + (heads * (shared * trips + start * n) / (_MI355X_CUS // 8)) ** p) ** (1 / p))
+    return us[0] < 1.03 * us[1]
 
 
 def kv_group_tiles(d: int, dv: int, batch_heads: int, seqlen_q: int, seqlen_kv: int, banded: bool):

@@ -110,6 +110,7 @@ class PrefillOp:
         if groups is not None:
             self.tiles = groups
         self._call_tiles = {}      # (B, H, Sq, Skv) other than the declared ones -> tiles_for()
+        self._causal_generic = {}  # (B, H, Sq, Skv) -> _causal_choice() takes the generic kernel
         # tune=True (attn_tl.py:465-521 of the reference): the tile configuration comes from the record of
         # this problem in tune_file, or is measured at the first call and recorded there.  Launches whose
         # tiles are bound to something else (split-KV, an external block mask) keep the fixed choice.
@@ -194,6 +195,7 @@ class PrefillOp:
             self.tiles = L.PrefillTiles()
         self._base = self._table_tiles = L.PrefillTiles()
         self._call_tiles.clear()
+        self._causal_generic.clear()
         self._variants.clear()
         self._plans.clear()
         self._host.clear()
@@ -258,12 +260,28 @@ class PrefillOp:
         """The tile configuration of a call with these extents."""
         key = (B, H, Sq, Skv)
         if key == self._declared or (self.tiles.kv_groups == 1 and self.tiles is not self._groups):
-            return self.tiles
+            return self._causal_choice(key, self.tiles)
         tiles = self._call_tiles.get(key)
         if tiles is None:
             tiles = self._call_tiles[key] = self._kv_group_choice(
                 *key, lambda found: self._plan(*key, device=None, tiles=found)) or self._base
-        return tiles
+        return self._causal_choice(key, tiles)
+
+    def _causal_choice(self, key, tiles):
+        """``tiles``, or the generic kernel's where they are the pipelined kernel's by this operator's own choice, would be at
+        these extents too, and a causal call is faster in the generic one (lower.pipelined_pays)."""
+        B, H, Sq, Skv = key
+        if (tiles.template != "ae_prefill_pipe.hip" or self.mask_mod is None or self._pipe_softmax is None or Sq != Skv or not Sq
+                or (self.D, self.DV) != (128, 128) or self._tiles_given or self._tune_file or self.extern_block_mask):
+            return tiles
+        generic = self._causal_generic.get(key)
+        if generic is None:
+            bf16 = self.dtype == torch.bfloat16
+            generic = self._causal_generic[key] = (
+                os.environ.get("AE_PREFILL_KERNEL", "") != "pipelined" and not L.pipelined_pays(bf16, B * H, Sq)
+                and L.choose_prefill_tiles(self.D, self.DV, Sq, self._pipe_softmax, B * H, seqlen_kv=Skv, bf16=bf16) == tiles
+                and self._plan(*key, device=None, tiles=tiles).mode == 1)
+        return L.PrefillTiles() if generic else tiles
 
     # ---- tuning ------------------------------------------------------------------------
     def _tune_candidates(self):

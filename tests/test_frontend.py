@@ -881,3 +881,26 @@ def test_tail_plan():
                 assert rest == slots % 32 and 2 <= n <= PrefillOp.MAX_TAIL_PARTS and (n - 1) * per < tiles <= n * per
     assert PrefillOp._tail_plan(64, 46, 32, 1.0) is None and PrefillOp._tail_plan(56, 56, 32, 1.0) is None
     assert PrefillOp._tail_plan(36, 46, 32, 1.0)[0] == 4
+
+
+def test_causal_prefill_takes_the_faster_kernel(monkeypatch):
+    """Causal softmax at head dim 128: the pipelined kernel where its 256-row tiles balance, the generic one elsewhere;
+    the caller's tiles, other masks and the environment's choice stay; short calls of a large engine keep its kernel."""
+    from core.lower import lower as L
+    from core.lower.prefill_op import PrefillOp
+    monkeypatch.delenv("AE_PREFILL_KERNEL", raising=False)
+    sm, f16 = C.make_scale_score_mod(0.1), torch.float16
+
+    def template(S, mask=C.causal_mask, H=32, B=1, **kw):
+        op = PrefillOp(_meta(B, H, H, S, S, 128, 128, f16), CustomIO({}), sm, mask, C.OnlineSoftmax(), "-inf", **kw)
+        return op, op.tiles_for(B, H, S, S).template
+    op, chosen = template(2009)
+    assert chosen == "ae_prefill.hip" and op.tiles.template == "ae_prefill_pipe.hip"
+    assert op.tiles_for(2, 32, 4096, 4096).template == "ae_prefill_pipe.hip"
+    assert op.tiles_for(1, 32, 100, 100) == op.tiles and op.tiles_for(1, 32, 2009, 4096) == op.tiles
+    assert template(4096, B=2)[1] == "ae_prefill_pipe.hip"
+    assert template(2009, mask=None)[1] == "ae_prefill_pipe.hip"
+    assert template(2009, tiles=L.pipelined_tiles(128, 128))[1] == "ae_prefill_pipe.hip"
+    assert not L.pipelined_pays(True, 64, 2867) and L.pipelined_pays(True, 16, 8192) and L.pipelined_pays(False, 16, 9131)
+    monkeypatch.setenv("AE_PREFILL_KERNEL", "pipelined")
+    assert template(2009)[1] == "ae_prefill_pipe.hip"
