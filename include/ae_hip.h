@@ -141,7 +141,9 @@ typedef struct ae_tile_cfg {
                           workgroup per (batch, kv head, head tile) merges its waves' partial results and
                           writes out itself: no combine kernel, no work buffers); 2 when it was compiled with
                           AE_MERGE_LAST 1 (the workgroup that finishes last merges: no combine kernel, work
-                          buffers with arrival counters, see ae_decode_fwd); else 0                        */
+                          buffers with arrival counters, see ae_decode_fwd); else 0.  Prefill: 2 for kernels
+                          compiled with AE_TAIL 1 (ae_attn_params.tail_slots), backward: 2 for AE_BWD_SPLIT 1
+                          (ae_attn_bwd_params.dkv_parts); else 0                                            */
   int32_t table_rows;  /* mask_mode 2: block-mask rows one q tile may span, the AE_TT_ROWS the kernel was
                           compiled with (1, 2, 4 or 8); 0 stands for the kernels' default of 8.
                           ae_prefill_bwd: 16 when the dk/dv kernel was compiled with AE_BWD_PAIRS 1 (its
