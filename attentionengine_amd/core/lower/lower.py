@@ -750,6 +750,8 @@ def kv_group_tiles(d: int, dv: int, batch_heads: int, seqlen_q: int, seqlen_kv: 
     D64 H32 S333 10.7 -> 7.3; but B4 H32 S333 17.4 -> 20 with any of them."""
     def wgs(rows):
         return batch_heads * -(-seqlen_q // rows)
+    if (d, dv) == (192, 128):
+        return _wide_key_group_tiles(wgs, batch_heads, seqlen_kv)
     slots = _MI355X_CUS if max(d, dv) > 64 else 2 * _MI355X_CUS
     if wgs(32) <= slots:
         return PrefillTiles(n_waves=1, kv_groups=4, block_n=32)
@@ -758,6 +760,22 @@ def kv_group_tiles(d: int, dv: int, batch_heads: int, seqlen_q: int, seqlen_kv: 
     if banded and seqlen_kv >= 512 and max(d, dv) > 64 and wgs(64) <= 2 * slots:
         return PrefillTiles(n_waves=2, kv_groups=2, block_n=32)
     if seqlen_kv >= 512 and wgs(128) <= (_MI355X_CUS * 3 // 2 if banded else _MI355X_CUS):
+        return PrefillTiles(kv_groups=2)
+    return None
+
+
+def _wide_key_group_tiles(wgs, batch_heads: int, seqlen_kv: int):
+    """The same for causal launches at head dims 192 / 128, whose tiles hold 160, 80 (two workgroups a CU) and 160 KiB of LDS.
+    Four groups where all 64-row tiles are resident at once, or few heads make them long; two groups while two a CU
+    hold them; two groups of 128 rows while few heads leave the longest tile behind its CU's share of all.  Measured
+    (us, default tiles -> these): B2 H16 S485 16.7 -> 13.1 and B1 H16 S1428 37.1 -> 26.6 (64 x 4 x 32), B2 H16 S1014
+    29.3 -> 24.5 (64 x 2 x 32), B1 H16 S2979 79.3 -> 62.6 and S3772 109 -> 92 (128 x 2 x 64); but B3 H16 S986 31.8 -> 32.6,
+    B1 H128 S433 19.4 -> 25.2, B1 H16 S5334 182 -> 184 with the best of them."""
+    if seqlen_kv >= 440 and (wgs(64) <= _MI355X_CUS or (wgs(64) <= 2 * _MI355X_CUS and batch_heads <= 18)):
+        return PrefillTiles(n_waves=2, kv_groups=4, block_n=32)
+    if wgs(64) <= 2 * _MI355X_CUS and (seqlen_kv >= 320 or wgs(64) <= _MI355X_CUS):
+        return PrefillTiles(n_waves=2, kv_groups=2, block_n=32)
+    if wgs(128) <= _MI355X_CUS * 9 // 4 and batch_heads <= 36:
         return PrefillTiles(kv_groups=2)
     return None
 

@@ -240,7 +240,10 @@ class PrefillOp:
         """Tiles whose waves share the kv axis, where this engine's graph, its mask (``mask_plan(tiles)``) and the extents
         allow and want them: a merge the kernel knows (the proven online softmax, or no row state), no mask table, no
         tensor read per score."""
-        if (not (B and H and Sq and Skv) or self.extern_block_mask or self.D not in (64, 128) or self.DV not in (64, 128)
+        wide = (self.D, self.DV) == (192, 128)          # (measured for causal softmax only)
+        if (not (B and H and Sq and Skv) or self.extern_block_mask
+                or not (wide or (self.D in (64, 128) and self.DV in (64, 128)))
+                or (wide and (self.mask_mod is None or self._pipe_softmax is None or self.split_kv))
                 or not (self._pipe_softmax is not None or self._pipe_elementwise)
                 or any(c.per_kv for c in self.functors.customs) or os.environ.get("AE_PREFILL_KERNEL", "")):
             return None
@@ -252,7 +255,7 @@ class PrefillOp:
             if lm.uses_b or lm.uses_h:
                 return None
             plan = mask_plan(found)
-            if not (plan.mode == 1 or plan.band is not None):
+            if not (plan.mode == 1 or (plan.band is not None and not wide)):
                 return None
         return found
 

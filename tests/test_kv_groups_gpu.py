@@ -56,6 +56,34 @@ def test_kv_groups_against_the_oracle(cuda_device, tiles, D, dtype, mask):
         assert (lse[~seen] == float("-inf")).all()
 
 
+def test_the_choice_of_wide_key_launches():
+    def choice(H, S, B=1):
+        return kv_group_tiles(192, 128, B * H, S, S, True)
+    assert choice(16, 485, 2) == choice(16, 1428) == TILES[1]
+    assert choice(16, 343) == choice(16, 1014, 2) == choice(32, 899) == TILES[2]
+    assert choice(16, 2979) == choice(32, 1514) == TILES[3]
+    assert choice(16, 986, 3) is None and choice(128, 433) is None and choice(16, 5334) is None and choice(32, 262, 3) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tiles", TILES[1:], ids=lambda t: f"{t.block_m}x{t.kv_groups}x{t.block_n}")
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_kv_groups_of_wide_keys(cuda_device, tiles, dtype):
+    """Head dims 192 / 128: one key, tiles and groups that end inside each other, more tiles than two per group."""
+    D, DV = 192, 128
+    for B, H, Hkv, S in ((1, 2, 2, 1), (1, 2, 1, 33), (2, 3, 3, 129), (1, 4, 2, 390), (1, 2, 2, 1000)):
+        print(f"case wide key groups {tiles.block_m}x{tiles.kv_groups}x{tiles.block_n} B{B} H{H} S{S} {dtype}", flush=True)
+        q, k, v = C.make_inputs(B, S, S, H, Hkv, D, DV, dtype, seed=S)
+        meta = (meta_tensor(B, H, S, D, dtype=dtype), meta_tensor(B, Hkv, S, D, dtype=dtype), meta_tensor(B, Hkv, S, DV, dtype=dtype))
+        op = PrefillOp(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), C.causal_mask, C.OnlineSoftmax(), "-inf",
+                       tiles=tiles)
+        assert op.tiles == tiles and "#define AE_KW " in op.source
+        out = op(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+        ref, rlse = R.softmax_attention(q, k, v, causal=True)
+        assert (out - ref).abs().max().item() <= 2e-2
+        assert (op.final_rowscales["lse"].cpu() - rlse).abs().max().item() <= 1e-3
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("Sq,Skv", [(1, 40), (1, 1000), (31, 129), (33, 700), (64, 2100)])
 def test_kv_groups_of_split_launches(cuda_device, Sq, Skv):
