@@ -780,6 +780,14 @@ def _wide_key_group_tiles(wgs, batch_heads: int, seqlen_kv: int):
     return None
 
 
+def window_group_tiles(batch_heads: int, seqlen_q: int):
+    """Tiles of a sliding window at head dim 64 whose 64-row tiles no longer all find a place as four groups of waves, while
+    the 128-row ones do not fill the chip twice; None elsewhere."""
+    if batch_heads * -(-seqlen_q // 64) > 7 * _MI355X_CUS // 4 and batch_heads * -(-seqlen_q // 128) <= 15 * _MI355X_CUS // 8:
+        return PrefillTiles(n_waves=2, kv_groups=2, block_n=32)
+    return None
+
+
 def kv_group_tiles_split(seqlen_q: int, batch_heads: int = 0):
     """The same for launches that also split the kv axis over workgroups (a few query tokens against a long cache): the
     query rows decide.  fp16 D128: B8 H32 Sq4 Skv4096 110 -> 95 us, B1 H32 Sq16 Skv16000 55 -> 46 (32 x 4 x 32); B2 H16 Sq40

@@ -93,10 +93,12 @@ class PrefillOp:
             self.tiles = L.PrefillTiles()
         self._table_tiles = L.PrefillTiles() if split_kv else self.tiles     # ... of a call that brings a block mask
         # Band masks are read in 32-key tiles (B2 H32 S4096 D128, window of 256: 94.8 -> 88.4 us with them, of 1024 184 -> 180):
-        # less of the band's edges is multiplied.
+        # less of the band's edges is multiplied.  At head dim 64, whose tiles cost more to start than to multiply, only
+        # narrow ones (B3 H16 S2719, window 133: 22.0 -> 20.3; B1 H16 S6102 of 655 55.5 against 59.6 with 32 keys, B4 H16
+        # S1278 of 856 23.5 against 24.4; 26 windows of 180 to 1000 keys: 3 % on average, 12 at most).
         if self.mask_mod is not None and self.tiles == L.PrefillTiles() and self.D in (64, 128) and self.DV in (64, 128):
             band = self._probe_mask(q_meta, v_meta).band
-            if band is not None and band[1] is not None:
+            if band is not None and band[1] is not None and (max(self.D, self.DV) > 64 or band[1] - band[0] < 180):
                 self.tiles = L.PrefillTiles(block_n=32)
         # Launches that leave the chip idle with these tiles: waves that share the kv axis.  That depends on the extents
         # of a call, so an engine declared at such extents decides again for every shape it is called with (tiles_for);
@@ -249,6 +251,14 @@ class PrefillOp:
             return None
         if self.split_kv:
             return L.kv_group_tiles_split(Sq, B * H) if self.mask_mod is None else None
+        if self.mask_mod is not None and max(self.D, self.DV) == 64:
+            # (a window's workgroups do not differ in length as a causal mask's do: four groups a CU are too many where
+            # 64-row tiles outnumber the places for them.  B3 H16 S755, window 121: 11.7 -> 8.4 us, B3 H16 S1155 of 862
+            # 24.1 -> 19.0, B1 H16 S3095 of 146 11.9 -> 11.1)
+            two = L.window_group_tiles(B * H, Sq)
+            band = mask_plan(two).band if two is not None else None
+            if band is not None and band[1] is not None and not (self.functors.mask.uses_b or self.functors.mask.uses_h):
+                return two
         found = L.kv_group_tiles(self.D, self.DV, B * H, Sq, Skv, self.mask_mod is not None)
         if found is not None and self.mask_mod is not None:
             lm = self.functors.mask
