@@ -780,6 +780,19 @@ def _wide_key_group_tiles(wgs, batch_heads: int, seqlen_kv: int):
     return None
 
 
+def short_key_tiles_pay(batch_heads: int, seqlen_q: int, seqlen_kv: int) -> bool:
+    """Whether an unmasked launch of the generic kernel at head dim 128 takes less time with 32-key tiles: half the LDS, so
+    that three workgroups share a CU instead of two, and less padding at the end of the keys, for 12 % more time a key.
+    One round of three where there were two of two (B24 H32 S73 bf16 16.8 -> 13.8 us, B18 H8 S481 32.6 -> 30.6, B17 H8 S387 29.4 ->
+    26.5), or padding saved over several rounds (B21 H32 S216 fp16 42.7 -> 34.7, B27 H32 S266 bf16 72.1 -> 63.3; B5 H32
+    S1328, which has none, 158.6 -> 160.4), or most of it in one round (B16 H32 S85 10.7 -> 10.3)."""
+    wgs = batch_heads * -(-seqlen_q // 128)
+    padding = 2 * -(-seqlen_kv // 64) / -(-seqlen_kv // 32)
+    if wgs <= 2 * _MI355X_CUS:
+        return padding >= 1.3 and wgs > 3 * _MI355X_CUS // 2
+    return wgs <= 3 * _MI355X_CUS or (padding >= 1.04 and wgs > 13 * _MI355X_CUS // 4)
+
+
 def window_group_tiles(batch_heads: int, seqlen_q: int):
     """Tiles of a sliding window at head dim 64 whose 64-row tiles no longer all find a place as four groups of waves, while
     the 128-row ones do not fill the chip twice; None elsewhere."""

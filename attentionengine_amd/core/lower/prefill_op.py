@@ -273,19 +273,31 @@ class PrefillOp:
         """The tile configuration of a call with these extents."""
         key = (B, H, Sq, Skv)
         if key == self._declared or (self.tiles.kv_groups == 1 and self.tiles is not self._groups):
-            return self._causal_choice(key, self.tiles)
+            return self._call_choice(key, self.tiles)
         tiles = self._call_tiles.get(key)
         if tiles is None:
             tiles = self._call_tiles[key] = self._kv_group_choice(
                 *key, lambda found: self._plan(*key, device=None, tiles=found)) or self._base
-        return self._causal_choice(key, tiles)
+        return self._call_choice(key, tiles)
+
+    def _call_choice(self, key, tiles):
+        """``tiles``, or where they are this operator's own choice what is faster for a call with these extents."""
+        if self._tiles_given or self._tune_file or self.extern_block_mask or self.split_kv or (self.D, self.DV) != (128, 128):
+            return tiles
+        if self.mask_mod is not None:
+            return self._causal_choice(key, tiles)
+        B, H, Sq, Skv = key
+        if (tiles == L.PrefillTiles() and (self._pipe_softmax is not None or self._pipe_elementwise) and Sq and Skv
+                and not any(c.per_kv for c in self.functors.customs) and not os.environ.get("AE_PREFILL_KERNEL", "")
+                and L.short_key_tiles_pay(B * H, Sq, Skv)):
+            return L.PrefillTiles(block_n=32)
+        return tiles
 
     def _causal_choice(self, key, tiles):
         """``tiles``, or the generic kernel's where they are the pipelined kernel's by this operator's own choice, would be at
         these extents too, and a causal call is faster in the generic one (lower.pipelined_pays)."""
         B, H, Sq, Skv = key
-        if (tiles.template != "ae_prefill_pipe.hip" or self.mask_mod is None or self._pipe_softmax is None or Sq != Skv or not Sq
-                or (self.D, self.DV) != (128, 128) or self._tiles_given or self._tune_file or self.extern_block_mask):
+        if tiles.template != "ae_prefill_pipe.hip" or self._pipe_softmax is None or Sq != Skv or not Sq:
             return tiles
         generic = self._causal_generic.get(key)
         if generic is None:

@@ -65,6 +65,35 @@ def test_the_choice_of_wide_key_launches():
     assert choice(16, 986, 3) is None and choice(128, 433) is None and choice(16, 5334) is None and choice(32, 262, 3) is None
 
 
+def test_the_choice_of_windows_and_short_keys():
+    """Windows at head dim 64: two groups while 128-row tiles do not fill the chip twice, then 64-key tiles unless the window is
+    narrow; short unmasked calls at head dim 128: 32-key tiles where three workgroups a CU or less padding pay."""
+    def window(B, S, w, D=64):
+        return _engine(S, C.make_sliding_window_mask(w), H=16, Hkv=16, D=D, B=B)._op.tiles_for(B, 16, S, S)
+    assert window(3, 755, 121) == TILES[2] and window(1, 6102, 655) == PrefillTiles()
+    assert window(3, 2719, 133) == PrefillTiles(block_n=32) == window(3, 4096, 655, D=128)
+    def full(B, H, S):
+        return _engine(S, None, H=H, Hkv=H, B=B)._op.tiles_for(B, H, S, S)
+    assert full(24, 32, 73) == full(21, 32, 216) == full(17, 8, 387) == PrefillTiles(block_n=32)
+    assert full(5, 32, 1328) == full(16, 16, 256) == PrefillTiles()
+    op = _engine(73, None, H=32, Hkv=32, B=24)._op
+    assert op.tiles_for(16, 16, 256, 256) == PrefillTiles() and op.tiles_for(8, 32, 349, 349) == PrefillTiles(block_n=32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,S", [(24, 32, 73), (17, 8, 387), (21, 32, 216)])
+def test_short_unmasked_calls(cuda_device, B, H, S):
+    """... computed with those tiles: the oracle's results on the first and the last (batch, head)."""
+    D, dtype = 128, torch.bfloat16
+    mod = _engine(S, None, H=H, Hkv=H, B=B)
+    q, k, v = C.make_inputs(B, S, S, H, H, D, D, dtype, seed=S)
+    out = mod(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+    for b, h in ((0, 0), (B - 1, H - 1)):
+        ref, rlse = R.softmax_attention(*(t[b:b + 1, :, h:h + 1] for t in (q, k, v)), causal=False)
+        assert (out[b:b + 1, :, h:h + 1] - ref).abs().max().item() <= 2e-2
+        assert (mod.final_rowscales["lse"].cpu()[b, h] - rlse[0, 0]).abs().max().item() <= 1e-3
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tiles", TILES[1:], ids=lambda t: f"{t.block_m}x{t.kv_groups}x{t.block_n}")
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
