@@ -447,7 +447,7 @@ class PrefillOp:
         best = None
         for n in range(2, cls.MAX_TAIL_PARTS + 1):
             per = -(-kv_tiles // n)
-            if -(-kv_tiles // per) != n:
+            if -(-kv_tiles // per) != n or 8 * rest * n * 0.136 * width > 128:      # (MB of partial results)
                 continue
             us = -(-rest * n // cus_per_xcd) * (start + trip * per) + 3.0 + 1.2 * n * width
             if best is None or us < best[0]:
