@@ -665,7 +665,7 @@ class PrefillOp:
                 shared = {"n_split": tail[1], "kv_per_split": p.kv_per_split, "tail_slots": tail[0], "counters": 8 * tail[0],
                           "o_rows": 8 * tail[0] * tail[1] * (tiles.block_m + 4 * tiles.threads // self.DV)}
                 partial_o = torch.empty((shared["o_rows"], self.DV), dtype=torch.float32, device=dev)
-                counters = self._host.work(1, 1, shared["counters"], dev.index, stream)[1]
+                counters = self._host.work(1, 1, shared["counters"], dev.index, stream, True)[1]
                 p.partial_o, p.partial_rs = partial_o.data_ptr(), counters.data_ptr() + 4
                 keep += [partial_o, counters]
             if self._clock_stamps(tiles):

@@ -142,14 +142,17 @@ at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dt, int device) {
 
 // The work buffers of a launch on `stream` (see Work).  A capture that finds none kept gets buffers of its own, which live
 // in the graph's memory, and records the clearing of their counters: what a capture allocates and clears is only there
-// when that graph has been replayed, so no other call may be given it.
-std::pair<at::Tensor, at::Tensor> get_work(Host* h, int64_t o_rows, int64_t rs_floats, int64_t counters, int device, void* stream) {
+// when that graph has been replayed, so no other call may be given it.  `eager_only`: a capture always gets its own, so
+// that its replays share nothing with any other call, on whatever streams they run (the clearing is one launch of about 2 us
+// in a graph whose kernel takes a hundred).
+std::pair<at::Tensor, at::Tensor> get_work(Host* h, int64_t o_rows, int64_t rs_floats, int64_t counters, int device, void* stream,
+                                           bool eager_only) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   bool capturing = true;
   if (hipStreamIsCapturing((hipStream_t)stream, &status) == hipSuccess) capturing = status != hipStreamCaptureStatusNone;
   else (void)hipGetLastError();         // (the default stream while another one captures)
   for (auto& w : *h->work)
-    if (w.device == device && w.stream == stream && w.o_rows == o_rows && w.rs_floats == rs_floats && w.counters == counters) {
+    if (!(eager_only && capturing) && w.device == device && w.stream == stream && w.o_rows == o_rows && w.rs_floats == rs_floats && w.counters == counters) {
       w.captured = w.captured || capturing;
       return {w.partial_o, w.partial_rs};
     }
@@ -404,9 +407,9 @@ PyObject* run(Host* h, PyObject* const* args, Py_ssize_t nargs, bool mla) {
   if (pl.tail_slots) {      // (only the counters are kept: the partial results are the size of a few thousand rows)
     p.tail_slots = pl.tail_slots;
     po = empty({pl.o_rows, h->DV}, at::kFloat, dev);
-    prs = get_work(h, 1, 1, pl.counters, dev, stream).second.narrow(0, 1, pl.counters);
+    prs = get_work(h, 1, 1, pl.counters, dev, stream, true).second.narrow(0, 1, pl.counters);
   } else if (pl.cfg.merge_in_wg == 2) {
-    std::tie(po, prs) = get_work(h, pl.o_rows, rs_floats, pl.counters, dev, stream);
+    std::tie(po, prs) = get_work(h, pl.o_rows, rs_floats, pl.counters, dev, stream, false);
   } else if (pl.n_split > 1 && pl.cfg.merge_in_wg == 0) {
     po = empty({pl.o_rows, h->DV}, at::kFloat, dev);
     prs = empty({rs_floats}, at::kFloat, dev);
@@ -535,14 +538,14 @@ PyObject* host_add_backward(PyObject* self, PyObject* d) {
   END_HANDLE_TH_ERRORS
 }
 
-// work(o_rows, rs_floats, counters, device, stream) -> (partial_o, partial_rs)
+// work(o_rows, rs_floats, counters, device, stream, eager_only) -> (partial_o, partial_rs)
 PyObject* host_work(PyObject* self, PyObject* args) {
   HANDLE_TH_ERRORS
   long long o_rows, rs_floats, counters, stream;
-  int device;
-  if (!PyArg_ParseTuple(args, "LLLiL", &o_rows, &rs_floats, &counters, &device, &stream)) return nullptr;
+  int device, eager_only = 0;
+  if (!PyArg_ParseTuple(args, "LLLiL|p", &o_rows, &rs_floats, &counters, &device, &stream, &eager_only)) return nullptr;
   TORCH_CHECK(o_rows > 0 && rs_floats > 0 && counters > 0, "work(): sizes must be positive");
-  auto w = get_work((Host*)self, o_rows, rs_floats, counters, device, (void*)(uintptr_t)stream);
+  auto w = get_work((Host*)self, o_rows, rs_floats, counters, device, (void*)(uintptr_t)stream, eager_only != 0);
   PyObject* res = PyTuple_New(2);
   if (!res) return nullptr;
   PyTuple_SET_ITEM(res, 0, THPVariable_Wrap(w.first));
@@ -587,7 +590,7 @@ PyMethodDef host_methods[] = {
      "run_mla(q, q_pe, kv, k_pe) or run_mla(q, cache[, block_table, cache_seqlens]) -> (out, *row scales) or None"},
     {"add", host_add, METH_O, "add(plan dict)"},
     {"add_backward", host_add_backward, METH_O, "add_backward(plan dict)"},
-    {"work", host_work, METH_VARARGS, "work(o_rows, rs_floats, counters, device, stream) -> (partial_o, partial_rs) with zero counters"},
+    {"work", host_work, METH_VARARGS, "work(o_rows, rs_floats, counters, device, stream[, eager_only]) -> (partial_o, partial_rs) with zero counters"},
     {"clear", host_clear, METH_NOARGS, "drop every plan"},
     {nullptr, nullptr, 0, nullptr}};
 PyType_Slot host_slots[] = {{Py_tp_new, (void*)host_new}, {Py_tp_dealloc, (void*)host_dealloc}, {Py_tp_methods, host_methods},

@@ -1143,6 +1143,59 @@ def test_q_tiles_shared_by_several_workgroups(cuda_device, monkeypatch, kind, B,
         torch.cuda.synchronize()
 
 
+def test_graphs_of_shared_q_tiles_have_counters_of_their_own(cuda_device, monkeypatch):
+    """Two graphs of a launch whose q tiles are shared, captured on a stream that has run it eagerly, replayed on two streams
+    next to eager calls on the first: each has the eager result.  A count left in the counters that the eager calls of that
+    stream keep (as a call still under way leaves one) does not reach the graphs."""
+    print("case graphs of shared q tiles", flush=True)
+    monkeypatch.setenv("AE_PREFILL_KERNEL", "pipelined")
+    B, H, S, D, dtype, tail = 1, 8, 1088, 128, torch.float16, (3, 4, 5)
+    inputs = [tuple(t.cuda() for t in C.make_inputs(B, S, S, H, H, D, D, dtype, seed=i)) for i in range(3)]
+    mod = _engine(B, H, S, D, D, dtype, C.make_scale_score_mod(1 / math.sqrt(D)), None, C.OnlineSoftmax())
+    op = mod.attention
+    op._tail_plan = lambda *a: tail
+    want = [mod(*x).clone() for x in inputs]
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    for warm in (False, True):                   # through Python, through the native host path
+        if not warm:
+            op._host.clear()
+        graphs, outs = [], []
+        with torch.cuda.stream(streams[0]):
+            mod(*inputs[0])
+            if not warm:
+                op._host.clear()
+        for x in inputs[:2]:
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1], stream=streams[0]):
+                outs.append(mod(*x))
+            if not warm:
+                op._host.clear()
+        torch.cuda.synchronize()
+        kept = op._host.work(1, 1, 8 * tail[0], 0, streams[0].cuda_stream, True)[1].view(torch.int32)
+        kept[1:] += 1
+        torch.cuda.synchronize()
+        for out in outs:
+            out.zero_()
+        torch.cuda.synchronize()
+        for g, out, x in zip(graphs, outs, want):
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, x)
+        assert kept[1:].eq(1).all()
+        kept[1:] -= 1
+        torch.cuda.synchronize()
+        for _ in range(20):                      # all three under way at once
+            for s, g in zip(streams[1:], graphs):
+                with torch.cuda.stream(s):
+                    g.replay()
+            with torch.cuda.stream(streams[0]):
+                eager = mod(*inputs[2])
+        torch.cuda.synchronize()
+        for got, x in zip(outs + [eager], want):
+            assert torch.equal(got, x)
+
+
 def test_a_share_without_visible_keys_weighs_nothing(cuda_device, monkeypatch):
     """A share whose scores are all -inf has no reference and adds nothing, also where the others' references are far
     below zero."""
