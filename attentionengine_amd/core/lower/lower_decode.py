@@ -88,12 +88,63 @@ def merges_in_any_order(online_func, final_rowscale_names) -> bool:
 
 
 def combine_rows(threads, dv):
-    """Output rows of a merge workgroup (AE_COMBINE_ROWS of csrc/kernels/ae_combine.h): four value columns a thread."""
+    """Output rows of a merge workgroup (AE_COMBINE_ROWS of csrc/kernels/ae_combine.hip): four value columns a thread."""
     return max(1, threads // (dv // 4))
 
 
+def merge_capacity(n, any_order):
+    """Partial results that a merge of ``n`` is built for.  The log-sum-exp merge gives places without a result no weight, so
+    it is built for powers of two: a cache that grows by a token a call meets a new kernel only where it has doubled.  What
+    the empty places cost: 0.1 us a call (B4 H64 Skv1723, 11 of 16 places: merge 3.72 -> 3.80 us).  Another combine() is
+    built for its exact count."""
+    return 1 << (n - 1).bit_length() if any_order else n
+
+
+def merge_config(dv, dtype, n_rowscales, capacity, threads, splits_per_partial=1):
+    """ae_config.h of csrc/kernels/ae_combine.hip."""
+    return "\n".join([
+        "// generated by core/lower/lower_decode.py -- do not edit",
+        f"#define AE_DV {dv}",
+        f"#define AE_DTYPE_BF16 {1 if dtype == torch.bfloat16 else 0}",
+        f"#define AE_N_ROWSCALES {n_rowscales}",
+        f"#define AE_NSPLIT {capacity}",
+        f"#define AE_SPLITS_PER_PARTIAL {splits_per_partial}",
+        f"#define AE_COMBINE_THREADS {threads}",
+        "",
+    ])
+
+
+class Merges:
+    """The merge kernels of one operator (csrc/kernels/ae_combine.hip)."""
+
+    def __init__(self, d, dv, dtype, n_rowscales, functor_src, any_order, threads, allow_spills=None):
+        self._dims, self._dtype, self._n_rowscales, self._functor_src = (d, dv), dtype, n_rowscales, functor_src
+        self._any_order, self._threads, self._allow_spills = any_order, threads, allow_spills
+        self._modules = {}
+
+    def config(self, n, splits_per_partial=1):
+        return merge_config(self._dims[1], self._dtype, self._n_rowscales, merge_capacity(n, self._any_order), self._threads,
+                            splits_per_partial)
+
+    def cfg(self, n, splits_per_partial=1):
+        """The launch configuration of a merge of ``n`` partial results a row."""
+        return rt.TileCfg(block_m=combine_rows(self._threads, self._dims[1]),
+                          block_n=merge_capacity(n, self._any_order) * splits_per_partial, threads=self._threads, lds_bytes=0,
+                          head_dim=self._dims[0], head_dim_v=self._dims[1], elem_bytes=2, n_rowscales=self._n_rowscales,
+                          mask_mode=0, merge_in_wg=int(self._any_order))
+
+    def module(self, n, splits_per_partial=1):
+        key = (merge_capacity(n, self._any_order), splits_per_partial)
+        m = self._modules.get(key)
+        if m is None:
+            m = self._modules[key] = rt.compile_module(
+                "ae_combine.hip", {"ae_config.h": self.config(n, splits_per_partial), "ae_functors.h": self._functor_src},
+                allow_spills=self._allow_spills)
+        return m
+
+
 def render_decode_config(d, dv, dtype, n_waves, waves_per_eu, v_pad, n_rowscales, o_scale_one,
-                         even_kv, n_split, combine_threads, merge_in_wg=False, merge_last=False, wg_first=False) -> str:
+                         even_kv, n_split, merge_in_wg=False, merge_last=False, wg_first=False) -> str:
     return "\n".join([
         "// generated by core/lower/lower_decode.py -- do not edit",
         f"#define AE_D {d}",
@@ -106,7 +157,6 @@ def render_decode_config(d, dv, dtype, n_waves, waves_per_eu, v_pad, n_rowscales
         f"#define AE_WAVES_PER_EU {waves_per_eu}",
         f"#define AE_V_PAD {v_pad}",
         f"#define AE_NSPLIT {n_split}",
-        f"#define AE_COMBINE_THREADS {combine_threads}",
         f"#define AE_MERGE_IN_WG {1 if merge_in_wg else 0}",
         f"#define AE_MERGE_LAST {1 if merge_last else 0}",
         f"#define AE_WG_FIRST {1 if wg_first else 0}",
@@ -182,8 +232,8 @@ class GQADecodeOp(_SplitTuning):
     SPLIT_COEFF = 0.117
     MAX_WGS_PER_KV_HEAD = 16
     # ... and where a workgroup merges its waves' partials first (AE_WG_FIRST of ae_decode.hip: a quarter of the merge
-    # traffic), the counts that _workgroups() chooses from: each is a kernel of its own, and a cache that grows by a
-    # token a call should not meet a new one every few calls
+    # traffic), the counts that _workgroups() chooses from: up to 8 any, beyond those that the builds of
+    # ae_decode.hip take as constants (5, 6, 7 or 8 eighths of a power of two)
     GROUPED_WGS_PER_KV_HEAD = (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 48, 64)
 
     def __init__(self, qkv_meta, custom_fwd_inputs, score_mod, mask_mod, online_func, mask_value,
@@ -214,6 +264,9 @@ class GQADecodeOp(_SplitTuning):
         # must not allocate; launches whose partials exceed rt.NOALLOC_SCRATCH_BYTES are refused
         self.static_workspace = False
         self.v_pad = (64 - (2 * self.DV) % 256) % 256 or 256
+        self._merges = Merges(self.D, self.DV, self.dtype, self.n_rowscales, self.functor_src, self.grouped_merge,
+                              64 if self.DV <= 256 else 128, allow_spills)
+        self._builds = {}             # what _variant() compiled: counts of splits share a kernel
         self.final_rowscales = {}
         self.block_mask = None
         self._variants = {}
@@ -345,7 +398,7 @@ class GQADecodeOp(_SplitTuning):
         return self.grouped_merge and merge != 1 and n_split > self.N_WAVES
 
     def _variant(self, n_split, even_kv, merge):
-        """(module, split cfg, combine cfg, config source) of one compiled kernel pair.  ``merge`` (0: two
+        """(module, split cfg, combine cfg, config source) of a launch's split kernel.  ``merge`` (0: two
         launches; 1: the split kernel merges its waves' partial results itself, AE_MERGE_IN_WG; 2: its last workgroup
         merges, AE_MERGE_LAST) is part of the key: it depends on ``static_workspace`` and environment variables, which
         may change between calls, and a kernel compiled for one form must never be launched as another (the kernel
@@ -354,32 +407,36 @@ class GQADecodeOp(_SplitTuning):
         key = (n_split, even_kv, merge)
         v = self._variants.get(key)
         if v is None:
-            combine_threads = 64 if self.DV <= 256 else 128
             lds = self.N_WAVES * self.TILE * (2 * self.DV + self.v_pad)
             # Two waves a SIMD (256 registers each) where the kernel fits them; a build that spills at that size
             # (value heads of 256: 85 registers through scratch memory, 1.56 ms where the chip's HBM allows 0.6 for
             # B64 Hq32 Hkv8 Skv8192) is built again for one wave a SIMD and the whole register file: 0.68 ms.
             # several workgroups per kv head: merged by workgroup first, where combine() allows it (AE_WG_FIRST)
             wg_first = self._wg_first(n_split, merge)
-            for waves_per_eu in (2, 1):
-                cfg_src = render_decode_config(self.D, self.DV, self.dtype, self.N_WAVES, waves_per_eu, self.v_pad,
-                                               self.n_rowscales, self.functors.o_scale_one, even_kv,
-                                               n_split // self.N_WAVES if wg_first else n_split, combine_threads,
-                                               merge == 1, merge == 2, wg_first)
-                headers = {"ae_config.h": cfg_src, "ae_functors.h": self.functor_src}
-                module = rt.compile_module("ae_decode.hip", headers, allow_spills=True)
-                if not module.kernel_info()["ae_decode_split_kernel"].get(".vgpr_spill_count", 0):
-                    break
-            rt.check_spills(module, "ae_decode.hip", self.allow_spills)
+            per = self.N_WAVES if wg_first else 1
+            # what the build holds the weights of: the partial results that its last workgroup merges, or its waves'
+            most = merge_capacity(n_split // per, self.grouped_merge) if merge == 2 else self.N_WAVES
+            build = self._builds.get((most, even_kv, merge, wg_first))
+            if build is None:
+                for waves_per_eu in (2, 1):
+                    cfg_src = render_decode_config(self.D, self.DV, self.dtype, self.N_WAVES, waves_per_eu, self.v_pad,
+                                                   self.n_rowscales, self.functors.o_scale_one, even_kv, most,
+                                                   merge == 1, merge == 2, wg_first)
+                    headers = {"ae_config.h": cfg_src, "ae_functors.h": self.functor_src}
+                    module = rt.compile_module("ae_decode.hip", headers, allow_spills=True)
+                    if not module.kernel_info()["ae_decode_split_kernel"].get(".vgpr_spill_count", 0):
+                        break
+                rt.check_spills(module, "ae_decode.hip", self.allow_spills)
+                build = self._builds[(most, even_kv, merge, wg_first)] = module, cfg_src
+            module, cfg_src = build
             if merge == 1 or wg_first:
                 lds += self.n_rowscales * self.N_WAVES * 16 * 4       # the waves' row scales, behind the V tiles
             cfg = rt.TileCfg(block_m=self.HEADS_PER_WG, block_n=self.TILE, threads=64 * self.N_WAVES,
                              lds_bytes=lds, head_dim=self.D, head_dim_v=self.DV, elem_bytes=2,
                              n_rowscales=self.n_rowscales, mask_mode=0, merge_in_wg=merge)
-            ccfg = rt.TileCfg(block_m=combine_rows(combine_threads, self.DV), block_n=n_split, threads=combine_threads, lds_bytes=0,
-                              head_dim=self.D, head_dim_v=self.DV, elem_bytes=2,
-                              n_rowscales=self.n_rowscales, mask_mode=0)
-            v = self._variants[key] = (module, cfg, ccfg, cfg_src)
+            if merge == 0:
+                cfg_src += self._merges.config(n_split // per, per)
+            v = self._variants[key] = (module, cfg, self._merges.cfg(n_split // per, per), cfg_src)
         return v
 
     def __call__(self, q, k, v, *extra):
@@ -454,10 +511,14 @@ class GQADecodeOp(_SplitTuning):
         p.batch, p.heads_q, p.heads_kv, p.seqlen_q, p.seqlen_kv = B, Hq, Hkv, 1, Skv
         p.num_splits, p.kv_per_split = n_split, kv_per_split
         launch = rt.decode_fwd_noalloc if self.static_workspace else rt.decode_fwd
-        split, combine = module.kernel("ae_decode_split_kernel"), None if merge else module.kernel("ae_decode_combine_kernel")
+        split, combine, modules = module.kernel("ae_decode_split_kernel"), None, (module,)
+        if not merge:
+            per = self.N_WAVES if self._wg_first(n_split, merge) else 1
+            modules += (self._merges.module(n_split // per, per),)
+            combine = modules[1].kernel("ae_decode_combine_kernel")
         launch(split, combine, p, cfg, ccfg, stream)
         if not self.static_workspace:
-            host.add_forward(self._host, host.DECODE, B, 1, Hq, Hkv, Skv, dev, module, split, cfg, combine=combine, ccfg=ccfg,
+            host.add_forward(self._host, host.DECODE, B, 1, Hq, Hkv, Skv, dev, modules, split, cfg, combine=combine, ccfg=ccfg,
                              n_split=n_split, kv_per_split=kv_per_split, o_rows=o_rows, counters=counters,
                              env=("AE_DECODE_MERGE_IN_WG", "AE_DECODE_MERGE_LAST"))
         self.final_rowscales = dict(zip(self.names, rowscales))
@@ -465,8 +526,8 @@ class GQADecodeOp(_SplitTuning):
         return out
 
 
-def render_mla_config(d1, d2, dv, dtype, block_n, k_pad, n_rowscales, o_scale_one, n_split,
-                      combine_threads, softmax=None, paged=False, heads_per_wg=64) -> str:
+def render_mla_config(d1, d2, dv, dtype, block_n, k_pad, n_rowscales, o_scale_one, n_split, softmax=None,
+                      paged=False, heads_per_wg=64) -> str:
     extra = [f"#define AE_PAGED {1 if paged else 0}"]
     if heads_per_wg != 64:
         extra.append(f"#define AE_HPW {heads_per_wg}")
@@ -483,7 +544,6 @@ def render_mla_config(d1, d2, dv, dtype, block_n, k_pad, n_rowscales, o_scale_on
         f"#define AE_O_SCALE_ONE {1 if o_scale_one else 0}",
         f"#define AE_K_PAD {k_pad}",
         f"#define AE_NSPLIT {n_split}",
-        f"#define AE_COMBINE_THREADS {combine_threads}",
         *extra,
         "",
     ])
@@ -542,6 +602,8 @@ class MLADecodeOp(_SplitTuning):
         self.target_workgroups = target_workgroups
         self.final_rowscales = {}
         self.block_mask = None
+        self._merges = Merges(self.D, self.DV, self.dtype, self.n_rowscales, self.functor_src,
+                              merges_in_any_order(online_func, self.names), 128, allow_spills)
         self._variants = {}
         self._plans = {}
         self.source = self.functor_src
@@ -549,7 +611,9 @@ class MLADecodeOp(_SplitTuning):
         if not any(isinstance(x, str) for x in shape):
             B, Hq, Hkv, Skv = (int(x) for x in shape)
             heads, n_split, _ = self.plan(B, Hq, Hkv, Skv)
-            self.source = self._variant(n_split, heads=heads)[3] + "\n" + self.functor_src
+            self.source = self._variant(n_split, heads=heads)[2] + "\n" + self.functor_src
+            if n_split > 1:
+                self.source = self._merges.config(n_split) + self.source
 
     def _cost(self, heads, n_split, B, Hkv, group, Skv, live=1.0):
         """Microseconds of a call of the wave-specialised kernel with ``heads`` query heads a workgroup, up to a constant:
@@ -621,14 +685,15 @@ class MLADecodeOp(_SplitTuning):
                 and os.environ.get("AE_MLA_KERNEL", "") != "generic")
 
     def _variant(self, n_split, paged=False, heads=64):
-        """``heads``: query heads of a workgroup (AE_HPW of the wave-specialised kernel)."""
-        v = self._variants.get((n_split, paged, heads))
+        """(module, cfg, config source) of the split kernel, one for every count of splits above 1.  ``heads``: query heads of a
+        workgroup (AE_HPW of the wave-specialised kernel)."""
+        key = (n_split > 1, paged, heads)
+        v = self._variants.get(key)
         if v is None:
-            combine_threads = 128
             ws = self._wave_specialised()
             self.template = "ae_mla_decode_ws.hip" if ws else "ae_mla_decode.hip"
             cfg_src = render_mla_config(self.DV, self.D2, self.DV, self.dtype, self.BLOCK_N, self.K_PAD,
-                                        self.n_rowscales, self.functors.o_scale_one, n_split, combine_threads,
+                                        self.n_rowscales, self.functors.o_scale_one, 2 if n_split > 1 else 1,
                                         self.functors.softmax if ws else None, paged, heads)
             # AE_CLOCK_STAMPS=1 (a measurement switch, read by ``bench.py --mfma-probe``): single-split launches of the
             # wave-specialised kernel report the shader clock their workgroups ran at (``self.clock_stamps``)
@@ -648,10 +713,7 @@ class MLADecodeOp(_SplitTuning):
             cfg = rt.TileCfg(block_m=heads, block_n=self.BLOCK_N, threads=threads, lds_bytes=lds,
                              head_dim=self.D, head_dim_v=self.DV, elem_bytes=2,
                              n_rowscales=self.n_rowscales, mask_mode=0, paged=1 if paged else 0)
-            ccfg = rt.TileCfg(block_m=combine_rows(combine_threads, self.DV), block_n=n_split, threads=combine_threads, lds_bytes=0,
-                              head_dim=self.D, head_dim_v=self.DV, elem_bytes=2,
-                              n_rowscales=self.n_rowscales, mask_mode=0)
-            v = self._variants[(n_split, paged, heads)] = (module, cfg, ccfg, cfg_src)
+            v = self._variants[key] = (module, cfg, cfg_src)
         return v
 
     def _call_paged(self, q, cache, block_table, cache_seqlens):
@@ -748,7 +810,8 @@ class MLADecodeOp(_SplitTuning):
             self._tune_splits(key, cands, lambda: self._launch(q1, q2, k1, k2, B, Hq, Hkv, Skv, paged),
                               lambda n: n > 0 and made_of(n) == n)
         heads, n_split, kv_per_split = self.plan(B, Hq, Hkv, Skv, page=paged[2] if paged is not None else None)
-        module, cfg, ccfg, _ = self._variant(n_split, paged is not None, heads)
+        module, cfg, _ = self._variant(n_split, paged is not None, heads)
+        ccfg = self._merges.cfg(n_split)
         out = torch.empty((B, 1, Hq, self.DV), dtype=self.dtype, device=dev)
         rowscales = [torch.empty((B, Hq, 1), dtype=torch.float32, device=dev) for _ in range(self.n_rowscales)]
         p = rt.AttnParams()
@@ -780,10 +843,13 @@ class MLADecodeOp(_SplitTuning):
             block_table, cache_seqlens, page, n_pages = paged
             p.block_table, p.seqlens_k = block_table.data_ptr(), cache_seqlens.data_ptr()
             p.block_table_stride, p.page_block_size, p.num_pages = block_table.stride(0), page, n_pages
-        split, combine = module.kernel("ae_mla_decode_split_kernel"), module.kernel("ae_decode_combine_kernel")
+        split, combine, modules = module.kernel("ae_mla_decode_split_kernel"), None, (module,)
+        if n_split > 1:
+            modules += (self._merges.module(n_split),)
+            combine = modules[1].kernel("ae_decode_combine_kernel")
         rt.mla_decode_fwd(split, combine, p, cfg, ccfg, rt.current_stream(dev))
         if not getattr(self, "_stamped", False) and (self.n_rowscales == 1 or not self.cute):
-            host.add_forward(self._host, host.MLA if paged is None else host.MLA_PAGED, B, 1, Hq, Hkv, Skv, dev, module, split,
+            host.add_forward(self._host, host.MLA if paged is None else host.MLA_PAGED, B, 1, Hq, Hkv, Skv, dev, modules, split,
                              cfg, combine=combine, ccfg=ccfg, n_split=n_split, kv_per_split=kv_per_split,
                              page=paged[2] if paged is not None else 0)
         self.final_rowscales = dict(zip(self.names, rowscales))

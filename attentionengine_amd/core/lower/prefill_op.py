@@ -18,7 +18,7 @@ from ..runtime import hip_rt as rt
 from ..runtime import host
 from ..transform.core import _convert_mask_to_block_mask, is_causal_mask
 from . import lower as L
-from .lower_decode import combine_rows
+from .lower_decode import Merges, lower_combine, merges_in_any_order
 from .mask import plan_mask, survey_mask
 
 
@@ -140,10 +140,12 @@ class PrefillOp:
                 raise NotImplementedError("split-KV prefill with a value head dim above 256")
             if not hasattr(online_func, "combine"):
                 raise NotImplementedError("split-KV needs OnlineFunc.combine to merge the partial results")
-            from .lower_decode import lower_combine
             if tiles is None and groups is None:
                 self.tiles = L.PrefillTiles()      # the generic kernel carries the split-KV mode
-            self.functor_src += lower_combine(online_func, self.functors.final_rowscale_names)
+            names = self.functors.final_rowscale_names
+            self.functor_src += lower_combine(online_func, names)
+            self._merges = Merges(self.D, self.DV, self.dtype, len(names), self.functor_src, merges_in_any_order(online_func, names),
+                                  self.COMBINE_THREADS, allow_spills)
         if self.extern_block_mask and self.tiles.rows_per_wave != 32 and (
                 self.mask_block[1] % self.tiles.block_n or
                 (self.tiles.block_m % self.mask_block[0] and self.mask_block[0] % self.tiles.block_m)):
@@ -215,6 +217,8 @@ class PrefillOp:
                                       plan.heavy_last and not self.extern_block_mask,
                                       None if self.extern_block_mask else self._band(plan, tiles))
         self.source = cfg_src + "\n" + self.functor_src
+        if n_split > 1:
+            self.source = self._merges.config(n_split) + self.source
         if infer_mask and mask_mod is not None and not self.extern_block_mask:
             self.block_mask = self._reference_block_mask(B, H, Sq, Skv)
 
@@ -496,7 +500,7 @@ class PrefillOp:
             table_rows = 1
         if mask_mode != 2:
             heavy_last = False
-        key = (mask_mode, even_q, even_kv, n_split, table_rows, bool(heavy_last), band, astuple(tiles), tail)
+        key = (mask_mode, even_q, even_kv, n_split > 1, table_rows, bool(heavy_last), band, astuple(tiles), tail)
         v = self._variants.get(key)
         if v is None:
             has_mask_mod = self.elementwise_mask and mask_mode != 1
@@ -518,7 +522,7 @@ class PrefillOp:
                 cfg_src += (f"#define AE_BAND 1\n#define AE_BAND_LO ({band[0]})\n"
                             f"#define AE_BAND_HI {'0x7fffffff' if band[1] is None else f'({band[1]})'}\n")
             if n_split > 1:
-                cfg_src += f"#define AE_NSPLIT {n_split}\n#define AE_COMBINE_THREADS {self.COMBINE_THREADS}\n"
+                cfg_src += "#define AE_NSPLIT 2\n"       # (a split launch; its count is the launch's)
             if self._clock_stamps(tiles):
                 cfg_src += "#define AE_CLOCK_STAMPS 1\n"
             if tail:
@@ -654,10 +658,8 @@ class PrefillOp:
             p.partial_o, p.partial_rs = partial_o.data_ptr(), partial_rs.data_ptr()
             p.num_splits, p.kv_per_split = n_split, kv_per_split
             keep += [partial_o, partial_rs]
-            ccfg = rt.TileCfg(block_m=combine_rows(self.COMBINE_THREADS, self.DV), block_n=n_split, threads=self.COMBINE_THREADS, lds_bytes=0,
-                              head_dim=self.D, head_dim_v=self.DV, elem_bytes=2,
-                              n_rowscales=self.n_rowscales, mask_mode=0)
-            rt.prefill_split_fwd(kern, module.kernel("ae_decode_combine_kernel"), p, cfg, ccfg, stream)
+            merge, ccfg = self._merges.module(n_split), self._merges.cfg(n_split)
+            rt.prefill_split_fwd(kern, merge.kernel("ae_decode_combine_kernel"), p, cfg, ccfg, stream)
         else:
             shared = {}
             if tail is not None:
@@ -683,8 +685,9 @@ class PrefillOp:
         if extern_mask is None and self.DV_launch == self.DV and not self._clock_stamps(tiles):
             if n_split > 1:
                 shared = {"n_split": n_split, "kv_per_split": kv_per_split}
-            host.add_forward(self._host, host.PREFILL_SPLIT if n_split > 1 else host.PREFILL, B, Sq, Hq, Hkv, Skv, dev, module,
-                             kern, cfg, combine=module.kernel("ae_decode_combine_kernel") if n_split > 1 else None,
+            host.add_forward(self._host, host.PREFILL_SPLIT if n_split > 1 else host.PREFILL, B, Sq, Hq, Hkv, Skv, dev,
+                             (module, merge) if n_split > 1 else (module,),
+                             kern, cfg, combine=merge.kernel("ae_decode_combine_kernel") if n_split > 1 else None,
                              ccfg=ccfg if n_split > 1 else None, **shared,
                              table=table if mode == 2 and band is None else None, mask_block=(mbm, mbn), env=("AE_CLOCK_STAMPS",))
         return out

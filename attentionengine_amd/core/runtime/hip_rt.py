@@ -533,7 +533,7 @@ def prefill_split_fwd(split: Kernel, combine: Kernel, params: AttnParams, cfg: T
 
 def mla_decode_fwd(split: Kernel, combine: Kernel, params: AttnParams, cfg: TileCfg,
                    combine_cfg: TileCfg, stream: int = 0):
-    _check(lib().ae_mla_decode_fwd(split.handle, combine.handle, C.byref(params), C.byref(cfg),
+    _check(lib().ae_mla_decode_fwd(split.handle, combine.handle if combine is not None else None, C.byref(params), C.byref(cfg),
                                    C.byref(combine_cfg), _VP(stream)))
 
 

@@ -53,16 +53,16 @@ def _handle(kernel):
     return kernel.handle.value if kernel is not None else 0
 
 
-def add_forward(host, kind, B, Sq, Hq, Hkv, Skv, device, module, kernel, cfg, combine=None, ccfg=None, n_split=1,
+def add_forward(host, kind, B, Sq, Hq, Hkv, Skv, device, modules, kernel, cfg, combine=None, ccfg=None, n_split=1,
                 kv_per_split=0, page=0, table=None, mask_block=(0, 0), env=(), o_rows=None, counters=0,
                 tail_slots=0):
     """Hands a forward launch that has just run to ``host``.  ``env``: switches read at every call; the plan holds
-    while they keep their values.  ``o_rows``: partial results a split launch writes (None: one per row and split);
+    while they keep their values.  ``modules``: what the kernels live in.  ``o_rows``: partial results a split launch writes (None: one per row and split);
     ``counters``: arrival counters of a launch whose last workgroup merges; ``tail_slots``: see ae_attn_params."""
     host.add({"kind": kind, "B": B, "Sq": Sq, "Hq": Hq, "Hkv": Hkv, "Skv": Skv, "page": page, "device": device.index,
               "k0": _handle(kernel), "k1": _handle(combine), "cfg": bytes(cfg), "ccfg": None if ccfg is None else bytes(ccfg),
               "n_split": n_split, "kv_per_split": kv_per_split, "o_rows": o_rows, "counters": counters, "tail_slots": tail_slots, "table": table, "mask_bm": mask_block[0],
-              "mask_bn": mask_block[1], "env": {n: os.environ.get(n, "") for n in env}, "keep": (module,)})
+              "mask_bn": mask_block[1], "env": {n: os.environ.get(n, "") for n in env}, "keep": tuple(modules)})
 
 
 def add_backward(host, B, Sq, Hq, Hkv, Skv, device, modules, delta, dkv, dq, cfg, n_rs, planes, tables=None, dkv_parts=0,

@@ -415,7 +415,17 @@ int ae_prefill_fwd(ae_kernel* k, const ae_attn_params* p, const ae_tile_cfg* cfg
   return ae_launch(k, p, sizeof *p, grid, block, (uint32_t)cfg->lds_bytes, stream);
 }
 
-// workgroups of the merge kernel for `rows` output rows of a batch entry: block_m rows each (ae_combine.h)
+// workgroups of the merge kernel for `rows` output rows of a batch entry: block_m rows each (ae_combine.hip)
+// the counts of splits that a kernel which merges takes
+static int check_merge_splits(const char* who, const ae_tile_cfg* c, int32_t num_splits) {
+  if (c->merge_in_wg != 0 && c->merge_in_wg != 1)
+    return fail(AE_ERR_INVALID_ARG, "%s: merge_in_wg=%d of a combine configuration", who, c->merge_in_wg);
+  if (c->merge_in_wg ? num_splits > c->block_n : num_splits != c->block_n)
+    return fail(AE_ERR_INVALID_ARG, "%s: combine kernel built for %s%d splits, got %d", who, c->merge_in_wg ? "up to " : "",
+                c->block_n, num_splits);
+  return AE_OK;
+}
+
 static uint32_t combine_grid(int32_t rows, const ae_tile_cfg* c) {
   const int32_t per = c->block_m > 0 ? c->block_m : 1;
   return (uint32_t)((rows + per - 1) / per);
@@ -453,11 +463,11 @@ static int decode_fwd_impl(ae_kernel* split, ae_kernel* combine, const ae_attn_p
       return fail(AE_ERR_INVALID_ARG, "ae_decode_fwd: a split kernel whose last workgroup merges takes no combine kernel");
     if (!p->partial_o || !p->partial_rs)
       return fail(AE_ERR_INVALID_ARG, "ae_decode_fwd: split-KV work buffers are NULL");
-    // (the kernel merges exactly the AE_NSPLIT partial results it was compiled for; the host cannot see that
-    // number, so it travels as it does for the merge kernel)
+    // (the host cannot see how many partial results the kernel was compiled to merge, so the number travels as it does
+    // for the merge kernel)
     if (!combine_cfg)
       return fail(AE_ERR_INVALID_ARG, "ae_decode_fwd: a split kernel whose last workgroup merges needs combine_cfg "
-                  "(its block_n is the number of splits the kernel was compiled for)");
+                  "(it says how many splits the kernel was compiled for)");
   }
   const bool merged = cfg->merge_in_wg == 1 || merge_last;
   if (merged && combine)
@@ -479,9 +489,7 @@ static int decode_fwd_impl(ae_kernel* split, ae_kernel* combine, const ae_attn_p
   if (p->num_splits % waves != 0)
     return fail(AE_ERR_INVALID_ARG, "ae_decode_fwd: num_splits=%d is not a multiple of %d waves",
                 p->num_splits, waves);
-  if (combine_cfg && combine_cfg->block_n != p->num_splits)
-    return fail(AE_ERR_INVALID_ARG, "ae_decode_fwd: combine kernel built for %d splits, got %d",
-                combine_cfg->block_n, p->num_splits);
+  if (combine_cfg && (rc = check_merge_splits("ae_decode_fwd", combine_cfg, p->num_splits))) return rc;
   int group = p->heads_q / p->heads_kv;
   int head_tiles = (group + cfg->block_m - 1) / cfg->block_m;
   uint32_t grid[3] = {(uint32_t)(p->num_splits / waves), (uint32_t)(head_tiles * p->heads_kv),
@@ -530,9 +538,7 @@ int ae_prefill_split_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_par
   if (p->kv_per_split % cfg->block_n != 0)
     return fail(AE_ERR_INVALID_ARG, "ae_prefill_split_fwd: kv_per_split=%d is not a multiple of block_n=%d",
                 p->kv_per_split, cfg->block_n);
-  if (combine_cfg->block_n != p->num_splits)
-    return fail(AE_ERR_INVALID_ARG, "ae_prefill_split_fwd: combine kernel built for %d splits, got %d",
-                combine_cfg->block_n, p->num_splits);
+  if ((rc = check_merge_splits("ae_prefill_split_fwd", combine_cfg, p->num_splits))) return rc;
   if (!p->partial_o || !p->partial_rs)
     return fail(AE_ERR_INVALID_ARG, "ae_prefill_split_fwd: split-KV work buffers are NULL");
   if (combine_cfg->threads <= 0 || combine_cfg->threads % 64 != 0 || combine_cfg->threads > 1024)
@@ -610,9 +616,7 @@ int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params
       (int64_t)p->num_splits * p->kv_per_split < p->seqlen_kv)
     return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: %d splits of %d do not cover Skv=%d",
                 p->num_splits, p->kv_per_split, p->seqlen_kv);
-  if (combine_cfg->block_n != p->num_splits)
-    return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: combine kernel built for %d splits, got %d",
-                combine_cfg->block_n, p->num_splits);
+  if ((rc = check_merge_splits("ae_mla_decode_fwd", combine_cfg, p->num_splits))) return rc;
   if (!direct && (!p->partial_o || !p->partial_rs))
     return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: split-KV work buffers are NULL");
   if (combine_cfg->threads <= 0 || combine_cfg->threads % 64 != 0 || combine_cfg->threads > 1024)
@@ -623,7 +627,7 @@ int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params
       return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: rowscale_out[%d] is NULL", i);
   // 1-D grid: head tiles of one (batch, kv head, split) sit 8 ids apart (same XCD); the
   // (batch, kv head, split) count is padded to a multiple of 8, surplus workgroups exit at once.  A large
-  // paged launch counts an odd number of splits per entry (ae_mla_units in ae_mla_paged.h).
+  // paged launch counts an odd number of splits per entry (ae_mla_odd_units in ae_mla_paged.h).
   int group = p->heads_q / p->heads_kv;
   int64_t n_ht = (group + cfg->block_m - 1) / cfg->block_m;
   int64_t units = (int64_t)p->batch * p->heads_kv * p->num_splits;

@@ -50,7 +50,7 @@
 // workgroup that finishes last instead of in a second launch: every workgroup writes its partial results with
 // device-scope stores, waits for them, then counts itself in with an atomic add on a counter of its (batch, kv head,
 // head tile); the one that reads gridDim.x - 1 is the last, sets the counter back to zero for the next launch, and
-// merges all AE_NSPLIT partial results in the order of ae_decode_combine_kernel (equal results to the last bit).  The
+// merges all partial results in the order of ae_decode_combine_kernel (equal results to the last bit).  The
 // counters are 32-bit integers behind the row scales in p.partial_rs (after max(1, AE_N_ROWSCALES) * batch * heads_q *
 // num_splits floats), one per (batch, blockIdx.y); they must be zero before the first launch and are left at zero by
 // every launch.  Saves the second launch and the gap in front of it: 2 to 4 us of a 20 us call at batch 1.
@@ -58,9 +58,14 @@
 #define AE_MERGE_LAST 0
 #endif
 static_assert(!(AE_MERGE_IN_WG && AE_MERGE_LAST), "one way to merge");
+// AE_NSPLIT: with AE_MERGE_LAST the most partial results that the build merges; the launch says how many there are.  So a
+// cache that grows by a token a call meets a new build at every doubling and not at every new count (0.4 to 1 s of
+// compilation each): B1 Hq32 Hkv8 from 128 to 32768 keys 6 builds, where every count of its own made 16.  Places beyond the
+// count weigh nothing; a combine() that is not known to take no notice of row scales of -inf gets a build for exactly the
+// launch's count.
 // 1 (where combine() is the log-sum-exp merge, whose result does not depend on the grouping): the waves of a workgroup
-// merge their partial results in LDS first and ONE partial result per workgroup goes to memory: AE_NSPLIT is then the
-// number of workgroups (p.num_splits / AE_NWAVES), with either form of the merge that follows.
+// merge their partial results in LDS first and ONE partial result per workgroup goes to memory, p.num_splits / AE_NWAVES
+// of them, with either form of the merge that follows.
 // A kv axis can then be shared out over four times as many workgroups for the same merge traffic, which is what a
 // batch of one to four needs: with one workgroup per 8 kv heads and 8 shares each wave walked eight tiles one memory
 // trip after the other (8.7 of 16.4 us of B1 Hq32 Hkv8 Skv8192).
@@ -75,6 +80,7 @@ static_assert(AE_DV % 16 == 0, "value head dim must be a multiple of 16");
 static_assert((AE_TILE * AE_VCPR) % 64 == 0, "V tile must split evenly over a wave");
 
 typedef __attribute__((address_space(3))) unsigned char ae_lds_byte;
+template <int N> struct ae_const_int { static constexpr int value = N; };
 
 extern "C" __global__ __launch_bounds__(AE_NT)
 __attribute__((amdgpu_waves_per_eu(AE_WAVES_PER_EU, AE_WAVES_PER_EU)))
@@ -291,11 +297,12 @@ void ae_decode_split_kernel(const ae_attn_params p) {
 #if AE_WG_FIRST
     // this workgroup's partial result of the tile's heads -> memory (device scope: see below)
     const int tile_heads = group - ht * 16 < 16 ? group - ht * 16 : 16;
-    const int64_t tile_row0 = ((int64_t)b * p.heads_q + hk * group + ht * 16) * AE_NSPLIT;
+    const int n_part = (unsigned)p.num_splits / AE_NWAVES;
+    const int64_t tile_row0 = ((int64_t)b * p.heads_q + hk * group + ht * 16) * n_part;
 #if AE_MERGE_LAST
     constexpr int kDeviceScope = 16;
     __amdgpu_buffer_rsrc_t po_buf = __builtin_amdgcn_make_buffer_rsrc(
-        p.partial_o + tile_row0 * AE_DV, 0, tile_heads * AE_NSPLIT * AE_DV * 4, 0x00020000);
+        p.partial_o + tile_row0 * AE_DV, 0, tile_heads * n_part * AE_DV * 4, 0x00020000);
 #endif
     for (int idx = tid; idx < tile_heads * (AE_DV / 4); idx += AE_NT) {
       const int hl = idx / (AE_DV / 4), dv = (idx % (AE_DV / 4)) * 4;
@@ -320,7 +327,7 @@ void ae_decode_split_kernel(const ae_attn_params p) {
 #pragma unroll
         for (int r = 0; r < 4; r++) acc[r] += v[r] * wk;
       }
-      const int row_in_tile = hl * AE_NSPLIT + blockIdx.x;
+      const int row_in_tile = hl * n_part + blockIdx.x;
 #if AE_MERGE_LAST
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(ae_u32x4, acc), po_buf, (row_in_tile * AE_DV + dv) * 4, 0,
                                              kDeviceScope);
@@ -368,9 +375,10 @@ void ae_decode_split_kernel(const ae_attn_params p) {
   // invalidates the whole L2: measured at several microseconds a workgroup, twice the call at batch 4).
   constexpr int kDeviceScope = 16;     // the sc1 bit of a buffer instruction's cache policy
   const int tile_heads = group - ht * 16 < 16 ? group - ht * 16 : 16;
-  const int64_t tile_row0 = ((int64_t)b * p.heads_q + hk * group + ht * 16) * AE_NSPLIT;
+  const int n_part = AE_WG_FIRST ? (unsigned)p.num_splits / AE_NWAVES : p.num_splits;
+  const int64_t tile_row0 = ((int64_t)b * p.heads_q + hk * group + ht * 16) * n_part;
   __amdgpu_buffer_rsrc_t po_buf = __builtin_amdgcn_make_buffer_rsrc(
-      p.partial_o + tile_row0 * AE_DV, 0, tile_heads * AE_NSPLIT * AE_DV * 4, 0x00020000);
+      p.partial_o + tile_row0 * AE_DV, 0, tile_heads * n_part * AE_DV * 4, 0x00020000);
 #if !AE_WG_FIRST
   if (head_ok) {
     const int row_in_tile = l16 * p.num_splits + split;
@@ -409,52 +417,81 @@ void ae_decode_split_kernel(const ae_attn_params p) {
     // Every other workgroup's partial results were in memory before it counted itself in.  One thread merges four
     // neighbouring output columns of one head; its loads of the row scales (the same addresses for the 32 threads
     // of a head) and of the first partial results go out together: one trip to memory, not one after the other.
-    for (int idx = tid; idx < tile_heads * (AE_DV / 4); idx += AE_NT) {
-      const int hl = idx / (AE_DV / 4), dv = (idx % (AE_DV / 4)) * 4;
-      const int hq2 = hk * group + ht * 16 + hl;
-      float rs[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1][AE_NSPLIT];
-#pragma unroll
-      for (int i = 0; i < AE_N_ROWSCALES; i++)
-#pragma unroll
-        for (int k = 0; k < AE_NSPLIT; k++)
-          rs[i][k] = __hip_atomic_load(p.partial_rs + (int64_t)i * p.batch * p.heads_q * AE_NSPLIT + tile_row0 +
-                                           hl * AE_NSPLIT + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      constexpr int G = AE_NSPLIT < 16 ? AE_NSPLIT : 16;     // partial results in flight at a time
-      ae_f32x4 val[G];
-#pragma unroll
-      for (int i = 0; i < G; i++)
-        val[i] = __builtin_bit_cast(ae_f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                  po_buf, ((hl * AE_NSPLIT + i) * AE_DV + dv) * 4, 0, kDeviceScope));
-      float w[AE_NSPLIT];
-      float merged[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1];
-      ae_combine(rs, w, merged);
-      // (the sum runs over the splits in ascending order, as in ae_decode_combine_kernel: equal to the last bit)
-      ae_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int k0 = 0; k0 < AE_NSPLIT; k0 += G) {
-        if (k0 > 0) {
-#pragma unroll
-          for (int i = 0; i < G; i++)
-            if (k0 + i < AE_NSPLIT)
-              val[i] = __builtin_bit_cast(ae_f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                        po_buf, ((hl * AE_NSPLIT + k0 + i) * AE_DV + dv) * 4, 0, kDeviceScope));
-        }
-#pragma unroll
-        for (int i = 0; i < G; i++)
-          if (k0 + i < AE_NSPLIT) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) acc[r] += val[i][r] * w[k0 + i];
-          }
-      }
-      ae_elem* orow = (ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)hq2 * p.o_stride_h + dv;
-#pragma unroll
-      for (int r = 0; r < 4; r++) orow[r] = (ae_elem)acc[r];
-      if (dv == 0) {
+    // `places`: the number of partial results where it is one of the four that plans ask for of this build (5, 6, 7 or 8
+    // eighths of AE_NSPLIT), a constant then, as are the offsets; 0 for any other, whose places beyond the count have a row scale of
+    // -inf and, from behind the buffer's end, a result of zero.  B1 Hq32 Hkv8 Skv8192, 32 places: 11.75 us; with the
+    // comparisons 12.2, and 20 of 32 places 12.1 against 13.1.
+    auto merge = [&](auto places) AE_LAMBDA {
+      constexpr bool kFixed = decltype(places)::value > 0;
+      constexpr int N = kFixed ? decltype(places)::value : AE_NSPLIT;
+      for (int idx = tid; idx < tile_heads * (AE_DV / 4); idx += AE_NT) {
+        const int hl = idx / (AE_DV / 4), dv = (idx % (AE_DV / 4)) * 4;
+        const int hq2 = hk * group + ht * 16 + hl;
+        // (the count is compared as a vector register, a copy for each use: 64 scalar conditions, or the results of as many
+        // vector ones kept from one use to the next, do not fit the scalar registers)
+        int n_row = n_part, n_load = n_part, n_weight = n_part;
+        if (!kFixed) asm volatile("" : "+v"(n_row), "+v"(n_load), "+v"(n_weight));
+        const int row_at = hl * (kFixed ? N : n_part);
+        float rs[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1][AE_NSPLIT];
 #pragma unroll
         for (int i = 0; i < AE_N_ROWSCALES; i++)
-          if (p.rowscale_out[i]) p.rowscale_out[i][(int64_t)b * p.heads_q + hq2] = merged[i];
+#pragma unroll
+          for (int k = 0; k < AE_NSPLIT; k++)
+            rs[i][k] = k >= N ? AE_NEG_INF
+                              : __hip_atomic_load(p.partial_rs + (int64_t)i * p.batch * p.heads_q * n_part + tile_row0 + row_at +
+                                                      (kFixed || k < n_row ? k : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        constexpr int G = N < 16 ? N : 16;     // partial results in flight at a time
+        ae_f32x4 val[G];
+        auto load_part = [&](int k) AE_LAMBDA -> ae_f32x4 {
+          return __builtin_bit_cast(ae_f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+              po_buf, kFixed || k < n_load ? ((row_at + k) * AE_DV + dv) * 4 : -1, 0, kDeviceScope));
+        };
+#pragma unroll
+        for (int i = 0; i < G; i++) val[i] = load_part(i);
+        if (!kFixed) {
+#pragma unroll
+          for (int i = 0; i < AE_N_ROWSCALES; i++)
+#pragma unroll
+            for (int k = 0; k < AE_NSPLIT; k++) rs[i][k] = k < n_weight ? rs[i][k] : AE_NEG_INF;
+        }
+        float w[AE_NSPLIT];
+        float merged[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1];
+        ae_combine(rs, w, merged);
+        // (the sum runs over the splits in ascending order, as in ae_decode_combine_kernel: equal to the last bit)
+        ae_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k0 = 0; k0 < N; k0 += G) {
+          if (k0 > 0) {
+#pragma unroll
+            for (int i = 0; i < G; i++)
+              if (k0 + i < N) val[i] = load_part(k0 + i);
+          }
+#pragma unroll
+          for (int i = 0; i < G; i++)
+            if (k0 + i < N) {
+#pragma unroll
+              for (int r = 0; r < 4; r++) acc[r] += val[i][r] * w[k0 + i];
+            }
+        }
+        ae_elem* orow = (ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)hq2 * p.o_stride_h + dv;
+#pragma unroll
+        for (int r = 0; r < 4; r++) orow[r] = (ae_elem)acc[r];
+        if (dv == 0) {
+#pragma unroll
+          for (int i = 0; i < AE_N_ROWSCALES; i++)
+            if (p.rowscale_out[i]) p.rowscale_out[i][(int64_t)b * p.heads_q + hq2] = merged[i];
+        }
       }
-    }
+    };
+    if (__builtin_expect(n_part == AE_NSPLIT, 1)) merge(ae_const_int<AE_NSPLIT>());
+#if AE_NSPLIT % 4 == 0
+    else if (n_part == AE_NSPLIT / 4 * 3) merge(ae_const_int<AE_NSPLIT / 4 * 3>());
+#endif
+#if AE_NSPLIT % 8 == 0
+    else if (n_part == AE_NSPLIT / 8 * 5) merge(ae_const_int<AE_NSPLIT / 8 * 5>());
+    else if (n_part == AE_NSPLIT / 8 * 7) merge(ae_const_int<AE_NSPLIT / 8 * 7>());
+#endif
+    else merge(ae_const_int<0>());
   }
 #elif !AE_WG_FIRST
   if (head_ok) {
@@ -474,6 +511,7 @@ void ae_decode_split_kernel(const ae_attn_params p) {
 #endif
 }
 
-#if !(AE_MERGE_IN_WG || AE_MERGE_LAST)
-#include "ae_combine.h"      // the merge kernel of the two-launch form
+#if defined(AE_COMBINE_THREADS) && !AE_MERGE_IN_WG && !AE_MERGE_LAST       // (a caller that wants both kernels in one module)
+#define AE_SPLITS_PER_PARTIAL (AE_WG_FIRST ? AE_NWAVES : 1)
+#include "ae_combine.h"
 #endif

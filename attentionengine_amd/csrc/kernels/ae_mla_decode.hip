@@ -93,6 +93,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #endif
   const int split = u % units;
   if (u >= p.batch * p.heads_kv * units || split >= p.num_splits) return;  // grid padding (whole workgroup exits)
+  if (AE_NSPLIT > 1 && !AE_PAGED && p.num_splits < 2) return;      // (a launch for the build that writes out)
   const int hk = (u / units) % p.heads_kv;
   const int b = u / (units * p.heads_kv);
   const int hblk = wave >> 1;     // which 16 heads of the workgroup
@@ -344,4 +345,6 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   }
 }
 
+#ifdef AE_COMBINE_THREADS       // (a caller that wants both kernels in one module)
 #include "ae_combine.h"
+#endif

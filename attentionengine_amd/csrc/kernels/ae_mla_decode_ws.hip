@@ -34,12 +34,12 @@
 // 16 or 32 heads.  Per head the tile is fetched and read two or four times as often as with 64 heads, which is why the
 // large launches keep that form.
 //
-// Configuration ("ae_config.h"): AE_HPW AE_D1 AE_D2 AE_DV AE_DTYPE_BF16 AE_N_ROWSCALES AE_NSPLIT
-// AE_COMBINE_THREADS AE_PAGED (1: the cache is paged, rows are found through ae_attn_params.block_table and
+// Configuration ("ae_config.h"): AE_HPW AE_D1 AE_D2 AE_DV AE_DTYPE_BF16 AE_N_ROWSCALES AE_NSPLIT (1: the kv axis is not split
+// and the kernel writes out; more: p.num_splits says how often, ae_combine.hip merges) AE_PAGED (1: the cache is paged, rows are found through ae_attn_params.block_table and
 // every batch entry has its own length seqlens_k[b], as in the reference's
 // cute_template_kvshared/kernels/params.h:33-36; a kv tile never straddles two pages), plus AE_SM_SCALE (the constant c > 0) and AE_SM_M / AE_SM_R (names of the
 // running-max and running-sum fields of ae_rowstate).  Functors used ("ae_functors.h"): ae_rowstate,
-// ae_rowstate_init, ae_epilogue, ae_load_custom, ae_combine.
+// ae_rowstate_init, ae_epilogue, ae_load_custom.
 
 #define AE_LAYOUT 1
 #include "ae_hip.h"
@@ -156,7 +156,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   // ---- which (head tile, split, kv head, batch): 1-D grid, ids 8 apart share their KV range ---------
   // (What a workgroup does before its first tile is requested is a serial chain that a short launch pays in full: the
   // integer divisions are left out where a shift does - one latent head, a power of two of head tiles, of tokens a page.
-  // The launch is planned with AE_NSPLIT splits.)
+  // The number of splits is the launch's: one build serves every count above one, and writes where the host planned.)
   int group = p.heads_q;
   if (__builtin_expect(p.heads_kv != 1, 0)) group /= p.heads_kv;
   const int n_ht = (int)((unsigned)(group + AE_HEADS_PER_WG - 1) / AE_HEADS_PER_WG);
@@ -170,11 +170,19 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     u8 = (wg >> 3) >> __builtin_ctz(n_ht);
   }
   const unsigned u = (unsigned)(u8 * 8 + (wg & 7));      // flattened (batch, kv head, split)
-  int split = u % AE_NSPLIT, b = u / AE_NSPLIT, hk = 0;
+#if AE_NSPLIT == 1
+  const int n_split = 1;
+  int split = 0, b = u, hk = 0;
+#else
+  const int n_split = p.num_splits;
+  int units = n_split, split, hk = 0;
 #if AE_PAGED
-  if (ae_mla_odd_units(p, n_ht)) split = u % (AE_NSPLIT | 1), b = u / (AE_NSPLIT | 1);
+  if (ae_mla_odd_units(p, n_ht)) units |= 1;
 #endif
-  if (b >= p.batch * p.heads_kv || split >= AE_NSPLIT) return;  // grid padding (whole workgroup exits)
+  int b = ae_divide((int)u, units, split);
+#endif
+  if (b >= p.batch * p.heads_kv || split >= n_split) return;  // grid padding (whole workgroup exits)
+  if (AE_NSPLIT > 1 && !AE_PAGED && n_split < 2) return;      // (a launch for the build that writes out)
   if (__builtin_expect(p.heads_kv != 1, 0)) {
     hk = b % p.heads_kv;
     b /= p.heads_kv;
@@ -864,10 +872,10 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     }
     // row scales: this lane's own head
     if (head_ok && hf == 0 && dvw == 0) {
-      const int64_t row = ((int64_t)b * p.heads_q + hq) * AE_NSPLIT + split;
+      const int64_t row = ((int64_t)b * p.heads_q + hq) * n_split + split;
 #pragma unroll
       for (int i = 0; i < AE_N_ROWSCALES; i++) {
-        if (!direct) p.partial_rs[(int64_t)i * p.batch * p.heads_q * AE_NSPLIT + row] = frs[i];
+        if (!direct) p.partial_rs[(int64_t)i * p.batch * p.heads_q * n_split + row] = frs[i];
         else if (p.rowscale_out[i]) p.rowscale_out[i][(int64_t)b * p.heads_q + hq] = frs[i];
       }
     }
@@ -908,12 +916,12 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
       }
     } else {
       constexpr int CPH = AE_DVW / 4, N = AE_HB * CPH / 64;
-      float* ob = p.partial_o + (((int64_t)b * p.heads_q + hk * group + ht * AE_HEADS_PER_WG) * AE_NSPLIT + split) * AE_DV + dvw * AE_DVW;
+      float* ob = p.partial_o + (((int64_t)b * p.heads_q + hk * group + ht * AE_HEADS_PER_WG) * n_split + split) * AE_DV + dvw * AE_DVW;
 #pragma unroll 8
       for (int i = 0; i < N && i * 64 < (heads_here - hb * AE_HB) * CPH; i++) {
         const int hs = hb * AE_HB + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
         const ae_f32x4 w = *(const __attribute__((address_space(3))) ae_f32x4*)(obuf + hs * (AE_DVW * 4) + ((c ^ (hs & AE_OSW)) << 4));
-        if (hs < heads_here) __builtin_nontemporal_store(w, (ae_f32x4*)(ob + (int64_t)hs * AE_NSPLIT * AE_DV + c * 4));
+        if (hs < heads_here) __builtin_nontemporal_store(w, (ae_f32x4*)(ob + (int64_t)hs * n_split * AE_DV + c * 4));
       }
     }
   }
@@ -937,4 +945,6 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #endif
 }
 
+#ifdef AE_COMBINE_THREADS       // (a caller that wants both kernels in one module)
 #include "ae_combine.h"
+#endif

@@ -1,5 +1,5 @@
 // Shared by the two MLA decode templates when they are built for a paged cache (AE_PAGED 1); included
-// after AE_DV, AE_NT, AE_HEADS_PER_WG, AE_NSPLIT and AE_N_ROWSCALES are defined.
+// after AE_DV, AE_NT, AE_HEADS_PER_WG and AE_N_ROWSCALES are defined.
 //
 // Splits of a batch entry that hold keys: ceil(length / kv_per_split).  An entry with at most one writes its
 // result itself (split 0: `out` and the row scales, as a launch without splits does) and the merge kernel

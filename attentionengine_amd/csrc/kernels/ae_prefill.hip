@@ -35,7 +35,7 @@
 #include "ae_hip.h"
 #include "ae_config.h"    // generated: the AE_* configuration macros
 #ifndef AE_NSPLIT
-#define AE_NSPLIT 1                // > 1: split-KV, fp32 partial results + the merge kernel of ae_combine.h
+#define AE_NSPLIT 1                // > 1: split-KV, p.num_splits fp32 partial results a row, merged by ae_combine.hip
 #endif
 #include "ae_device.h"
 // custom inputs with a kv dimension (one element per score) are fetched a tile ahead: a lane's groups of four
@@ -247,8 +247,9 @@ void ae_prefill_kernel(const ae_attn_params p) {
   const int n_bh = p.batch * p.heads_q;
 #if AE_NSPLIT > 1
   // split-KV ("decode" with several query tokens): consecutive ids are the splits of one q tile
-  const int split = blockIdx.x % AE_NSPLIT;
-  const int wg = blockIdx.x / AE_NSPLIT;
+  const int n_split = p.num_splits;
+  int split;
+  const int wg = ae_divide(blockIdx.x, n_split, split);
 #else
   const int wg = blockIdx.x;
 #endif
@@ -780,7 +781,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
     }
     if (q_ok[0]) {
 #if AE_NSPLIT > 1
-      const int64_t prow = ((((int64_t)b * p.seqlen_q + qrow[0]) * p.heads_q + h) * AE_NSPLIT) + split;
+      const int64_t prow = ((((int64_t)b * p.seqlen_q + qrow[0]) * p.heads_q + h) * n_split) + split;
       float* po = p.partial_o + prow * AE_DV;
 #else
       ae_elem* po = (ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)qrow[0] * p.o_stride_s + (int64_t)h * p.o_stride_h;
@@ -799,7 +800,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #pragma unroll
         for (int i = 0; i < AE_N_ROWSCALES; i++)
 #if AE_NSPLIT > 1
-          p.partial_rs[(int64_t)i * p.batch * p.seqlen_q * p.heads_q * AE_NSPLIT + prow] = frs[i];
+          p.partial_rs[(int64_t)i * p.batch * p.seqlen_q * p.heads_q * n_split + prow] = frs[i];
 #else
           p.rowscale_out[i][((int64_t)b * p.heads_q + h) * p.seqlen_q + qrow[0]] = frs[i];
 #endif
@@ -889,7 +890,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
       asm volatile("" : "+v"(le));
       ae_lds_byte* os = lds + wave * REGION;
       const int64_t row0 = ((int64_t)b * p.seqlen_q + q0w) * p.heads_q + h;
-      const bool past = (int64_t)p.batch * p.seqlen_q * p.heads_q * (AE_NSPLIT * AE_DV * 4) <= 12 << 20;
+      const bool past = (int64_t)p.batch * p.seqlen_q * p.heads_q * (n_split * AE_DV * 4) <= 12 << 20;
 #pragma unroll
       for (int ps = 0; ps < NP; ps++) {
         ae_lds_byte* orow = os + (le & 31) * (CPR * 16);
@@ -909,7 +910,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
           for (int i = 0; i < 32 * CPR / 64; i++) {
             const int row = (i * 64 + le) / CPR, c = (i * 64 + le) % CPR;
             const ae_f32x4 w = *(const lds_f4*)(os + row * (CPR * 16) + ((c ^ (row & SW)) << 4));
-            ae_f32x4* at = (ae_f32x4*)(p.partial_o + ((row0 + (int64_t)row * p.heads_q) * AE_NSPLIT + split) * AE_DV + (ps * CPR + c) * 4);
+            ae_f32x4* at = (ae_f32x4*)(p.partial_o + ((row0 + (int64_t)row * p.heads_q) * n_split + split) * AE_DV + (ps * CPR + c) * 4);
             if (AE_EVEN_Q || q0w + row < p.seqlen_q) {
               if (decltype(past_tag)::value) __builtin_nontemporal_store(w, at);
               else *at = w;
@@ -925,10 +926,10 @@ void ae_prefill_kernel(const ae_attn_params p) {
       }
     }
     if (q_ok[rb] && hf == 0) {
-      const int64_t prow = ((((int64_t)b * p.seqlen_q + qrow[rb]) * p.heads_q + h) * AE_NSPLIT) + split;
+      const int64_t prow = ((((int64_t)b * p.seqlen_q + qrow[rb]) * p.heads_q + h) * n_split) + split;
 #pragma unroll
       for (int i = 0; i < AE_N_ROWSCALES; i++)
-        p.partial_rs[(int64_t)i * p.batch * p.seqlen_q * p.heads_q * AE_NSPLIT + prow] = frs[i];
+        p.partial_rs[(int64_t)i * p.batch * p.seqlen_q * p.heads_q * n_split + prow] = frs[i];
     }
 #elif AE_O_VIA_LDS
     {
@@ -990,6 +991,6 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #endif  // wide value heads
 }
 
-#if AE_NSPLIT > 1
+#ifdef AE_COMBINE_THREADS       // (a caller that wants both kernels in one module)
 #include "ae_combine.h"
 #endif

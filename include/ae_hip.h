@@ -143,7 +143,9 @@ typedef struct ae_tile_cfg {
                           AE_MERGE_LAST 1 (the workgroup that finishes last merges: no combine kernel, work
                           buffers with arrival counters, see ae_decode_fwd); else 0.  Prefill: 2 for kernels
                           compiled with AE_TAIL 1 (ae_attn_params.tail_slots), backward: 2 for AE_BWD_SPLIT 1
-                          (ae_attn_bwd_params.dkv_parts); else 0                                            */
+                          (ae_attn_bwd_params.dkv_parts); else 0.  Combine configurations: 1 when the kernel
+                          merges any number of splits up to block_n (places without a result count as row scales
+                          of -inf, which its combine() gives no weight), 0 when num_splits must equal block_n  */
   int32_t table_rows;  /* mask_mode 2: block-mask rows one q tile may span, the AE_TT_ROWS the kernel was
                           compiled with (1, 2, 4 or 8); 0 stands for the kernels' default of 8.
                           ae_prefill_bwd: 16 when the dk/dv kernel was compiled with AE_BWD_PAIRS 1 (its
@@ -268,12 +270,13 @@ int ae_launch(ae_kernel* k, const void* params, size_t params_bytes,
  *   (attn_gqa_decode_tl.py:150-151, 224-266). Every WAVE of the split kernel produces one partial,
  *   so its grid is (num_splits / (threads/64), ceil(Hq/Hkv / block_m)*Hkv, B); kv_per_split is the
  *   share of one partial and must be a multiple of block_n; combine_cfg->block_n is the number of
- *   splits the combine kernel was compiled for and must equal num_splits.  A split kernel compiled with
+ *   splits the combine kernel was compiled for: num_splits must equal it, or with combine_cfg->merge_in_wg = 1
+ *   not exceed it.  A split kernel compiled with
  *   AE_MERGE_IN_WG 1 is announced by cfg->merge_in_wg = 1: num_splits must then equal the waves of one
  *   workgroup, `combine` must be NULL (that workgroup merges its waves' partial results itself and writes
  *   out: one launch, no work buffers).  A split kernel compiled with AE_MERGE_LAST 1 is announced by
  *   cfg->merge_in_wg = 2: `combine` must be NULL, both work buffers and combine_cfg are required (block_n = the
- *   number of splits the kernel was compiled for, which must equal num_splits); the workgroup of a (batch,
+ *   number of splits the kernel was compiled for, as above); the workgroup of a (batch,
  *   kv head, head tile) that finishes last merges all partial results and writes out (one launch).  Its arrival
  *   counters are 32-bit integers BEHIND the row scales in partial_rs -- after max(1, n_rowscales) * batch * heads_q *
  *   num_splits floats, batch * ceil(Hq/Hkv / block_m) * Hkv of them -- which must be zero before the first launch
@@ -290,8 +293,8 @@ int ae_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params* p,
 /*
  * ae_prefill_split_fwd: split-KV attention for a FEW query tokens against a long KV ("MHA decode",
  *   the reference's generic decode template core/template/tl_template/attn/attn_decode_tl.py:47-205,
- *   selected in attn_engine/attn_engine.py:273-290).  The prefill kernel compiled with AE_NSPLIT =
- *   num_splits runs once per (q tile, head, batch, split) on kv_per_split positions (a multiple of
+ *   selected in attn_engine/attn_engine.py:273-290).  The prefill kernel compiled with AE_NSPLIT above 1
+ *   (num_splits is read at run time) runs once per (q tile, head, batch, split) on kv_per_split positions (a multiple of
  *   block_n) and writes fp32 partials ordered (batch, q position, head, split); the combine kernel then
  *   merges them with the user's combine() into `out`, which must be contiguous [B,Sq,Hq,DV], and writes
  *   the merged rowscales to rowscale_out as fp32 [B,Hq,Sq], the layout of ae_prefill_fwd.
@@ -306,7 +309,9 @@ int ae_prefill_split_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_par
  *   (cute_template_kvshared/flash_api.cpp:61-210). Every workgroup covers cfg->block_m query heads
  *   of one (batch, kv head, split); 1-D grid ordered so workgroups sharing a KV range run on one XCD.
  *   With num_splits == 1 the split kernel writes `out` / `rowscale_out` itself: no merge pass runs,
- *   `combine` may be NULL and the partial buffers are not touched.
+ *   `combine` may be NULL and the partial buffers are not touched.  A kernel compiled with AE_NSPLIT above 1
+ *   takes any num_splits above 1, one compiled with AE_NSPLIT 1 only num_splits == 1 (the other one's launch leaves `out`
+ *   unwritten or wrong, but strays nowhere).
  */
 int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params* p,
                       const ae_tile_cfg* cfg, const ae_tile_cfg* combine_cfg, void* stream);

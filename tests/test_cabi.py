@@ -251,6 +251,40 @@ def test_decode_merge_form_is_checked_before_any_launch():
     assert rc == 1 and "combine configuration is NULL" in msg, msg
 
 
+def test_a_merge_takes_no_more_splits_than_it_was_built_for():
+    """A combine configuration says how many splits its kernel merges: exactly block_n (merge_in_wg 0) or up to block_n
+    (1).  Every split launch holds num_splits to it; the refusals come before the kernel handles are used."""
+    lib = rt.lib()
+    fake = ctypes.c_void_p(8)
+    buf = ctypes.create_string_buffer(64)
+    addr = ctypes.addressof(buf)
+
+    def run(entry, num_splits, combine, **kw):
+        p = rt.AttnParams()
+        p.q = p.k = p.v = p.out = p.q2 = p.k2 = addr
+        p.partial_o = p.partial_rs = addr
+        p.batch, p.heads_q, p.heads_kv, p.seqlen_q, p.seqlen_kv = 2, 32, 8, 1, 256
+        p.num_splits, p.kv_per_split = num_splits, 64
+        c = rt.TileCfg(block_m=16, block_n=32, threads=256, lds_bytes=1024, head_dim=128, head_dim_v=128, elem_bytes=2,
+                       n_rowscales=0, mask_mode=0, merge_in_wg=0 if combine else 2)
+        cc = rt.TileCfg(block_m=1, threads=64, n_rowscales=1, **kw)
+        rc = entry(fake, fake if combine else None, ctypes.byref(p), ctypes.byref(c), ctypes.byref(cc), None)
+        return rc, lib.ae_last_error().decode()
+    for entry, combine in ((lib.ae_decode_fwd, True), (lib.ae_decode_fwd, False), (lib.ae_mla_decode_fwd, True),
+                           (lib.ae_prefill_split_fwd, True)):
+        for block_n in (4, 16):
+            rc, msg = run(entry, 8, combine, block_n=block_n)
+            assert rc == 1 and f"built for {block_n} splits, got 8" in msg, msg
+        rc, msg = run(entry, 12, combine, block_n=8, merge_in_wg=1)
+        assert rc == 1 and "built for up to 8 splits, got 12" in msg, msg
+        rc, msg = run(entry, 8, combine, block_n=8, merge_in_wg=2)
+        assert rc == 1 and "merge_in_wg=2 of a combine configuration" in msg, msg
+        if combine:                  # accepted counts go on to the next check (a row scale without a place to go)
+            for kw in ({"block_n": 8}, {"block_n": 16, "merge_in_wg": 1}):
+                rc, msg = run(entry, 8, combine, **kw)
+                assert rc == 1 and "rowscale_out[0] is NULL" in msg, msg
+
+
 def test_block_table_geometry_is_checked_before_any_launch():
     """mask_mode 2: both prefill launches refuse a table whose blocks do not fit the kernel's tiles - rows that
     neither divide nor are divided by the q tile, columns that are not whole kv tiles, and more table rows per q

@@ -664,3 +664,64 @@ def test_a_workgroup_whose_keys_are_all_masked_adds_nothing(cuda_device, monkeyp
         out = mod(q.cuda(), k.cuda(), v.cuda()).float().cpu()
         assert torch.isfinite(out).all() and (out - ref).abs().max().item() <= 2e-2
         assert (mod.final_rowscales["lse"].cpu().view(-1) - rlse.view(-1)).abs().max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("kind,n", [("gqa", 3), ("gqa", 8), ("gqa two launches", 5), ("mha", 5)])
+def test_an_infinite_value_stays_one_through_the_merge(cuda_device, monkeypatch, kind, n):
+    """The merge is built for a power of two of partial results; places beyond the launch's count must not turn an infinite
+    column (an infinite value, seen with positive weight) into no number, nor touch the others."""
+    print(f"case infinite value {kind} {n}", flush=True)
+    dtype, D, S = torch.float16, 128, 32 * 4 * 8
+    heads = 4 if kind == "mha" else 8
+    q, k, v = C.make_inputs(1, 1 if kind != "mha" else 3, S, heads, heads if kind == "mha" else 2, D, D, dtype, seed=n)
+    q *= 0.25
+    v[0, -1, :, 7] = float("inf")
+    if kind == "mha":
+        mod = _mha_decode_engine(1, heads, 3, S, D, dtype, C.OnlineSoftmax())
+        per = -(-(S // 32) // n) * 32
+        mod.attention.plan_splits = lambda *a: (n, per)
+    else:
+        monkeypatch.setenv("AE_DECODE_MERGE_LAST", "0" if "two" in kind else "1")
+        mod = _decode_engine(1, heads, 2, S, D, D, dtype, C.make_scale_score_mod(1 / math.sqrt(D)), C.OnlineSoftmax())
+        mod.attention._workgroups = lambda *a: n
+        assert mod.attention.plan_splits(1, heads, 2, S)[0] == 4 * n
+    out = mod(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+    v[0, -1, :, 7] = 0.0
+    ref, _ = R.softmax_attention(q, k, v, causal=False)
+    assert torch.isposinf(out[..., 7]).all()
+    ref[..., 7] = out[..., 7] = 0.0
+    assert (out - ref).abs().max().item() <= OUT_TOL
+
+
+def test_an_mla_split_kernel_takes_its_count_from_the_launch(cuda_device):
+    """One build of the split kernel, launched with 3 and with 5 splits through the C ABI's typed launch: the oracle's
+    result, and nothing written behind the work buffers that the count asks for."""
+    from core.runtime import hip_rt as rt
+    B, H, S, D, DV, dtype, scale = 2, 40, 700, 576, 512, torch.bfloat16, 1 / math.sqrt(192)
+    print("case mla split kernel, counts of the launch", flush=True)
+    q, q_pe, kv, k_pe = _mla_inputs(B, H, 1, S, DV, D - DV, dtype, seed=3)
+    ref, rlse = R.mla_decode(q[:, 0], q_pe[:, 0], kv, k_pe, scale=scale)
+    op = _mla_engine(B, H, 1, S, D, DV, dtype, scale).attention
+    dev = [t.cuda() for t in (q, q_pe, kv, k_pe)]
+    modules = set()
+    for n in (3, 5):
+        module, cfg, _ = op._variant(n, heads=32)
+        modules.add(module)
+        out = torch.zeros(B, 1, H, DV, dtype=dtype, device="cuda")
+        lse = torch.zeros(B, H, 1, device="cuda")
+        po, prs = (torch.full((size + 4096,), 7.0, device="cuda") for size in (B * H * n * DV, B * H * n))
+        p = rt.AttnParams()
+        p.q, p.q2, p.k, p.k2, p.v, p.out = (t.data_ptr() for t in (*dev[:2], *dev[2:], dev[2], out))
+        p.rowscale_out[0], p.partial_o, p.partial_rs = lse.data_ptr(), po.data_ptr(), prs.data_ptr()
+        for name, t in (("q", dev[0]), ("q2", dev[1]), ("k", dev[2]), ("k2", dev[3]), ("v", dev[2]), ("o", out)):
+            for i, ax in enumerate("bsh"):
+                setattr(p, f"{name}_stride_{ax}", t.stride(i))
+        p.batch, p.heads_q, p.heads_kv, p.seqlen_q, p.seqlen_kv = B, H, 1, 1, S
+        p.num_splits, p.kv_per_split = n, -(-22 // n) * 32
+        rt.mla_decode_fwd(module.kernel("ae_mla_decode_split_kernel"), op._merges.module(n).kernel("ae_decode_combine_kernel"), p,
+                          cfg, op._merges.cfg(n), torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert (out[:, 0].float().cpu() - ref).abs().max().item() <= OUT_TOL
+        assert (lse[:, :, 0].cpu() - rlse).abs().max().item() <= LSE_TOL
+        assert (po[-4096:] == 7.0).all() and (prs[-4096:] == 7.0).all()
+    assert len(modules) == 1

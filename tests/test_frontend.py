@@ -904,3 +904,51 @@ def test_causal_prefill_takes_the_faster_kernel(monkeypatch):
     assert not L.pipelined_pays(True, 64, 2867) and L.pipelined_pays(True, 16, 8192) and L.pipelined_pays(False, 16, 9131)
     monkeypatch.setenv("AE_PREFILL_KERNEL", "pipelined")
     assert template(2009)[1] == "ae_prefill_pipe.hip"
+
+
+def test_a_growing_cache_meets_few_kernels(monkeypatch):
+    """Every count of splits that a cache asks for while it grows a token a call runs in a few compiled kernels: the split
+    kernels take the count from the launch, merges are built for powers of two.  A combine() that is not the log-sum-exp merge
+    has one for its exact count."""
+    from core.lower.lower_decode import merge_capacity
+    from core.runtime import hip_rt as rt
+    built = set()
+
+    class Module:
+        def kernel_info(self):
+            return {"ae_decode_split_kernel": {}}
+
+    def compiled(template, headers, *a, **kw):
+        built.add((template, headers["ae_config.h"]))
+        return Module()
+    monkeypatch.setattr(rt, "compile_module", compiled)
+    monkeypatch.setattr(rt, "check_spills", lambda *a, **kw: None)
+    sm, f16 = C.make_scale_score_mod(0.1), torch.float16
+    for B, Hq, Hkv in ((1, 32, 8), (4, 32, 8), (19, 64, 8)):
+        op = AttentionEngine(_meta(B, Hq, Hkv, 1, 128, 128, 128, f16), CustomIO({}), sm, None, C.OnlineSoftmax()).attention
+        built.clear()
+        counts = {op.plan_splits(B, Hq, Hkv, S)[0] for S in range(128, 32769, 32)}
+        for n in counts:
+            _, cfg, ccfg, _ = op._variant(n, True, op._merge_mode(n))
+            assert n <= ccfg.block_n < 2 * n and (n == ccfg.block_n or ccfg.merge_in_wg == 1)
+        assert len(built) <= 6
+    for B, H in ((1, 128), (1, 16), (16, 64)):
+        op = AttentionEngine(_meta(B, H, 1, 1, 256, 576, 512, f16), CustomIO({}), sm, None, C.OnlineSoftmax(),
+                             kv_shared=True).attention
+        built.clear()
+        for S in range(256, 8193, 32):
+            heads, n, _ = op.plan(B, H, 1, S)
+            op._variant(n, False, heads)
+            if n > 1:
+                op._merges.module(n)
+        assert len([1 for t, _ in built if t == "ae_combine.hip"]) <= 6 and len(built) <= 6 + 6
+    op = AttentionEngine(_meta(5, 16, 16, 3, 512, 128, 128, f16), CustomIO({}), sm, None, C.OnlineSoftmax()).attention
+    built.clear()
+    for S in range(512, 16385, 32):
+        tiles = op.tiles_for(5, 16, 3, S)
+        n, _ = op.plan_splits(5, 16, 3, S, tiles)
+        op._variant(tiles, 0, 3, S, n)
+        if n > 1:
+            op._merges.module(n)
+    assert len(built) <= 2 * 2 + 6
+    assert [merge_capacity(n, True) for n in (2, 3, 4, 5, 8, 9, 64)] == [2, 4, 4, 8, 8, 16, 64] and merge_capacity(5, False) == 5
