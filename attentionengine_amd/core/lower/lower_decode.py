@@ -605,7 +605,6 @@ class MLADecodeOp(_SplitTuning):
         self._merges = Merges(self.D, self.DV, self.dtype, self.n_rowscales, self.functor_src,
                               merges_in_any_order(online_func, self.names), 128, allow_spills)
         self._variants = {}
-        self._plans = {}
         self.source = self.functor_src
         shape = [q_meta.shape[0], q_meta.shape[1], v_meta.shape[1], v_meta.shape[2]]
         if not any(isinstance(x, str) for x in shape):
@@ -615,22 +614,45 @@ class MLADecodeOp(_SplitTuning):
             if n_split > 1:
                 self.source = self._merges.config(n_split) + self.source
 
-    def _cost(self, heads, n_split, B, Hkv, group, Skv, live=1.0):
-        """Microseconds of a call of the wave-specialised kernel with ``heads`` query heads a workgroup, up to a constant:
-        one workgroup fits a CU, so it takes as many rounds as there are workgroups per CU, each a start and an end (f)
-        and its tiles (c); the cache cannot arrive faster than it is read (5.7 TB/s); partial results cost by the byte
-        (written, and read again by the merge), the merge by the split.  Fitted to 1073 timings - 40 shapes, batch 1 to
-        128, 16 / 64 / 128 heads, 300 to 8000 keys, bf16, every split count up to 64 -, where the choice by it is 0.2 %
-        slower on average than the best one measured, 2.8 % at most.  ``live``: the share of the splits that hold keys; those that
-        do are not spread evenly, so a round is full at 1/1.4 of the CUs (B8 H128, 2048 tokens at most, 16 heads: 5 splits,
-        192 live workgroups 19.4 us, 6, 224 22.9)."""
-        f, c = self.ROUND_COST[heads]
-        n_wg = math.ceil(B * Hkv * -(-group // heads) * n_split * (live if live == 1 or n_split == 1 else live * 1.4) - 1e-6)
-        tiles = -(-Skv // self.BLOCK_N)
-        body = -(-n_wg // self.target_workgroups) * (f + c * -(-tiles // n_split))
-        read = B * Hkv * Skv * 2e-6 * self.D * (live if live == 1 else 0.5) / 5.7
-        merge = 1.2 + 0.077 * n_split + 0.31 * B * Hkv * group * n_split * live * 4e-6 * self.DV if n_split > 1 else 0.0
-        return (body ** 4 + read ** 4) ** 0.25 + merge
+    @staticmethod
+    @functools.lru_cache(maxsize=1024)
+    def _cheapest(units, group, tiles, n_splits, cus, d, dv, paged):
+        """(query heads of a workgroup, splits) that a call of the wave-specialised kernel over ``units`` (batch entry, latent
+        head) of ``group`` heads and ``tiles`` kv tiles takes least time with; ``n_splits``: the candidates, first and last.
+
+        Its microseconds, up to a constant: one workgroup fits a CU, so it takes as many rounds as there are workgroups per
+        CU, each a start and an end (f) and its tiles (c); the cache cannot arrive faster than it is read (5.7 TB/s); partial
+        results cost by the byte (written, and read again by the merge), the merge by the split.  Fitted to 1073 timings - 40
+        shapes, batch 1 to 128, 16 / 64 / 128 heads, 300 to 8000 keys, bf16, every split count up to 64 -, where the choice by
+        it is 0.2 % slower on average than the best one measured, 2.8 % at most.  A paged cache counts half as if every entry
+        filled its table, half as if they were spread evenly up to that: ``live``, the share of the splits that hold keys;
+        those that do are not spread evenly, so a round is full at 1/1.4 of the CUs (B8 H128, 2048 tokens at most, 16 heads: 5
+        splits, 192 live workgroups 19.4 us, 6, 224 22.9).
+
+        Kept by the number of tiles: a latent cache that grows by a token a call asks anew every 32 calls (20 to 40 us; the 3 x 64
+        candidates evaluated at every length took 130 to 270, more than the choice gains)."""
+        read = units * tiles * MLADecodeOp.BLOCK_N * 2e-6 * d / 5.7
+        partial = 0.31 * units * group * 4e-6 * dv
+        splits = sorted({-(-tiles // -(-tiles // n)) for n in range(n_splits[0], n_splits[1] + 1)})      # (none without tiles)
+        best = None
+        for heads, (f, c) in MLADecodeOp.ROUND_COST.items():
+            if heads != 16 and group <= heads // 2:
+                continue
+            wgs = units * -(-group // heads)
+            for n in splits:
+                trip = f + c * -(-tiles // n)
+                us = ((-(-wgs * n // cus) * trip) ** 4 + read ** 4) ** 0.25
+                if n > 1:
+                    us += 1.2 + 0.077 * n + partial * n
+                if paged:
+                    live = (n + 1) / (2 * n)
+                    rounds = math.ceil(math.ceil(wgs * n * (live * 1.4 if n > 1 else 1.0) - 1e-6) / cus)
+                    us += ((rounds * trip) ** 4 + (read * (0.5 if n > 1 else 1.0)) ** 4) ** 0.25
+                    if n > 1:
+                        us += 1.2 + 0.077 * n + partial * n * live
+                if best is None or (us, -heads, n) < best:
+                    best = us, -heads, n
+        return -best[1], best[2]
 
     def plan(self, B, Hq, Hkv, Skv, page=None):
         """(query heads of a workgroup, number of splits, kv positions per split); with a paged cache a split spans at
@@ -645,33 +667,20 @@ class MLADecodeOp(_SplitTuning):
         tiles = -(-Skv // self.BLOCK_N)
         least = 1 if page is None else -(-Skv // ((self.PAGE_TABLE_ENTRIES - 2) * page))
         tuned = self._tuned.get((B, Hq, Hkv, Skv))
-        key = (B, Hq, Hkv, Skv, page, tuned, self.target_workgroups, self._wave_specialised())
-        got = self._plans.get(key)
-        if got is not None:
-            return got
 
-        def whole(n):                                        # no split without tiles
-            return -(-tiles // -(-tiles // n))
-        if not key[-1]:
+        def clamped(n):
+            return max(1, min(tiles, max(n, least)))
+        if self._wave_specialised():
+            span = (clamped(tuned),) * 2 if tuned else (clamped(least), clamped(self.MAX_SPLITS))
+            heads, n_split = self._cheapest(B * Hkv, group, tiles, span, self.target_workgroups, self.D, self.DV, page is not None)
+        else:
             # as many splits as fill the chip, but no more than the merge is worth: B1 H128 Skv4096 takes 24 us with
             # 16 splits, 92 us with the 128 that would occupy every CU
             base = B * Hkv * -(-group // self.HEADS_PER_WG)
-            want = tuned or min(-(-self.target_workgroups // base), self._balanced_splits(self.SPLIT_COEFF, Skv),
-                                self.MAX_SPLITS)
-            heads, n_split = self.HEADS_PER_WG, whole(max(1, min(tiles, max(want, least))))
-        else:
-            wants = [tuned] if tuned else range(least, max(least, self.MAX_SPLITS) + 1)
-            splits = sorted({whole(max(1, min(tiles, max(n, least)))) for n in wants})
-            def cost(h, n):
-                # a paged cache: half as if every entry filled its table, half as if they were spread evenly up to that
-                full = self._cost(h, n, B, Hkv, group, Skv)
-                return full if page is None else full + self._cost(h, n, B, Hkv, group, Skv, (n + 1) / (2 * n))
-            heads, n_split = min(((h, n) for h in self.ROUND_COST for n in splits if h == 16 or group > h // 2),
-                                 key=lambda x: (cost(*x), -x[0], x[1]))
-        if len(self._plans) >= 64:
-            self._plans.clear()
-        got = self._plans[key] = (heads, n_split, -(-tiles // n_split) * self.BLOCK_N)
-        return got
+            want = clamped(tuned or min(-(-self.target_workgroups // base), self._balanced_splits(self.SPLIT_COEFF, Skv),
+                                        self.MAX_SPLITS))
+            heads, n_split = self.HEADS_PER_WG, -(-tiles // -(-tiles // want))           # no split without tiles
+        return heads, n_split, -(-tiles // n_split) * self.BLOCK_N
 
     def plan_splits(self, B, Hq, Hkv, Skv, page=None):
         """(number of splits, kv positions per split) of ``plan``."""

@@ -952,3 +952,18 @@ def test_a_growing_cache_meets_few_kernels(monkeypatch):
             op._merges.module(n)
     assert len(built) <= 2 * 2 + 6
     assert [merge_capacity(n, True) for n in (2, 3, 4, 5, 8, 9, 64)] == [2, 4, 4, 8, 8, 16, 64] and merge_capacity(5, False) == 5
+
+
+def test_a_latent_cache_that_grows_is_planned_once_a_tile():
+    """A dense latent cache asks for a plan at every length: the splits are worked out once for all lengths of as many
+    tiles, and lengths that were asked for before stay known."""
+    from core.lower.lower_decode import MLADecodeOp
+    op = AttentionEngine(_meta(3, 128, 1, 1, 256, 576, 512, torch.bfloat16), CustomIO({}), C.make_scale_score_mod(0.1), None,
+                         C.OnlineSoftmax(), kv_shared=True).attention
+    MLADecodeOp._cheapest.cache_clear()
+    plans = [op.plan(3, 128, 1, S) for S in range(4001, 4641)]
+    assert MLADecodeOp._cheapest.cache_info().misses == 21 and len(set(plans)) > 1
+    assert [op.plan(3, 128, 1, S) for S in range(4001, 4641)] == plans
+    assert MLADecodeOp._cheapest.cache_info().misses == 21
+    assert all(n * per >= S > (n - 1) * per for S, (_, n, per) in zip(range(4001, 4641), plans))
+    assert op.plan(3, 128, 1, 4000, 64)[1] * op.plan(3, 128, 1, 4000, 64)[2] >= 4000         # (a paged call has its own)
