@@ -962,8 +962,8 @@ def test_a_latent_cache_that_grows_is_planned_once_a_tile():
                          C.OnlineSoftmax(), kv_shared=True).attention
     MLADecodeOp._cheapest.cache_clear()
     plans = [op.plan(3, 128, 1, S) for S in range(4001, 4641)]
-    assert MLADecodeOp._cheapest.cache_info().misses == 21 and len(set(plans)) > 1
+    assert MLADecodeOp._cheapest.cache_info().misses == 20 and len(set(plans)) > 1
     assert [op.plan(3, 128, 1, S) for S in range(4001, 4641)] == plans
-    assert MLADecodeOp._cheapest.cache_info().misses == 21
+    assert MLADecodeOp._cheapest.cache_info().misses == 20
     assert all(n * per >= S > (n - 1) * per for S, (_, n, per) in zip(range(4001, 4641), plans))
     assert op.plan(3, 128, 1, 4000, 64)[1] * op.plan(3, 128, 1, 4000, 64)[2] >= 4000         # (a paged call has its own)
