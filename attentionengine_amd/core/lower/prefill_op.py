@@ -133,6 +133,10 @@ class PrefillOp:
         # core/lower/lower_decode.py:287-313 of the reference): the kv axis is shared out over several
         # workgroups per q tile and the partial results are merged with the user's combine().
         self.target_workgroups = int(target_workgroups)
+        # Bytes of work memory that one call may take for launches that share tiles out over several workgroups where the chip
+        # would idle (_tail, PrefillBwdOp.dkv_parts): allocated per call, given back with it.  None: 128 MB in the forward,
+        # 256 MB in the backward.  0: no tile is shared out.
+        self._work_limit = None
         if self.split_kv:
             if self.tiles.template == "ae_prefill_simple.hip" or max(self.D, self.DV) > 128:
                 raise NotImplementedError("split-KV prefill needs head dims 64 or 128")
@@ -186,6 +190,18 @@ class PrefillOp:
                 if not self._gives_way_to_the_generic_kernel():
                     raise
                 self._compile_declared_shape(B, H, Sq, Skv, infer_mask, mask_mod)
+
+    @property
+    def work_limit(self):
+        return self._work_limit
+
+    @work_limit.setter
+    def work_limit(self, n):
+        self._work_limit = n
+        self._host.clear()         # (plans made under the old one)
+
+    def work_limit_mb(self, default):
+        return default if self._work_limit is None else self._work_limit * 1e-6
 
     def _gives_way_to_the_generic_kernel(self) -> bool:
         """A build of the software-pipelined kernel that spills registers is refused (hip_rt.check_spills).  Where
@@ -333,9 +349,9 @@ class PrefillOp:
         best, op, times = tuner.pick(
             cands, lambda t: self if t == self.tiles else PrefillOp(*args, **kw, tiles=t), run, log)
         if op is not self:
-            keep = (self._ctor, self._tune_file, self._tune_keys, self._tune_bwd, mine)
+            keep = (self._ctor, self._tune_file, self._tune_keys, self._tune_bwd, self._work_limit, mine)
             self.__dict__.update(op.__dict__)
-            self._ctor, self._tune_file, self._tune_keys, self._tune_bwd, self.block_mask = keep
+            self._ctor, self._tune_file, self._tune_keys, self._tune_bwd, self._work_limit, self.block_mask = keep
             self._bwd = None        # the backward reads this operator's mask plans: built again on demand
         self._tune_pending = False
         self.tune_times = {tuple(tuner.encode_tiles(cands[i])): ms for i, ms in times.items()}
@@ -435,7 +451,7 @@ class PrefillOp:
 
     @classmethod
     @functools.lru_cache(maxsize=1024)
-    def _tail_plan(cls, slots, kv_tiles, cus_per_xcd, width):
+    def _tail_plan(cls, slots, kv_tiles, cus_per_xcd, width, limit_mb=128):
         """(q tiles of an XCD, workgroups of each, kv tiles of a workgroup) that share their kv axes in an unmasked launch of the
         pipelined kernel with ``slots`` q tiles an XCD (AE_TAIL of ae_prefill_pipe.hip), or None: what is left over when the
         CUs have been filled as often as possible would take a round of its own.  A workgroup takes 7 us to start and end
@@ -451,7 +467,7 @@ class PrefillOp:
         best = None
         for n in range(2, cls.MAX_TAIL_PARTS + 1):
             per = -(-kv_tiles // n)
-            if -(-kv_tiles // per) != n or 8 * rest * n * 0.136 * width > 128:      # (MB of partial results)
+            if -(-kv_tiles // per) != n or 8 * rest * n * 0.136 * width > limit_mb:      # (MB of partial results)
                 continue
             us = -(-rest * n // cus_per_xcd) * (start + trip * per) + 3.0 + 1.2 * n * width
             if best is None or us < best[0]:
@@ -465,7 +481,7 @@ class PrefillOp:
                 or self._clock_stamps(tiles)):
             return None
         return self._tail_plan(-(-Sq // tiles.block_m) * -(-(B * H) // 8), -(-Skv // tiles.block_n),
-                               L._MI355X_CUS // 8, (self.D + self.DV) / 256)
+                               L._MI355X_CUS // 8, (self.D + self.DV) / 256, self.work_limit_mb(128))
 
     def _kv_custom_scratch(self, tiles) -> int:
         """LDS a launch needs beyond its K / V stages: the direct-to-LDS kernel redistributes the tiles of custom

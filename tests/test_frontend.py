@@ -967,3 +967,37 @@ def test_a_latent_cache_that_grows_is_planned_once_a_tile():
     assert MLADecodeOp._cheapest.cache_info().misses == 20
     assert all(n * per >= S > (n - 1) * per for S, (_, n, per) in zip(range(4001, 4641), plans))
     assert op.plan(3, 128, 1, 4000, 64)[1] * op.plan(3, 128, 1, 4000, 64)[2] >= 4000         # (a paged call has its own)
+
+
+def test_the_caller_limits_the_work_memory_of_shared_tiles():
+    """``work_limit`` bounds what a call allocates for tiles that several workgroups share, in the forward and in the
+    backward: fewer shares, or none; plans made under another limit are dropped."""
+    from core.lower.lower import pipelined_tiles
+    meta = _meta(2, 32, 8, 2048, 2048, 128, 128, torch.float16)
+    op = AttentionEngine(meta, CustomIO({}), C.make_scale_score_mod(0.1), C.causal_mask, C.OnlineSoftmax())._op
+    bwd, B, S = op.backward_op(), 2, 1000
+
+    def mb(parts):
+        return -(-S // 128) * B * 8 * parts * 128 * 256 * 4e-6 if parts > 1 else 0.0
+    free = bwd.dkv_parts(B, 32, 8, S, S, True)
+    assert free > 2 and op.work_limit is None
+    limits = [int(mb(2) * 1e6) + 1, 0]
+    for limit in limits:
+        op.work_limit = limit
+        got = bwd.dkv_parts(B, 32, 8, S, S, True)
+        assert got == (2 if limit else 1) and mb(got) * 1e6 <= limit
+    full = AttentionEngine(_meta(3, 8, 8, 2944, 2944, 128, 128, torch.float16), CustomIO({}), C.make_scale_score_mod(0.1), None,
+                           C.OnlineSoftmax())._op
+    tiles = pipelined_tiles(128, 128)
+    rest, n, _ = full._tail(3, 8, 2944, 2944, tiles, 0, 1)
+    cleared = []
+
+    class Host:
+        def clear(self):
+            cleared.append(1)
+    full._host = Host()
+    full.work_limit = int(8 * rest * (n - 1) * 0.14e6)
+    fewer = full._tail(3, 8, 2944, 2944, tiles, 0, 1)
+    assert fewer is None or fewer[1] < n
+    full.work_limit = 0
+    assert full._tail(3, 8, 2944, 2944, tiles, 0, 1) is None and len(cleared) == 2
