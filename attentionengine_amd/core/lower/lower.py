@@ -770,7 +770,8 @@ def _wide_key_group_tiles(wgs, batch_heads: int, seqlen_kv: int):
     hold them; two groups of 128 rows while few heads leave the longest tile behind its CU's share of all.  Measured
     (us, default tiles -> these): B2 H16 S485 16.7 -> 13.1 and B1 H16 S1428 37.1 -> 26.6 (64 x 4 x 32), B2 H16 S1014
     29.3 -> 24.5 (64 x 2 x 32), B1 H16 S2979 79.3 -> 62.6 and S3772 109 -> 92 (128 x 2 x 64); but B3 H16 S986 31.8 -> 32.6,
-    B1 H128 S433 19.4 -> 25.2, B1 H16 S5334 182 -> 184 with the best of them."""
+    B1 H128 S433 19.4 -> 25.2, B1 H16 S5334 182 -> 184 with the best of them.  On 40 shapes beside those (batch 1 to 4, 16 to
+    128 heads, 256 to 8192 positions) the choice is 0.03 % off the best of the four on average, 1.1 % at most."""
     if seqlen_kv >= 440 and (wgs(64) <= _MI355X_CUS or (wgs(64) <= 2 * _MI355X_CUS and batch_heads <= 18)):
         return PrefillTiles(n_waves=2, kv_groups=4, block_n=32)
     if wgs(64) <= 2 * _MI355X_CUS and (seqlen_kv >= 320 or wgs(64) <= _MI355X_CUS):
@@ -785,7 +786,9 @@ def short_key_tiles_pay(batch_heads: int, seqlen_q: int, seqlen_kv: int) -> bool
     that three workgroups share a CU instead of two, and less padding at the end of the keys, for 12 % more time a key.
     One round of three where there were two of two (B24 H32 S73 bf16 16.8 -> 13.8 us, B18 H8 S481 32.6 -> 30.6, B17 H8 S387 29.4 ->
     26.5), or padding saved over several rounds (B21 H32 S216 fp16 42.7 -> 34.7, B27 H32 S266 bf16 72.1 -> 63.3; B5 H32
-    S1328, which has none, 158.6 -> 160.4), or most of it in one round (B16 H32 S85 10.7 -> 10.3)."""
+    S1328, which has none, 158.6 -> 160.4), or most of it in one round (B16 H32 S85 10.7 -> 10.3).  On 28 shapes beside those it
+    is 2.1 % off the better of the two on average: it takes nothing that is more than 2 % slower, but leaves some (B28 H32 S186
+    fp16 41.3 us, 36.7 with 32 keys)."""
     wgs = batch_heads * -(-seqlen_q // 128)
     padding = 2 * -(-seqlen_kv // 64) / -(-seqlen_kv // 32)
     if wgs <= 2 * _MI355X_CUS:
@@ -795,7 +798,9 @@ def short_key_tiles_pay(batch_heads: int, seqlen_q: int, seqlen_kv: int) -> bool
 
 def window_group_tiles(batch_heads: int, seqlen_q: int):
     """Tiles of a sliding window at head dim 64 whose 64-row tiles no longer all find a place as four groups of waves, while
-    the 128-row ones do not fill the chip twice; None elsewhere."""
+    the 128-row ones do not fill the chip twice; None elsewhere.  On 50 shapes beside those that it was made from (batch 1
+    to 4, 16 and 32 heads, 512 to 8192 positions, windows of 64 to 1024) the tiles that this and the other rules choose are
+    2.3 % off the best of six on average, 23 % at most (B1 H16 S1216 of 166 bf16: four groups 9.0 us, two 7.3)."""
     if batch_heads * -(-seqlen_q // 64) > 7 * _MI355X_CUS // 4 and batch_heads * -(-seqlen_q // 128) <= 15 * _MI355X_CUS // 8:
         return PrefillTiles(n_waves=2, kv_groups=2, block_n=32)
     return None

@@ -305,14 +305,22 @@ class GQADecodeOp(_SplitTuning):
         XCDs idle (B19 Hq64 Hkv8 Skv2204: 8 workgroups 40.8 us, 7 30.8).
 
         Fitted to 1819 timings (216 shapes of fp16 and bf16, batch 1 to 128, 128 to 32768 keys, D128), where the choice is
-        0.4 % slower than the best one on average, 7 % at most.  Against the power of two that fills the CUs, which was
+        0.4 % slower than the best one on average, 7 % at most; at D256 (25 shapes) 0.1 and 2 %.  Head dim 64 has constants
+        of its own: three workgroups share a CU, and starting and ending them is what more of them cost (fitted to 114 shapes; on 37 others the
+        choice is 1.2 % off the best on average, 11 % at most, and by the constants of D128 B48 Hq16 Hkv2 Skv871 took 10.3 us
+        instead of 7.5).  Against the power of two that fills the CUs, which was
         the rule before: B67 Hq32 Hkv4 Skv13634 471 -> 346 us, B71 Skv3876 138 -> 113, B65 Hq16 Hkv2 Skv2082 32.6 -> 25.5,
         B19 Hq64 Hkv8 Skv3372 54 -> 42."""
         kib = 16 * width                                     # of keys and values in a wave's tile
         cached = units * tiles * kib <= 300e3                # (of 256 MB: some of it still hits a little beyond)
-        alone, rate = (1.4, 8.1) if cached else (1.7, 6.2)
-        alone *= 0.2 + 0.8 * width if width <= 1 else 1 + 1.7 * (width - 1)
-        shared = alone * (2.15 if width <= 1 else 2.75)      # (wider rows: one workgroup fits a CU)
+        if width <= 0.5:
+            per_cu, power, fixed, ends, gap, merge = 3, 1.41, 1.7, 0.98, 0.0, (1.18, 0.068)
+            alone, rate, share = 0.68 if cached else 0.65, 12.3 if cached else 7.3, 0.632
+        else:
+            per_cu, power, fixed, ends, gap, merge = 2, 4, 3.6, 0.0, 0.45, (0.8, 0.08)
+            alone, rate = (1.4, 8.1) if cached else (1.7, 6.2)
+            alone *= 0.2 + 0.8 * width if width <= 1 else 1 + 1.7 * (width - 1)
+            share = alone * (2.15 if width <= 1 else 2.75) / 2       # (wider rows: one workgroup fits a CU)
         best = []
         for x in GQADecodeOp.GROUPED_WGS_PER_KV_HEAD:
             if x > most:
@@ -320,15 +328,16 @@ class GQADecodeOp(_SplitTuning):
             trips = -(-tiles // (GQADecodeOp.N_WAVES * x))
             live = -(-tiles // (GQADecodeOp.N_WAVES * trips))
             xcds = math.gcd(x, 8)
-            rounds, rest = divmod(units * xcds * -(-live // xcds), 2 * cus)
+            rounds, rest = divmod(units * xcds * -(-live // xcds), per_cu * cus)
 
             def trip(n):
-                return (max(alone, shared if n > cus else 0.0) ** 4 + (n * 4096e-6 * kib / rate) ** 4) ** 0.25
-            full, last = trip(2 * cus), trip(rest) if rest else 0.0
+                here = -(-n // cus)
+                return (max(alone, share * here if here > 1 else 0.0) ** power + (n * 4096e-6 * kib / rate) ** power) ** (1 / power)
+            full, last = trip(per_cu * cus), trip(rest) if rest else 0.0
             us = full if rounds else last
             if rounds + (rest > 0) > 1:
-                us = 0.5 * (rounds * full + last + (rounds + rest / (2 * cus)) * full + 0.45)
-            best.append((3.6 + us * trips + (0.8 + 0.08 * x if x > 1 else 0.0), x))
+                us = 0.5 * (rounds * full + last + (rounds + rest / (per_cu * cus)) * full + gap)
+            best.append((fixed + us * trips + ends * max(1.0, units * x / cus) + (merge[0] + merge[1] * x if x > 1 else 0.0), x))
         least = min(best)[0]
         return next(x for us, x in best if us <= 1.01 * least)
 

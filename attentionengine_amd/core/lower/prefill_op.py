@@ -9,6 +9,7 @@ rowscales, launches on torch's current stream, returns ``o``.
 from __future__ import annotations
 
 import functools
+import math
 import os
 from dataclasses import astuple
 
@@ -398,6 +399,8 @@ class PrefillOp:
 
     # microseconds of a workgroup's start and end, and of a trip over its kv groups' next tiles, by the rows of its q tile
     SPLIT_COST = {32: (3.0, 0.92), 64: (1.8, 0.66), 128: (1.3, 0.91), 256: (5.2, 1.39)}
+    # head dim 64: (start and end, trip, what a trip takes of each workgroup that shares the CU, workgroups a CU holds)
+    SPLIT_COST_64 = {32: (2.04, 0.63, 0.44, 2), 64: (2.25, 0.53, 0.31, 4), 128: (1.66, 0.77, 0.57, 4), 256: (4.7, 1.0, 0.0, 2)}
 
     @classmethod
     @functools.lru_cache(maxsize=1024)
@@ -409,7 +412,14 @@ class PrefillOp:
         and the partial results: written and merged.  Fitted to 1926 timings (150 shapes, batch 1 to 8, 8 to 32 heads, 1
         to 256 rows, 512 to 16384 keys, D128): 1 % above the best count on average.  Measured, one split for every CU ->
         this: B7 H16 Sq31 Skv522 17.6 -> 9.2 us, B6 H16 Sq25 Skv1118 22.0 -> 15.3, B6 H8 Sq78 Skv2854 26.1 -> 21.6,
-        B3 H32 Sq2 Skv9161 109 -> 88.  ``width``: bytes of a key and a value row in units of 512."""
+        B3 H32 Sq2 Skv9161 109 -> 88.  ``width``: bytes of a key and a value row in units of 512.
+
+        At head dim 64 two to four workgroups fit a CU, and a launch of two on some CUs is no second round: with the costs of
+        D128 17 of 71 choices were slower than one split for every CU (B7 H32 Sq47 Skv5777 70.5 -> 93.9 us).  Its own costs
+        are fitted to 130 shapes; where the count is chosen by them, 40 others take 0.89 of the time on average, 1.04 at most
+        (that one 63.5 us)."""
+        if width <= 0.5:
+            return cls._cheapest_splits_64(wgs, rows, kv_tiles, block_m, block_n, kv_groups, cus, heads)
         start, trip = cls.SPLIT_COST[block_m]
         read = heads * kv_tiles * block_n * 512e-6 * width
         read /= 8.4 if read <= 300 else 6.2
@@ -428,6 +438,28 @@ class PrefillOp:
             best.append((2.3 + (body ** 1.85 + read ** 1.85) ** (1 / 1.85) + merge, per))
         least = min(best)[0]
         return next(per for us, per in best if us <= 1.01 * least)
+
+    @classmethod
+    def _cheapest_splits_64(cls, wgs, rows, kv_tiles, block_m, block_n, kv_groups, cus, heads):
+        start, trip, share, fit = cls.SPLIT_COST_64[block_m]
+        read = heads * kv_tiles * block_n * 256e-6
+        read /= 7.1 if read <= 300 else 5.3
+        best = []
+        for x in range(1, min(64, kv_tiles) + 1):
+            per = -(-kv_tiles // x)
+            if -(-kv_tiles // per) != x:
+                continue
+            trips, a_cu = -(-per // kv_groups), wgs * x / cus
+            if a_cu > 8 and x > 1:
+                break
+            full = start + max(trip, share * fit) * trips                  # a round of as many workgroups as a CU holds
+            rounds, rest = divmod(a_cu, fit)
+            body = rounds * full + (start + max(trip, share * math.ceil(rest)) * trips if rest > 0 else 0.0)
+            if a_cu > fit:
+                body = 0.5 * (body + a_cu / fit * full) + 0.3 * start
+            merge = 3.5 + 0.061 * x + 0.315 * rows * x * 256e-6 if x > 1 else 0.0
+            best.append((1.2 + (body ** 2.46 + read ** 2.46) ** (1 / 2.46) + merge, per))
+        return min(best)[1]
 
     def plan_splits(self, B, Hq, Sq, Skv, tiles=None):
         """(number of KV splits, kv positions per split): a workgroup for every CU of the chip (more splits cost
@@ -458,7 +490,9 @@ class PrefillOp:
         and 2.0 us a kv tile (D128); shares are few (the last workgroup reads all of them, about 1.2 us each), and taken
         where the call gains 6 % by this count - what it says is 3 % turned out between -7 and +2.  Measured: softmax B3 H8
         S2944 D128 fp16 162 -> 117 us, bf16 174 -> 120, B1 H32 S2560 sigmoid bf16 155 -> 115 (40 tiles an XCD), B1 H40 S3584
-        (70) 301 -> 250, D64 B2 H16 S4200 231 -> 178, sigmoid fp16 B3 H16 S1325 83 -> 68; 56 of 64 tiles: 232 -> 230."""
+        (70) 301 -> 250, D64 B2 H16 S4200 231 -> 178, sigmoid fp16 B3 H16 S1325 83 -> 68; 56 of 64 tiles: 232 -> 230.  On 49
+        shapes beside those the choice is 0.5 % off the best count on average (B2 H8 S2293 bf16, 18 tiles an XCD: 71.7 us, 64.2
+        unshared; else 3 % at most), at D64 on 48 shapes 0.4 %, 7 at most."""
         rounds, rest = divmod(slots, cus_per_xcd)
         if not rest:
             return None

@@ -1001,3 +1001,21 @@ def test_the_caller_limits_the_work_memory_of_shared_tiles():
     assert fewer is None or fewer[1] < n
     full.work_limit = 0
     assert full._tail(3, 8, 2944, 2944, tiles, 0, 1) is None and len(cleared) == 2
+
+
+def test_plans_at_head_dim_64_have_costs_of_their_own():
+    """Narrow rows: several workgroups fit a CU, so one split more than a CU each is no second round (split prefill), and a
+    short cache is not cut into a workgroup a tile (GQA decode); splits cover the cache with none empty."""
+    f16, sm = torch.float16, C.make_scale_score_mod(0.1)
+    op = AttentionEngine(_meta(7, 32, 32, 47, 5777, 64, 64, f16), CustomIO({}), sm, None, C.OnlineSoftmax())._op
+    assert op.split_kv and op.plan_splits(7, 32, 47, 5777)[0] > 1
+    for B, H, Sq in ((1, 8, 1), (5, 16, 40), (7, 32, 130), (3, 16, 250)):
+        tiles = op.tiles_for(B, H, Sq, 5000)
+        for Skv in (1, 100, 522, 16001):
+            n, per = op.plan_splits(B, H, Sq, Skv, tiles)
+            assert per % tiles.block_n == 0 and n * per >= Skv > (n - 1) * per
+    gqa = AttentionEngine(_meta(48, 16, 2, 1, 871, 64, 64, f16), CustomIO({}), sm, None, C.OnlineSoftmax()).attention
+    assert gqa.plan_splits(48, 16, 2, 871)[0] <= 2 * gqa.N_WAVES
+    for B, Skv in ((1, 128), (3, 5000), (128, 16000)):
+        n, per = gqa.plan_splits(B, 16, 2, Skv)
+        assert n // gqa.N_WAVES in gqa.GROUPED_WGS_PER_KV_HEAD and n * per >= Skv
