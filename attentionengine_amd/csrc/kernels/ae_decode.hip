@@ -400,6 +400,10 @@ void ae_decode_split_kernel(const ae_attn_params p) {
     // Every wave waits until its stores above have been acknowledged (stores count in vmcnt; the barrier alone
     // does not wait for them: a workgroup-scope release on this target orders only what the waves of one CU see),
     // then the workgroup meets and counts itself in: no partial result is still travelling when the counter moves.
+    // (where this thread starts to merge, should the workgroup be the last, is worked out while the stores are on their way)
+    constexpr int kQuads = AE_DV / 4;
+    int rs_at = tid / kQuads * n_part, po_at = (rs_at * AE_DV + tid % kQuads * 4) * 4;
+    asm volatile("" : "+v"(rs_at), "+v"(po_at));
     __builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0), the other counters left alone
     __syncthreads();                   // (every wave is also past its last tile: the V tile regions are free)
     __attribute__((address_space(3))) int* flag = (__attribute__((address_space(3))) int*)ae_smem;
@@ -424,27 +428,25 @@ void ae_decode_split_kernel(const ae_attn_params p) {
     auto merge = [&](auto places) AE_LAMBDA {
       constexpr bool kFixed = decltype(places)::value > 0;
       constexpr int N = kFixed ? decltype(places)::value : AE_NSPLIT;
-      for (int idx = tid; idx < tile_heads * (AE_DV / 4); idx += AE_NT) {
-        const int hl = idx / (AE_DV / 4), dv = (idx % (AE_DV / 4)) * 4;
-        const int hq2 = hk * group + ht * 16 + hl;
+      for (int idx = tid; idx < tile_heads * kQuads;
+           idx += AE_NT, rs_at = idx / kQuads * n_part, po_at = (rs_at * AE_DV + idx % kQuads * 4) * 4) {
         // (the count is compared as a vector register, a copy for each use: 64 scalar conditions, or the results of as many
         // vector ones kept from one use to the next, do not fit the scalar registers)
         int n_row = n_part, n_load = n_part, n_weight = n_part;
         if (!kFixed) asm volatile("" : "+v"(n_row), "+v"(n_load), "+v"(n_weight));
-        const int row_at = hl * (kFixed ? N : n_part);
         float rs[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1][AE_NSPLIT];
 #pragma unroll
         for (int i = 0; i < AE_N_ROWSCALES; i++)
 #pragma unroll
           for (int k = 0; k < AE_NSPLIT; k++)
             rs[i][k] = k >= N ? AE_NEG_INF
-                              : __hip_atomic_load(p.partial_rs + (int64_t)i * p.batch * p.heads_q * n_part + tile_row0 + row_at +
+                              : __hip_atomic_load(p.partial_rs + (int64_t)i * p.batch * p.heads_q * n_part + tile_row0 + rs_at +
                                                       (kFixed || k < n_row ? k : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         constexpr int G = N < 16 ? N : 16;     // partial results in flight at a time
         ae_f32x4 val[G];
         auto load_part = [&](int k) AE_LAMBDA -> ae_f32x4 {
           return __builtin_bit_cast(ae_f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-              po_buf, kFixed || k < n_load ? ((row_at + k) * AE_DV + dv) * 4 : -1, 0, kDeviceScope));
+              po_buf, kFixed || k < n_load ? po_at + k * (AE_DV * 4) : -1, 0, kDeviceScope));
         };
 #pragma unroll
         for (int i = 0; i < G; i++) val[i] = load_part(i);
@@ -473,7 +475,10 @@ void ae_decode_split_kernel(const ae_attn_params p) {
               for (int r = 0; r < 4; r++) acc[r] += val[i][r] * w[k0 + i];
             }
         }
-        ae_elem* orow = (ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)hq2 * p.o_stride_h + dv;
+        const int hq2 = hk * group + ht * 16 + idx / kQuads, dv = idx % kQuads * 4;
+        int b_out = b;
+        asm volatile("" : "+s"(b_out));       // (the address is worked out here, behind the requests, not in front of the loop)
+        ae_elem* orow = (ae_elem*)p.out + (int64_t)b_out * p.o_stride_b + (int64_t)hq2 * p.o_stride_h + dv;
 #pragma unroll
         for (int r = 0; r < 4; r++) orow[r] = (ae_elem)acc[r];
         if (dv == 0) {
@@ -483,7 +488,9 @@ void ae_decode_split_kernel(const ae_attn_params p) {
         }
       }
     };
-    if (__builtin_expect(n_part == AE_NSPLIT, 1)) merge(ae_const_int<AE_NSPLIT>());
+    int n_first = n_part;
+    asm("" : "+s"(n_first));             // (else the comparisons become a search whose first case is another one)
+    if (__builtin_expect(n_first == AE_NSPLIT, 1)) merge(ae_const_int<AE_NSPLIT>());
 #if AE_NSPLIT % 4 == 0
     else if (n_part == AE_NSPLIT / 4 * 3) merge(ae_const_int<AE_NSPLIT / 4 * 3>());
 #endif
