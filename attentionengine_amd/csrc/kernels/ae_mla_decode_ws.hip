@@ -28,7 +28,8 @@
 // AE_HPW (heads per workgroup): 64 is the form above.  32 and 16 are for launches that 64-head workgroups spread thin -
 // few query heads, or so few sequences that the kv axis is split over many workgroups and every one of them pays for the
 // fp32 partial results of 64 heads.  A trip of the 64-head form is one score wave's instruction stream (36 MFMAs, 36
-// fragment reads, the softmax of 16 scores a lane: 0.92 us); here 16 heads and 16 of the tile's 32 keys make up a score
+// fragment reads, the softmax of 16 scores a lane: 0.81 us in split launches of a small batch, 1.1 where every CU is busy
+// and the clock at the power cap); here 16 heads and 16 of the tile's 32 keys make up a score
 // wave's share (v_mfma_f32_16x16x32: 18 MFMAs, 18 reads, 4 scores a lane), two waves per 16 heads, which exchange their
 // maxima through LDS at the end of a trip and so keep one reference.  The value waves take 16x16x32 too: 128 columns x
 // 16 or 32 heads.  Per head the tile is fetched and read two or four times as often as with 64 heads, which is why the
