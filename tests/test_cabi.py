@@ -432,6 +432,21 @@ def test_code_object_cache_is_keyed_by_content(tmp_path, monkeypatch):
     rt._modules.clear()
 
 
+def test_a_module_may_hold_the_split_and_the_merge_kernel():
+    """A configuration that defines AE_COMBINE_THREADS gets the merge kernel in the split kernel's own module (callers of
+    the C ABI that fetch both from one); without it, and from ae_combine.hip, each is alone."""
+    import __graft_entry__ as G
+    sets = G.representative_headers()
+    alone = [h for t, h in sets if t == "ae_combine.hip"]
+    assert set(rt.compile_module("ae_combine.hip", alone[0]).kernel_info()) == {"ae_decode_combine_kernel"}
+    for template, name in (("ae_decode.hip", "ae_decode_split_kernel"), ("ae_mla_decode.hip", "ae_mla_decode_split_kernel"),
+                           ("ae_mla_decode_ws.hip", "ae_mla_decode_split_kernel")):
+        headers = [h for t, h in sets if t == template][0]
+        assert set(rt.compile_module(template, headers).kernel_info()) == {name}
+        both = {**headers, "ae_config.h": headers["ae_config.h"] + "#define AE_COMBINE_THREADS 128\n"}
+        assert set(rt.compile_module(template, both).kernel_info()) == {name, "ae_decode_combine_kernel"}
+
+
 def test_benchmarked_kernels_do_not_spill_registers():
     """The code objects hipRTC builds for the benchmark configurations (and the backward of the causal one) keep
     every value in registers: a kernel that spills pays for it with scratch-memory traffic in every workgroup, and
