@@ -702,10 +702,15 @@ class MLADecodeOp(_SplitTuning):
                 and self.D // 16 >= 27      # its softmax is spread over 27 of the D/16 k-steps
                 and os.environ.get("AE_MLA_KERNEL", "") != "generic")
 
+    def _stamped(self, n_split):
+        """AE_CLOCK_STAMPS=1 (a measurement switch, read by ``bench.py --mfma-probe``): single-split launches of the
+        wave-specialised kernel report the shader clock their workgroups ran at (``self.clock_stamps``)."""
+        return n_split == 1 and os.environ.get("AE_CLOCK_STAMPS", "") == "1" and self._wave_specialised()
+
     def _variant(self, n_split, paged=False, heads=64):
         """(module, cfg, config source) of the split kernel, one for every count of splits above 1.  ``heads``: query heads of a
         workgroup (AE_HPW of the wave-specialised kernel)."""
-        key = (n_split > 1, paged, heads)
+        key = (n_split > 1, paged, heads, self._stamped(n_split))
         v = self._variants.get(key)
         if v is None:
             ws = self._wave_specialised()
@@ -713,10 +718,7 @@ class MLADecodeOp(_SplitTuning):
             cfg_src = render_mla_config(self.DV, self.D2, self.DV, self.dtype, self.BLOCK_N, self.K_PAD,
                                         self.n_rowscales, self.functors.o_scale_one, 2 if n_split > 1 else 1,
                                         self.functors.softmax if ws else None, paged, heads)
-            # AE_CLOCK_STAMPS=1 (a measurement switch, read by ``bench.py --mfma-probe``): single-split launches of the
-            # wave-specialised kernel report the shader clock their workgroups ran at (``self.clock_stamps``)
-            self._stamped = ws and n_split == 1 and os.environ.get("AE_CLOCK_STAMPS", "") == "1"
-            if self._stamped:
+            if key[-1]:
                 cfg_src += "#define AE_CLOCK_STAMPS 1\n"
             module = rt.compile_module(self.template, {"ae_config.h": cfg_src, "ae_functors.h": self.functor_src},
                                        allow_spills=self.allow_spills)
@@ -840,7 +842,7 @@ class MLADecodeOp(_SplitTuning):
             partial_o = torch.empty((B, Hq, n_split, self.DV), dtype=torch.float32, device=dev)
             partial_rs = torch.empty((max(1, self.n_rowscales), B, Hq, n_split), dtype=torch.float32, device=dev)
             p.partial_o, p.partial_rs = partial_o.data_ptr(), partial_rs.data_ptr()
-        if n_split == 1 and getattr(self, "_stamped", False):
+        if self._stamped(n_split):
             n_ht = -(-(Hq // Hkv) // heads)
             n_wg = -(-(B * Hkv) // 8) * 8 * n_ht
             self._stamp_buffer = torch.zeros(6 * n_wg, dtype=torch.int64, device=dev)
@@ -866,7 +868,7 @@ class MLADecodeOp(_SplitTuning):
             modules += (self._merges.module(n_split),)
             combine = modules[1].kernel("ae_decode_combine_kernel")
         rt.mla_decode_fwd(split, combine, p, cfg, ccfg, rt.current_stream(dev))
-        if not getattr(self, "_stamped", False) and (self.n_rowscales == 1 or not self.cute):
+        if not self._stamped(n_split) and (self.n_rowscales == 1 or not self.cute):
             host.add_forward(self._host, host.MLA if paged is None else host.MLA_PAGED, B, 1, Hq, Hkv, Skv, dev, modules, split,
                              cfg, combine=combine, ccfg=ccfg, n_split=n_split, kv_per_split=kv_per_split,
                              page=paged[2] if paged is not None else 0)

@@ -550,7 +550,8 @@ class PrefillOp:
             table_rows = 1
         if mask_mode != 2:
             heavy_last = False
-        key = (mask_mode, even_q, even_kv, n_split > 1, table_rows, bool(heavy_last), band, astuple(tiles), tail)
+        key = (mask_mode, even_q, even_kv, n_split > 1, table_rows, bool(heavy_last), band, astuple(tiles), tail,
+               self._clock_stamps(tiles))
         v = self._variants.get(key)
         if v is None:
             has_mask_mod = self.elementwise_mask and mask_mode != 1
@@ -573,7 +574,7 @@ class PrefillOp:
                             f"#define AE_BAND_HI {'0x7fffffff' if band[1] is None else f'({band[1]})'}\n")
             if n_split > 1:
                 cfg_src += "#define AE_NSPLIT 2\n"       # (a split launch; its count is the launch's)
-            if self._clock_stamps(tiles):
+            if key[-1]:
                 cfg_src += "#define AE_CLOCK_STAMPS 1\n"
             if tail:
                 cfg_src += "#define AE_TAIL 1\n"

@@ -1019,3 +1019,26 @@ def test_plans_at_head_dim_64_have_costs_of_their_own():
     for B, Skv in ((1, 128), (3, 5000), (128, 16000)):
         n, per = gqa.plan_splits(B, 16, 2, Skv)
         assert n // gqa.N_WAVES in gqa.GROUPED_WGS_PER_KV_HEAD and n * per >= Skv
+
+
+def test_a_build_with_clock_stamps_is_launched_as_one_only(monkeypatch):
+    """Kernels built under AE_CLOCK_STAMPS=1 write their stamps through the partial-result pointer, which only a call under
+    the same switch sets: builds with and without stamps are kept apart, whatever was compiled in between."""
+    sm, f16 = C.make_scale_score_mod(0.1), torch.float16
+    mla = AttentionEngine(_meta(128, 128, 1, 1, 256, 576, 512, f16), CustomIO({}), sm, None, C.OnlineSoftmax(),
+                          kv_shared=True).attention
+    pre = AttentionEngine(_meta(2, 32, 32, 4096, 4096, 128, 128, f16), CustomIO({}), sm, None, C.OnlineSoftmax()).attention
+    assert pre.tiles.template == "ae_prefill_pipe.hip"
+
+    def builds():
+        got = mla._variant(1), pre._variant(pre.tiles, 0, 4096, 4096)
+        assert mla._stamped(1) == ("AE_CLOCK_STAMPS" in got[0][2]) and not mla._stamped(2)
+        assert pre._clock_stamps(pre.tiles) == ("#define AE_CLOCK_STAMPS" in got[1][2])
+        return got
+    plain = builds()
+    monkeypatch.setenv("AE_CLOCK_STAMPS", "1")
+    stamped = builds()
+    mla._variant(4)
+    assert builds()[0] is stamped[0] and stamped[0][0] is not plain[0][0] and stamped[1][0] is not plain[1][0]
+    monkeypatch.delenv("AE_CLOCK_STAMPS")
+    assert builds()[0] is plain[0] and builds()[1] is plain[1]
