@@ -58,10 +58,15 @@ def lower_combine(online_func, final_rowscale_names):
     for i in range(len(final_rowscale_names)):
         body.append(f"  merged[{i}] = {merged.get(i, undefined)};")
     text = "\n".join(body)
-    return f"""AE_DEV void ae_combine(const float (&rs)[{nrs}][AE_NSPLIT], float (&w)[AE_NSPLIT],
+    # (a template over the number of partial results, whatever the configuration's macro of that name says)
+    return f"""#pragma push_macro("AE_NSPLIT")
+#undef AE_NSPLIT
+template <int AE_NSPLIT>
+AE_DEV void ae_combine(const float (&rs)[{nrs}][AE_NSPLIT], float (&w)[AE_NSPLIT],
                        float (&merged)[{nrs}]) {{
 {text}
 }}
+#pragma pop_macro("AE_NSPLIT")
 """
 
 
@@ -94,9 +99,9 @@ def combine_rows(threads, dv):
 
 def merge_capacity(n, any_order):
     """Partial results that a merge of ``n`` is built for.  The log-sum-exp merge gives places without a result no weight, so
-    it is built for powers of two: a cache that grows by a token a call meets a new kernel only where it has doubled.  What
-    the empty places cost: 0.1 us a call (B4 H64 Skv1723, 11 of 16 places: merge 3.72 -> 3.80 us).  Another combine() is
-    built for its exact count."""
+    it is built for powers of two: a cache that grows by a token a call meets a new kernel only where it has doubled.  Up to
+    16 places every count, beyond that 5, 6, 7 and 8 eighths of the places are constants of the build and cost what a build
+    for the exact count does; others up to 0.1 us a call (B1 H64 Skv4009, 21 of 32 places: merge 3.92 us on both).  Another combine() is built for its exact count."""
     return 1 << (n - 1).bit_length() if any_order else n
 
 

@@ -66,7 +66,7 @@ class AttnParams(C.Structure):
         ("mask_b", C.c_int32), ("mask_h", C.c_int32), ("mask_nq", C.c_int32), ("mask_nkv", C.c_int32),
         ("mask_block_m", C.c_int32), ("mask_block_n", C.c_int32),
         ("num_splits", C.c_int32), ("kv_per_split", C.c_int32),
-        ("tail_slots", C.c_int32), ("reserved", C.c_int32 * 2),
+        ("tail_slots", C.c_int32), ("units_reciprocal", C.c_uint32), ("reserved", C.c_int32),
         ("block_table", C.c_void_p), ("seqlens_k", C.c_void_p),
         ("block_table_stride", C.c_int32), ("page_block_size", C.c_int32), ("num_pages", C.c_int32),
         ("reserved2", C.c_int32),

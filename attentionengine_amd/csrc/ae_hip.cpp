@@ -630,13 +630,20 @@ int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params
   // paged launch counts an odd number of splits per entry (ae_mla_odd_units in ae_mla_paged.h).
   int group = p->heads_q / p->heads_kv;
   int64_t n_ht = (group + cfg->block_m - 1) / cfg->block_m;
-  int64_t units = (int64_t)p->batch * p->heads_kv * p->num_splits;
-  if (cfg->paged && units * n_ht > 128) units = (int64_t)p->batch * p->heads_kv * (p->num_splits | 1);
+  int64_t units = (int64_t)p->batch * p->heads_kv * p->num_splits, a_head = p->num_splits;
+  if (cfg->paged && units * n_ht > 128) a_head |= 1;
+  units = (int64_t)p->batch * p->heads_kv * a_head;
   int64_t total = ((units + 7) / 8) * 8 * n_ht;
   if (total > 0x7fffffffll) return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: grid too large");
   uint32_t grid[3] = {(uint32_t)total, 1, 1};
   uint32_t block[3] = {(uint32_t)cfg->threads, 1, 1};
-  rc = ae_launch(split, p, sizeof *p, grid, block, (uint32_t)cfg->lds_bytes, stream);
+  // (id / a_head as a multiplication: exact while ids * a_head < 2^32, since the reciprocal is less than 2^-32 * a_head off.
+  // A division in front of the first request costs 0.1 us of the call)
+  ae_attn_params q = *p;
+  q.units_reciprocal = (uint64_t)(units + 8) * (uint64_t)a_head < (1ull << 32) && a_head > 1
+                           ? (uint32_t)(((1ull << 32) + (uint64_t)a_head - 1) / (uint64_t)a_head)
+                           : 0;
+  rc = ae_launch(split, &q, sizeof q, grid, block, (uint32_t)cfg->lds_bytes, stream);
   if (rc || direct) return rc;
   uint32_t cgrid[3] = {combine_grid(p->heads_q, combine_cfg), (uint32_t)p->batch, 1};
   uint32_t cblock[3] = {(uint32_t)combine_cfg->threads, 1, 1};

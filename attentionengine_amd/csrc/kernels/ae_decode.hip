@@ -434,14 +434,13 @@ void ae_decode_split_kernel(const ae_attn_params p) {
         // vector ones kept from one use to the next, do not fit the scalar registers)
         int n_row = n_part, n_load = n_part, n_weight = n_part;
         if (!kFixed) asm volatile("" : "+v"(n_row), "+v"(n_load), "+v"(n_weight));
-        float rs[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1][AE_NSPLIT];
+        float rs[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1][N];
 #pragma unroll
         for (int i = 0; i < AE_N_ROWSCALES; i++)
 #pragma unroll
-          for (int k = 0; k < AE_NSPLIT; k++)
-            rs[i][k] = k >= N ? AE_NEG_INF
-                              : __hip_atomic_load(p.partial_rs + (int64_t)i * p.batch * p.heads_q * n_part + tile_row0 + rs_at +
-                                                      (kFixed || k < n_row ? k : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          for (int k = 0; k < N; k++)
+            rs[i][k] = __hip_atomic_load(p.partial_rs + (int64_t)i * p.batch * p.heads_q * n_part + tile_row0 + rs_at +
+                                             (kFixed || k < n_row ? k : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         constexpr int G = N < 16 ? N : 16;     // partial results in flight at a time
         ae_f32x4 val[G];
         auto load_part = [&](int k) AE_LAMBDA -> ae_f32x4 {
@@ -454,9 +453,9 @@ void ae_decode_split_kernel(const ae_attn_params p) {
 #pragma unroll
           for (int i = 0; i < AE_N_ROWSCALES; i++)
 #pragma unroll
-            for (int k = 0; k < AE_NSPLIT; k++) rs[i][k] = k < n_weight ? rs[i][k] : AE_NEG_INF;
+            for (int k = 0; k < N; k++) rs[i][k] = k < n_weight ? rs[i][k] : AE_NEG_INF;
         }
-        float w[AE_NSPLIT];
+        float w[N];
         float merged[AE_N_ROWSCALES > 0 ? AE_N_ROWSCALES : 1];
         ae_combine(rs, w, merged);
         // (the sum runs over the splits in ascending order, as in ae_decode_combine_kernel: equal to the last bit)

@@ -180,7 +180,13 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #if AE_PAGED
   if (ae_mla_odd_units(p, n_ht)) units |= 1;
 #endif
-  int b = ae_divide((int)u, units, split);
+  int b;
+  if (__builtin_expect(p.units_reciprocal != 0, 1)) {
+    b = (int)(((uint64_t)u * (uint32_t)p.units_reciprocal) >> 32);
+    split = (int)u - b * units;
+  } else {
+    b = ae_divide((int)u, units, split);
+  }
 #endif
   if (b >= p.batch * p.heads_kv || split >= n_split) return;  // grid padding (whole workgroup exits)
   if (AE_NSPLIT > 1 && !AE_PAGED && n_split < 2) return;      // (a launch for the build that writes out)

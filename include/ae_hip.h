@@ -105,7 +105,10 @@ typedef struct ae_attn_params {
    * the one that finishes last merges.  partial_o: 8 * tail_slots * num_splits * (block_m * DV + 4 * threads) floats;
    * partial_rs: 8 * tail_slots int32 arrival counters, zero when the launch starts and when it ends.  Else 0. */
   int32_t tail_slots;
-  int32_t reserved[2];
+  /* Filled in by ae_mla_decode_fwd for its split kernel, whatever the caller left there: ceil(2^32 / u) of the number u of
+   * workgroup ids per (batch, kv head), or 0 where ids times u do not fit 32 bits. */
+  uint32_t units_reciprocal;
+  int32_t reserved;
   /* MLA decode on a paged cache (kernels whose ae_tile_cfg.paged is 1; NULL / 0 otherwise): the cache is
    * [num_pages, page_block_size, Hkv, D] (k_stride_b = elements between pages, k_stride_s between the
    * rows of a page), token t of batch entry b is row t % page_block_size of page

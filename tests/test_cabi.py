@@ -447,6 +447,27 @@ def test_a_module_may_hold_the_split_and_the_merge_kernel():
         assert set(rt.compile_module(template, both).kernel_info()) == {name, "ae_decode_combine_kernel"}
 
 
+@pytest.mark.parametrize("dv", [64, 128, 512])
+@pytest.mark.parametrize("places", [2, 8, 16, 32, 64])
+def test_merge_kernels_keep_their_weights_in_registers(dv, places):
+    """Every merge build and every last-workgroup merge of the decode kernel: no spilled vector or scalar register, and
+    buffer descriptors in scalar registers (in vector registers every load becomes a loop over the lanes' descriptors, which
+    multiplies the code: 32 places at 512 columns once took 5.6 us instead of 3.9)."""
+    import __graft_entry__ as G
+    from core.lower import lower_decode as LD
+    functors = [h for t, h in G.representative_headers() if t == "ae_combine.hip"][0]["ae_functors.h"]
+    built = [rt.compile_module("ae_combine.hip", {"ae_config.h": LD.merge_config(dv, torch.bfloat16, 1, places, 128 if dv > 256 else 64),
+                                                  "ae_functors.h": functors})]
+    if dv <= 128:
+        config = LD.render_decode_config(dv, dv, torch.bfloat16, 4, 2, (64 - (2 * dv) % 256) % 256 or 256, 1, False, True, places,
+                                         False, True, True)
+        built.append(rt.compile_module("ae_decode.hip", {"ae_config.h": config, "ae_functors.h": functors}, allow_spills=True))
+    for m in built:
+        for k in m.kernel_info().values():
+            assert k[".vgpr_spill_count"] == 0 and k[".sgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0
+        assert len(m.code()) < (48 << 10), len(m.code())
+
+
 def test_benchmarked_kernels_do_not_spill_registers():
     """The code objects hipRTC builds for the benchmark configurations (and the backward of the causal one) keep
     every value in registers: a kernel that spills pays for it with scratch-memory traffic in every workgroup, and
