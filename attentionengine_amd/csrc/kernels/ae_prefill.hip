@@ -71,6 +71,16 @@
 #define AE_BAND_HI 0x7fffffff
 #endif
 
+// AE_ROTATE 1 (bands with two ends): a q tile starts at the kv tile whose index is a multiple of AE_PERIOD - the most tiles that
+// a q tile's band can have, so its range holds at most one - and takes the front of its range last.  A kv tile is read by the
+// (AE_BM + width) / AE_BM q tiles whose bands hold it; walked from the front of each range they come to it AE_BM / AE_BN trips
+// apart, by when the 64 workgroups of an XCD have pushed it out of the 4 MB L2 (20 % hits, 410 MB read for 201 MB of q, k and v).
+// Started this way, workgroups in step with each other read the same tile in the same trip.  Inputs not in the caches, B2 H32
+// S4096 D128 fp16: window 256 85.9 -> 76.8 us; calls one after the other, window 1024 162.4 -> 155.8, B4 S4000 bf16 window 64
+// 119.8 -> 116.4, B3 S5188 bf16 window 388 179.2 -> 169.3.  Not at narrower heads: the keys and values of 64 neighbouring q
+// tiles are 2 MB there and stay in the L2 anyway (B2 H16 S2886 D64 window 843 32.8 -> 33.8).
+#define AE_ROTATE (AE_MASK_MODE == 3 && AE_BAND_HI != 0x7fffffff && AE_NSPLIT == 1 && AE_KW == 1 && AE_D + AE_DV >= 256)
+
 // AE_KW > 1: the waves of a workgroup also share the kv axis.  AE_NWAVES waves own 32 query rows each, as always; AE_KW
 // such sets of waves ("kv groups") walk the kv tiles in turn, each with its own pair of LDS stages, and meet at the end:
 // every wave leaves its unscaled O in LDS, rescales a share of the value columns to the common reference and sums it
@@ -116,6 +126,10 @@
 #define AE_GT (AE_NWAVES * 64)     // threads of a kv group
 #define AE_NT (AE_GT * AE_KW)
 #define AE_NB (AE_BN / 32)        // 32-wide kv blocks per tile
+#if AE_ROTATE
+constexpr int ae_floor_div(int a, int b) { return a >= 0 ? a / b : -((b - 1 - a) / b); }
+#define AE_PERIOD (ae_floor_div(AE_BM - 1 - (AE_BAND_LO), AE_BN) - ae_floor_div(-(AE_BAND_HI), AE_BN) + 1)
+#endif
 #define AE_NS (AE_NB * 16)        // score elements per lane per tile
 #define AE_NDB (AE_DV / 32)       // 32-wide dv blocks
 #define AE_NO (AE_NDB * 16)       // output elements per lane
@@ -430,6 +444,9 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #else
   int j = next_tile(j_begin);
 #endif
+#elif AE_ROTATE
+  int j = (j_first + AE_PERIOD - 1) / AE_PERIOD * AE_PERIOD;
+  j = j < j_end ? j : j_first;
 #elif AE_ANALYTIC
   int j = j_first;
 #else
@@ -444,6 +461,14 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #else
   const int j_trips = j_end;
 #define AE_J_LIVE true
+#endif
+#if AE_ROTATE
+  int left = j_end - j_first;          // tiles still to be multiplied
+#define AE_TRIPS_LEFT (left > 0)
+#define AE_HAS_NEXT (left > 1)
+#else
+#define AE_TRIPS_LEFT (j < j_trips)
+#define AE_HAS_NEXT (jn < j_end)
 #endif
   int cls[AE_RB];          // class of tile j for this lane's row of each row block
   // 1 once this lane's row of a row block has met a key it may see.  A row that never does - inside a q tile whose
@@ -477,12 +502,16 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #endif
 
   int stage = 0;
-  while (j < j_trips) {
+  while (AE_TRIPS_LEFT) {
+#if AE_ROTATE
+    const int jn = j + 1 == j_end ? j_first : j + 1;
+#else
     const int jn = next_tile(j + AE_KW);
+#endif
     int cls_n[AE_RB];
 #pragma unroll
     for (int rb = 0; rb < AE_RB; rb++) cls_n[rb] = row_class(jn, rb);
-    if (jn < j_end) load_tile(jn, stage ^ 1);   // streams into the other stage while this one is used
+    if (AE_HAS_NEXT) load_tile(jn, stage ^ 1);   // streams into the other stage while this one is used
 
     ae_lds_byte* ks_ = lds + stage * AE_STAGE_BYTES;
     ae_lds_byte* vs_ = ks_ + AE_K_BYTES;
@@ -623,7 +652,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #ifdef AE_HAS_KV_PREFETCH
       // the functors are done with this tile's elements of the per-score custom inputs: request the next
       // tile's, which travel while the second product runs
-      if (jn < j_end) ae_prefetch_custom(cust[rb], jn * AE_BN + 4 * hf, q0w + rb * 32, jn * AE_BN, p);
+      if (AE_HAS_NEXT) ae_prefetch_custom(cust[rb], jn * AE_BN + 4 * hf, q0w + rb * 32, jn * AE_BN, p);
 #endif
 
 #if AE_PAD_WEIGHTS
@@ -701,6 +730,9 @@ void ae_prefill_kernel(const ae_attn_params p) {
     __syncthreads();
     stage ^= 1;
     j = jn;
+#if AE_ROTATE
+    left--;
+#endif
 #pragma unroll
     for (int rb = 0; rb < AE_RB; rb++) cls[rb] = cls_n[rb];
   }

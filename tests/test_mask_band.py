@@ -70,6 +70,28 @@ def test_banded_masks_against_the_oracle(cuda_device, name, Sq, Skv, D):
     assert torch.equal(torch.isfinite(lse[b]), seen) and (lse[b][seen] - rlse[seen]).abs().max().item() <= 1e-3
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("lo,hi", [(0, 0), (0, 31), (0, 96), (0, 97), (0, 128), (0, 500), (-70, 30), (65, 200), (-40, 0)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_bands_with_two_ends_start_inside_their_range(cuda_device, lo, hi, D):
+    """Every kv tile of a q tile's range is multiplied once, wherever the walk starts (AE_ROTATE)."""
+    B, H, S, dtype = (9 if D == 64 else 3), 32, 555, torch.float16          # (no groups of waves along the kv axis)
+    mask = lambda b, h, q, kv: (q - lo >= kv) & (q - hi <= kv)  # noqa: E731
+    q, k, v = C.make_inputs(B, S, S, H, H, D, D, dtype, seed=7)
+    meta = tuple(meta_tensor(B, H, S, D, dtype=dtype) for _ in range(3))
+    mod = AttentionEngine(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), mask, C.OnlineSoftmax())
+    assert "#define AE_BAND 1" in mod.tl_code
+    out = mod(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+    lse = mod.final_rowscales["lse"].cpu()
+    b = slice(B - 1, B)
+    ref, rlse = R.softmax_attention(q[b], k[b], v[b], causal=False, mask=torch.from_numpy(OM.dense_mask_grid(mask, 1, H, S, S)))
+    seen = torch.isfinite(rlse)
+    assert torch.equal(torch.isfinite(lse[b]), seen) and (lse[b][seen] - rlse[seen]).abs().max().item() <= 1e-3
+    # sum of |P rounding| <= 2^-11 (the weights sum to 1), times the largest |v|, and the result's own rounding
+    bound = 2.0 ** -10 * v.float().abs().max().item() + 2.0 ** -11 * ref.nan_to_num(0.0).abs().max().item()
+    assert (out[b] - ref.nan_to_num(0.0)).abs().max().item() <= bound
+
+
 @pytest.mark.parametrize("Sq,Skv", [(1, 1), (31, 33), (300, 300), (130, 517), (517, 130), (256, 64)])
 @pytest.mark.parametrize("name", ["causal", "plus_one", "window", "head", "holes", "all", "none"])
 def test_tables_put_together_from_one_survey(name, Sq, Skv):
