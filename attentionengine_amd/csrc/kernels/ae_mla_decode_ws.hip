@@ -19,7 +19,7 @@
 //     fragment feeding both 32-head blocks.
 // Wave i runs on SIMD i % 4.  The workgroup is launched with 8 waves: waves 0, 1 are the score waves
 // (SIMD 0, 1: 1152 matrix-pipe cycles per tile each), waves 2, 3, 6, 7 the value waves (two each on SIMD
-// 2, 3: 2 x 512 cycles), waves 4, 5 leave at once - so the four SIMDs carry about the same MFMA work.
+// 2, 3: 2 x 512 cycles), waves 4, 5 leave at once (AE_HPW 16, paged cache: they request the tiles, AE_LOADER_WAVES) - so the four SIMDs carry about the same MFMA work.
 // The score waves run one tile ahead of the value waves: one workgroup barrier per tile hands P over.
 // Scores are computed once: 124 KiB of LDS reads per tile instead of 416.  KV tiles go HBM -> LDS
 // directly (16 B per lane, chunk-swizzled as in ae_mla_decode.hip), AE_NSTAGE tiles deep; a trip ends by
@@ -48,6 +48,9 @@
 #include "ae_device.h"
 #include "ae_functors.h"
 
+#ifndef AE_PAGED
+#define AE_PAGED 0
+#endif
 #define AE_D (AE_D1 + AE_D2)
 #define AE_NWAVES 8
 #define AE_NT (AE_NWAVES * 64)
@@ -63,7 +66,15 @@
 #else
 #define AE_NKS (AE_D / 32)                // 32-deep ones
 #endif
-#define AE_NLOADERS 4                     // the value waves also request the KV tiles
+// 1: the tiles are requested by two waves of their own - waves 4 and 5, which 16 heads a workgroup leave idle - on the score
+// waves' SIMDs.  A trip of 16 heads is bound by the serial chain of each wave (the LDS pipe busy for 830 of its 1500 cycles):
+// a value wave that first issues nine requests, 16 cycles each, comes late to its products.  Paged cache, 128 heads, one
+// split: 0.647 -> 0.533 us a trip, 0.9 us more until the first; B8 H128, 2048 tokens at most 19.8 -> 18.4 us, B6 H64 5568
+// 21.5 -> 19.9, splits of two to four tiles the same.  Not for the dense cache: its requests take two VALU instructions
+// each to step an address, which there delay the score waves (0.600 -> 0.606; four request waves of three a SIMD 0.592
+// and, paged, 0.568).  Nor with 32 heads, where the score waves are waves 4 and 5 too (four more waves: 0.81 -> 0.87).
+#define AE_LOADER_WAVES (AE_HPW == 16 && AE_PAGED)
+#define AE_NLOADERS (AE_LOADER_WAVES ? 2 : 4)      // else the value waves also request the KV tiles
 #define AE_DVW (AE_DV / 4)                // value columns of one value wave
 #if AE_HPW == 64
 #define AE_NDB (AE_DVW / 32)              // 32-wide dv blocks of a value wave
@@ -78,8 +89,8 @@
 #define AE_CPR1 (AE_D1 / 8)
 #define AE_BLOCKS ((AE_BN * AE_CPR) / 64) // 1 KiB blocks per tile
 #define AE_LOADS ((AE_BLOCKS + AE_NLOADERS - 1) / AE_NLOADERS)
-#define AE_L1 ((AE_LOADS + 1) / 2)        // a wave's loads of one tile go out as two bursts
-#define AE_L2 (AE_LOADS - AE_L1)
+#define AE_BURSTS (AE_LOADS <= 16 ? 2 : 3)   // a wave's loads of one tile go out as two or three bursts, burst i from load AE_LB(i)
+#define AE_LB(i) (((i) * AE_LOADS + AE_BURSTS - 1) / AE_BURSTS)
 #ifndef AE_NSTAGE
 #define AE_NSTAGE 4
 #define AE_PTAB 1024      // paged cache: block-table entries of one split kept in LDS
@@ -104,7 +115,8 @@ static_assert(AE_D % 64 == 0, "two accumulation chains over the k-steps");
 static_assert(AE_DV % 128 == 0 && AE_DV <= AE_D1, "V must be a prefix of the latent part, four 32-column blocks wide");
 static_assert(AE_CPR % 8 == 0 && AE_CPR1 % 8 == 0, "chunk groups of eight must not straddle the two K tensors");
 static_assert((AE_BN * AE_CPR) % 64 == 0, "tile must be a whole number of 1 KiB blocks");
-static_assert(AE_L1 <= 8 && AE_L2 >= 1 && AE_BLOCKS >= AE_LOADS, "two bursts of at most eight loads per wave and tile");
+static_assert(AE_LB(1) <= 8 && AE_LOADS >= AE_BURSTS && AE_BLOCKS >= AE_LOADS, "bursts of at most eight loads per wave and tile");
+static_assert(2 * AE_LOADS <= 63 && AE_NSTAGE == 4, "the wait counter holds the requests in flight");
 // chunk exchange of the results in LDS: inside groups that divide a head's chunks (16 where there are as many)
 #define AE_OSW1 ((AE_DVW / 8) & -(AE_DVW / 8))
 #define AE_OSW (AE_OSW1 < 16 ? AE_OSW1 - 1 : 15)
@@ -112,9 +124,6 @@ static_assert(AE_DV * AE_HEADS_PER_WG * 4 <= AE_NSTAGE * AE_STAGE_BYTES, "the re
 static_assert(AE_DVW % 64 == 0, "a value wave's first chunk is a multiple of eight, a block of heads leaves in whole instructions");
 static_assert(AE_NSTAGE >= 3, "a tile is multiplied by K one trip before it is multiplied as V");
 
-#ifndef AE_PAGED
-#define AE_PAGED 0
-#endif
 // 1 (single-split builds only, a measurement switch): every workgroup reports the shader-clock cycles (s_memtime)
 // and the constant-rate 100 MHz ticks (s_memrealtime) between its entry and its last store, as two 64-bit values
 // at ((unsigned long long*)p.partial_o)[2 * blockIdx.x] - a buffer a single-split launch does not otherwise use -
@@ -132,6 +141,7 @@ typedef __attribute__((address_space(3))) unsigned char ae_lds_byte;
 typedef __attribute__((address_space(3))) float ae_lds_f32;
 typedef __attribute__((address_space(3))) int ae_lds_i32;
 template <bool B> struct ae_const_bool { static constexpr bool value = B; };
+template <int I> struct ae_const_int { static constexpr int value = I; };
 
 extern "C" __global__ __launch_bounds__(AE_NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void ae_mla_decode_split_kernel(const ae_attn_params p) {
@@ -149,6 +159,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool score_wave = wave < 2 || (AE_HPW == 32 && (wave == 4 || wave == 5));
+  const bool requests = AE_LOADER_WAVES ? wave == 4 || wave == 5 : !score_wave;      // (waves that request the tiles)
 #if AE_CLOCK_STAMPS
   const unsigned long long ae_t0 = __builtin_amdgcn_s_memtime();
   const unsigned long long ae_w0 = __builtin_amdgcn_s_memrealtime();
@@ -221,7 +232,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   // row; what an entry shorter than that left unset is read, but never followed.
   int seqlen_b = p.seqlens_k[b];
   int table0 = 0;
-  if (!score_wave && rq_slot0 + lane <= top_slot) table0 = pages[rq_slot0 + lane];
+  if (requests && rq_slot0 + lane <= top_slot) table0 = pages[rq_slot0 + lane];
 #else
   const ae_elem* k1 = (const ae_elem*)p.k + (int64_t)b * p.k_stride_b + (int64_t)hk * p.k_stride_h;
   const ae_elem* k2 = (const ae_elem*)p.k2 + (int64_t)b * p.k2_stride_b + (int64_t)hk * p.k2_stride_h;
@@ -230,6 +241,80 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 
 #if AE_PAGED
   asm volatile("" ::: "memory");   // (both requests stay in front of the first wait and of the exits below)
+#endif
+
+  // ============================== tile requests =========================================================
+  // Direct HBM -> LDS tile load, by the four value waves or by waves of their own: wave w fills AE_LOADS consecutive 1 KiB blocks of
+  // the tile, starting at block min(w*AE_LOADS, AE_BLOCKS-AE_LOADS) (the last wave overlaps its neighbour, so
+  // every wave issues the same number of loads); LDS chunk c' of row r receives global chunk c' ^ f(r).
+  // Which row and chunk a lane fetches never changes: its byte offset inside a tile is computed once (one
+  // register per load) and added per tile to the tile's wave-uniform address in the latent or in the rope
+  // tensor.  The loads of a wave go out as bursts, each behind a single write of M0 (see
+  // ae_load_lds16_burst; the offsets carry the compensation for its immediate offsets).  Rows past the
+  // end re-read the last row.  Tiles past the end are not requested, so the waits for a tile ask whether a newer one
+  // is on its way (a split of four tiles asked for nine when every trip requested one, and waited for them at its end).
+  const int loader = AE_LOADER_WAVES ? wave - 4 : wave < 4 ? wave - 2 : wave - 4;
+  const int blk0 = loader * AE_LOADS < AE_BLOCKS - AE_LOADS ? loader * AE_LOADS : AE_BLOCKS - AE_LOADS;
+  // (the row and chunk of load i are carried along, and their row's offset with them: a division and a multiplication
+  // per load were a third of the instructions in front of the first request)
+  const int stride1 = (int)p.k_stride_s * 2, stride2 = (int)p.k2_stride_s * 2;   // bytes per kv row
+#if AE_PAGED
+  unsigned ld_uoff[AE_LOADS];
+#else
+  const char* ld_ptr[AE_LOADS];
+  unsigned ld_adv[AE_LOADS];
+#endif
+  auto set_up_requests = [&]() AE_LAMBDA {
+    int ld_row = (blk0 * 64 + lane) / AE_CPR, ld_cp = (blk0 * 64 + lane) % AE_CPR;
+#if AE_PAGED
+    // Paged cache: the latent and the rope part are column ranges of ONE cache tensor (equal strides, the rope
+    // columns rope_delta bytes behind the latent ones: checked by ae_mla_decode_fwd), so every load of a tile is
+    // (the tile's wave-uniform address) + (an offset of the lane that never changes): scalar base + 32-bit offset
+    // loads, no address arithmetic per tile at all.  Bases are passed 4 KiB low and the offsets 4 KiB high, so
+    // that the offsets, which carry the compensation for the immediate offsets, stay >= 0.
+    const int rope_off = (int)((const char*)k2 - (const char*)k1) - AE_CPR1 * 16;
+    int ld_roff = ld_row * stride1 + 4096;
+#else
+    // Dense cache: the requests go tile by tile, so a lane keeps the source address of each of its loads for the
+    // NEXT tile to request and adds the tile pitch after every request - two instructions per load and tile.
+    // (Two waves share a SIMD here: address arithmetic of ~140 instructions per tile and wave, as a base + offset
+    // form needs, made these waves, not the matrix pipe, set the pace of the whole workgroup.)
+    const char* const ld_base1 = (const char*)k1 + (uint64_t)((unsigned)kv_begin * (uint64_t)(unsigned)stride1);
+    const char* const ld_base2 = (const char*)k2 + (uint64_t)((unsigned)kv_begin * (uint64_t)(unsigned)stride2);
+    int ld_roff1 = ld_row * stride1, ld_roff2 = ld_row * stride2 - AE_CPR1 * 16;
+#endif
+#pragma unroll
+    for (int i = 0; i < AE_LOADS; i++) {
+      const int c = ld_cp ^ AE_SWZ(ld_row);
+      const bool rope = c >= AE_CPR1;
+      // immediate offset of load i inside its burst
+      const int burst = i < AE_LB(1) ? 0 : i < AE_LB(2) ? 1 : 2;
+      const int imm = (i - AE_LB(burst) - (AE_LB(burst + 1) - AE_LB(burst)) / 2) * 1024;
+#if AE_PAGED
+      ld_uoff[i] = (unsigned)(c * 16 + ld_roff + (rope ? rope_off : 0) - imm);
+#else
+      ld_ptr[i] = (rope ? ld_base2 : ld_base1) + (int64_t)(c * 16 + (rope ? ld_roff2 : ld_roff1) - imm);
+      ld_adv[i] = AE_BN * (unsigned)(rope ? stride2 : stride1);
+#endif
+      ld_cp += 64 % AE_CPR;
+      const bool wrap = ld_cp >= AE_CPR;
+      const int rows = 64 / AE_CPR + (wrap ? 1 : 0);
+      ld_cp -= wrap ? AE_CPR : 0;
+      ld_row += rows;
+#if AE_PAGED
+      ld_roff += 64 / AE_CPR * stride1 + (wrap ? stride1 : 0);
+#else
+      ld_roff1 += 64 / AE_CPR * stride1 + (wrap ? stride1 : 0);
+      ld_roff2 += 64 / AE_CPR * stride2 + (wrap ? stride2 : 0);
+#endif
+    }
+  };
+#if AE_PAGED
+  if (requests) {
+    set_up_requests();                       // while the entry's length and the table are on their way
+#pragma unroll
+    for (int i = 0; i < AE_LOADS; i++) asm volatile("" : "+v"(ld_uoff[i]));
+  }
   seqlen_b = seqlen_b < p.seqlen_kv ? seqlen_b : p.seqlen_kv;
   seqlen_b = __builtin_amdgcn_readfirstlane(seqlen_b > 0 ? seqlen_b : 0);
 #endif
@@ -255,7 +340,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #else
   constexpr bool direct = false;
 #endif
-  if (!score_wave && (wave == 4 || wave == 5)) return;      // placeholders: they only steer the value waves onto SIMD 2, 3
+  if (!AE_LOADER_WAVES && !score_wave && (wave == 4 || wave == 5)) return;      // placeholders: they only steer the value waves onto SIMD 2, 3
 
 #if AE_HPW != 64
   if (score_wave) {
@@ -528,74 +613,12 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   }
 #endif
 
-  // ============================== value wave: AE_DVW value columns, AE_HPW heads =======================
-#if AE_HPW == 64
-  const int lhd = lane & 31;       // the lane's head in a block of heads
-  const int hf = lane >> 5;        // ... and which part of the block's rows
-#else
-  const int lhd = lane & 15;
-  const int hf = lane >> 4;
+#if AE_LOADER_WAVES
+  if (requests) {
 #endif
-  const int dvw = wave < 4 ? wave - 2 : wave - 4;   // waves 2, 3, 6, 7
-  // Direct HBM -> LDS tile load, by the four value waves: wave w fills AE_LOADS consecutive 1 KiB blocks of
-  // the tile, starting at block min(w*AE_LOADS, AE_BLOCKS-AE_LOADS) (the last wave overlaps its neighbour, so
-  // every wave issues the same number of loads); LDS chunk c' of row r receives global chunk c' ^ f(r).
-  // Which row and chunk a lane fetches never changes: its byte offset inside a tile is computed once (one
-  // register per load) and added per tile to the tile's wave-uniform address in the latent or in the rope
-  // tensor.  The loads of a wave go out as two bursts, each behind a single write of M0 (see
-  // ae_load_lds16_burst; the offsets carry the compensation for its immediate offsets).  Rows past the
-  // end re-read the last row.  Tiles past the end are not requested, so the waits for a tile ask whether a newer one
-  // is on its way (a split of four tiles asked for nine when every trip requested one, and waited for them at its end).
-  const int blk0 = dvw * AE_LOADS < AE_BLOCKS - AE_LOADS ? dvw * AE_LOADS : AE_BLOCKS - AE_LOADS;
-  // (the row and chunk of load i are carried along, and their row's offset with them: a division and a multiplication
-  // per load were a third of the instructions in front of the first request)
-  const int stride1 = (int)p.k_stride_s * 2, stride2 = (int)p.k2_stride_s * 2;   // bytes per kv row
-  int ld_row = (blk0 * 64 + lane) / AE_CPR, ld_cp = (blk0 * 64 + lane) % AE_CPR;
-#if AE_PAGED
-  // Paged cache: the latent and the rope part are column ranges of ONE cache tensor (equal strides, the rope
-  // columns rope_delta bytes behind the latent ones: checked by ae_mla_decode_fwd), so every load of a tile is
-  // (the tile's wave-uniform address) + (an offset of the lane that never changes): scalar base + 32-bit offset
-  // loads, no address arithmetic per tile at all.  Bases are passed 4 KiB low and the offsets 4 KiB high, so
-  // that the offsets, which carry the compensation for the immediate offsets, stay >= 0.
-  const int rope_off = (int)((const char*)k2 - (const char*)k1) - AE_CPR1 * 16;
-  unsigned ld_uoff[AE_LOADS];
-  int ld_roff = ld_row * stride1 + 4096;
+#if !AE_PAGED
+  set_up_requests();
 #else
-  // Dense cache: the requests go tile by tile, so a lane keeps the source address of each of its loads for the
-  // NEXT tile to request and adds the tile pitch after every request - two instructions per load and tile.
-  // (Two waves share a SIMD here: address arithmetic of ~140 instructions per tile and wave, as a base + offset
-  // form needs, made these waves, not the matrix pipe, set the pace of the whole workgroup.)
-  const char* ld_ptr[AE_LOADS];
-  unsigned ld_adv[AE_LOADS];
-  const char* const ld_base1 = (const char*)k1 + (uint64_t)((unsigned)kv_begin * (uint64_t)(unsigned)stride1);
-  const char* const ld_base2 = (const char*)k2 + (uint64_t)((unsigned)kv_begin * (uint64_t)(unsigned)stride2);
-  int ld_roff1 = ld_row * stride1, ld_roff2 = ld_row * stride2 - AE_CPR1 * 16;
-#endif
-#pragma unroll
-  for (int i = 0; i < AE_LOADS; i++) {
-    const int c = ld_cp ^ AE_SWZ(ld_row);
-    const bool rope = c >= AE_CPR1;
-    // immediate offset of load i inside its burst
-    const int imm = i < AE_L1 ? (i - AE_L1 / 2) * 1024 : (i - AE_L1 - AE_L2 / 2) * 1024;
-#if AE_PAGED
-    ld_uoff[i] = (unsigned)(c * 16 + ld_roff + (rope ? rope_off : 0) - imm);
-#else
-    ld_ptr[i] = (rope ? ld_base2 : ld_base1) + (int64_t)(c * 16 + (rope ? ld_roff2 : ld_roff1) - imm);
-    ld_adv[i] = AE_BN * (unsigned)(rope ? stride2 : stride1);
-#endif
-    ld_cp += 64 % AE_CPR;
-    const bool wrap = ld_cp >= AE_CPR;
-    const int rows = 64 / AE_CPR + (wrap ? 1 : 0);
-    ld_cp -= wrap ? AE_CPR : 0;
-    ld_row += rows;
-#if AE_PAGED
-    ld_roff += 64 / AE_CPR * stride1 + (wrap ? stride1 : 0);
-#else
-    ld_roff1 += 64 / AE_CPR * stride1 + (wrap ? stride1 : 0);
-    ld_roff2 += 64 / AE_CPR * stride2 + (wrap ? stride2 : 0);
-#endif
-  }
-#if AE_PAGED
   // Paged cache: page, and row inside it, of the tile the NEXT request reads (wave-uniform; requests go tile by
   // tile, so no division per tile).  The split's part of the block table is copied into LDS first and looked up
   // there: once the tile loads are in flight, a table entry read from memory comes back through the same counter
@@ -622,53 +645,53 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     int page = rq_page < 0 ? 0 : (rq_page < p.num_pages ? rq_page : p.num_pages - 1);
     page = __builtin_amdgcn_readfirstlane(page);
     const char* tile = (const char*)k1 + ((int64_t)page * p.k_stride_b + (int64_t)rq_in_page * p.k_stride_s) * 2 - 4096;
-    unsigned o1[8], o2[8];
+    unsigned o[AE_LOADS];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      o1[i] = ld_uoff[i < AE_L1 ? i : 0];
-      o2[i] = ld_uoff[i < AE_L2 ? AE_L1 + i : AE_L1];
-    }
+    for (int i = 0; i < AE_LOADS; i++) o[i] = ld_uoff[i];
     if (__builtin_expect(ragged, 0)) {                        // rows past the end re-read the last row
       int ln = lane;
       asm volatile("" : "+v"(ln)::"memory");                  // (keeps this ONE branch, out of the common path, rows and all)
 #pragma unroll
-      for (int i = 0; i < 16; i++) {
-        const int j = i < 8 ? (i < AE_L1 ? i : 0) : (i - 8 < AE_L2 ? AE_L1 + i - 8 : AE_L1);
-        const int row = ((blk0 + j) * 64 + ln) / AE_CPR;
+      for (int i = 0; i < AE_LOADS; i++) {
+        const int row = ((blk0 + i) * 64 + ln) / AE_CPR;
         int over = kv0 + row - (seqlen_b - 1);
         over = over > 0 ? over : 0;                           // <= row: the offset stays >= 0
-        const unsigned back = (unsigned)(over * stride1);
-        if (i < 8) o1[i] -= back;
-        else o2[i - 8] -= back;
+        o[i] -= (unsigned)(over * stride1);
       }
     }
-    ae_load_lds16_burst_base<AE_L1>(tile, o1, dst + (blk0 + AE_L1 / 2) * 1024);
-    ae_load_lds16_burst_base<AE_L2>(tile, o2, dst + (blk0 + AE_L1 + AE_L2 / 2) * 1024);
-#else
-    const char* g1[8];
-    const char* g2[8];
+    auto burst = [&](auto which) AE_LAMBDA {
+      constexpr int LO = AE_LB(which.value), N = AE_LB(which.value + 1) - LO;
+      unsigned ob[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      g1[i] = ld_ptr[i < AE_L1 ? i : 0];
-      g2[i] = ld_ptr[i < AE_L2 ? AE_L1 + i : AE_L1];
-    }
+      for (int i = 0; i < 8; i++) ob[i] = o[LO + (i < N ? i : 0)];
+      ae_load_lds16_burst_base<N>(tile, ob, dst + (blk0 + LO + N / 2) * 1024);
+    };
+#else
+    const char* g[AE_LOADS];
+#pragma unroll
+    for (int i = 0; i < AE_LOADS; i++) g[i] = ld_ptr[i];
     if (__builtin_expect(ragged, 0)) {                        // rows past the end re-read the last row
       int ln = lane;
       asm volatile("" : "+v"(ln)::"memory");                  // (keeps this ONE branch, out of the common path, rows and all)
 #pragma unroll
-      for (int i = 0; i < 16; i++) {
-        const int j = i < 8 ? (i < AE_L1 ? i : 0) : (i - 8 < AE_L2 ? AE_L1 + i - 8 : AE_L1);
-        const int row = ((blk0 + j) * 64 + ln) / AE_CPR, cp = ((blk0 + j) * 64 + ln) % AE_CPR;
+      for (int i = 0; i < AE_LOADS; i++) {
+        const int row = ((blk0 + i) * 64 + ln) / AE_CPR, cp = ((blk0 + i) * 64 + ln) % AE_CPR;
         int over = kv0 + row - (seqlen_b - 1);
         over = over > 0 ? over : 0;
-        const int back = over * ((cp ^ AE_SWZ(row)) >= AE_CPR1 ? stride2 : stride1);
-        if (i < 8) g1[i] -= back;
-        else g2[i - 8] -= back;
+        g[i] -= over * ((cp ^ AE_SWZ(row)) >= AE_CPR1 ? stride2 : stride1);
       }
     }
-    ae_load_lds16_burst<AE_L1>((const void* const*)g1, dst + (blk0 + AE_L1 / 2) * 1024);
-    ae_load_lds16_burst<AE_L2>((const void* const*)g2, dst + (blk0 + AE_L1 + AE_L2 / 2) * 1024);
+    auto burst = [&](auto which) AE_LAMBDA {
+      constexpr int LO = AE_LB(which.value), N = AE_LB(which.value + 1) - LO;
+      const char* gb[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) gb[i] = g[LO + (i < N ? i : 0)];
+      ae_load_lds16_burst<N>((const void* const*)gb, dst + (blk0 + LO + N / 2) * 1024);
+    };
 #endif
+    burst(ae_const_int<0>());
+    burst(ae_const_int<1>());
+    if constexpr (AE_BURSTS == 3) burst(ae_const_int<2>());
 #if !AE_PAGED
 #pragma unroll
     for (int i = 0; i < AE_LOADS; i++) ld_ptr[i] += ld_adv[i];
@@ -681,18 +704,42 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     }
 #endif
   };
-  // end of a trip: tile t+2 has landed when only the newest request (tile t+3) is outstanding; after the barrier
-  // everyone is done with tile t, whose stage takes the next request
-  auto end_trip = [&](int t) AE_LAMBDA {
-    if (t + AE_NSTAGE - 1 < n_tiles) __builtin_amdgcn_s_waitcnt(AE_VMCNT_LGKM0(AE_LOADS));   // ... and this trip's LDS reads have returned
+  // end of trip n, in which the score waves multiplied tile n and the value waves read tile n - 1: tile n + 1 has landed when
+  // only the newest request (tile n + 2) is outstanding; after the barrier everyone is done with tile n - 1, whose stage
+  // takes the next request
+  auto end_trip = [&](int n) AE_LAMBDA {
+    if (n + 2 < n_tiles) __builtin_amdgcn_s_waitcnt(AE_VMCNT_LGKM0(AE_LOADS));   // ... and this trip's LDS reads have returned
     else __builtin_amdgcn_s_waitcnt(AE_VMCNT_LGKM0(0));     // (the last tile has been requested: nothing is newer)
     __syncthreads();
-    load_tile(t + AE_NSTAGE);
+    load_tile(n + 3);
   };
 
   __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
 #pragma unroll
-  for (int t = 0; t < AE_NSTAGE - 1; t++) load_tile(t);
+  for (int t = 0; t < 3; t++) load_tile(t);
+  if (n_tiles >= 3) __builtin_amdgcn_s_waitcnt(AE_VMCNT(2 * AE_LOADS));
+  else if (n_tiles == 2) __builtin_amdgcn_s_waitcnt(AE_VMCNT(AE_LOADS));
+  else __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
+#if AE_LOADER_WAVES
+    __syncthreads();
+    for (int n = 0; n <= n_tiles + 1; n++) end_trip(n);      // (the barriers of the value waves' trips)
+    return;
+  }
+  auto end_trip = [&](int) AE_LAMBDA {
+    __builtin_amdgcn_s_waitcnt(AE_VMCNT_LGKM0(63));            // (the trip's LDS reads have returned)
+    __syncthreads();
+  };
+#endif
+
+  // ============================== value wave: AE_DVW value columns, AE_HPW heads =======================
+#if AE_HPW == 64
+  const int lhd = lane & 31;       // the lane's head in a block of heads
+  const int hf = lane >> 5;        // ... and which part of the block's rows
+#else
+  const int lhd = lane & 15;
+  const int hf = lane >> 4;
+#endif
+  const int dvw = wave < 4 ? wave - 2 : wave - 4;   // waves 2, 3, 6, 7
 #if AE_HPW == 64
   typedef ae_f32x16 ae_acc;
 #else
@@ -706,9 +753,6 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     for (int db = 0; db < AE_NDB; db++)
 #pragma unroll
       for (int r = 0; r < NR; r++) oacc[hb][db][r] = 0.f;
-  if (n_tiles >= AE_NSTAGE - 1) __builtin_amdgcn_s_waitcnt(AE_VMCNT((AE_NSTAGE - 2) * AE_LOADS));
-  else if (n_tiles == 2) __builtin_amdgcn_s_waitcnt(AE_VMCNT(AE_LOADS));
-  else __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
   __syncthreads();
 #if AE_CLOCK_STAMPS
   const unsigned long long ae_w1 = __builtin_amdgcn_s_memrealtime();     // tile 0 (and Q) have landed
@@ -820,16 +864,16 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  end_trip(-1);                                                    // trip 0: the score waves multiply tile 0
+  end_trip(0);                                                     // trip 0: the score waves multiply tile 0
   value_trip(1, ae_const_bool<false>(), ae_const_bool<true>());    // trip 1: fragments of tile 0
-  end_trip(0);
+  end_trip(1);
   for (int n = 2; n <= n_tiles; n++) {
     value_trip(n, ae_const_bool<true>(), ae_const_bool<true>());
-    end_trip(n - 1);
+    end_trip(n);
   }
   if (n_tiles > 0) {                                               // trip n_tiles + 1: the last tile's product
     value_trip(n_tiles + 1, ae_const_bool<true>(), ae_const_bool<false>());
-    end_trip(n_tiles);
+    end_trip(n_tiles + 1);
   }
   __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));   // (the last barrier also made the final (m, r) of every head visible)
 #if AE_CLOCK_STAMPS

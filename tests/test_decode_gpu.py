@@ -424,6 +424,37 @@ def test_mla_decode_paged_cache(cuda_device, monkeypatch, kernel, dtype, B, H, p
     assert (out2[:, 0].float().cpu() - ref).abs().max().item() <= OUT_TOL
 
 
+@pytest.mark.parametrize("dtype,H,page,n_split,lens", [
+    (torch.bfloat16, 16, 32, 1, [1, 32, 33, 64, 65, 96, 97, 128, 129, 161]),     # one to six tiles, one page each
+    (torch.float16, 40, 64, 2, [0, 320, 161, 160, 129, 31]),                     # dead heads; second splits of 0 to 5 tiles
+    (torch.bfloat16, 16, 128, 3, [2500, 833, 1, 1664]),                          # 27 tiles a split through the stage ring
+])
+def test_paged_cache_with_16_heads_a_workgroup(cuda_device, dtype, H, page, n_split, lens):
+    """The tiles are requested by waves of their own (AE_LOADER_WAVES): every count of tiles around the three that are
+    requested ahead, lengths that end inside a tile."""
+    print(f"case mla paged 16 heads {dtype} H{H} page{page} splits{n_split} lens{lens}", flush=True)
+    B, D, DV, scale = len(lens), 576, 512, 1 / math.sqrt(576)
+    max_pages = -(-max(lens) // page)
+    q, q_pe, kv, k_pe = _mla_inputs(B, H, 1, max_pages * page, DV, D - DV, dtype, seed=6)
+    order = torch.randperm(B * max_pages, generator=torch.Generator().manual_seed(3))
+    cache = torch.empty((B * max_pages, page, 1, D), dtype=dtype)
+    cache[order] = torch.cat([kv, k_pe], -1).reshape(-1, page, 1, D)
+    mod = _mla_engine(B, H, 1, max_pages * page, D, DV, dtype, scale, backend="cute")
+    tiles = max_pages * page // 32
+    mod.attention.plan = lambda *a, **k: (16, n_split, -(-tiles // n_split) * 32)
+    args = (torch.cat([q, q_pe], -1).cuda(), cache.cuda())
+    pages = dict(block_table=order.view(B, max_pages).to(torch.int32).cuda(), cache_seqlens=torch.tensor(lens, dtype=torch.int32).cuda())
+    for _ in range(2):                        # through Python, then through the native host path
+        out, lse = mod(*args, **pages)
+        for b, n in enumerate(lens):
+            if n == 0:
+                assert (out[b] == 0).all() and (lse[b] == float("-inf")).all()
+                continue
+            ref, lref = R.mla_decode(q[b:b + 1, 0], q_pe[b:b + 1, 0], kv[b:b + 1, :n], k_pe[b:b + 1, :n], scale=scale)
+            assert (out[b:b + 1, 0].float().cpu() - ref).abs().max().item() <= OUT_TOL, b
+            assert (lse[b:b + 1, :, 0].cpu() - lref).abs().max().item() <= LSE_TOL, b
+
+
 def test_decode_split_counts_are_tuned_and_recorded(cuda_device, tmp_path):
     """tune=True for the decode engines (the reference tunes num_split whenever it builds the MLA decode kernel,
     mla_decode_tl.py:13-24, 308-319): the first call of a shape measures the planned split count, its half and its
