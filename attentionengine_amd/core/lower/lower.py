@@ -859,7 +859,7 @@ def render_config(d: int, dv: int, dtype, tiles: PrefillTiles, mask_mode: int, h
         f"#define AE_WAVES_PER_EU {tiles.waves_per_eu}",
         f"#define AE_K_PAD {tiles.k_pad}",
         f"#define AE_V_PAD {tiles.v_pad}",
-        *([f"#define AE_KV_STAGES {tiles.kv_stages}"] if tiles.template == "ae_prefill_pipe.hip" else []),
+        *([f"#define AE_KV_STAGES {tiles.kv_stages}"] if tiles.template == "ae_prefill_pipe.hip" or tiles.kv_stages > 2 else []),
         # (measurement switch of the pipelined kernel: the order of a causal launch's workgroups)
         *([f"#define AE_CAUSAL_ORDER {os.environ['AE_CAUSAL_ORDER']}"]
           if tiles.template == "ae_prefill_pipe.hip" and os.environ.get("AE_CAUSAL_ORDER", "") in ("0", "1") else []),

@@ -225,7 +225,7 @@ class PrefillOp:
         return True
 
     def _compile_declared_shape(self, B, H, Sq, Skv, infer_mask, mask_mod):
-        tiles = self.tiles_for(B, H, Sq, Skv)
+        tiles = self._launch_tiles(B, H, Sq, Skv, self.tiles_for(B, H, Sq, Skv))
         plan = self._plan(B, H, Sq, Skv, device=None, tiles=tiles)
         mode = 2 if self.extern_block_mask else plan.mode
         n_split, _ = self.plan_splits(B, H, Sq, Skv, tiles)
@@ -264,11 +264,9 @@ class PrefillOp:
         allow and want them: a merge the kernel knows (the proven online softmax, or no row state), no mask table, no
         tensor read per score."""
         wide = (self.D, self.DV) == (192, 128)          # (measured for causal softmax only)
-        if (not (B and H and Sq and Skv) or self.extern_block_mask
-                or not (wide or (self.D in (64, 128) and self.DV in (64, 128)))
+        if (not (B and H and Sq and Skv) or not (wide or (self.D in (64, 128) and self.DV in (64, 128)))
                 or (wide and (self.mask_mod is None or self._pipe_softmax is None or self.split_kv))
-                or not (self._pipe_softmax is not None or self._pipe_elementwise)
-                or any(c.per_kv for c in self.functors.customs) or os.environ.get("AE_PREFILL_KERNEL", "")):
+                or not self._groups_can_meet()):
             return None
         if self.split_kv:
             return L.kv_group_tiles_split(Sq, B * H) if self.mask_mod is None else None
@@ -289,6 +287,11 @@ class PrefillOp:
             if not (plan.mode == 1 or (plan.band is not None and not wide)):
                 return None
         return found
+
+    def _groups_can_meet(self):
+        """Whether this engine's graph lets waves share the kv axis, and nothing asks for another kernel."""
+        return not (self.extern_block_mask or not (self._pipe_softmax is not None or self._pipe_elementwise)
+                    or any(c.per_kv for c in self.functors.customs) or os.environ.get("AE_PREFILL_KERNEL", ""))
 
     def tiles_for(self, B, H, Sq, Skv):
         """The tile configuration of a call with these extents."""
@@ -397,6 +400,64 @@ class PrefillOp:
     # ---- kernels -------------------------------------------------------------------------
     COMBINE_THREADS = 128
 
+    # Head dim 128: tiles of a split launch whose workgroups have a CU each.  Three stages keep two tiles on their way while one
+    # is multiplied; with two, what is on its way drains at the end of every trip (not where eight waves multiply for 1.4 us:
+    # B7 H16 Sq192 Skv12126 199.9 us, 201.1 with three).  name -> (tiles, microseconds of a
+    # workgroup's start and end, of a trip over its kv groups' next tiles)
+    SPLIT_FORMS = {"32": (dict(n_waves=1, kv_groups=2, block_n=32, kv_stages=3), 3.14, 0.69),
+                   "64": (dict(n_waves=2, kv_groups=2, block_n=32, kv_stages=3), 3.2, 0.72),
+                   "128": (dict(kv_stages=3), 3.3, 1.0),
+                   "256": (dict(n_waves=8), 3.3, 1.43)}
+
+    def _launch_tiles(self, B, H, Sq, Skv, tiles):
+        """The tiles of a split launch with these extents: those of ``SPLIT_FORMS`` that cost least instead of ``tiles``
+        (``tiles_for``), where the graph allows them.  Not at other head dims, nor where 128- or 256-row tiles fill the chip
+        without a split (two workgroups a CU then hide each other's waits: B10 H32 Sq108 Skv2102 79 us, 92 with three stages)."""
+        if (not self.split_kv or self.mask_mod is not None or (self.D, self.DV) != (128, 128) or self._tiles_given
+                or not (B and H and Sq and Skv) or Sq > 256 or (Sq > 64 and -(-(B * H) // 8) * 8 > self.target_workgroups)
+                or not self._groups_can_meet()):
+            return tiles
+        names = ("32",) if Sq <= 32 else ("64",) if Sq <= 64 else ("64", "128", "256")
+        return L.PrefillTiles(**self.SPLIT_FORMS[self._cheapest_form(names, B * H, Sq, -(-Skv // 32), self.target_workgroups)[0]][0])
+
+    def _split_form_of(self, tiles):
+        """The name in ``SPLIT_FORMS`` of tiles that ``_launch_tiles`` chose, or None."""
+        if (self.D, self.DV) != (128, 128):
+            return None
+        return next((n for n, f in self.SPLIT_FORMS.items() if tiles == L.PrefillTiles(**f[0])), None)
+
+    @classmethod
+    @functools.lru_cache(maxsize=1024)
+    def _cheapest_form(cls, names, heads, rows, kv_tiles, cus):
+        """(tiles, splits) of a split launch at head dim 128 that takes least time, ``kv_tiles`` counted in 32 keys.  Every CU has
+        one workgroup at a time, so a launch takes whole rounds of starts and trips; the cache arrives at 6.4 TB/s; partial
+        results are written and merged.  Fitted to 1000 timings of 94 shapes (batch 1 to 8, 8 to 32 heads, 1 to 256 rows, 512
+        to 16384 keys, bf16), 3.6 % off in the root mean square; the choice is 0.6 % off the best measured on average and
+        takes 0.93 of the time of two stages with a split for every CU (1.05 at most).  us: B6 H32 Sq50 Skv2562 60 -> 51,
+        B8 H8 Sq115 Skv521 15.9 -> 12.2, B1 H16 Sq4 Skv8393 20.7 -> 19.2, B5 H32 Sq216 Skv3498 112 -> 99, B1 H32 Sq128 Skv8192
+        42.2 -> 39.4; B5 H32 Sq61 Skv15254 232 -> 244."""
+        read = heads * kv_tiles * 32 * 512e-6 / 6.4
+        best = []
+        for name in names:
+            tiles, start, trip = cls.SPLIT_FORMS[name]
+            tiles = L.PrefillTiles(**tiles)
+            n = -(-kv_tiles * 32 // tiles.block_n)
+            wgs = -(-rows // tiles.block_m) * (-(-heads // 8) * 8)
+            for x in range(1, min(64, n) + 1):
+                if x > 1 and wgs * x > 4 * cus:
+                    break
+                per = -(-n // x)
+                if -(-n // per) != x:
+                    continue
+                body = -(-wgs * x // cus) * (start + trip * -(-per // tiles.kv_groups))
+                us = (body ** 2.25 + read ** 2.25) ** (1 / 2.25)
+                if x > 1:
+                    us += 1.8 + 0.047 * x + 0.42 * heads * rows * x * 512e-6
+                best.append((us, x, name))
+        least = min(best)[0]
+        _, x, name = min((b for b in best if b[0] <= 1.01 * least), key=lambda b: (b[1], b[0]))
+        return name, x
+
     # microseconds of a workgroup's start and end, and of a trip over its kv groups' next tiles, by the rows of its q tile
     SPLIT_COST = {32: (3.0, 0.92), 64: (1.8, 0.66), 128: (1.3, 0.91), 256: (5.2, 1.39)}
     # head dim 64: (start and end, trip, what a trip takes of each workgroup that shares the CU, workgroups a CU holds)
@@ -465,12 +526,17 @@ class PrefillOp:
         """(number of KV splits, kv positions per split): a workgroup for every CU of the chip (more splits cost
         more in partial results and their merge than they gain: B1 H32 Sq128 Skv8192, the shape of
         attn_script/mha_inference.py, 43 us with 8 splits, 44 with 16, 75 with 32), whole kv tiles per split, no
-        empty split.  Where that leaves some CUs with two workgroups the cheapest count is taken (``_cheapest_splits``)."""
+        empty split.  Where that leaves some CUs with two workgroups the cheapest count is taken (``_cheapest_splits``), and
+        always for the tiles that are chosen with it (``_launch_tiles``)."""
         if not self.split_kv:
             return 1, Skv
         tiles = tiles or self.tiles_for(B, Hq, Sq, Skv)
         bn = tiles.block_n
         kv_tiles = -(-Skv // bn)
+        form = self._split_form_of(tiles)
+        if form:
+            x = self._cheapest_form((form,), B * Hq, Sq, -(-Skv // 32), self.target_workgroups)[1]
+            return x, -(-kv_tiles // x) * bn
         wgs = -(-Sq // tiles.block_m) * (-(-(B * Hq) // 8) * 8)
         want = max(1, min(kv_tiles, -(-self.target_workgroups // wgs)))
         per = -(-kv_tiles // want)
@@ -673,6 +739,7 @@ class PrefillOp:
             table = table.to(dev).contiguous()
             mode, mbm, mbn, band = 2, bm, bn, None
         else:
+            tiles = self._launch_tiles(B, Hq, Sq, Skv, tiles)
             plan = self._plan(B, Hq, Sq, Skv, dev, tiles)
             mode, table, mbm, mbn, band = plan.mode, plan.table, plan.block_m, plan.block_n, self._band(plan, tiles)
         n_split, kv_per_split = self.plan_splits(B, Hq, Sq, Skv, tiles)

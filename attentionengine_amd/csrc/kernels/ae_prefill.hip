@@ -96,6 +96,17 @@
 #define AE_KW_SOFTMAX 0
 #endif
 
+// K / V tiles in LDS.  2: tile j + 1 is requested at the start of trip j and waited for at its end.  3 (split launches at head
+// dim 128, a workgroup a CU): tile j + 2 is, into the stage of tile j - 1, and the wait at the end is for tile j + 1 alone.  Such
+// a launch is bound by the cache's bytes, and with two stages nothing is on its way from the last byte's arrival until the
+// next trip.  us: B1 H32 Sq128 Skv8192 42.2 -> 39.4, B3 H32 Sq48 Skv5012 62.7 -> 52.5, B3 H32 Sq3 Skv1218 18.8 -> 17.3 (four
+// stages 40.7, 53.3, 18.2).  Not where the workgroups share CUs: a sliding window B2 H32 S4096 D128 75.5 -> 74.9 (four 80.7),
+// causal 192 / 128 columns 293 -> 322 (two workgroups a CU instead of three).
+#ifndef AE_KV_STAGES
+#define AE_KV_STAGES 2
+#endif
+#define AE_DEEP (AE_KV_STAGES == 3)
+
 // value given to score positions past seqlen_kv before the user functors run: -inf, or 0 for graphs
 // declared with mask_value="0" (no additive -inf mask anywhere, attn_tl.py:124-137 / lower.py:637)
 #if defined(AE_MASK_VALUE_ZERO) && AE_MASK_VALUE_ZERO
@@ -130,6 +141,7 @@
 constexpr int ae_floor_div(int a, int b) { return a >= 0 ? a / b : -((b - 1 - a) / b); }
 #define AE_PERIOD (ae_floor_div(AE_BM - 1 - (AE_BAND_LO), AE_BN) - ae_floor_div(-(AE_BAND_HI), AE_BN) + 1)
 #endif
+#define AE_VMCNT(n) (0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
 #define AE_NS (AE_NB * 16)        // score elements per lane per tile
 #define AE_NDB (AE_DV / 32)       // 32-wide dv blocks
 #define AE_NO (AE_NDB * 16)       // output elements per lane
@@ -155,6 +167,7 @@ static_assert((AE_BN * AE_KCPR) % AE_GT == 0, "K tile must split evenly over the
 static_assert((AE_BN * AE_VCPR) % AE_GT == 0, "V tile must split evenly over the waves that load it");
 static_assert(AE_KW == 1 || (AE_MASK_MODE != 2 && AE_RB == 1 && AE_NO % (4 * AE_KW) == 0 && AE_WAVES_PER_EU >= 2),
               "kv groups: 32 rows a wave, no tile table, a whole number of 4-column pieces of O per group");
+static_assert(AE_KV_STAGES == 2 || (AE_DEEP && AE_MASK_MODE == 0), "two or three stages; tiles requested ahead follow one another");
 static_assert(AE_K_LOADS >= 1 && AE_K_LOADS <= 8 && AE_V_LOADS >= 1 && AE_V_LOADS <= 8, "one burst per tile and wave");
 static_assert(AE_KCPR == 8 || AE_KCPR == 16 || AE_KCPR == 32 || AE_KCPR % 8 == 4 || AE_KCPR % 16 == 8,
               "swizzle is written for K rows of 128, 256 or 512 bytes, or an odd multiple of 64 or 128 bytes");
@@ -198,7 +211,7 @@ AE_DEV int ae_k_swz(int c, int row) {
 // A lane that loads its own row's fragments, or stores its own row's results, touches 32 rows per instruction,
 // 16 bytes of each: the workgroups of a launch start and end together and queue behind each other's requests
 // (measured in the pipelined kernel: 3.5 us until the first tile could be multiplied, 4.4 us to get O out).
-// Q uses stage 1 of the tile ring, which is free until the loop's first prefetch, swizzled like a K tile; O the
+// Q uses the last stage of the tile ring, which is free until the loop's first prefetch, swizzled like a K tile; O the
 // whole ring after the last tile.  Builds whose rows do not fit there keep the direct accesses.
 #define AE_Q_LOADS ((AE_WROWS * AE_KCPR) / 64)     // direct loads per lane for the wave's Q rows
 #define AE_Q_VIA_LDS (AE_BM * AE_KSTR <= AE_STAGE_BYTES)
@@ -239,7 +252,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
   const int wave_wg = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kg = wave_wg / AE_NWAVES;         // kv group
   const int wave = wave_wg % AE_NWAVES;       // ... and which 32 rows
-  ae_lds_byte* lds = (ae_lds_byte*)ae_smem + kg * (2 * AE_STAGE_BYTES);
+  ae_lds_byte* lds = (ae_lds_byte*)ae_smem + kg * (AE_KV_STAGES * AE_STAGE_BYTES);
 #endif
   const int l32 = lane & 31;
   const int hf = lane >> 5;
@@ -303,7 +316,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
   // ---- Q fragments: B operand of S^T = K Q^T, resident for the whole kernel -------------
   ae_elem8 qf[AE_RB][AE_D / 16];
 #if AE_Q_VIA_LDS
-  ae_lds_byte* qs = lds + AE_STAGE_BYTES + wave * (AE_WROWS * AE_KSTR);
+  ae_lds_byte* qs = lds + (AE_KV_STAGES - 1) * AE_STAGE_BYTES + wave * (AE_WROWS * AE_KSTR);
   {
     const int q0c = q0w < p.seqlen_q ? q0w : p.seqlen_q - 1;
     const char* qg = (const char*)((const ae_elem*)p.q + (int64_t)b * p.q_stride_b + (int64_t)q0c * p.q_stride_s +
@@ -462,8 +475,23 @@ void ae_prefill_kernel(const ae_attn_params p) {
   const int j_trips = j_end;
 #define AE_J_LIVE true
 #endif
+#if AE_DEEP
+  int rq_j = j, rq_stage = 0;          // the group's next tile to request, and the stage it goes into
+  auto request_next = [&]() AE_LAMBDA {
+    if (rq_j < j_end) load_tile(rq_j, rq_stage);
+    rq_j += AE_KW;
+    rq_stage = rq_stage == 2 ? 0 : rq_stage + 1;
+  };
+  // tile jt has landed: the one behind it, if there is one, is the only one outstanding
+  auto wait_tile = [&](int jt) AE_LAMBDA {
+    if (jt + AE_KW < j_end) __builtin_amdgcn_s_waitcnt(AE_VMCNT(AE_K_LOADS + AE_V_LOADS));
+    else __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
+  };
+#endif
 #if AE_ROTATE
   int left = j_end - j_first;          // tiles still to be multiplied
+#endif
+#if AE_ROTATE
 #define AE_TRIPS_LEFT (left > 0)
 #define AE_HAS_NEXT (left > 1)
 #else
@@ -479,7 +507,9 @@ void ae_prefill_kernel(const ae_attn_params p) {
   for (int rb = 0; rb < AE_RB; rb++) seen[rb] = 0.f;
 #pragma unroll
   for (int rb = 0; rb < AE_RB; rb++) cls[rb] = row_class(j, rb);
+#if !AE_DEEP
   if (any_tile && AE_J_LIVE) load_tile(j, 0);
+#endif
 #ifdef AE_HAS_KV_PREFETCH
   if (any_tile) {
 #pragma unroll
@@ -489,7 +519,14 @@ void ae_prefill_kernel(const ae_attn_params p) {
   // Drain every outstanding load (Q fragments, first tile) before the loop: with loads still
   // pending at the loop header the compiler's wait-count insertion makes the QK^T MFMAs of every
   // iteration wait for that iteration's K/V prefetch, which serialises the pipeline.
+#if AE_DEEP
+  __builtin_amdgcn_s_waitcnt(0xc07f);            // lgkmcnt(0); the Q rows and the first tile are waited for together
+  request_next();
+  request_next();
+  wait_tile(j);
+#else
   __builtin_amdgcn_s_waitcnt(0);
+#endif
   __syncthreads();
 #if AE_Q_VIA_LDS
 #pragma unroll
@@ -498,7 +535,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
     for (int ks = 0; ks < AE_D / 16; ks++)
       qf[rb][ks] = *(const __attribute__((address_space(3))) ae_elem8*)(
           qs + (rb * 32 + l32) * AE_KSTR + (ae_k_swz(2 * ks + hf, l32) << 4));
-  __syncthreads();      // every wave has its fragments before the loop's first prefetch refills stage 1
+  __syncthreads();      // every wave has its fragments before the next request refills the rows' stages
 #endif
 
   int stage = 0;
@@ -511,7 +548,11 @@ void ae_prefill_kernel(const ae_attn_params p) {
     int cls_n[AE_RB];
 #pragma unroll
     for (int rb = 0; rb < AE_RB; rb++) cls_n[rb] = row_class(jn, rb);
+#if AE_DEEP
+    request_next();                              // into the stage that the last trip left
+#else
     if (AE_HAS_NEXT) load_tile(jn, stage ^ 1);   // streams into the other stage while this one is used
+#endif
 
     ae_lds_byte* ks_ = lds + stage * AE_STAGE_BYTES;
     ae_lds_byte* vs_ = ks_ + AE_K_BYTES;
@@ -645,7 +686,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
       // ---- user functors ----------------------------------------------------------------------
 #if defined(AE_HAS_KV_PREFETCH) && AE_KV_COALESCED
       // per-score custom inputs: from the coalesced layout they were fetched in to the lanes that own them
-      ae_stage_custom(cust[rb], lds + 2 * AE_STAGE_BYTES + (wave * AE_RB + rb) * AE_KV_SCRATCH);
+      ae_stage_custom(cust[rb], lds + AE_KV_STAGES * AE_STAGE_BYTES + (wave * AE_RB + rb) * AE_KV_SCRATCH);
 #endif
       ae_score_mod<AE_NS>(s, ctx[rb], cust[rb]);
       float o_scale = ae_online_fwd<AE_NS>(s, st[rb], ctx[rb], cust[rb]);
@@ -726,9 +767,15 @@ void ae_prefill_kernel(const ae_attn_params p) {
     }
 
     // the next tile must have landed before anyone reads it: direct loads are tracked by vmcnt
+#if AE_DEEP
+    wait_tile(j + AE_KW);
+    __syncthreads();
+    stage = stage == 2 ? 0 : stage + 1;
+#else
     __builtin_amdgcn_s_waitcnt(0x0070 | 0x0f00 | 0x0000);  // vmcnt(0), expcnt/lgkmcnt untouched
     __syncthreads();
     stage ^= 1;
+#endif
     j = jn;
 #if AE_ROTATE
     left--;

@@ -237,3 +237,46 @@ def test_an_engine_for_short_prompts_at_other_lengths(cuda_device):
     assert (out - ref).abs().max().item() <= 2e-2
     assert op.tiles == TILES[1]
     check(333)
+
+
+def test_split_launches_take_the_cheapest_tiles():
+    """Head dim 128: tiles and splits of a launch by one cost, splits that cover the cache with none empty; other engines
+    and launches that fill the chip keep the tiles they had."""
+    op = _engine(8, None, H=8, Hkv=8, Skv=4096)._op
+    for B, H in ((1, 8), (3, 16), (7, 32), (40, 32)):
+        for Sq in (1, 32, 33, 64, 65, 128, 129, 256, 257):
+            for Skv in (1, 31, 33, 522, 16001):
+                own = op.tiles_for(B, H, Sq, Skv)
+                tiles = op._launch_tiles(B, H, Sq, Skv, own)
+                n, per = op.plan_splits(B, H, Sq, Skv, tiles)
+                assert per % tiles.block_n == 0 and n * per >= Skv > (n - 1) * per
+                assert tiles.lds_bytes(128, 128) <= 160 * 1024
+                assert (Sq <= 256 and (Sq <= 64 or B * H <= 256)) or tiles == own
+    three = [PrefillTiles(**f[0]) for f in op.SPLIT_FORMS.values()]
+    assert op._launch_tiles(1, 8, 8, 4096, None) == three[0] and op._launch_tiles(1, 8, 64, 4096, None) == three[1]
+    assert op._launch_tiles(1, 32, 128, 8192, None) == three[2] and op._launch_tiles(5, 32, 216, 3498, None) == three[3]
+    assert op._launch_tiles(8, 8, 115, 521, None) == three[1]                    # 128 workgroups, not three splits of 64
+    narrow = _engine(8, None, H=8, Hkv=8, Skv=4096, D=64)._op
+    assert narrow._launch_tiles(1, 8, 8, 4096, TILES[0]) == TILES[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["32", "64", "128", "256"])
+@pytest.mark.parametrize("Sq", [1, 33, 128, 150])
+def test_three_tile_stages(cuda_device, form, Sq):
+    """AE_KV_STAGES 3: none to seven tiles of a kv group, ragged last tiles, with and without a split; through Python, then
+    natively."""
+    B, H, D, dtype = 2, 3, 128, torch.float16
+    for Skv, n in ((1, 1), (31, 1), (33, 1), (64, 1), (65, 2), (129, 1), (200, 1), (300, 2), (449, 1), (700, 3)):
+        print(f"case three stages {form} Sq{Sq} Skv{Skv} splits {n}", flush=True)
+        q, k, v = C.make_inputs(B, Sq, Skv, H, H, D, D, dtype, seed=Skv)
+        op = _engine(Sq, None, H=H, Hkv=H, B=B, Skv=4096, dtype=dtype)._op
+        assert op.split_kv
+        tiles = PrefillTiles(**op.SPLIT_FORMS[form][0])
+        op._launch_tiles = lambda *a: tiles
+        op.plan_splits = lambda *a: (n, -(-Skv // (64 * n)) * 64)
+        ref, lse = R.softmax_attention(q, k, v, causal=False)
+        for _ in range(2):
+            out = op(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+            assert (out - ref).abs().max().item() <= 2e-2
+            assert (op.final_rowscales["lse"].cpu() - lse).abs().max().item() <= 1e-3
