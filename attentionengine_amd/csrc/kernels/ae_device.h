@@ -245,7 +245,7 @@ AE_DEV float ae_row_max(const float (&s)[N]) {
   return ae_group_max(m);
 }
 template <int N>
-AE_DEV float ae_row_sum(const float (&s)[N]) {
+AE_DEV float ae_lane_sum(const float (&s)[N]) {
   // four independent chains keep the adds off one dependency path
   float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
 #pragma unroll
@@ -257,7 +257,11 @@ AE_DEV float ae_row_sum(const float (&s)[N]) {
   }
 #pragma unroll
   for (int e = N & ~3; e < N; e++) a0 += s[e];
-  return ae_group_sum((a0 + a1) + (a2 + a3));
+  return (a0 + a1) + (a2 + a3);
+}
+template <int N>
+AE_DEV float ae_row_sum(const float (&s)[N]) {
+  return ae_group_sum(ae_lane_sum<N>(s));
 }
 template <int N>
 AE_DEV float ae_row_abssum(const float (&s)[N]) {

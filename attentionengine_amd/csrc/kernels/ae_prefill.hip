@@ -132,6 +132,21 @@
 #ifndef AE_RB
 #define AE_RB 1
 #endif
+// AE_SUM_CHECK 1 (the proven online softmax of score * AE_SM_SCALE, fields AE_SM_M and AE_SM_R): no row maxima in the common
+// trip.  The reference that the exponents are taken against may lag behind the running maximum as long as the weights fit
+// their type, and a weight that does not shows in the sum of its lane's weights, which is needed anyway: sums up to
+// AE_SUM_MOST go on; after a larger one (or a NaN) the wave makes the trip again - the tile is still in LDS, it requests
+// nothing and waits for nobody - and takes the maxima, as it does on its first tiles, until every row has a reference.  The
+// row sum stays per lane until the end.  These kernels are bound by the VALU at head dim 64 (70 % busy, 11.6 instructions an
+// MFMA): a tile's 32 scores of a lane take 132 VALU instructions instead of 160, row maxima and (below) addresses
+// together.  us: bf16 B16 H16 S1000 D64 85.8 -> 83.2, causal B2 H32/8 S3407 D64 115.7 -> 111.2, B17 H32 S577 75.5 -> 73.6,
+// window of 256, B2 H32 S4096 D128 fp16 75.5 -> 74.1; causal D128 0 to 1 %.
+// (As a way back inside the trip instead of a trip of its own, the compiler keeps 20 registers more through all of it.)
+#ifndef AE_SUM_CHECK
+#define AE_SUM_CHECK 0
+#endif
+#define AE_SUM_MOST 32768.f        // (half of what fp16 holds)
+#define AE_SM_TAU 5.545177444479562f     // the reference moves when a maximum exceeds it by 8 log2 units
 #define AE_WROWS (AE_RB * 32)     // query rows per wave
 #define AE_BM (AE_NWAVES * AE_WROWS)
 #define AE_GT (AE_NWAVES * 64)     // threads of a kv group
@@ -155,6 +170,7 @@ constexpr int ae_floor_div(int a, int b) { return a >= 0 ? a / b : -((b - 1 - a)
 #define AE_K_LOADS ((AE_BN * AE_KCPR) / AE_GT)   // direct loads per lane per K tile
 #define AE_V_LOADS ((AE_BN * AE_VCPR) / AE_GT)
 #define AE_V_RPI (64 / AE_VCPR)
+#define AE_KGRP ((AE_KCPR & (AE_KCPR - 1)) == 0 ? AE_KCPR : (AE_KCPR % 16 == 8 ? 8 : 4))    // chunks that ae_k_swz exchanges
 #define AE_VPPR (AE_VCPR / 2)     // 32-byte pairs per V row
 // the pairs of a V row are exchanged by the row's low bits: at most three of them, so that rows 8 apart (the
 // two halves of a transposed fragment) share one permutation whatever the row length
@@ -193,11 +209,14 @@ AE_DEV int ae_k_swz(int c, int row) {
 }
 
 // Fragments that a wave reads from LDS ahead of the MFMA that takes them: rings with one scheduling fence per MFMA (left
-// to itself the compiler keeps one or two reads in flight and waits for each).  Not where the head is so wide that
-// the ring's registers cost a wave per SIMD (D 192, DV 128, 32-key tiles: 168 -> 180 registers, 294 -> 313 us), nor in
-// the builds that run one wave per SIMD with every register taken.  bf16, without a mask, B16 H16 S1000: D 64 90.0 ->
-// 88.2 us, D 128 160.3 -> 155.6 us (with the shorter epilogue); causal B8 H32 S1000 D128 112.3 -> 110.0 us.
-#if AE_D <= 128 && AE_DV <= 128 && AE_RB == 1
+// to itself the compiler keeps one or two reads in flight and waits for each).  Not in the builds that run one wave per SIMD
+// with every register taken.  bf16, without a mask, B16 H16 S1000: D 64 90.0 -> 88.2 us, D 128 160.3 -> 155.6 us (with the
+// shorter epilogue); causal B8 H32 S1000 D128 112.3 -> 110.0 us.  At D 192, DV 128 the rings have cost a wave per SIMD (180
+// registers, 294 -> 313 us); without row maxima and with fragment addresses by constants 168 suffice: B1 H128 S2500 299.6 ->
+// 290.0, B1 H16 S8088 345 -> 329, B2 H32 S1968 105.9 -> 101.5, B1 H32 S570 16.5 -> 15.8, B3 H16 S789 26.7 -> 27.1 (rings of
+// two and two, three and three, six and three fragments: 289.8, 291.0, 305.7 for the first; none 280 to 288 there, 44.7
+// against 42.8 for B2 H32 S1098).
+#if (AE_D <= 128 || AE_D == 192) && AE_DV <= 128 && AE_RB == 1
 #define AE_K_AHEAD 4
 #define AE_V_AHEAD 3
 #define AE_RING_FENCE() __builtin_amdgcn_sched_barrier(0)
@@ -242,7 +261,7 @@ AE_DEV void ae_q_rows_to_lds(const char* qg, ae_lds_byte* qs, int lane, int row0
 extern "C" __global__ __launch_bounds__(AE_NT)
 __attribute__((amdgpu_waves_per_eu(AE_WAVES_PER_EU)))
 void ae_prefill_kernel(const ae_attn_params p) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char ae_smem[];
+  extern __shared__ __attribute__((aligned(1024))) unsigned char ae_smem[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
 #if AE_KW == 1
@@ -435,15 +454,18 @@ void ae_prefill_kernel(const ae_attn_params p) {
       for (int r = 0; r < 16; r++) oacc[rb][db][r] = 0.f;
   }
 
-  // lane-constant pieces of the swizzled LDS read addresses
-  // K fragment (row l32 of a 32-row block, d chunk 2*ks+hf): chunk' = (2*ks+hf) ^ (l32 mod CPR)
-  const int k_row_off = l32 * AE_KSTR;
+  // Lane parts of the LDS read addresses.  The k-step and the column block only flip bits of the chunk (pair) index inside the
+  // group of chunks that the swizzle exchanges, and stages and rows start on multiples of it, so a fragment's address is
+  // ((stage + lane part) ^ constant) + immediate: an addition a tile and an instruction per constant.  (From the chunk
+  // positions as they are the compiler forms every address by additions: 35 of the 160 VALU instructions of a tile at head dim 64.)
+  // K fragment (row l32 of a 32-row block, d chunk 2*ks+hf): see ae_k_swz
+  const unsigned k_lane = (unsigned)(l32 * AE_KSTR + (ae_k_swz(hf, l32) << 4));
   // V transpose read: lane i of a 16-lane group reads row 4*hf + i/4 (+8), 8 bytes at pair
   // (2*db + g) ^ (row mod PPR), g = (lane%32)/16; rows of one group differ only in their low bits
   const int v_row = 4 * hf + ((lane & 15) >> 2);
-  const int v_row_off = v_row * AE_VSTR + (lane & 3) * 8;
-  const int v_sw = v_row & AE_VSWM;
-  const int v_g = l32 >> 4;
+  const unsigned v_lane = (unsigned)(v_row * AE_VSTR + (lane & 3) * 8 + (((l32 >> 4) ^ (v_row & AE_VSWM)) << 5));
+  static_assert(AE_STAGE_BYTES % (AE_KGRP * 16) == 0 && AE_K_BYTES % ((AE_VSWM + 1) * 32) == 0 && AE_KSTR % (AE_KGRP * 16) == 0 &&
+                AE_STAGE_BYTES % ((AE_VSWM + 1) * 32) == 0, "the exchanged bits of a stage's and a row's address are zero");
 
 #if AE_NSPLIT > 1
   // this workgroup's share of the kv axis: kv_per_split positions (a multiple of the tile)
@@ -538,6 +560,12 @@ void ae_prefill_kernel(const ae_attn_params p) {
   __syncthreads();      // every wave has its fragments before the next request refills the rows' stages
 #endif
 
+#if AE_SUM_CHECK
+  static_assert(AE_RB == 1 && AE_WAVES_PER_EU >= 2, "one row block a wave, O in ordinary registers");
+  bool by_maxima = true;      // (wave uniform) this trip takes the maxima: some row has no reference yet, or the sums were large
+  bool again = false; // ... the trip is made once more for them: nothing is requested, nobody is waited for
+  float minus_ref = 0.f;       // the lane's row's reference, log2 units, negative
+#endif
   int stage = 0;
   while (AE_TRIPS_LEFT) {
 #if AE_ROTATE
@@ -548,6 +576,9 @@ void ae_prefill_kernel(const ae_attn_params p) {
     int cls_n[AE_RB];
 #pragma unroll
     for (int rb = 0; rb < AE_RB; rb++) cls_n[rb] = row_class(jn, rb);
+#if AE_SUM_CHECK
+    if (__builtin_expect(!again, 1))
+#endif
 #if AE_DEEP
     request_next();                              // into the stage that the last trip left
 #else
@@ -589,9 +620,12 @@ void ae_prefill_kernel(const ae_attn_params p) {
       for (int nb = 0; nb < AE_NB; nb++)
 #pragma unroll
         for (int r = 0; r < 16; r++) sacc[rb][nb][r] = 0.f;
+    unsigned k_at = (unsigned)(unsigned long)ks_ + k_lane;
+    asm("" : "+v"(k_at));                        // (a value of its own: not rebuilt per read from its parts)
     auto k_frag = [&](int f) AE_LAMBDA -> ae_elem8 {
-      return *(__attribute__((address_space(3))) ae_elem8*)(
-          ks_ + k_row_off + f % AE_NB * 32 * AE_KSTR + (ae_k_swz(2 * (f / AE_NB) + hf, l32) << 4));
+      const int c = 2 * (f / AE_NB);
+      return *(const __attribute__((address_space(3))) ae_elem8*)(
+          (const ae_lds_byte*)(k_at ^ (unsigned)((c & (AE_KGRP - 1)) << 4)) + ((c & -AE_KGRP) << 4) + f % AE_NB * 32 * AE_KSTR);
     };
     constexpr int NKF = (AE_D / 16) * AE_NB;
     ae_elem8 kring[AE_K_AHEAD + 1];
@@ -615,8 +649,8 @@ void ae_prefill_kernel(const ae_attn_params p) {
       for (int nb = 0; nb < AE_NB; nb++)
 #pragma unroll
         for (int r = 0; r < 16; r++) s[nb * 16 + r] = sacc[rb][nb][r];
-      ctx[rb].kv_base = kv0 + 4 * hf;
-      const int kvb = ctx[rb].kv_base;
+      const int kvb = kv0 + 4 * hf;
+      ctx[rb].kv_base = kvb;
 
       // ---- mask (additive -inf before score_mod, attn_tl.py:124-137) --------------------------
 #if !AE_ANALYTIC
@@ -658,7 +692,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #if AE_PAD_SCORES          // (not causal over equal lengths: behind the diagonal of every row)
       if (kv0 + AE_BN > p.seqlen_kv) {
 #pragma unroll
-        for (int e = 0; e < AE_NS; e++) s[e] = (kvb + ae_kv_off(e) < p.seqlen_kv) ? s[e] : AE_KV_PAD;
+        for (int e = 0; e < AE_NS; e++) s[e] = ae_kv_off(e) < p.seqlen_kv - kvb ? s[e] : AE_KV_PAD;
       }
 #endif
 #if AE_ANALYTIC
@@ -683,6 +717,33 @@ void ae_prefill_kernel(const ae_attn_params p) {
       }
 #endif
 
+#if AE_SUM_CHECK
+      const bool took_maxima = by_maxima;
+      if (by_maxima) {
+        again = false;
+        const float top = ae_row_max<AE_NS>(s) * AE_SM_SCALE;
+        const float ref = top - st[rb].AE_SM_M > AE_SM_TAU ? top : st[rb].AE_SM_M;
+        const float o_scale = ae_exp(st[rb].AE_SM_M - ref);
+        minus_ref = -ref * AE_LOG2E;
+        st[rb].AE_SM_M = ref;
+        st[rb].AE_SM_R *= o_scale;
+        by_maxima = __builtin_amdgcn_ballot_w64(ref <= -1e30f) != 0;
+        if (__builtin_amdgcn_ballot_w64(o_scale != 1.0f) != 0) {
+#pragma unroll
+          for (int db = 0; db < AE_NDB; db++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) oacc[rb][db][r] *= o_scale;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < AE_NS; e++) s[e] = ae_exp2(__builtin_fmaf(s[e], AE_SM_SCALE * AE_LOG2E, minus_ref));
+      const float sum = ae_lane_sum<AE_NS>(s);
+      if (!took_maxima && __builtin_expect(__builtin_amdgcn_ballot_w64(!(sum <= AE_SUM_MOST)) != 0, 0)) {
+        by_maxima = again = true;
+      } else {
+        st[rb].AE_SM_R += sum;
+      }
+#else
       // ---- user functors ----------------------------------------------------------------------
 #if defined(AE_HAS_KV_PREFETCH) && AE_KV_COALESCED
       // per-score custom inputs: from the coalesced layout they were fetched in to the lanes that own them
@@ -690,6 +751,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #endif
       ae_score_mod<AE_NS>(s, ctx[rb], cust[rb]);
       float o_scale = ae_online_fwd<AE_NS>(s, st[rb], ctx[rb], cust[rb]);
+#endif
 #ifdef AE_HAS_KV_PREFETCH
       // the functors are done with this tile's elements of the per-score custom inputs: request the next
       // tile's, which travel while the second product runs
@@ -699,7 +761,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #if AE_PAD_WEIGHTS
       if (kv0 + AE_BN > p.seqlen_kv) {
 #pragma unroll
-        for (int e = 0; e < AE_NS; e++) s[e] = (kvb + ae_kv_off(e) < p.seqlen_kv) ? s[e] : 0.f;
+        for (int e = 0; e < AE_NS; e++) s[e] = ae_kv_off(e) < p.seqlen_kv - kvb ? s[e] : 0.f;
       }
 #endif
 
@@ -715,7 +777,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
           pf[rb][kk][t + 1] = y2[1];
         }
 
-#if !AE_O_SCALE_ONE
+#if !AE_O_SCALE_ONE && !AE_SUM_CHECK
       // skip the rescale when no row of this block changed its scale (wave-uniform branch)
       if (__builtin_amdgcn_ballot_w64(o_scale != 1.0f) != 0) {
 #pragma unroll
@@ -734,18 +796,25 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #endif
           }
       }
-#else
+#elif !AE_SUM_CHECK
       (void)o_scale;
 #endif
     }
 
     // ---- O^T += V^T P^T: every V fragment feeds one MFMA per row block ------------------------
+#if AE_SUM_CHECK
+    if (__builtin_expect(!again, 1))
+#endif
+    {
+    unsigned v_at = (unsigned)(unsigned long)vs_ + v_lane;
+    asm("" : "+v"(v_at));
     auto v_frag = [&](int f) AE_LAMBDA -> ae_elem8 {
       // slots 0..3 of k-step kk are kv rows rb0+4*hf+0..3, slots 4..7 rows rb0+8+4*hf+0..3
       // (rb0 and +8 are multiples of 8, so they do not change the swizzle)
       const int kk = f / AE_NDB;
       const int rb0 = (kk >> 1) * 32 + (kk & 1) * 16;
-      ae_lds_byte* a0 = vs_ + v_row_off + rb0 * AE_VSTR + (((2 * (f % AE_NDB) + v_g) ^ v_sw) << 5);
+      const int pair = 2 * (f % AE_NDB);
+      const ae_lds_byte* a0 = (const ae_lds_byte*)(v_at ^ (unsigned)((pair & AE_VSWM) << 5)) + ((pair & ~AE_VSWM) << 5) + rb0 * AE_VSTR;
       ae_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)a0);
       ae_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
           (__attribute__((address_space(3))) ae_s16x4*)(a0 + 8 * AE_VSTR));
@@ -765,6 +834,11 @@ void ae_prefill_kernel(const ae_attn_params p) {
       AE_RING_FENCE();
     }
     }
+    }
+#if AE_SUM_CHECK
+    if (__builtin_expect(!again, 1))
+#endif
+    {
 
     // the next tile must have landed before anyone reads it: direct loads are tracked by vmcnt
 #if AE_DEEP
@@ -782,9 +856,13 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #endif
 #pragma unroll
     for (int rb = 0; rb < AE_RB; rb++) cls[rb] = cls_n[rb];
+    }
   }
 
   // ---- epilogue -------------------------------------------------------------------------------
+#if AE_SUM_CHECK
+  st[0].AE_SM_R = ae_group_sum(st[0].AE_SM_R);
+#endif
 #if AE_KW > 1
   // Every wave leaves its O and its row state in LDS (the stages are free: the loop ended with a barrier; element e of
   // lane l at 16 * ((e / 4) * 64 + l) + 4 * (e % 4), so that all accesses are 16 bytes a lane in lane order), then takes

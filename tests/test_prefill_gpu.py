@@ -1217,3 +1217,49 @@ def test_a_share_without_visible_keys_weighs_nothing(cuda_device, monkeypatch):
     for out, lse in outs.values():
         assert (out - ref).abs().max().item() <= OUT_TOL
         assert ((lse - rlse).abs() <= LSE_TOL + 2e-6 * rlse.abs()).all()
+
+
+@pytest.mark.parametrize("D,DV,dtype", [(64, 64, torch.float16), (64, 64, torch.bfloat16), (128, 128, torch.float16), (192, 128, torch.bfloat16)])
+@pytest.mark.parametrize("mask", ["none", "causal", "window"])
+def test_references_that_lag_behind_the_maxima(cuda_device, D, DV, dtype, mask):
+    """AE_SUM_CHECK: scores that grow along the keys (every few tiles the weights would leave their type), that fall, and one
+    key far above all others; rows whose first tiles hide every key from them."""
+    B, H, S = 2, 24, 700                                   # (enough q tiles that no groups of waves share the kv axis at D 64)
+    mod = {"none": None, "causal": C.causal_mask, "window": C.make_sliding_window_mask(150)}[mask]
+    q, k, v = C.make_inputs(B, S, S, H, H, D, DV, dtype, seed=D)
+    ramp = torch.linspace(0.05, 6.0, S)
+    ramp[400:500] = 0.1
+    ramp[611] = 25.0
+    k = (k.float() * ramp[None, :, None, None]).to(dtype)
+    meta = (meta_tensor(B, H, S, D, dtype=dtype), meta_tensor(B, H, S, D, dtype=dtype), meta_tensor(B, H, S, DV, dtype=dtype))
+    eng = AttentionEngine(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), mod, C.OnlineSoftmax())
+    assert "#define AE_SUM_CHECK 1" in eng.tl_code
+    out = eng(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+    lse = eng.final_rowscales["lse"].cpu()
+    i = torch.arange(S)
+    dense = torch.ones(S, S, dtype=torch.bool) if mask == "none" else (i[:, None] >= i[None, :])
+    if mask == "window":
+        dense = dense & (i[:, None] < i[None, :] + 150)
+    ref, rlse = R.softmax_attention(q, k, v, causal=False, mask=dense.expand(B, H, S, S))
+    # weights rounded to the type (they sum to 1) times the largest value, and the result's own rounding
+    eps = 2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12
+    assert (out - ref).abs().max().item() <= 2 * eps * v.float().abs().max().item() + 2 * eps * ref.abs().max().item()
+    assert ((lse - rlse).abs() <= 1e-3 + 2e-6 * rlse.abs()).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_scores_that_are_no_numbers_reach_their_rows_only(cuda_device, D):
+    B, H, S, dtype = 2, 24, 500, torch.float16
+    q, k, v = C.make_inputs(B, S, S, H, H, D, D, dtype, seed=3)
+    meta = tuple(meta_tensor(B, H, S, D, dtype=dtype) for _ in range(3))
+    eng = AttentionEngine(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), C.causal_mask, C.OnlineSoftmax())
+    assert "#define AE_SUM_CHECK 1" in eng.tl_code
+    clean = eng(q.cuda(), k.cuda(), v.cuda()).cpu()
+    k[0, 300, :, 5] = float("nan")
+    q[1, 77, :, 5] = float("nan")
+    out = eng(q.cuda(), k.cuda(), v.cuda()).cpu()
+    assert torch.isnan(out[0, 300:]).all() and torch.equal(out[0, :300], clean[0, :300])
+    assert torch.isnan(out[1, 77]).all()
+    rest = torch.arange(S) != 77
+    # (the wave of a row without a number takes the maxima on every tile: another reference, another rounding)
+    assert (out[1, rest].float() - clean[1, rest].float()).abs().max().item() <= 2.0 ** -10 * v.abs().max().item()
