@@ -135,8 +135,9 @@ class PrefillOp:
         # workgroups per q tile and the partial results are merged with the user's combine().
         self.target_workgroups = int(target_workgroups)
         # Bytes of work memory that one call may take for launches that share tiles out over several workgroups where the chip
-        # would idle (_tail, PrefillBwdOp.dkv_parts): allocated per call, given back with it.  None: 128 MB in the forward,
-        # 256 MB in the backward.  0: no tile is shared out.
+        # would idle (_tail, PrefillBwdOp.dkv_parts), or that keep ds for the dq launch (PrefillBwdOp.keeps_ds): allocated per
+        # call, given back with it.  None: 128 MB in the forward, 256 MB and, for ds, 1 GB in the backward.  0: no tile is
+        # shared out, nothing kept.
         self._work_limit = None
         if self.split_kv:
             if self.tiles.template == "ae_prefill_simple.hip" or max(self.D, self.DV) > 128:

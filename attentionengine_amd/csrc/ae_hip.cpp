@@ -687,6 +687,14 @@ int ae_prefill_bwd(ae_kernel* delta, ae_kernel* dkv, ae_kernel* dq, const ae_att
       cfg->lds_bytes > 160 * 1024 || cfg->head_dim_v <= 0 || cfg->head_dim_v % 8 != 0)
     return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: bad tile configuration (bm=%d bn=%d threads=%d lds=%d dv=%d)",
                 cfg->block_m, cfg->block_n, cfg->threads, cfg->lds_bytes, cfg->head_dim_v);
+  const bool keeps_ds = cfg->merge_in_wg == 3;
+  if (keeps_ds) {
+    if (!delta || !p->lse || dkv_waves != 8 || cfg->mask_mode == 2 || cfg->head_dim != 128 || cfg->head_dim_v != 128 ||
+        cfg->block_m != 256)
+      return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: ds is kept by launches of wave pairs at head dim 128, delta first, dq of 256 rows");
+    if (((uintptr_t)p->delta & 15) != 0)
+      return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: the work buffer must start on a 16-byte boundary");
+  }
   if (cfg->mask_mode == 2) {
     if (!p->mask_dq || !p->mask_dkv)
       return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: tile-class kernels without their tables");
@@ -715,7 +723,7 @@ int ae_prefill_bwd(ae_kernel* delta, ae_kernel* dkv, ae_kernel* dq, const ae_att
     if (((uintptr_t)p->delta & 15) != 0)
       return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: the work buffer must start on a 16-byte boundary");
     g_dkv *= (uint64_t)p->dkv_parts;
-  } else if (cfg->merge_in_wg != 0) {
+  } else if (cfg->merge_in_wg != 0 && !keeps_ds) {
     return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: merge_in_wg=%d", cfg->merge_in_wg);
   }
   const uint64_t g_dq = (((uint64_t)p->seqlen_q + cfg->block_m - 1) / cfg->block_m) * ((((uint64_t)p->batch * p->heads_q) + 7) / 8) * 8;
@@ -742,7 +750,9 @@ int ae_prefill_bwd(ae_kernel* delta, ae_kernel* dkv, ae_kernel* dq, const ae_att
   if (rc) return rc;
   grid[0] = (uint32_t)g_dq;
   block[0] = (uint32_t)cfg->threads;
-  return ae_launch(dq, p, sizeof *p, grid, block, (uint32_t)cfg->lds_bytes, stream);
+  // (dq from ds in memory: three stages of 32 rows of K and of four blocks of ds, two workgroups a CU)
+  const uint32_t dq_lds = keeps_ds ? 3 * (32 * 256 + 4 * 4096) : (uint32_t)cfg->lds_bytes;
+  return ae_launch(dq, p, sizeof *p, grid, block, dq_lds, stream);
 }
 
 int ae_event_create(ae_event** out) {

@@ -171,6 +171,15 @@ AE_DEV int ae_bwd_chunk_pos(int r, int c) {
 #ifndef AE_BWD_SPLIT
 #define AE_BWD_SPLIT 0
 #endif
+// 1 (dk/dv launch in pairs of waves): ds goes to memory as well, in the layout of ae_bwd_ds.h, and the dq launch multiplies it by
+// K (ae_bwd_dq.hip) instead of forming s, dp and ds once more: 5 tile products instead of 7 for 2 bytes a score out and in.
+#ifndef AE_BWD_KEEP_DS
+#define AE_BWD_KEEP_DS 0
+#endif
+#if AE_BWD_KEEP_DS
+#include "ae_bwd_ds.h"
+static_assert(AE_BWD_PAIRS && !AE_BWD_SPLIT && AE_MASK_MODE != 2, "ds is kept by the waves that form it, softmax without a tile table");
+#endif
 static_assert(!AE_BWD_SPLIT || (AE_BWD_FUSE_DELTA && AE_MASK_MODE != 2), "shared kv tiles: softmax without a tile table");
 static_assert(!AE_BWD_PAIRS || (AE_BWD_ROLE == 1 && AE_BWD_KIND == 0 && AE_NWAVES == 8 && AE_RES_VIA_LDS && AE_OUT_VIA_LDS), "pairs");
 static_assert(!AE_BWD_FUSE_DELTA || (AE_RES_VIA_LDS && AE_BWD_KIND == 0), "the fused row sums need the staged resident rows");
@@ -882,6 +891,12 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   typedef __attribute__((address_space(3))) ae_u32x4 ae_lds_u32x4;
   unsigned st_use = 0, st_req = AE_STAGE_BYTES;
   if (wave < AE_NRW) {
+#if AE_BWD_KEEP_DS
+    // (carried along, as the requests' addresses are)
+    char* ds_at = ae_ds_row(p, b * p.heads_q + us_h, us_t) + (int64_t)(rt * 4 + rw) * 4096 + lane * 16;
+    const bool ds_triangle = AE_MASK_MODE == 1 && p.seqlen_q == p.seqlen_kv;
+    const int ds_pairs = 2 * n_rt;
+#endif
     while (x0 < n_items) {
       request_item(x1, st_req);
       const tile_at at = tile_in_use(st_use);
@@ -893,6 +908,11 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
           *(ae_lds_u32x4*)(ho + (2 * nb + i) * 1024) = pf[2 * nb + i];
           *(ae_lds_u32x4*)(ho + (4 + 2 * nb + i) * 1024) = dsf[2 * nb + i];
         }
+#if AE_BWD_KEEP_DS
+        // (past the caches: another launch reads it, hundreds of MB later)
+#pragma unroll
+        for (int i = 0; i < 2; i++) __builtin_nontemporal_store(dsf[2 * nb + i], (ae_u32x4*)(ds_at + (2 * nb + i) * 1024));
+#endif
       };
       if (need_vis) block(0, ae_bwd_true{}, at, pf, dsf);
       else block(0, ae_bwd_false{}, at, pf, dsf);
@@ -901,11 +921,23 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
       if (need_vis) block(1, ae_bwd_true{}, at, pf, dsf);
       else block(1, ae_bwd_false{}, at, pf, dsf);
       hand_over(1);
+#if AE_BWD_KEEP_DS
+      __builtin_amdgcn_s_waitcnt(AE_VMCNT(4));                 // (the tile: this trip's four stores of ds are newer)
+#else
       __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
+#endif
       __syncthreads();                                         // B
+#if AE_BWD_KEEP_DS
+      ds_at += (ds_triangle ? 2 * (us_t / 2 + 1) : ds_pairs) * 8192;
+#endif
 #if AE_MASK_MODE != 2
       us_t++;
-      if (us_t == t_hi) us_t = t_lo, us_h++;
+      if (us_t == t_hi) {
+        us_t = t_lo, us_h++;
+#if AE_BWD_KEEP_DS
+        ds_at = ae_ds_row(p, b * p.heads_q + us_h, us_t) + (int64_t)(rt * 4 + rw) * 4096 + lane * 16;
+#endif
+      }
 #endif
       st_use = st_use == 2 * AE_STAGE_BYTES ? 0 : st_use + AE_STAGE_BYTES;
       st_req = st_req == 2 * AE_STAGE_BYTES ? 0 : st_req + AE_STAGE_BYTES;
@@ -1160,52 +1192,5 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 }
 
 #if AE_BWD_ROLE == 0
-// Work buffer fp32 [2,B,Hq,Sq]: plane 0 = rowsum(do * o) (softmax: its negative), the `doosum` row scale of the reference's
-// backward (flashattn_bwd_preprocess, attn_tl.py:196-221); plane 1 = lse in log2 units, the form the two
-// other launches subtract inside exp2.  DV/8 lanes share a row, 16 bytes each.
-extern "C" __global__ __launch_bounds__(256)
-void ae_bwd_delta_kernel(const ae_attn_bwd_params p) {
-  constexpr int LPR = AE_DV / 8;                   // lanes per row
-  constexpr int RPB = 256 / LPR;                   // rows per workgroup
-  const int tid = threadIdx.x;
-  const int64_t n_rows = (int64_t)p.batch * p.seqlen_q * p.heads_q;
-  const int64_t row = (int64_t)blockIdx.x * RPB + tid / LPR;
-  const int c = tid % LPR;
-  float acc = 0.f;
-  int b = 0, s = 0, h = 0;
-  if (row < n_rows) {
-    h = (int)(row % p.heads_q);
-    s = (int)((row / p.heads_q) % p.seqlen_q);
-    b = (int)(row / ((int64_t)p.heads_q * p.seqlen_q));
-    const ae_elem8 o = *(const ae_elem8*)((const ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)s * p.o_stride_s + (int64_t)h * p.o_stride_h + c * 8);
-    const ae_elem8 d = *(const ae_elem8*)((const ae_elem*)p.dout + (int64_t)b * p.do_stride_b + (int64_t)s * p.do_stride_s + (int64_t)h * p.do_stride_h + c * 8);
-#pragma unroll
-    for (int j = 0; j < 8; j++) acc += (float)o[j] * (float)d[j];
-  }
-  // the LPR lanes of a row are consecutive and aligned: butterfly inside the group
-#pragma unroll
-  for (int m = 1; m < LPR; m <<= 1) {
-    const int lane = tid & 63;
-    acc += __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ m) << 2, __builtin_bit_cast(int, acc)));
-  }
-  if (row < n_rows && c == 0) {
-    const int64_t ri = ((int64_t)b * p.heads_q + h) * p.seqlen_q + s;
-    const float l = p.lse ? p.lse[ri] : 0.f;
-#if AE_BWD_KIND == 0
-    p.delta[ri] = -acc;             // (the sign in which the two launches start their dp products)
-#else
-    p.delta[ri] = acc;
-#endif
-#if AE_BWD_KIND == 2
-    // further planes: the online function's final row scales, as the forward wrote them
-    p.delta[(int64_t)p.batch * p.heads_q * p.seqlen_q + ri] = l;
-#pragma unroll
-    for (int i = 1; i < AE_BWD_NRS; i++)
-      p.delta[(int64_t)(1 + i) * p.batch * p.heads_q * p.seqlen_q + ri] = p.more_rowscales[i - 1][ri];
-#else
-    // second plane: lse in log2 units, +inf for a row without a visible key (its p is 0 everywhere)
-    p.delta[(int64_t)p.batch * p.heads_q * p.seqlen_q + ri] = (l == AE_NEG_INF) ? __builtin_inff() : l * AE_LOG2E;
-#endif
-  }
-}
+#include "ae_bwd_delta.h"
 #endif

@@ -201,7 +201,10 @@ typedef struct ae_attn_bwd_params {
   /* kernels compiled with AE_BWD_SPLIT 1 (announced by cfg->merge_in_wg = 2): workgroups per kv tile of the dk/dv launch,
    * 2 .. 64.  `delta` then has, behind its two planes (their length rounded up to a multiple of 4), ceil(Skv/128) * B * Hkv
    * arrival counters (rounded up likewise; the dq launch clears them) and, per kv tile, dkv_parts * 128 * (D + DV) floats
-   * of partial sums.  Ignored otherwise. */
+   * of partial sums.  Ignored otherwise.
+   * Kernels that keep ds (cfg->merge_in_wg = 3: dk/dv compiled with AE_BWD_KEEP_DS 1, delta and dq from ae_bwd_dq.hip) use `delta`
+   * behind its two planes, rounded up likewise, for it: for every (batch, q head) and every 64 q rows 8 KiB for each 64 keys of
+   * ceil(Skv/128) * 128, under a causal mask over equal lengths only of the 128-key tiles up to the diagonal. */
   int32_t dkv_parts;
 } ae_attn_bwd_params;
 
@@ -333,6 +336,8 @@ int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params
  *   kernels compiled with AE_BWD_KIND 1 and the generated derivative of score_mod; lse is NULL then).
  *   `delta` may be NULL for softmax kernels compiled with AE_BWD_FUSE_DELTA 1: the dq launch then forms
  *   rowsum(dout*out) for its own rows, fills the work buffer and runs first, dkv second (two launches).
+ *   cfg->merge_in_wg = 3 (kernels that keep ds: dkv compiled with AE_BWD_KEEP_DS 1 in wave pairs, dq and delta from
+ *   ae_bwd_dq.hip): the order is delta, dkv, dq, and dq multiplies the ds that dkv left in the work buffer; block_m is 256.
  */
 int ae_prefill_bwd(ae_kernel* delta, ae_kernel* dkv, ae_kernel* dq, const ae_attn_bwd_params* p,
                    const ae_tile_cfg* cfg, void* stream);

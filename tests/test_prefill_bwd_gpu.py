@@ -462,3 +462,60 @@ def test_backward_rows_of_the_dq_launch_follow_the_problem(cuda_device, S, rows)
     ref = R.softmax_attention_grads(*one, scale=1 / math.sqrt(D), causal=True)
     for g, want, what in zip(got, ref, ("dq", "dk", "dv")):
         _check(g[:, :, 3:4], want, what, (S, rows))
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,H,Hkv,Sq,Skv,dtype", [
+    (1, 2, 2, 1, 1, torch.float16),
+    (2, 3, 3, 64, 64, torch.bfloat16),
+    (1, 4, 2, 65, 65, torch.float16),         # a q tile of one row; grouped heads
+    (2, 2, 1, 129, 129, torch.bfloat16),      # a key tile of one key
+    (1, 3, 3, 300, 300, torch.float16),       # two workgroups, the second's last waves without rows
+    (1, 9, 3, 577, 577, torch.bfloat16),
+    (1, 2, 2, 100, 300, torch.float16),       # unequal lengths: every block of ds exists
+    (2, 2, 2, 390, 70, torch.bfloat16),
+])
+def test_backward_with_ds_kept_in_memory(cuda_device, monkeypatch, B, H, Hkv, Sq, Skv, dtype, causal):
+    """AE_BWD_KEEP_DS and ae_bwd_dq.hip at sizes where the plan would not take them: against the oracle, and against the launches
+    that form ds twice."""
+    from core.lower.prefill_bwd_op import PrefillBwdOp
+    print(f"case ds kept B{B} H{H} Hkv{Hkv} Sq{Sq} Skv{Skv} {dtype} causal={causal}", flush=True)
+    D, scale = 128, 1 / math.sqrt(128)
+    q, k, v = C.make_inputs(B, Sq, Skv, H, Hkv, D, D, dtype, seed=Sq)
+    do = torch.randn(B, Sq, H, D, generator=torch.Generator().manual_seed(5)).to(dtype)
+    monkeypatch.setattr(PrefillBwdOp, "dkv_parts", lambda self, *a: 1)
+    grads = []
+    for keep in (False, True):
+        monkeypatch.setattr(PrefillBwdOp, "keeps_ds", lambda self, *a: keep and a[4] != 2)      # (unequal lengths: a mask table)
+        mod = _engine(B, H, Hkv, Sq, D, D, dtype, C.causal_mask if causal else None, scale)
+        for _ in range(2):                    # through Python, then through the native host path
+            leaves = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+            mod(*leaves).backward(do.cuda())
+        grads.append([t.grad.float().cpu() for t in leaves])
+        assert any(key[-1] for key in mod.attention.backward_op()._variants) == (keep and (Sq == Skv or not causal))
+    case = (B, H, Hkv, Sq, Skv, dtype, causal)
+    ref = R.softmax_attention_grads(q, k, v, do, scale=scale, causal=causal)
+    for got, want, what in zip(grads[1], ref, ("dq", "dk", "dv")):
+        _check(got, want, what, case)
+    # the row sums rowsum(do * o) come from another order of 128 fp32 terms, which moves ds by up to that and perhaps to the
+    # next value of the input type; dv does not use them
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    out, _ = R.softmax_attention(q, k, v, scale=scale, causal=causal)
+    moved = 128 * 2.0 ** -24 * (out * do.float()).abs().sum(-1).max().item() * scale
+    for got, want, rows in zip(grads[1], grads[0], (k, q)):
+        slack = moved * rows.float().abs().max().item() * (1 if rows is k else Sq * H // Hkv) * want.numel() ** 0.5
+        assert (got - want).norm().item() <= eps * want.norm().item() + slack
+    assert torch.equal(grads[1][2], grads[0][2])
+
+
+def test_when_ds_is_kept(cuda_device):
+    """By the visible pairs and the size of its buffer; not for other graphs, masks by table or a caller's own dq rows."""
+    op = _engine(4, 32, 32, 2048, 128, 128, torch.bfloat16, C.causal_mask, 0.1).attention
+    bwd = op.backward_op()
+    assert bwd.keeps_ds(4, 32, 2048, 2048, 1, False) and not bwd.keeps_ds(4, 32, 2048, 2048, 2, False)
+    assert not bwd.keeps_ds(1, 32, 1024, 1024, 1, False) and not bwd.keeps_ds(64, 32, 8192, 8192, 1, False)
+    # q tiles t of 64 rows see the 128-key tiles 0 .. t / 2
+    assert bwd.ds_floats(1, 1, 300, 300, 1) == sum(t // 2 + 1 for t in range(5)) * 64 * 128 // 2
+    assert bwd.ds_floats(2, 3, 300, 300, 0) == 6 * 5 * 3 * 64 * 128 // 2
+    op.work_limit = 100 << 20
+    assert not bwd.keeps_ds(4, 32, 2048, 2048, 1, False)
