@@ -124,22 +124,22 @@ class Merges:
 
     def __init__(self, d, dv, dtype, n_rowscales, functor_src, any_order, threads, allow_spills=None):
         self._dims, self._dtype, self._n_rowscales, self._functor_src = (d, dv), dtype, n_rowscales, functor_src
-        self._any_order, self._threads, self._allow_spills = any_order, threads, allow_spills
+        self.any_order, self._threads, self._allow_spills = any_order, threads, allow_spills
         self._modules = {}
 
     def config(self, n, splits_per_partial=1):
-        return merge_config(self._dims[1], self._dtype, self._n_rowscales, merge_capacity(n, self._any_order), self._threads,
+        return merge_config(self._dims[1], self._dtype, self._n_rowscales, merge_capacity(n, self.any_order), self._threads,
                             splits_per_partial)
 
     def cfg(self, n, splits_per_partial=1):
         """The launch configuration of a merge of ``n`` partial results a row."""
         return rt.TileCfg(block_m=combine_rows(self._threads, self._dims[1]),
-                          block_n=merge_capacity(n, self._any_order) * splits_per_partial, threads=self._threads, lds_bytes=0,
+                          block_n=merge_capacity(n, self.any_order) * splits_per_partial, threads=self._threads, lds_bytes=0,
                           head_dim=self._dims[0], head_dim_v=self._dims[1], elem_bytes=2, n_rowscales=self._n_rowscales,
-                          mask_mode=0, merge_in_wg=int(self._any_order))
+                          mask_mode=0, merge_in_wg=int(self.any_order))
 
     def module(self, n, splits_per_partial=1):
-        key = (merge_capacity(n, self._any_order), splits_per_partial)
+        key = (merge_capacity(n, self.any_order), splits_per_partial)
         m = self._modules.get(key)
         if m is None:
             m = self._modules[key] = rt.compile_module(

@@ -610,6 +610,25 @@ class PrefillOp:
         """The mask's band (MaskPlan.band) where the kernel takes one instead of the tile table."""
         return plan.band if tiles.template == "ae_prefill.hip" else None
 
+    MERGED_SPLITS, MERGED_VALUES = 8, 8192      # (the first: of ae_merge_last.h)
+
+    def _merges_in_last(self, Hq, Sq, tiles, n_split):
+        """Whether the workgroup that finishes last of a q tile merges (AE_MERGE_LAST of ae_prefill.hip) instead of a second
+        launch (not in a graph: see ae_host.cpp): few values are read by that one workgroup, few counts are constants of its
+        build.  48 shapes (batch 1 to 8, 8 to 32 heads, 1 to 25 rows, 512 to 16384 keys, head dims 64 and 128), time of the call in
+        units of that with two launches: 0.94 on average, 0.81 to 1.003 (D64 B3 H8 Sq8 Skv764, 8 splits, 9.9 us -> 8.0; D128
+        B4 H32 Sq5 Skv1496, 2 splits, 23.2 -> 21.8; B4 H16 Sq12 Skv14418, 4 splits, 89.4 -> 89.6).  Beyond: 8192 to 16384
+        values 0.92 to 1.20, 10 to 15 splits 0.95 to 1.06."""
+        return (1 < n_split <= self.MERGED_SPLITS and self._can_merge_in_last(tiles)
+                and min(Sq, tiles.block_m) * n_split * self.DV <= self.MERGED_VALUES
+                and tiles.block_m * Hq * n_split * self.DV < 2**29)
+
+    def _can_merge_in_last(self, tiles):
+        """Whether a split launch's build can: the merge's 32 loads a thread in flight take up to 190 registers, which those of 32
+        rows have (at most two waves a SIMD)."""
+        return (tiles.template == "ae_prefill.hip" and tiles.block_m == 32 and tiles.kv_groups > 1 and tiles.waves_per_eu == 2
+                and self._merges.any_order)
+
     def _variant(self, tiles, mask_mode, Sq, Skv, n_split=1, table_rows=1, heavy_last=False, band=None,
                  tail=False):
         even_q, even_kv = Sq % tiles.block_m == 0, Skv % tiles.block_n == 0
@@ -644,6 +663,8 @@ class PrefillOp:
                 cfg_src += "#define AE_SUM_CHECK 1\n"
             if n_split > 1:
                 cfg_src += "#define AE_NSPLIT 2\n"       # (a split launch; its count is the launch's)
+                if self._can_merge_in_last(tiles):
+                    cfg_src += "#define AE_MERGE_LAST 1\n"
             if key[-1]:
                 cfg_src += "#define AE_CLOCK_STAMPS 1\n"
             if tail:
@@ -777,13 +798,17 @@ class PrefillOp:
         if n_split > 1:
             partial_o = torch.empty((B, Sq, Hq, n_split, self.DV), dtype=torch.float32, device=dev)
             partial_rs = torch.empty((max(1, self.n_rowscales), B, Sq, Hq, n_split), dtype=torch.float32, device=dev)
+            modules, ccfg = (module, self._merges.module(n_split)), self._merges.cfg(n_split)
+            combine = modules[1].kernel("ae_decode_combine_kernel")
+            shared = {"n_split": n_split, "kv_per_split": kv_per_split}
+            if self._merges_in_last(Hq, Sq, tiles, n_split):       # (from the next call on: the host path keeps the counters)
+                shared["counters"] = B * Hq * -(-Sq // tiles.block_m)
             p.partial_o, p.partial_rs = partial_o.data_ptr(), partial_rs.data_ptr()
             p.num_splits, p.kv_per_split = n_split, kv_per_split
             keep += [partial_o, partial_rs]
-            merge, ccfg = self._merges.module(n_split), self._merges.cfg(n_split)
-            rt.prefill_split_fwd(kern, merge.kernel("ae_decode_combine_kernel"), p, cfg, ccfg, stream)
+            rt.prefill_split_fwd(kern, combine, p, cfg, ccfg, stream)
         else:
-            shared = {}
+            modules, combine, ccfg, shared = (module,), None, None, {}
             if tail is not None:
                 p.tail_slots, p.num_splits, p.kv_per_split = tail[0], tail[1], tail[2] * tiles.block_n
                 shared = {"n_split": tail[1], "kv_per_split": p.kv_per_split, "tail_slots": tail[0], "counters": 8 * tail[0],
@@ -805,12 +830,8 @@ class PrefillOp:
         self.final_rowscales = dict(zip(self.functors.final_rowscale_names, rowscales))
         self._keepalive = keep
         if extern_mask is None and self.DV_launch == self.DV and not self._clock_stamps(tiles):
-            if n_split > 1:
-                shared = {"n_split": n_split, "kv_per_split": kv_per_split}
             host.add_forward(self._host, host.PREFILL_SPLIT if n_split > 1 else host.PREFILL, B, Sq, Hq, Hkv, Skv, dev,
-                             (module, merge) if n_split > 1 else (module,),
-                             kern, cfg, combine=merge.kernel("ae_decode_combine_kernel") if n_split > 1 else None,
-                             ccfg=ccfg if n_split > 1 else None, **shared,
+                             modules, kern, cfg, combine=combine, ccfg=ccfg, **shared,
                              table=table if mode == 2 and band is None else None, mask_block=(mbm, mbn), env=("AE_CLOCK_STAMPS",))
         return out
 

@@ -412,6 +412,8 @@ def _compile_module(template: str, headers: dict, arch: str = None, use_cache: b
     }
     if template in ("ae_prefill_bwd.hip", "ae_bwd_dq.hip"):
         all_headers.update({n: _read(osp.join(KERNEL_DIR, n)) for n in ("ae_bwd_delta.h", "ae_bwd_ds.h")})
+    if template == "ae_prefill.hip":
+        all_headers["ae_merge_last.h"] = _read(osp.join(KERNEL_DIR, "ae_merge_last.h"))
     all_headers.update(headers)
     opts = COMPILE_OPTS + TEMPLATE_OPTS.get(template, [])
     hsh = hashlib.sha256()

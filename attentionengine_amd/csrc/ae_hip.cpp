@@ -525,7 +525,9 @@ extern "C" __attribute__((visibility("hidden"))) int ae_internal_decode_check(
 
 int ae_prefill_split_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params* p,
                          const ae_tile_cfg* cfg, const ae_tile_cfg* combine_cfg, void* stream) {
-  if (!split || !combine || !combine_cfg)
+  // merge_in_wg 2: a kernel compiled with AE_MERGE_LAST 1, whose last workgroup of a q tile is to merge
+  const bool merged = cfg && cfg->merge_in_wg == 2;
+  if (!split || (!combine && !merged) || !combine_cfg)
     return fail(AE_ERR_INVALID_ARG, "ae_prefill_split_fwd: kernel/cfg is NULL");
   int rc = check_common("ae_prefill_split_fwd", p, cfg);
   if (rc) return rc;
@@ -538,6 +540,9 @@ int ae_prefill_split_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_par
   if (p->kv_per_split % cfg->block_n != 0)
     return fail(AE_ERR_INVALID_ARG, "ae_prefill_split_fwd: kv_per_split=%d is not a multiple of block_n=%d",
                 p->kv_per_split, cfg->block_n);
+  if (merged && (p->num_splits > 8 || (int64_t)cfg->block_m * p->heads_q * p->num_splits * cfg->head_dim_v >= (1 << 29)))
+    return fail(AE_ERR_INVALID_ARG, "ae_prefill_split_fwd: the last workgroup merges at most 8 splits and 2 GiB between a tile's first "
+                "and last result (%d splits, %d heads)", p->num_splits, p->heads_q);
   if ((rc = check_merge_splits("ae_prefill_split_fwd", combine_cfg, p->num_splits))) return rc;
   if (!p->partial_o || !p->partial_rs)
     return fail(AE_ERR_INVALID_ARG, "ae_prefill_split_fwd: split-KV work buffers are NULL");
@@ -559,11 +564,12 @@ int ae_prefill_split_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_par
                 (unsigned long long)total);
   uint32_t grid[3] = {(uint32_t)total, 1, 1};
   uint32_t block[3] = {(uint32_t)cfg->threads, 1, 1};
-  rc = ae_launch(split, p, sizeof *p, grid, block, (uint32_t)cfg->lds_bytes, stream);
-  if (rc) return rc;
+  ae_attn_params cp = *p;
+  cp.tail_slots = merged;
+  rc = ae_launch(split, &cp, sizeof cp, grid, block, (uint32_t)cfg->lds_bytes, stream);
+  if (rc || merged) return rc;
   // the merge kernel sees the (q position, head) pairs as the heads of a one-token decode; seqlen_q stays, and
   // tells it to write the merged row scales in [B, Hq, Sq] order
-  ae_attn_params cp = *p;
   cp.heads_q = (int32_t)rows;
   uint32_t cgrid[3] = {combine_grid((int32_t)rows, combine_cfg), (uint32_t)p->batch, 1};
   uint32_t cblock[3] = {(uint32_t)combine_cfg->threads, 1, 1};

@@ -140,6 +140,13 @@ at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dt, int device) {
   return at::Tensor(at::detail::empty_cuda(sizes, dt, c10::Device(c10::kCUDA, (c10::DeviceIndex)device), std::nullopt));
 }
 
+bool is_capturing(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();              // (the default stream while another one captures)
+  return true;
+}
+
 // The work buffers of a launch on `stream` (see Work).  A capture that finds none kept gets buffers of its own, which live
 // in the graph's memory, and records the clearing of their counters: what a capture allocates and clears is only there
 // when that graph has been replayed, so no other call may be given it.  `eager_only`: a capture always gets its own, so
@@ -147,10 +154,7 @@ at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dt, int device) {
 // in a graph whose kernel takes a hundred).
 std::pair<at::Tensor, at::Tensor> get_work(Host* h, int64_t o_rows, int64_t rs_floats, int64_t counters, int device, void* stream,
                                            bool eager_only) {
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  bool capturing = true;
-  if (hipStreamIsCapturing((hipStream_t)stream, &status) == hipSuccess) capturing = status != hipStreamCaptureStatusNone;
-  else (void)hipGetLastError();         // (the default stream while another one captures)
+  const bool capturing = is_capturing(stream);
   for (auto& w : *h->work)
     if (!(eager_only && capturing) && w.device == device && w.stream == stream && w.o_rows == o_rows && w.rs_floats == rs_floats && w.counters == counters) {
       w.captured = w.captured || capturing;
@@ -401,6 +405,7 @@ PyObject* run(Host* h, PyObject* const* args, Py_ssize_t nargs, bool mla) {
     p.mask_nq = (int)pl.table.size(2), p.mask_nkv = (int)pl.table.size(3);
     p.mask_block_m = pl.mask_bm, p.mask_block_n = pl.mask_bn;
   }
+  ae_tile_cfg cfg = pl.cfg;
   const int64_t rs_floats = (h->n_rs > 0 ? h->n_rs : 1) * B * Sq * Hq * pl.n_split;
   at::Tensor po, prs;
   if (pl.kind != kPrefill || pl.tail_slots) p.num_splits = pl.n_split, p.kv_per_split = pl.kv_per_split;
@@ -408,6 +413,12 @@ PyObject* run(Host* h, PyObject* const* args, Py_ssize_t nargs, bool mla) {
     p.tail_slots = pl.tail_slots;
     po = empty({pl.o_rows, h->DV}, at::kFloat, dev);
     prs = get_work(h, 1, 1, pl.counters, dev, stream, true).second.narrow(0, 1, pl.counters);
+  } else if (pl.kind == kPrefillSplit && pl.counters && !is_capturing(stream)) {
+    // (the last workgroup merges; not in a graph, where the clearing of its counters costs what the merge launch does:
+    // B3 H8 Sq8 Skv1680 D64 9.1 us a replay, 10.2 so)
+    cfg.merge_in_wg = 2;
+    po = empty({pl.o_rows, h->DV}, at::kFloat, dev);
+    prs = get_work(h, 1, rs_floats, pl.counters, dev, stream, true).second;
   } else if (pl.cfg.merge_in_wg == 2) {
     std::tie(po, prs) = get_work(h, pl.o_rows, rs_floats, pl.counters, dev, stream, false);
   } else if (pl.n_split > 1 && pl.cfg.merge_in_wg == 0) {
@@ -419,8 +430,8 @@ PyObject* run(Host* h, PyObject* const* args, Py_ssize_t nargs, bool mla) {
   int rc;
   PyThreadState* thread = PyEval_SaveThread();
   switch (pl.kind) {
-    case kPrefill: rc = ae_prefill_fwd(pl.k0, &p, &pl.cfg, stream); break;
-    case kPrefillSplit: rc = ae_prefill_split_fwd(pl.k0, pl.k1, &p, &pl.cfg, &pl.ccfg, stream); break;
+    case kPrefill: rc = ae_prefill_fwd(pl.k0, &p, &cfg, stream); break;
+    case kPrefillSplit: rc = ae_prefill_split_fwd(pl.k0, pl.k1, &p, &cfg, &pl.ccfg, stream); break;
     case kDecode: rc = ae_decode_fwd(pl.k0, pl.k1, &p, &pl.cfg, pl.has_ccfg ? &pl.ccfg : nullptr, stream); break;
     default: rc = ae_mla_decode_fwd(pl.k0, pl.k1, &p, &pl.cfg, &pl.ccfg, stream); break;
   }

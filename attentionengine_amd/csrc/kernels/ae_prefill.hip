@@ -105,6 +105,15 @@
 #ifndef AE_KV_STAGES
 #define AE_KV_STAGES 2
 #endif
+// 1 (split builds with kv groups): where p.tail_slots is not 0 the workgroup that finishes last of a q tile merges, see
+// ae_merge_last.h; p.num_splits at most 8 then
+#ifndef AE_MERGE_LAST
+#define AE_MERGE_LAST 0
+#endif
+#if AE_MERGE_LAST
+#include "ae_merge_last.h"
+static_assert(AE_NSPLIT > 1 && AE_KW > 1, "merged by the last workgroup: builds whose groups meet in LDS");
+#endif
 #define AE_DEEP (AE_KV_STAGES == 3)
 
 // value given to score positions past seqlen_kv before the user functors run: -inf, or 0 for graphs
@@ -936,7 +945,18 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #pragma unroll
       for (int i = 0; i < AE_N_ROWSCALES; i++) frs[i] = AE_NEG_INF;
     }
+#if AE_MERGE_LAST
+    const int64_t first = (((int64_t)b * p.seqlen_q + q0) * p.heads_q + h) * n_split;
+    const int rows_here = p.seqlen_q - q0 < AE_BM ? p.seqlen_q - q0 : AE_BM;
+    const int row_step = p.heads_q * n_split;
+    __amdgpu_buffer_rsrc_t part = __builtin_amdgcn_make_buffer_rsrc(
+        p.partial_o + first * AE_DV, 0, ((rows_here - 1) * row_step + n_split) * (AE_DV * 4), 0x00020000);
+    const bool merged = p.tail_slots != 0;
+#endif
     if (q_ok[0]) {
+#if AE_MERGE_LAST
+      const int at = (qrow[0] - q0) * row_step + split;
+#endif
 #if AE_NSPLIT > 1
       const int64_t prow = ((((int64_t)b * p.seqlen_q + qrow[0]) * p.heads_q + h) * n_split) + split;
       float* po = p.partial_o + prow * AE_DV;
@@ -947,6 +967,12 @@ void ae_prefill_kernel(const ae_attn_params p) {
       for (int e = 0; e < AE_NE; e += 4) {
         const int ea = kg * AE_NE + e;                      // element ea .. ea + 3: four neighbouring columns
         const int col = (ea >> 4) * 32 + ((ea & 15) >> 2) * 8 + hf * 4;
+#if AE_MERGE_LAST
+        if (merged)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(ae_u32x4, (ae_f32x4){o[e], o[e + 1], o[e + 2], o[e + 3]}), part,
+                                                 (at * AE_DV + col) * 4, 0, kAeDeviceScope);
+        else
+#endif
 #if AE_NSPLIT > 1
         *(ae_f32x4*)(po + col) = (ae_f32x4){o[e], o[e + 1], o[e + 2], o[e + 3]};
 #else
@@ -956,6 +982,10 @@ void ae_prefill_kernel(const ae_attn_params p) {
       if (hf == 0 && kg == 0) {
 #pragma unroll
         for (int i = 0; i < AE_N_ROWSCALES; i++)
+#if AE_MERGE_LAST
+          if (merged) __hip_atomic_store(p.partial_rs + first + at, frs[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          else
+#endif
 #if AE_NSPLIT > 1
           p.partial_rs[(int64_t)i * p.batch * p.seqlen_q * p.heads_q * n_split + prow] = frs[i];
 #else
@@ -963,6 +993,18 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #endif
       }
     }
+#if AE_MERGE_LAST
+    if (!merged) return;
+    int* const counter = (int*)(p.partial_rs + (int64_t)p.batch * p.seqlen_q * p.heads_q * n_split) + (int64_t)bh * n_qt + qt;
+    if (!ae_count_in(counter, n_split, tid == 0, (__attribute__((address_space(3))) int*)xs)) return;
+    ae_merge_rows<AE_NT>(p, first, row_step, tid, rows_here, n_split, [&](int r, int col, ae_f32x4 acc, float merged) AE_LAMBDA {
+      ae_elem4 w;
+#pragma unroll
+      for (int c = 0; c < 4; c++) w[c] = (ae_elem)acc[c];
+      *(ae_elem4*)((ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)(q0 + r) * p.o_stride_s + (int64_t)h * p.o_stride_h + col) = w;
+      if (col == 0) p.rowscale_out[0][((int64_t)b * p.heads_q + h) * p.seqlen_q + q0 + r] = merged;
+    });
+#endif
   }
 #elif AE_NO > 128 && AE_NSPLIT == 1
   // wide value heads: the epilogue functor (elementwise over the value columns) runs one 32-column block at a

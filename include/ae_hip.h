@@ -103,7 +103,8 @@ typedef struct ae_attn_params {
   /* prefill kernels compiled with AE_TAIL 1 (announced by cfg->merge_in_wg = 2): of the q-tile slots of every XCD (see
    * ae_prefill_fwd) the last tail_slots are shared by num_splits workgroups each, kv_per_split positions a workgroup;
    * the one that finishes last merges.  partial_o: 8 * tail_slots * num_splits * (block_m * DV + 4 * threads) floats;
-   * partial_rs: 8 * tail_slots int32 arrival counters, zero when the launch starts and when it ends.  Else 0. */
+   * partial_rs: 8 * tail_slots int32 arrival counters, zero when the launch starts and when it ends.  Else 0
+   * (ae_prefill_split_fwd fills it in for its split kernel). */
   int32_t tail_slots;
   /* Filled in by ae_mla_decode_fwd for its split kernel, whatever the caller left there: ceil(2^32 / u) of the number u of
    * workgroup ids per (batch, kv head), or 0 where ids times u do not fit 32 bits. */
@@ -145,7 +146,8 @@ typedef struct ae_tile_cfg {
                           writes out itself: no combine kernel, no work buffers); 2 when it was compiled with
                           AE_MERGE_LAST 1 (the workgroup that finishes last merges: no combine kernel, work
                           buffers with arrival counters, see ae_decode_fwd); else 0.  Prefill: 2 for kernels
-                          compiled with AE_TAIL 1 (ae_attn_params.tail_slots), backward: 2 for AE_BWD_SPLIT 1
+                          compiled with AE_TAIL 1 (ae_attn_params.tail_slots), split: 2 where a kernel
+                          compiled with AE_MERGE_LAST 1 is to merge (ae_prefill_split_fwd), backward: 2 for AE_BWD_SPLIT 1
                           (ae_attn_bwd_params.dkv_parts); else 0.  Combine configurations: 1 when the kernel
                           merges any number of splits up to block_n (places without a result count as row scales
                           of -inf, which its combine() gives no weight), 0 when num_splits must equal block_n  */
@@ -304,6 +306,10 @@ int ae_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params* p,
  *   block_n) and writes fp32 partials ordered (batch, q position, head, split); the combine kernel then
  *   merges them with the user's combine() into `out`, which must be contiguous [B,Sq,Hq,DV], and writes
  *   the merged rowscales to rowscale_out as fp32 [B,Hq,Sq], the layout of ae_prefill_fwd.
+ *   cfg->merge_in_wg = 2 (a split kernel compiled with AE_MERGE_LAST 1, at most 8 splits): the workgroup of a
+ *   (batch, head, q tile) that finishes last merges instead; `combine` is not launched and may be NULL.  Behind the row
+ *   scales in partial_rs it needs batch * heads_q * ceil(seqlen_q / block_m) 32-bit arrival counters, which must be zero before
+ *   the launch and are zero behind it; launches that share them must not overlap.
  */
 int ae_prefill_split_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params* p,
                          const ae_tile_cfg* cfg, const ae_tile_cfg* combine_cfg, void* stream);

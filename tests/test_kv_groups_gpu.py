@@ -280,3 +280,61 @@ def test_three_tile_stages(cuda_device, form, Sq):
             out = op(q.cuda(), k.cuda(), v.cuda()).float().cpu()
             assert (out - ref).abs().max().item() <= 2e-2
             assert (op.final_rowscales["lse"].cpu() - lse).abs().max().item() <= 1e-3
+
+
+def test_which_split_launches_merge_in_their_last_workgroup():
+    op = _engine(8, None, H=8, Hkv=8, Skv=4096)._op
+    forms = {n: PrefillTiles(**f[0]) for n, f in op.SPLIT_FORMS.items()}
+    assert op._merges_in_last(8, 8, forms["32"], 8) and op._merges_in_last(8, 32, forms["32"], 2)
+    assert not op._merges_in_last(8, 9, forms["32"], 8) and not op._merges_in_last(8, 1, forms["32"], 9)
+    assert not op._merges_in_last(8, 8, forms["32"], 1) and not op._merges_in_last(8, 8, forms["64"], 2)
+    assert not op._merges_in_last(1 << 14, 8, forms["32"], 8)                    # 2 GiB between a tile's results
+    op._merges.any_order = False                                                  # (another combine() counts its places)
+    assert not op._merges_in_last(8, 8, forms["32"], 8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16)])
+@pytest.mark.parametrize("Sq,n", [(1, 2), (1, 8), (3, 5), (4, 8), (5, 7), (8, 8), (16, 4), (17, 3), (21, 3), (32, 2)])
+def test_the_last_workgroup_merges(cuda_device, D, dtype, Sq, n):
+    """AE_MERGE_LAST against the same splits merged by a second launch, bit for bit: passes that the rows fill, exceed by one
+    and do not fill, every capacity; on two streams in turn, and in a graph (two launches again) between eager calls."""
+    H, Skv, B = 3, 64 * n - 5, 2
+    tiles = TILES[0] if D == 64 else PrefillTiles(**PrefillOp.SPLIT_FORMS["32"][0])
+    print(f"case last workgroup merges D{D} Sq{Sq} splits {n}", flush=True)
+    q, k, v = (t.cuda() for t in C.make_inputs(B, Sq, Skv, H, H, D, D, dtype, seed=Sq * 8 + n))
+    ops = []
+    for most in (0, 8192):
+        op = _engine(Sq, None, H=H, Hkv=H, B=B, Skv=4096, D=D, dtype=dtype)._op
+        op.MERGED_VALUES = most
+        op._launch_tiles = lambda *a: tiles
+        op.plan_splits = lambda *a: (n, 64)
+        assert op.split_kv and op._merges_in_last(H, Sq, tiles, n) == (most > 0)
+        ops.append(op)
+    two = ops[0](q, k, v).float()
+    two_lse = ops[0].final_rowscales["lse"]
+
+    def check(out, lse):
+        assert torch.equal(out.float(), two) and torch.equal(lse, two_lse)
+
+    ref, rlse = R.softmax_attention(q.cpu(), k.cpu(), v.cpu(), causal=False)
+    assert (two.cpu() - ref).abs().max().item() <= 2e-2 and (two_lse.cpu() - rlse).abs().max().item() <= 1e-3
+    streams = [torch.cuda.current_stream(), torch.cuda.Stream()]
+    for i in range(6):                                                # through Python, then natively; two streams in turn
+        s = streams[i % 2]
+        s.wait_stream(streams[1 - i % 2])
+        with torch.cuda.stream(s):
+            out = ops[1](q, k, v)
+            lse = ops[1].final_rowscales["lse"]
+        s.synchronize()
+        check(out, lse)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops[1](q, k, v)
+        lse = ops[1].final_rowscales["lse"]
+    for _ in range(3):
+        out.zero_(), lse.zero_()
+        graph.replay()
+        check(ops[1](q, k, v), ops[1].final_rowscales["lse"])
+        torch.cuda.synchronize()
+        check(out, lse)
