@@ -600,7 +600,7 @@ class PrefillTiles:
     v_pad: int = 0
     rows_per_wave: int = 32
     kv_groups: int = 1                 # sets of n_waves waves that share the kv axis (AE_KW of ae_prefill.hip)
-    kv_stages: int = 2                 # K / V tile stages in LDS (AE_KV_STAGES of the pipelined kernel: 2 or 3)
+    kv_stages: int = 2                 # K / V tile stages in LDS (AE_KV_STAGES: 2 or 3, 3 in the pipelined kernel and in split launches)
 
     @property
     def block_m(self):
@@ -808,7 +808,7 @@ def window_group_tiles(batch_heads: int, seqlen_q: int):
 
 def kv_group_tiles_split(seqlen_q: int, batch_heads: int = 0):
     """The same for launches that also split the kv axis over workgroups (a few query tokens against a long cache): the
-    query rows decide.  fp16 D128: B8 H32 Sq4 Skv4096 110 -> 95 us, B1 H32 Sq16 Skv16000 55 -> 46 (32 x 4 x 32); B2 H16 Sq40
+    query rows decide; at head dim 128 only where PrefillOp._launch_tiles does not choose.  fp16 D128, two tile stages: B8 H32 Sq4 Skv4096 110 -> 95 us, B1 H32 Sq16 Skv16000 55 -> 46 (32 x 4 x 32); B2 H16 Sq40
     Skv3000 19.1 -> 17.7 (64 x 2 x 32); from 65 rows on the 128-row tiles already read the cache at 5.8 TB/s.  Rows that fill a
     256-row tile better than two of 128 take one workgroup of eight waves, which reads the cache once, where the heads leave
     room for several splits: B4 H8 Sq213 Skv11337 78 -> 71 us, B1 H32 Sq237 Skv15274 98 -> 91; B8 H16 Sq220 Skv1909 51 -> 53."""

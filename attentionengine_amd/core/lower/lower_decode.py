@@ -673,8 +673,8 @@ class MLADecodeOp(_SplitTuning):
         most as many pages as the kernel keeps table entries for.
 
         The wave-specialised kernel has forms for 16, 32 and 64 heads a workgroup: the fewer, the shorter a trip over
-        one tile (0.59 / 0.73 / 0.81 us) and the fewer splits - partial results - fill the chip, but the tiles are fetched
-        by as many more workgroups.  B4 H128 Skv2048: 18.8 us with 64 heads and 16 splits, 13.9 with 16 and 8; B85 H64
+        one tile (0.59 / 0.73 / 0.81 us, paged 0.53 with 16 heads: the plans by this cost are 0.7 % off the best there)
+        and the fewer splits - partial results - fill the chip, but the tiles are fetched by as many more workgroups.  B4 H128 Skv2048: 18.8 us with 64 heads and 16 splits, 13.9 with 16 and 8; B85 H64
         Skv445 39.4 us with 64 and 4 splits (340 workgroups: a second round for 84 of them), 18.4 with 32 and none;
         B128 H128 Skv4096 163.6 us with 64, 225.6 with 32."""
         group = Hq // Hkv

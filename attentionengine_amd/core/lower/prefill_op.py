@@ -526,7 +526,7 @@ class PrefillOp:
     def plan_splits(self, B, Hq, Sq, Skv, tiles=None):
         """(number of KV splits, kv positions per split): a workgroup for every CU of the chip (more splits cost
         more in partial results and their merge than they gain: B1 H32 Sq128 Skv8192, the shape of
-        attn_script/mha_inference.py, 43 us with 8 splits, 44 with 16, 75 with 32), whole kv tiles per split, no
+        attn_script/mha_inference.py, two tile stages, 43 us with 8 splits, 44 with 16, 75 with 32), whole kv tiles per split, no
         empty split.  Where that leaves some CUs with two workgroups the cheapest count is taken (``_cheapest_splits``), and
         always for the tiles that are chosen with it (``_launch_tiles``)."""
         if not self.split_kv:

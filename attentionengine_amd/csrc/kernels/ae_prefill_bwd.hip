@@ -11,7 +11,8 @@
 // The reference accumulates dq with fp32 atomics from the kernel that owns a kv tile and converts it
 // in a third kernel.  Here the work is split by OUTPUT instead, with no atomics and a fixed summation
 // order: one launch owns q rows and produces dq, one owns kv rows and produces dk and dv; both
-// recompute s and dp (7 tile products per tile pair instead of 5).  They are the same code with the
+// recompute s and dp (7 tile products per tile pair instead of 5; with AE_BWD_KEEP_DS the dk/dv launch goes first and leaves its
+// ds for ae_bwd_dq.hip: 5).  They are the same code with the
 // operands exchanged (AE_BWD_ROLE):
 //     role 0 (dq):      resident rows = q  (Q, dO in registers), streamed tiles = K, V
 //     role 1 (dk, dv):  resident rows = kv (K, V in registers),  streamed tiles = Q, dO of every q head
