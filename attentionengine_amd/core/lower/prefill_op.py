@@ -136,7 +136,7 @@ class PrefillOp:
         self.target_workgroups = int(target_workgroups)
         # Bytes of work memory that one call may take for launches that share tiles out over several workgroups where the chip
         # would idle (_tail, PrefillBwdOp.dkv_parts), or that keep ds for the dq launch (PrefillBwdOp.keeps_ds): allocated per
-        # call, given back with it.  None: 128 MB in the forward, 256 MB and, for ds, 1 GB in the backward.  0: no tile is
+        # call, given back with it.  None: 128 MB in the forward, 256 MB and, for ds, 2.5 GB in the backward.  0: no tile is
         # shared out, nothing kept.
         self._work_limit = None
         if self.split_kv:

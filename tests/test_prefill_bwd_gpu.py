@@ -517,5 +517,33 @@ def test_when_ds_is_kept(cuda_device):
     # q tiles t of 64 rows see the 128-key tiles 0 .. t / 2
     assert bwd.ds_floats(1, 1, 300, 300, 1) == sum(t // 2 + 1 for t in range(5)) * 64 * 128 // 2
     assert bwd.ds_floats(2, 3, 300, 300, 0) == 6 * 5 * 3 * 64 * 128 // 2
+    assert bwd.keeps_ds(1, 32, 8192, 8192, 1, False)
     op.work_limit = 100 << 20
     assert not bwd.keeps_ds(4, 32, 2048, 2048, 1, False)
+
+
+@pytest.mark.gpu
+def test_no_memory_for_ds(cuda_device, monkeypatch):
+    """A first backward whose ds cannot be had takes the two launches, as one that may not keep it does."""
+    B, H, S = 1, 16, 2048
+    q, k, v = (t.cuda().requires_grad_(True) for t in C.make_inputs(B, S, S, H, H, 128, 128, torch.bfloat16, seed=3))
+    dout = torch.randn(B, S, H, 128, device="cuda", dtype=torch.bfloat16)
+    grads = []
+    for limit in (0, None):
+        op = _engine(B, H, H, S, 128, 128, torch.bfloat16, C.causal_mask, 0.1).attention
+        op.work_limit = limit
+        bwd = op.backward_op()
+        assert bwd.keeps_ds(B, H, S, S, 1, False) == (limit is None)
+        bwd.dkv_parts = lambda *a: 1
+        empty, refused = torch.empty, []
+
+        def short(*a, **kw):
+            if a and isinstance(a[0], int) and a[0] > 1 << 24:
+                refused.append(a[0])
+                raise torch.OutOfMemoryError("no memory")
+            return empty(*a, **kw)
+        monkeypatch.setattr(torch, "empty", short)
+        grads.append(torch.autograd.grad(op(q, k, v), (q, k, v), dout))
+        monkeypatch.setattr(torch, "empty", empty)
+        assert len(refused) == (limit is None)
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
