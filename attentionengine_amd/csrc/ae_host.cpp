@@ -72,6 +72,7 @@ struct BwdPlan {
   int64_t work_more = 0;    // fp32 values of the work buffer behind its planes
   at::Tensor table_dq, table_dkv;     // tile classes of the two launches (mask mode 2)
   std::shared_ptr<Keep> keep;
+  std::shared_ptr<Keep> again;        // weak reference to the Python operator, which can do without `work_more` (or none)
 };
 
 struct Plan {
@@ -192,6 +193,29 @@ struct AeBackward : public torch::autograd::Node {
     q_.reset_data(), k_.reset_data(), v_.reset_data(), out_.reset_data();
     for (auto& s : scales_) s.reset_data();
   }
+  // (dq, dk, dv) from the operator behind the weak reference, called as a backward is the first time
+  static torch::autograd::variable_list in_python(const Keep& again, const std::vector<at::Tensor>& args) {
+    PyGILState_STATE g = PyGILState_Ensure();
+    PyObject *op = PyObject_CallObject(again.obj, nullptr), *res = nullptr;
+    torch::autograd::variable_list grads;
+    if (op && op != Py_None) {
+      PyObject* t = PyTuple_New((Py_ssize_t)args.size());
+      for (size_t i = 0; t && i < args.size(); i++) PyTuple_SET_ITEM(t, (Py_ssize_t)i, THPVariable_Wrap(args[i]));
+      res = t ? PyObject_CallObject(op, t) : nullptr;
+      Py_XDECREF(t);
+      for (Py_ssize_t i = 0; res && PyTuple_Check(res) && i < PyTuple_GET_SIZE(res); i++)
+        grads.push_back(THPVariable_Unpack(PyTuple_GET_ITEM(res, i)));
+    }
+    const bool failed = PyErr_Occurred() != nullptr;
+    python_error err;
+    if (failed) err.persist();
+    Py_XDECREF(res);
+    Py_XDECREF(op);
+    PyGILState_Release(g);
+    if (failed) throw err;
+    TORCH_CHECK_WITH(OutOfMemoryError, grads.size() == 3, "no memory for the work buffer of the backward, and its operator is gone");
+    return grads;
+  }
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     if (!grads[0].defined()) return torch::autograd::variable_list(3);
@@ -205,8 +229,14 @@ struct AeBackward : public torch::autograd::Node {
     if (!readable(dout)) dout = dout.contiguous();
     const int dev = q.get_device();
     const int64_t B = q.size(0), Sq = q.size(1), Hq = q.size(2), Skv = k.size(1), Hkv = k.size(2);
+    at::Tensor work;
+    try {
+      work = empty({pl.planes * B * Hq * Sq + pl.work_more}, at::kFloat, dev);
+    } catch (const c10::OutOfMemoryError&) {
+      if (!pl.again) throw;
+    }
+    if (!work.defined()) return in_python(*pl.again, {q, k, v, out, rs[0], dout});
     at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
-    at::Tensor work = empty({pl.planes * B * Hq * Sq + pl.work_more}, at::kFloat, dev);
     ae_attn_bwd_params p{};
     p.q = q.const_data_ptr(), p.k = k.const_data_ptr(), p.v = v.const_data_ptr(), p.out = out.const_data_ptr();
     p.dout = dout.const_data_ptr();
@@ -541,6 +571,8 @@ PyObject* host_add_backward(PyObject* self, PyObject* d) {
   bw->dkv_parts = (int)get_int(d, "dkv_parts"), bw->work_more = get_int(d, "work_more");
   bw->table_dq = get_tensor(d, "table_dq"), bw->table_dkv = get_tensor(d, "table_dkv");
   bw->keep = std::make_shared<Keep>(PyDict_GetItemString(d, "keep"));
+  PyObject* again = PyDict_GetItemString(d, "again");
+  if (again && again != Py_None) bw->again = std::make_shared<Keep>(again);
   for (auto& pl : *h->plans)
     if (pl->kind == kPrefill && pl->B == get_int(d, "B") && pl->Sq == get_int(d, "Sq") && pl->Hq == get_int(d, "Hq") &&
         pl->Hkv == get_int(d, "Hkv") && pl->Skv == get_int(d, "Skv") && pl->device == (int)get_int(d, "device"))

@@ -524,7 +524,7 @@ def test_when_ds_is_kept(cuda_device):
 
 @pytest.mark.gpu
 def test_no_memory_for_ds(cuda_device, monkeypatch):
-    """A first backward whose ds cannot be had takes the two launches, as one that may not keep it does."""
+    """A backward whose ds cannot be had takes the two launches, as one that may not keep it does."""
     B, H, S = 1, 16, 2048
     q, k, v = (t.cuda().requires_grad_(True) for t in C.make_inputs(B, S, S, H, H, 128, 128, torch.bfloat16, seed=3))
     dout = torch.randn(B, S, H, 128, device="cuda", dtype=torch.bfloat16)
@@ -547,3 +547,23 @@ def test_no_memory_for_ds(cuda_device, monkeypatch):
         monkeypatch.setattr(torch, "empty", empty)
         assert len(refused) == (limit is None)
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+    # natively, from the second call of a shape on: the allocator may take less than ds (284 MB) needs
+    S = 4096
+    q, k, v = (t.cuda().requires_grad_(True) for t in C.make_inputs(B, S, S, H, H, 128, 128, torch.bfloat16, seed=4))
+    dout = torch.randn(B, S, H, 128, device="cuda", dtype=torch.bfloat16)
+    for limit in (0, None):
+        op.work_limit = limit
+        want = [torch.autograd.grad(op(q, k, v), (q, k, v), dout) for _ in range(2)]
+        if limit == 0:
+            grads = want[1]
+    assert bwd.keeps_ds(B, H, S, S, 1, False) and not torch.equal(grads[0], want[1][0])
+    del want
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (160 << 20)) / total)
+    try:
+        again = torch.autograd.grad(op(q, k, v), (q, k, v), dout)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert all(torch.equal(a, b) for a, b in zip(grads, again))
