@@ -618,7 +618,7 @@ class PrefillOp:
         build.  48 shapes (batch 1 to 8, 8 to 32 heads, 1 to 25 rows, 512 to 16384 keys, head dims 64 and 128), time of the call in
         units of that with two launches: 0.94 on average, 0.81 to 1.003 (D64 B3 H8 Sq8 Skv764, 8 splits, 9.9 us -> 8.0; D128
         B4 H32 Sq5 Skv1496, 2 splits, 23.2 -> 21.8; B4 H16 Sq12 Skv14418, 4 splits, 89.4 -> 89.6).  Beyond: 8192 to 16384
-        values 0.92 to 1.20, 10 to 15 splits 0.95 to 1.06."""
+        values 0.92 to 1.20, 9 to 12 splits 0.93 to 1.10 (the more, the faster the host), 13 to 16 0.95 to 1.18."""
         return (1 < n_split <= self.MERGED_SPLITS and self._can_merge_in_last(tiles)
                 and min(Sq, tiles.block_m) * n_split * self.DV <= self.MERGED_VALUES
                 and tiles.block_m * Hq * n_split * self.DV < 2**29)
