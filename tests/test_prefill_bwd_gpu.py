@@ -522,6 +522,26 @@ def test_when_ds_is_kept(cuda_device):
     assert not bwd.keeps_ds(4, 32, 2048, 2048, 1, False)
 
 
+def test_a_backward_keeps_no_work_buffer(cuda_device):
+    """The first backward of a shape, through Python, and later native ones leave their gradients allocated and no more: not
+    ds (71 MB here), nor the row sums, nor what they were called with."""
+    B, H, S, D = 1, 16, 2048, 128
+    mod = _engine(B, H, H, S, D, D, torch.bfloat16, C.causal_mask, 1 / math.sqrt(D))
+    bwd = mod.attention.backward_op()
+    bwd.dkv_parts = lambda *a: 1
+    assert bwd.keeps_ds(B, H, S, S, 1, False)
+    q, k, v = (t.cuda().requires_grad_(True) for t in C.make_inputs(B, S, S, H, H, D, D, torch.bfloat16, seed=9))
+    for _ in range(3):
+        out = mod(q, k, v)
+        before = torch.cuda.memory_allocated()
+        dout = torch.ones_like(out)
+        grads = torch.autograd.grad(out, (q, k, v), dout)
+        del dout
+        kept = torch.cuda.memory_allocated() - before - sum(g.numel() * g.element_size() for g in grads)
+        assert kept <= 0, kept
+        del grads, out
+
+
 @pytest.mark.gpu
 def test_no_memory_for_ds(cuda_device, monkeypatch):
     """A backward whose ds cannot be had takes the two launches, as one that may not keep it does."""
