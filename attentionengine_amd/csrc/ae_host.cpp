@@ -229,14 +229,14 @@ struct AeBackward : public torch::autograd::Node {
     if (!readable(dout)) dout = dout.contiguous();
     const int dev = q.get_device();
     const int64_t B = q.size(0), Sq = q.size(1), Hq = q.size(2), Skv = k.size(1), Hkv = k.size(2);
-    at::Tensor work;
+    at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), work;     // (in front of ds, which a call can do without)
     try {
       work = empty({pl.planes * B * Hq * Sq + pl.work_more}, at::kFloat, dev);
     } catch (const c10::OutOfMemoryError&) {
       if (!pl.again) throw;
+      dq.reset(), dk.reset(), dv.reset();
     }
     if (!work.defined()) return in_python(*pl.again, {q, k, v, out, rs[0], dout});
-    at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     ae_attn_bwd_params p{};
     p.q = q.const_data_ptr(), p.k = k.const_data_ptr(), p.v = v.const_data_ptr(), p.out = out.const_data_ptr();
     p.dout = dout.const_data_ptr();

@@ -17,6 +17,13 @@ from oracle import masks as M
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def _nothing_cached():
+    """Tests that limit the allocator's memory count on no room inside what earlier tests' tensors left to it."""
+    if torch.cuda.is_available():
+        torch.cuda.empty_cache()
+
+
 class OnlineSoftmaxTwoScales(C.OnlineSoftmax):
     """The online softmax of attn_script/mha.py with its reference point and its row sum exported as TWO final row
     scales (instead of their combination lse), and the recompute / backward rules written against both, in the
@@ -587,3 +594,48 @@ def test_no_memory_for_ds(cuda_device, monkeypatch):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert all(torch.equal(a, b) for a, b in zip(grads, again))
+
+
+class _MemoryLeft:
+    """Inside, torch's allocator has ``mib`` MiB beyond what it holds."""
+
+    def __init__(self, mib):
+        self.mib = mib
+
+    def __enter__(self):
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        total = torch.cuda.get_device_properties(0).total_memory
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (self.mib << 20)) / total)
+
+    def __exit__(self, *exc):
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+def _ds_engine(S, limit=None, B=1, H=16):
+    mod = _engine(B, H, H, S, 128, 128, torch.bfloat16, C.causal_mask, 0.1)
+    mod.attention.work_limit = limit
+    bwd = mod.attention.backward_op()
+    bwd.dkv_parts = lambda *a: 1
+    assert bwd.keeps_ds(B, H, S, S, 1, False) == (limit is None)
+    q, k, v = (t.cuda().requires_grad_(True) for t in C.make_inputs(B, S, S, H, H, 128, 128, torch.bfloat16, seed=4))
+    dout = torch.randn(B, S, H, 128, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16).cuda()
+    return mod, lambda: mod(q, k, v), lambda out: torch.autograd.grad(out, (q, k, v), dout)
+
+
+def _same(a, b):
+    return all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("natively", [False, True])
+def test_memory_for_ds_but_not_for_the_gradients_beside_it(cuda_device, natively):
+    """264 MiB of ds and 48 MiB of gradients where 290 are left: the launches that need no ds run, as they did before."""
+    _, forward, backward = _ds_engine(4096, limit=0)
+    two = backward(forward())
+    _, forward, backward = _ds_engine(4096)
+    if natively:
+        assert not _same(backward(forward()), two)
+    out = forward()
+    with _MemoryLeft(290):
+        got = backward(out)
+    assert _same(got, two)
