@@ -66,10 +66,12 @@ def add_forward(host, kind, B, Sq, Hq, Hkv, Skv, device, modules, kernel, cfg, c
 
 
 def add_backward(host, B, Sq, Hq, Hkv, Skv, device, modules, delta, dkv, dq, cfg, n_rs, planes, tables=None, dkv_parts=0,
-                 work_more=0, again=None):
+                 work_more=0, again=None, retry=0, skip=0):
     """Hands the backward launches of the forward plan with these extents to ``host``.  ``work_more``: fp32 values of the
-    work buffer behind its planes; ``again``: weak reference to the operator that is called instead where they cannot be had."""
+    work buffer behind its planes; ``again``: weak reference to the operator that is called instead where they cannot be had,
+    then for the next ``retry`` calls too, and for the first ``skip``."""
     host.add_backward({"B": B, "Sq": Sq, "Hq": Hq, "Hkv": Hkv, "Skv": Skv, "device": device.index,
                        "delta": _handle(delta), "dkv": _handle(dkv), "dq": _handle(dq), "cfg": bytes(cfg), "n_rs": n_rs,
                        "planes": planes, "dkv_parts": dkv_parts, "work_more": work_more, "table_dq": tables[0] if tables else None,
-                       "table_dkv": tables[1] if tables else None, "keep": tuple(modules), "again": again})
+                       "table_dkv": tables[1] if tables else None, "keep": tuple(modules), "again": again,
+                       "retry": retry, "skip": skip})

@@ -32,6 +32,7 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
+#include <atomic>
 #include <cstdlib>
 #include <memory>
 #include <string>
@@ -72,7 +73,9 @@ struct BwdPlan {
   int64_t work_more = 0;    // fp32 values of the work buffer behind its planes
   at::Tensor table_dq, table_dkv;     // tile classes of the two launches (mask mode 2)
   std::shared_ptr<Keep> keep;
-  std::shared_ptr<Keep> again;        // weak reference to the Python operator, which can do without `work_more` (or none)
+  std::shared_ptr<Keep> again;        // weak reference to the Python operator, which can do without `work_more` (or none) ...
+  int retry = 0;                      // ... and is called this many times more once it has been refused
+  std::atomic<int> skip{0};           // calls left of these
 };
 
 struct Plan {
@@ -193,16 +196,17 @@ struct AeBackward : public torch::autograd::Node {
     q_.reset_data(), k_.reset_data(), v_.reset_data(), out_.reset_data();
     for (auto& s : scales_) s.reset_data();
   }
-  // (dq, dk, dv) from the operator behind the weak reference, called as a backward is the first time
+  // (dq, dk, dv) from the operator behind the weak reference: a call of it that keeps no ds
   static torch::autograd::variable_list in_python(const Keep& again, const std::vector<at::Tensor>& args) {
     PyGILState_STATE g = PyGILState_Ensure();
     PyObject *op = PyObject_CallObject(again.obj, nullptr), *res = nullptr;
     torch::autograd::variable_list grads;
     if (op && op != Py_None) {
-      PyObject* t = PyTuple_New((Py_ssize_t)args.size());
+      PyObject *t = PyTuple_New((Py_ssize_t)args.size()), *more = Py_BuildValue("{s:O}", "without_ds", Py_True);
       for (size_t i = 0; t && i < args.size(); i++) PyTuple_SET_ITEM(t, (Py_ssize_t)i, THPVariable_Wrap(args[i]));
-      res = t ? PyObject_CallObject(op, t) : nullptr;
+      res = t && more ? PyObject_Call(op, t, more) : nullptr;
       Py_XDECREF(t);
+      Py_XDECREF(more);
       for (Py_ssize_t i = 0; res && PyTuple_Check(res) && i < PyTuple_GET_SIZE(res); i++)
         grads.push_back(THPVariable_Unpack(PyTuple_GET_ITEM(res, i)));
     }
@@ -220,7 +224,7 @@ struct AeBackward : public torch::autograd::Node {
     std::lock_guard<std::mutex> lock(mutex_);
     if (!grads[0].defined()) return torch::autograd::variable_list(3);
     at::NoGradGuard no_grad;
-    const BwdPlan& pl = *plan;
+    BwdPlan& pl = *plan;
     const at::Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack(), out = out_.unpack(shared_from_this());
     std::vector<at::Tensor> rs;
     for (auto& s : scales_) rs.push_back(s.unpack());
@@ -229,12 +233,14 @@ struct AeBackward : public torch::autograd::Node {
     if (!readable(dout)) dout = dout.contiguous();
     const int dev = q.get_device();
     const int64_t B = q.size(0), Sq = q.size(1), Hq = q.size(2), Skv = k.size(1), Hkv = k.size(2);
+    if (pl.skip > 0 && pl.skip-- > 0) return in_python(*pl.again, {q, k, v, out, rs[0], dout});
     at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), work;     // (in front of ds, which a call can do without)
     try {
       work = empty({pl.planes * B * Hq * Sq + pl.work_more}, at::kFloat, dev);
     } catch (const c10::OutOfMemoryError&) {
       if (!pl.again) throw;
       dq.reset(), dk.reset(), dv.reset();
+      pl.skip = pl.retry;
     }
     if (!work.defined()) return in_python(*pl.again, {q, k, v, out, rs[0], dout});
     ae_attn_bwd_params p{};
@@ -572,7 +578,8 @@ PyObject* host_add_backward(PyObject* self, PyObject* d) {
   bw->table_dq = get_tensor(d, "table_dq"), bw->table_dkv = get_tensor(d, "table_dkv");
   bw->keep = std::make_shared<Keep>(PyDict_GetItemString(d, "keep"));
   PyObject* again = PyDict_GetItemString(d, "again");
-  if (again && again != Py_None) bw->again = std::make_shared<Keep>(again);
+  if (again && again != Py_None)
+    bw->again = std::make_shared<Keep>(again), bw->retry = (int)get_int(d, "retry"), bw->skip = (int)get_int(d, "skip");
   for (auto& pl : *h->plans)
     if (pl->kind == kPrefill && pl->B == get_int(d, "B") && pl->Sq == get_int(d, "Sq") && pl->Hq == get_int(d, "Hq") &&
         pl->Hkv == get_int(d, "Hkv") && pl->Skv == get_int(d, "Skv") && pl->device == (int)get_int(d, "device"))

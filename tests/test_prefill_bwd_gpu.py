@@ -639,3 +639,21 @@ def test_memory_for_ds_but_not_for_the_gradients_beside_it(cuda_device, natively
     with _MemoryLeft(290):
         got = backward(out)
     assert _same(got, two)
+
+
+@pytest.mark.parametrize("natively", [False, True])
+def test_a_refused_ds_is_asked_for_again(cuda_device, monkeypatch, natively):
+    """A moment without memory does not leave a shape with the slower launches: after DS_RETRY calls ds is tried again."""
+    from core.lower import prefill_bwd_op as B
+    monkeypatch.setattr(B, "DS_RETRY", 2, raising=False)
+    _, forward, backward = _ds_engine(4096, limit=0)
+    two = backward(forward())
+    _, forward, backward = _ds_engine(4096)
+    if natively:
+        backward(forward())
+    out = forward()
+    with _MemoryLeft(160):
+        assert _same(backward(out), two)
+    assert _same(backward(forward()), two) and _same(backward(forward()), two)
+    kept = backward(forward())
+    assert not _same(kept, two) and _same(kept, backward(forward()))
