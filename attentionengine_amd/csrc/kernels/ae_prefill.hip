@@ -573,6 +573,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
   static_assert(AE_RB == 1 && AE_WAVES_PER_EU >= 2, "one row block a wave, O in ordinary registers");
   bool by_maxima = true;      // (wave uniform) this trip takes the maxima: some row has no reference yet, or the sums were large
   bool again = false; // ... the trip is made once more for them: nothing is requested, nobody is waited for
+  bool sharp = false;          // ... has been made once more: every later trip takes the maxima
   float minus_ref = 0.f;       // the lane's row's reference, log2 units, negative
 #endif
   int stage = 0;
@@ -736,7 +737,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
         minus_ref = -ref * AE_LOG2E;
         st[rb].AE_SM_M = ref;
         st[rb].AE_SM_R *= o_scale;
-        by_maxima = __builtin_amdgcn_ballot_w64(ref <= -1e30f) != 0;
+        by_maxima = sharp || __builtin_amdgcn_ballot_w64(ref <= -1e30f) != 0;
         if (__builtin_amdgcn_ballot_w64(o_scale != 1.0f) != 0) {
 #pragma unroll
           for (int db = 0; db < AE_NDB; db++)
@@ -748,7 +749,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
       for (int e = 0; e < AE_NS; e++) s[e] = ae_exp2(__builtin_fmaf(s[e], AE_SM_SCALE * AE_LOG2E, minus_ref));
       const float sum = ae_lane_sum<AE_NS>(s);
       if (!took_maxima && __builtin_expect(__builtin_amdgcn_ballot_w64(!(sum <= AE_SUM_MOST)) != 0, 0)) {
-        by_maxima = again = true;
+        by_maxima = again = sharp = true;
       } else {
         st[rb].AE_SM_R += sum;
       }

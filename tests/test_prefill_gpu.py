@@ -1263,3 +1263,35 @@ def test_scores_that_are_no_numbers_reach_their_rows_only(cuda_device, D):
     rest = torch.arange(S) != 77
     # (the wave of a row without a number takes the maxima on every tile: another reference, another rounding)
     assert (out[1, rest].float() - clean[1, rest].float()).abs().max().item() <= 2.0 ** -10 * v.abs().max().item()
+
+
+def test_scores_that_outgrow_their_references_cost_one_trip_a_wave(cuda_device):
+    """AE_SUM_CHECK: in every tile of 64 keys some row of each wave meets a score far above all before it.  The first of them
+    sends its wave over to the row maxima; were every such tile multiplied twice, a launch would take 1.4 times as long."""
+    B, H, S, D = 16, 16, 1024, 64
+    meta = tuple(meta_tensor(B, H, S, D, dtype=torch.bfloat16) for _ in range(3))
+    eng = AttentionEngine(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), None, C.OnlineSoftmax())
+    assert "#define AE_SUM_CHECK 1" in eng.tl_code
+    i = torch.arange(S)
+    k = torch.zeros(S, D)
+    k[i, i // 64] = 1.0                                      # tile t's keys answer rows r with r % 16 == t: 25 nats
+    q = torch.zeros(S, D)
+    q[i, i % 16] = 25.0 * math.sqrt(D)
+    q, k = (t[None, :, None].expand(B, S, H, D).to(torch.bfloat16).cuda().contiguous() for t in (q, k))
+    v = C.make_inputs(1, S, S, 1, 1, D, D, torch.bfloat16, seed=2)[2].expand(B, S, H, D).cuda().contiguous()
+    flat = (q * 0.01).contiguous()
+    out = eng(q, k, v)[0, :, 0].float().cpu()
+    want = v[0, :, 0].float().cpu().view(16, 64, D).mean(1)[i % 16]
+    assert (out - want).abs().max().item() <= 2.0 ** -8 * want.abs().max().item() + 1e-5
+
+    def us(q):
+        a, b = torch.cuda.Event(True), torch.cuda.Event(True)
+        a.record()
+        for _ in range(50):
+            eng(q, k, v)
+        b.record()
+        b.synchronize()
+        return a.elapsed_time(b) * 20
+    us(q), us(flat)
+    times = [(us(flat), us(q)) for _ in range(7)]
+    assert min(t[1] for t in times) <= 1.25 * min(t[0] for t in times), times
