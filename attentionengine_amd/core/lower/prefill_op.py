@@ -641,10 +641,10 @@ class PrefillOp:
         v = self._variants.get(key)
         if v is None:
             has_mask_mod = self.elementwise_mask and mask_mode != 1
-            sum_check = tiles.template == "ae_prefill.hip" and self._pipe_softmax is not None and tiles.waves_per_eu >= 2
+            own_softmax = tiles.template == "ae_prefill.hip" and self._pipe_softmax is not None and tiles.waves_per_eu >= 2
             cfg_src = L.render_config(self.D, self.DV_launch, self.dtype, tiles, mask_mode, has_mask_mod,
                                       self.n_rowscales, self.functors.o_scale_one, even_q, even_kv,
-                                      self._pipe_softmax if tiles.rows_per_wave == 64 or tiles.kv_groups > 1 or sum_check else None,
+                                      self._pipe_softmax if tiles.rows_per_wave == 64 or tiles.kv_groups > 1 or own_softmax else None,
                                       elementwise=self._pipe_elementwise and tiles.rows_per_wave == 64,
                                       exact_scale=self.exact_scale)
             if self.mask_value_zero:
@@ -659,8 +659,8 @@ class PrefillOp:
             if band is not None:
                 cfg_src += (f"#define AE_BAND 1\n#define AE_BAND_LO ({band[0]})\n"
                             f"#define AE_BAND_HI {'0x7fffffff' if band[1] is None else f'({band[1]})'}\n")
-            if sum_check:
-                cfg_src += "#define AE_SUM_CHECK 1\n"
+            if own_softmax:
+                cfg_src += "#define AE_OWN_SOFTMAX 1\n"
             if n_split > 1:
                 cfg_src += "#define AE_NSPLIT 2\n"       # (a split launch; its count is the launch's)
                 if self._can_merge_in_last(tiles):

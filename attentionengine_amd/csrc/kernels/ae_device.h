@@ -255,11 +255,15 @@ AE_DEV float ae_group_sum(float v) {
 // (ReduceMax / ReduceSum / ReduceAbsSum over dim=1 of the [block_M, block_N] tile,
 //  core/codegen/tl_gen.py:9-21.)
 template <int N>
-AE_DEV float ae_row_max(const float (&s)[N]) {
+AE_DEV float ae_lane_max(const float (&s)[N]) {
   float m = s[0];
 #pragma unroll
   for (int e = 1; e < N; e++) m = __builtin_fmaxf(m, s[e]);
-  return ae_group_max(m);
+  return m;
+}
+template <int N>
+AE_DEV float ae_row_max(const float (&s)[N]) {
+  return ae_group_max(ae_lane_max<N>(s));
 }
 template <int N>
 AE_DEV float ae_lane_sum(const float (&s)[N]) {

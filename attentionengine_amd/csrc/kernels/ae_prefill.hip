@@ -141,21 +141,19 @@ static_assert(AE_NSPLIT > 1 && AE_KW > 1, "merged by the last workgroup: builds 
 #ifndef AE_RB
 #define AE_RB 1
 #endif
-// AE_SUM_CHECK 1 (the proven online softmax of score * AE_SM_SCALE, fields AE_SM_M and AE_SM_R): no row maxima in the common
-// trip.  The reference that the exponents are taken against may lag behind the running maximum as long as the weights fit
-// their type, and a weight that does not shows in the sum of its lane's weights, which is needed anyway: sums up to
-// AE_SUM_MOST go on; after a larger one (or a NaN) the wave makes the trip again - the tile is still in LDS, it requests
-// nothing and waits for nobody - and takes the maxima, as it does on its first tiles, until every row has a reference.  The
-// row sum stays per lane until the end.  These kernels are bound by the VALU at head dim 64 (70 % busy, 11.6 instructions an
-// MFMA): a tile's 32 scores of a lane take 132 VALU instructions instead of 160, row maxima and (below) addresses
-// together.  us: bf16 B16 H16 S1000 D64 85.8 -> 83.2, causal B2 H32/8 S3407 D64 115.7 -> 111.2, B17 H32 S577 75.5 -> 73.6,
-// window of 256, B2 H32 S4096 D128 fp16 75.5 -> 74.1; causal D128 0 to 1 %.
-// (As a way back inside the trip instead of a trip of its own, the compiler keeps 20 registers more through all of it.)
-#ifndef AE_SUM_CHECK
-#define AE_SUM_CHECK 0
+// AE_OWN_SOFTMAX 1 (the proven online softmax of score * AE_SM_SCALE, fields AE_SM_M and AE_SM_R): written out here.  A row's
+// reference moves where a score exceeds it by AE_SM_TAU, which a lane sees by itself: two lanes share a row, and only where some
+// lane of the wave has such a score do they exchange their maxima and does anything move.  The row sum stays per lane until
+// the end.  These kernels are bound by the VALU at head dim 64.  us, generated functors (which exchange maxima and sums on every
+// tile) -> this, addresses by constants (below) included, at scores with a standard deviation of 1 | 4 | 16: bf16 B16 H16 S1000
+// D64 86.3 -> 83.3 | 90.0 -> 88.0 | 91.7 -> 90.4, causal B2 H32/8 S3407 D64 116.1 -> 110.5 | 118.8 -> 115.2 | 120.6 -> 118.5,
+// B4 H32 S1500 D128 99.6 -> 97.8 | 102.7 -> 101.5 | 104.5 -> 103.8, B1 H128 S2500 192 / 128 columns 290 -> 275 | 302 -> 290 |
+// 307 -> 297.  (Without any maxima, a tile whose weights' sum is too large multiplied again: 84 | 86.7 | 119.5 for the
+// first, 281 | 290 | 359 for the last; and what one row makes its wave do twice changed the rounding of the others.)
+#ifndef AE_OWN_SOFTMAX
+#define AE_OWN_SOFTMAX 0
 #endif
-#define AE_SUM_MOST 32768.f        // (half of what fp16 holds)
-#define AE_SM_TAU 5.545177444479562f     // the reference moves when a maximum exceeds it by 8 log2 units
+#define AE_SM_TAU 5.545177444479562f     // 8 log2 units: weights up to 256
 #define AE_WROWS (AE_RB * 32)     // query rows per wave
 #define AE_BM (AE_NWAVES * AE_WROWS)
 #define AE_GT (AE_NWAVES * 64)     // threads of a kv group
@@ -569,11 +567,8 @@ void ae_prefill_kernel(const ae_attn_params p) {
   __syncthreads();      // every wave has its fragments before the next request refills the rows' stages
 #endif
 
-#if AE_SUM_CHECK
+#if AE_OWN_SOFTMAX
   static_assert(AE_RB == 1 && AE_WAVES_PER_EU >= 2, "one row block a wave, O in ordinary registers");
-  bool by_maxima = true;      // (wave uniform) this trip takes the maxima: some row has no reference yet, or the sums were large
-  bool again = false; // ... the trip is made once more for them: nothing is requested, nobody is waited for
-  bool sharp = false;          // ... has been made once more: every later trip takes the maxima
   float minus_ref = 0.f;       // the lane's row's reference, log2 units, negative
 #endif
   int stage = 0;
@@ -586,9 +581,6 @@ void ae_prefill_kernel(const ae_attn_params p) {
     int cls_n[AE_RB];
 #pragma unroll
     for (int rb = 0; rb < AE_RB; rb++) cls_n[rb] = row_class(jn, rb);
-#if AE_SUM_CHECK
-    if (__builtin_expect(!again, 1))
-#endif
 #if AE_DEEP
     request_next();                              // into the stage that the last trip left
 #else
@@ -727,32 +719,25 @@ void ae_prefill_kernel(const ae_attn_params p) {
       }
 #endif
 
-#if AE_SUM_CHECK
-      const bool took_maxima = by_maxima;
-      if (by_maxima) {
-        again = false;
-        const float top = ae_row_max<AE_NS>(s) * AE_SM_SCALE;
-        const float ref = top - st[rb].AE_SM_M > AE_SM_TAU ? top : st[rb].AE_SM_M;
-        const float o_scale = ae_exp(st[rb].AE_SM_M - ref);
+#if AE_OWN_SOFTMAX
+      const float lane_top = ae_lane_max<AE_NS>(s);
+      float over = __builtin_fmaf(lane_top, AE_SM_SCALE, -st[rb].AE_SM_M);
+      if (__builtin_amdgcn_ballot_w64(over > AE_SM_TAU) != 0) {      // (the first tile; seldom later)
+        over = ae_group_max(over);
+        const float ref = over > AE_SM_TAU ? ae_group_max(lane_top) * AE_SM_SCALE : st[rb].AE_SM_M;
+        const float o_scale = ae_exp(st[rb].AE_SM_M - ref);          // (1 for rows whose reference stays)
         minus_ref = -ref * AE_LOG2E;
         st[rb].AE_SM_M = ref;
         st[rb].AE_SM_R *= o_scale;
-        by_maxima = sharp || __builtin_amdgcn_ballot_w64(ref <= -1e30f) != 0;
-        if (__builtin_amdgcn_ballot_w64(o_scale != 1.0f) != 0) {
 #pragma unroll
-          for (int db = 0; db < AE_NDB; db++)
+        for (int db = 0; db < AE_NDB; db++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) oacc[rb][db][r] *= o_scale;
-        }
+          for (int r = 0; r < 16; r++) oacc[rb][db][r] *= o_scale;
       }
 #pragma unroll
       for (int e = 0; e < AE_NS; e++) s[e] = ae_exp2(__builtin_fmaf(s[e], AE_SM_SCALE * AE_LOG2E, minus_ref));
-      const float sum = ae_lane_sum<AE_NS>(s);
-      if (!took_maxima && __builtin_expect(__builtin_amdgcn_ballot_w64(!(sum <= AE_SUM_MOST)) != 0, 0)) {
-        by_maxima = again = sharp = true;
-      } else {
-        st[rb].AE_SM_R += sum;
-      }
+      st[rb].AE_SM_R += ae_lane_sum<AE_NS>(s);
+      asm("" : "+v"(st[rb].AE_SM_R));          // (now: put off, the weights stay beside their fragments, 13 registers more)
 #else
       // ---- user functors ----------------------------------------------------------------------
 #if defined(AE_HAS_KV_PREFETCH) && AE_KV_COALESCED
@@ -787,7 +772,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
           pf[rb][kk][t + 1] = y2[1];
         }
 
-#if !AE_O_SCALE_ONE && !AE_SUM_CHECK
+#if !AE_O_SCALE_ONE && !AE_OWN_SOFTMAX
       // skip the rescale when no row of this block changed its scale (wave-uniform branch)
       if (__builtin_amdgcn_ballot_w64(o_scale != 1.0f) != 0) {
 #pragma unroll
@@ -806,16 +791,12 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #endif
           }
       }
-#elif !AE_SUM_CHECK
+#elif !AE_OWN_SOFTMAX
       (void)o_scale;
 #endif
     }
 
     // ---- O^T += V^T P^T: every V fragment feeds one MFMA per row block ------------------------
-#if AE_SUM_CHECK
-    if (__builtin_expect(!again, 1))
-#endif
-    {
     unsigned v_at = (unsigned)(unsigned long)vs_ + v_lane;
     asm("" : "+v"(v_at));
     auto v_frag = [&](int f) AE_LAMBDA -> ae_elem8 {
@@ -844,11 +825,6 @@ void ae_prefill_kernel(const ae_attn_params p) {
       AE_RING_FENCE();
     }
     }
-    }
-#if AE_SUM_CHECK
-    if (__builtin_expect(!again, 1))
-#endif
-    {
 
     // the next tile must have landed before anyone reads it: direct loads are tracked by vmcnt
 #if AE_DEEP
@@ -866,11 +842,10 @@ void ae_prefill_kernel(const ae_attn_params p) {
 #endif
 #pragma unroll
     for (int rb = 0; rb < AE_RB; rb++) cls[rb] = cls_n[rb];
-    }
   }
 
   // ---- epilogue -------------------------------------------------------------------------------
-#if AE_SUM_CHECK
+#if AE_OWN_SOFTMAX
   st[0].AE_SM_R = ae_group_sum(st[0].AE_SM_R);
 #endif
 #if AE_KW > 1
