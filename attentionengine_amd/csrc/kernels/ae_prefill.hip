@@ -154,6 +154,15 @@ static_assert(AE_NSPLIT > 1 && AE_KW > 1, "merged by the last workgroup: builds 
 #define AE_OWN_SOFTMAX 0
 #endif
 #define AE_SM_TAU 5.545177444479562f     // 8 log2 units: weights up to 256
+// AE_FIRST_REST 1 (split launches whose tiles PrefillOp._cheapest_form chooses): what the rounding of its first tile's weights
+// leaves over is multiplied as well.  The largest weight of every reference is 1, which has no rounding error, and the
+// plans with fewer splits and kv groups have fewer references: by that alone the error against fp64 was 1.019 of what four
+// groups and a split for every CU gave (40 shapes of 1 to 256 rows, 512 to 16384 keys, N(0, 1) scores; 1.08 at most), the more the
+// shorter the cache.  So it is 0.988 (1.02), and 0.997 on 50 shapes of more than 32 rows (1.012 without).  0.2 to 0.3 us a call
+// (1.6 % of 60 calls of 9 to 330 us; every tile's: 7 %, error 0.74; the references that there were, by the plan: 3.5 % and more).
+#ifndef AE_FIRST_REST
+#define AE_FIRST_REST 0
+#endif
 #define AE_WROWS (AE_RB * 32)     // query rows per wave
 #define AE_BM (AE_NWAVES * AE_WROWS)
 #define AE_GT (AE_NWAVES * 64)     // threads of a kv group
@@ -571,6 +580,10 @@ void ae_prefill_kernel(const ae_attn_params p) {
   static_assert(AE_RB == 1 && AE_WAVES_PER_EU >= 2, "one row block a wave, O in ordinary registers");
   float minus_ref = 0.f;       // the lane's row's reference, log2 units, negative
 #endif
+#if AE_FIRST_REST
+  static_assert(AE_OWN_SOFTMAX, "weights up to 256");
+  bool first = true;
+#endif
   int stage = 0;
   while (AE_TRIPS_LEFT) {
 #if AE_ROTATE
@@ -643,6 +656,20 @@ void ae_prefill_kernel(const ae_attn_params p) {
       AE_RING_FENCE();
     }
 
+    unsigned v_at = (unsigned)(unsigned long)vs_ + v_lane;
+    asm("" : "+v"(v_at));
+    auto v_frag = [&](int f) AE_LAMBDA -> ae_elem8 {
+      // slots 0..3 of k-step kk are kv rows rb0+4*hf+0..3, slots 4..7 rows rb0+8+4*hf+0..3
+      // (rb0 and +8 are multiples of 8, so they do not change the swizzle)
+      const int kk = f / AE_NDB;
+      const int rb0 = (kk >> 1) * 32 + (kk & 1) * 16;
+      const int pair = 2 * (f % AE_NDB);
+      const ae_lds_byte* a0 = (const ae_lds_byte*)(v_at ^ (unsigned)((pair & AE_VSWM) << 5)) + ((pair & ~AE_VSWM) << 5) + rb0 * AE_VSTR;
+      ae_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)a0);
+      ae_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (__attribute__((address_space(3))) ae_s16x4*)(a0 + 8 * AE_VSTR));
+      return __builtin_bit_cast(ae_elem8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
     ae_elem8 pf[AE_RB][AE_BN / 16];
 #pragma unroll
     for (int rb = 0; rb < AE_RB; rb++) {
@@ -772,6 +799,20 @@ void ae_prefill_kernel(const ae_attn_params p) {
           pf[rb][kk][t + 1] = y2[1];
         }
 
+#if AE_FIRST_REST
+      if (first) {
+        first = false;
+#pragma unroll
+        for (int kk = 0; kk < AE_BN / 16; kk++) {
+          ae_elem8 rest;
+#pragma unroll
+          for (int t = 0; t < 8; t++) rest[t] = (ae_elem)(s[kk * 8 + t] - (float)pf[rb][kk][t]);
+#pragma unroll
+          for (int db = 0; db < AE_NDB; db++) oacc[rb][db] = ae_mfma32(v_frag(kk * AE_NDB + db), rest, oacc[rb][db]);
+        }
+      }
+#endif
+
 #if !AE_O_SCALE_ONE && !AE_OWN_SOFTMAX
       // skip the rescale when no row of this block changed its scale (wave-uniform branch)
       if (__builtin_amdgcn_ballot_w64(o_scale != 1.0f) != 0) {
@@ -797,20 +838,6 @@ void ae_prefill_kernel(const ae_attn_params p) {
     }
 
     // ---- O^T += V^T P^T: every V fragment feeds one MFMA per row block ------------------------
-    unsigned v_at = (unsigned)(unsigned long)vs_ + v_lane;
-    asm("" : "+v"(v_at));
-    auto v_frag = [&](int f) AE_LAMBDA -> ae_elem8 {
-      // slots 0..3 of k-step kk are kv rows rb0+4*hf+0..3, slots 4..7 rows rb0+8+4*hf+0..3
-      // (rb0 and +8 are multiples of 8, so they do not change the swizzle)
-      const int kk = f / AE_NDB;
-      const int rb0 = (kk >> 1) * 32 + (kk & 1) * 16;
-      const int pair = 2 * (f % AE_NDB);
-      const ae_lds_byte* a0 = (const ae_lds_byte*)(v_at ^ (unsigned)((pair & AE_VSWM) << 5)) + ((pair & ~AE_VSWM) << 5) + rb0 * AE_VSTR;
-      ae_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)a0);
-      ae_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (__attribute__((address_space(3))) ae_s16x4*)(a0 + 8 * AE_VSTR));
-      return __builtin_bit_cast(ae_elem8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-    };
     constexpr int NVF = (AE_BN / 16) * AE_NDB;
     ae_elem8 vring[AE_V_AHEAD + 1];
 #pragma unroll

@@ -282,6 +282,34 @@ def test_three_tile_stages(cuda_device, form, Sq):
             assert (op.final_rowscales["lse"].cpu() - lse).abs().max().item() <= 1e-3
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("form,Sq", [("32", 5), ("64", 61), ("128", 100), ("256", 200)])
+def test_the_first_tile_leaves_no_rounding_of_weights(cuda_device, form, Sq, dtype):
+    """AE_FIRST_REST: where only the first 32 keys count, the result is as good as its own rounding, at every edge of the cache;
+    with one split and with two."""
+    B, H, D = 2, 3, 128
+    for Skv, n in ((31, 1), (32, 1), (300, 1), (700, 2)):
+        print(f"case first tile {form} Sq{Sq} Skv{Skv} splits {n} {dtype}", flush=True)
+        q, k, v = C.make_inputs(B, Sq, Skv, H, H, D, D, dtype, seed=Skv + Sq)
+        q[..., 0] = 40.0
+        k[..., 0] = 0.0
+        k[:, 32:, :, 0] = -20.0                       # 70 nats below
+        op = _engine(Sq, None, H=H, Hkv=H, B=B, Skv=4096, dtype=dtype)._op
+        tiles = PrefillTiles(**op.SPLIT_FORMS[form][0])
+        op._launch_tiles = lambda *a: tiles
+        op.plan_splits = lambda *a: (n, -(-Skv // (64 * n)) * 64)
+        p = torch.softmax(torch.einsum("bqhd,bkhd->bhqk", q.double(), k.double()) / math.sqrt(D), -1)
+        ref = torch.einsum("bhqk,bkhd->bqhd", p, v.double())
+        # u = 2^-8 or 2^-11 (8 or 11 significant bits): the result's rounding is within u |result|, a weight's and then its rest's
+        # within u^2 of it, and the weights sum to 1; 2^-18 for fp32 scores of at most 2^4, exponentials and sums
+        u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+        bound = u * ref.abs() + (u * u + 2.0 ** -18) * v.abs().max().item()
+        for _ in range(2):
+            err = (op(q.cuda(), k.cuda(), v.cuda()).cpu().double() - ref).abs()
+            assert (err <= bound).all(), (err - bound).max().item()
+
+
 def test_which_split_launches_merge_in_their_last_workgroup():
     op = _engine(8, None, H=8, Hkv=8, Skv=4096)._op
     forms = {n: PrefillTiles(**f[0]) for n, f in op.SPLIT_FORMS.items()}
