@@ -413,13 +413,25 @@ class PrefillOp:
     def _launch_tiles(self, B, H, Sq, Skv, tiles):
         """The tiles of a split launch with these extents: those of ``SPLIT_FORMS`` that cost least instead of ``tiles``
         (``tiles_for``), where the graph allows them.  Not at other head dims, nor where 128- or 256-row tiles fill the chip
-        without a split (two workgroups a CU then hide each other's waits: B10 H32 Sq108 Skv2102 79 us, 92 with three stages)."""
+        without a split (two workgroups a CU then hide each other's waits: B10 H32 Sq108 Skv2102 79 us, 92 with three stages),
+        nor where ``tiles`` are one launch that is as good (``_own_tiles_pay``)."""
         if (not self.split_kv or self.mask_mod is not None or (self.D, self.DV) != (128, 128) or self._tiles_given
                 or not (B and H and Sq and Skv) or Sq > 256 or (Sq > 64 and -(-(B * H) // 8) * 8 > self.target_workgroups)
-                or not self._groups_can_meet()):
+                or not self._groups_can_meet() or self._own_tiles_pay(B, H, Sq, Skv, tiles)):
             return tiles
         names = ("32",) if Sq <= 32 else ("64",) if Sq <= 64 else ("64", "128", "256")
         return L.PrefillTiles(**self.SPLIT_FORMS[self._cheapest_form(names, B * H, Sq, -(-Skv // 32), self.target_workgroups)[0]][0])
+
+    def _own_tiles_pay(self, B, H, Sq, Skv, tiles):
+        """Whether up to 64 rows keep ``tiles``: one split of them, with two stages, against the cheapest of ``SPLIT_FORMS``.  Short
+        caches, where four kv groups share the trips (32-row tiles) and no partial result is written, up to a number of heads:
+        B3 H32 Sq30 Skv704 12.9 -> 11.2 us, B3 H16 Sq19 Skv353 9.6 -> 7.7, B3 H32 Sq37 Skv651 14.2 -> 12.7; 0.956 of the time
+        on 101 shapes of at most 32 rows (1.06 at most); but B5 H32 Sq45 Skv500 1.11.  More than 32 rows of more heads than there
+        are CUs: two workgroups share a CU, with three stages the last ones wait for a place: B9 H32 Sq61 Skv521 28.7 -> 23.2, B16 H32
+        Sq61 Skv521 35.5 -> 31.2, 0.80 of the time up to 800 keys, 0.97 at 3000 to 4000, where the plan starts to split."""
+        heads, cus = B * H, self.target_workgroups
+        short = Skv <= 768 and heads <= (cus * 5 // 8 if Sq <= 32 else cus // 2)
+        return Sq <= 64 and (short or (Sq > 32 and heads > cus)) and self.plan_splits(B, H, Sq, Skv, tiles)[0] == 1
 
     def _split_form_of(self, tiles):
         """The name in ``SPLIT_FORMS`` of tiles that ``_launch_tiles`` chose, or None."""
@@ -436,7 +448,8 @@ class PrefillOp:
         to 16384 keys, bf16), 3.6 % off in the root mean square; the choice is 0.6 % off the best measured on average and
         takes 0.93 of the time of two stages with a split for every CU (1.05 at most).  us: B6 H32 Sq50 Skv2562 60 -> 51,
         B8 H8 Sq115 Skv521 15.9 -> 12.2, B1 H16 Sq4 Skv8393 20.7 -> 19.2, B5 H32 Sq216 Skv3498 112 -> 99, B1 H32 Sq128 Skv8192
-        42.2 -> 39.4; B5 H32 Sq61 Skv15254 232 -> 244."""
+        42.2 -> 39.4.  Splits that take a second round where one split would not start and drain twice, 12 % of
+        the read by 3600 shapes: B5 H32 Sq61 Skv15254, 232 with two stages, 244 with three splits, 226 with one."""
         read = heads * kv_tiles * 32 * 512e-6 / 6.4
         best = []
         for name in names:
@@ -452,6 +465,8 @@ class PrefillOp:
                     continue
                 body = -(-wgs * x // cus) * (start + trip * -(-per // tiles.kv_groups))
                 us = (body ** 2.25 + read ** 2.25) ** (1 / 2.25)
+                if wgs <= cus < wgs * x:
+                    us += 0.12 * read
                 if x > 1:
                     us += 1.8 + 0.047 * x + 0.42 * heads * rows * x * 512e-6
                 best.append((us, x, name))

@@ -256,6 +256,13 @@ def test_split_launches_take_the_cheapest_tiles():
     assert op._launch_tiles(1, 8, 8, 4096, None) == three[0] and op._launch_tiles(1, 8, 64, 4096, None) == three[1]
     assert op._launch_tiles(1, 32, 128, 8192, None) == three[2] and op._launch_tiles(5, 32, 216, 3498, None) == three[3]
     assert op._launch_tiles(8, 8, 115, 521, None) == three[1]                    # 128 workgroups, not three splits of 64
+    # short caches, and more heads than CUs: the engine's own tiles, unsplit; a long cache that one split reads best
+    for B, Sq, Skv, tiles in ((3, 30, 704, TILES[0]), (3, 37, 651, TILES[2]), (9, 61, 521, TILES[2]), (16, 40, 2000, TILES[2]),
+                              (5, 61, 15254, three[1]), (5, 45, 500, three[1]), (3, 30, 1100, three[0]), (9, 61, 8000, three[1])):
+        got = op._launch_tiles(B, 32, Sq, Skv, op.tiles_for(B, 32, Sq, Skv))
+        assert got == tiles, (B, Sq, Skv, got)
+        if (B, Skv) != (9, 8000) and Skv != 1100:
+            assert op.plan_splits(B, 32, Sq, Skv, got)[0] == 1, (B, Sq, Skv)
     narrow = _engine(8, None, H=8, Hkv=8, Skv=4096, D=64)._op
     assert narrow._launch_tiles(1, 8, 8, 4096, TILES[0]) == TILES[0]
 
