@@ -676,7 +676,7 @@ class PrefillOp:
                             f"#define AE_BAND_HI {'0x7fffffff' if band[1] is None else f'({band[1]})'}\n")
             if own_softmax:
                 cfg_src += "#define AE_OWN_SOFTMAX 1\n"
-                if self.split_kv and self._split_form_of(tiles):
+                if self.split_kv and tiles.kv_groups > 1 and self._split_form_of(tiles):
                     cfg_src += "#define AE_FIRST_REST 1\n"
             if n_split > 1:
                 cfg_src += "#define AE_NSPLIT 2\n"       # (a split launch; its count is the launch's)

@@ -154,12 +154,13 @@ static_assert(AE_NSPLIT > 1 && AE_KW > 1, "merged by the last workgroup: builds 
 #define AE_OWN_SOFTMAX 0
 #endif
 #define AE_SM_TAU 5.545177444479562f     // 8 log2 units: weights up to 256
-// AE_FIRST_REST 1 (split launches whose tiles PrefillOp._cheapest_form chooses): what the rounding of its first tile's weights
-// leaves over is multiplied as well.  The largest weight of every reference is 1, which has no rounding error, and the
-// plans with fewer splits and kv groups have fewer references: by that alone the error against fp64 was 1.019 of what four
-// groups and a split for every CU gave (40 shapes of 1 to 256 rows, 512 to 16384 keys, N(0, 1) scores; 1.08 at most), the more the
-// shorter the cache.  So it is 0.988 (1.02), and 0.997 on 50 shapes of more than 32 rows (1.012 without).  0.2 to 0.3 us a call
-// (1.6 % of 60 calls of 9 to 330 us; every tile's: 7 %, error 0.74; the references that there were, by the plan: 3.5 % and more).
+// AE_FIRST_REST 1 (split launches with kv groups whose tiles PrefillOp._cheapest_form chooses): what the rounding of its first
+// tile's weights leaves over is multiplied as well.  The largest weight of every reference is 1, which has no rounding error,
+// and the plans with fewer splits and kv groups have fewer references: by that alone the error against fp64 was 1.019 of what
+// four groups and a split for every CU gave (40 shapes of 1 to 256 rows, 512 to 16384 keys, N(0, 1) scores; 1.08 at most), the
+// more the shorter the cache.  So it is 0.990 (1.02); on 50 shapes of more than 32 rows 1.012 without, 1.000 so (1.09 at most,
+// where ten splits have become one).  0.2 to 0.3 us a call; every tile's: 7 % of 60 calls of 9 to 330 us, error 0.74; the
+// references that there were, by the plan: 3.5 % of calls of at most 32 rows.
 #ifndef AE_FIRST_REST
 #define AE_FIRST_REST 0
 #endif
