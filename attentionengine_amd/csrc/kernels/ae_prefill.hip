@@ -232,8 +232,10 @@ AE_DEV int ae_k_swz(int c, int row) {
 // registers, 294 -> 313 us); without row maxima and with fragment addresses by constants 168 suffice: B1 H128 S2500 299.6 ->
 // 290.0, B1 H16 S8088 345 -> 329, B2 H32 S1968 105.9 -> 101.5, B1 H32 S570 16.5 -> 15.8, B3 H16 S789 26.7 -> 27.1 (rings of
 // two and two, three and three, six and three fragments: 289.8, 291.0, 305.7 for the first; none 280 to 288 there, 44.7
-// against 42.8 for B2 H32 S1098).
-#if (AE_D <= 128 || AE_D == 192) && AE_DV <= 128 && AE_RB == 1
+// against 42.8 for B2 H32 S1098).  At D 160 fragment addresses by constants without the rings cost up to 9 % (B4 H16 S1000 causal
+// 36.4 -> 38.1, B1 H32 S333 14.1 -> 15.0), with them 192 calls (DV 64 and 128, softmax, sigmoid and relu, every kind of mask) take
+// 0.92 of the time before either, none more than 1.01: 33.1 and 12.7 for those two.
+#if AE_D <= 192 && AE_DV <= 128 && AE_RB == 1
 #define AE_K_AHEAD 4
 #define AE_V_AHEAD 3
 #define AE_RING_FENCE() __builtin_amdgcn_sched_barrier(0)

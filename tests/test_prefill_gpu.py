@@ -736,6 +736,27 @@ def test_head_dims_whose_rows_are_not_a_power_of_two(cuda_device, B, H, Hkv, Sq,
     assert (mod.final_rowscales["lse"].cpu() - lse).abs().max().item() <= LSE_TOL
 
 
+@pytest.mark.parametrize("D,DV,S,dtype", [(160, 64, 33, torch.bfloat16), (160, 64, 257, torch.float16), (160, 128, 191, torch.bfloat16)])
+@pytest.mark.parametrize("mask_mod", [None, C.causal_mask, C.make_sliding_window_mask(70), C.head_dependent_mask])
+def test_fragment_rings_at_160_columns(cuda_device, D, DV, S, dtype, mask_mod):
+    """Ten k-steps a K fragment ring of five, every kind of mask, a last tile of one key and one that is nearly full."""
+    B, H = 1, 3
+    q, k, v = C.make_inputs(B, S, S, H, H, D, DV, dtype, seed=S)
+    meta = (meta_tensor(B, H, S, D, dtype=dtype), meta_tensor(B, H, S, D, dtype=dtype), meta_tensor(B, H, S, DV, dtype=dtype))
+    eng = AttentionEngine(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), mask_mod, C.OnlineSoftmax())
+    assert eng.attention.tiles.template == "ae_prefill.hip" and eng.attention.tiles.waves_per_eu == 2
+    out = eng(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+    mk = None
+    if mask_mod is not None:
+        mk = mask_mod(torch.arange(B)[:, None, None, None], torch.arange(H)[None, :, None, None],
+                      torch.arange(S)[:, None], torch.arange(S)[None, :]).expand(B, H, S, S)
+    ref, lse = R.softmax_attention(q, k, v, mask=mk)
+    # weights rounded to the type (they sum to 1) times the largest value, and the result's own rounding
+    eps = 2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12
+    assert (out - ref).abs().max().item() <= 2 * eps * v.float().abs().max().item() + 2 * eps * ref.abs().max().item()
+    assert (eng.final_rowscales["lse"].cpu() - lse).abs().max().item() <= LSE_TOL
+
+
 @pytest.mark.parametrize("how", ["keyword", "environment"])
 def test_pipelined_kernel_exact_scale_switch(cuda_device, monkeypatch, how):
     """``AttentionEngine(..., exact_scale=True)`` (or AE_PREFILL_PRESCALE=0 in the environment): the pipelined
