@@ -808,10 +808,12 @@ def window_group_tiles(batch_heads: int, seqlen_q: int):
 
 def kv_group_tiles_split(seqlen_q: int, batch_heads: int = 0):
     """The same for launches that also split the kv axis over workgroups (a few query tokens against a long cache): the
-    query rows decide; at head dim 128 only where PrefillOp._launch_tiles does not choose.  fp16 D128, two tile stages: B8 H32 Sq4 Skv4096 110 -> 95 us, B1 H32 Sq16 Skv16000 55 -> 46 (32 x 4 x 32); B2 H16 Sq40
-    Skv3000 19.1 -> 17.7 (64 x 2 x 32); from 65 rows on the 128-row tiles already read the cache at 5.8 TB/s.  Rows that fill a
-    256-row tile better than two of 128 take one workgroup of eight waves, which reads the cache once, where the heads leave
-    room for several splits: B4 H8 Sq213 Skv11337 78 -> 71 us, B1 H32 Sq237 Skv15274 98 -> 91; B8 H16 Sq220 Skv1909 51 -> 53."""
+    query rows decide.  At head dim 128 PrefillOp._launch_tiles takes other tiles except where one launch of these is as good
+    (PrefillOp._own_tiles_pay).  fp16 D128, two tile stages, which is what they were made from: B8 H32 Sq4 Skv4096 110 -> 95 us, B1 H32
+    Sq16 Skv16000 55 -> 46 (32 x 4 x 32); B2 H16 Sq40 Skv3000 19.1 -> 17.7 (64 x 2 x 32); from 65 rows on the 128-row tiles already
+    read the cache at 5.8 TB/s.  Rows that fill a 256-row tile better than two of 128 take one workgroup of eight waves, which reads
+    the cache once, where the heads leave room for several splits: B4 H8 Sq213 Skv11337 78 -> 71 us, B1 H32 Sq237 Skv15274 98 -> 91;
+    B8 H16 Sq220 Skv1909 51 -> 53."""
     if seqlen_q <= 32:
         return PrefillTiles(n_waves=1, kv_groups=4, block_n=32)
     if seqlen_q <= 64:

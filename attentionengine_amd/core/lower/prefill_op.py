@@ -487,9 +487,9 @@ class PrefillOp:
         rounds.  A call takes its rounds of starts and trips (half rounds beyond the second, where workgroups no longer
         end together), at least what memory needs for the cache (8.4 TB/s while the memory-side cache holds it, else 6.2),
         and the partial results: written and merged.  Fitted to 1926 timings (150 shapes, batch 1 to 8, 8 to 32 heads, 1
-        to 256 rows, 512 to 16384 keys, D128): 1 % above the best count on average.  Measured, one split for every CU ->
-        this: B7 H16 Sq31 Skv522 17.6 -> 9.2 us, B6 H16 Sq25 Skv1118 22.0 -> 15.3, B6 H8 Sq78 Skv2854 26.1 -> 21.6,
-        B3 H32 Sq2 Skv9161 109 -> 88.  ``width``: bytes of a key and a value row in units of 512.
+        to 256 rows, 512 to 16384 keys, D128, two tile stages): 1 % above the best count on average.  Measured, one split for every CU ->
+        this: B7 H16 Sq31 Skv522 17.6 -> 9.2 us.  (At head dim 128 only for tiles that ``_launch_tiles`` leaves as they are, as there, and
+        at 64 / 128 columns; the others have ``_cheapest_form``.)  ``width``: bytes of a key and a value row in units of 512.
 
         At head dim 64 two to four workgroups fit a CU, and a launch of two on some CUs is no second round: with the costs of
         D128 17 of 71 choices were slower than one split for every CU (B7 H32 Sq47 Skv5777 70.5 -> 93.9 us).  Its own costs
@@ -633,7 +633,7 @@ class PrefillOp:
         build.  48 shapes (batch 1 to 8, 8 to 32 heads, 1 to 25 rows, 512 to 16384 keys, head dims 64 and 128), time of the call in
         units of that with two launches: 0.94 on average, 0.81 to 1.003 (D64 B3 H8 Sq8 Skv764, 8 splits, 9.9 us -> 8.0; D128
         B4 H32 Sq5 Skv1496, 2 splits, 23.2 -> 21.8; B4 H16 Sq12 Skv14418, 4 splits, 89.4 -> 89.6).  Beyond: 8192 to 16384
-        values 0.92 to 1.20, 9 to 12 splits 0.93 to 1.10 (the more, the faster the host), 13 to 16 0.95 to 1.18."""
+        values 0.92 to 1.20, 9 to 12 splits 0.93 to 1.10, 13 to 16 0.95 to 1.18."""
         return (1 < n_split <= self.MERGED_SPLITS and self._can_merge_in_last(tiles)
                 and min(Sq, tiles.block_m) * n_split * self.DV <= self.MERGED_VALUES
                 and tiles.block_m * Hq * n_split * self.DV < 2**29)

@@ -11,7 +11,7 @@
 // 64 slots of q rows a q tile (a wave uses 32 of the slots; where slot n lies among the rows is undone when the rows leave).
 // Three stages of 24 KiB, filled by direct loads two steps ahead.
 //
-// B4 H32 S2048 D128 bf16 causal (537 MB of ds): 145 us where the launch that forms ds takes 219.  Loads of ds alone 135 us at
+// B4 H32 S2048 D128 bf16 causal (570 MB of ds): 145 us where the launch that forms ds takes 219.  Loads of ds alone 135 us at
 // first - while 256 MB of them still sat dirty in the memory-side cache and had to leave it -, 164 with K and the products; two
 // workgroups a CU instead of one 160, from the last keys to the first 152, past the caches 145.  Launched for one batch
 // entry at a time, so that all of ds stays in that cache, the longest workgroup of each launch costs more than it saves (the

@@ -77,7 +77,9 @@
 // apart, by when the 64 workgroups of an XCD have pushed it out of the 4 MB L2 (20 % hits, 410 MB read for 201 MB of q, k and v).
 // Started this way, workgroups in step with each other read the same tile in the same trip.  Inputs not in the caches, B2 H32
 // S4096 D128 fp16: window 256 85.9 -> 76.8 us; calls one after the other, window 1024 162.4 -> 155.8, B4 S4000 bf16 window 64
-// 119.8 -> 116.4, B3 S5188 bf16 window 388 179.2 -> 169.3.  Not at narrower heads: the keys and values of 64 neighbouring q
+// 119.8 -> 116.4, B3 S5188 bf16 window 388 179.2 -> 169.3; B1 H128 S2500 192 / 128 columns window 512 162.2 -> 142.5, sigmoid weights,
+// window 256, 82.0 -> 73.4 and at 192 / 128 99.8 -> 86.2, B2 H32 S3000 160 / 128 64.9 -> 61.3 (14 launches of wide heads and of graphs
+// without a softmax: 0.86 to 0.98 of the time).  Not at narrower heads: the keys and values of 64 neighbouring q
 // tiles are 2 MB there and stay in the L2 anyway (B2 H16 S2886 D64 window 843 32.8 -> 33.8).
 #define AE_ROTATE (AE_MASK_MODE == 3 && AE_BAND_HI != 0x7fffffff && AE_NSPLIT == 1 && AE_KW == 1 && AE_D + AE_DV >= 256)
 
@@ -230,7 +232,7 @@ AE_DEV int ae_k_swz(int c, int row) {
 // with every register taken.  bf16, without a mask, B16 H16 S1000: D 64 90.0 -> 88.2 us, D 128 160.3 -> 155.6 us (with the
 // shorter epilogue); causal B8 H32 S1000 D128 112.3 -> 110.0 us.  At D 192, DV 128 the rings have cost a wave per SIMD (180
 // registers, 294 -> 313 us); without row maxima and with fragment addresses by constants 168 suffice: B1 H128 S2500 299.6 ->
-// 290.0, B1 H16 S8088 345 -> 329, B2 H32 S1968 105.9 -> 101.5, B1 H32 S570 16.5 -> 15.8, B3 H16 S789 26.7 -> 27.1 (rings of
+// 290.0, B1 H16 S8088 345 -> 329, B2 H32 S1968 105.9 -> 101.5, B1 H32 S570 16.5 -> 15.8, B3 H16 S789 26.7 -> 27.1 (24.8 with AE_OWN_SOFTMAX as well; rings of
 // two and two, three and three, six and three fragments: 289.8, 291.0, 305.7 for the first; none 280 to 288 there, 44.7
 // against 42.8 for B2 H32 S1098).  At D 160 fragment addresses by constants without the rings cost up to 9 % (B4 H16 S1000 causal
 // 36.4 -> 38.1, B1 H32 S333 14.1 -> 15.0), with them 192 calls (DV 64 and 128, softmax, sigmoid and relu, every kind of mask) take
