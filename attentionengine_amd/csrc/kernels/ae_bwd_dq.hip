@@ -69,8 +69,10 @@ void ae_bwd_dq_kernel(const ae_attn_bwd_params p) {
   const int n_bh = p.batch * p.heads_q;
   const int n_bg = (n_bh + 7) >> 3;
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int bh = (slot % n_bg) * 8 + xcd;
-  const int rt = AE_MASK_MODE == 1 ? n_rt - 1 - slot / n_bg : slot / n_bg;
+  int turn;
+  const int tile = ae_divide(slot, n_bg, turn);
+  const int bh = ae_head_of_xcd(turn, xcd, n_bh, p.heads_q != p.heads_kv && n_bg >= AE_RUNS_FROM);
+  const int rt = AE_MASK_MODE == 1 ? n_rt - 1 - tile : tile;
   if (bh >= n_bh) return;
   const int h = bh % p.heads_q, b = bh / p.heads_q;
   const int hk = h / (p.heads_q / p.heads_kv);

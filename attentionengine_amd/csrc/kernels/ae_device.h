@@ -39,21 +39,67 @@ typedef unsigned int ae_u32x2 __attribute__((ext_vector_type(2)));
 // Quotient and remainder of wave-uniform numbers, a >= 0 and d > 0.  The compiler's division is a chain of some thirty
 // dependent instructions, and which tile a workgroup has takes four of them in front of its first request: a shift where d
 // is a power of two, else a reciprocal whose quotient is off by at most one below 2^22.
+AE_DEV int ae_divide_small(int a, int d, int& rem) {       // a below 2^22
+  int q = __builtin_amdgcn_readfirstlane((int)((float)a * __builtin_amdgcn_rcpf((float)d)));
+  rem = a - q * d;
+  if (rem < 0) q--, rem += d;
+  if (rem >= d) q++, rem -= d;
+  return q;
+}
 AE_DEV int ae_divide(int a, int d, int& rem) {
   int q;
   if ((d & (d - 1)) == 0) {
     q = a >> __builtin_ctz(d);
     rem = a & (d - 1);
   } else if (__builtin_expect(a < 1 << 22, 1)) {
-    q = __builtin_amdgcn_readfirstlane((int)((float)a * __builtin_amdgcn_rcpf((float)d)));
-    rem = a - q * d;
-    if (rem < 0) q--, rem += d;
-    if (rem >= d) q++, rem -= d;
+    q = ae_divide_small(a, d, rem);
   } else {
     q = a / d;
     rem = a - q * d;
   }
   return q;
+}
+
+// Which head and which tile a workgroup has.  Consecutive ids are dealt round-robin to the 8 XCDs, each with an L2 of 4 MB of
+// its own, so the workgroups of id 8 * slot + xcd share one.
+// ae_head_of_xcd: the (batch, query head) whose turn among the heads of its XCD is i; n_bh or more: none.  in_runs (launches whose
+// query heads share kv heads): an XCD has neighbouring heads, so that K and V of fewer kv heads go through its L2; else turn i
+// of the eight XCDs are eight neighbours, whose rows lie side by side in memory.  us, dealt singly -> in runs: causal bf16 B4 Hq64
+// Hkv8 D128 S1000 104.3 -> 88.8, S2000 348 -> 291, fp16 S333 26.3 -> 22.9, B4 Hq32 Hkv8 S3000 D64 181.8 -> 172.5, B2 Hq32 Hkv8 S4096
+// D128 275.5 -> 270.7, without a mask B1 Hq64 Hkv8 S700 25.0 -> 24.6, forward and backward of B8 Hq32 Hkv8 S1500 D64 451 -> 432.
+// (Heads with K and V of their own in runs: 0.99 to 1.015.)
+// With fewer than eight heads an XCD (AE_RUNS_FROM) the whole K and V fit every L2, and one head's lines asked for by all workgroups of
+// an XCD are late: B1 Hq32 Hkv8 S333 with inputs in the caches 8.77 -> 8.95 (not in them 9.19 -> 8.97); B1 Hq64 Hkv8 S333 10.87 ->
+// 10.71 (11.69 -> 11.25).
+#define AE_RUNS_FROM 8
+AE_DEV int ae_head_of_xcd(int i, int xcd, int n_bh, bool in_runs) {
+  if (!in_runs) return i * 8 + xcd;
+  const int lo = n_bh >> 3, more = n_bh & 7;
+  return i < lo + (xcd < more ? 1 : 0) ? xcd * lo + (xcd < more ? xcd : more) + i : n_bh;
+}
+// ae_heavy_first: q tiles that differ in work, the tile with the most work first across the heads of the XCD (longest job first
+// keeps the tail short).  Returns how many tiles of the head lie in front of it in that order; i: the head's turn.  in_eights: the
+// first three quarters of the tiles go eight heads at a time - the tiles in flight are then of few heads, which keeps their K
+// and V in the L2, and what is left for the end is short.  Pays where an XCD has more heads than that, each with K and V of its own, and
+// more than two rounds of workgroups.  us, all heads -> eight at a time: causal 192 / 128 columns B1 H128 S2500 269 -> 265 (bf16), B2
+// H128 S1400 208 -> 197 (fp16), B4 H128 S700 158 -> 133 (bf16); 128 columns, 128-row tiles, B8 H32 S875 87.5 -> 80.0, B4 H32 S2048 162.9 ->
+// 159.8; 64 columns B8 H32 S1700 143 -> 135; 256-row tiles of the pipelined kernel, B4 H32 S4096 570 -> 557, S2500 249 -> 241.  Where
+// there is less it costs: B1 H128 S400 (64 tiles an XCD) 19.7 -> 21.1, D64 B4 H32 S1200 (160) 39.6 -> 40.1.  Two or four heads at
+// a time, or all tiles that way: up to 15 % worse at some lengths.  The launches of the backward: no difference beyond 1 %.
+AE_DEV int ae_heavy_first(int slot, int n_bg, int n_t, bool in_eights, int& i) {
+  if (in_eights) {
+    const int n_long = n_t - n_t / 4;
+    if (slot < n_long * n_bg) {
+      int r;
+      const int i0 = ae_divide_small(slot, 8 * n_long, r) * 8;
+      int t = r >> 3;
+      i = r & 7;
+      if (n_bg - i0 < 8) t = ae_divide_small(r, n_bg - i0, i);
+      i += i0;
+      return t;
+    }
+  }
+  return ae_divide(slot, n_bg, i);
 }
 
 // D[m][n] += sum_k A[m][k] B[k][n], 32x32 output, 16-deep. Lane l supplies A[l%32][8*(l/32)+j]

@@ -166,6 +166,7 @@ static_assert(AE_NSPLIT > 1 && AE_KW > 1, "merged by the last workgroup: builds 
 #ifndef AE_FIRST_REST
 #define AE_FIRST_REST 0
 #endif
+#define AE_TWO_ROUNDS (AE_D <= 64 ? 256 : 128)      // workgroups of two rounds of an XCD's 32 CUs
 #define AE_WROWS (AE_RB * 32)     // query rows per wave
 #define AE_BM (AE_NWAVES * AE_WROWS)
 #define AE_GT (AE_NWAVES * 64)     // threads of a kv group
@@ -327,13 +328,17 @@ void ae_prefill_kernel(const ae_attn_params p) {
   // (longest-job-first keeps the tail short); the heads of one XCD still meet in its L2.  A tile table whose
   // late q tiles are the long ones (AE_HEAVY_LAST, found on the host: causal variants, long sliding windows)
   // takes the same order: B2 H32 S4096, "kv <= q + 1": 0.40 -> 0.35 ms.
+  int turn;
   const int n_bg = (n_bh + 7) >> 3;
-  int bh;
-  const int qt = n_qt - 1 - ae_divide(slot, n_bg, bh);
-  bh = bh * 8 + xcd;
+  const bool own_kv = p.heads_q == p.heads_kv;
+  const int n_tiles = n_bg * n_qt;
+  const int qt = n_qt - 1 - ae_heavy_first(slot, n_bg, n_qt, AE_NSPLIT == 1 && AE_KW == 1 && own_kv && n_bg > 8 && n_tiles > AE_TWO_ROUNDS &&
+                                           n_tiles < 1 << 22, turn);
+  const int bh = ae_head_of_xcd(turn, xcd, n_bh, AE_NSPLIT == 1 && !own_kv && n_bg >= AE_RUNS_FROM);
 #else
   int qt;
-  const int bh = ae_divide(slot, n_qt, qt) * 8 + xcd;
+  const int turn = ae_divide(slot, n_qt, qt);
+  const int bh = ae_head_of_xcd(turn, xcd, n_bh, AE_NSPLIT == 1 && p.heads_q != p.heads_kv && n_bh >= 8 * AE_RUNS_FROM);
 #endif
   if (bh >= n_bh) return;
   int h, rest;

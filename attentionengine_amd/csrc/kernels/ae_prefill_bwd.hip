@@ -257,13 +257,15 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #else
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
 #endif
-  const int bh = (slot % n_bg) * 8 + xcd;
+  int turn;
+  const int tile = ae_divide(slot, n_bg, turn);
+  const int bh = ae_head_of_xcd(turn, xcd, n_bh, AE_BWD_ROLE == 0 && p.heads_q != p.heads_kv && n_bg >= AE_RUNS_FROM);
 #if AE_BWD_ROLE == 0 && (AE_MASK_MODE == 1 || (AE_MASK_MODE == 2 && AE_HEAVY_LAST))
   // (the q tiles with the most visible keys first: the last ones under a causal mask, and under a tile table
   // that the host found to be heavier towards the end - AE_HEAVY_LAST)
-  const int rt = n_rt - 1 - slot / n_bg;
+  const int rt = n_rt - 1 - tile;
 #else
-  const int rt = slot / n_bg;
+  const int rt = tile;
 #endif
   if (bh >= n_bh) return;
   const int h = bh % heads;            // role 0: q head; role 1: kv head

@@ -185,8 +185,10 @@ void ae_prefill_kernel(const ae_attn_params p) {
   // takes the same order: B2 H32 S4096, "kv <= q + 1": 0.40 -> 0.35 ms.
   const int n_bg = (n_bh + 7) >> 3;
 #if AE_CAUSAL_ORDER == 0
-  const int qt = n_qt - 1 - slot / n_bg;
-  const int bh = (slot % n_bg) * 8 + xcd;
+  int turn;
+  const bool own_kv = p.heads_q == p.heads_kv;
+  const int qt = n_qt - 1 - ae_heavy_first(slot, n_bg, n_qt, own_kv && n_bg > 8 && n_bg * n_qt > 64 && n_bg * n_qt < 1 << 22, turn);
+  const int bh = ae_head_of_xcd(turn, xcd, n_bh, !own_kv && n_bg >= AE_RUNS_FROM);
 #else
   // (measurement switch) head by head: the q tiles of one (batch, head) are adjacent in time, heaviest first, so
   // that its K / V stay in the XCD's L2 while they are used - at the price of a longer tail

@@ -1338,3 +1338,41 @@ def test_a_row_does_not_depend_on_the_rows_of_its_wave(cuda_device, D, DV, dtype
     rest = torch.arange(S) % 32 != 31
     assert not torch.equal(loud[:, ~rest], out[:, ~rest])
     assert torch.equal(loud[:, rest], out[:, rest]) and torch.equal(loud_lse[:, :, rest], lse[:, :, rest])
+
+
+@pytest.mark.parametrize("kernel,B,H,Hkv,S,D,DV,dtype,mask", [
+    # more than eight heads an XCD and more than two rounds of workgroups: eight heads at a time, the last group smaller
+    ("generic", 9, 9, 9, 1700, 128, 128, torch.float16, "causal"),
+    ("generic", 3, 27, 27, 3001, 64, 64, torch.bfloat16, "causal"),
+    ("generic", 9, 8, 8, 2100, 192, 128, torch.bfloat16, "causal"),
+    ("pipelined", 9, 8, 8, 2100, 128, 128, torch.float16, "causal"),
+    # one tile too few for that, and just enough
+    ("generic", 16, 8, 8, 1024, 128, 128, torch.bfloat16, "causal"),
+    ("generic", 16, 8, 8, 1025, 128, 128, torch.bfloat16, "causal"),
+    # heads that share K and V, their number no multiple of the eight XCDs, fewer than XCDs among them
+    ("generic", 5, 15, 5, 300, 128, 128, torch.float16, "causal"),
+    ("pipelined", 5, 6, 3, 600, 128, 128, torch.bfloat16, "causal"),
+    ("generic", 3, 10, 2, 300, 64, 64, torch.bfloat16, "none"),
+    ("generic", 2, 6, 2, 700, 128, 128, torch.float16, "window"),
+    ("generic", 2, 2, 1, 300, 64, 64, torch.float16, "causal"),
+])
+def test_every_head_has_its_turn(cuda_device, monkeypatch, kernel, B, H, Hkv, S, D, DV, dtype, mask):
+    """Which workgroup has which tile of which head depends on how many heads there are; a head's result does not: bit for
+    bit what its batch entry gives in a call of its own, whose order is another one."""
+    print(f"case turns {kernel} B{B} H{H}/{Hkv} S{S} D{D} {mask}", flush=True)
+    monkeypatch.setenv("AE_PREFILL_KERNEL", kernel)
+    masks = {"none": None, "causal": C.causal_mask, "window": C.make_sliding_window_mask(100)}
+    meta = (meta_tensor(B, H, S, D, dtype=dtype), meta_tensor(B, Hkv, S, D, dtype=dtype), meta_tensor(B, Hkv, S, DV, dtype=dtype))
+    eng = AttentionEngine(meta, CustomIO({}), C.make_scale_score_mod(1 / math.sqrt(D)), masks[mask], C.OnlineSoftmax())
+    q, k, v = (t.cuda() for t in C.make_inputs(B, S, S, H, Hkv, D, DV, dtype, seed=H))
+    out, lse = eng(q, k, v), eng.final_rowscales["lse"]
+    for b in range(B):
+        one = eng(q[b:b + 1], k[b:b + 1], v[b:b + 1])
+        assert torch.equal(out[b], one[0]) and torch.equal(lse[b], eng.final_rowscales["lse"][0]), b
+    # (the rows of the last entry's last head against fp32: no tile is missing from both)
+    s = q[-1, :, -1].float() @ k[-1, :, -1].float().T / math.sqrt(D)
+    if mask != "none":
+        pos = torch.arange(S, device="cuda")
+        gap = pos[:, None] - pos[None]
+        s = s.masked_fill((gap < 0) | (gap >= (S if mask == "causal" else 100)), -math.inf)
+    assert (out[-1, :, -1].float() - s.softmax(-1) @ v[-1, :, -1].float()).abs().max().item() <= OUT_TOL
