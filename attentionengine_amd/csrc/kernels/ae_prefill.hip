@@ -166,6 +166,14 @@ static_assert(AE_NSPLIT > 1 && AE_KW > 1, "merged by the last workgroup: builds 
 #ifndef AE_FIRST_REST
 #define AE_FIRST_REST 0
 #endif
+// 1: a wave's priority on its SIMD goes up as it goes through a trip - scores 0, softmax 1, second product 2 -, so that of the waves
+// that share the SIMD the one that has got furthest finishes and they fall out of step: one's products run under another's
+// softmax.  us: causal 192 / 128 columns B1 H128 S2500 278 -> 270, B2 H128 S1400 222 -> 208, B1 H32 S5000 249 -> 236, B4 H128 S700 163 ->
+// 158; sigmoid at 64 columns B2 H32 S3000 175 -> 173, B4 H16 S1000 25.6 -> 24.7.  Not at 128 columns (causal B4 Hq32 Hkv8 S1400 79.2 ->
+// 81.6) or for the softmax at 64 (155.5 -> 157.1), and not where the groups of a workgroup wait for each other (192 / 128 B1 H16
+// S8000 315 -> 320).
+#define AE_PRIO (AE_KW == 1 && AE_NSPLIT == 1 && AE_WAVES_PER_EU >= 2 && (AE_D >= 192 || (AE_ELEMENTWISE && AE_D <= 64)))
+#define AE_SETPRIO(n) do { if (AE_PRIO) __builtin_amdgcn_s_setprio(n); } while (0)
 #define AE_TWO_ROUNDS (AE_D <= 64 ? 256 : 128)      // workgroups of two rounds of an XCD's 32 CUs
 #define AE_WROWS (AE_RB * 32)     // query rows per wave
 #define AE_BM (AE_NWAVES * AE_WROWS)
@@ -654,6 +662,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
     };
     constexpr int NKF = (AE_D / 16) * AE_NB;
     ae_elem8 kring[AE_K_AHEAD + 1];
+    AE_SETPRIO(0);
 #pragma unroll
     for (int f = 0; f < AE_K_AHEAD && f < NKF; f++) kring[f] = k_frag(f);
     AE_RING_FENCE();
@@ -666,6 +675,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
       AE_RING_FENCE();
     }
 
+    AE_SETPRIO(1);
     unsigned v_at = (unsigned)(unsigned long)vs_ + v_lane;
     asm("" : "+v"(v_at));
     auto v_frag = [&](int f) AE_LAMBDA -> ae_elem8 {
@@ -850,6 +860,7 @@ void ae_prefill_kernel(const ae_attn_params p) {
     // ---- O^T += V^T P^T: every V fragment feeds one MFMA per row block ------------------------
     constexpr int NVF = (AE_BN / 16) * AE_NDB;
     ae_elem8 vring[AE_V_AHEAD + 1];
+    AE_SETPRIO(2);
 #pragma unroll
     for (int f = 0; f < AE_V_AHEAD && f < NVF; f++) vring[f] = v_frag(f);
     AE_RING_FENCE();
