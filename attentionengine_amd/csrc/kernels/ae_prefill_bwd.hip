@@ -34,7 +34,7 @@
 // straddles blocks of both kinds - looks every element up in the user's mask (ae_attn_bwd_params.block_mask).
 //
 // Waves per workgroup (AE_BWD_NWAVES, 32 resident rows each): dk/dv runs four, one per SIMD with the
-// whole register file (two accumulators), or, softmax attention without a tile table, eight in pairs at head dims 128
+// whole register file (two accumulators), or, softmax attention without a tile table, eight of two kinds at head dims 128
 // (AE_BWD_PAIRS) and two workgroups a CU at head dims 64. dq has one accumulator and fits 256 registers, so it runs
 // eight, two per SIMD (AE_BWD_WAVES_PER_EU 2, AE_AHEAD 3): a wave spends about half of its time waiting
 // (LDS fragments, MFMA results, the p/ds arithmetic between two sets of MFMAs) and the second wave
@@ -70,8 +70,8 @@
 #endif
 #define AE_NWAVES AE_BWD_NWAVES
 #define AE_NT (AE_NWAVES * 64)
-// 1 (dk/dv launch of softmax attention at head dim 128, eight waves): waves in pairs that share 32 kv rows, see
-// "two waves a pair" below.
+// 1 (dk/dv launch of softmax attention at head dim 128, eight waves): four waves form p and ds, four add the products, see
+// "two kinds of waves" below.
 #ifndef AE_BWD_PAIRS
 #define AE_BWD_PAIRS 0
 #endif
@@ -289,7 +289,9 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   ae_custom cust;
   ae_bwd_load_custom(cust, p);
 #endif
+#if !AE_BWD_PAIRS
   ae_elem8 rf1[AE_NKS1], rf2[AE_NKS2];
+#endif
 #if !AE_RES_VIA_LDS
 #pragma unroll
   for (int ks = 0; ks < AE_NKS1; ks++) rf1[ks] = *(const ae_elem8*)(r1p + ks * 16 + hf * 8);
@@ -610,8 +612,10 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
     ae_bwd_rows_to_lds<AE_CPR1>(g1 - 4096, rs, lane, rw0 - rw0c, n_res - 1 - rw0c, rs1);
     ae_bwd_rows_to_lds<AE_CPR2>(g2 - 4096, rs + AE_R1B, lane, rw0 - rw0c, n_res - 1 - rw0c, rs2);
     __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
+#if !AE_BWD_PAIRS
     ae_bwd_frags_from_lds<AE_NKS1, AE_CPR1>(rf1, rs, l32, hf);
     ae_bwd_frags_from_lds<AE_NKS2, AE_CPR2>(rf2, rs + AE_R1B, l32, hf);
+#endif
 #else
     ae_lds_byte* rs = lds + AE_STAGE_BYTES + rw * (AE_R1B > AE_R2B ? AE_R1B : AE_R2B);
     ae_bwd_rows_to_lds<AE_CPR1>(g1 - 4096, rs, lane, rw0 - rw0c, n_res - 1 - rw0c, rs1);
@@ -650,7 +654,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
     asm volatile("" :: "v"(lse2_r), "v"(delta_r));
 #endif
   }
-  __syncthreads();       // every wave has its fragments: stages 1 and 2 go back to the ring
+  __syncthreads();       // every wave has its fragments (pairs: has sent its rows): stages 1 and 2 go back to the ring
   if (!AE_BWD_PAIRS && x0 < n_items) request_item(x1, AE_STAGE_BYTES);
 #else
   if (x0 < n_items) {
@@ -682,6 +686,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
     return at;
   };
+#if !AE_BWD_PAIRS
   // only tiles that touch the diagonal, the end of a sequence or an elementwise mask test visibility
   const int r0w = r0 + rw * 32;
   auto tests_visibility = [&](int s0) AE_LAMBDA {
@@ -879,51 +884,122 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+#endif      // !AE_BWD_PAIRS
 #if AE_BWD_PAIRS
-  // Two waves a pair.  dk and dv of 32 rows are 128 accumulators, the resident operands 64 registers, the scores 64: one
-  // wave a SIMD with the whole file, which issues its LDS reads, its p / ds arithmetic and its MFMAs one after the other
-  // and moves every score out of the accumulator file.  Here wave w (w < 4) holds K and V of the pair's rows and forms p
-  // and ds of tile n, and wave w + 4, on the same SIMD, holds dk and dv and adds tile n - 1's products: 32 MFMAs a tile
-  // each, 256 registers suffice, and one's arithmetic runs under the other's MFMAs.  p and ds go over through 8 KiB of
-  // LDS a pair, in the operand layout.  A tile's two barriers: A, half-way, the second wave has p and ds of n - 1 in its
-  // registers (the first may write those of n); B, at the end, tile n + 1 has landed and p and ds of n are written.
-  // Tile n + 1 goes into the stage of tile n - 2, which the second wave left at the last B.
-  // Against one wave a SIMD: causal backward of B2 H32 S4096 fp16 1047 -> 1005 us, B4 H32 S2048 bf16 594 -> 558, B2 H16
-  // S1000 88.5 -> 77.
-  ae_lds_byte* ho = lds + 3 * AE_STAGE_BYTES + rw * 8192 + lane * 16;      // fragment i (p: 0..3, ds: 4..7) at + 1024 * i
+  // Two kinds of waves.  dk and dv of 32 rows are 128 accumulators, the resident operands 64 registers, the scores 64: one
+  // wave a SIMD with the whole file would issue its LDS reads, its p / ds arithmetic and its MFMAs one after the other
+  // and move every score out of the accumulator file.  Here waves 0 .. 3 form p and ds of tile n and waves 4 .. 7, one of either
+  // kind on a SIMD, add tile n - 1's products: 32 MFMAs a tile each, 256 registers suffice, and one's arithmetic runs under the
+  // other's MFMAs.  Wave w of the first kind holds K and V of 64 of the 128 rows (w % 2) and takes 32 of the tile's 64 q rows
+  // (w / 2); wave 4 + w holds 64 rows (w % 2) of dk or of dv (w / 2).  So every fragment that is read from LDS feeds two MFMAs,
+  // and a wave of the second kind reads one of the two tensors.  p and ds go over through 32 KiB of LDS, in the operand layout.
+  // A tile's two barriers: A, the second kind has p and ds of n - 1 in registers (the first may write those of n); B, at the
+  // end, tile n + 1 has landed and p and ds of n are written.  Tile n + 1 goes into the stage of tile n - 2, which the second kind
+  // left at the last B.
+  // LDS bound this: a wave of the first kind held 32 rows and took all 64 q rows, one of the second 32 rows of dk and of dv, and each
+  // fragment fed one MFMA, 320 KB of fragments, row values and hand-over a tile at 128 bytes a clock, now 224.  dk/dv launch,
+  // us: causal fp16 B2 H32 S4096 644 -> 598, B2 Hq32 Hkv8 S2500 251 -> 233, bf16 B4 H32 S2048 356 -> 335, B2 H32 S1000 53.2 -> 51.5.
+  // Bits are the same.  What is left of B4 H32 S2048: without the stores of ds 308, with every tile in the L2 297, without the
+  // exponentials too 286, on inputs of zeros 277 (the power cap).  Priorities of either kind, and barrier A a quarter earlier
+  // or later: within 1 %.
+  static_assert(AE_D == AE_DV && AE_NKS1 == AE_NKS2 && AE_RES_ONEPASS, "pairs: one head dim");
+  ae_lds_byte* const ho = lds + 3 * AE_STAGE_BYTES + lane * 16;      // fragment i (p: 0..3, ds: 4..7) of 32 rows kb at + 8192 * kb + 1024 * i
   typedef __attribute__((address_space(3))) ae_u32x4 ae_lds_u32x4;
   unsigned st_use = 0, st_req = AE_STAGE_BYTES;
+  const int half = wave & 1, nb = (wave >> 1) & 1;
   if (wave < AE_NRW) {
+    ae_elem8 rf1[2][AE_NKS1], rf2[2][AE_NKS2];         // (its 64 rows have come by two waves)
+#pragma unroll
+    for (int rb = 0; rb < 2; rb++) {
+      const ae_lds_byte* rs = lds + AE_STAGE_BYTES + (2 * half + rb) * (AE_R1B + AE_R2B);
+      ae_bwd_frags_from_lds<AE_NKS1, AE_CPR1>(rf1[rb], rs, l32, hf);
+      ae_bwd_frags_from_lds<AE_NKS2, AE_CPR2>(rf2[rb], rs + AE_R1B, l32, hf);
+    }
+    __syncthreads();                                           // every wave has its fragments
 #if AE_BWD_KEEP_DS
     // (carried along, as the requests' addresses are)
-    char* ds_at = ae_ds_row(p, b * p.heads_q + us_h, us_t) + (int64_t)(rt * 4 + rw) * 4096 + lane * 16;
+    const int64_t ds_lane = (int64_t)(rt * 4 + 2 * half) * 4096 + nb * 2048 + lane * 16;
+    char* ds_at = ae_ds_row(p, b * p.heads_q + us_h, us_t) + ds_lane;
     const bool ds_triangle = AE_MASK_MODE == 1 && p.seqlen_q == p.seqlen_kv;
     const int ds_pairs = 2 * n_rt;
 #endif
+    const int r0w = r0 + half * 64;
     while (x0 < n_items) {
       request_item(x1, st_req);
       const tile_at at = tile_in_use(st_use);
-      const bool need_vis = tests_visibility(at.s0);
-      ae_u32x4 pf[4], dsf[4];
-      auto hand_over = [&](int nb) AE_LAMBDA {
+      const int qb = at.s0 + 32 * nb;                // the first of the wave's 32 q rows
+      bool need_vis = qb + 32 > n_str || r0w + 64 > n_res;
+#if AE_MASK_MODE == 1
+      need_vis = need_vis || qb < r0w + 63;
+#endif
+      auto row_values = [&](int slot, int rg) AE_LAMBDA -> ae_f32x4 {
+        return *(const __attribute__((address_space(3))) ae_f32x4*)(lds + at.rows + (slot * AE_BS + nb * 32 + 8 * rg) * 4);
+      };
+      // S = Q K^T and dP = dO V^T, [q row][resident row]; dP starts at -rowsum(do * o)
+      ae_f32x16 sacc[2], pacc[2];
+#pragma unroll
+      for (int r = 0; r < 16; r++) sacc[0][r] = 0.f, sacc[1][r] = 0.f, pacc[0][r] = row_values(1, r >> 2)[r & 3];
+      pacc[1] = pacc[0];
+      const unsigned v0 = at.v1 + (unsigned)(nb * 32 * AE_STR1);
+      constexpr int NF = 2 * AE_NKS1;
+      auto frag = [&](int f) AE_LAMBDA -> ae_elem8 { return row_frag(v0, AE_STR1, 0, f >> 1, f & 1 ? AE_T1_BYTES : 0); };
+      ae_elem8 ring[AE_RING];
+#pragma unroll
+      for (int f = 0; f < AE_AHEAD; f++) ring[f] = frag(f);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int f = 0; f < NF; f++) {
+        if (f + AE_AHEAD < NF) ring[(f + AE_AHEAD) % AE_RING] = frag(f + AE_AHEAD);
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) {
+          if (f & 1) pacc[rb] = ae_mfma32(ring[f % AE_RING], rf2[rb][f >> 1], pacc[rb]);
+          else sacc[rb] = ae_mfma32(ring[f % AE_RING], rf1[rb][f >> 1], sacc[rb]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      ae_f32x4 lse2[4];
+#pragma unroll
+      for (int rg = 0; rg < 4; rg++) lse2[rg] = row_values(0, rg);
+      // p and ds of the wave's q rows and 32 resident rows, packed as B operands: k-step i holds the lane's elements 8*i .. 8*i+7
+      auto weights = [&](int rb, auto masked, ae_u32x4 (&pf)[2], ae_u32x4 (&dsf)[2]) AE_LAMBDA {
+        const int row = r0w + rb * 32 + l32;
+        // masked tiles: the q rows that see the lane's row are one interval, tested with one comparison a score
+        const int lo = AE_MASK_MODE == 1 ? row : 0, hi = row < n_res ? n_str : 0;
+        const int vis_lo = lo - qb - 4 * hf;
+        const unsigned vis_span = hi > lo ? (unsigned)(hi - lo) : 0u;
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+          typedef float ae_f32x2 __attribute__((ext_vector_type(2)));
+          ae_f32x2 p2, d2;
+#pragma unroll
+          for (int u = 0; u < 2; u++) {
+            const int e = r + u;
+            float pv = ae_exp2(__builtin_fmaf(sacc[rb][e], AE_SM_SCALE * AE_LOG2E, -lse2[e >> 2][e & 3]));
+            if (decltype(masked)::value) pv = (unsigned)(8 * (e >> 2) + (e & 3) - vis_lo) < vis_span ? pv : 0.f;
+            p2[u] = pv;
+            d2[u] = pv * pacc[rb][e];                  // score_mod's derivative (the scale) is applied to the sums
+          }
+          pf[r >> 3][(r & 7) >> 1] = __builtin_bit_cast(unsigned, __builtin_convertvector(p2, ae_elem2));
+          dsf[r >> 3][(r & 7) >> 1] = __builtin_bit_cast(unsigned, __builtin_convertvector(d2, ae_elem2));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+#pragma unroll
+      for (int rb = 0; rb < 2; rb++) {
+        ae_u32x4 pf[2], dsf[2];
+        if (need_vis) weights(rb, ae_bwd_true{}, pf, dsf);
+        else weights(rb, ae_bwd_false{}, pf, dsf);
+        if (rb == 0) __syncthreads();                            // A
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-          *(ae_lds_u32x4*)(ho + (2 * nb + i) * 1024) = pf[2 * nb + i];
-          *(ae_lds_u32x4*)(ho + (4 + 2 * nb + i) * 1024) = dsf[2 * nb + i];
-        }
+          *(ae_lds_u32x4*)(ho + (2 * half + rb) * 8192 + (2 * nb + i) * 1024) = pf[i];
+          *(ae_lds_u32x4*)(ho + (2 * half + rb) * 8192 + (4 + 2 * nb + i) * 1024) = dsf[i];
 #if AE_BWD_KEEP_DS
-        // (past the caches: another launch reads it, hundreds of MB later)
-#pragma unroll
-        for (int i = 0; i < 2; i++) __builtin_nontemporal_store(dsf[2 * nb + i], (ae_u32x4*)(ds_at + (2 * nb + i) * 1024));
+          // (past the caches: another launch reads it, hundreds of MB later)
+          __builtin_nontemporal_store(dsf[i], (ae_u32x4*)(ds_at + rb * 4096 + i * 1024));
 #endif
-      };
-      if (need_vis) block(0, ae_bwd_true{}, at, pf, dsf);
-      else block(0, ae_bwd_false{}, at, pf, dsf);
-      __syncthreads();                                         // A
-      hand_over(0);
-      if (need_vis) block(1, ae_bwd_true{}, at, pf, dsf);
-      else block(1, ae_bwd_false{}, at, pf, dsf);
-      hand_over(1);
+        }
+      }
 #if AE_BWD_KEEP_DS
       __builtin_amdgcn_s_waitcnt(AE_VMCNT(4));                 // (the tile: this trip's four stores of ds are newer)
 #else
@@ -933,47 +1009,60 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #if AE_BWD_KEEP_DS
       ds_at += (ds_triangle ? 2 * (us_t / 2 + 1) : ds_pairs) * 8192;
 #endif
-#if AE_MASK_MODE != 2
       us_t++;
       if (us_t == t_hi) {
         us_t = t_lo, us_h++;
 #if AE_BWD_KEEP_DS
-        ds_at = ae_ds_row(p, b * p.heads_q + us_h, us_t) + (int64_t)(rt * 4 + rw) * 4096 + lane * 16;
+        ds_at = ae_ds_row(p, b * p.heads_q + us_h, us_t) + ds_lane;
 #endif
       }
-#endif
       st_use = st_use == 2 * AE_STAGE_BYTES ? 0 : st_use + AE_STAGE_BYTES;
       st_req = st_req == 2 * AE_STAGE_BYTES ? 0 : st_req + AE_STAGE_BYTES;
-      x0 = x1, cls0 = cls1;
+      x0 = x1;
       x1 = next_item(x1 + 1, cls1);
     }
     __syncthreads();                                           // the ring goes to the results
     return;
   }
+  __syncthreads();
+  // (acc1, acc2: the two blocks of 32 rows, of dk where nb is 0, else of dv)
   clear(acc1);
   clear(acc2);
-  // the tile's products with p and ds as they were handed over
+  // the tile's products with what was handed over: fragment f = (k-step f / 4, output block f % 4)
   auto add_handed_over = [&](unsigned stage, auto all_read) AE_LAMBDA {
-    ae_u32x4 pf[4], dsf[4];
-    auto take = [&](int i0) AE_LAMBDA {
-#pragma unroll
-      for (int i = i0; i < i0 + 2; i++) {
-        pf[i] = *(const ae_lds_u32x4*)(ho + i * 1024);
-        dsf[i] = *(const ae_lds_u32x4*)(ho + (4 + i) * 1024);
-      }
+    unsigned w = tr1 + stage + (unsigned)(nb * AE_T1_BYTES);
+    asm("" : "+v"(w));
+    ae_u32x4 b0[4], b1[4];
+    auto take = [&](int kk) AE_LAMBDA {
+      b0[kk] = *(const ae_lds_u32x4*)(ho + 2 * half * 8192 + (4 - 4 * nb + kk) * 1024);
+      b1[kk] = *(const ae_lds_u32x4*)(ho + (2 * half + 1) * 8192 + (4 - 4 * nb + kk) * 1024);
     };
+    constexpr int NF = 4 * AE_NDB1;
+    auto frag = [&](int f) AE_LAMBDA -> ae_elem8 { return tr_frag(w, AE_STR1, AE_CPR1, f / AE_NDB1, f % AE_NDB1, 0); };
+    ae_elem8 ring[AE_RING];
     take(0);
-    add_products(stage, pf, dsf, [&]() AE_LAMBDA {
-      take(2);
-      all_read();
-    });
+#pragma unroll
+    for (int f = 0; f < AE_AHEAD; f++) ring[f] = frag(f);
+    take(1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+      if (f + AE_AHEAD < NF) ring[(f + AE_AHEAD) % AE_RING] = frag(f + AE_AHEAD);
+      if (f == AE_NDB1) take(2);
+      if (f == AE_NDB1 + 1) take(3);
+      if (f == NF / 2) all_read();
+      const int kk = f / AE_NDB1, j = f % AE_NDB1;
+      acc1[j] = ae_mfma32(ring[f % AE_RING], __builtin_bit_cast(ae_elem8, b0[kk]), acc1[j]);
+      acc2[j] = ae_mfma32(ring[f % AE_RING], __builtin_bit_cast(ae_elem8, b1[kk]), acc2[j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   };
   unsigned st_prev = 2 * AE_STAGE_BYTES;
   bool first = true;
   while (x0 < n_items) {
     request_item(x1, st_req);
     if (first) __syncthreads();                                // A (nothing is handed over yet)
-    else add_handed_over(st_prev, [&]() AE_LAMBDA { __syncthreads(); });
+    else add_handed_over(st_prev, [&]() AE_LAMBDA { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __syncthreads(); });
     first = false;
     __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
     __syncthreads();                                           // B
@@ -1093,6 +1182,12 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
     int le = lane;
     asm volatile("" : "+v"(le));
     ae_lds_byte* os1 = lds + rw * AE_OUT_BYTES;
+#if AE_BWD_PAIRS
+    const float scale1 = nb == 0 ? AE_SM_SCALE : 1.f, scale2 = scale1;
+#else
+    constexpr float scale1 = AE_SM_SCALE, scale2 = 1.f;
+    (void)scale2;
+#endif
 #if AE_BWD_SPLIT && AE_BWD_ROLE == 1
     merge_parts(acc1, 0);
 #endif
@@ -1105,7 +1200,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
         for (int rg = 0; rg < 4; rg++) {
           ae_elem4 w;
 #pragma unroll
-          for (int t = 0; t < 4; t++) w[t] = (ae_elem)(acc1[db][rg * 4 + t] * AE_SM_SCALE);
+          for (int t = 0; t < 4; t++) w[t] = (ae_elem)(acc1[db][rg * 4 + t] * scale1);
           *(__attribute__((address_space(3))) ae_elem4*)(orow + (((db * 4 + rg) ^ osw) << 4)) = w;
         }
     }
@@ -1122,14 +1217,22 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
         for (int rg = 0; rg < 4; rg++) {
           ae_elem4 w;
 #pragma unroll
-          for (int t = 0; t < 4; t++) w[t] = (ae_elem)acc2[db][rg * 4 + t];
+          for (int t = 0; t < 4; t++) w[t] = (ae_elem)(acc2[db][rg * 4 + t] * scale2);
           *(__attribute__((address_space(3))) ae_elem4*)(orow + (((db * 4 + rg) ^ osw) << 4)) = w;
         }
     }
 #endif
     // (the rows were written by other lanes of this wave: LDS instructions of a wave complete in order)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    const int rw0 = r0 + rw * 32;
+#if AE_BWD_PAIRS
+    const int rw0 = r0 + half * 64, rw2 = rw0 + 32;
+    ae_elem* o1 = nb == 0 ? (ae_elem*)p.dk + (int64_t)b * p.dk_stride_b + (int64_t)h * p.dk_stride_h
+                          : (ae_elem*)p.dv + (int64_t)b * p.dv_stride_b + (int64_t)h * p.dv_stride_h;
+    ae_elem* o2 = o1;
+    const int64_t os1s = nb == 0 ? p.dk_stride_s : p.dv_stride_s, os2s = os1s;
+#else
+    const int rw0 = r0 + rw * 32, rw2 = rw0;
+    (void)rw2;
 #if AE_BWD_ROLE == 0
     ae_elem* o1 = (ae_elem*)p.dq + (int64_t)b * p.dq_stride_b + (int64_t)h * p.dq_stride_h;
     const int64_t os1s = p.dq_stride_s;
@@ -1137,6 +1240,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
     ae_elem* o1 = (ae_elem*)p.dk + (int64_t)b * p.dk_stride_b + (int64_t)h * p.dk_stride_h;
     ae_elem* o2 = (ae_elem*)p.dv + (int64_t)b * p.dv_stride_b + (int64_t)h * p.dv_stride_h;
     const int64_t os1s = p.dk_stride_s, os2s = p.dv_stride_s;
+#endif
 #endif
 #pragma unroll
     for (int i = 0; i < AE_CPR1 / 2; i++) {
@@ -1153,7 +1257,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
       const int row = n / AE_CPR2, c = n % AE_CPR2;
       const ae_elem8 w = *(const __attribute__((address_space(3))) ae_elem8*)(
           os1 + AE_R1B + row * AE_STR2 + ((c ^ (row & (AE_CPR2 - 1))) << 4));
-      if (rw0 + row < n_res) *(ae_elem8*)(o2 + (int64_t)(rw0 + row) * os2s + c * 8) = w;
+      if (rw2 + row < n_res) *(ae_elem8*)(o2 + (int64_t)(rw2 + row) * os2s + c * 8) = w;
     }
 #endif
   }

@@ -117,6 +117,16 @@ def test_softmax_backward_item_walk(cuda_device, B, H, Hkv, Sq, Skv, D, causal):
     _run(B, H, Hkv, Sq, Skv, D, D, torch.float16, C.causal_mask if causal else None, causal and Sq == Skv)
 
 
+@pytest.mark.parametrize("Sq,Skv,causal", [(1, 1, True), (33, 33, True), (64, 64, True), (65, 65, True), (95, 95, True), (129, 129, True),
+                                           (1, 129, False), (31, 65, False), (32, 64, False), (33, 97, False), (63, 31, False), (96, 128, False)])
+@pytest.mark.parametrize("Hkv,dtype", [(3, torch.bfloat16), (1, torch.float16)])
+def test_dk_dv_at_the_edges_of_their_waves(cuda_device, Sq, Skv, causal, Hkv, dtype):
+    """Head dim 128, softmax (AE_BWD_PAIRS): a wave holds 64 kv rows and takes 32 q rows, another 64 rows of dk or of dv: lengths
+    around those, so that whole waves have no rows, or no q rows."""
+    print(f"case dk dv edges Sq{Sq} Skv{Skv} causal={causal} Hkv{Hkv} {dtype}", flush=True)
+    _run(2, 3, Hkv, Sq, Skv, 128, 128, dtype, C.causal_mask if causal else None, causal, seed=Sq)
+
+
 def test_softmax_backward_headline_shape(cuda_device):
     """The shape bench.py times the backward on (B2 H32 S4096 D128 fp16, causal): every gradient finite,
     and dq, dk, dv of two (batch, head) slices -- which depend on that slice's tensors only -- against the
