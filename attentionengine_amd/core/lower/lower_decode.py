@@ -585,6 +585,8 @@ class MLADecodeOp(_SplitTuning):
     HEADS_PER_WG = 64
     # wave-specialised kernel, per round of workgroups: query heads a workgroup -> (us to start and end, us per tile)
     ROUND_COST = {16: (1.9, 0.585), 32: (3.7, 0.73), 64: (4.9, 0.81)}
+    # ... and where the entries of a paged cache are split by their lengths
+    LENGTH_COST = {16: (3.03, 0.591), 32: (4.53, 0.784), 64: (6.48, 0.937)}
     K_PAD = 0
     # sqrt(a / b) of _balanced_splits(): B1 H128 Skv4096 takes 112 us unsplit and about 0.3 us more per split
     SPLIT_COEFF = 0.30
@@ -645,32 +647,81 @@ class MLADecodeOp(_SplitTuning):
 
         Kept by the number of tiles: a latent cache that grows by a token a call asks anew every 32 calls (20 to 40 us; the 3 x 64
         candidates evaluated at every length took 130 to 270, more than the choice gains)."""
-        read = units * tiles * MLADecodeOp.BLOCK_N * 2e-6 * d / 5.7
-        partial = 0.31 * units * group * 4e-6 * dv
         splits = sorted({-(-tiles // -(-tiles // n)) for n in range(n_splits[0], n_splits[1] + 1)})      # (none without tiles)
         best = None
-        for heads, (f, c) in MLADecodeOp.ROUND_COST.items():
+        for heads in MLADecodeOp.ROUND_COST:
             if heads != 16 and group <= heads // 2:
                 continue
-            wgs = units * -(-group // heads)
             for n in splits:
-                trip = f + c * -(-tiles // n)
-                us = ((-(-wgs * n // cus) * trip) ** 4 + read ** 4) ** 0.25
-                if n > 1:
-                    us += 1.2 + 0.077 * n + partial * n
-                if paged:
-                    live = (n + 1) / (2 * n)
-                    rounds = math.ceil(math.ceil(wgs * n * (live * 1.4 if n > 1 else 1.0) - 1e-6) / cus)
-                    us += ((rounds * trip) ** 4 + (read * (0.5 if n > 1 else 1.0)) ** 4) ** 0.25
-                    if n > 1:
-                        us += 1.2 + 0.077 * n + partial * n * live
+                us = sum(MLADecodeOp._call_us(units, group, tiles, heads, n, cus, d, dv, spread) for spread in ((False, True) if paged else (False,)))
                 if best is None or (us, -heads, n) < best:
                     best = us, -heads, n
         return -best[1], best[2]
 
+    @staticmethod
+    def _call_us(units, group, tiles, heads, n, cus, d, dv, spread):
+        """``_cheapest``'s cost of one choice; ``spread``: entries spread evenly up to the table's width."""
+        f, c = MLADecodeOp.ROUND_COST[heads]
+        read = units * tiles * MLADecodeOp.BLOCK_N * 2e-6 * d / 5.7
+        wgs = units * -(-group // heads)
+        live = (n + 1) / (2 * n) if spread else 1.0
+        rounds = math.ceil(math.ceil(wgs * n * (live * 1.4 if spread and n > 1 else 1.0) - 1e-6) / cus)
+        us = ((rounds * (f + c * -(-tiles // n))) ** 4 + (read * (0.5 if spread and n > 1 else 1.0)) ** 4) ** 0.25
+        return us + (1.2 + 0.077 * n + 0.31 * units * group * 4e-6 * dv * n * live if n > 1 else 0.0)
+
+    @staticmethod
+    @functools.lru_cache(maxsize=1024)
+    def _splits_by_length(batch, group, tiles, fixed, cus, d, dv):
+        """(query heads of a workgroup, the most splits of an entry, workgroups a head tile) for a paged call whose kernel cuts the
+        entries by their lengths (``ae_split_by_length`` of csrc/kernels/ae_device.h), None where ``fixed``, (heads, splits) of
+        equal spans of the table, is the better plan.
+
+        With equal spans the host plans for entries that fill their tables, and shorter ones leave workgroups without keys (B8
+        H128, up to 2048 tokens: 96 of 256).  Cut by length, every workgroup of a whole number of rounds has about as many tiles.  Costs
+        fitted to 1738 calls (62 shapes, every form), 5 % off; a batch spread evenly counts 1, one that fills its tables 0.7, and may
+        take 1.08 of its time at most.  Over those shapes, evenly spread 0.98 of the time (30 shapes keep their plan; B8 H128
+        2048 18.4 -> 16.4 us, B64 H128 4096 85 -> 64, B30 H64 2560 26.8 -> 24.1), full tables 0.99 (18.7 -> 19.1, 139 -> 102, 49.4 ->
+        31.6; 1.07 at most, B24 H128 1024 25.4 -> 27.2).  Fewer than four entries have little to share: up to 1.5 us slower, the lengths are waited for."""
+        if batch < 4 or tiles < 8:
+            return None
+
+        def cut(lengths, n_wgs, most):
+            per = max(4, -(-sum(lengths) // n_wgs), -(-max(lengths) // most))
+            while True:
+                splits = [max(1, -(-t // per)) for t in lengths]
+                if sum(splits) <= n_wgs:
+                    return per, sum(splits)
+                per += max(1, per // 16)
+
+        def us(heads, n_wgs, most, spread):
+            lengths = [-(-tiles * (i + 1) // batch) for i in range(batch)] if spread else [tiles] * batch
+            per, n = cut(lengths, n_wgs, most)
+            f, c = MLADecodeOp.LENGTH_COST[heads]
+            read = sum(lengths) * MLADecodeOp.BLOCK_N * 2e-6 * d / 4.8
+            return (((-(-n * -(-group // heads) // cus) * (f + c * per)) ** 4 + read ** 4) ** 0.25 + 0.32 * group * 4e-6 * dv * n
+                    + 0.05 * most + 0.5)
+        full, spread = (MLADecodeOp._call_us(batch, group, tiles, *fixed, cus, d, dv, s) for s in (False, True))
+        best = None
+        for heads in MLADecodeOp.LENGTH_COST:
+            if heads != 16 and group <= heads // 2:
+                continue
+            for rounds in range(1, 5):
+                n_wgs = rounds * cus // -(-group // heads)
+                if not batch <= n_wgs <= 64 * batch:
+                    continue
+                for most in (2, 4, 8, 16):
+                    if 2 * most > tiles or most * batch < 0.45 * n_wgs or most > 4 * n_wgs / batch + 2:
+                        continue
+                    this_full = us(heads, n_wgs, most, False)
+                    cost = us(heads, n_wgs, most, True) + 0.7 * this_full
+                    if this_full <= 1.08 * full and cost < spread + 0.7 * full and (best is None or cost < best[0]):
+                        best = cost, heads, most, n_wgs
+        return best[1:] if best else None
+
     def plan(self, B, Hq, Hkv, Skv, page=None):
         """(query heads of a workgroup, number of splits, kv positions per split); with a paged cache a split spans at
-        most as many pages as the kernel keeps table entries for.
+        most as many pages as the kernel keeps table entries for, and where the kernel cuts the entries by their lengths
+        (``_splits_by_length``) there is a fourth number, the workgroups a head tile that share them, and the second is the most splits of an entry.
 
         The wave-specialised kernel has forms for 16, 32 and 64 heads a workgroup: the fewer, the shorter a trip over
         one tile (0.59 / 0.73 / 0.81 us, paged 0.53 with 16 heads: the plans by this cost are 0.7 % off the best there)
@@ -687,6 +738,10 @@ class MLADecodeOp(_SplitTuning):
         if self._wave_specialised():
             span = (clamped(tuned),) * 2 if tuned else (clamped(least), clamped(self.MAX_SPLITS))
             heads, n_split = self._cheapest(B * Hkv, group, tiles, span, self.target_workgroups, self.D, self.DV, page is not None)
+            if page is not None and Hkv == 1 and B <= 64 and Skv // page + 2 <= self.PAGE_TABLE_ENTRIES and Skv <= 1 << 24 and not tuned:
+                by_length = self._splits_by_length(B, group, tiles, (heads, n_split), self.target_workgroups, self.D, self.DV)
+                if by_length is not None:
+                    return by_length[0], by_length[1], -(-tiles // by_length[1]) * self.BLOCK_N, by_length[2]
         else:
             # as many splits as fill the chip, but no more than the merge is worth: B1 H128 Skv4096 takes 24 us with
             # 16 splits, 92 us with the 128 that would occupy every CU
@@ -698,7 +753,7 @@ class MLADecodeOp(_SplitTuning):
 
     def plan_splits(self, B, Hq, Hkv, Skv, page=None):
         """(number of splits, kv positions per split) of ``plan``."""
-        return self.plan(B, Hq, Hkv, Skv, page)[1:]
+        return self.plan(B, Hq, Hkv, Skv, page)[1:3]
 
     def _wave_specialised(self):
         """The wave-specialised kernel (scores computed once, a third of the LDS traffic) runs where the graph is the
@@ -737,7 +792,7 @@ class MLADecodeOp(_SplitTuning):
                 lds = self.N_STAGES * self.BLOCK_N * 2 * self.D
             cfg = rt.TileCfg(block_m=heads, block_n=self.BLOCK_N, threads=threads, lds_bytes=lds,
                              head_dim=self.D, head_dim_v=self.DV, elem_bytes=2,
-                             n_rowscales=self.n_rowscales, mask_mode=0, paged=1 if paged else 0)
+                             n_rowscales=self.n_rowscales, mask_mode=0, paged=(2 if ws else 1) if paged else 0)
             v = self._variants[key] = (module, cfg, cfg_src)
         return v
 
@@ -819,8 +874,8 @@ class MLADecodeOp(_SplitTuning):
         if self._tune_file and key not in self._tuned:
             page = paged[2] if paged is not None else None
             n0 = self.plan_splits(*key, page=page)[0]
+            cands = [0] if len(self.plan(*key, page=page)) == 4 else []      # (0: the entries split by their lengths)
             self._tuned[key] = n0
-            cands = []
 
             def made_of(n):
                 self._tuned[key] = n
@@ -834,7 +889,7 @@ class MLADecodeOp(_SplitTuning):
             self._tuned[key] = n0
             self._tune_splits(key, cands, lambda: self._launch(q1, q2, k1, k2, B, Hq, Hkv, Skv, paged),
                               lambda n: n > 0 and made_of(n) == n)
-        heads, n_split, kv_per_split = self.plan(B, Hq, Hkv, Skv, page=paged[2] if paged is not None else None)
+        heads, n_split, kv_per_split, *by_length = self.plan(B, Hq, Hkv, Skv, page=paged[2] if paged is not None else None)
         module, cfg, _ = self._variant(n_split, paged is not None, heads)
         ccfg = self._merges.cfg(n_split)
         out = torch.empty((B, 1, Hq, self.DV), dtype=self.dtype, device=dev)
@@ -845,7 +900,7 @@ class MLADecodeOp(_SplitTuning):
         partial_o = partial_rs = None
         if n_split > 1:      # a single split writes `out` directly, no work buffers
             partial_o = torch.empty((B, Hq, n_split, self.DV), dtype=torch.float32, device=dev)
-            partial_rs = torch.empty((max(1, self.n_rowscales), B, Hq, n_split), dtype=torch.float32, device=dev)
+            partial_rs = torch.empty(max(1, self.n_rowscales) * B * Hq * n_split + (B if by_length else 0), dtype=torch.float32, device=dev)
             p.partial_o, p.partial_rs = partial_o.data_ptr(), partial_rs.data_ptr()
         if self._stamped(n_split):
             n_ht = -(-(Hq // Hkv) // heads)
@@ -868,6 +923,7 @@ class MLADecodeOp(_SplitTuning):
             block_table, cache_seqlens, page, n_pages = paged
             p.block_table, p.seqlens_k = block_table.data_ptr(), cache_seqlens.data_ptr()
             p.block_table_stride, p.page_block_size, p.num_pages = block_table.stride(0), page, n_pages
+            p.tail_slots = by_length[0] if by_length else 0
         split, combine, modules = module.kernel("ae_mla_decode_split_kernel"), None, (module,)
         if n_split > 1:
             modules += (self._merges.module(n_split),)
@@ -876,7 +932,7 @@ class MLADecodeOp(_SplitTuning):
         if not self._stamped(n_split) and (self.n_rowscales == 1 or not self.cute):
             host.add_forward(self._host, host.MLA if paged is None else host.MLA_PAGED, B, 1, Hq, Hkv, Skv, dev, modules, split,
                              cfg, combine=combine, ccfg=ccfg, n_split=n_split, kv_per_split=kv_per_split,
-                             page=paged[2] if paged is not None else 0)
+                             page=paged[2] if paged is not None else 0, tail_slots=by_length[0] if by_length else 0)
         self.final_rowscales = dict(zip(self.names, rowscales))
         self._keepalive = [partial_o, partial_rs, q1, q2, k1, k2, paged]
         if self.cute:

@@ -596,8 +596,14 @@ int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params
     if (p->kv_per_split % cfg->block_n != 0)
       return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: kv_per_split=%d is not a multiple of the %d-token kv tile",
                   p->kv_per_split, cfg->block_n);
+    // splits by the entries' lengths: kernels that cut them (paged 2), a lane of a wave an entry, a split of any length
+    if (p->tail_slots != 0 && (cfg->paged != 2 || p->heads_kv != 1 || p->batch > 64 || p->tail_slots < p->batch ||
+                               p->tail_slots > (1 << 20) || p->seqlen_kv > (1 << 24) || p->num_splits < 2))
+      return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: %d workgroups a head tile for the splits of %d entries of %d kv heads, at "
+                                      "most %d each, by a kernel with paged=%d", p->tail_slots, p->batch, p->heads_kv, p->num_splits,
+                  cfg->paged);
     // (the wave-specialised kernel keeps a split's part of the block table in LDS: AE_PTAB = 1024 entries)
-    if (p->kv_per_split / p->page_block_size + 2 > 1024)
+    if ((p->tail_slots != 0 ? p->seqlen_kv : p->kv_per_split) / p->page_block_size + 2 > 1024)
       return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: a split of %d tokens spans more than 1022 pages of %d tokens "
                                       "(use more splits)", p->kv_per_split, p->page_block_size);
     // the paged kernels address the rope columns as an offset from the latent ones inside one cache tensor
@@ -639,6 +645,7 @@ int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params
   int64_t units = (int64_t)p->batch * p->heads_kv * p->num_splits, a_head = p->num_splits;
   if (cfg->paged && units * n_ht > 128) a_head |= 1;
   units = (int64_t)p->batch * p->heads_kv * a_head;
+  if (cfg->paged && p->tail_slots != 0) units = p->tail_slots;
   int64_t total = ((units + 7) / 8) * 8 * n_ht;
   if (total > 0x7fffffffll) return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: grid too large");
   uint32_t grid[3] = {(uint32_t)total, 1, 1};

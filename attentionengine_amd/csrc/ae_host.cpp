@@ -445,7 +445,8 @@ PyObject* run(Host* h, PyObject* const* args, Py_ssize_t nargs, bool mla) {
   const int64_t rs_floats = (h->n_rs > 0 ? h->n_rs : 1) * B * Sq * Hq * pl.n_split;
   at::Tensor po, prs;
   if (pl.kind != kPrefill || pl.tail_slots) p.num_splits = pl.n_split, p.kv_per_split = pl.kv_per_split;
-  if (pl.tail_slots) {      // (only the counters are kept: the partial results are the size of a few thousand rows)
+  if (pl.kind == kMlaPaged) p.tail_slots = pl.tail_slots;
+  if (pl.kind != kMlaPaged && pl.tail_slots) {      // (only the counters are kept: the partial results are the size of a few thousand rows)
     p.tail_slots = pl.tail_slots;
     po = empty({pl.o_rows, h->DV}, at::kFloat, dev);
     prs = get_work(h, 1, 1, pl.counters, dev, stream, true).second.narrow(0, 1, pl.counters);
@@ -459,7 +460,7 @@ PyObject* run(Host* h, PyObject* const* args, Py_ssize_t nargs, bool mla) {
     std::tie(po, prs) = get_work(h, pl.o_rows, rs_floats, pl.counters, dev, stream, false);
   } else if (pl.n_split > 1 && pl.cfg.merge_in_wg == 0) {
     po = empty({pl.o_rows, h->DV}, at::kFloat, dev);
-    prs = empty({rs_floats}, at::kFloat, dev);
+    prs = empty({rs_floats + (pl.tail_slots ? B : 0)}, at::kFloat, dev);
   }
   if (po.defined()) p.partial_o = (float*)po.mutable_data_ptr(), p.partial_rs = (float*)prs.mutable_data_ptr();
 

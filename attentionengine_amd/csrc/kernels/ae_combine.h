@@ -31,16 +31,20 @@ void ae_decode_combine_kernel(const ae_attn_params p) {
   constexpr int TPR = AE_DV / 4 < AE_COMBINE_THREADS ? AE_DV / 4 : AE_COMBINE_THREADS;      // threads per row
   const int h = AE_COMBINE_ROWS == 1 ? blockIdx.x : blockIdx.x * AE_COMBINE_ROWS + threadIdx.x / TPR;
   const int b = blockIdx.y;
-  if (threadIdx.x >= AE_COMBINE_ROWS * TPR || h >= p.heads_q) return;
   const int n_part = (unsigned)p.num_splits / AE_SPLITS_PER_PARTIAL;
+  if (threadIdx.x >= AE_COMBINE_ROWS * TPR || h >= p.heads_q) return;
   // Paged cache (per-entry lengths): only the first ceil(length / kv_per_split) splits of an entry hold keys and
   // wrote partial results; an entry with at most one wrote `out` itself.
   int n_used = n_part;
   if (p.seqlens_k != nullptr) {
-    int len = p.seqlens_k[b];
-    len = len < p.seqlen_kv ? len : p.seqlen_kv;
-    const int n = (int)((unsigned)((len > 0 ? len : 0) + p.kv_per_split - 1) / (unsigned)p.kv_per_split);
-    n_used = n < n_part ? n : n_part;
+    if (p.tail_slots != 0) {           // (the split kernel has cut the entries, and says how often)
+      n_used = ((const int*)(p.partial_rs + (int64_t)AE_N_ROWSCALES * p.batch * p.heads_q * n_part))[b];
+    } else {
+      int len = p.seqlens_k[b];
+      len = len < p.seqlen_kv ? len : p.seqlen_kv;
+      const int n = (int)((unsigned)((len > 0 ? len : 0) + p.kv_per_split - 1) / (unsigned)p.kv_per_split);
+      n_used = n < n_part ? n : n_part;
+    }
     if (n_used <= 1) return;
   }
   // The partial results are read 16 splits at a time, unconditionally, so that the loads of a group all go
@@ -139,6 +143,11 @@ void ae_decode_combine_kernel(const ae_attn_params p) {
 #if AE_NSPLIT % 8 == 0
   else if (n_used == AE_NSPLIT / 8 * 5) merge(ae_places<AE_NSPLIT / 8 * 5>());
   else if (n_used == AE_NSPLIT / 8 * 7) merge(ae_places<AE_NSPLIT / 8 * 7>());
+#endif
+#if AE_NSPLIT == 8 || AE_NSPLIT == 16
+  else if (n_used == AE_NSPLIT / 2) merge(ae_places<AE_NSPLIT / 2>());       // (paged entries have any count)
+  else if (n_used == AE_NSPLIT / 8 * 3) merge(ae_places<AE_NSPLIT / 8 * 3>());
+  else if (n_used == AE_NSPLIT / 4) merge(ae_places<AE_NSPLIT / 4>());
 #endif
 #if AE_NSPLIT == 16
   else if (n_used == 9) merge(ae_places<9>());

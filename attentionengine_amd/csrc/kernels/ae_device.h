@@ -385,4 +385,51 @@ AE_DEV constexpr int ae_kv_off(int e) { return (e >> 2) * 16 + (e & 3); }
 AE_DEV constexpr int ae_kv_off(int e) { return (e >> 4) * 32 + ((e & 15) >> 2) * 8 + (e & 3); }
 #endif
 
+// ---- paged launches whose splits follow the entries' lengths (ae_attn_params.tail_slots; batches of at most 64) ------------
+// inclusive scan over the wave's lanes, all of them active: sums, or maxima of numbers >= 0
+template <bool MAX>
+AE_DEV int ae_wave_scan(int x) {
+  auto step = [&](int y) AE_LAMBDA { x = MAX ? (x > y ? x : y) : x + y; };
+  step(__builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false));      // row_shr 1, 2, 4, 8
+  step(__builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false));      // row_bcast 15, 31
+  step(__builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false));
+  return x;
+}
+// The kv axes of all entries cut into splits of `tiles` kv tiles, the fewest with which p.tail_slots workgroups a head tile
+// suffice and no entry has more than p.num_splits: lane b's entry has `mine` of them (one at least), the entries up to it `upto`.
+// Equal spans of the table, which the host can plan, leave the workgroups without keys whose spans lie behind an entry's end, and the
+// launch takes as long as the longest entry's.  Every wave works this out from the lengths (0.2 us, and they are one trip to
+// memory that the first requests wait for).  us, equal spans -> so, entries spread evenly up to the table's width | all of that
+// width: B8 H128 2048 tokens 18.4 -> 16.4 | 18.7 -> 19.1, B64 H128 4096 85 -> 64 | 139 -> 102, B30 H64 2560 26.8 -> 24.1 | 49.4 -> 31.6,
+// B5 H128 4736 23.5 -> 19.6 | 24.1 -> 24.5.  Which calls take it: MLADecodeOp._splits_by_length.
+struct ae_paged_splits { int tiles, mine, upto; };
+#define AE_LEAST_TILES 4      // (a split's start and end, and its partial result, take as long as four trips)
+AE_DEV ae_paged_splits ae_split_by_length(const ae_attn_params& p, int lane, int entry_tiles) {
+  ae_paged_splits s;
+  const bool there = lane < p.batch;
+  entry_tiles = there ? entry_tiles : 0;
+  const int total = __builtin_amdgcn_readlane(ae_wave_scan<false>(entry_tiles), 63);
+  int rest;
+  s.tiles = ae_divide_small(total + p.tail_slots - 1, p.tail_slots, rest);
+  s.tiles = s.tiles > AE_LEAST_TILES ? s.tiles : AE_LEAST_TILES;
+  for (;;) {            // (ends: with s.tiles at the longest entry's every entry has one split, and there are at most p.tail_slots entries)
+    const int a = entry_tiles + s.tiles - 1;
+    int n = (int)((float)a * __builtin_amdgcn_rcpf((float)s.tiles));       // off by at most one below 2^22
+    n -= n * s.tiles > a ? 1 : 0;
+    n += a - n * s.tiles >= s.tiles ? 1 : 0;
+    s.mine = there ? (n > 1 ? n : 1) : 0;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(s.mine > p.num_splits) != 0, 0)) {      // (one entry far longer than the others)
+      const int most = __builtin_amdgcn_readlane(ae_wave_scan<true>(entry_tiles), 63);
+      s.tiles = ae_divide_small(most + p.num_splits - 1, p.num_splits, rest);
+      continue;
+    }
+    s.upto = ae_wave_scan<false>(s.mine);
+    if (__builtin_amdgcn_readlane(s.upto, 63) <= p.tail_slots) return s;
+    s.tiles += s.tiles >> 4 > 1 ? s.tiles >> 4 : 1;
+  }
+}
+
 #endif  // AE_DEVICE_H

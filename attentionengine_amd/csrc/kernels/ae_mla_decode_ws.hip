@@ -93,6 +93,7 @@
 #define AE_LB(i) (((i) * AE_LOADS + AE_BURSTS - 1) / AE_BURSTS)
 #ifndef AE_NSTAGE
 #define AE_NSTAGE 4
+#define AE_WHOLE_TABLE 512     // ... or the whole table, up to this
 #define AE_PTAB 1024      // paged cache: block-table entries of one split kept in LDS
 #endif
 #define AE_PSTR 80                        // LDS pitch of one head's P row (32 kv * 2 B, padded against bank conflicts)
@@ -183,8 +184,13 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   }
   const unsigned u = (unsigned)(u8 * 8 + (wg & 7));      // flattened (batch, kv head, split)
 #if AE_NSPLIT == 1
-  const int n_split = 1;
+  const int n_split = 1, per_split = p.kv_per_split;
   int split = 0, b = u, hk = 0;
+#if AE_PAGED
+  constexpr bool by_length = false;
+  constexpr int len_b = 0;
+  constexpr bool whole_table = false;
+#endif
 #else
   const int n_split = p.num_splits;
   int units = n_split, split, hk = 0;
@@ -192,6 +198,43 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   if (ae_mla_odd_units(p, n_ht)) units |= 1;
 #endif
   int b;
+#if AE_PAGED
+  // (splits by the entries' lengths: see ae_split_by_length)
+  const bool by_length = p.tail_slots != 0;
+  const int table_ints = (p.batch - 1) * p.block_table_stride + ((p.page_block_size & (p.page_block_size - 1)) == 0
+                                        ? (p.seqlen_kv + p.page_block_size - 1) >> __builtin_ctz(p.page_block_size)
+                                        : (p.seqlen_kv + p.page_block_size - 1) / p.page_block_size);
+  int table_all[AE_WHOLE_TABLE / 64];
+  bool whole_table = false;
+  int per_split = p.kv_per_split, n_mine = 0, len_b = 0;
+  if (by_length) {
+    if ((int)u >= p.tail_slots) return;                        // grid padding
+    int len = lane < p.batch ? p.seqlens_k[lane] : 0;
+    // a small block table is requested whole, together with the lengths (what an entry left unset is read, but never followed);
+    // of a larger one the split's part, once it is known which that is: another trip to memory
+    whole_table = table_ints <= AE_WHOLE_TABLE;
+    if (whole_table && requests) {
+#pragma unroll
+      for (int i = 0; i < AE_WHOLE_TABLE / 64; i++)
+        if (i * 64 + lane < table_ints) table_all[i] = p.block_table[i * 64 + lane];
+    }
+    len = len < p.seqlen_kv ? len : p.seqlen_kv;
+    len = len > 0 ? len : 0;
+    const ae_paged_splits s = ae_split_by_length(p, lane, (len + AE_BN - 1) / AE_BN);
+    b = __builtin_popcountll(__builtin_amdgcn_ballot_w64(s.upto <= (int)u));     // entries in front of the unit's
+    b = b < p.batch ? b : p.batch;
+    if (b >= p.batch) return;                                  // (fewer splits than units)
+    n_mine = __builtin_amdgcn_readlane(s.mine, b);
+    split = (int)u - (__builtin_amdgcn_readlane(s.upto, b) - n_mine);
+    per_split = s.tiles * AE_BN;
+    len_b = __builtin_amdgcn_readlane(len, b);
+    // (for the merge kernel: behind the row scales)
+    if (split == 0 && ht == 0 && tid == 0)
+      ((int*)(p.partial_rs + (int64_t)AE_N_ROWSCALES * p.batch * p.heads_q * n_split))[b] = n_mine;
+  } else
+#else
+  const int per_split = p.kv_per_split;
+#endif
   if (__builtin_expect(p.units_reciprocal != 0, 1)) {
     b = (int)(((uint64_t)u * (uint32_t)p.units_reciprocal) >> 32);
     split = (int)u - b * units;
@@ -208,7 +251,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 
   // (wave-uniform values are pinned to scalar registers: a copy in a vector register that gets spilled is
   // reloaded with a scratch load, which the tile loads' vmcnt bookkeeping would have to wait for)
-  const int kv_begin = __builtin_amdgcn_readfirstlane(split * p.kv_per_split);
+  const int kv_begin = __builtin_amdgcn_readfirstlane(split * per_split);
 #if AE_PAGED
   const ae_elem* k1 = (const ae_elem*)p.k + (int64_t)hk * p.k_stride_h;
   const ae_elem* k2 = (const ae_elem*)p.k2 + (int64_t)hk * p.k2_stride_h;
@@ -216,8 +259,9 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   const int page_size = p.page_block_size;
   int rq_slot0, top_slot;          // table slots of the split's first token and of the last one that it could hold
   {
-    int top = kv_begin + p.kv_per_split;
-    top = (top < p.seqlen_kv ? top : p.seqlen_kv) - 1;
+    const int limit = by_length ? len_b : p.seqlen_kv;
+    int top = kv_begin + per_split;
+    top = (top < limit ? top : limit) - 1;
     top = top > 0 ? top : 0;
     if (__builtin_expect((page_size & (page_size - 1)) != 0, 0)) {
       rq_slot0 = kv_begin / page_size;
@@ -230,9 +274,9 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   // The entry's length and the split's first 64 table entries are requested together (one after the other they held the
   // first tile back by another trip to memory).  So the entries are those that the split COULD hold: inside the table's
   // row; what an entry shorter than that left unset is read, but never followed.
-  int seqlen_b = p.seqlens_k[b];
+  int seqlen_b = by_length ? len_b : p.seqlens_k[b];
   int table0 = 0;
-  if (requests && rq_slot0 + lane <= top_slot) table0 = pages[rq_slot0 + lane];
+  if (requests && !whole_table && rq_slot0 + lane <= top_slot) table0 = pages[rq_slot0 + lane];
 #else
   const ae_elem* k1 = (const ae_elem*)p.k + (int64_t)b * p.k_stride_b + (int64_t)hk * p.k_stride_h;
   const ae_elem* k2 = (const ae_elem*)p.k2 + (int64_t)b * p.k2_stride_b + (int64_t)hk * p.k2_stride_h;
@@ -319,7 +363,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   seqlen_b = __builtin_amdgcn_readfirstlane(seqlen_b > 0 ? seqlen_b : 0);
 #endif
 
-  int kv_end_ = kv_begin + p.kv_per_split;
+  int kv_end_ = kv_begin + per_split;
   kv_end_ = kv_end_ < seqlen_b ? kv_end_ : seqlen_b;
   const int kv_end = __builtin_amdgcn_readfirstlane(kv_end_);
   const int n_tiles = __builtin_amdgcn_readfirstlane(kv_end > kv_begin ? (kv_end - kv_begin + AE_BN - 1) / AE_BN : 0);
@@ -336,7 +380,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #if AE_NSPLIT == 1
   constexpr bool direct = true;
 #elif AE_PAGED
-  const bool direct = seqlen_b <= p.kv_per_split;      // ae_mla_splits_used() <= 1
+  const bool direct = seqlen_b <= per_split;           // (one split with keys at most)
 #else
   constexpr bool direct = false;
 #endif
@@ -626,9 +670,25 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   // waiting for every tile requested so far - 0.190 against 0.170 ms for the dense cache at B128 H128 S4096,
   // 0.166 ms with the table in LDS.  Every value wave writes the same entries and reads them back itself (a wave's
   // LDS operations complete in order), so no barrier is needed.
+  int rq_idx = 0;
+#if AE_NSPLIT > 1
+  if (whole_table) {
+#pragma unroll
+    for (int i = 0; i < AE_WHOLE_TABLE / 64; i++)
+      if (i * 64 + lane < table_ints) ptab[i * 64 + lane] = table_all[i];
+    // (the first page from the registers: what goes through LDS is there when the second is looked up)
+    rq_idx = b * p.block_table_stride + rq_slot0;
+    const int at = rq_idx >> 6;
+    table0 = table_all[0];
+#pragma unroll
+    for (int i = 1; i < AE_WHOLE_TABLE / 64; i++) table0 = at == i ? table_all[i] : table0;
+    table0 = __builtin_amdgcn_readlane(table0, rq_idx & 63);
+  } else
+#endif
+  {
   if (rq_slot0 + lane <= top_slot) ptab[lane] = table0;
   for (int i = 64 + lane; i < AE_PTAB && rq_slot0 + i <= top_slot; i += 64) ptab[i] = pages[rq_slot0 + i];   // (<= AE_PTAB: checked by ae_mla_decode_fwd)
-  int rq_idx = 0;
+  }
   int rq_in_page = kv_begin - rq_slot0 * page_size;
   int rq_page = __builtin_amdgcn_readfirstlane(table0);
 #endif

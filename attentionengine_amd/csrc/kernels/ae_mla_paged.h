@@ -4,7 +4,8 @@
 // Splits of a batch entry that hold keys: ceil(length / kv_per_split).  An entry with at most one writes its
 // result itself (split 0: `out` and the row scales, as a launch without splits does) and the merge kernel
 // passes it over; the merge of a longer entry reads only the splits that hold keys.  Splits without keys
-// write nothing.
+// write nothing.  Where the wave-specialised kernel cuts the entries by their lengths (ae_split_by_length in ae_device.h) an entry
+// has at least one split and all of them hold keys; the merge reads their number, which the split kernel leaves behind the row scales.
 //
 // ae_mla_write_no_keys: result of an entry of length 0, written by the whole workgroup of its split 0: zero
 // output and -inf row scales, the values the kernels' epilogues produce for an empty range.

@@ -103,14 +103,18 @@ typedef struct ae_attn_params {
   /* prefill kernels compiled with AE_TAIL 1 (announced by cfg->merge_in_wg = 2): of the q-tile slots of every XCD (see
    * ae_prefill_fwd) the last tail_slots are shared by num_splits workgroups each, kv_per_split positions a workgroup;
    * the one that finishes last merges.  partial_o: 8 * tail_slots * num_splits * (block_m * DV + 4 * threads) floats;
-   * partial_rs: 8 * tail_slots int32 arrival counters, zero when the launch starts and when it ends.  Else 0
-   * (ae_prefill_split_fwd fills it in for its split kernel). */
+   * partial_rs: 8 * tail_slots int32 arrival counters, zero when the launch starts and when it ends.
+   * MLA decode on a paged cache, kernels whose ae_tile_cfg.paged is 2: not 0 where the kernel cuts the entries into splits by
+   * their lengths (one kv head, at most 64 entries): the workgroups a head tile that share the splits, one an entry at
+   * least; num_splits is then the most splits of an entry, kv_per_split is not read, and partial_rs has, behind the row
+   * scales, an int32 an entry (the kernel leaves the entry's number of splits there for the merge).
+   * Else 0 (ae_prefill_split_fwd fills it in for its split kernel). */
   int32_t tail_slots;
   /* Filled in by ae_mla_decode_fwd for its split kernel, whatever the caller left there: ceil(2^32 / u) of the number u of
    * workgroup ids per (batch, kv head), or 0 where ids times u do not fit 32 bits. */
   uint32_t units_reciprocal;
   int32_t reserved;
-  /* MLA decode on a paged cache (kernels whose ae_tile_cfg.paged is 1; NULL / 0 otherwise): the cache is
+  /* MLA decode on a paged cache (kernels whose ae_tile_cfg.paged is not 0; NULL / 0 otherwise): the cache is
    * [num_pages, page_block_size, Hkv, D] (k_stride_b = elements between pages, k_stride_s between the
    * rows of a page), token t of batch entry b is row t % page_block_size of page
    * block_table[b * block_table_stride + t / page_block_size], and entry b holds
@@ -118,7 +122,8 @@ typedef struct ae_attn_params {
    * block_table_batch_stride, page_block_size and seqlens_k_ptr
    * (core/template/cute_template_kvshared/kernels/params.h:33-36, flash_api.cpp:61-72).
    * The latent part (k) and the rope part (k2) are column ranges of that ONE cache tensor: equal strides,
-   * k2 at most 1 MiB behind k.  A split spans at most 1022 pages (kv_per_split / page_block_size + 2 <= 1024).
+   * k2 at most 1 MiB behind k.  A split spans at most 1022 pages (kv_per_split / page_block_size + 2 <= 1024;
+   * splits by the entries' lengths: seqlen_kv / page_block_size + 2).
    * In a split launch an entry whose keys all lie in the first split writes `out` itself; splits without
    * keys write nothing and the merge reads only the splits that hold keys. */
   const int32_t* block_table;                /* int32 [B, block_table_stride]             */
@@ -140,7 +145,8 @@ typedef struct ae_tile_cfg {
   int32_t elem_bytes;  /* 2 for fp16/bf16                                                 */
   int32_t n_rowscales; /* number of final rowscales the kernel writes                     */
   int32_t mask_mode;   /* 0 none, 1 analytic causal, 2 block table                        */
-  int32_t paged;       /* MLA decode: 1 when the kernel reads KV through block_table / seqlens_k */
+  int32_t paged;       /* MLA decode: 1 when the kernel reads KV through block_table / seqlens_k, 2 when it can also cut
+                          the entries into splits by their lengths (ae_attn_params.tail_slots) */
   int32_t merge_in_wg; /* GQA decode: 1 when the split kernel was compiled with AE_MERGE_IN_WG 1 (its one
                           workgroup per (batch, kv head, head tile) merges its waves' partial results and
                           writes out itself: no combine kernel, no work buffers); 2 when it was compiled with

@@ -180,6 +180,14 @@ def test_paged_cache_arguments_are_checked_before_any_launch():
     assert rc == 1 and "do not cover Skv=256" in msg
     rc, msg = mla(params(**{**table, "num_pages": 0}), cfg(paged=1))
     assert rc == 1 and "num_pages" in msg
+    # splits by the entries' lengths: a kernel that cuts them, one kv head, 64 entries and a workgroup an entry at the least
+    for wrong, c in ((dict(tail_slots=8), cfg(paged=1)), (dict(tail_slots=1), cfg(paged=2)), (dict(tail_slots=8, num_splits=1), cfg(paged=2)),
+                     (dict(tail_slots=8, heads_kv=2), cfg(paged=2)), (dict(tail_slots=99, batch=65), cfg(paged=2)), (dict(tail_slots=-1), cfg(paged=2))):
+        rc, msg = mla(params(**{**table, "num_splits": 2, "kv_per_split": 128, **wrong}), c)
+        assert rc == 1 and "for the splits of" in msg, (wrong, msg)
+    wide = dict(block_table_stride=2000, page_block_size=32, seqlen_kv=64000, num_splits=64, kv_per_split=1024)
+    rc, msg = mla(params(**{**table, **wide, "tail_slots": 8}), cfg(paged=2))
+    assert rc == 1 and "more than 1022 pages" in msg
     p = params(**table)
     assert lib.ae_prefill_fwd(fake, ctypes.byref(p), ctypes.byref(cfg()), None) == 1
     assert "reads a dense cache" in lib.ae_last_error().decode()

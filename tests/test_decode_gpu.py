@@ -756,3 +756,60 @@ def test_an_mla_split_kernel_takes_its_count_from_the_launch(cuda_device):
         assert (lse[:, :, 0].cpu() - rlse).abs().max().item() <= LSE_TOL
         assert (po[-4096:] == 7.0).all() and (prs[-4096:] == 7.0).all()
     assert len(modules) == 1
+
+
+@pytest.mark.parametrize("dtype,H,heads,page,most,n_wgs,lens", [
+    (torch.bfloat16, 16, 16, 32, 8, 40, [1, 128, 129, 0, 700, 511, 512, 513]),     # entries of one split, one without keys
+    (torch.float16, 40, 32, 64, 4, 9, [64, 1, 32, 33, 2000, 63, 65, 31, 0]),       # as many workgroups as entries: none is split; dead heads
+    (torch.bfloat16, 16, 16, 96, 16, 64, [6000, 1, 1, 1]),                         # one long entry: bounded by the most splits; pages of 96
+    (torch.float16, 64, 64, 32, 2, 128, [320] * 17),                               # full tables, more ids than the whole-table read takes
+    (torch.bfloat16, 16, 16, 32, 8, 200, [17 + 29 * i for i in range(64)]),        # a lane an entry: all 64 of them
+])
+def test_paged_entries_split_by_their_lengths(cuda_device, dtype, H, heads, page, most, n_wgs, lens):
+    """ae_split_by_length: the kernels cut the entries so that every workgroup has about as many tiles.  Table entries beyond an
+    entry's pages are out of range and its unused pages NaN; through Python, through the native host path, and as a graph
+    whose replays meet other lengths than its capture."""
+    print(f"case mla by length {dtype} H{H} heads{heads} page{page} most{most} wgs{n_wgs} B{len(lens)}", flush=True)
+    B, D, DV, scale = len(lens), 576, 512, 1 / math.sqrt(576)
+    width = max(-(-max(lens) // page), 8)
+    tiles = width * page // 32
+    q, q_pe, kv, k_pe = _mla_inputs(B, H, 1, width * page, DV, D - DV, dtype, seed=7)
+    dense = torch.cat([kv, k_pe], -1)
+    order = torch.randperm(B * width, generator=torch.Generator().manual_seed(4)).view(B, width)
+
+    def paged(lens):
+        table = torch.full((B, width), 10 ** 6, dtype=torch.int32)
+        cache = torch.full((B * width, page, 1, D), float("nan"), dtype=dtype)
+        for b, n in enumerate(lens):
+            for j in range(-(-n // page)):
+                table[b, j] = order[b, j]
+                cache[order[b, j]] = dense[b, j * page:(j + 1) * page]
+        return cache.cuda(), table.cuda(), torch.tensor(lens, dtype=torch.int32).cuda()
+    mod = _mla_engine(B, H, 1, width * page, D, DV, dtype, scale, backend="cute")
+    mod.attention.plan = lambda *a, **k: (heads, most, -(-tiles // most) * 32, n_wgs)
+    qq = torch.cat([q, q_pe], -1).cuda()
+    cache, table, seqlens = paged(lens)
+
+    def check(out, lse, lens):
+        for b, n in enumerate(lens):
+            if n == 0:
+                assert (out[b] == 0).all() and (lse[b] == float("-inf")).all()
+                continue
+            ref, lref = R.mla_decode(q[b:b + 1, 0], q_pe[b:b + 1, 0], kv[b:b + 1, :n], k_pe[b:b + 1, :n], scale=scale)
+            assert (out[b:b + 1, 0].float().cpu() - ref).abs().max().item() <= OUT_TOL, b
+            assert (lse[b:b + 1, :, 0].cpu() - lref).abs().max().item() <= LSE_TOL, b
+    for _ in range(2):
+        check(*mod(qq, cache, block_table=table, cache_seqlens=seqlens), lens)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        mod(qq, cache, block_table=table, cache_seqlens=seqlens)
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            out, lse = mod(qq, cache, block_table=table, cache_seqlens=seqlens)
+    for other in (lens[::-1], [max(lens)] * B, lens):
+        for mine, new in zip((cache, table, seqlens), paged(other)):
+            mine.copy_(new)
+        graph.replay()
+        torch.cuda.synchronize()
+        check(out, lse, other)
