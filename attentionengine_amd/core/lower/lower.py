@@ -726,10 +726,15 @@ def pipelined_pays(bf16: bool, batch_heads: int, seqlen: int) -> bool:
     one.  Under the mask the q tiles differ in work, and a launch takes as long as its longest tile or as its share of all
     tiles and their starts, whichever is more: 256-row tiles are longer, fewer and waste more rows at the end of a ragged
     sequence, but multiply faster.  Fitted to both kernels' times of 170 shapes (22 to 400 of the larger tiles an XCD, 1024 to
-    12000 positions; windows of 60 ms, since the first 20 favour the generic one), where the choice (a tie
-    goes to the pipelined kernel) is 0.3 % slower than the better one on average; the lengths of choose_prefill_tiles alone: 7 %.  Pipelined -> generic where it now goes there,
+    12000 positions; windows of 60 ms, since the first 20 favour the generic one), where the choice is 0.3 % slower than the better one on average; the lengths of choose_prefill_tiles alone: 7 %.  Pipelined -> generic where it now goes there,
     us: fp16 B3 H32 S1400 76 -> 64, B1 H32 S2009 56 -> 49, bf16 B4 H16 S2680 146 -> 127, B2 H32 S2867 166 -> 149; the other
-    way it is 270 against 290 for fp16 B2 H32 S4096 and 257 against 280 for bf16 B1 H16 S8192."""
+    way it is 270 against 290 for fp16 B2 H32 S4096 and 257 against 280 for bf16 B1 H16 S8192.
+
+    The factor: past eight heads an XCD their order (ae_heavy_first, ae_head_of_xcd in csrc/kernels/ae_device.h) gave the generic
+    kernel more than the other.  Over 43 such shapes (1100 to 7000 positions) the two kernels are level where the estimates' ratio
+    is 0.945: the pipelined one is 0 to 2 % faster below it, the generic one 1 to 3 % between 0.95 and 0.96 and 1 to 11 % above
+    (bf16 B6 H32 S4352 1058 -> 947, B5 H32 S2999 436 -> 406, B8 Hq24 Hkv8 S3328 599 -> 551, fp16 B8 H32 S1729 281 -> 260,
+    B4 H24 S1763 104 -> 101).  Up to eight a tie goes to the pipelined kernel, as the fit above has it."""
     heads, kv_tiles = -(-batch_heads // 8), -(-seqlen // 64)
     us = []
     for rows, (call, start, longest, shared, p) in zip((256, 128), _CAUSAL_COST[bf16]):
@@ -737,7 +742,7 @@ def pipelined_pays(bf16: bool, batch_heads: int, seqlen: int) -> bool:
         trips = (rows // 64) * n * (n + 1) // 2                    # of a head: q tile i sees (i + 1) * rows / 64 kv tiles
         trips -= (rows // 64) * n - kv_tiles                        # (the last one no more than there are)
         us.append(call + ((longest * kv_tiles) ** p + (heads * (shared * trips + start * n) / (_MI355X_CUS // 8)) ** p) ** (1 / p))
-    return us[0] < 1.03 * us[1]
+    return us[0] < (0.95 if heads > 8 else 1.03) * us[1]
 
 
 def kv_group_tiles(d: int, dv: int, batch_heads: int, seqlen_q: int, seqlen_kv: int, banded: bool):
