@@ -15,12 +15,8 @@
 //     waves' fragment reads, 144 KiB per tile, took 2.6x the time of their MFMAs), lazy online softmax,
 //     P^T written to LDS as the B operand of the second product, per-head rescale factors next to it;
 //   * 4 "value waves" (a quarter of the value columns each, all 64 heads): O^T[dv,head] += V^T P^T with
-//     v_mfma_f32_16x16x32, V^T fragments read from the SAME LDS rows through ds_read_b64_tr_b16, every
-//     fragment feeding all four 16-head blocks.  That shape of the instruction takes the same matrix-pipe cycles and a sixth
-//     less power a product than 32x32x16, twice the instructions: these waves have the issue slots, and the launch is at the
-//     socket's power cap.  With 32x32x16: B128 H128 Skv4096 bf16 171.4 -> 166.8 us, fp16 184.3 -> 177.5, B64 Skv2000
-//     58.6 -> 57.6, B24 Skv4000 47.0 -> 46.2, B16 H64 Skv8000 42.7 either way.  The score waves, whose instruction
-//     stream is the trip, keep 32x32x16.
+//     v_mfma_f32_16x16x32, paged 32x32x16 (AE_VB), V^T fragments read from the SAME LDS rows through ds_read_b64_tr_b16,
+//     every fragment feeding all blocks of heads.
 // Wave i runs on SIMD i % 4.  The workgroup is launched with 8 waves: waves 0, 1 are the score waves
 // (SIMD 0, 1: 1152 matrix-pipe cycles per tile each), waves 2, 3, 6, 7 the value waves (two each on SIMD
 // 2, 3: 2 x 512 cycles), waves 4, 5 leave at once (AE_HPW 16, paged cache: they request the tiles, AE_LOADER_WAVES) - so the four SIMDs carry about the same MFMA work.
@@ -61,8 +57,15 @@
 #define AE_HPW 64
 #endif
 #define AE_HEADS_PER_WG AE_HPW
-#define AE_NHB (AE_HPW / 16)              // a value wave's head blocks
 #define AE_NSB (AE_HPW == 64 ? 2 : AE_HPW / 16)      // head blocks of the score waves: of 32 heads, or of 16
+// Heads of a value wave's block, and columns of its V^T fragments: 16 (v_mfma_f32_16x16x32) or 32 (32x32x16).  16x16x32 takes the
+// same matrix-pipe cycles and a sixth less power a product, twice the instructions.  The dense launch of 64 heads a workgroup is at the
+// socket's power cap and its value waves have the issue slots: 32 -> 16, us, B128 H128 Skv4096 bf16 171.4 -> 166.8, fp16 184.3 ->
+// 177.5, B64 Skv2000 fp16 58.6 -> 57.6, split B24 Skv4000 bf16 45.8 -> 45.0, B16 H64 Skv8000 42.7 either way.  A paged batch whose
+// entries have different lengths leaves CUs idle and the clock up, and there the instructions count: B23 H128 up to 6848 tokens
+// 52.4 -> 53.6, B56 5056 80.6 -> 82.1, B44 H64 2944 33.7 -> 34.4.  (The score waves' instruction stream is the trip: 32x32x16.)
+#define AE_VB (AE_HPW == 64 && AE_PAGED ? 32 : 16)
+#define AE_NHB (AE_HPW / AE_VB)           // head blocks of a value wave
 #define AE_BN 32                          // kv rows per tile
 #if AE_HPW == 64
 #define AE_NKS (AE_D / 16)                // 16-deep k-steps of S^T = K Q^T
@@ -79,8 +82,8 @@
 #define AE_LOADER_WAVES (AE_HPW == 16 && AE_PAGED)
 #define AE_NLOADERS (AE_LOADER_WAVES ? 2 : 4)      // else the value waves also request the KV tiles
 #define AE_DVW (AE_DV / 4)                // value columns of one value wave
-#define AE_NDB (AE_DVW / 16)              // 16-wide dv blocks of a value wave
-#define AE_NO (AE_NDB * 4)                // output elements per lane and head block
+#define AE_NDB (AE_DVW / AE_VB)           // dv blocks of a value wave
+#define AE_NO (AE_DVW * AE_VB / 64)       // output elements per lane and head block
 #define AE_KSTR (AE_D * 2)                // LDS row pitch, bytes (unpadded: swizzled)
 #define AE_STAGE_BYTES (AE_BN * AE_KSTR)
 #define AE_CPR (AE_D / 8)                 // 16-byte chunks per K row
@@ -562,7 +565,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
       }
       mx = AE_NEG_INF;
       rs = 0.f;
-      prow = pbuf + (tp & 1) * AE_P_BYTES + (wave * 32 + l32s) * AE_PSTR + 16 * hfs;
+      prow = pbuf + (tp & 1) * AE_P_BYTES + (wave * 32 + l32s) * AE_PSTR + (AE_VB == 32 ? 8 : 16) * hfs;
       xb = xbuf + (tp & 1) * AE_X_BYTES;
     };
     // the softmax of one tile in AE_NKS pieces, piece f issued behind the MFMA of k-step f
@@ -588,8 +591,8 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
         ae_elem4 w;
 #pragma unroll
         for (int i = 0; i < 4; i++) w[i] = (ae_elem)xs[4 * rb + i];
-        // P^T [head][slot]: a value wave's lane takes slots 8*g .. + 7, keys 4*g .. + 3 of the tile's first half and of its second
-        *(__attribute__((address_space(3))) ae_elem4*)(prow + 32 * (rb & 1) + 8 * (rb >> 1)) = w;
+        // (P^T [head][key]; 16-wide blocks [head][slot]: a value wave's lane takes slots 8*g .. + 7, keys 4*g .. + 3 of either half)
+        *(__attribute__((address_space(3))) ae_elem4*)(prow + (AE_VB == 32 ? 16 * rb : 32 * (rb & 1) + 8 * (rb >> 1))) = w;
       } else if (f == 26) {
         r_run = r_run * osc + rs;
         if (hfs == 0) ((ae_lds_f32*)xb)[wave * 32 + l32s] = osc;
@@ -791,11 +794,21 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #endif
 
   // ============================== value wave: AE_DVW value columns, AE_HPW heads =======================
-  const int lhd = lane & 15;       // the lane's head in a block of 16
-  const int hf = lane >> 4;        // ... and which part of the block's rows
+#if AE_VB == 32
+  const int lhd = lane & 31;       // the lane's head in a block of heads
+  const int hf = lane >> 5;        // ... and which part of the block's rows
+#else
+  const int lhd = lane & 15;
+  const int hf = lane >> 4;
+#endif
   const int dvw = wave < 4 ? wave - 2 : wave - 4;   // waves 2, 3, 6, 7
-  constexpr int NR = 4;
-  ae_f32x4 oacc[AE_NHB][AE_NDB];     // [head block][dv block]: O^T
+#if AE_VB == 32
+  typedef ae_f32x16 ae_acc;
+#else
+  typedef ae_f32x4 ae_acc;
+#endif
+  constexpr int NR = sizeof(ae_acc) / 4;
+  ae_acc oacc[AE_NHB][AE_NDB];     // [head block][dv block]: O^T
 #pragma unroll
   for (int hb = 0; hb < AE_NHB; hb++)
 #pragma unroll
@@ -807,6 +820,33 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   const unsigned long long ae_w1 = __builtin_amdgcn_s_memrealtime();     // tile 0 (and Q) have landed
 #endif
 
+#if AE_VB == 32
+  // V^T fragment (k-step kk, dv block db): A[m = dv][k = kv]: lane i of a 16-lane group supplies the
+  // address of row 16*kk + 8*hf + i/4 (+4 for slots 4..7), 8 bytes at value column
+  // 32*db + 16*((lane%32)/16) + 4*(i%4), and receives column i of those four rows.  The swizzle of a
+  // row's chunks touches the three low bits of the chunk number only, so a lane has four distinct
+  // offsets (parity of db, first / second group of four rows) and everything else is an immediate.
+  const int v_row = 8 * hf + ((lane & 15) >> 2);
+  const int v_c0 = 2 * (lhd >> 4) + ((lane & 3) >> 1);
+  const int v_half = (lane & 1) * 8;
+  int v_base[2][2];     // [db & 1][row group]
+#pragma unroll
+  for (int par = 0; par < 2; par++)
+#pragma unroll
+    for (int rg = 0; rg < 2; rg++) {
+      const int r = v_row + 4 * rg;
+      v_base[par][rg] = r * AE_KSTR + ((((4 * par + v_c0) ^ AE_SWZ(r)) + 4 * AE_NDB * dvw) << 4) + v_half;
+    }
+  auto read_vfrag = [&](const int (&va)[2][2], int kk, int db) AE_LAMBDA -> ae_elem8 {
+    const int imm = 16 * kk * AE_KSTR + (db >> 1) * 128;
+    ae_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)(
+        lds + va[db & 1][0] + imm));
+    ae_s16x4 hi2 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)(
+        lds + va[db & 1][1] + imm));
+    return __builtin_bit_cast(ae_elem8, __builtin_shufflevector(lo, hi2, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+
+#else
   // V^T fragment of dv block db (16 columns, all 32 keys): A[m = dv][k]: k = 8*(lane/16) + j is key 4*(lane/16) + j of the
   // tile's first half (j < 4) or second half (the order in which the score waves leave P): the 16 rows of one transposed
   // read then lie in 16 different places of the swizzle, where rows 0-3 and 8-11 would share theirs.
@@ -815,7 +855,7 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #pragma unroll
   for (int i = 0; i < 4; i++)
     v_base[i] = v_row * AE_KSTR + ((((2 * i + ((lane & 3) >> 1)) ^ AE_SWZ(v_row)) + (AE_DVW / 8) * dvw) << 4) + (lane & 1) * 8;
-  auto read_vfrag = [&](const int (&va)[4], int db) AE_LAMBDA -> ae_elem8 {
+  auto read_vfrag = [&](const int (&va)[4], int, int db) AE_LAMBDA -> ae_elem8 {
     const int imm = (db >> 2) * 128;
     ae_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)(
         lds + va[db & 3] + imm));
@@ -823,21 +863,29 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
         lds + va[db & 3] + imm + 16 * AE_KSTR));
     return __builtin_bit_cast(ae_elem8, __builtin_shufflevector(lo, hi2, 0, 1, 2, 3, 4, 5, 6, 7));
   };
+#endif
 
   // A trip of a value wave: O^T += V^T P^T for tile n - 2 with the V^T fragments it holds in registers (PV),
   // and the fragments of tile n - 1 read from LDS into those registers as they fall free (RD) - the read
   // has a whole trip to complete, and tile n - 1's stage can take the next request when the trip ends.
-  ae_elem8 vreg[AE_NDB];           // fragment of dv block f
+  constexpr int NKK = AE_VB == 32 ? 2 : 1;      // k-steps over the tile's keys
+  ae_elem8 vreg[NKK * AE_NDB];     // fragment f = (k-step f / AE_NDB, dv block f % AE_NDB)
 #pragma unroll
-  for (int f = 0; f < AE_NDB; f++) vreg[f] = (ae_elem8){};
+  for (int f = 0; f < NKK * AE_NDB; f++) vreg[f] = (ae_elem8){};
   auto value_trip = [&](int n, auto with_pv, auto with_rd) AE_LAMBDA {
     constexpr bool PV = decltype(with_pv)::value;
     constexpr bool RD = decltype(with_rd)::value;
     // the lane's four fragment offsets inside tile n - 1's stage
+#if AE_VB == 32
+    int va[2][2];
+#pragma unroll
+    for (int i = 0; i < 4; i++) va[i >> 1][i & 1] = v_base[i >> 1][i & 1] + ((n - 1) % AE_NSTAGE) * AE_STAGE_BYTES;
+#else
     int va[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) va[i] = v_base[i] + ((n - 1) % AE_NSTAGE) * AE_STAGE_BYTES;
-    ae_elem8 pf[AE_NHB];
+#endif
+    ae_elem8 pf[AE_NHB][NKK];
     if (PV) {
       const int t = n - 2;
       const ae_lds_byte* pb = pbuf + (t & 1) * AE_P_BYTES;
@@ -847,26 +895,34 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
       if (__builtin_amdgcn_readfirstlane(flags[0] | flags[AE_NSB - 1]) != 0) {
 #pragma unroll
         for (int hb = 0; hb < AE_NHB; hb++) {
-          const float osc = ((const ae_lds_f32*)xb)[hb * 16 + lhd];
+          const float osc = ((const ae_lds_f32*)xb)[hb * AE_VB + lhd];
 #pragma unroll
           for (int db = 0; db < AE_NDB; db++)
 #pragma unroll
             for (int r = 0; r < NR; r++) oacc[hb][db][r] *= osc;
         }
       }
-      // P^T fragments: B[k = slot = 8*hf + j][n = head = 16*hb + lhd]
+      // P^T fragments: B[k = kv = 16*kk + 8*hf + j][n = head = 32*hb + lhd] (16 heads a block: all 32 kv, k = 8*hf + j)
 #pragma unroll
       for (int hb = 0; hb < AE_NHB; hb++)
-        pf[hb] = *(const __attribute__((address_space(3))) ae_elem8*)(pb + (hb * 16 + lhd) * AE_PSTR + 16 * hf);
+#pragma unroll
+        for (int kk = 0; kk < NKK; kk++)
+          pf[hb][kk] = *(const __attribute__((address_space(3))) ae_elem8*)(
+              pb + (hb * AE_VB + lhd) * AE_PSTR + 32 * kk + 16 * hf);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int f = 0; f < AE_NDB; f++) {
+    for (int f = 0; f < NKK * AE_NDB; f++) {
       if (PV) {
 #pragma unroll
-        for (int hb = 0; hb < AE_NHB; hb++) oacc[hb][f] = ae_mfma16(vreg[f], pf[hb], oacc[hb][f]);
+        for (int hb = 0; hb < AE_NHB; hb++)
+#if AE_VB == 32
+          oacc[hb][f % AE_NDB] = ae_mfma32(vreg[f], pf[hb][f / AE_NDB], oacc[hb][f % AE_NDB]);
+#else
+          oacc[hb][f] = ae_mfma16(vreg[f], pf[hb][0], oacc[hb][f]);
+#endif
       }
-      if (RD) vreg[f] = read_vfrag(va, f);
+      if (RD) vreg[f] = read_vfrag(va, f / AE_NDB, f % AE_NDB);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -891,11 +947,12 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   ae_lds_byte* obuf = lds + dvw * (AE_HEADS_PER_WG * AE_DVW * 4);
   const int heads_left = group - ht * AE_HEADS_PER_WG;          // heads of the tile that exist
   const int heads_here = heads_left < AE_HEADS_PER_WG ? heads_left : AE_HEADS_PER_WG;
-  // ---- per-split epilogue: lane owns head 16*hb + lhd, columns AE_DVW*dvw + 16*db + 4*hf + r
+  // ---- per-split epilogue: lane owns head 32*hb + lhd, value columns AE_DVW*dvw + 32*db + 8*(r/4) + 4*hf + r%4
+  //      (16 heads a block: head 16*hb + lhd, columns AE_DVW*dvw + 16*db + 4*hf + r)
 #pragma unroll
   for (int hb = 0; hb < AE_NHB; hb++) {
-    if (hb * 16 >= heads_here) break;                        // (wave uniform)
-    const int hl = hb * 16 + lhd;
+    if (hb * AE_VB >= heads_here) break;                        // (wave uniform)
+    const int hl = hb * AE_VB + lhd;
     const int head_in_group = ht * AE_HEADS_PER_WG + hl;
     const bool head_ok = head_in_group < group;
     const int hq = hk * group + (head_ok ? head_in_group : 0);
@@ -944,7 +1001,11 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     // (piece e of a lane, four columns: fp32 chunk at4, in the output type half at4 % 2 of chunk at4 / 2)
 #pragma unroll
     for (int e = 0; e < AE_NO / 4; e++) {
+#if AE_VB == 32
+      const int at4 = e * 2 + hf;                   // (dv block e / 4)
+#else
       const int at4 = e * 4 + hf;
+#endif
       if (direct) {
         ae_elem4 w;
 #pragma unroll
@@ -958,20 +1019,20 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the wave's own region: its LDS writes have been made)
     // (the heads of a block leave while the next block's results are scaled and written)
     if (direct) {
-      constexpr int CPH = AE_DVW / 8, N = 16 * CPH / 64;      // 16-byte chunks of a head's piece, instructions of the block
+      constexpr int CPH = AE_DVW / 8, N = AE_VB * CPH / 64;      // 16-byte chunks of a head's piece, instructions of the block
       ae_elem* ob = (ae_elem*)p.out + (int64_t)b * p.o_stride_b + (int64_t)(hk * group + ht * AE_HEADS_PER_WG) * p.o_stride_h + dvw * AE_DVW;
 #pragma unroll 4
-      for (int i = 0; i < N && i * 64 < (heads_here - hb * 16) * CPH; i++) {
-        const int hs = hb * 16 + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
+      for (int i = 0; i < N && i * 64 < (heads_here - hb * AE_VB) * CPH; i++) {
+        const int hs = hb * AE_VB + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
         const ae_elem8 w = *(const __attribute__((address_space(3))) ae_elem8*)(obuf + hs * (AE_DVW * 2) + ((c ^ (hs & AE_OSW)) << 4));
         if (hs < heads_here) *(ae_elem8*)(ob + (int64_t)hs * p.o_stride_h + c * 8) = w;
       }
     } else {
-      constexpr int CPH = AE_DVW / 4, N = 16 * CPH / 64;
+      constexpr int CPH = AE_DVW / 4, N = AE_VB * CPH / 64;
       float* ob = p.partial_o + (((int64_t)b * p.heads_q + hk * group + ht * AE_HEADS_PER_WG) * n_split + split) * AE_DV + dvw * AE_DVW;
 #pragma unroll 8
-      for (int i = 0; i < N && i * 64 < (heads_here - hb * 16) * CPH; i++) {
-        const int hs = hb * 16 + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
+      for (int i = 0; i < N && i * 64 < (heads_here - hb * AE_VB) * CPH; i++) {
+        const int hs = hb * AE_VB + (i * 64 + lane) / CPH, c = (i * 64 + lane) % CPH;
         const ae_f32x4 w = *(const __attribute__((address_space(3))) ae_f32x4*)(obuf + hs * (AE_DVW * 4) + ((c ^ (hs & AE_OSW)) << 4));
         if (hs < heads_here) __builtin_nontemporal_store(w, (ae_f32x4*)(ob + (int64_t)hs * n_split * AE_DV + c * 4));
       }
