@@ -723,9 +723,9 @@ int ae_prefill_bwd(ae_kernel* delta, ae_kernel* dkv, ae_kernel* dq, const ae_att
   } else if (p->block_mask) {
     return fail(AE_ERR_INVALID_ARG, "ae_prefill_bwd: a block mask was passed to kernels built without tile-class tables");
   }
-  const uint64_t rows = (uint64_t)p->batch * p->seqlen_q * p->heads_q;
-  const uint64_t rows_per_wg = 256u / (uint32_t)(cfg->head_dim_v / 8);
-  const uint64_t g_delta = (rows + rows_per_wg - 1) / rows_per_wg;
+  // (32 positions of the heads that 64 lanes of 16 bytes span: AE_DELTA_S and AE_DELTA_H of ae_bwd_delta.h)
+  const uint64_t delta_heads = cfg->head_dim_v < 512 ? 64u / (uint32_t)(cfg->head_dim_v / 8) : 1u;
+  const uint64_t g_delta = (((uint64_t)p->seqlen_q + 31) / 32) * (((uint64_t)p->heads_q + delta_heads - 1) / delta_heads) * (uint64_t)p->batch;
   // ids are 8*slot + xcd, slot = tile*ceil(batch*heads/8) + head group (see ae_prefill_bwd.hip)
   uint64_t g_dkv = (((uint64_t)p->seqlen_kv + 127) / 128) * ((((uint64_t)p->batch * p->heads_kv) + 7) / 8) * 8;
   if (cfg->merge_in_wg == 2) {         // kernels that share a kv tile out over several workgroups

@@ -402,6 +402,12 @@ def test_traced_backward_with_two_final_row_scales(cuda_device, B, H, Hkv, S, D,
     _check(vd.grad, dv, "dv", case)
 
 
+@pytest.mark.parametrize("B,H,Hkv,S,D", [(2, 9, 3, 33, 64), (1, 17, 17, 31, 64), (3, 8, 8, 64, 64), (2, 5, 5, 65, 128), (1, 1, 1, 1, 64)])
+def test_row_sums_at_the_edges_of_their_workgroups(cuda_device, B, H, Hkv, S, D):
+    """ae_bwd_delta_kernel: 32 positions of 8 heads (D 64) or 4 a workgroup, heads and positions past the end among them."""
+    test_traced_backward_with_two_final_row_scales(cuda_device, B, H, Hkv, S, D, torch.float16, True)
+
+
 def test_backward_of_other_graphs_is_refused(cuda_device):
     """An online function that keeps row scales of its own but defines no forward() / backward() rules
     (here: the running sum of |s| without them) has no backward.  Its forward still runs on tensors that
