@@ -97,15 +97,16 @@
 #define AE_NKS2 (AE_DV / 16)       // k-steps of dP
 #define AE_NDB1 (AE_D / 32)        // 32-wide output blocks of dQ / dK
 #define AE_NDB2 (AE_DV / 32)       // ... of dV
-#define AE_L1 ((AE_BS * AE_CPR1) / AE_NT)   // 1 KiB load instructions per wave and tile
-#define AE_L2 ((AE_BS * AE_CPR2) / AE_NT)
+#define AE_RQW (AE_BWD_PAIRS ? AE_NWAVES / 2 : AE_NWAVES)       // waves that request the tiles (pairs: those of the second kind)
+#define AE_L1 ((AE_BS * AE_CPR1) / (AE_RQW * 64))   // 1 KiB load instructions per such wave and tile
+#define AE_L2 ((AE_BS * AE_CPR2) / (AE_RQW * 64))
 #ifndef AE_NSTAGE
 #define AE_NSTAGE 3                // LDS stages: a tile is requested AE_NSTAGE - 1 iterations before it is multiplied
 #endif
 #ifndef AE_BWD_WAVES_PER_EU
 #define AE_BWD_WAVES_PER_EU 1
 #endif
-#define AE_RSL ((AE_RS_PLANES + AE_NWAVES - 1) / AE_NWAVES)      // row-value loads per wave and tile (dk / dv launch)
+#define AE_RSL ((AE_RS_PLANES + AE_RQW - 1) / AE_RQW)      // row-value loads per wave and tile (dk / dv launch)
 #define AE_NLOADS (AE_L1 + AE_L2 + (AE_BWD_ROLE == 1 ? AE_RSL : 0))   // load instructions per wave and tile
 #define AE_VMCNT(n) (0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
 #ifndef AE_AHEAD
@@ -228,6 +229,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rw = AE_BWD_PAIRS ? wave % AE_NRW : wave;      // the wave's 32 resident rows
+  const int rqw = AE_BWD_PAIRS ? wave % AE_RQW : wave;     // ... and its share of the requests
   const int l32 = lane & 31;
   const int hf = lane >> 5;
   const int group = p.heads_q / p.heads_kv;
@@ -405,13 +407,13 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   // ae_load_lds16_burst_base: bases are passed 4 KiB low and offsets 4 KiB high).  Rows past the end of
   // the sequence re-read its last row (they are masked).
   auto lane_off1 = [&](int i, int64_t st) AE_LAMBDA -> unsigned {
-    const int sidx = (wave * AE_L1 + i) * 64 + lane;
+    const int sidx = (rqw * AE_L1 + i) * 64 + lane;
     const int r = sidx / AE_CPR1;
     const int c = ae_bwd_chunk_pos<AE_CPR1>(r, sidx % AE_CPR1);
     return (unsigned)((r * (int)st + c * 8) * 2 + 4096 - (i - AE_L1 / 2) * 1024);
   };
   auto lane_off2 = [&](int i, int64_t st) AE_LAMBDA -> unsigned {
-    const int sidx = (wave * AE_L2 + i) * 64 + lane;
+    const int sidx = (rqw * AE_L2 + i) * 64 + lane;
     const int r = sidx / AE_CPR2;
     const int c = ae_bwd_chunk_pos<AE_CPR2>(r, sidx % AE_CPR2);
     return (unsigned)((r * (int)st + c * 8) * 2 + 4096 - (i - AE_L2 / 2) * 1024);
@@ -445,7 +447,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   const float* rq_d[AE_RSL];
 #pragma unroll
   for (int i = 0; i < AE_RSL; i++) {
-    const int plane = (wave + AE_NWAVES * i) % AE_RS_PLANES;
+    const int plane = (rqw + AE_RQW * i) % AE_RS_PLANES;
     rq_d[i] = p.delta + ((int64_t)plane * p.batch * p.heads_q + (int64_t)b * p.heads_q + str_h) * p.seqlen_q;
   }
 #endif
@@ -489,14 +491,14 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
       const int last = n_str - 1 - s0;
 #pragma unroll
       for (int i = 0; i < 8; i++) {
-        const int over1 = ((wave * AE_L1 + (i < AE_L1 ? i : 0)) * 64 + le) / AE_CPR1 - last;
-        const int over2 = ((wave * AE_L2 + (i < AE_L2 ? i : 0)) * 64 + le) / AE_CPR2 - last;
+        const int over1 = ((rqw * AE_L1 + (i < AE_L1 ? i : 0)) * 64 + le) / AE_CPR1 - last;
+        const int over2 = ((rqw * AE_L2 + (i < AE_L2 ? i : 0)) * 64 + le) / AE_CPR2 - last;
         g1[i] -= (unsigned)((over1 > 0 ? over1 : 0) * (int)st1 * 2);
         g2[i] -= (unsigned)((over2 > 0 ? over2 : 0) * (int)st2 * 2);
       }
     }
-    ae_load_lds16_burst_base<AE_L1>(x1 - 4096, g1, t1 + (wave * AE_L1 + AE_L1 / 2) * 1024);
-    ae_load_lds16_burst_base<AE_L2>(x2 - 4096, g2, t2 + (wave * AE_L2 + AE_L2 / 2) * 1024);
+    ae_load_lds16_burst_base<AE_L1>(x1 - 4096, g1, t1 + (rqw * AE_L1 + AE_L1 / 2) * 1024);
+    ae_load_lds16_burst_base<AE_L2>(x2 - 4096, g2, t2 + (rqw * AE_L2 + AE_L2 / 2) * 1024);
 #if AE_BWD_ROLE == 1
     {
       // rowsum(do * o) and lse in log2 units (kind 2: the final row scales) of the tile's 64 q rows: the waves share
@@ -506,7 +508,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
       row = row < n_str ? row : n_str - 1;
 #pragma unroll
       for (int i = 0; i < AE_RSL; i++) {
-        const int plane = (wave + AE_NWAVES * i) % AE_RS_PLANES;
+        const int plane = (rqw + AE_RQW * i) % AE_RS_PLANES;
 #if AE_MASK_MODE != 2
         const float* src = rq_d[i] + row;
 #else
@@ -591,7 +593,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   int cls0, cls1, cls2;                 // ... and the classes of those three items
   int x0 = next_item(x_first, cls0), x1 = next_item(x0 + 1, cls1), x2 = next_item(x1 + 1, cls2);
 #if AE_RES_VIA_LDS
-  if (x0 < n_items) request_item(x0, 0);
+  if (x0 < n_items && (!AE_BWD_PAIRS || wave >= AE_NRW)) request_item(x0, 0);
   if (AE_BWD_PAIRS && wave >= AE_NRW) {
     __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
   } else {
@@ -895,13 +897,17 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   // and a wave of the second kind reads one of the two tensors.  p and ds go over through 32 KiB of LDS, in the operand layout.
   // A tile's two barriers: A, the second kind has p and ds of n - 1 in registers (the first may write those of n); B, at the
   // end, tile n + 1 has landed and p and ds of n are written.  Tile n + 1 goes into the stage of tile n - 2, which the second kind
-  // left at the last B.
+  // left at the last B, and is requested by the second kind alone: the first kind's stream (3900 of 4100 cycles a tile: 1200 scores,
+  // 550 weights, 1130 hand-over, ds and the other weights, 250 from B to the first score, barriers) is the longer one, and with all
+  // eight waves asking for the tile behind B each of them was held there for 850 to 950 cycles.  A lies behind a third of the
+  // second kind's products, where the first kind comes to it.  dk/dv launch, us, before and after: bf16 B4 H32 S2048 366 -> 351,
+  // fp16 B2 H32 S4096 617 -> 577, bf16 B8 H32 S875 197 -> 186, B2 Hq32 Hkv8 S2500 244 -> 235, fp16 B2 H16 S1000 36.0 -> 33.8.  With A
+  // or the requests elsewhere 1 to 6 % of that again; ds stored by dk's waves 394 where this took 364; kv tiles that follow each
+  // other in one workgroup without a gap 380 for 371 (K and V straight into registers: 5.7 us a tile, as long as the edges).
   // LDS bound this: a wave of the first kind held 32 rows and took all 64 q rows, one of the second 32 rows of dk and of dv, and each
   // fragment fed one MFMA, 320 KB of fragments, row values and hand-over a tile at 128 bytes a clock, now 224.  dk/dv launch,
   // us: causal fp16 B2 H32 S4096 644 -> 598, B2 Hq32 Hkv8 S2500 251 -> 233, bf16 B4 H32 S2048 356 -> 335, B2 H32 S1000 53.2 -> 51.5.
-  // Bits are the same.  What is left of B4 H32 S2048: without the stores of ds 308, with every tile in the L2 297, without the
-  // exponentials too 286, on inputs of zeros 277 (the power cap).  Priorities of either kind, and barrier A a quarter earlier
-  // or later: within 1 %.
+  // Bits are the same.  The launch runs at the socket's power cap: 1.56 GHz, on inputs of zeros 2.1 (B4 H32 S2048 273 us).
   static_assert(AE_D == AE_DV && AE_NKS1 == AE_NKS2 && AE_RES_ONEPASS, "pairs: one head dim");
   ae_lds_byte* const ho = lds + 3 * AE_STAGE_BYTES + lane * 16;      // fragment i (p: 0..3, ds: 4..7) of 32 rows kb at + 8192 * kb + 1024 * i
   typedef __attribute__((address_space(3))) ae_u32x4 ae_lds_u32x4;
@@ -925,7 +931,6 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
     const int r0w = r0 + half * 64;
     while (x0 < n_items) {
-      request_item(x1, st_req);
       const tile_at at = tile_in_use(st_use);
       const int qb = at.s0 + 32 * nb;                // the first of the wave's 32 q rows
       bool need_vis = qb + 32 > n_str || r0w + 64 > n_res;
@@ -1000,11 +1005,6 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
         }
       }
-#if AE_BWD_KEEP_DS
-      __builtin_amdgcn_s_waitcnt(AE_VMCNT(4));                 // (the tile: this trip's four stores of ds are newer)
-#else
-      __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
-#endif
       __syncthreads();                                         // B
 #if AE_BWD_KEEP_DS
       ds_at += (ds_triangle ? 2 * (us_t / 2 + 1) : ds_pairs) * 8192;
@@ -1017,7 +1017,6 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
 #endif
       }
       st_use = st_use == 2 * AE_STAGE_BYTES ? 0 : st_use + AE_STAGE_BYTES;
-      st_req = st_req == 2 * AE_STAGE_BYTES ? 0 : st_req + AE_STAGE_BYTES;
       x0 = x1;
       x1 = next_item(x1 + 1, cls1);
     }
@@ -1028,41 +1027,48 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   // (acc1, acc2: the two blocks of 32 rows, of dk where nb is 0, else of dv)
   clear(acc1);
   clear(acc2);
-  // the tile's products with what was handed over: fragment f = (k-step f / 4, output block f % 4)
-  auto add_handed_over = [&](unsigned stage, auto all_read) AE_LAMBDA {
+  // The tile's products with what was handed over: fragment f = (k-step f / 4, output block f % 4).  All of what was handed over
+  // is read first; all_read() comes behind a third of the products.
+  auto add_handed_over = [&](unsigned stage, auto request, auto all_read) AE_LAMBDA {
     unsigned w = tr1 + stage + (unsigned)(nb * AE_T1_BYTES);
     asm("" : "+v"(w));
     ae_u32x4 b0[4], b1[4];
-    auto take = [&](int kk) AE_LAMBDA {
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) {
       b0[kk] = *(const ae_lds_u32x4*)(ho + 2 * half * 8192 + (4 - 4 * nb + kk) * 1024);
       b1[kk] = *(const ae_lds_u32x4*)(ho + (2 * half + 1) * 8192 + (4 - 4 * nb + kk) * 1024);
-    };
+    }
     constexpr int NF = 4 * AE_NDB1;
     auto frag = [&](int f) AE_LAMBDA -> ae_elem8 { return tr_frag(w, AE_STR1, AE_CPR1, f / AE_NDB1, f % AE_NDB1, 0); };
     ae_elem8 ring[AE_RING];
-    take(0);
+    __builtin_amdgcn_sched_barrier(0);
+    request();
 #pragma unroll
     for (int f = 0; f < AE_AHEAD; f++) ring[f] = frag(f);
-    take(1);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int f = 0; f < NF; f++) {
       if (f + AE_AHEAD < NF) ring[(f + AE_AHEAD) % AE_RING] = frag(f + AE_AHEAD);
-      if (f == AE_NDB1) take(2);
-      if (f == AE_NDB1 + 1) take(3);
-      if (f == NF / 2) all_read();
       const int kk = f / AE_NDB1, j = f % AE_NDB1;
       acc1[j] = ae_mfma32(ring[f % AE_RING], __builtin_bit_cast(ae_elem8, b0[kk]), acc1[j]);
       acc2[j] = ae_mfma32(ring[f % AE_RING], __builtin_bit_cast(ae_elem8, b1[kk]), acc2[j]);
       __builtin_amdgcn_sched_barrier(0);
+      if (f == NF / 3) {
+        all_read();
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   };
   unsigned st_prev = 2 * AE_STAGE_BYTES;
   bool first = true;
   while (x0 < n_items) {
-    request_item(x1, st_req);
-    if (first) __syncthreads();                                // A (nothing is handed over yet)
-    else add_handed_over(st_prev, [&]() AE_LAMBDA { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __syncthreads(); });
+    if (first) {
+      request_item(x1, st_req);
+      __syncthreads();                                         // A (nothing is handed over yet)
+    } else {
+      add_handed_over(st_prev, [&]() AE_LAMBDA { request_item(x1, st_req); },
+                      [&]() AE_LAMBDA { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __syncthreads(); });      // A
+    }
     first = false;
     __builtin_amdgcn_s_waitcnt(AE_VMCNT(0));
     __syncthreads();                                           // B
@@ -1071,7 +1077,7 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
     x0 = x1;
     x1 = next_item(x1 + 1, cls1);
   }
-  if (!first) add_handed_over(st_prev, []() AE_LAMBDA {});
+  if (!first) add_handed_over(st_prev, []() AE_LAMBDA {}, []() AE_LAMBDA {});
   (void)st_use;
 #else
   unsigned st_use = 0, st_req = (AE_NSTAGE - 1) * AE_STAGE_BYTES;      // stages of this iteration: multiplied, filled
