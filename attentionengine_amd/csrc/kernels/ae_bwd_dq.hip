@@ -11,11 +11,12 @@
 // 64 slots of q rows a q tile (a wave uses 32 of the slots; where slot n lies among the rows is undone when the rows leave).
 // Three stages of 24 KiB, filled by direct loads two steps ahead.
 //
-// B4 H32 S2048 D128 bf16 causal (570 MB of ds): 145 us where the launch that forms ds takes 219.  Loads of ds alone 135 us at
-// first - while 256 MB of them still sat dirty in the memory-side cache and had to leave it -, 164 with K and the products; two
-// workgroups a CU instead of one 160, from the last keys to the first 152, past the caches 145.  Launched for one batch
-// entry at a time, so that all of ds stays in that cache, the longest workgroup of each launch costs more than it saves (the
-// backward 573 us against 538).
+// B4 H32 S2048 D128 bf16 causal (570 MB of ds, 812 MB moved): 141 us, 5.8 TB/s, where the launch that forms ds takes 219.  One workgroup
+// a CU 160 at first, two 152 with the steps from the last keys to the first, past the caches 145 (loads that stay in them: 150 for 141).
+// Loads whose neighbouring lanes read neighbouring bytes, us, before and after: that call 149 -> 141, fp16 B2 H32 S4096 247 -> 235, bf16 B8
+// H32 S875 84.7 -> 77.3, B5 Hq32 Hkv8 S2676 289 -> 259.  With all of ds in the L2 it would be 90.  Heads four or eight at a time, so that
+// their K stays in the L2: 150, 148 for 141; for one batch entry at a time, so that ds stays in the memory-side cache, the longest
+// workgroup of each launch costs more than it saves (the backward 573 us against 538).
 //
 // Configuration ("ae_config.h"): AE_D (128) AE_DTYPE_BF16 AE_MASK_MODE (0, 1) AE_SM_SCALE, and for the delta kernel AE_DV AE_BWD_KIND (0).
 
@@ -48,11 +49,8 @@ static_assert(AE_MASK_MODE == 0 || AE_MASK_MODE == 1, "none or causal");
 
 typedef __attribute__((address_space(3))) unsigned char ae_lds_byte;
 
-// LDS position of 16-byte chunk c of row r (CPR chunks a row), as in ae_prefill_bwd.hip: an involution in c
-template <int CPR>
-AE_DEV int ae_chunk_pos(int r, int c) {
-  return ((((c >> 1) ^ (r & (CPR / 2 - 1))) << 1) | ((c ^ (r >> (CPR == 16 ? 3 : 2))) & 1));
-}
+// LDS position of 16-byte chunk c of row r of K, as in ae_prefill_bwd.hip: an involution in c
+AE_DEV int ae_chunk_pos(int r, int c) { return ((((c >> 1) ^ (r & 7)) << 1) | ((c ^ (r >> 3)) & 1)); }
 
 extern "C" __global__ __launch_bounds__(AE_NWAVES * 64) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void ae_bwd_dq_kernel(const ae_attn_bwd_params p) {
@@ -86,11 +84,16 @@ void ae_bwd_dq_kernel(const ae_attn_bwd_params p) {
   n_mine = (r0w + 31) / AE_BS + 1 < n_items ? (r0w + 31) / AE_BS + 1 : n_items;
 #endif
 
-  // ---- requests: K rows wave * 4 .. + 3 of the step's 32, and half a block of ds: keys 16 * (wave % 2) .. of q tile wave / 2 ----
+  // ---- requests: K rows wave * 4 .. + 3 of the step's 32, and half a block of ds: 1 KiB pieces kk = 2 * (wave % 2) .. + 1 of q tile
+  // wave / 2.  A piece lands as it lies in memory but for its groups of four keys (64 bytes), which are exchanged inside 256 bytes: a
+  // transposed read takes four of them, of two pieces and of either half of a piece, that would share their banks.  (A load whose
+  // sixteen neighbouring lanes read 32 bytes each of eight lines - ds with its rows of 64 slots side by side in LDS - is
+  // held at issue: 520 to 1370 of 2800 cycles a step.)
+  auto group_at = [](int kk, int half, int g) AE_LAMBDA -> int { return half * 8 + (g & 4) + ((g + 2 * half + kk) & 3); };
   const int ks = (int)p.k_stride_s;
   auto k_off = [&](int i, int back) AE_LAMBDA -> unsigned {
     const int n = (wave * AE_KL + i) * 64 + lane;
-    const int r = n / 16, c = ae_chunk_pos<16>(r, n % 16);
+    const int r = n / 16, c = ae_chunk_pos(r, n % 16);
     const int over = r - back;                    // (rows past the end re-read the last one: their ds is zero)
     return (unsigned)(((r - (over > 0 ? over : 0)) * ks + c * 8) * 2 + 4096 - (i - AE_KL / 2) * 1024);
   };
@@ -98,9 +101,8 @@ void ae_bwd_dq_kernel(const ae_attn_bwd_params p) {
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     koff[i] = k_off(i < AE_KL ? i : 0, AE_BS);
-    const int n = (i < AE_DL ? i : 0) * 64 + lane;       // chunk of the block's rows, in LDS order
-    const int r = 16 * (wave & 1) + n / 8, c = ae_chunk_pos<8>(r, n % 8);
-    doff[i] = (unsigned)((c >> 1) * 1024 + ((c & 1) * 32 + r) * 16 + 4096 - ((i < AE_DL ? i : 0) - AE_DL / 2) * 1024);
+    const int kk = 2 * (wave & 1) + (i < AE_DL ? i : 0), u = lane >> 2, g = (u & 4) | ((u - 2 * (u >> 3) - kk) & 3);
+    doff[i] = (unsigned)(kk * 1024 + ((u >> 3) * 32 + g * 4 + (lane & 3)) * 16 + 4096 - ((i < AE_DL ? i : 0) - AE_DL / 2) * 1024);
   }
   // The steps run from the last keys to the first: the dk/dv launch goes through the key tiles from the first to the last, so
   // its last blocks are those that the memory-side cache still holds.
@@ -131,8 +133,10 @@ void ae_bwd_dq_kernel(const ae_attn_bwd_params p) {
   // transposed fragments, see tr_frag of ae_prefill_bwd.hip: rows 16*kk + 4*hf + 0..3 and + 8 of column 32*db + l32
   const int t_row = 4 * hf + ((lane & 15) >> 2), t_g = l32 >> 4;
   const unsigned k_lane = (unsigned)(t_row * AE_STR + ((t_g ^ (t_row & 7)) << 5) + (((lane & 3) * 8) ^ (((t_row >> 3) & 1) * 16)));
-  const unsigned d_lane = (unsigned)(AE_K_BYTES + (wave >> 1) * AE_DS_BYTES + t_row * 128 +
-                                     (((2 * (wave & 1) + t_g) ^ (t_row & 3)) << 5) + (((lane & 3) * 8) ^ (((t_row >> 2) & 1) * 16)));
+  // (key 4*g + i of slots 16*kk + 8*half ..: group g; 8 keys on the group's low bits change by 2)
+  const int d_kk = 2 * (wave & 1) + t_g, d_half = (lane & 3) >> 1;
+  const unsigned d_lane = (unsigned)(AE_K_BYTES + (wave >> 1) * AE_DS_BYTES + d_kk * 1024 + group_at(d_kk, d_half, hf) * 64 +
+                                     ((lane & 15) >> 2) * 16 + (lane & 1) * 8);
   auto pair_of = [](const ae_lds_byte* a_lo, const ae_lds_byte* a_hi) AE_LAMBDA -> ae_elem8 {
     ae_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)a_lo);
     ae_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ae_s16x4*)a_hi);
@@ -162,7 +166,7 @@ void ae_bwd_dq_kernel(const ae_attn_bwd_params p) {
       };
       ae_elem8 ds[AE_NKK], ring[AE_AHEAD + 1];
 #pragma unroll
-      for (int kk = 0; kk < AE_NKK; kk++) ds[kk] = pair_of((const ae_lds_byte*)da + kk * 16 * 128, (const ae_lds_byte*)da + (kk * 16 + 8) * 128);
+      for (int kk = 0; kk < AE_NKK; kk++) ds[kk] = pair_of((const ae_lds_byte*)da + kk * 256, (const ae_lds_byte*)(da ^ 128u) + kk * 256);
 #pragma unroll
       for (int f = 0; f < AE_AHEAD; f++) ring[f] = k_frag(f);
       __builtin_amdgcn_sched_barrier(0);
