@@ -767,10 +767,10 @@ class MLADecodeOp(_SplitTuning):
         wave-specialised kernel report the shader clock their workgroups ran at (``self.clock_stamps``)."""
         return n_split == 1 and os.environ.get("AE_CLOCK_STAMPS", "") == "1" and self._wave_specialised()
 
-    def _variant(self, n_split, paged=False, heads=64):
+    def _variant(self, n_split, paged=False, heads=64, by_length=False):
         """(module, cfg, config source) of the split kernel, one for every count of splits above 1.  ``heads``: query heads of a
-        workgroup (AE_HPW of the wave-specialised kernel)."""
-        key = (n_split > 1, paged, heads, self._stamped(n_split))
+        workgroup (AE_HPW of the wave-specialised kernel); ``by_length``: the entries of a paged cache are split by their lengths."""
+        key = (n_split > 1, paged, heads, by_length, self._stamped(n_split))
         v = self._variants.get(key)
         if v is None:
             ws = self._wave_specialised()
@@ -778,6 +778,8 @@ class MLADecodeOp(_SplitTuning):
             cfg_src = render_mla_config(self.DV, self.D2, self.DV, self.dtype, self.BLOCK_N, self.K_PAD,
                                         self.n_rowscales, self.functors.o_scale_one, 2 if n_split > 1 else 1,
                                         self.functors.softmax if ws else None, paged, heads)
+            if paged and ws and not by_length:
+                cfg_src += "#define AE_BY_LENGTH 0\n"
             if key[-1]:
                 cfg_src += "#define AE_CLOCK_STAMPS 1\n"
             module = rt.compile_module(self.template, {"ae_config.h": cfg_src, "ae_functors.h": self.functor_src},
@@ -792,7 +794,7 @@ class MLADecodeOp(_SplitTuning):
                 lds = self.N_STAGES * self.BLOCK_N * 2 * self.D
             cfg = rt.TileCfg(block_m=heads, block_n=self.BLOCK_N, threads=threads, lds_bytes=lds,
                              head_dim=self.D, head_dim_v=self.DV, elem_bytes=2,
-                             n_rowscales=self.n_rowscales, mask_mode=0, paged=(2 if ws else 1) if paged else 0)
+                             n_rowscales=self.n_rowscales, mask_mode=0, paged=(2 if by_length else 1) if paged else 0)
             v = self._variants[key] = (module, cfg, cfg_src)
         return v
 
@@ -890,7 +892,7 @@ class MLADecodeOp(_SplitTuning):
             self._tune_splits(key, cands, lambda: self._launch(q1, q2, k1, k2, B, Hq, Hkv, Skv, paged),
                               lambda n: n > 0 and made_of(n) == n)
         heads, n_split, kv_per_split, *by_length = self.plan(B, Hq, Hkv, Skv, page=paged[2] if paged is not None else None)
-        module, cfg, _ = self._variant(n_split, paged is not None, heads)
+        module, cfg, _ = self._variant(n_split, paged is not None, heads, bool(by_length))
         ccfg = self._merges.cfg(n_split)
         out = torch.empty((B, 1, Hq, self.DV), dtype=self.dtype, device=dev)
         rowscales = [torch.empty((B, Hq, 1), dtype=torch.float32, device=dev) for _ in range(self.n_rowscales)]

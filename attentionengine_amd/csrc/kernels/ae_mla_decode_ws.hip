@@ -50,6 +50,12 @@
 #ifndef AE_PAGED
 #define AE_PAGED 0
 #endif
+// 0 (paged cache): never asked to split the entries by their lengths (ae_tile_cfg.paged 1).  Asked at run time, a launch of equal
+// spans waits for the answer in front of its first request, 64 heads a workgroup: B33 H128 up to 3968 tokens 52.8 us, 52.0 with 0, B56
+// 5056 81.0 and 80.4.
+#ifndef AE_BY_LENGTH
+#define AE_BY_LENGTH 1
+#endif
 #define AE_D (AE_D1 + AE_D2)
 #define AE_NWAVES 8
 #define AE_NT (AE_NWAVES * 64)
@@ -201,7 +207,11 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
   int b;
 #if AE_PAGED
   // (splits by the entries' lengths: see ae_split_by_length)
+#if AE_BY_LENGTH
   const bool by_length = p.tail_slots != 0;
+#else
+  constexpr bool by_length = false;
+#endif
   const int table_ints = (p.batch - 1) * p.block_table_stride + ((p.page_block_size & (p.page_block_size - 1)) == 0
                                         ? (p.seqlen_kv + p.page_block_size - 1) >> __builtin_ctz(p.page_block_size)
                                         : (p.seqlen_kv + p.page_block_size - 1) / p.page_block_size);
