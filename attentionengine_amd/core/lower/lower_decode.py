@@ -681,7 +681,9 @@ class MLADecodeOp(_SplitTuning):
         fitted to 1738 calls (62 shapes, every form), 5 % off; a batch spread evenly counts 1, one that fills its tables 0.7, and may
         take 1.08 of its time at most.  Over those shapes, evenly spread 0.98 of the time (30 shapes keep their plan; B8 H128
         2048 18.4 -> 16.4 us, B64 H128 4096 85 -> 64, B30 H64 2560 26.8 -> 24.1), full tables 0.99 (18.7 -> 19.1, 139 -> 102, 49.4 ->
-        31.6; 1.07 at most, B24 H128 1024 25.4 -> 27.2).  Fewer than four entries have little to share: up to 1.5 us slower, the lengths are waited for."""
+        31.6; 1.07 at most, B9 H128 1792 20.3 -> 21.7 with 19.7 -> 17.1 where spread).  Fewer than four entries have little to share: up to 1.5 us slower, the lengths are waited for.
+        In tables of up to 32 tiles a split has few trips, and the cost of full ones is 4 to 8 % low (spread | full, us: B14 H128 768 15.8 -> 15.8 |
+        17.4 -> 18.5, B26 H64 768 15.9 -> 15.0 | 16.6 -> 18.4, B24 H128 1024 23.3 -> 21.2 | 25.3 -> 27.1): they may not take longer by it."""
         if batch < 4 or tiles < 8:
             return None
 
@@ -701,6 +703,7 @@ class MLADecodeOp(_SplitTuning):
             return (((-(-n * -(-group // heads) // cus) * (f + c * per)) ** 4 + read ** 4) ** 0.25 + 0.32 * group * 4e-6 * dv * n
                     + 0.05 * most + 0.5)
         full, spread = (MLADecodeOp._call_us(batch, group, tiles, *fixed, cus, d, dv, s) for s in (False, True))
+        may_take = (1.08 if tiles > 32 else 1.0) * full
         best = None
         for heads in MLADecodeOp.LENGTH_COST:
             if heads != 16 and group <= heads // 2:
@@ -714,7 +717,7 @@ class MLADecodeOp(_SplitTuning):
                         continue
                     this_full = us(heads, n_wgs, most, False)
                     cost = us(heads, n_wgs, most, True) + 0.7 * this_full
-                    if this_full <= 1.08 * full and cost < spread + 0.7 * full and (best is None or cost < best[0]):
+                    if this_full <= may_take and cost < spread + 0.7 * full and (best is None or cost < best[0]):
                         best = cost, heads, most, n_wgs
         return best[1:] if best else None
 
