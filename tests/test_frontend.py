@@ -1042,3 +1042,23 @@ def test_a_build_with_clock_stamps_is_launched_as_one_only(monkeypatch):
     assert builds()[0] is stamped[0] and stamped[0][0] is not plain[0][0] and stamped[1][0] is not plain[1][0]
     monkeypatch.delenv("AE_CLOCK_STAMPS")
     assert builds()[0] is plain[0] and builds()[1] is plain[1]
+
+
+def test_which_paged_tables_are_cut_by_their_entries_lengths():
+    """MLADecodeOp._splits_by_length: no plan below its batch and table limits, none up to 32 tiles where full tables would take
+    longer, and every plan has a workgroup an entry at least and no more splits than tiles."""
+    from core.lower.lower_decode import MLADecodeOp as Op
+
+    def plan(batch, group, tiles):
+        fixed = Op._cheapest(batch, group, tiles, (1, min(Op.MAX_SPLITS, tiles)), 256, 576, 512, True)
+        return Op._splits_by_length(batch, group, tiles, fixed, 256, 576, 512)
+    assert plan(3, 128, 64) is None and plan(8, 128, 7) is None
+    assert plan(8, 128, 64) is not None
+    assert all(plan(*c) is None for c in ((14, 128, 24), (26, 64, 24), (24, 128, 32)))
+    for batch in (4, 17, 33, 64):
+        for group in (16, 40, 64, 128):
+            for tiles in (8, 32, 33, 150):
+                by_length = plan(batch, group, tiles)
+                if by_length is not None:
+                    heads, most, n_wgs = by_length
+                    assert heads in (16, 32, 64) and 2 <= most <= tiles and n_wgs >= batch
