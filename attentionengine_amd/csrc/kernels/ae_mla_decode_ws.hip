@@ -212,9 +212,11 @@ void ae_mla_decode_split_kernel(const ae_attn_params p) {
 #else
   constexpr bool by_length = false;
 #endif
-  const int table_ints = (p.batch - 1) * p.block_table_stride + ((p.page_block_size & (p.page_block_size - 1)) == 0
+  // (rows may lie any distance apart: 64 bits, as for `pages` below)
+  const int64_t all_ints = (int64_t)(p.batch - 1) * p.block_table_stride + ((p.page_block_size & (p.page_block_size - 1)) == 0
                                         ? (p.seqlen_kv + p.page_block_size - 1) >> __builtin_ctz(p.page_block_size)
                                         : (p.seqlen_kv + p.page_block_size - 1) / p.page_block_size);
+  const int table_ints = all_ints <= AE_WHOLE_TABLE ? (int)all_ints : AE_WHOLE_TABLE + 1;
   int table_all[AE_WHOLE_TABLE / 64];
   bool whole_table = false;
   int per_split = p.kv_per_split, n_mine = 0, len_b = 0;

@@ -813,3 +813,28 @@ def test_paged_entries_split_by_their_lengths(cuda_device, dtype, H, heads, page
         graph.replay()
         torch.cuda.synchronize()
         check(out, lse, other)
+
+
+@pytest.mark.parametrize("stride", [8, 9, 66, 1000, 34087043])
+def test_paged_entries_split_by_their_lengths_from_a_strided_table(cuda_device, stride):
+    """Rows of the block table that lie further apart than they are wide: read whole up to 512 integers from the first to the
+    last, else a split's part; 63 rows of 34087043 integers are more than 32 bits count."""
+    print(f"case mla by length, table rows {stride} apart", flush=True)
+    dtype, H, page, width, D, DV, scale = torch.float16, 16, 32, 8, 576, 512, 1 / math.sqrt(576)
+    B = 64 if stride > 2000 else 8
+    lens = [(37 * b) % (width * page) + 1 for b in range(B)]
+    q, q_pe, kv, k_pe = _mla_inputs(B, H, 1, width * page, DV, D - DV, dtype, seed=stride % 100)
+    pages = torch.randperm(B * width, generator=torch.Generator().manual_seed(1)).to(torch.int32)
+    cache = torch.empty(B * width, page, 1, D, dtype=dtype)
+    cache[pages.long()] = torch.cat([kv, k_pe], -1).view(B * width, page, 1, D)
+    table = torch.empty(B * stride, dtype=torch.int32, device="cuda").view(B, stride)[:, :width]
+    table.copy_(pages.view(B, width))
+    mod = _mla_engine(B, H, 1, width * page, D, DV, dtype, scale, backend="cute")
+    mod.attention.plan = lambda *a, **k: (16, 2, 128, 2 * B)
+    seqlens = torch.tensor(lens, dtype=torch.int32).cuda()
+    for _ in range(2):                       # through Python, then through the native host path
+        out, lse = mod(torch.cat([q, q_pe], -1).cuda(), cache.cuda(), block_table=table, cache_seqlens=seqlens)
+        for b, n in enumerate(lens):
+            ref, lref = R.mla_decode(q[b:b + 1, 0], q_pe[b:b + 1, 0], kv[b:b + 1, :n], k_pe[b:b + 1, :n], scale=scale)
+            assert (out[b:b + 1, 0].float().cpu() - ref).abs().max().item() <= OUT_TOL, b
+            assert (lse[b:b + 1, :, 0].cpu() - lref).abs().max().item() <= LSE_TOL, b
