@@ -645,15 +645,28 @@ class MLADecodeOp(_SplitTuning):
         those that do are not spread evenly, so a round is full at 1/1.4 of the CUs (B8 H128, 2048 tokens at most, 16 heads: 5
         splits, 192 live workgroups 19.4 us, 6, 224 22.9).
 
-        Kept by the number of tiles: a latent cache that grows by a token a call asks anew every 32 calls (20 to 40 us; the 3 x 64
-        candidates evaluated at every length took 130 to 270, more than the choice gains)."""
+        Kept by the number of tiles: a latent cache that grows by a token a call asks anew every 32 calls (25 to 35 us, paged 45 to
+        65; the 3 x 64 candidates evaluated at every length took 130 to 270, more than the choice gains, and with a function called
+        for each candidate it is 60 to 85, 105 to 145)."""
+        read = units * tiles * MLADecodeOp.BLOCK_N * 2e-6 * d / 5.7
+        partial = 0.31 * units * group * 4e-6 * dv
         splits = sorted({-(-tiles // -(-tiles // n)) for n in range(n_splits[0], n_splits[1] + 1)})      # (none without tiles)
         best = None
-        for heads in MLADecodeOp.ROUND_COST:
+        for heads, (f, c) in MLADecodeOp.ROUND_COST.items():
             if heads != 16 and group <= heads // 2:
                 continue
+            wgs = units * -(-group // heads)
             for n in splits:
-                us = sum(MLADecodeOp._call_us(units, group, tiles, heads, n, cus, d, dv, spread) for spread in ((False, True) if paged else (False,)))
+                trip = f + c * -(-tiles // n)
+                us = ((-(-wgs * n // cus) * trip) ** 4 + read ** 4) ** 0.25
+                if n > 1:
+                    us += 1.2 + 0.077 * n + partial * n
+                if paged:
+                    live = (n + 1) / (2 * n)
+                    rounds = math.ceil(math.ceil(wgs * n * (live * 1.4 if n > 1 else 1.0) - 1e-6) / cus)
+                    us += ((rounds * trip) ** 4 + (read * (0.5 if n > 1 else 1.0)) ** 4) ** 0.25
+                    if n > 1:
+                        us += 1.2 + 0.077 * n + partial * n * live
                 if best is None or (us, -heads, n) < best:
                     best = us, -heads, n
         return -best[1], best[2]

@@ -2,6 +2,7 @@
 force), mask_mod lowering, functor emission + hipRTC compilation (no GPU needed), engine dispatch
 and error behaviour."""
 import math
+import sys
 
 import numpy as np
 import pytest
@@ -1062,3 +1063,33 @@ def test_which_paged_tables_are_cut_by_their_entries_lengths():
                 if by_length is not None:
                     heads, most, n_wgs = by_length
                     assert heads in (16, 32, 64) and 2 <= most <= tiles and n_wgs >= batch
+
+
+def _work_of(f, *args):
+    """Interpreter steps of one call: what planning costs, without a clock."""
+    steps = 0
+
+    def trace(frame, event, _):
+        nonlocal steps
+        frame.f_trace_opcodes, frame.f_trace_lines = True, False
+        steps += event == "opcode"
+        return trace
+    before = sys.gettrace()
+    sys.settrace(trace)
+    try:
+        f(*args)
+    finally:
+        sys.settrace(before)
+    return steps
+
+
+def test_the_choice_among_equal_spans_is_cheap():
+    """MLADecodeOp._cheapest is asked anew whenever the cache grows by a tile: some 80 interpreter steps a
+    candidate and kind of batch (160 with a function called for each)."""
+    from core.lower.lower_decode import MLADecodeOp as Op
+    for batch, group, tiles in ((1, 128, 64), (8, 128, 64), (33, 128, 128), (64, 64, 128), (21, 64, 66)):
+        splits = {-(-tiles // -(-tiles // n)) for n in range(1, min(Op.MAX_SPLITS, tiles) + 1)}
+        forms = sum(h == 16 or group > h // 2 for h in Op.ROUND_COST)
+        for paged in (False, True):
+            work = _work_of(Op._cheapest.__wrapped__, batch, group, tiles, (1, min(Op.MAX_SPLITS, tiles)), 256, 576, 512, paged)
+            assert work <= 110 * len(splits) * forms * (1 + paged), (batch, tiles, paged, work)
