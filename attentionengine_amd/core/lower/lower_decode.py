@@ -683,56 +683,98 @@ class MLADecodeOp(_SplitTuning):
         return us + (1.2 + 0.077 * n + 0.31 * units * group * 4e-6 * dv * n * live if n > 1 else 0.0)
 
     @staticmethod
+    def _length_us(batch, group, tiles, heads, most, n_wgs, cus, d, dv, spread):
+        """... and of one plan by the entries' lengths.  The kernel's cut in closed form: of full tables every entry has as many
+        splits as its share of the workgroups; of lengths that are spread evenly (``total`` tiles) an entry's last split is half
+        full on average."""
+        total = (tiles * (batch + 1) + batch - 1) / 2 if spread else tiles * batch
+        if spread:
+            per = max(4, math.ceil((total - batch / 2) / (n_wgs - batch / 2)), -(-tiles // most))
+            splits = min(n_wgs, math.ceil(total / per + batch / 2 * (1 - 1 / per)))
+        else:
+            per = max(4, -(-tiles // min(most, n_wgs // batch)))
+            splits = batch * -(-tiles // per)
+        f, c = MLADecodeOp.LENGTH_COST[heads]
+        read = total * MLADecodeOp.BLOCK_N * 2e-6 * d / 4.8
+        return (((-(-splits * -(-group // heads) // cus) * (f + c * per)) ** 4 + read ** 4) ** 0.25 + 0.32 * group * 4e-6 * dv * splits
+                + 0.05 * most + 0.5)
+
+    @staticmethod
+    def _second_round(spans, n, n_ht, cus):
+        """Whether equal spans, ``n`` an entry and ``n_ht`` head tiles each, take a second round of the CUs; ``spans``: how many of
+        them hold keys, by entry.  More workgroups than CUs do.  Fewer may have to wait: ``ae_mla_decode_fwd`` pads an entry's ids
+        to an odd number, an XCD deals its workgroups to its four shader engines in turn, in the order of their ids, and
+        where the turn comes to an engine whose CUs are taken - by an empty workgroup too -, all behind it wait until one of those
+        has ended.  Right about 1022 of 1026 calls of 460 shapes, full tables and lengths of 0.8 to 1 of them (B21 H64 2624 tokens, 32 heads a
+        workgroup, 6 splits, 252 workgroups: full tables 40.6 us, entries spread evenly 23.7)."""
+        if sum(spans) * n_ht > cus:
+            return True
+        ids = n | 1 if len(spans) * n * n_ht > 128 else n
+        engine = max(1, cus // 32)
+        for xcd in range(8):
+            taken, waits, turn = [0] * 4, False, 0
+            for unit in range(xcd, len(spans) * ids, 8):
+                live = unit % ids < spans[unit // ids]
+                for _ in range(n_ht):
+                    waits = waits or taken[turn & 3] == engine
+                    if waits and live:
+                        return True
+                    taken[turn & 3] += live
+                    turn += 1
+        return False
+
+    @staticmethod
     @functools.lru_cache(maxsize=1024)
     def _splits_by_length(batch, group, tiles, fixed, cus, d, dv):
         """(query heads of a workgroup, the most splits of an entry, workgroups a head tile) for a paged call whose kernel cuts the
         entries by their lengths (``ae_split_by_length`` of csrc/kernels/ae_device.h), None where ``fixed``, (heads, splits) of
         equal spans of the table, is the better plan.
 
-        With equal spans the host plans for entries that fill their tables, and shorter ones leave workgroups without keys (B8
-        H128, up to 2048 tokens: 96 of 256).  Cut by length, every workgroup of a whole number of rounds has about as many tiles.  Costs
-        fitted to 1738 calls (62 shapes, every form), 5 % off; a batch spread evenly counts 1, one that fills its tables 0.7, and may
-        take 1.08 of its time at most.  Over those shapes, evenly spread 0.98 of the time (30 shapes keep their plan; B8 H128
-        2048 18.4 -> 16.4 us, B64 H128 4096 85 -> 64, B30 H64 2560 26.8 -> 24.1), full tables 0.99 (18.7 -> 19.1, 139 -> 102, 49.4 ->
-        31.6; 1.07 at most, B9 H128 1792 20.3 -> 21.7 with 19.7 -> 17.1 where spread).  Fewer than four entries have little to share: up to 1.5 us slower, the lengths are waited for.
-        In tables of up to 32 tiles a split has few trips, and the cost of full ones is 4 to 8 % low (spread | full, us: B14 H128 768 15.8 -> 15.8 |
-        17.4 -> 18.5, B26 H64 768 15.9 -> 15.0 | 16.6 -> 18.4, B24 H128 1024 23.3 -> 21.2 | 25.3 -> 27.1): they may not take longer by it."""
-        if batch < 4 or tiles < 8:
+        Equal spans are planned for tables that may be full, and shorter entries leave workgroups without keys.  Cut by length,
+        the workgroups of one round have about as many tiles each, but they wait for the lengths in front of their first request,
+        0.2 to 0.8 us.  So tables whose equal spans are one round keep them: full ones would lose what spread entries gain (us,
+        spread | full: B8 H128 2048 tokens 18.7 -> 17.4 | 19.9 -> 20.2, B9 H128 1792 20.0 -> 17.2 | 20.2 -> 21.7, B5 H128 4736 23.7 -> 20.7 |
+        23.7 -> 24.5, B11 H64 3712 21.3 -> 19.0 | 22.5 -> 24.3).  By length go tables
+
+        - whose equal spans take more than one round when they are full and also with lengths of 0.8 to 1 of the table (``_second_round``):
+          of many spans the last ones of such entries are empty, and the others may fit a round (B16 H64, 8 spans: 1.05 of the time);
+        - whose head tiles share a round's workgroups evenly (cut in shares of 85 and 42, 96 heads took up to 1.4 of the time),
+          with no more than a fifth of them without a split when the entries are full (B46 H96: 1.02 of the time on full tables with a third);
+        - with as many splits for a long entry as twice its share, so that it may be twice the mean, and more than equal spans
+          give it (one long entry of 64: 46 us with 4 splits, 40 with 6, equal spans 43);
+        - if by the costs spread entries take at most 0.96 of the time, and a spread and 0.7 of a full call no more than with equal
+          spans (the costs of spread entries are 6 % off, of full tables 12 %: these decide little, the rounds most).
+
+        905 such shapes (5 to 64 entries, 32 to 128 heads), time over that of equal spans, geometric mean (largest): lengths spread 0.76 (1.00), full
+        0.75 (1.00), drawn evenly 0.77 (1.01), 0.8 to 1 of the table 0.79 (0.95), all half of it 0.69 (0.97), a quarter and all of it in
+        turn 0.79 (1.02), one long entry among short ones 0.79 (0.98).  us, spread | full: B64 H128 4096 85.7 -> 61.9 | 130.8 -> 93.1, B21 H64 2624
+        23.7 -> 20.9 | 40.6 -> 26.8.  Planned in 5 to 60 us, once a table width."""
+        heads_fixed, n_fixed = fixed
+        if batch < 4 or n_fixed == 1:
             return None
-
-        def cut(lengths, n_wgs, most):
-            per = max(4, -(-sum(lengths) // n_wgs), -(-max(lengths) // most))
-            while True:
-                splits = [max(1, -(-t // per)) for t in lengths]
-                if sum(splits) <= n_wgs:
-                    return per, sum(splits)
-                per += max(1, per // 16)
-
-        def us(heads, n_wgs, most, spread):
-            lengths = [-(-tiles * (i + 1) // batch) for i in range(batch)] if spread else [tiles] * batch
-            per, n = cut(lengths, n_wgs, most)
-            f, c = MLADecodeOp.LENGTH_COST[heads]
-            read = sum(lengths) * MLADecodeOp.BLOCK_N * 2e-6 * d / 4.8
-            return (((-(-n * -(-group // heads) // cus) * (f + c * per)) ** 4 + read ** 4) ** 0.25 + 0.32 * group * 4e-6 * dv * n
-                    + 0.05 * most + 0.5)
-        full, spread = (MLADecodeOp._call_us(batch, group, tiles, *fixed, cus, d, dv, s) for s in (False, True))
-        may_take = (1.08 if tiles > 32 else 1.0) * full
         best = None
         for heads in MLADecodeOp.LENGTH_COST:
-            if heads != 16 and group <= heads // 2:
+            n_ht = -(-group // heads)
+            n_wgs = cus // n_ht
+            if (heads != 16 and group <= heads // 2) or cus % n_ht or batch > n_wgs or batch * (n_wgs // batch) < 0.8 * n_wgs:
                 continue
-            for rounds in range(1, 5):
-                n_wgs = rounds * cus // -(-group // heads)
-                if not batch <= n_wgs <= 64 * batch:
-                    continue
-                for most in (2, 4, 8, 16):
-                    if 2 * most > tiles or most * batch < 0.45 * n_wgs or most > 4 * n_wgs / batch + 2:
-                        continue
-                    this_full = us(heads, n_wgs, most, False)
-                    cost = us(heads, n_wgs, most, True) + 0.7 * this_full
-                    if this_full <= may_take and cost < spread + 0.7 * full and (best is None or cost < best[0]):
-                        best = cost, heads, most, n_wgs
-        return best[1:] if best else None
+            least = max(2 * n_wgs / batch, n_fixed + 1 if heads >= heads_fixed else 0)
+            most = next((n for n in (2, 3, 4, 6, 8, 12, 16, 24) if n >= least), None)
+            if most is None or 2 * most > tiles:
+                continue
+            full, spread = (MLADecodeOp._length_us(batch, group, tiles, heads, most, n_wgs, cus, d, dv, s) for s in (False, True))
+            if best is None or spread + 0.7 * full < best[0]:
+                best = spread + 0.7 * full, spread, (heads, most, n_wgs)
+        if best is None:
+            return None
+        full, spread = (MLADecodeOp._call_us(batch, group, tiles, *fixed, cus, d, dv, s) for s in (False, True))
+        if best[1] > 0.96 * spread or best[0] > spread + 0.7 * full:
+            return None
+        n_ht, per = -(-group // heads_fixed), -(-tiles // n_fixed)
+        nearly_full = [min(n_fixed, math.ceil(tiles * (0.8 + i * 37 % 64 / 320) / per)) for i in range(batch)]
+        if all(MLADecodeOp._second_round(spans, n_fixed, n_ht, cus) for spans in ([n_fixed] * batch, nearly_full)):
+            return best[2]
+        return None
 
     def plan(self, B, Hq, Hkv, Skv, page=None):
         """(query heads of a workgroup, number of splits, kv positions per split); with a paged cache a split spans at

@@ -398,13 +398,13 @@ AE_DEV int ae_wave_scan(int x) {
   step(__builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false));
   return x;
 }
-// The kv axes of all entries cut into splits of `tiles` kv tiles, the fewest with which p.tail_slots workgroups a head tile
-// suffice and no entry has more than p.num_splits: lane b's entry has `mine` of them (one at least), the entries up to it `upto`.
+// The kv axes of all entries cut into splits of `tiles` kv tiles, at most a sixteenth above the least with which p.tail_slots workgroups
+// a head tile suffice and no entry has more than p.num_splits: lane b's entry has `mine` of them (one at least), the entries up to it `upto`.
 // Equal spans of the table, which the host can plan, leave the workgroups without keys whose spans lie behind an entry's end, and the
 // launch takes as long as the longest entry's.  Every wave works this out from the lengths (0.2 us, and they are one trip to
-// memory that the first requests wait for).  us, equal spans -> so, entries spread evenly up to the table's width | all of that
-// width: B8 H128 2048 tokens 18.4 -> 16.4 | 18.7 -> 19.1, B64 H128 4096 85 -> 64 | 139 -> 102, B30 H64 2560 26.8 -> 24.1 | 49.4 -> 31.6,
-// B5 H128 4736 23.5 -> 19.6 | 24.1 -> 24.5.  Which calls take it: MLADecodeOp._splits_by_length.
+// memory that the first requests wait for: 0.2 to 0.8 us of a call).  us, equal spans -> so, entries spread evenly up to the table's width |
+// all of that width: B64 H128 4096 85.7 -> 61.9 | 130.8 -> 93.1, B21 H64 2624 23.7 -> 20.9 | 40.6 -> 26.8.  Where equal spans are one round of
+// the CUs, full tables are the slower for it (B8 H128 2048 18.7 -> 17.4 | 19.9 -> 20.2).  Which calls take it: MLADecodeOp._splits_by_length.
 struct ae_paged_splits { int tiles, mine, upto; };
 #define AE_LEAST_TILES 4      // (a split's start and end, and its partial result, take as long as four trips)
 AE_DEV ae_paged_splits ae_split_by_length(const ae_attn_params& p, int lane, int entry_tiles) {

@@ -838,3 +838,53 @@ def test_paged_entries_split_by_their_lengths_from_a_strided_table(cuda_device, 
             ref, lref = R.mla_decode(q[b:b + 1, 0], q_pe[b:b + 1, 0], kv[b:b + 1, :n], k_pe[b:b + 1, :n], scale=scale)
             assert (out[b:b + 1, 0].float().cpu() - ref).abs().max().item() <= OUT_TOL, b
             assert (lse[b:b + 1, :, 0].cpu() - lref).abs().max().item() <= LSE_TOL, b
+
+
+@pytest.mark.parametrize("B,H,page,width,dtype", [(31, 64, 64, 33, torch.bfloat16), (5, 128, 32, 80, torch.float16)])
+def test_a_paged_call_whose_plan_is_by_length(cuda_device, tmp_path, B, H, page, width, dtype):
+    """The plan that such a call gets by itself, against the oracle; ``tune=True`` times it beside equal spans and keeps what
+    the file says: 0 for it, else a number of equal spans, with which an entry's result does not depend on the others' lengths
+    (by length it does, in the rounding of the weights)."""
+    import json
+    print(f"case mla plan by length B{B} H{H} {width} pages of {page} {dtype}", flush=True)
+    D, DV, scale = 576, 512, 1 / math.sqrt(576)
+    key = (B, H, 1, width * page)
+    lens = [1 + (i * 977) % (width * page) for i in range(B)]
+    lens[1] = width * page
+    q, q_pe, kv, k_pe = _mla_inputs(B, H, 1, width * page, DV, D - DV, dtype, seed=B)
+    pages = torch.randperm(B * width, generator=torch.Generator().manual_seed(1)).to(torch.int32)
+    cache = torch.empty(B * width, page, 1, D, dtype=dtype)
+    cache[pages.long()] = torch.cat([kv, k_pe], -1).view(B * width, page, 1, D)
+    qq, cache, table = torch.cat([q, q_pe], -1).cuda(), cache.cuda(), pages.view(B, width).cuda()
+
+    def engine(**tuning):
+        return _mla_engine(B, H, 1, width * page, D, DV, dtype, scale, backend="cute", **tuning)
+
+    def call(mod, lens):
+        return [t.clone() for t in mod(qq, cache, block_table=table, cache_seqlens=torch.tensor(lens, dtype=torch.int32).cuda())]
+    mod = engine()
+    assert len(mod.attention.plan(*key, page)) == 4
+    out, lse = call(mod, lens)
+    for b, n in enumerate(lens):
+        ref, lref = R.mla_decode(q[b:b + 1, 0], q_pe[b:b + 1, 0], kv[b:b + 1, :n], k_pe[b:b + 1, :n], scale=scale)
+        assert (out[b:b + 1, 0].float().cpu() - ref).abs().max().item() <= OUT_TOL, b
+        assert (lse[b:b + 1, :, 0].cpu() - lref).abs().max().item() <= LSE_TOL, b
+    tuned = engine(tune=True, tune_file=str(tmp_path / "tuned.json"))
+    call(tuned, lens)
+    assert 0 in tuned.attention.tune_times and len(tuned.attention.tune_times) >= 3
+    for count in (0, 4):
+        file = tmp_path / f"{count}.json"
+        file.write_text((tmp_path / "tuned.json").read_text())
+        rec = json.loads(file.read_text())
+        rec[0]["tuned_config"] = [count]
+        file.write_text(json.dumps(rec))
+        again = engine(tune=True, tune_file=str(file))
+        for _ in range(2):                   # through Python, then through the native host path
+            got = call(again, lens)
+        assert again.attention.tune_times is None and again.attention._tuned[key] == count
+        assert len(again.attention.plan(*key, page)) == (4 if count == 0 else 3)
+        if count == 0:
+            assert torch.equal(got[0], out) and torch.equal(got[1], lse)
+        else:
+            other = call(again, [n if b == 1 else 1 + n // 3 for b, n in enumerate(lens)])
+            assert torch.equal(other[0][1], got[0][1]) and torch.equal(other[1][1], got[1][1])

@@ -1046,23 +1046,70 @@ def test_a_build_with_clock_stamps_is_launched_as_one_only(monkeypatch):
 
 
 def test_which_paged_tables_are_cut_by_their_entries_lengths():
-    """MLADecodeOp._splits_by_length: no plan below its batch and table limits, none up to 32 tiles where full tables would take
-    longer, and every plan has a workgroup an entry at least and no more splits than tiles."""
+    """MLADecodeOp._splits_by_length: no plan below its batch and table limits, none where the equal spans of full tables are
+    one round - cut by length those would take longer -, and every plan has a workgroup an entry at least, no more splits
+    than tiles, and more splits for a long entry than equal spans give it."""
     from core.lower.lower_decode import MLADecodeOp as Op
 
     def plan(batch, group, tiles):
         fixed = Op._cheapest(batch, group, tiles, (1, min(Op.MAX_SPLITS, tiles)), 256, 576, 512, True)
-        return Op._splits_by_length(batch, group, tiles, fixed, 256, 576, 512)
-    assert plan(3, 128, 64) is None and plan(8, 128, 7) is None
-    assert plan(8, 128, 64) is not None
-    assert all(plan(*c) is None for c in ((14, 128, 24), (26, 64, 24), (24, 128, 32)))
-    for batch in (4, 17, 33, 64):
+        return fixed, Op._splits_by_length(batch, group, tiles, fixed, 256, 576, 512)
+    assert plan(3, 128, 64)[1] is None and plan(8, 128, 7)[1] is None
+    assert all(plan(*c)[1] is None for c in ((14, 128, 24), (26, 64, 24), (24, 128, 32), (8, 128, 64), (9, 128, 56), (5, 128, 148), (16, 64, 130)))
+    by_length = {c: plan(*c) for c in ((64, 128, 128), (5, 128, 80), (21, 64, 82), (32, 64, 80), (31, 64, 66))}
+    assert all(p is not None for _, p in by_length.values())
+    for batch in range(4, 65):
         for group in (16, 40, 64, 128):
-            for tiles in (8, 32, 33, 150):
-                by_length = plan(batch, group, tiles)
-                if by_length is not None:
-                    heads, most, n_wgs = by_length
-                    assert heads in (16, 32, 64) and 2 <= most <= tiles and n_wgs >= batch
+            for tiles in (8, 32, 33, 64, 150):
+                c = batch, group, tiles
+                fixed, p = plan(*c)
+                if p is not None:
+                    by_length[c] = fixed, p
+    assert len(by_length) >= 15
+    for (batch, group, tiles), ((heads0, n0), (heads, most, n_wgs)) in by_length.items():
+        assert heads in (16, 32, 64) and 2 <= 2 * most <= tiles and n_wgs >= batch
+        assert n_wgs * -(-group // heads) == 256 and most >= 2 * n_wgs / batch
+        assert most > n0 or heads < heads0
+
+
+@pytest.mark.parametrize("spans,n,n_ht,second", [
+    ([4] * 8, 4, 8, False),       # 256 workgroups whose padding fits between them
+    ([6] * 5, 6, 8, True),        # 240, but an XCD has five units of eight
+    ([8] * 16, 8, 1, False),      # 128: not padded
+    ([8] * 16, 8, 2, True), ([8] * 16, 8, 3, True),
+    ([7] * 16, 8, 2, False),      # the last span of every entry is empty
+    ([4] * 3, 4, 8, False), ([1] * 8, 1, 32, False), ([1] * 4, 1, 64, True),
+])
+def test_when_equal_spans_take_a_second_round(spans, n, n_ht, second):
+    """MLADecodeOp._second_round over 256 CUs in 8 XCDs of 4 shader engines, against the same dispatch one workgroup at a time."""
+    from core.lower.lower_decode import MLADecodeOp as Op
+    assert Op._second_round(spans, n, n_ht, 256) is second
+    ids = n | 1 if len(spans) * n * n_ht > 128 else n
+    waits = sum(spans) * n_ht > 256
+    for xcd in range(8):
+        free, stuck = [8] * 4, False
+        queue = [unit % ids < spans[unit // ids] for unit in range(len(spans) * ids) if unit % 8 == xcd for _ in range(n_ht)]
+        for turn, live in enumerate(queue):
+            stuck = stuck or not free[turn % 4]
+            waits = waits or (stuck and live)
+            free[turn % 4] -= live and not stuck
+    assert bool(waits) is second
+
+
+def test_which_paged_calls_ask_for_splits_by_length():
+    """MLADecodeOp.plan: a fourth number where the kernel cuts the entries; equal spans for two latent heads, more entries than
+    a wave has lanes, tables of more pages than a workgroup keeps, a dense cache, and a split count that was tuned."""
+    from core.lower.lower_decode import MLADecodeOp as Op
+    op = AttentionEngine(_meta(64, 128, 1, 1, 256, 576, 512, torch.bfloat16), CustomIO({}), C.make_scale_score_mod(0.1), None,
+                         C.OnlineSoftmax(), kv_shared=True).attention
+    assert op.plan(64, 128, 1, 4096, 64) == (64, 6, -(-128 // 6) * 32, 128) and op.plan_splits(64, 128, 1, 4096, 64) == (6, 704)
+    assert len(op.plan(64, 128, 1, 32 * 1022, 32)) == 4
+    for args in ((65, 128, 1, 4096, 64), (64, 128, 1, 4096), (32, 256, 2, 4096, 64), (64, 128, 1, 32 * 1023, 32), (8, 128, 1, 2048, 64)):
+        assert len(op.plan(*args)) == 3, args
+    op._tuned[64, 128, 1, 4096] = 4
+    assert op.plan(64, 128, 1, 4096, 64) == (64, 4, 1024)
+    op._tuned[64, 128, 1, 4096] = 0
+    assert len(op.plan(64, 128, 1, 4096, 64)) == 4
 
 
 def _work_of(f, *args):
@@ -1093,3 +1140,15 @@ def test_the_choice_among_equal_spans_is_cheap():
         for paged in (False, True):
             work = _work_of(Op._cheapest.__wrapped__, batch, group, tiles, (1, min(Op.MAX_SPLITS, tiles)), 256, 576, 512, paged)
             assert work <= 110 * len(splits) * forms * (1 + paged), (batch, tiles, paged, work)
+
+
+def test_the_choice_of_splits_by_length_is_cheap():
+    """MLADecodeOp._splits_by_length is asked for every new batch and table width: no walk over the entries for each
+    candidate (190000 interpreter steps at 64 entries), and the dispatch is followed for the plans that are left."""
+    from core.lower.lower_decode import MLADecodeOp as Op
+    for batch in (4, 5, 8, 16, 17, 33, 64):
+        for group in (16, 64, 128):
+            for tiles in (8, 33, 64, 128, 250):
+                fixed = Op._cheapest(batch, group, tiles, (1, min(Op.MAX_SPLITS, tiles)), 256, 576, 512, True)
+                work = _work_of(Op._splits_by_length.__wrapped__, batch, group, tiles, fixed, 256, 576, 512)
+                assert work <= 20000, (batch, group, tiles, work)
