@@ -52,7 +52,12 @@ AE_DEV int ae_divide(int a, int d, int& rem) {
     q = a >> __builtin_ctz(d);
     rem = a & (d - 1);
   } else if (__builtin_expect(a < 1 << 22, 1)) {
-    q = ae_divide_small(a, d, rem);
+    // (ae_divide_small, written out: with a call of it the compiler lays the latent decode out differently, B8 H128 of 2048 tokens,
+    // paged, 18.55 -> 18.75 us)
+    q = __builtin_amdgcn_readfirstlane((int)((float)a * __builtin_amdgcn_rcpf((float)d)));
+    rem = a - q * d;
+    if (rem < 0) q--, rem += d;
+    if (rem >= d) q++, rem -= d;
   } else {
     q = a / d;
     rem = a - q * d;
