@@ -593,7 +593,7 @@ int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params
     if ((int64_t)p->block_table_stride * p->page_block_size < p->seqlen_kv)
       return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: %d table entries of %d tokens do not cover Skv=%d",
                   p->block_table_stride, p->page_block_size, p->seqlen_kv);
-    if (p->kv_per_split % cfg->block_n != 0)
+    if (p->tail_slots == 0 && p->kv_per_split % cfg->block_n != 0)
       return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: kv_per_split=%d is not a multiple of the %d-token kv tile",
                   p->kv_per_split, cfg->block_n);
     // splits by the entries' lengths: kernels that cut them (paged 2), a lane of a wave an entry, a split of any length
@@ -603,7 +603,10 @@ int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params
                                       "most %d each, by a kernel with paged=%d", p->tail_slots, p->batch, p->heads_kv, p->num_splits,
                   cfg->paged);
     // (the wave-specialised kernel keeps a split's part of the block table in LDS: AE_PTAB = 1024 entries)
-    if ((p->tail_slots != 0 ? p->seqlen_kv : p->kv_per_split) / p->page_block_size + 2 > 1024)
+    if (p->tail_slots != 0 && p->seqlen_kv / p->page_block_size + 2 > 1024)
+      return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: splits by the entries' lengths of a table of %d tokens, more than 1022 pages of %d "
+                                      "(use equal spans, or larger pages)", p->seqlen_kv, p->page_block_size);
+    if (p->tail_slots == 0 && p->kv_per_split / p->page_block_size + 2 > 1024)
       return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: a split of %d tokens spans more than 1022 pages of %d tokens "
                                       "(use more splits)", p->kv_per_split, p->page_block_size);
     // the paged kernels address the rope columns as an offset from the latent ones inside one cache tensor
@@ -624,8 +627,8 @@ int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params
   if (p->seqlen_q != 1)
     return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: seqlen_q=%d (decode handles one query token)",
                 p->seqlen_q);
-  if (p->num_splits <= 0 || p->kv_per_split <= 0 ||
-      (int64_t)p->num_splits * p->kv_per_split < p->seqlen_kv)
+  const bool by_length = cfg->paged && p->tail_slots != 0;      // (the kernel cuts the entries: kv_per_split is not read)
+  if (p->num_splits <= 0 || (!by_length && (p->kv_per_split <= 0 || (int64_t)p->num_splits * p->kv_per_split < p->seqlen_kv)))
     return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: %d splits of %d do not cover Skv=%d",
                 p->num_splits, p->kv_per_split, p->seqlen_kv);
   if ((rc = check_merge_splits("ae_mla_decode_fwd", combine_cfg, p->num_splits))) return rc;
@@ -645,7 +648,7 @@ int ae_mla_decode_fwd(ae_kernel* split, ae_kernel* combine, const ae_attn_params
   int64_t units = (int64_t)p->batch * p->heads_kv * p->num_splits, a_head = p->num_splits;
   if (cfg->paged && units * n_ht > 128) a_head |= 1;
   units = (int64_t)p->batch * p->heads_kv * a_head;
-  if (cfg->paged && p->tail_slots != 0) units = p->tail_slots;
+  if (by_length) units = p->tail_slots;
   int64_t total = ((units + 7) / 8) * 8 * n_ht;
   if (total > 0x7fffffffll) return fail(AE_ERR_INVALID_ARG, "ae_mla_decode_fwd: grid too large");
   uint32_t grid[3] = {(uint32_t)total, 1, 1};

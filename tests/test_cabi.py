@@ -188,6 +188,14 @@ def test_paged_cache_arguments_are_checked_before_any_launch():
     wide = dict(block_table_stride=2000, page_block_size=32, seqlen_kv=64000, num_splits=64, kv_per_split=1024)
     rc, msg = mla(params(**{**table, **wide, "tail_slots": 8}), cfg(paged=2))
     assert rc == 1 and "more than 1022 pages" in msg
+    assert "table of 64000 tokens" in msg and "equal spans" in msg and "more splits" not in msg
+    # ... for which kv_per_split is not read: every check of it is passed, and the next one names the work buffers
+    for unread in (0, -1, 31, 64):
+        rc, msg = mla(params(**{**table, "num_splits": 2, "kv_per_split": unread, "tail_slots": 8}), cfg(paged=2))
+        assert rc == 1 and "work buffers are NULL" in msg, (unread, msg)
+    for c in (1, 2):
+        rc, msg = mla(params(**{**table, "num_splits": 2, "kv_per_split": 64}), cfg(paged=c))
+        assert rc == 1 and "2 splits of 64 do not cover" in msg
     p = params(**table)
     assert lib.ae_prefill_fwd(fake, ctypes.byref(p), ctypes.byref(cfg()), None) == 1
     assert "reads a dense cache" in lib.ae_last_error().decode()
