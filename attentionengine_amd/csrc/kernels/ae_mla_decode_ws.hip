@@ -100,9 +100,9 @@
 #define AE_LB(i) (((i) * AE_LOADS + AE_BURSTS - 1) / AE_BURSTS)
 #ifndef AE_NSTAGE
 #define AE_NSTAGE 4
-#define AE_WHOLE_TABLE 512     // ... or the whole table, up to this
-#define AE_PTAB 1024      // paged cache: block-table entries of one split kept in LDS
 #endif
+#define AE_PTAB 1024                      // paged cache: block-table entries of one split kept in LDS
+#define AE_WHOLE_TABLE 512                // ... or of the whole table, up to this
 #define AE_PSTR 80                        // LDS pitch of one head's P row (32 kv * 2 B, padded against bank conflicts)
 #define AE_P_BYTES (AE_HEADS_PER_WG * AE_PSTR)
 #define AE_X_BYTES (AE_HEADS_PER_WG * 4 + 16)   // per-head rescale factors + one flag word per head block

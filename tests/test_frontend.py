@@ -1152,3 +1152,14 @@ def test_the_choice_of_splits_by_length_is_cheap():
                 fixed = Op._cheapest(batch, group, tiles, (1, min(Op.MAX_SPLITS, tiles)), 256, 576, 512, True)
                 work = _work_of(Op._splits_by_length.__wrapped__, batch, group, tiles, fixed, 256, 576, 512)
                 assert work <= 20000, (batch, group, tiles, work)
+
+
+def test_a_paged_build_takes_a_number_of_stages():
+    """AE_NSTAGE of the wave-specialised latent decode (4: its waits count the requests in flight) may come with the configuration,
+    for a paged cache too."""
+    from core.lower.lower_decode import render_mla_config
+    from core.runtime import hip_rt as rt
+    f = L.trace_functors(C.make_scale_score_mod(0.1), None, C.OnlineSoftmax(), CustomIO({}), torch.bfloat16)
+    cfg = render_mla_config(512, 64, 512, torch.bfloat16, 32, 0, 1, False, 2, f.softmax, True, 16) + "#define AE_NSTAGE 4\n"
+    names = f.final_rowscale_names
+    rt.compile_module("ae_mla_decode_ws.hip", {"ae_config.h": cfg, "ae_functors.h": L.render_functors(f) + lower_combine(C.OnlineSoftmax(), names)})
