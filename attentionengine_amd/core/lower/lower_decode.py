@@ -684,9 +684,10 @@ class MLADecodeOp(_SplitTuning):
 
     @staticmethod
     def _length_us(batch, group, tiles, heads, most, n_wgs, cus, d, dv, spread):
-        """... and of one plan by the entries' lengths.  The kernel's cut in closed form: of full tables every entry has as many
-        splits as its share of the workgroups; of lengths that are spread evenly (``total`` tiles) an entry's last split is half
-        full on average."""
+        """... and of one plan by the entries' lengths: rounds, the read at 4.8 TB/s, 0.32 us a MB of partial results (written, and
+        read by the merge), 0.05 a place of an entry in the merge, 0.5 for it.  The kernel's cut in closed form: of full tables every
+        entry has as many splits as its share of the workgroups; of lengths that are spread evenly (``total`` tiles) an entry's last
+        split is half full on average.  Fitted to 1738 calls of 62 shapes, every form."""
         total = (tiles * (batch + 1) + batch - 1) / 2 if spread else tiles * batch
         if spread:
             per = max(4, math.ceil((total - batch / 2) / (n_wgs - batch / 2)), -(-tiles // most))

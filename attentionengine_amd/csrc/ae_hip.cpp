@@ -694,7 +694,7 @@ int ae_prefill_bwd(ae_kernel* delta, ae_kernel* dkv, ae_kernel* dq, const ae_att
                     (long long)st);
   }
   // block_m / threads describe the dq launch (4 or 8 waves of 32 resident rows); dk/dv owns 128 rows, with 4 waves or 8
-  // in pairs, whose p and ds take 8 KiB of LDS a pair behind the tile ring
+  // of two kinds, whose p and ds take 8 KiB of LDS for 32 rows behind the tile ring
   // (table_rows 16: a value that no forward configuration has)
   const uint32_t dkv_waves = cfg->table_rows == 16 ? 8u : 4u;
   if (dkv_waves == 8 && (cfg->head_dim <= 0 || cfg->lds_bytes < 3 * (128 * (cfg->head_dim + cfg->head_dim_v) + 512) + 4 * 8192))

@@ -92,7 +92,8 @@ struct Plan {
   std::shared_ptr<Keep> keep;
   std::shared_ptr<BwdPlan> bwd;
   int64_t o_rows = 0, counters = 0;   // partial results a split launch writes; arrival counters behind the row scales
-  int tail_slots = 0;                 // prefill: q-tile slots of an XCD that several workgroups share
+  int tail_slots = 0;                 // prefill: q-tile slots of an XCD that several workgroups share; paged MLA: workgroups a
+                                      // head tile that share splits by the entries' lengths
 };
 
 // Work buffers of launches whose last workgroup merges: the arrival counters behind the row scales are zero when a

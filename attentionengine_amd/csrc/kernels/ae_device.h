@@ -38,8 +38,8 @@ typedef unsigned int ae_u32x2 __attribute__((ext_vector_type(2)));
 
 // Quotient and remainder of wave-uniform numbers, a >= 0 and d > 0.  The compiler's division is a chain of some thirty
 // dependent instructions, and which tile a workgroup has takes four of them in front of its first request: a shift where d
-// is a power of two, else a reciprocal whose quotient is off by at most one below 2^22.
-AE_DEV int ae_divide_small(int a, int d, int& rem) {       // a below 2^22
+// is a power of two, else a reciprocal, whose quotient is off by at most one below 2^22 (three roundings, 2^-22 of it together).
+AE_DEV int ae_divide_small(int a, int d, int& rem) {       // a below 2^31, a / d below 2^22
   int q = __builtin_amdgcn_readfirstlane((int)((float)a * __builtin_amdgcn_rcpf((float)d)));
   rem = a - q * d;
   if (rem < 0) q--, rem += d;
@@ -417,7 +417,7 @@ AE_DEV ae_paged_splits ae_split_by_length(const ae_attn_params& p, int lane, int
   const bool there = lane < p.batch;
   entry_tiles = there ? entry_tiles : 0;
   const int total = __builtin_amdgcn_readlane(ae_wave_scan<false>(entry_tiles), 63);
-  int rest;
+  int rest;           // (an entry has at most 2^19 tiles, and there are at most p.tail_slots entries: the quotient is no more than that)
   s.tiles = ae_divide_small(total + p.tail_slots - 1, p.tail_slots, rest);
   s.tiles = s.tiles > AE_LEAST_TILES ? s.tiles : AE_LEAST_TILES;
   for (;;) {            // (ends: with s.tiles at the longest entry's every entry has one split, and there are at most p.tail_slots entries)

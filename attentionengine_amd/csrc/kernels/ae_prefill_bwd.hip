@@ -17,8 +17,8 @@
 //     role 0 (dq):      resident rows = q  (Q, dO in registers), streamed tiles = K, V
 //     role 1 (dk, dv):  resident rows = kv (K, V in registers),  streamed tiles = Q, dO of every q head
 //                       of the kv head's group, with their lse and rowsum(do * o)
-// A wave owns 32 resident rows as the B operand (n = row) of v_mfma_f32_32x32x16, so a lane owns ONE
-// resident row: S[streamed, resident] = X1 R1^T and dP = X2 R2^T come out with the streamed rows in
+// A wave owns 32 resident rows (of AE_BWD_PAIRS 64, in two blocks) as the B operand (n = row) of v_mfma_f32_32x32x16, so a lane owns ONE
+// resident row of a block: S[streamed, resident] = X1 R1^T and dP = X2 R2^T come out with the streamed rows in
 // a lane's 16 accumulator registers, which makes the packed p and ds the B operand of the second
 // set of products, OUT^T[d, resident] += X^T[d, streamed] ds[streamed, resident], with X^T read from
 // the same LDS tile through ds_read_b64_tr_b16.  Streamed tiles (64 rows) go HBM -> LDS directly
@@ -35,7 +35,7 @@
 //
 // Waves per workgroup (AE_BWD_NWAVES, 32 resident rows each): dk/dv runs four, one per SIMD with the
 // whole register file (two accumulators), or, softmax attention without a tile table, eight of two kinds at head dims 128
-// (AE_BWD_PAIRS) and two workgroups a CU at head dims 64. dq has one accumulator and fits 256 registers, so it runs
+// (AE_BWD_PAIRS: 128 rows, 64 a wave) and two workgroups a CU at head dims 64. dq has one accumulator and fits 256 registers, so it runs
 // eight, two per SIMD (AE_BWD_WAVES_PER_EU 2, AE_AHEAD 3): a wave spends about half of its time waiting
 // (LDS fragments, MFMA results, the p/ds arithmetic between two sets of MFMAs) and the second wave
 // fills it - 0.59 -> 0.44 ms for B2 H32 S4096 D128 causal.
@@ -900,14 +900,15 @@ void AE_BWD_KERNEL(const ae_attn_bwd_params p) {
   // left at the last B, and is requested by the second kind alone: the first kind's stream (3900 of 4100 cycles a tile: 1200 scores,
   // 550 weights, 1130 hand-over, ds and the other weights, 250 from B to the first score, barriers) is the longer one, and with all
   // eight waves asking for the tile behind B each of them was held there for 850 to 950 cycles.  A lies behind a third of the
-  // second kind's products, where the first kind comes to it.  dk/dv launch, us, before and after: bf16 B4 H32 S2048 366 -> 351,
-  // fp16 B2 H32 S4096 617 -> 577, bf16 B8 H32 S875 197 -> 186, B2 Hq32 Hkv8 S2500 244 -> 235, fp16 B2 H16 S1000 36.0 -> 33.8.  With A
-  // or the requests elsewhere 1 to 6 % of that again; ds stored by dk's waves 394 where this took 364; kv tiles that follow each
-  // other in one workgroup without a gap 380 for 371 (K and V straight into registers: 5.7 us a tile, as long as the edges).
+  // second kind's products, where the first kind comes to it.  With A or the requests elsewhere it takes 1 to 6 % longer; B4 H32
+  // S2048, each beside a run of this: ds stored by dk's waves 394 us for 364; kv tiles that follow each other in one workgroup
+  // without a gap 380 for 371 (K and V straight into registers: 5.7 us a tile, as long as the edges).
   // LDS bound this: a wave of the first kind held 32 rows and took all 64 q rows, one of the second 32 rows of dk and of dv, and each
   // fragment fed one MFMA, 320 KB of fragments, row values and hand-over a tile at 128 bytes a clock, now 224.  dk/dv launch,
-  // us: causal fp16 B2 H32 S4096 644 -> 598, B2 Hq32 Hkv8 S2500 251 -> 233, bf16 B4 H32 S2048 356 -> 335, B2 H32 S1000 53.2 -> 51.5.
-  // Bits are the same.  The launch runs at the socket's power cap: 1.56 GHz, on inputs of zeros 2.1 (B4 H32 S2048 273 us).
+  // us, that -> fragments for two MFMAs -> requests by the second kind, one card: bf16 B4 H32 S2048 355 -> 339 -> 319, fp16 B2 H32 S4096
+  // 656 -> 620 -> 577, bf16 B8 H32 S875 178 -> 169 -> 166, B2 Hq32 Hkv8 S2500 244 -> 227 -> 224, fp16 B2 H16 S1000 36.4 -> 34.0 -> 32.2.
+  // Bits are the same.  The launch runs at the socket's power cap: 1.56 GHz, on inputs of zeros 2.1 (B4 H32 S2048 273 us).  At that clock the
+  // issue slots hold it: its waves are ready but not issued for 47 % of their time, the matrix pipe is 45 % busy.
   static_assert(AE_D == AE_DV && AE_NKS1 == AE_NKS2 && AE_RES_ONEPASS, "pairs: one head dim");
   ae_lds_byte* const ho = lds + 3 * AE_STAGE_BYTES + lane * 16;      // fragment i (p: 0..3, ds: 4..7) of 32 rows kb at + 8192 * kb + 1024 * i
   typedef __attribute__((address_space(3))) ae_u32x4 ae_lds_u32x4;
